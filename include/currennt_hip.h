@@ -130,19 +130,19 @@ typedef struct {
     float bias;  /* the layer's constant bias input ("bias" in the JSON)    */
 } cnt_lstm_desc;
 
-/* LstmLayer::LstmLayer (layers/LstmLayer.cu:1078-1268): allocates the per-direction state.  Layers with 64, 128,
- * 256 or 512 cells per direction and at most 32 parallel sequences run their recursions as persistent kernels;
- * any other geometry runs them step by step (one batched recurrent product and one cell kernel per time step, the
- * reference's own schedule), with the same results.
- * With 64, 128 or 256 cells per direction both recursions run on teams of workgroups that share one XCD's L2: a job
- * is a direction and up to four sequences, its team exchanges each step's outputs (forward) or partial errors
- * (backward) through that L2, and the launch asks for a little more than half of a compute unit's LDS so that every
- * workgroup of a team gets a compute unit of its own (two on one unit take their steps at the same moments and cost
- * a fifth of the step time).  Environment, read when a handle is created: CNT_LSTM_LOCAL=0 / CNT_LSTM_FWD_LOCAL=0
- * (the kernels that exchange across XCDs instead), CNT_LSTM_SPREAD_LDS=<bytes> (the LDS request, 0: none),
- * CNT_LSTM_LOCAL_JB=16 (16 instead of 8 cells per workgroup for 256-cell layers), CNT_LSTM_WARM=1 (a full-bandwidth
- * read of the states into the memory-side cache in front of the backward recursion), CNT_LSTM_MEM_DELAY=<units of 64
- * clocks> (how long the backward recursion's memory wave sleeps after a step's barrier), CNT_LSTM_STEPWISE=1. */
+/* LstmLayer::LstmLayer (layers/LstmLayer.cu:1078-1268): allocates the per-direction state.  Layers with up to 512 cells
+ * per direction run their recursions as persistent kernels, for any number of parallel sequences; larger ones run them
+ * step by step (one batched recurrent product and one cell kernel per time step, the reference's own schedule), with
+ * the same results.  A job is a direction and up to four sequences.  Up to 64 cells a job is one workgroup.  Above, it
+ * is a team of workgroups that share one XCD's L2 and exchange each step's outputs (forward) or partial errors
+ * (backward) through it; the launch asks for so much of a compute unit's LDS that every workgroup of a team gets a
+ * compute unit of its own (two on one unit take their steps at the same moments and cost a fifth of the step time).
+ * Environment, read when a handle is created: CNT_LSTM_SPREAD_LDS=<bytes> (the LDS request, 0: none),
+ * CNT_LSTM_LOCAL_JB=8|16 (cells per workgroup of a team), CNT_LSTM_SLOTS=<n> (workgroups of a recursion a compute unit may
+ * take), CNT_LSTM_SOLO=<cells> (largest layer run by one workgroup per job), CNT_LSTM_WARM=1 (a
+ * full-bandwidth read of the states into the memory-side cache in front of the backward recursion),
+ * CNT_LSTM_MEM_DELAY=<units of 64 clocks> (how long the backward recursion's memory wave sleeps after a step's barrier),
+ * CNT_LSTM_STEPWISE=1. */
 int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out);
 int cnt_lstm_destroy(cnt_lstm *h);
 /* LstmLayer::loadSequences (layers/LstmLayer.cu:1488-1533): records the fraction's geometry and
@@ -181,8 +181,8 @@ int cnt_lstm_backward_prev_errors(cnt_lstm *h, void *stream, const float *weight
  * pass stands at: a range that starts anywhere else is refused (CNT_ERR_ARG), and a pass that is abandoned half way
  * -- a range from step 0, cnt_lstm_backward_errors, cnt_lstm_forward or cnt_lstm_load_sequences before step curMaxT
  * was reached -- is dropped cleanly (the partial errors it left in the mailbox are discarded).  Only where
- * cnt_lstm_backward_can_split returns 1 (layers whose backward recursion runs as one persistent kernel per group of
- * sequences); elsewhere it is an error.
+ * cnt_lstm_backward_can_split returns 1 (layers of 64 cells per direction and more whose backward recursion runs as a
+ * persistent kernel); elsewhere it is an error.
  * cnt_lstm_backward_steps_done: the time steps [t_begin, t_end) whose deltas are final once `steps` steps have run
  * (both directions have passed them), i.e. what cnt_lstm_backward_prev_errors_range may already compute:
  * prev_errors columns of the time steps [t_begin, t_end) only.

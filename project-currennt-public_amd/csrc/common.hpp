@@ -53,12 +53,11 @@ constexpr float kMinLarg = 1.1754944e-038f;
 constexpr float kMinLogExp = -69.0776f;
 }  // namespace lim
 
+// The clamps are selects, not branches: a divergent branch costs a recursion's step more than the whole function.
 __device__ __forceinline__ float logistic(float x) {
-    if (x < lim::kExpLimit) {
-        if (x > -lim::kExpLimit) return 1.0f / (1.0f + expf(-x));
-        return 0.0f;
-    }
-    return 1.0f;
+    float y = 1.0f / (1.0f + expf(-x));
+    y = x > -lim::kExpLimit ? y : 0.0f;
+    return x < lim::kExpLimit ? y : 1.0f;
 }
 // The same functions from the hardware's exp2 and reciprocal (the library routines above spend about twenty instructions
 // on denormal results and on an exactly rounded quotient), for the forward recursion, where the five of them per cell
@@ -67,11 +66,9 @@ __device__ __forceinline__ float logistic(float x) {
 // relative error of |x| * 6e-8 in exp(-x).  The result stays within 4e-6 absolute of the exact logistic function
 // (8e-6 for tanh) over the whole unclamped range, which tests/test_gpu_core.py checks against the CPU functions.
 __device__ __forceinline__ float logistic_quick(float x) {
-    if (x < lim::kExpLimit) {
-        if (x > -lim::kExpLimit) return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * x));
-        return 0.0f;
-    }
-    return 1.0f;
+    float y = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * x));
+    y = x > -lim::kExpLimit ? y : 0.0f;
+    return x < lim::kExpLimit ? y : 1.0f;
 }
 __device__ __forceinline__ float tanh_quick(float x) { return 2.0f * logistic_quick(2.0f * x) - 1.0f; }
 __device__ __forceinline__ float logistic_deriv(float y) { return y * (1.0f - y); }
@@ -245,7 +242,7 @@ int lstm_take_failure(cnt_lstm *h);
 // every recursion launch anyway): what a stream needs that consumes the recursion's results, without another event
 // record on the launching stream
 int lstm_wait_recursion(cnt_lstm *h, hipStream_t other);
-int lstm_is_persistent(const cnt_lstm *h);  // its recursions are single launches (not the step-by-step schedule)
+int lstm_is_persistent(const cnt_lstm *h);  // its recursions are launches behind which lstm_wait_recursion finds an event
 int report_failure(cnt_network *net, hipStream_t stream);
 
 // ----- error halves that also do the backward step of the skip layer in front of them ----------------

@@ -1,8 +1,8 @@
 // XCD-local BPTT error recursion (included by lstm.hip inside its anonymous namespace).
 //
 // The parallel sequences of a fraction are independent chains, and so are the two directions of a bidirectional
-// layer.  The recursion is therefore cut into up to eight JOBS = (direction, group of at most four sequences), and
-// every job is run by a TEAM of G = H/JB workgroups that sit on ONE XCD: the all-to-all exchange of a step then
+// layer.  The recursion is therefore cut into JOBS = (direction, group of at most four sequences), and
+// every job is run by a TEAM of G = ceil(H/JB) workgroups that sit on ONE XCD: the all-to-all exchange of a step then
 // stays inside that XCD's L2 (plain stores, loads that only bypass the per-CU cache), which takes about half as
 // long as a hop through the memory side, and a step moves G*G*4*JB words per job instead of G*G*S*JB per direction.
 //
@@ -12,39 +12,47 @@
 // give the other XCDs' first teams a head start, so that with an even spread every XCD runs one job on its own
 // compute units, while any other spread still finds a team for every job: with W launched workgroups at least
 // (W - 8*(G-1)) / G teams complete, whatever the spread, and the launch uses W = njobs*G + 8*(G-1).  Workgroups
-// without a job end at once.
+// without a job end at once.  A launch never holds more jobs than complete teams fit the compute units at once (the
+// host cuts the jobs into launches): a team whose members could only become resident after another team has ended is not
+// waited for -- with 19-workgroup teams, one workgroup per compute unit and a second team left half resident, the
+// remaining workgroups were never dispatched and the launch gave up.
 //
 // Per workgroup (cells j0 .. j0+JB-1 of the job's direction, all T steps): the recurrent weights that read this
 // workgroup's gate deltas, W[h][k] for every cell h of the direction and k = (gate, own cell), live in registers
 // as operands of v_mfma_f32_4x4x1 (sixteen independent 4 x 4 outer products per instruction: four receiving cells
 // times the four sequences of the job).  Waves and roles, ONE LDS-only barrier per step (every LDS buffer exists twice,
 // by step parity):
-//   cell wave (1)      polls all words addressed to the workgroup (H/64 16-byte loads per lane, in address order: lane
+//   cell wave (1)      polls all words addressed to the workgroup (PW 16-byte loads per lane, in address order: lane
 //                      = sender * JB + chunk), sums them in registers and across lanes, and runs the cell update of the
 //                      4*JB elements straight from those registers; the step's coefficients were fetched from LDS
 //                      while the poll was in flight.  It issues no stores.
 //   product waves      after the barrier: multiply the fresh deltas with the weight slice, publish, hand the
-//   (H/64)             consumed words back as empty.  They never wait for a load.
+//   (PW = ceil(H/64))  consumed words back as empty.  They never wait for a load.
 //   memory wave (1)    every other global access: loads the inputs of the cell update three steps ahead, folds what
 //                      does not depend on the recursion into coefficients two steps ahead, writes the results of the
 //                      finished step to the state arrays.
 //
 // Mailbox of a job: plain 4-byte words [slot][receiver][sender][sequence][cell of the receiver], kEmpty = not
-// written yet, four slots, the receiver hands its words back as empty after use.  The ordering argument is the one
-// given for lstm_backward_chain; a store is acknowledged once the XCD's L2 holds it, which is where the team's
+// written yet, four slots, the receiver hands its words back as empty after use.  A store is acknowledged once the XCD's L2 holds it, which is where the team's
 // polls read.
 
 constexpr int kLocalSeqs = 4;     // sequences of a job (padded)
-constexpr int kLocalMaxJobs = 8;
-constexpr int kLocalTeams = 16;   // teams counted per XCD
-// control words (zero before every launch): tickets per XCD, jobs claimed, per (XCD, team) arrivals and job
-constexpr int kCtlTickets = 0, kCtlClaimed = 8, kCtlArrived = 16, kCtlTeamJob = kCtlArrived + 8 * kLocalTeams;
-constexpr int kCtlWords = kCtlTeamJob + 8 * kLocalTeams;
+constexpr int kLocalXcds = 8;
+// control words (zero before every launch): tickets per XCD, jobs claimed, per (XCD, team) arrivals and job; teams are
+// counted up to ChainParams::ctl_teams per XCD, which the launch makes large enough for all of its workgroups on one XCD
+constexpr int kCtlTickets = 0, kCtlClaimed = 8, kCtlArrived = 16;
+constexpr int ctl_words(int teams) { return kCtlArrived + 2 * kLocalXcds * teams; }
 constexpr unsigned kNoJob = 0xFFFFFFFFu;
 
-constexpr int local_threads(int H) { return (H / 64 + 2) * 64; }
-constexpr size_t local_job_words(int H, int JB) {
-    return (size_t)kMailSlots * (H / JB) * (H / JB) * kLocalSeqs * JB;
+constexpr int local_threads(int PW) { return (PW + 2) * 64; }
+constexpr size_t local_job_words(int G, int JB) { return (size_t)kMailSlots * G * G * kLocalSeqs * JB; }
+
+// Job -> direction and sequences: the sequences are dealt to the groups as evenly as possible, in order.
+struct LocalJob { int dir, seq0, nseq; };
+__device__ __forceinline__ LocalJob local_job(const ChainParams &p, int job) {
+    const int dir = job / p.groups, q = job % p.groups;
+    const int each = p.S / p.groups, more = p.S % p.groups;
+    return LocalJob{dir, q * each + min(q, more), each + (q < more ? 1 : 0)};
 }
 
 // The placement counters carry nothing but their own values (everything else a workgroup reads was written by earlier
@@ -54,24 +62,25 @@ __device__ __forceinline__ unsigned ctl_load(const unsigned *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Role of this workgroup: job * 64 + member, or -1.  Called by one thread.
+// Role of this workgroup: job * 64 + member (a team has at most 32 workgroups), or -1.  Called by one thread.
 __device__ int local_claim_role(const ChainParams &p, int G) {
     const unsigned xcd = __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15u;  // XCC_ID, bits 3:0
     if (xcd >= 8u) return -1;
     const unsigned ticket = __hip_atomic_fetch_add(p.ctl + kCtlTickets + xcd, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned team = ticket / (unsigned)G, member = ticket % (unsigned)G;
-    if (team >= (unsigned)kLocalTeams) return -1;
-    unsigned *arrived = p.ctl + kCtlArrived + xcd * kLocalTeams + team;
-    unsigned *team_job = p.ctl + kCtlTeamJob + xcd * kLocalTeams + team;
+    if (team >= (unsigned)p.ctl_teams) return -1;
+    unsigned *arrived = p.ctl + kCtlArrived + xcd * (unsigned)p.ctl_teams + team;
+    unsigned *team_job = arrived + kLocalXcds * p.ctl_teams;
     unsigned *claimed = p.ctl + kCtlClaimed;
     const unsigned before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     unsigned job = 0;  // 0: undecided, j + 1: job j, kNoJob: none
     if (before == (unsigned)G - 1u) {
         // this arrival completes the team
         if (team > 0) {
-            // head start for the first teams of the other XCDs: about 20 us, or until every job is taken
+            // head start for the earlier teams of the other XCDs: about 20 us, or until they can all have taken a job
             const long long t0 = wall_clock64();
-            while (ctl_load(claimed) < (unsigned)p.njobs && wall_clock64() - t0 < 2000) __builtin_amdgcn_s_sleep(8);
+            const unsigned enough = min((unsigned)p.njobs, team * (unsigned)kLocalXcds);
+            while (ctl_load(claimed) < enough && wall_clock64() - t0 < 2000) __builtin_amdgcn_s_sleep(8);
         }
         const unsigned c = __hip_atomic_fetch_add(claimed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         job = c < (unsigned)p.njobs ? c + 1u : kNoJob;
@@ -92,7 +101,7 @@ __device__ int local_claim_role(const ChainParams &p, int G) {
         }
     }
     if (job == kNoJob) return -1;
-    return (int)((job - 1u) * 64u + member);
+    return (int)((p.job0 + job - 1u) * 64u + member);
 }
 
 // Sum over the lanes that share lane % JB (the senders polled side by side, JB = 4 or 8); every lane ends up with
@@ -125,25 +134,26 @@ __device__ __forceinline__ float sender_sum(float v) {
 // Diagnostic trace (CNT_LSTM_TIMING): for four steps in the middle of the recursion every workgroup records when its
 // waves pass five points of a step, on the 100 MHz clock all compute units share.  32 entries per workgroup behind the
 // phase counters: [0] job, [1] member, [2] XCD, [4 + 5*i + k] stamp k of traced step i.
-constexpr int kTraceFirstStep = 100, kTraceSteps = 4, kTraceBase = 8 * 512, kTraceStride = 32;
+constexpr unsigned kTraceBlocks = 512;  // workgroups that record
+constexpr int kTraceFirstStep = 100, kTraceSteps = 4, kTraceBase = 8 * kTraceBlocks, kTraceStride = 32;
 __device__ __forceinline__ void trace_stamp(const ChainParams &p, int step, int k) {
-    if (p.phase_ticks && step >= kTraceFirstStep && step < kTraceFirstStep + kTraceSteps)
+    if (p.phase_ticks && blockIdx.x < kTraceBlocks && step >= kTraceFirstStep && step < kTraceFirstStep + kTraceSteps)
         p.phase_ticks[kTraceBase + (size_t)blockIdx.x * kTraceStride + 4 + 5 * (step - kTraceFirstStep) + k] = wall_clock64();
 }
 
-template <int H, int JB>
-__global__ __launch_bounds__(local_threads(H)) void lstm_backward_local(const ChainParams p) {
-    constexpr int G = H / JB;
+// PW = ceil(cells per direction / 64) product waves, JB cells per workgroup
+template <int PW, int JB>
+__global__ __launch_bounds__(local_threads(PW)) void lstm_backward_local(const ChainParams p) {
+    const int H = p.H, G = p.team;    // G = ceil(H / JB) workgroups; the last one may own fewer than JB cells
     constexpr int NSQ = kLocalSeqs;
-    constexpr int PW = H / 64;        // product waves
     constexpr int SPW = 64 / JB;      // senders side by side in the polling wave
-    constexpr int NL = G / SPW;       // 16-byte loads per polling lane
+    constexpr int NL = PW;            // 16-byte loads per polling lane; the last one may lie past the last sender
     constexpr int EL = NSQ * JB;      // (sequence, cell) elements of this workgroup: e = sequence * JB + cell
     constexpr int KW = 4 * JB;        // k extent of the product: (gate, own cell)
     constexpr int DP = KW + 4;        // pitch of a sequence's deltas in LDS (16-byte reads of four sequences: no bank shared)
     constexpr int PAIR = NSQ * JB;    // words of one (receiver, sender) pair
-    constexpr int RECV = G * PAIR;    // words one receiver gets per step
-    static_assert((JB == 4 || JB == 8 || JB == 16) && EL <= 64 && G % SPW == 0 && NL == PW, "local recursion geometry");
+    const unsigned RECV = (unsigned)(G * PAIR);  // words one receiver gets per step
+    static_assert((JB == 4 || JB == 8 || JB == 16) && EL <= 64 && PW >= 2, "local recursion geometry");
     enum { C_OG = 0, C_CE, C_NI, C_FG, C_IG, C_E, C_DOG, C_FGACT, C_DUMMY, NCOEF };
 
     __shared__ __attribute__((aligned(16))) float dl[2][NSQ][DP];
@@ -161,22 +171,24 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_backward_local(const Ch
     const int role = role_sh;
     if (role < 0) return;
     const int job = role >> 6, me = role & 63;
-    const int dir = p.job[job].dir, seq0 = p.job[job].seq0, nseq = p.job[job].nseq;
+    const LocalJob part = local_job(p, job);
+    const int dir = part.dir, seq0 = part.seq0, nseq = part.nseq;
     const DirPtrs &D = p.d[dir];
     const int S = p.S, T = p.T;
     const int j0 = me * JB;
     const int n = S * H;
-    float *const mailbox = p.lmail + (size_t)job * local_job_words(H, JB);
-    constexpr unsigned slot_words = (unsigned)G * RECV;
+    float *const mailbox = p.lmail + (size_t)job * local_job_words(G, JB);
+    const unsigned slot_words = (unsigned)G * RECV;
     const __amdgpu_buffer_rsrc_t mail =
-        __builtin_amdgcn_make_buffer_rsrc(mailbox, 0, (int)(local_job_words(H, JB) * sizeof(float)), 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(mailbox, 0, (int)(local_job_words(G, JB) * sizeof(float)), 0x00020000);
+    const int last_vectors = G * JB - 64 * (NL - 1);  // lanes whose last poll lies inside the senders' words
     auto slot_of = [&](int step) { return dir ? step : (T - 1 - step); };
 
     if (wave == PW + 1) {
         // ------------------------------------------------------------------ memory wave
         struct StepIn { float e, ni, ig, fg, og, dog_old, c, c_earlier; char pat; };
         const int ej = lane / JB, ec = lane % JB;  // element `lane`: sequence seq0 + ej, cell j0 + ec
-        const bool valid = lane < EL && ej < nseq;
+        const bool valid = lane < EL && ej < nseq && j0 + ec < H;
         const int s = seq0 + ej;
         auto load_step = [&](int step, StepIn &v) {
             v = StepIn{0, 0, 0, 0, 0, 0, 0, 0, 1};
@@ -214,7 +226,7 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_backward_local(const Ch
             put_coef(sb, first); put_coef(sb + 1, second);
         }
         load_step(sb + 2, in);
-        const bool mtiming = p.phase_ticks != nullptr;
+        const bool mtiming = p.phase_ticks != nullptr && blockIdx.x < kTraceBlocks;
         long long mbusy = 0;
         lds_barrier();  // start of the recursion
         for (int step = sb; step < p.step_end; ++step) {
@@ -244,9 +256,10 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_backward_local(const Ch
                 // front of the next poll in the compute unit's queue.
                 const u32x4 empty = {kEmpty, kEmpty, kEmpty, kEmpty};
 #pragma unroll
-                for (int q = 0; q < RECV / 256; ++q)
-                    __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)((step - 1) % kMailSlots) * slot_words * 4u +
-                                                           ((unsigned)me * RECV + (unsigned)(q * 64 + lane) * 4u) * 4u), 0, 0);
+                for (int q = 0; q < NL; ++q)
+                    if (q + 1 < NL || lane < last_vectors)
+                        __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)((step - 1) % kMailSlots) * slot_words * 4u +
+                                                               ((unsigned)me * RECV + (unsigned)(q * 64 + lane) * 4u) * 4u), 0, 0);
             }
             if (mtiming) mbusy += wall_clock64() - tm0;
         }
@@ -264,15 +277,16 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_backward_local(const Ch
 #pragma unroll
         for (int k = 0; k < KW; ++k) {
             const int g = k / JB, jj = k % JB;
-            wreg[k] = D.w_int[(size_t)g * p.L * H + (size_t)(j0 + jj) * H + h];
+            wreg[k] = h < H && j0 + jj < H ? D.w_int[(size_t)g * p.L * H + (size_t)(j0 + jj) * H + h] : 0.0f;
         }
         // the accumulator's four rows of lane (block b, sequence j) are the receiving cells 64*pw + 4*b .. + 3
         const int bj = lane & 3, first_cell = 64 * pw + 4 * (lane >> 2);
         const unsigned pub_off = ((unsigned)(first_cell / JB) * RECV + (unsigned)me * PAIR + (unsigned)bj * JB +
                                   (unsigned)(first_cell % JB)) * 4u;
+        const bool publishes = first_cell < G * JB;
         wait_all_vmem();
         lds_barrier();  // start of the recursion
-        const bool timing = p.phase_ticks != nullptr;
+        const bool timing = p.phase_ticks != nullptr && blockIdx.x < kTraceBlocks;
         long long busy = 0;
         for (int step = p.step_begin; step < p.step_end; ++step) {
             lds_barrier();  // the deltas of this step are in LDS
@@ -300,7 +314,8 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_backward_local(const Ch
                 // a NaN that happens to look like the empty marker is sent as the default NaN
                 v.x = v.x == kEmpty ? 0x7FC00000u : v.x; v.y = v.y == kEmpty ? 0x7FC00000u : v.y;
                 v.z = v.z == kEmpty ? 0x7FC00000u : v.z; v.w = v.w == kEmpty ? 0x7FC00000u : v.w;
-                __builtin_amdgcn_raw_buffer_store_b128(v, mail, (int)((unsigned)(step % kMailSlots) * slot_words * 4u + pub_off), 0, 0);
+                if (publishes)
+                    __builtin_amdgcn_raw_buffer_store_b128(v, mail, (int)((unsigned)(step % kMailSlots) * slot_words * 4u + pub_off), 0, 0);
             }
             if (tid == 64) trace_stamp(p, step, 4);
             if (failed) return;
@@ -317,22 +332,26 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_backward_local(const Ch
     // workgroup, i.e. chunk q = l % JB (four cells of one sequence) of sender i*SPW + l / JB
     const unsigned poll_off = ((unsigned)me * RECV + (unsigned)lane * 4u) * 4u;
     constexpr unsigned poll_stride = (unsigned)SPW * PAIR * 4u;
+    // lanes past the last sender poll their first vector once more and leave it out of the sum
+    const bool last_counts = lane < last_vectors;
+    const unsigned poll_off_last = last_counts ? poll_off + (unsigned)(NL - 1) * poll_stride : poll_off;
     // cell-update role: after the sum every lane holds its chunk's four totals; lane q + JB*r takes cell r of chunk q,
     // which is element e = q*4 + r = sequence*JB + cell
     const bool cell_lane = lane < EL;
     const int cr = cell_lane ? lane / JB : 0;
     const int e_id = cell_lane ? (lane % JB) * 4 + cr : 0;
     const int cj = e_id / JB, cc = e_id % JB;
+    const bool real_cell = cell_lane && j0 + cc < H;
     float p_ig = 0, p_fg = 0, p_og = 0;
-    if (cell_lane) { p_ig = D.peep[0][j0 + cc]; p_fg = D.peep[1][j0 + cc]; p_og = D.peep[2][j0 + cc]; }
+    if (real_cell) { p_ig = D.peep[0][j0 + cc]; p_fg = D.peep[1][j0 + cc]; p_og = D.peep[2][j0 + cc]; }
     float fg_later = 0, cerr_later = 0, dig_later = 0, dfg_later = 0;
-    if (p.step_begin > 0 && cell_lane && cj < nseq) {
+    if (p.step_begin > 0 && real_cell && cj < nseq) {
         // a launch that starts in the middle: what the step before carried over stands in the state arrays
         const size_t gi = (size_t)slot_of(p.step_begin - 1) * n + (size_t)(seq0 + cj) * H + j0 + cc;
         fg_later = D.fg[gi]; cerr_later = D.cerr[gi]; dig_later = D.dig[gi]; dfg_later = D.dfg[gi];
     }
     long long ph0 = 0, ph1 = 0, ph3 = 0, ph6 = 0, poll_rounds = 0;
-    const bool timing = p.phase_ticks != nullptr;
+    const bool timing = p.phase_ticks != nullptr && blockIdx.x < kTraceBlocks;
     const long long tk_begin = timing ? wall_clock64() : 0;
 
     wait_all_vmem();  // peepholes are in registers before the recursion starts
@@ -357,7 +376,7 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_backward_local(const Ch
             for (int d = 0; d < p.poll_delay; ++d) __builtin_amdgcn_s_sleep(1);
             for (;;) {
                 const long long tq0 = timing ? wall_clock64() : 0;
-                poll_load<NL>(slot, poll_off, poll_stride, w);
+                poll_load<NL>(slot, poll_off, poll_stride, poll_off_last, w);
                 unsigned worst = 0;
 #pragma unroll
                 for (int i = 0; i < NL; ++i) worst = max(max(worst, w[i].x), max(max(w[i].y, w[i].z), w[i].w));
@@ -373,7 +392,10 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_backward_local(const Ch
             }
             f32x4 sum = __builtin_bit_cast(f32x4, w[0]);
 #pragma unroll
-            for (int i = 1; i < NL; ++i) sum += __builtin_bit_cast(f32x4, w[i]);
+            for (int i = 1; i + 1 < NL; ++i) sum += __builtin_bit_cast(f32x4, w[i]);
+            const f32x4 far = __builtin_bit_cast(f32x4, w[NL - 1]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum[r] += last_counts ? far[r] : 0.0f;
             sum[0] = sender_sum<JB>(sum[0]); sum[1] = sender_sum<JB>(sum[1]);
             sum[2] = sender_sum<JB>(sum[2]); sum[3] = sender_sum<JB>(sum[3]);
             e += cr == 0 ? sum[0] : cr == 1 ? sum[1] : cr == 2 ? sum[2] : sum[3];

@@ -20,19 +20,21 @@
 //   memory wave (1)      input projections two steps ahead; gate activations, cell states and outputs of the finished
 //                        step to the state arrays.
 
-template <int H, int JB>
-__global__ __launch_bounds__(local_threads(H)) void lstm_forward_local(const ChainParams p) {
-    constexpr int G = H / JB;
+// PW = ceil(cells per direction / 64) gather waves, JB cells per workgroup
+template <int PW, int JB>
+__global__ __launch_bounds__(local_threads(PW)) void lstm_forward_local(const ChainParams p) {
+    const int H = p.H, G = p.team;       // G = ceil(H / JB) workgroups; the last one may own fewer than JB cells
     constexpr int NSQ = kLocalSeqs;
-    constexpr int PW = H / 64;           // gather waves
     constexpr int ROWS = 4 * JB;         // (gate, cell) rows of this workgroup: row = gate * JB + cell
-    constexpr int NQ = H / 64;           // 16-byte vectors per polling lane: 16 blocks x NQ x 4 cells = H
+    constexpr int NQ = PW;               // 16-byte vectors per lane that hand a block back; the last may lie past its end
     constexpr int EL = NSQ * JB;         // (sequence, cell) elements: e = sequence * JB + cell
     constexpr int PAIR = NSQ * JB;       // words one sender leaves in one receiver's block
     constexpr int CH = PAIR / 4;         // 16-byte chunks of those
-    constexpr int RECV = G * PAIR;       // words of a receiver's block = NSQ * H
-    constexpr int PUB = G / (64 / CH);   // publishing stores per lane
-    static_assert(EL <= 64 && G % (64 / CH) == 0 && RECV == 64 * 4 * NQ, "local forward geometry");
+    constexpr int RPS = 64 / CH;         // receivers served by one publishing store
+    constexpr int PUB = (64 * PW / JB + RPS - 1) / RPS;  // publishing stores per lane; the last may lie past the team
+    const unsigned RECV = (unsigned)(G * PAIR);  // words of a receiver's block
+    const int vectors = G * JB;          // 16-byte vectors of a receiver's block
+    static_assert(EL <= 64, "local forward geometry");
     enum { R_NI = 0, R_IG, R_FG, R_OG, R_C, R_H, NRES };
 
     __shared__ float red[2][PW][ROWS][NSQ];   // recurrent sums of the step, one share per gather wave
@@ -56,22 +58,23 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_forward_local(const Cha
     const int role = role_sh;
     if (role < 0) return;
     const int job = role >> 6, me = role & 63;
-    const int dir = p.job[job].dir, seq0 = p.job[job].seq0, nseq = p.job[job].nseq;
+    const LocalJob part = local_job(p, job);
+    const int dir = part.dir, seq0 = part.seq0, nseq = part.nseq;
     const DirPtrs &D = p.d[dir];
     const int S = p.S, T = p.T;
     const int j0 = me * JB;
     const int n = S * H;
-    float *const mailbox = p.flmail + (size_t)job * local_job_words(H, JB);
-    constexpr unsigned slot_words = (unsigned)G * RECV;
+    float *const mailbox = p.flmail + (size_t)job * local_job_words(G, JB);
+    const unsigned slot_words = (unsigned)G * RECV;
     const __amdgpu_buffer_rsrc_t mail =
-        __builtin_amdgcn_make_buffer_rsrc(mailbox, 0, (int)(local_job_words(H, JB) * sizeof(float)), 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(mailbox, 0, (int)(local_job_words(G, JB) * sizeof(float)), 0x00020000);
     auto slot_of = [&](int step) { return dir ? (T - 1 - step) : step; };
 
     if (wave == PW + 1) {
         // ------------------------------------------------------------------ memory wave
         struct StepIn { float a[4]; char pat; };
         const int cs = lane / JB, cj = lane % JB;
-        const bool valid = lane < EL && cs < nseq;
+        const bool valid = lane < EL && cs < nseq && j0 + cj < H;
         const int s = seq0 + cs;
         auto load_step = [&](int step, StepIn &v) {
             v = StepIn{{0, 0, 0, 0}, 1};
@@ -129,7 +132,7 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_forward_local(const Cha
         // ------------------------------------------------------------------ cell wave
         const int cs = lane / JB, cj = lane % JB;
         const bool cell_lane = lane < EL;
-        const bool cell_valid = cell_lane && cs < nseq;
+        const bool cell_valid = cell_lane && cs < nseq && j0 + cj < H;
         float b_ni = 0, b_ig = 0, b_fg = 0, b_og = 0, p_ig = 0, p_fg = 0, p_og = 0;
         if (cell_valid) {
             b_ni = p.bias * D.b[0][j0 + cj]; b_ig = p.bias * D.b[1][j0 + cj];
@@ -140,7 +143,8 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_forward_local(const Cha
         // receivers l / CH + (64 / CH) * i
         const int ch = lane % CH, ch_half = ch / NSQ, ch_seq = ch % NSQ;
         const unsigned pub_off = (((unsigned)(lane / CH)) * RECV + (unsigned)me * PAIR + (unsigned)ch * 4u) * 4u;
-        constexpr unsigned pub_stride = (unsigned)(64 / CH) * RECV * 4u;
+        const unsigned pub_stride = (unsigned)RPS * RECV * 4u;
+        const int pub_last = G - (PUB - 1) * RPS;   // receivers of the last store
         const unsigned reset_off = ((unsigned)me * RECV + (unsigned)lane * 4u) * 4u;
         float c_prev = 0.0f;
         wait_all_vmem();
@@ -198,14 +202,16 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_forward_local(const Cha
                 v.z = v.z == kEmpty ? 0x7FC00000u : v.z; v.w = v.w == kEmpty ? 0x7FC00000u : v.w;
 #pragma unroll
                 for (int i = 0; i < PUB; ++i)
-                    __builtin_amdgcn_raw_buffer_store_b128(v, mail, (int)((unsigned)(step % kMailSlots) * slot_words * 4u + pub_off + (unsigned)i * pub_stride), 0, 0);
+                    if (i + 1 < PUB || lane / CH < pub_last)
+                        __builtin_amdgcn_raw_buffer_store_b128(v, mail, (int)((unsigned)(step % kMailSlots) * slot_words * 4u + pub_off + (unsigned)i * pub_stride), 0, 0);
             }
             if (step > 0) {
                 // the words the gather waves read for this step are empty again
                 const u32x4 empty = {kEmpty, kEmpty, kEmpty, kEmpty};
 #pragma unroll
                 for (int q = 0; q < NQ; ++q)
-                    __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)((step - 1) % kMailSlots) * slot_words * 4u + reset_off + (unsigned)q * 1024u), 0, 0);
+                    if (q + 1 < NQ || lane < vectors - 64 * (NQ - 1))
+                        __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)((step - 1) % kMailSlots) * slot_words * 4u + reset_off + (unsigned)q * 1024u), 0, 0);
             }
         }
         lds_barrier();  // results of the last step are in LDS
@@ -222,21 +228,26 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_forward_local(const Cha
     constexpr int RG = ROWS / 4;         // groups of four rows
     constexpr int KQ = 16 / RG;          // residues of the source cell index dealt to the blocks
     constexpr int NI = 64 / KQ;          // MFMA instructions per step
-    static_assert(RG * KQ == 16 && (KQ == 2 || KQ == 4), "blocks of the recurrent product");
+    static_assert(RG * KQ == 16 && (KQ == 1 || KQ == 2 || KQ == 4), "blocks of the recurrent product");
     const int blk = lane >> 2, sub = lane & 3;  // A operand: row sub of the block; B operand and accumulator: sequence sub
     const int rg = blk % RG, kq = blk / RG;
     float wreg[NI];
     {
         const int o = rg * 4 + sub, g = o / JB, jj = o % JB;
-        const float *wg = D.w_int + (size_t)g * p.L * H + (size_t)(j0 + jj) * H + 64 * pw;
+        const float *wg = D.w_int + (size_t)g * p.L * H + (size_t)(j0 + jj) * H;
 #pragma unroll
-        for (int i = 0; i < NI; ++i) wreg[i] = wg[NI * kq + i];
+        for (int i = 0; i < NI; ++i) {
+            const int from = 64 * pw + NI * kq + i;
+            wreg[i] = from < H && j0 + jj < H ? wg[from] : 0.0f;
+        }
     }
     // the wave's own staging buffer: [sequence][cell], written as the words arrive, read back as B operands
     float (*hb)[64 + 4] = hstage[pw];
-    const unsigned poll_off = ((unsigned)me * RECV + (unsigned)(64 * pw + lane) * 4u) * 4u;
+    // a lane past the end of the block polls its wave's first vector instead and stages zeros
+    const bool inside = 64 * pw + lane < vectors;
+    const unsigned poll_off = ((unsigned)me * RECV + (unsigned)(64 * pw + (inside ? lane : 0)) * 4u) * 4u;
     long long ph0 = 0, ph1 = 0, ph2 = 0, ph3 = 0, poll_rounds = 0;
-    const bool timing = p.phase_ticks != nullptr;
+    const bool timing = p.phase_ticks != nullptr && blockIdx.x < kTraceBlocks;
     const long long tk_begin = timing ? wall_clock64() : 0;
     wait_all_vmem();
     lds_barrier();  // start of the recursion
@@ -250,7 +261,7 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_forward_local(const Cha
         unsigned spins = 0;
         for (int d = 0; d < p.poll_delay_fwd; ++d) __builtin_amdgcn_s_sleep(1);
         for (;;) {
-            poll_load<1>(slot, poll_off, 0u, w);
+            poll_load<1>(slot, poll_off, 0u, poll_off, w);
             const unsigned worst = max(max(w[0].x, w[0].y), max(w[0].z, w[0].w));
             if (timing) ++poll_rounds;
             if (worst != kEmpty) break;
@@ -264,6 +275,7 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_forward_local(const Cha
         }
         if (timing) ph1 += wall_clock64() - tk0;
         // this lane's vector: sequence sub, source cells 4*blk .. + 3 of the wave's 64
+        if (!inside) w[0] = u32x4{0, 0, 0, 0};
         *reinterpret_cast<f32x4 *>(&hb[sub][4 * blk]) = __builtin_bit_cast(f32x4, w[0]);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -277,7 +289,7 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_forward_local(const Cha
             acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(wreg[i4 + 3], hv[3], acc1, 0, 0, 0);
         }
         f32x4 sum = acc0 + acc1;
-        // the residues sit in lane bits 4 and 5 (KQ = 4) or in lane bit 5 (KQ = 2)
+        // the residues sit in lane bits 4 and 5 (KQ = 4), in lane bit 5 (KQ = 2), or there is only one (KQ = 1)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             float v = sum[r];
@@ -286,7 +298,7 @@ __global__ __launch_bounds__(local_threads(H)) void lstm_forward_local(const Cha
                 const auto x = __builtin_amdgcn_permlane16_swap(u, u, false, false);
                 v = __builtin_bit_cast(float, (unsigned)x[0]) + __builtin_bit_cast(float, (unsigned)x[1]);
             }
-            {
+            if (KQ >= 2) {
                 const unsigned u = __builtin_bit_cast(unsigned, v);
                 const auto x = __builtin_amdgcn_permlane32_swap(u, u, false, false);
                 v = __builtin_bit_cast(float, (unsigned)x[0]) + __builtin_bit_cast(float, (unsigned)x[1]);

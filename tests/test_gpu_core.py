@@ -491,3 +491,23 @@ def test_lstm_partial_recursion_rejects_what_it_cannot_do():
     assert layer.backward_steps_done(9) == (3, 9)
     assert layer.backward_steps_done(4) == (8, 8)   # nothing final yet in a bidirectional layer
     layer.close()
+
+
+@pytest.mark.parametrize("L,bidir,lengths", [
+    # one workgroup per job: one cell, the edges of its sixteen-cell waves, sequence groups that do not come out even
+    (1, False, [3]), (30, True, [9, 4]), (32, True, [1, 6, 6, 2, 5]), (34, True, [13, 8, 13]), (63, False, [7] * 9),
+    (128, True, [21, 3, 17] * 7),
+    # teams: the first size above, last workgroups and waves that own few cells, as many jobs as XCDs and one more
+    (65, False, [8, 8, 5]), (254, True, [6, 9]), (129, False, [5, 7] * 4), (300, True, [6, 4, 6] * 6), (385, True, [5, 5, 2]),
+    # 16 cells per workgroup, two teams per XCD, more jobs than one launch holds
+    (512, True, [12, 9] * 10), (257, False, [4, 6]), (450, False, [3] * 7), (512, False, [6, 5] * 20), (512, True, [4] * 70),
+    # the first size the step-by-step schedule takes
+    (513, False, [3, 2]),
+])
+def test_lstm_recursion_geometries(L, bidir, lengths):
+    """Persistent recursions against the step-by-step schedule at the sizes where their dispatch and their remainders
+    change (cells per direction, number of (direction, four sequences) jobs)."""
+    print("lstm geometry", L, bidir, lengths, flush=True)
+    if bidir and L % 2:
+        L += 1
+    assert PC.run_lstm_two_recursions(19, L, bidir, lengths, seed=L + len(lengths)) < TOL
