@@ -1282,6 +1282,36 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     // what the skip layers' forward passes clear (layers/SkipAddLayer.cu:195-205)
     if (net->skip_error_count) CNT_TRY(fill_zero(stream, net->skip_errors, net->skip_error_count));
+    static const bool fuse_blocks = [] { const char *e = std::getenv("CNT_NET_FUSE_BLOCKS"); return !e || std::atoi(e) != 0; }();
+    // a WaveNet residual block seen from its convolution layer i: [cnn 2R (i)][wavnetc R][dense R, identity]
+    // [skipadd of the block's input and that layer][skipini, shares the sum][dense K, identity]
+    auto block_at = [&](size_t i) {
+        if (!fuse_blocks || i < 1 || i + 5 >= net->layers.size()) return false;
+        const NetLayer &in = net->layers[i - 1], &cnn = net->layers[i], &wav = net->layers[i + 1], &out = net->layers[i + 2];
+        const NetLayer &add = net->layers[i + 3], &ini = net->layers[i + 4], &sk = net->layers[i + 5];
+        const int R = in.size;
+        if (cnn.kind != K_CNN || wav.kind != K_WAVNETC || out.kind != K_DENSE || add.kind != K_SKIPADD || ini.kind != K_SKIPINI ||
+            sk.kind != K_DENSE) return false;
+        if (wav.size != R || out.size != R || add.size != R || out.act != ACT_IDENTITY || sk.act != ACT_IDENTITY) return false;
+        if (add.pre.size() != 2 || ini.out != add.out || add.out == in.out) return false;
+        const float *s0 = net->layers[(size_t)add.pre[0]].out, *s1 = net->layers[(size_t)add.pre[1]].out;
+        if (!((s0 == in.out && s1 == out.out) || (s0 == out.out && s1 == in.out))) return false;
+        for (const NetLayer *l : {&cnn, &wav, &out, &add, &ini, &sk})
+            if (l->N != in.N || l->pat != in.pat) return false;
+        return wavenet_block_forward_supported(cnn.cnn, R, sk.size, wav.ctx_dim);
+    };
+    auto conditioning = [&](size_t i) -> int {
+        const NetLayer &L = net->layers[i];
+        CNT_REQUIRE(L.ctx_dim == 0 || net->ctx, "network_forward: wavnetc layer '%s' has no conditioning features "
+                    "(cnt_network_set_context)", L.name.c_str());
+        if ((int)i != net->first_wavnetc || net->flagged < 0) return CNT_OK;
+        // WavNetCore::__loadContextBuff (layers/wavNetCore.cu:455-492) and the clearing of the gradient
+        // buffer for the conditioning sub-network (:645-647)
+        const NetLayer &f = net->layers[(size_t)net->flagged];
+        CNT_TRY(fill_zero(stream, net->ctx_grad, (size_t)L.ctx_dim * L.N));
+        return cnt_wavnetc_load_context(stream, L.ctx_dim, net->S, L.N, f.T, f.res == 1 ? 1 : 0, f.out,
+                                        net->layers.front().out, net->ctx_mv, L.pat, net->ctx_own);
+    };
     for (size_t i = 1; i < net->layers.size(); ++i) {
         NetLayer &L = net->layers[i];
         const NetLayer &prev = net->layers[i - 1];
@@ -1331,19 +1361,20 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
                 CNT_HIP(hipGetLastError());
                 break;
             case K_CNN:
+                if (block_at(i)) {
+                    const NetLayer &wav = net->layers[i + 1], &out = net->layers[i + 2], &sk = net->layers[i + 5];
+                    CNT_TRY(conditioning(i + 1));
+                    const BlockForward block = {prev.out, net->ctx, W, net->weights + wav.w_off, net->weights + out.w_off,
+                                                net->weights + sk.w_off, out.bias, sk.bias, L.out, wav.core, wav.cth, wav.out,
+                                                out.out, net->layers[i + 3].out, sk.out};
+                    CNT_TRY(wavenet_block_forward(stream, L.cnn, prev.size, sk.size, wav.ctx_dim, N, L.pat, block));
+                    i += 5;
+                    break;
+                }
                 CNT_TRY(cnt_cnn_forward(L.cnn, stream, L.pat, L.T, W, prev.out, L.out));
                 break;
             case K_WAVNETC:
-                CNT_REQUIRE(L.ctx_dim == 0 || net->ctx, "network_forward: wavnetc layer '%s' has no conditioning features "
-                            "(cnt_network_set_context)", L.name.c_str());
-                if ((int)i == net->first_wavnetc && net->flagged >= 0) {
-                    // WavNetCore::__loadContextBuff (layers/wavNetCore.cu:455-492) and the clearing of the gradient
-                    // buffer for the conditioning sub-network (:645-647)
-                    const NetLayer &f = net->layers[(size_t)net->flagged];
-                    CNT_TRY(fill_zero(stream, net->ctx_grad, (size_t)L.ctx_dim * N));
-                    CNT_TRY(cnt_wavnetc_load_context(stream, L.ctx_dim, net->S, N, f.T, f.res == 1 ? 1 : 0, f.out,
-                                                     net->layers.front().out, net->ctx_mv, L.pat, net->ctx_own));
-                }
+                CNT_TRY(conditioning(i));
                 CNT_TRY(cnt_wavnetc_forward(stream, L.size, L.ctx_dim, N, L.pat, W, net->ctx, prev.out, L.core, L.cth,
                                             L.out));
                 break;

@@ -12,6 +12,7 @@
 // buffer.  The dead "future" tap of a causal window is never computed; its gradient columns are the
 // zeros of the weight-update clear.  The elementwise parts are fused streaming kernels.
 #include "common.hpp"
+#include "wavenet_block.hpp"
 
 #include <cstring>
 #include <new>
@@ -909,6 +910,47 @@ int cnt_wavnetc_forward(void *stream_, int D, int C, int N, const char *patTypes
         CNT_TRY(gemm_launch(stream, ga));
     }
     return cnt_gatedact_forward(stream_, D, N, patTypes, core_buf, outputs);
+}
+
+extern "C++" bool cnt::wavenet_block_forward_supported(const cnt_cnn *cnn, int R, int K, int C) {
+    return cnn_foldable(cnn, R) && pick_block_forward_kernel(R, 1) && K > 0 && K % 16 == 0 && (C == 0 || C >= 4) && C <= kBlockMaxContext;
+}
+
+extern "C++" int cnt::wavenet_block_forward(hipStream_t stream, const cnt_cnn *cnn, int R, int K, int C, int N,
+                                            const char *patTypes, const BlockForward &b) {
+    CNT_REQUIRE(wavenet_block_forward_supported(cnn, R, K, C), "wavenet_block_forward: no kernel for this block");
+    CNT_REQUIRE(N > 0 && patTypes && b.x && b.conv_weights && b.out_weights && b.skip_weights && b.conv && b.core && b.gated &&
+                b.out && b.sum && b.skip && (C == 0 || (b.ctx && b.ctx_weights && b.ctx_tanh)),
+                "wavenet_block_forward: null argument");
+    const cnt_cnn_group &g = cnn->groups[0];
+    BlockFwdArgs a = {};
+    a.N = N; a.K = K; a.C = C; a.pat = patTypes; a.x = b.x; a.ctx = b.ctx;
+    a.shift = g.dil * cnn->desc.S;
+    a.conv_ld = (2 * g.hw + 1) * R;
+    for (int tap = 0; tap < 2; ++tap) a.conv_w[tap] = b.conv_weights + (size_t)(g.col0 + g.hw + tap - 1) * R;
+    a.conv_bias = b.conv_weights + (size_t)R * cnn->Lw;
+    a.conv_scale = cnn->desc.bias; a.conv_tanh = cnn->desc.output_tanh;
+    a.ctx_w = b.ctx_weights;
+    a.out_w = b.out_weights; a.out_bias = b.out_weights + (size_t)R * R; a.out_scale = b.out_bias;
+    a.skip_w = b.skip_weights; a.skip_bias = b.skip_weights + (size_t)R * K; a.skip_scale = b.skip_bias;
+    a.conv = b.conv; a.core = b.core; a.ctx_tanh = b.ctx_tanh; a.gated = b.gated; a.out = b.out; a.sum = b.sum; a.skip = b.skip;
+    for (const void *p : {(const void *)a.x, (const void *)a.conv, (const void *)a.core, (const void *)a.ctx_tanh,
+                          (const void *)a.gated, (const void *)a.out, (const void *)a.sum, (const void *)a.skip})
+        CNT_REQUIRE((reinterpret_cast<uintptr_t>(p) & 15) == 0, "wavenet_block_forward: buffers must be 16-byte aligned");
+    // Samples per workgroup (16, 32 or 64): the more, the fewer times a block's weights are read, the fewer, the more
+    // workgroups share the chip.  Measured with 80 conditioning features (us at 16 / 32 / 64 samples): 64 channels, 4 000
+    // samples 10.3 / 13.9 / 21.1, 16 000 samples 27.4 / 21.5 / 22.1, 24 000 samples 38.3 / 32.9 / 34.5, 32 000 samples
+    // 50.8 / 41.0 / 35.4; 32 channels (60 features), 4 000 samples 6.9 / 9.5 / 15.3, 24 000 samples 15.6 / 15.9 / 24.3,
+    // 32 000 samples 23.7 / 17.7 / 24.6.
+    const int st = N <= 4096 || (R < 64 && N <= 24576) ? 1 : R == 32 || N <= 24576 ? 2 : 4;
+    const block_fwd_kernel_t kernel = pick_block_forward_kernel(R, st);
+    const int lds = 16 * block_forward_lds_words(R, st, C);
+    if (lds > 65536)
+        CNT_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    ProfileScope prof(stream, "wavenet_block_forward");
+    hipLaunchKernelGGL(kernel, dim3((N + 16 * st - 1) / (16 * st)), dim3(4 * R), lds, stream, a);
+    CNT_HIP(hipGetLastError());
+    return CNT_OK;
 }
 
 extern "C++" bool cnt::wavenet_block_errors_supported(int R, int K) { return pick_block_errors_kernel(R, K, false) != nullptr; }

@@ -440,6 +440,54 @@ class _CondOracleBackend(OM.OracleBackend):
         O.wavnetc_backward(D, C, N, pat, W, ctx, core, cth, err, prev_err, dW, self.ctx_grad)
 
 
+# one launch per residual block: tiles of 16, 32 and 64 samples with a ragged last one, conditioning rows that end inside
+# a 16-byte piece or start off a 16-byte boundary, fewer skip than residual channels, the widest conditioning
+@pytest.mark.parametrize("cnn_tanh,R,K,C,lengths", [
+    (1, 32, 32, 4, [1]), (1, 64, 32, 7, [40, 33, 1]), (0, 48, 96, 45, [70, 51]), (1, 48, 256, 112, [17]), (1, 64, 80, 81, [2050, 1999]),
+    (1, 32, 64, 20, [12300, 12295]), (1, 64, 128, 100, [8200, 7000, 8199]),
+])
+def test_wavenet_block_forward_edges(cnn_tanh, R, K, C, lengths):
+    import torch
+
+    print("wavenet block forward", cnn_tanh, R, K, C, lengths, flush=True)
+    capi, networks = PC.pkg().capi, PC.networks()
+    O.use_all_cores()
+    nb, Q, S, T = 2, 32, len(lengths), max(lengths)
+    pat, _, ctx, target, N = WD.make(lengths, Q, C, upsample=5, seed=7)
+    onehot = np.zeros((N, Q), np.float32)  # the feedback layer's: also in the first padding slot behind a sequence
+    follows = np.flatnonzero(pat[: N - S] != 0)
+    onehot[follows + S, np.asarray(target).reshape(-1)[follows].astype(int)] = 1
+    ref = networks.WaveNet(OM.OracleBackend(), nb, S, T, Q=Q, R=R, K=K, C=C, cnn_tanh=cnn_tanh, dilation_cycle=10)
+    W = WD.init_weights({k: len(ref.buf[k]["W"]) for k in ref.weight_names()}, seed=3)
+    for k, w in W.items():
+        ref.buf[k]["W"][:] = w
+    ref.set_inputs(pat, onehot.reshape(-1), ctx, target)
+    ref.forward()
+    net = capi.Network(json.dumps(PC.pkg().specs.wavenet_network_doc(nb, Q, R, K, C, cnn_tanh, 10)), S, T, mdn_config=[1, 0, Q, 0, 1, -1])
+    for L in net.layers:
+        if L["weight_count"]:
+            L["weights"].copy_(torch.from_numpy(W[L["name"]]))
+    ctx_d = PC.dev(ctx)
+    net.set_context(ctx_d)
+    net.load_sequences(PC.dev(pat), T, min(lengths), torch.zeros(N, dtype=torch.float32, device="cuda"), PC.dev(target))
+    for layer in net.layers:
+        if layer["type"] == "cnn":
+            layer["outputs"].fill_(3.0)  # padding slots of a convolution layer keep what they hold
+    net.forward()
+    torch.cuda.synchronize()
+    valid = (pat != 0).repeat(2 * R)
+    for layer in net.layers:
+        name = layer["name"]
+        if name not in ref.buf or name == "postoutput":
+            continue
+        got, want = layer["outputs"].cpu().numpy()[: ref.buf[name]["out"].size], ref.buf[name]["out"]
+        if layer["type"] == "cnn":
+            assert np.all(got[~valid] == 3.0)
+            got, want = got[valid], want[valid]
+        assert np.abs(got - want).max() <= 2e-5 * max(1.0, np.abs(want).max()), name
+    net.close()
+
+
 @pytest.mark.parametrize("context_mv", [False, True])
 def test_wavenet_with_frame_rate_conditioning_network(context_mv, tmp_path):
     """The reference example's layout in full: externalloader -> skipini -> blstm -> cnn -> skipcat at one slot per
