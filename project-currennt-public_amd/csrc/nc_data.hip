@@ -13,22 +13,30 @@
 // libnetcdf is not used: the classic format (CDF-1) and its 64-bit-offset variant (CDF-2) are a flat
 // big-endian header followed by the variables' row-major data, parsed here.  Record (unlimited-dimension)
 // variables are refused with a clear message.  The reference copies every sequence into a cache file under
-// /tmp first and builds fractions from there; here a fraction is built straight from the .nc file with one
-// positioned read per sequence and variable.
+// /tmp first and builds fractions from there; here a fraction is built straight from the .nc file, in blocks of rows
+// that go from a positioned read through a cache-sized buffer into their places, by several threads for a large one.
 // Not covered (refused or absent): several .nc files in one set, input context windows and output time lag,
 // noise injection, external / auxiliary data, sequence and fraction shuffling, ordered file lists.
 #include "common.hpp"
 
 #include <random>
 #include <algorithm>
+#include <atomic>
 #include <cerrno>
+#include <condition_variable>
 #include <cstring>
+#include <functional>
 #include <limits>
+#include <memory>
+#include <mutex>
 #include <new>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include <fcntl.h>
+#include <sched.h>
 #include <sys/stat.h>
 #include <unistd.h>
 
@@ -55,16 +63,17 @@ struct NcFile {
 
     bool fail(const std::string &m) { error = m; return false; }
 
-    bool read_at(long long off, void *dst, size_t n) {
+    bool pread_all(long long off, void *dst, size_t n) const {
         char *p = static_cast<char *>(dst);
         while (n > 0) {
             const ssize_t r = ::pread(fd, p, n, off);
             if (r < 0 && errno == EINTR) continue;
-            if (r <= 0) return fail("unexpected end of file");
+            if (r <= 0) return false;
             p += r; off += r; n -= (size_t)r;
         }
         return true;
     }
+    bool read_at(long long off, void *dst, size_t n) { return pread_all(off, dst, n) || fail("unexpected end of file"); }
 
     // --- header -------------------------------------------------------------------------------------
     std::vector<unsigned char> hdr;
@@ -196,24 +205,116 @@ struct NcFile {
         return e;
     }
 
-    // rows [row0, row0 + nrows) of a variable whose first dimension is the row index, as T (float or int)
+    // where rows [row0, row0 + nrows) of a variable whose first dimension is the row index stand, or -1
+    long long rows_at(const char *nm, int want_type, long long row0, long long nrows, long long row_len) {
+        const NcVar *v = variable(nm);
+        const char *wrong = !v ? "variable not found" : v->dimids.empty() || elements(*v) < (row0 + nrows) * row_len
+            ? "index exceeds dimension bound" : nullptr;
+        if (v && v->record) fail(std::string("variable '") + nm + "' uses the unlimited dimension, which is not supported");
+        else if (v && v->type != want_type) fail(std::string("variable '") + nm + "' has an unexpected type");
+        else if (wrong) fail(std::string("Cannot read array '") + nm + "': " + wrong);
+        else return v->begin + row0 * row_len * (long long)type_size(want_type);
+        return -1;
+    }
+
+    // those rows as T (float, int or char)
     template <typename T>
     bool read_rows(const char *nm, int want_type, long long row0, long long nrows, long long row_len, T *dst) {
-        const NcVar *v = variable(nm);
-        if (!v) return fail(std::string("Cannot read array '") + nm + "': variable not found");
-        if (v->record) return fail(std::string("variable '") + nm + "' uses the unlimited dimension, which is not supported");
-        if (v->type != want_type) return fail(std::string("variable '") + nm + "' has an unexpected type");
-        if (v->dimids.empty() || elements(*v) < (row0 + nrows) * row_len)
-            return fail(std::string("Cannot read array '") + nm + "': index exceeds dimension bound");
-        const size_t count = (size_t)(nrows * row_len);
+        const long long at = rows_at(nm, want_type, row0, nrows, row_len);
+        if (at < 0) return false;
+        const size_t count = (size_t)(nrows * row_len), es = type_size(want_type);
         if (count == 0) return true;
-        const size_t es = type_size(want_type);
-        if (!read_at(v->begin + row0 * row_len * (long long)es, dst, count * es)) return false;
+        if (!read_at(at, dst, count * es)) return false;
         if (es == 4) {
             unsigned *w = reinterpret_cast<unsigned *>(dst);
             for (size_t i = 0; i < count; ++i) w[i] = __builtin_bswap32(w[i]);
         }
         return true;
+    }
+};
+
+// big-endian words to host order; sixteen or thirty-two bytes per instruction where the processor has a byte shuffle
+#if !defined(__HIP_DEVICE_COMPILE__)
+__attribute__((target_clones("avx2", "default")))
+#endif
+void swapped_copy(unsigned *dst, const unsigned *src, size_t n) {
+    for (size_t i = 0; i < n; ++i) dst[i] = __builtin_bswap32(src[i]);
+}
+
+// Threads that help the caller through a list of independent pieces of work; they are started by the first list and joined
+// with the pool.  The caller works through the list itself and waits only for helpers that have taken a piece, so a list
+// also ends where no helper is left (a forked child) or none could be started.
+class Helpers {
+    std::mutex m, busy;
+    std::condition_variable wake, idle;
+    std::vector<std::thread> threads;
+    const std::function<void(size_t)> *job = nullptr;
+    std::atomic<size_t> next{0};
+    size_t count = 0;
+    unsigned generation = 0;
+    int active = 0;
+    bool stop = false;
+    pid_t owner = 0;
+
+    static void work(const std::function<void(size_t)> &f, std::atomic<size_t> &next, size_t count) {
+        for (size_t i; (i = next.fetch_add(1, std::memory_order_relaxed)) < count;) f(i);
+    }
+    void help() {
+        unsigned seen = 0;
+        std::unique_lock<std::mutex> lock(m);
+        for (;;) {
+            wake.wait(lock, [&] { return stop || (job && generation != seen); });
+            if (stop) return;
+            seen = generation;
+            const std::function<void(size_t)> &f = *job;
+            const size_t n = count;
+            ++active;
+            lock.unlock();
+            work(f, next, n);
+            lock.lock();
+            if (--active == 0) idle.notify_one();
+        }
+    }
+    static int helpers_wanted() {
+        // memory bandwidth is used up by about eight threads, and a process may be one of several on its machine
+        cpu_set_t set;
+        const int cpus = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : 1;
+        return std::min(7, cpus - 1);
+    }
+
+public:
+    void run(size_t n, const std::function<void(size_t)> &f) {
+        std::unique_lock<std::mutex> mine(busy, std::try_to_lock);
+        if (!mine.owns_lock() || !owned()) {  // another thread's list is in work, or a forked child
+            for (size_t i = 0; i < n; ++i) f(i);
+            return;
+        }
+        if (owner == 0) {
+            owner = getpid();
+            try {
+                for (int k = helpers_wanted(); k > 0; --k) threads.emplace_back([this] { help(); });
+            } catch (const std::system_error &) {
+            }  // fewer helpers then
+        }
+        {
+            std::lock_guard<std::mutex> lock(m);
+            next = 0; count = n; job = &f; ++generation;
+        }
+        wake.notify_all();
+        work(f, next, n);
+        std::unique_lock<std::mutex> lock(m);
+        job = nullptr;
+        idle.wait(lock, [&] { return active == 0; });
+    }
+    // false in a forked child, which has the objects but not the threads: nothing there may be waited for or destroyed
+    bool owned() const { return owner == 0 || owner == getpid(); }
+    ~Helpers() {
+        {
+            std::lock_guard<std::mutex> lock(m);
+            stop = true;
+        }
+        wake.notify_all();
+        for (std::thread &t : threads) t.join();
     }
 };
 
@@ -236,6 +337,10 @@ struct cnt_dataset {
     std::vector<cnt::Sequence> sequences;
     std::mt19937 shuffle_gen;  // one generator for every shuffle of this data set, seeded by the first one
     bool shuffle_seeded = false;
+    cnt::Helpers *helpers = new cnt::Helpers();
+    ~cnt_dataset() {
+        if (helpers->owned()) delete helpers;
+    }
 };
 
 namespace {
@@ -423,29 +528,65 @@ int cnt_dataset_fraction_fill(cnt_dataset *d, int first_seq, char *patTypes, flo
                 "dataset_fraction: the target buffer of this data set's kind is missing");
     const int S = d->desc.parallel_sequences, P = d->input_size, Q = d->output_size;
     const size_t slots = (size_t)T * S;
+    // A fraction is written once, row by row: the rows of a sequence in blocks of up to 128 KB that go from the file
+    // through a buffer which stays in cache, byte order and place changed on the way out of it; zeros only where there is
+    // no row.  (Reading a sequence whole, swapping it in place and copying its rows over a cleared fraction moves every
+    // byte five times.)  From two megabytes on several threads share the blocks; below, waking them takes what they save.
+    // 10 sequences of 300 to 600 rows of 382 inputs and 187 targets, 13.7 MB, into fresh pages: 907 -> 491 us with eight
+    // threads, what is left is mostly the kernel's zeroing of the pages; 8 x 48 rows of 432 + 4 values, 0.7 MB, by the
+    // caller alone: 54 -> 32 us.
+    struct Block { long long at; float *out; int col, t0, t1, rows, width; };  // rows of t0 .. t1 from the file, the rest zeros
+    std::vector<Block> blocks;
+    auto add = [&](const char *name, int width, float *out) {
+        const int step = std::max(1, 32768 / std::max(1, width));
+        for (int i = 0; i < S; ++i) {
+            const Sequence *s = i < n ? &d->sequences[(size_t)(first_seq + i)] : nullptr;
+            const int length = s ? s->length : 0;
+            const long long at = s ? d->file.rows_at(name, 5, s->begin, length, width) : 0;
+            if (at < 0) return false;
+            for (int t = 0; t < T; t += step) {
+                const int end = std::min(T, t + step), rows = std::max(0, std::min(end, length) - t);
+                blocks.push_back({at + (long long)t * width * 4, out, i, t, end, rows, width});
+            }
+        }
+        return true;
+    };
+    if (!add("inputs", P, inputs) || (!d->is_classification && !add("targetPatterns", Q, targets)))
+        return dataset_error(d, "dataset_fraction");
+    std::atomic<bool> short_file{false};
+    const std::function<void(size_t)> fill = [&](size_t k) {
+        const Block &b = blocks[k];
+        const size_t width = (size_t)b.width;
+        static thread_local std::vector<unsigned> buffer;
+        buffer.resize((size_t)b.rows * width);
+        if (b.rows > 0 && !d->file.pread_all(b.at, buffer.data(), buffer.size() * 4)) {
+            short_file = true;
+            return;
+        }
+        for (int t = b.t0; t < b.t1; ++t) {
+            unsigned *dst = reinterpret_cast<unsigned *>(b.out + ((size_t)t * S + b.col) * width);
+            if (t < b.t0 + b.rows) swapped_copy(dst, buffer.data() + (size_t)(t - b.t0) * width, width);
+            else std::memset(dst, 0, width * 4);
+        }
+    };
+    const size_t values = slots * (size_t)(P + (d->is_classification ? 0 : Q));
+    if (values >= (1u << 19)) d->helpers->run(blocks.size(), fill);
+    else
+        for (size_t k = 0; k < blocks.size(); ++k) fill(k);
+    if (short_file) {
+        d->file.fail("unexpected end of file");
+        return dataset_error(d, "dataset_fraction");
+    }
     std::memset(patTypes, 0, slots);
-    std::fill(inputs, inputs + slots * P, 0.0f);
     if (d->is_classification) std::fill(target_classes, target_classes + slots, -1);
-    else std::fill(targets, targets + slots * Q, 0.0f);
-    std::vector<float> rows;
     std::vector<int> classes;
     for (int i = 0; i < n; ++i) {
         const Sequence &s = d->sequences[(size_t)(first_seq + i)];
-        rows.resize((size_t)s.length * P);
-        if (!d->file.read_rows<float>("inputs", 5, s.begin, s.length, P, rows.data())) return dataset_error(d, "dataset_fraction");
-        for (int t = 0; t < s.length; ++t)
-            std::memcpy(inputs + ((size_t)t * S + i) * P, rows.data() + (size_t)t * P, sizeof(float) * P);
         if (d->is_classification) {
             classes.resize((size_t)s.length);
             if (!d->file.read_rows<int>("targetClasses", 4, s.begin, s.length, 1, classes.data()))
                 return dataset_error(d, "dataset_fraction");
             for (int t = 0; t < s.length; ++t) target_classes[(size_t)t * S + i] = classes[(size_t)t];
-        } else {
-            rows.resize((size_t)s.length * Q);
-            if (!d->file.read_rows<float>("targetPatterns", 5, s.begin, s.length, Q, rows.data()))
-                return dataset_error(d, "dataset_fraction");
-            for (int t = 0; t < s.length; ++t)
-                std::memcpy(targets + ((size_t)t * S + i) * Q, rows.data() + (size_t)t * Q, sizeof(float) * Q);
         }
         for (int t = 0; t < s.length; ++t)
             patTypes[(size_t)t * S + i] = t == 0 ? 1 : (t == s.length - 1 ? 3 : 2);  // FIRST, LAST, NORMAL

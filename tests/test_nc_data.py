@@ -223,3 +223,42 @@ def test_damaged_header_is_rejected(tmp_path):
         except RuntimeError:
             pass
         ds.close()
+
+
+# blocks of rows that end with a sequence, inside it and behind it, rows wider than a block, fewer sequences than
+# parallel slots; small fractions (filled by the caller) and large ones (shared with helper threads), the latter also by
+# two threads at once and in a forked child, which has the data set but not its threads
+@pytest.mark.parametrize("lengths,P,Q,classes,S", [
+    ([256, 255, 257, 1], 128, 3, 0, 4), ([900, 512, 300, 130], 128, 37, 0, 5), ([2, 3], 40000, 1, 0, 2), ([900, 40], 320, 0, 7, 2),
+])
+def test_fractions_in_blocks(tmp_path, lengths, P, Q, classes, S):
+    import threading
+
+    capi = load_package().capi
+    p = str(tmp_path / "blocks.nc")
+    write_nc(p, lengths, P, Q, 2, classes=classes, seed=3)
+    want = NF.make_fraction(p, NF.segments(p, training_mode=True), 0, S)
+    ds = capi.Dataset(p, S, True, 0, 1.0)
+
+    def same():
+        got = ds.fraction(0)
+        return all(np.array_equal(got[k], want[k]) for k in ("patTypes", "inputs", "target_classes" if classes else "targets"))
+
+    results = []
+    threads = [threading.Thread(target=lambda: results.extend(same() for _ in range(5))) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert results == [True] * 10
+    pid = os.fork()
+    if pid == 0:
+        ok = False
+        try:
+            ok = same()
+            ds.close()
+        finally:
+            os._exit(0 if ok else 1)
+    assert os.waitpid(pid, 0)[1] == 0
+    assert same()
+    ds.close()
