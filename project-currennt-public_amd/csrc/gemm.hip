@@ -1,4 +1,4 @@
-// fp32 MFMA matrix product for gfx950.
+// fp32 matrix product for gfx950 on the bf16 matrix instructions.
 //
 // This is the seam that the reference reaches through helpers::Matrix::assignProduct/addProduct
 // (helpers/Matrix.cu:353-377 -> helpers/cublas.cu:52-84).  One kernel covers every operand
@@ -6,12 +6,25 @@
 // products of a BLSTM become one pass), several independent problems per launch, split-K for the
 // long-K weight-gradient shapes, and a fused bias + activation epilogue for the dense forward.
 //
+// Arithmetic: the fp32 matrix instructions end at 157 TFLOP/s and reached 88 here, with the matrix units 56% busy.  Every
+// operand value is therefore split into three bf16 parts, x = h + m + l exactly (round to nearest, so m <= 2^-9 |x| and
+// l <= 2^-18 |x|), and a product is the sum of the six part products h*h, h*m, m*h, m*m, h*l, l*h, which the bf16
+// instructions form exactly and add in fp32, the small ones first.  What is left out (m*l, l*m, l*l) is below 2^-25 of
+// |a||b|, less than the rounding of one fp32 product.  An instruction adds sixteen products before it rounds, where the fp32 one
+// adds two, so the result is closer to a 64-bit product than before: 2-norm error 4.9e-7 against 5.7e-7 at k = 1024, 1.2e-6
+// against 1.4e-6 at k = 6000, 1.6e-7 against 2.0e-7 at k = 128.  Values that are infinite, or round to an infinite bf16
+// value, leave infinity minus infinity in their parts; a sum that is not finite is formed again in plain fp32.
+//   1024 x 12000 x 1024: 283 -> 167 us (150 TFLOP/s), 512 x 6000 x 512: 40 -> 30 us, 1024 x 6000 x 512: 74 -> 55 us,
+//   1024 x 32000 x 128: 108 -> 72 us, 425 x 12000 x 1024: 141 -> 100 us.
+// What bounds it now, at the first size per SIMD: 69 us of matrix instructions, 38 us of conversions, 51 us of LDS traffic,
+// which overlap only in part.  Measured and not taken: the conversion of the next tile between the matrix instructions of
+// this one, with two LDS buffers and one or two tiles of loads in flight (245 us: one wave per SIMD issues a vector
+// instruction every eight clocks, not four); 128 x 64 tiles (182 us).
+//
 // Tiling: T x T x 32 per workgroup with T = 128 or 64, four 64-lane waves in a 2 x 2 arrangement, each wave
-// owning a T/2 x T/2 block as tiles of v_mfma_f32_32x32x2_f32.  An operand tile sits in LDS in the
-// orientation it has in memory, so that staging never transposes: k-contiguous operands as [row][k] with
-// a (BK+4)-float pitch (16-byte fragment reads, conflict free), row-contiguous operands as [k][row]
-// (4-byte fragment reads along consecutive rows).  A transposing store of the latter into [row][k]
-// costs a 16-way LDS bank conflict.
+// owning a T/2 x T/2 block as tiles of v_mfma_f32_32x32x16_bf16.  The parts lie in LDS in the order the instruction takes
+// them (TileLayout); 50 KB (T = 128) and 26 KB (T = 64) per workgroup leave room for three and five of them per compute unit, whose
+// phases overlap.  Two workgroups of T = 128 instead of three: 197 us at the first size above.
 // The MFMA operands are swapped (the B tile feeds the instruction's A port) so that lane%32 walks
 // along the column-major output's contiguous dimension and every store is a 128-byte segment.
 #include "gemm_kernel.hpp"
@@ -42,17 +55,17 @@ inline int pick_vec(const GemmArgs &a, bool for_a) {
     return v;
 }
 
-// Tile edge.  128 x 128 tiles give the most MFMA work per byte staged, but a launch that yields only a few of
-// them per compute unit leaves the machine waiting on memory latency (one or two workgroups of four waves per
-// CU) and on the last, partly filled round of workgroups.  Measured on MI355X, 64 x 64 tiles -- four times as
-// many workgroups -- are faster for every product of the benchmark networks (the acoustic model's 512 x 5880
-// error products by 1.4x, the WaveNet layers' K = 64..384 products over 32 000 slots by 2x); the large tile is
-// kept for launches that fill the machine many times over anyway.
-int pick_tile(const GemmArgs &a) {
+// Tile edge.  128 x 128 tiles convert and read half as much per matrix instruction, but three of them fill a compute unit, so a
+// launch needs some 600 of them, and a run over k long enough that filling and draining the pipeline does not show
+// (64 / 128, us: 1024 x 12000 x 1024 with 752 large tiles 200 / 165; 1024 x 6000 x 512 with 376 of them 54 / 56; 512 x
+// 6000 x 512 with 188 30 / 51; 1024 x 32000 x 128 with 2000 71 / 103).  They exist for operands with 16-byte vectors only: with narrower
+// ones the loader's registers spill (425 x 12000 x 1024: 100 / 396).
+int pick_tile(const GemmArgs &a, int va, int vb) {
     static const int forced = [] { const char *e = std::getenv("CNT_GEMM_TILE"); return e ? std::atoi(e) : 0; }();
+    if (va != 4 || vb != 4 || a.masked || a.epilogue == EPI_FAN) return 64;
     if (forced == 64 || forced == 128) return forced;
     const long t128 = (long)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.splitk * a.nprob;
-    return t128 < 2048 ? 64 : 128;
+    return t128 >= 600 && (long)a.k * a.nseg / a.splitk >= 512 ? 128 : 64;
 }
 
 // ----- split-K through partial products ---------------------------------------------------------------------
@@ -270,7 +283,7 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
     const int va = pick_vec(args, true), vb = pick_vec(args, false);
     gemm_plan(args, stream);
     if (args.epilogue != EPI_PARTIAL) args.rowsum = 0;
-    const int tile = pick_tile(args);
+    const int tile = pick_tile(args, va, vb);
     static const bool use_lines = [] { const char *e = std::getenv("CNT_GEMM_K_ORDER"); return !e || std::atoi(e) != 0; }();
     if (!use_lines) args.k_order = nullptr;
     // a list of k lines is used where the kernel that reads through it exists, and ignored otherwise (the lines it leaves

@@ -1,18 +1,21 @@
-// Kernel template and launch ladder of the fp32 MFMA matrix product (design notes: gemm.hip).
+// Kernel template and launch ladder of the fp32 matrix product (design notes: gemm.hip).
 #pragma once
 
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace cnt {
+
 namespace {
 
-constexpr int BK = 32;  // k depth of a staged tile (16 measured 5-8% slower on the acoustic model's products: twice the
-                        // barriers per flop); the tile edge (rows of A = columns of B per workgroup) is a template
-                        // parameter: 128 or 64
-constexpr int PITCH = BK + 4;
+constexpr int BK = 32;  // k depth of a staged tile: two matrix instructions deep
 constexpr int NTHREADS = 256;
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // workgroup barrier that orders LDS traffic only; global loads issued before it stay in flight
 __device__ __forceinline__ void lds_only_barrier() {
@@ -30,6 +33,113 @@ struct VecT<2> { typedef float2 type; };
 template <>
 struct VecT<4> { typedef float4 type; };
 
+// Two fp32 values as three bf16 pairs (the lower half of a word belongs to x0): x = h + m + l exactly, each part the
+// nearest bf16 value to what the parts before it leave (8 + 8 + 8 bits of significand hold the 24 of x).
+__device__ __forceinline__ unsigned nearest_bf16(float x0, float x1) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x0, x1}), bf16x2));
+}
+__device__ __forceinline__ void split_pair(float x0, float x1, unsigned (&part)[3]) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        part[q] = nearest_bf16(x0, x1);
+        if (q == 2) break;
+        x0 -= __uint_as_float(part[q] << 16);
+        x1 -= __uint_as_float(part[q] & 0xffff0000u);
+    }
+}
+
+// Where the parts of a ROWS-row x BK-k operand tile lie in LDS.  The 16-byte unit is what one lane of a matrix instruction
+// takes: eight consecutive k of one row.  Units are ordered [part][k / 8][position of the row]; the position of a row is the
+// row itself where a thread loads along k, and r * GROUP + t for row VEC * t + r where it loads VEC rows at once, so that in
+// both cases the lanes of one store, and those of one read, fall on distinct banks (the pads of GROUP and LINE see to it).
+template <int VEC, bool KCONTIG, int ROWS>
+struct TileLayout {
+    static constexpr int NLOAD = (ROWS * BK) / (NTHREADS * VEC);  // vectors per thread
+    static_assert(NLOAD >= 1, "tile too small for this vector width");
+    static constexpr int GROUP = ROWS / VEC + (VEC == 4 ? 4 : VEC == 2 ? 8 : 0);
+    static constexpr int LINE = KCONTIG ? ROWS + 4 : VEC * GROUP;  // units per k / 8
+    static constexpr int PART = (BK / 8) * LINE;                   // units per part
+    static constexpr int UNITS = 3 * PART;
+    typedef typename VecT<VEC>::type vec_t;
+
+    // k-contiguous: the thread's vectors start at k position first_k of the rows row(p); row-contiguous: they hold the VEC
+    // rows from first_row on, of the NLOAD consecutive k positions from first_k on
+    static constexpr int TPR = BK / VEC, RPP = NTHREADS / TPR;
+    static constexpr int TPK = ROWS / VEC;
+    static __device__ __forceinline__ int column(int tid) {  // t above
+        if (TPK == 32) return (tid & 15) | ((tid & 32) >> 1);  // sixteen lanes along the rows, two halves of a unit
+        return tid % TPK;
+    }
+    static __device__ __forceinline__ int first_k(int tid) {
+        if (KCONTIG) return (tid % TPR) * VEC;
+        if (TPK == 32) return (2 * (tid >> 6) + ((tid >> 4) & 1)) * NLOAD;
+        return (tid / TPK) * NLOAD;
+    }
+    static __device__ __forceinline__ int first_row(int tid) { return KCONTIG ? tid / TPR : column(tid) * VEC; }
+    static __device__ __forceinline__ int row(int tid, int p) { return KCONTIG ? tid / TPR + p * RPP : column(tid) * VEC; }
+
+    static __device__ __forceinline__ void put(uint4 *__restrict__ lds, int tid, const vec_t (&v)[NLOAD]) {
+        const int k = first_k(tid);
+        if (KCONTIG) {
+            char *at = reinterpret_cast<char *>(lds + (k / 8) * LINE + tid / TPR) + 2 * (k % 8);
+            if constexpr (VEC == 1) {
+#pragma unroll
+                for (int p = 0; p < NLOAD; p += 2) {
+                    unsigned x[3];
+                    split_pair(v[p], v[p + 1], x);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) {
+                        *reinterpret_cast<unsigned short *>(at + 16 * (q * PART + p * RPP)) = (unsigned short)x[q];
+                        *reinterpret_cast<unsigned short *>(at + 16 * (q * PART + (p + 1) * RPP)) = (unsigned short)(x[q] >> 16);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int p = 0; p < NLOAD; ++p) {
+                    const float *e = reinterpret_cast<const float *>(&v[p]);
+                    unsigned x[VEC / 2][3];
+#pragma unroll
+                    for (int j = 0; j < VEC / 2; ++j) split_pair(e[2 * j], e[2 * j + 1], x[j]);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) {
+                        char *to = at + 16 * (q * PART + p * RPP);
+                        if constexpr (VEC == 4) *reinterpret_cast<uint2 *>(to) = uint2{x[0][q], x[1][q]};
+                        else *reinterpret_cast<unsigned *>(to) = x[0][q];
+                    }
+                }
+            }
+        } else {
+            char *at = reinterpret_cast<char *>(lds + (k / 8) * LINE + column(tid)) + 2 * (k % 8);
+#pragma unroll
+            for (int r = 0; r < VEC; ++r) {
+                unsigned x[NLOAD / 2][3];
+#pragma unroll
+                for (int p = 0; p < NLOAD; p += 2)
+                    split_pair(reinterpret_cast<const float *>(&v[p])[r], reinterpret_cast<const float *>(&v[p + 1])[r], x[p / 2]);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    char *to = at + 16 * (q * PART + r * GROUP);
+                    if constexpr (NLOAD == 2) *reinterpret_cast<unsigned *>(to) = x[0][q];
+                    else if constexpr (NLOAD == 4) *reinterpret_cast<uint2 *>(to) = uint2{x[0][q], x[1][q]};
+                    else {
+#pragma unroll
+                        for (int u = 0; u < NLOAD / 8; ++u)
+                            *reinterpret_cast<uint4 *>(to + 16 * u * LINE) =
+                                uint4{x[4 * u][q], x[4 * u + 1][q], x[4 * u + 2][q], x[4 * u + 3][q]};
+                    }
+                }
+            }
+        }
+    }
+
+    // the three parts of k positions [8 * k8, 8 * k8 + 8) of tile row `row`
+    static __device__ __forceinline__ void fragment(const uint4 *__restrict__ lds, int row, int k8, bf16x8 (&f)[3]) {
+        const uint4 *at = lds + k8 * LINE + (KCONTIG ? row : (row % VEC) * GROUP + row / VEC);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) f[q] = __builtin_bit_cast(bf16x8, at[q * PART]);
+    }
+};
+
 // Stages one ROWS-row x BK-k operand tile: global -> registers -> LDS.
 //
 // A load always executes, on a clamped address, and what decides whether its vector counts (inside the matrix; in
@@ -39,8 +149,8 @@ struct VecT<4> { typedef float4 type; };
 // tile have arrived"; zeroing the vector right after the load would make every iteration wait for its own loads.
 template <int VEC, bool KCONTIG, int ROWS>
 struct TileStage {
-    static constexpr int NLOAD = (ROWS * BK) / (NTHREADS * VEC);
-    static_assert(NLOAD >= 1, "tile too small for this vector width");
+    typedef TileLayout<VEC, KCONTIG, ROWS> L;
+    static constexpr int NLOAD = L::NLOAD;
     typename VecT<VEC>::type r[NLOAD];
     bool inside_[NLOAD];      // known at load time (indices only)
     char pat_own_[NLOAD], pat_src_[NLOAD];  // masked mode: loaded next to the data, looked at in store()
@@ -51,13 +161,10 @@ struct TileStage {
                                          int rows_total, int k_total, int tid, const char *__restrict__ pat = nullptr,
                                          int shift = 0, int n_slots = 0, bool time_on_k = false) {
         if (KCONTIG) {
-            constexpr int TPR = BK / VEC;        // threads per row
-            constexpr int RPP = NTHREADS / TPR;  // rows per pass
-            const int kq = (tid % TPR) * VEC;
-            const int rr = tid / TPR;
+            const int kq = L::first_k(tid);
 #pragma unroll
             for (int p = 0; p < NLOAD; ++p) {
-                const int row = row0 + rr + p * RPP;
+                const int row = row0 + L::row(tid, p);
                 typename VecT<VEC>::type v = {};
                 pat_own_[p] = 1; pat_src_[p] = 1;
                 if (!pat) {
@@ -88,13 +195,11 @@ struct TileStage {
                 r[p] = v;
             }
         } else {
-            constexpr int TPK = ROWS / VEC;      // threads per k line
-            constexpr int KPP = NTHREADS / TPK;  // k lines per pass
-            const int rq = (tid % TPK) * VEC;
-            const int kk = tid / TPK;
+            const int rq = L::first_row(tid);
+            const int kk = L::first_k(tid);
 #pragma unroll
             for (int p = 0; p < NLOAD; ++p) {
-                const int k = k0 + kk + p * KPP;
+                const int k = k0 + kk + p;
                 typename VecT<VEC>::type v = {};
                 pat_own_[p] = 1; pat_src_[p] = 1;
                 if (!pat) {
@@ -131,40 +236,11 @@ struct TileStage {
         return keep ? r[p] : typename VecT<VEC>::type{};
     }
 
-    // k values [k_first, k_first + BK/2) of tile row `row`, in MFMA issue order
-    static __device__ __forceinline__ void fragment(const float *__restrict__ lds, int row, int k_first,
-                                                    float (&f)[BK / 2]) {
-        if (KCONTIG) {
-            const float *p = lds + row * PITCH + k_first;
+    __device__ __forceinline__ void store(uint4 *__restrict__ lds, int tid) const {
+        typename VecT<VEC>::type v[NLOAD];
 #pragma unroll
-            for (int q = 0; q < BK / 8; ++q) {
-                const float4 v = *reinterpret_cast<const float4 *>(p + 4 * q);
-                f[4 * q] = v.x; f[4 * q + 1] = v.y; f[4 * q + 2] = v.z; f[4 * q + 3] = v.w;
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < BK / 2; ++q) f[q] = lds[(k_first + q) * ROWS + row];
-        }
-    }
-
-    __device__ __forceinline__ void store(float *__restrict__ lds, int tid) const {
-        if (KCONTIG) {
-            constexpr int TPR = BK / VEC;
-            constexpr int RPP = NTHREADS / TPR;
-            const int kq = (tid % TPR) * VEC;
-            const int rr = tid / TPR;
-#pragma unroll
-            for (int p = 0; p < NLOAD; ++p)
-                *reinterpret_cast<typename VecT<VEC>::type *>(lds + (rr + p * RPP) * PITCH + kq) = kept(p);
-        } else {
-            constexpr int TPK = ROWS / VEC;
-            constexpr int KPP = NTHREADS / TPK;
-            const int rq = (tid % TPK) * VEC;
-            const int kk = tid / TPK;
-#pragma unroll
-            for (int p = 0; p < NLOAD; ++p)
-                *reinterpret_cast<typename VecT<VEC>::type *>(lds + (kk + p * KPP) * ROWS + rq) = kept(p);
-        }
+        for (int p = 0; p < NLOAD; ++p) v[p] = kept(p);
+        L::put(lds, tid, v);
     }
 };
 
@@ -176,37 +252,31 @@ struct TileStage {
 // the workgroup (`special`), every other tile is stored as it arrived.
 template <int VEC, bool KCONTIG, int ROWS>
 struct FastStage {
-    static constexpr int NLOAD = (ROWS * BK) / (NTHREADS * VEC);
+    typedef TileLayout<VEC, KCONTIG, ROWS> L;
+    static constexpr int NLOAD = L::NLOAD;
     typedef typename VecT<VEC>::type vec_t;
     vec_t r[NLOAD];
     unsigned voff[NLOAD];    // byte offsets at k = 0
     unsigned koff[NLOAD];    // what has to be taken off voff to reach k position 0 of the tile (used in a k tail only)
     int kpos[NLOAD];         // first k of the vector inside the tile
-    bool row_ok[NLOAD];
-    bool edge;               // uniform: some row of this tile lies outside the matrix
     int k_valid;             // uniform: k values of the tile in registers that lie inside the operand pair
 
     __device__ __forceinline__ void init(int ld, int row0, int rows_total, int tid) {
-        edge = row0 + ROWS > rows_total;
         if (KCONTIG) {
-            constexpr int TPR = BK / VEC, RPP = NTHREADS / TPR;
-            const int kq = (tid % TPR) * VEC, rr = tid / TPR;
+            const int kq = L::first_k(tid);
 #pragma unroll
             for (int p = 0; p < NLOAD; ++p) {
-                const int row = row0 + rr + p * RPP;
-                row_ok[p] = row < rows_total;
+                const int row = row0 + L::row(tid, p);
                 voff[p] = (unsigned)(((size_t)min(row, rows_total - 1) * ld + kq) * sizeof(float));
                 koff[p] = (unsigned)(kq * sizeof(float));
                 kpos[p] = kq;
             }
         } else {
-            constexpr int TPK = ROWS / VEC, KPP = NTHREADS / TPK;
-            const int rq = (tid % TPK) * VEC, kk = tid / TPK;
+            const int rq = L::first_row(tid), kk = L::first_k(tid);
 #pragma unroll
             for (int p = 0; p < NLOAD; ++p) {
-                const int k = kk + p * KPP;
-                row_ok[p] = (row0 + rq) < rows_total;
-                const int rc = row_ok[p] ? row0 + rq : 0;
+                const int k = kk + p;
+                const int rc = (row0 + rq) < rows_total ? row0 + rq : 0;
                 voff[p] = (unsigned)(((size_t)k * ld + rc) * sizeof(float));
                 koff[p] = (unsigned)((size_t)k * ld * sizeof(float));
                 kpos[p] = k;
@@ -228,26 +298,14 @@ struct FastStage {
                 r[p] = *reinterpret_cast<const vec_t *>(b + (kpos[p] < kv ? voff[p] : voff[p] - koff[p]));
         }
     }
-    __device__ __forceinline__ void store(float *__restrict__ lds, int tid) const {
-        const bool special = edge || k_valid < BK;
-        if (KCONTIG) {
-            constexpr int TPR = BK / VEC, RPP = NTHREADS / TPR;
-            const int kq = (tid % TPR) * VEC, rr = tid / TPR;
+    __device__ __forceinline__ void store(uint4 *__restrict__ lds, int tid) const {
+        if (k_valid < BK) {
+            vec_t v[NLOAD];
 #pragma unroll
-            for (int p = 0; p < NLOAD; ++p) {
-                vec_t v = r[p];
-                if (special && !(row_ok[p] && kpos[p] < k_valid)) v = vec_t{};
-                *reinterpret_cast<vec_t *>(lds + (rr + p * RPP) * PITCH + kq) = v;
-            }
+            for (int p = 0; p < NLOAD; ++p) v[p] = kpos[p] < k_valid ? r[p] : vec_t{};
+            L::put(lds, tid, v);
         } else {
-            constexpr int TPK = ROWS / VEC, KPP = NTHREADS / TPK;
-            const int rq = (tid % TPK) * VEC, kk = tid / TPK;
-#pragma unroll
-            for (int p = 0; p < NLOAD; ++p) {
-                vec_t v = r[p];
-                if (special && !(row_ok[p] && kpos[p] < k_valid)) v = vec_t{};
-                *reinterpret_cast<vec_t *>(lds + (kk + p * KPP) * ROWS + rq) = v;
-            }
+            L::put(lds, tid, r);
         }
     }
 };
@@ -257,21 +315,17 @@ struct FastStage {
 // share them) and handed to load(); everything else is FastStage.
 template <int ROWS>
 struct GatherStage {
-    static constexpr int NLOAD = (ROWS * BK) / (NTHREADS * 4);
-    static constexpr int TPK = ROWS / 4, KPP = NTHREADS / TPK;
+    typedef TileLayout<4, false, ROWS> L;
+    static constexpr int NLOAD = L::NLOAD;
     float4 r[NLOAD];
     unsigned roff;   // byte offset of the thread's four rows inside a k line (clamped into the matrix)
-    int kk;          // the thread's first k line inside a tile; its others follow at a distance of KPP
-    bool row_ok;
-    bool edge;       // uniform: some row of this tile lies outside the matrix
+    int kk;          // the thread's first k line inside a tile; its others follow
     int k_valid;     // uniform: k lines of the tile in registers that are listed
 
     __device__ __forceinline__ void init(int row0, int rows_total, int tid) {
-        edge = row0 + ROWS > rows_total;
-        const int rq = (tid % TPK) * 4;
-        kk = tid / TPK;
-        row_ok = (row0 + rq) < rows_total;
-        roff = (unsigned)((row_ok ? row0 + rq : 0) * sizeof(float));
+        const int rq = L::first_row(tid);
+        kk = L::first_k(tid);
+        roff = (unsigned)(((row0 + rq) < rows_total ? row0 + rq : 0) * sizeof(float));
     }
     // line_bytes and the indices are below 2^24 and the operand below 4 GiB (checked by the launcher): a 24-bit multiply-add
     // gives the 32-bit offset beside the uniform base
@@ -282,35 +336,64 @@ struct GatherStage {
         for (int p = 0; p < NLOAD; ++p)
             r[p] = *reinterpret_cast<const float4 *>(b + (__umul24((unsigned)idx[p], line_bytes) + roff));
     }
-    __device__ __forceinline__ void store(float *__restrict__ lds, int tid) const {
-        const bool special = edge || k_valid < BK;
-        const int rq = (tid % TPK) * 4;
+    __device__ __forceinline__ void store(uint4 *__restrict__ lds, int tid) const {
+        if (k_valid < BK) {
+            float4 v[NLOAD];
 #pragma unroll
-        for (int p = 0; p < NLOAD; ++p) {
-            float4 v = r[p];
-            if (special && !(row_ok && kk + p * KPP < k_valid)) v = float4{0.0f, 0.0f, 0.0f, 0.0f};
-            *reinterpret_cast<float4 *>(lds + (kk + p * KPP) * ROWS + rq) = v;
+            for (int p = 0; p < NLOAD; ++p) v[p] = kk + p < k_valid ? r[p] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+            L::put(lds, tid, v);
+        } else {
+            L::put(lds, tid, r);
         }
     }
 };
 
+// One element of the product over the k tiles [it_begin, it_end) in plain fp32, for the few that the split product cannot
+// form: an operand that is infinite or rounds to an infinite bf16 value leaves infinity minus infinity in its parts.
+template <bool AK, bool BK_, bool MASKED, bool GATHER>
+__device__ __forceinline__ float plain_element(const GemmArgs &args, const GemmProblem &pb, int m, int n, int it_begin,
+                                                         int it_end, int kt_per_seg, int k_extent, int k_lo) {
+    float sum = 0.0f;
+    for (int it = it_begin; it < it_end; ++it) {
+        const int seg = it / kt_per_seg, k0 = (it % kt_per_seg) * BK, k1 = min(k0 + BK, k_extent);
+        for (int kk = k0; kk < k1; ++kk) {
+            const int k = GATHER ? args.k_order[k_lo + kk] + pb.k_shift : kk;
+            int bk = k, bn = n;
+            bool keep = true;
+            if (MASKED && args.pat) {
+                const int u = args.b_time_on_k ? k : n, src = u + pb.b_shift[seg];
+                keep = args.pat[u] != 0 && src >= 0 && src < args.n_slots && args.pat[src] != 0;
+                if (args.b_time_on_k) bk = src; else bn = src;
+            }
+            const float a = pb.A[seg][AK ? (size_t)m * args.lda + k : (size_t)k * args.lda + m];
+            const float b = keep ? pb.B[seg][BK_ ? (size_t)bn * args.ldb + bk : (size_t)bk * args.ldb + bn] : 0.0f;
+            sum = __builtin_fmaf(a, b, sum);
+        }
+    }
+    return sum;
+}
+
 // MASKED selects the time-shifted, padding-masked B loader at compile time: its per-element predication is a lot
-// of code, and four copies of it (two prologue fetches, two in the unrolled loop) inside the plain kernels would
+// of code, which inside the plain kernels would
 // push their hot loop out of the instruction cache.
 // FAN: the EPI_FAN epilogue, a kernel of its own (instantiated for 16-byte row-contiguous A and k-contiguous B only,
 // the shapes of the error products that use it) so that its registers and code stay out of every other product.
 // GATHER: the k lines of both (row-contiguous, 16-byte aligned) operands are those a list names (GemmArgs::k_order).
+// The workgroups a compute unit is to hold (by registers; LDS allows as many) are what hides one's loads and conversions
+// behind another's matrix instructions.
 template <int VA, bool AK, int VB, bool BK_, bool MASKED, int TILE, bool FAN = false, bool GATHER = false>
-__global__ __launch_bounds__(NTHREADS) void gemm_f32_kernel(const GemmArgs args) {
+__global__ __launch_bounds__(NTHREADS, TILE == 128 ? 3 : VA == 1 || VB == 1 ? 4 : 5) void gemm_split_kernel(const GemmArgs args) {
     constexpr int BM = TILE, BN = TILE;
     constexpr int WT = TILE / 2;   // edge of a wave's block (waves are arranged 2 x 2)
     constexpr int NB = WT / 32;    // 32 x 32 MFMA tiles per wave and dimension
-    __shared__ __attribute__((aligned(16))) float lds_a[2][BM * PITCH];
-    __shared__ __attribute__((aligned(16))) float lds_b[2][BN * PITCH];
+    typedef TileLayout<VA, AK, TILE> LA;
+    typedef TileLayout<VB, BK_, TILE> LB;
+    __shared__ uint4 lds[LA::UNITS + LB::UNITS];
+    uint4 *const lds_a = lds, *const lds_b = lds + LA::UNITS;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 1, wn = wave >> 1;
 
     // Which tile, k range and problem this workgroup takes.  Workgroups go to the eight XCDs in turn, in launch
@@ -363,83 +446,69 @@ __global__ __launch_bounds__(NTHREADS) void gemm_f32_kernel(const GemmArgs args)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-    // Two register sets per operand: tile it+1 waits in one of them while tile it+2 is being fetched into the
-    // other, so that a global load has two k-iterations of MFMA work (about 4000 clocks) to arrive in; with one
-    // workgroup per compute unit, which is what the benchmark's shapes give, nothing else hides that latency.
-    // The loop is unrolled by two so that the sets swap roles without register copies, and its barrier orders
-    // LDS only (__syncthreads() would also drain the loads in flight).
     const char *mask_pat = MASKED ? args.pat : nullptr;
-    constexpr bool kStoreEarly = true;
 
-    // sum of the B operand over this split's k range, per row (dense bias gradient); kept by the waves with wm == 0
-    const bool rowsum = args.rowsum != 0;
+    // sum of the B operand over this split's k range, per row (dense bias gradient); the waves that keep it run a loop
+    // of their own, and only the operand kinds of a weight gradient have one
+    const bool rowsum = !AK && !BK_ && !MASKED && args.rowsum != 0 && wm == 0 && m0 == 0;
     float rs[NB];
 #pragma unroll
     for (int j = 0; j < NB; ++j) rs[j] = 0.0f;
 
     const int frag_row = lane & 31;
-    constexpr int FK = BK / 2;  // k values per half-wave and tile
-    const int frag_k = (lane >> 5) * FK;
+    const int half = lane >> 5;
 
-    // `fetch_next(a, b)` loads the next tile of the walk into a pair of register sets; after the last tile it loads
-    // that one again, so that the count of loads in flight is the same on every path.
-    auto run = [&](auto &a0, auto &b0, auto &a1, auto &b1, auto &fetch_next) __attribute__((always_inline)) {
-        fetch_next(a0, b0);
-        fetch_next(a1, b1);
-        a0.store(lds_a[0], tid);
-        b0.store(lds_b[0], tid);
-        lds_only_barrier();
-        // one k-iteration on LDS buffer `cur`; `held` carries tile it+1, `recv` receives tile it+2
-        auto iterate = [&](int it, int cur, auto &held_a, auto &held_b, auto &recv_a, auto &recv_b) __attribute__((always_inline)) {
-            fetch_next(recv_a, recv_b);
-            __builtin_amdgcn_sched_barrier(0);  // keep the loads ahead of the MFMA block: the scheduler would sink them
-            if (kStoreEarly && it + 1 < it_end) {
-                // the tile that arrived during the last iteration goes to the other LDS buffer (free since the barrier)
-                // while this iteration's fragments are on their way, not behind the last MFMA
-                held_a.store(lds_a[cur ^ 1], tid);
-                held_b.store(lds_b[cur ^ 1], tid);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-
-            float fa[NB][FK], fb[NB][FK];
+    // `fetch_next(a, b)` loads the next tile of the walk into the register sets; after the last tile it loads that one
+    // again, so that the count of loads in flight is the same on every path.  The loads of tile it+1 are in flight during
+    // the matrix instructions of tile it; the barriers order LDS only (__syncthreads() would also wait for those loads).
+    auto loop = [&](auto &ra, auto &rb, auto &fetch_next, auto sums) __attribute__((always_inline)) {
+        fetch_next(ra, rb);
+        for (int it = it_begin; it < it_end; ++it) {
+            ra.store(lds_a, tid);
+            rb.store(lds_b, tid);
+            fetch_next(ra, rb);
+            lds_only_barrier();
 #pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                TileStage<VA, AK, TILE>::fragment(lds_a[cur], wm * WT + i * 32 + frag_row, frag_k, fa[i]);
-                TileStage<VB, BK_, TILE>::fragment(lds_b[cur], wn * WT + i * 32 + frag_row, frag_k, fb[i]);
-            }
+            for (int s = 0; s < BK / 16; ++s) {
+                bf16x8 fa[NB][3], fb[NB][3];
 #pragma unroll
-            for (int kk = 0; kk < FK; ++kk) {
+                for (int i = 0; i < NB; ++i) LA::fragment(lds_a, wm * WT + i * 32 + frag_row, 2 * s + half, fa[i]);
 #pragma unroll
-                for (int i = 0; i < NB; ++i) {
+                for (int j = 0; j < NB; ++j) LB::fragment(lds_b, wn * WT + j * 32 + frag_row, 2 * s + half, fb[j]);
+                // h*l, l*h, m*m, h*m, m*h, h*h: the small terms first
+                constexpr int QA[6] = {0, 2, 1, 0, 1, 0}, QB[6] = {2, 0, 1, 1, 0, 0};
+#pragma unroll
+                for (int t = 0; t < 6; ++t)
+#pragma unroll
+                    for (int i = 0; i < NB; ++i)
+#pragma unroll
+                        for (int j = 0; j < NB; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j][QB[t]], fa[i][QA[t]], acc[i][j], 0, 0, 0);
+                if constexpr (decltype(sums)::value) {
 #pragma unroll
                     for (int j = 0; j < NB; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j][kk], fa[i][kk], acc[i][j], 0, 0, 0);
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) rs[j] += ((float)fb[j][2][e] + (float)fb[j][1][e]) + (float)fb[j][0][e];
                 }
             }
-            if (rowsum) {
-#pragma unroll
-                for (int j = 0; j < NB; ++j)
-#pragma unroll
-                    for (int kk = 0; kk < FK; ++kk) rs[j] += fb[j][kk];
-            }
-
-            if (!kStoreEarly && it + 1 < it_end) {
-                held_a.store(lds_a[cur ^ 1], tid);
-                held_b.store(lds_b[cur ^ 1], tid);
-            }
             lds_only_barrier();
-        };
-        for (int it = it_begin; it < it_end; it += 2) {
-            iterate(it, 0, a1, b1, a0, b0);
-            if (it + 1 < it_end) iterate(it + 1, 1, a0, b0, a1, b1);
         }
+    };
+    auto run = [&](auto &ra, auto &rb, auto &fetch_next) __attribute__((always_inline)) {
+        if constexpr (!AK && !BK_ && !MASKED) {
+            if (rowsum) {
+                loop(ra, rb, fetch_next, std::true_type());
+                return;
+            }
+        }
+        loop(ra, rb, fetch_next, std::false_type());
     };
     if constexpr (GATHER) {
         static_assert(VA == 4 && VB == 4 && !AK && !BK_ && !MASKED, "the gathering loader is for two row-contiguous operands");
-        GatherStage<TILE> ga0, ga1, gb0, gb1;
-        ga0.init(m0, args.m, tid); ga1.init(m0, args.m, tid);
-        gb0.init(n0, args.n, tid); gb1.init(n0, args.n, tid);
-        constexpr int NL = GatherStage<TILE>::NLOAD, KPP = GatherStage<TILE>::KPP;
+        GatherStage<TILE> ga, gb;
+        ga.init(m0, args.m, tid);
+        gb.init(n0, args.n, tid);
+        constexpr int NL = GatherStage<TILE>::NLOAD;
         const int *__restrict__ order = args.k_order + k_lo;
         const int k_shift = pb.k_shift;
         const unsigned a_line = (unsigned)(args.lda * sizeof(float)), b_line = (unsigned)(args.ldb * sizeof(float));
@@ -449,7 +518,7 @@ __global__ __launch_bounds__(NTHREADS) void gemm_f32_kernel(const GemmArgs args)
         int idx[NL];
         auto lines_of = [&](int tile) __attribute__((always_inline)) {
 #pragma unroll
-            for (int p = 0; p < NL; ++p) idx[p] = order[max(min(tile * BK + ga0.kk + p * KPP, k_extent - 1), 0)] + k_shift;
+            for (int p = 0; p < NL; ++p) idx[p] = order[max(min(tile * BK + ga.kk + p, k_extent - 1), 0)] + k_shift;
         };
         lines_of(kin);
         auto fetch_next = [&](GatherStage<TILE> &qa, GatherStage<TILE> &qb) __attribute__((always_inline)) {
@@ -465,10 +534,10 @@ __global__ __launch_bounds__(NTHREADS) void gemm_f32_kernel(const GemmArgs args)
             }
             lines_of(kin);
         };
-        if (it_begin < it_end) run(ga0, gb0, ga1, gb1, fetch_next);
+        if (it_begin < it_end) run(ga, gb, fetch_next);
     } else if constexpr (MASKED) {
-        TileStage<VA, AK, TILE> sa0, sa1;
-        TileStage<VB, BK_, TILE> sb0, sb1;
+        TileStage<VA, AK, TILE> sa;
+        TileStage<VB, BK_, TILE> sb;
         int next_it = it_begin;
         auto fetch_next = [&](TileStage<VA, AK, TILE> &ra, TileStage<VB, BK_, TILE> &rb) __attribute__((always_inline)) {
             const int it = min(next_it, it_end - 1);
@@ -479,14 +548,14 @@ __global__ __launch_bounds__(NTHREADS) void gemm_f32_kernel(const GemmArgs args)
             rb.load(pb.B[seg], args.ldb, n0, k0, args.n, args.k, tid, mask_pat, pb.b_shift[seg], args.n_slots,
                     args.b_time_on_k != 0);
         };
-        run(sa0, sb0, sa1, sb1, fetch_next);
+        run(sa, sb, fetch_next);
     } else {
         // the tile cursor: operand pair `seg`, k tile `kin` inside it; the operands' base pointers are looked up only
         // when the pair changes
-        FastStage<VA, AK, TILE> qa0, qa1;
-        FastStage<VB, BK_, TILE> qb0, qb1;
-        qa0.init(args.lda, m0, args.m, tid); qa1.init(args.lda, m0, args.m, tid);
-        qb0.init(args.ldb, n0, args.n, tid); qb1.init(args.ldb, n0, args.n, tid);
+        FastStage<VA, AK, TILE> sa;
+        FastStage<VB, BK_, TILE> sb;
+        sa.init(args.lda, m0, args.m, tid);
+        sb.init(args.ldb, n0, args.n, tid);
         int seg = it_begin / kt_per_seg, kin = it_begin % kt_per_seg, left = it_end - it_begin - 1;
         const float *pa = pb.A[seg], *pbb = pb.B[seg];
         const size_t ka = AK ? 1 : (size_t)args.lda, kb = BK_ ? 1 : (size_t)args.ldb;  // floats per k step
@@ -502,12 +571,40 @@ __global__ __launch_bounds__(NTHREADS) void gemm_f32_kernel(const GemmArgs args)
                 }
             }
         };
-        run(qa0, qb0, qa1, qb1, fetch_next);
+        run(sa, sb, fetch_next);
+    }
+
+    // what came out infinite or not a number is formed again (plain_element)
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) finite = finite && __builtin_fabsf(acc[i][j][r]) <= lim::kMax;
+    if (__builtin_expect(!finite, 0)) {
+        // through LDS, where a rolled loop can index a thread's sums: this code is cold and should take no registers
+        static_assert(NB * 16 * NTHREADS * sizeof(float) <= sizeof(lds), "a row of accumulators fits the tile's buffer");
+        float *mine = reinterpret_cast<float *>(lds) + tid;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+#pragma unroll
+            for (int e = 0; e < NB * 16; ++e) mine[e * NTHREADS] = acc[i][e / 16][e % 16];
+            const int m = m0 + wm * WT + i * 32 + frag_row;
+#pragma unroll 1
+            for (int e = 0; e < NB * 16; ++e) {
+                const int r = e % 16, n = n0 + wn * WT + (e / 16) * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+                if (!(__builtin_fabsf(mine[e * NTHREADS]) <= lim::kMax) && m < args.m && n < args.n)
+                    mine[e * NTHREADS] =
+                        plain_element<AK, BK_, MASKED, GATHER>(args, pb, m, n, it_begin, it_end, kt_per_seg, k_extent, k_lo);
+            }
+#pragma unroll
+            for (int e = 0; e < NB * 16; ++e) acc[i][e / 16][e % 16] = mine[e * NTHREADS];
+        }
     }
 
     // epilogue: lane%32 runs along m (contiguous), the 16 accumulators along n
     float *__restrict__ C = pb.C;
-    const int half = lane >> 5;
     if (args.epilogue == EPI_PARTIAL) {
         // this split's partial product, m x n column-major without padding, after those of the problems before it
         float *__restrict__ P = args.partial + (size_t)split_id * args.partial_stride +
@@ -525,7 +622,7 @@ __global__ __launch_bounds__(NTHREADS) void gemm_f32_kernel(const GemmArgs args)
                 }
             }
         }
-        if (rowsum && wm == 0 && m0 == 0) {
+        if (rowsum) {
             float *__restrict__ R = args.partial + (size_t)split_id * args.partial_stride +
                                     (size_t)args.nprob * args.m * args.n + (size_t)prob_id * args.n;
 #pragma unroll
@@ -616,31 +713,30 @@ __global__ __launch_bounds__(NTHREADS) void gemm_f32_kernel(const GemmArgs args)
     }
 }
 
-template <int VA, bool AK, int VB, bool BK_, int TILE>
-void launch_m(const GemmArgs &a, dim3 grid, hipStream_t s) {
-    if (a.epilogue == EPI_FAN) {
-        // gemm_launch has checked that the operands are of the one kind this exists for
-        if constexpr (VA == 4 && !AK && VB == 4 && BK_) {
-            if (a.masked)
-                hipLaunchKernelGGL((gemm_f32_kernel<VA, AK, VB, BK_, true, TILE, true>), grid, dim3(NTHREADS), 0, s, a);
-            else
-                hipLaunchKernelGGL((gemm_f32_kernel<VA, AK, VB, BK_, false, TILE, true>), grid, dim3(NTHREADS), 0, s, a);
-        }
-        return;
-    }
-    if (a.k_order) {
-        // gemm_launch has checked that the operands are of the one kind this exists for
-        if constexpr (VA == 4 && !AK && VB == 4 && !BK_ && TILE == 64)
-            hipLaunchKernelGGL((gemm_f32_kernel<VA, AK, VB, BK_, false, TILE, false, true>), grid, dim3(NTHREADS), 0, s, a);
-        return;
-    }
-    if (a.masked) hipLaunchKernelGGL((gemm_f32_kernel<VA, AK, VB, BK_, true, TILE>), grid, dim3(NTHREADS), 0, s, a);
-    else hipLaunchKernelGGL((gemm_f32_kernel<VA, AK, VB, BK_, false, TILE>), grid, dim3(NTHREADS), 0, s, a);
-}
 template <int VA, bool AK, int VB, bool BK_>
 void launch_t(const GemmArgs &a, dim3 grid, hipStream_t s, int tile) {
-    if (tile == 64) launch_m<VA, AK, VB, BK_, 64>(a, grid, s);
-    else launch_m<VA, AK, VB, BK_, 128>(a, grid, s);
+    // gemm_launch has checked the operand kinds of the two special products and that they, and the masked one, come with
+    // the small tile
+    if (a.epilogue == EPI_FAN) {
+        if constexpr (VA == 4 && !AK && VB == 4 && BK_) {
+            if (a.masked)
+                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, true, 64, true>), grid, dim3(NTHREADS), 0, s, a);
+            else
+                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64, true>), grid, dim3(NTHREADS), 0, s, a);
+        }
+    } else if (a.k_order) {
+        if constexpr (VA == 4 && !AK && VB == 4 && !BK_)
+            hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64, false, true>), grid, dim3(NTHREADS), 0, s, a);
+    } else if (a.masked) {
+        hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, true, 64>), grid, dim3(NTHREADS), 0, s, a);
+    } else {
+        if constexpr (VA == 4 && VB == 4)
+            if (tile == 128) {
+                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128>), grid, dim3(NTHREADS), 0, s, a);
+                return;
+            }
+        hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64>), grid, dim3(NTHREADS), 0, s, a);
+    }
 }
 template <int VA, bool AK, int VB>
 void launch_b(const GemmArgs &a, dim3 grid, hipStream_t s, bool bk, int tile) {

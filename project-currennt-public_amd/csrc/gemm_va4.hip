@@ -1,4 +1,4 @@
-// Instantiates one share of the fp32 MFMA matrix-product kernels (see gemm_kernel.hpp, gemm.hip).
+// Instantiates one share of the fp32 matrix-product kernels (see gemm_kernel.hpp, gemm.hip).
 #include "gemm_kernel.hpp"
 
 namespace cnt {

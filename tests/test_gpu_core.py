@@ -511,3 +511,56 @@ def test_lstm_recursion_geometries(L, bidir, lengths):
     if bidir and L % 2:
         L += 1
     assert PC.run_lstm_two_recursions(19, L, bidir, lengths, seed=L + len(lengths)) < TOL
+
+
+def _product(m, n, k, tA, tB, A, B):
+    import torch
+    C = torch.empty(m * n, device="cuda")
+    PC.pkg().capi.matrix_product(C, m, n, k, A, tA, B, tB, False)
+    A64 = (A.view(m, k) if tA else A.view(k, m).t()).double()
+    B64 = (B.view(k, n) if tB else B.view(n, k).t()).double()
+    return C.view(n, m).t().double(), A64, B64
+
+
+# sizes around the two tiles' edges, k around the staged depth, every vector width and both orientations; the last two take
+# the 128 x 128 tile (600 tiles and k >= 512)
+@pytest.mark.parametrize("m,n,k,tA,tB", [
+    (63, 65, 31, False, False), (64, 64, 32, True, False), (66, 130, 33, False, True), (132, 68, 36, True, False),
+    (257, 129, 97, False, False), (130, 66, 34, False, True), (1, 1, 1, False, False), (4, 1000, 100, False, True),
+    (3100, 3076, 516, True, False), (3076, 3100, 540, False, True),
+])
+def test_matrix_product_is_as_exact_as_fp32_sums(m, n, k, tA, tB):
+    """The operands are multiplied as three bf16 parts each: what the six part products leave out is below 2^-25 of
+    |a||b| per term, and every sum is fp32, so the bound of a plain fp32 product holds: (k + 2) * 2^-24 * |A||B|."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + 7 * n + 31 * k)
+    A = torch.randn(m * k, device="cuda", generator=g) * torch.exp2(
+        torch.randint(-20, 20, (m * k,), device="cuda", generator=g).float())
+    B = torch.randn(n * k, device="cuda", generator=g)
+    C, A64, B64 = _product(m, n, k, tA, tB, A, B)
+    bound = (k + 2) * 2.0 ** -24 * (A64.abs() @ B64.abs())
+    assert bool(((C - A64 @ B64).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m,n,k,tA,tB", [(70, 66, 37, True, False), (3100, 3076, 516, False, False)])
+def test_matrix_product_of_infinite_huge_and_missing_values(m, n, k, tA, tB):
+    """Values that have no finite bf16 parts give what fp32 arithmetic gives."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(5)
+    A, B = torch.randn(m * k, device="cuda", generator=g), torch.randn(n * k, device="cuda", generator=g)
+    row = (lambda i, q: i * k + q) if tA else (lambda i, q: q * m + i)
+    A[row(3, 5)], A[row(9, 0)], A[row(20, k - 1)] = float("inf"), float("nan"), -float("inf")
+    A[row(40, 2)] = 3.402823e38                          # rounds to an infinite bf16 value
+    A[row(50, 7)], A[row(50, 8)] = float("inf"), -float("inf")
+    B64 = B.view(n, k)
+    B64[:, 2] = 0.25                                     # keeps the huge row finite
+    B64[11, 5] = 0.0                                     # infinity times zero
+    C, A64, B64 = _product(m, n, k, tA, tB, A, B)
+    want = torch.zeros_like(C)
+    for q in range(k):                                   # term by term: a library product may treat infinities its own way
+        want += A64[:, q:q + 1] * B64[q:q + 1, :]
+    assert torch.equal(C.isnan(), want.isnan())
+    assert torch.equal(C.isposinf(), want.isposinf()) and torch.equal(C.isneginf(), want.isneginf())
+    finite = want.isfinite()
+    scale = (k + 2) * 2.0 ** -24 * (torch.nan_to_num(A64, 0.0, 0.0, 0.0).abs() @ torch.nan_to_num(B64).abs())
+    assert bool(((C - want).abs() <= scale)[finite].all())
