@@ -207,7 +207,7 @@ struct GemmArgs {
     // or both NULL): only the k lines k_order[lo .. lo + n) of the operands are read, the others being all zero in at least
     // one operand.  k_count[0] = number of listed lines; with GemmProblem::k_trim = 1 the problem leaves out the first
     // k_count[1] of them (the lines of the first time step), with 2 the last k_count[2] (those of the last time step).  The
-    // launcher uses the list where both operands are row-contiguous and 16-byte aligned and the tile is 64 x 64, and
+    // launcher uses the list where both operands are row-contiguous and 16-byte aligned, and
     // multiplies all k lines otherwise -- so the operands' base pointers must be valid for both readings.
     const int *k_order;
     const int *k_count;

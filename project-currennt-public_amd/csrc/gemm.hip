@@ -60,11 +60,24 @@ inline int pick_vec(const GemmArgs &a, bool for_a) {
 // (64 / 128, us: 1024 x 12000 x 1024 with 752 large tiles 200 / 165; 1024 x 6000 x 512 with 376 of them 54 / 56; 512 x
 // 6000 x 512 with 188 30 / 51; 1024 x 32000 x 128 with 2000 71 / 103).  They exist for operands with 16-byte vectors only: with narrower
 // ones the loader's registers spill (425 x 12000 x 1024: 100 / 396).
+inline long large_tiles(const GemmArgs &a) { return (long)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.nprob; }
+
+// The weight gradient of one dense layer of 64 large tiles or more (1024 x 1024 weights) also takes the large tile, and as
+// many splits of k as make two workgroups per compute unit (the parts of two row-contiguous operands take 55 KB of LDS, so more do not
+// fit): the feed-forward model of five such layers 2320 -> 2224 us per pass, 768 workgroups 2230.  The gradients of a
+// recurrent layer, several problems per launch, run beside the recursion of the layer below and leave it less LDS and
+// issue slots then: with them on the large tile the acoustic model's pass takes 3787 instead of 3767 us.
+constexpr long kWideGradientGroups = 512;
+inline bool wide_gradient(const GemmArgs &a) {
+    return a.nprob == 1 && !a.masked && !a.a_kcontig && !a.b_kcontig && large_tiles(a) >= 64 && large_tiles(a) <= kWideGradientGroups / 2;
+}
+
 int pick_tile(const GemmArgs &a, int va, int vb) {
     static const int forced = [] { const char *e = std::getenv("CNT_GEMM_TILE"); return e ? std::atoi(e) : 0; }();
     if (va != 4 || vb != 4 || a.masked || a.epilogue == EPI_FAN) return 64;
     if (forced == 64 || forced == 128) return forced;
-    const long t128 = (long)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.splitk * a.nprob;
+    const long t128 = large_tiles(a) * a.splitk;
+    if (wide_gradient(a) && t128 >= kWideGradientGroups / 2) return 128;
     return t128 >= 600 && (long)a.k * a.nseg / a.splitk >= 512 ? 128 : 64;
 }
 
@@ -226,6 +239,8 @@ void gemm_plan(GemmArgs &args, hipStream_t stream) {
     const int target = forced_target > 0 ? forced_target : ((long)args.m * args.n <= 16384 ? 1024 : tiles >= 64 ? 768 : 512);
     const long kt = ((long)args.k + BK - 1) / BK * args.nseg;
     long s = (target + tiles - 1) / tiles;
+    if (forced_target == 0 && wide_gradient(args) && pick_vec(args, true) == 4 && pick_vec(args, false) == 4)
+        s = kWideGradientGroups / large_tiles(args);
     s = std::min(s, std::max(1L, kt / 8));
     s = std::max(1L, s);
     // no empty split: every split of the partial-product path has to write its share
@@ -288,7 +303,7 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
     if (!use_lines) args.k_order = nullptr;
     // a list of k lines is used where the kernel that reads through it exists, and ignored otherwise (the lines it leaves
     // out are zero)
-    if (args.k_order && !(args.k_count && !args.masked && !args.a_kcontig && !args.b_kcontig && va == 4 && vb == 4 && tile == 64 &&
+    if (args.k_order && !(args.k_count && !args.masked && !args.a_kcontig && !args.b_kcontig && va == 4 && vb == 4 &&
                           args.epilogue != EPI_FAN && args.k < (1 << 24) && args.lda < (1 << 22) && args.ldb < (1 << 22)))
         args.k_order = nullptr;
     const int tiles = ((args.m + tile - 1) / tile) * ((args.n + tile - 1) / tile);

@@ -725,8 +725,12 @@ void launch_t(const GemmArgs &a, dim3 grid, hipStream_t s, int tile) {
                 hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64, true>), grid, dim3(NTHREADS), 0, s, a);
         }
     } else if (a.k_order) {
-        if constexpr (VA == 4 && !AK && VB == 4 && !BK_)
-            hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64, false, true>), grid, dim3(NTHREADS), 0, s, a);
+        if constexpr (VA == 4 && !AK && VB == 4 && !BK_) {
+            if (tile == 128)
+                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128, false, true>), grid, dim3(NTHREADS), 0, s, a);
+            else
+                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64, false, true>), grid, dim3(NTHREADS), 0, s, a);
+        }
     } else if (a.masked) {
         hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, true, 64>), grid, dim3(NTHREADS), 0, s, a);
     } else {

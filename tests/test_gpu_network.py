@@ -152,6 +152,48 @@ def test_weight_gradients_of_a_fraction_that_is_mostly_padding():
     net.close()
 
 
+@pytest.mark.parametrize("lengths", [(400, 250, 3), (353, 352, 352)])
+def test_weight_gradients_of_wide_dense_layers(lengths):
+    """1024 x 1028 weights take the large tile, with the fraction's valid slots or all of them as the inner dimension."""
+    import torch
+
+    print("network case: wide dense layers", lengths, flush=True)
+    capi, networks = PC.pkg().capi, PC.networks()
+    P, Q, S, T = 20, 8, 3, lengths[0]
+    specs = [{"name": "ff1", "type": "feedforward_tanh", "size": 1024, "bias": 1.0},
+             {"name": "ff2", "type": "feedforward_logistic", "size": 1028, "bias": 0.5},
+             {"name": "out", "type": "feedforward_identity", "size": Q, "bias": 1.0},
+             {"name": "postoutput", "type": "sse", "size": Q}]
+    weights = OM.init_weights(P, specs, 19, 0.1)
+    doc = {"layers": [{"size": P, "name": "input", "type": "input"}] + specs, "weights": {}}
+    wi, prev = iter(weights), P
+    for sp in specs:
+        n_in, n_bias, _ = networks.weight_sections(sp, prev)
+        if n_in:
+            _sections(doc["weights"], sp["name"], next(wi), n_in, n_bias)
+        prev = sp["size"]
+    net = capi.Network(json.dumps(doc), S, T)
+    rng = np.random.default_rng(20)
+    pat = make_pat_types(list(lengths), T)
+    x = rng.standard_normal((T, S, P)).astype(np.float32)
+    tgt = (0.3 * rng.standard_normal((T, S, Q))).astype(np.float32)
+    valid = (pat != 0).reshape(T, S)
+    x[~valid] = 0
+    tgt[~valid] = 0
+    net.load_sequences(PC.dev(pat), T, min(lengths), PC.dev(x.reshape(-1)), PC.dev(tgt.reshape(-1)))
+    net.forward()
+    net.backward()
+    net.check()
+    ref = OM.OracleNetwork(P, specs, S, T, min(lengths), pat, [w.copy() for w in weights])
+    ref.forward(x.reshape(-1), tgt.reshape(-1))
+    ref.backward()
+    grads = [L["updates"] for L in ref.layers if "updates" in L]
+    torch.cuda.synchronize()
+    for L, g in zip([L for L in net.layers if L["weight_count"]], grads):
+        assert PC.relerr(L["updates"].cpu().numpy(), g) < TOL, L["name"]
+    net.close()
+
+
 def test_network_reports_a_later_lstm_layer_that_gave_up_and_keeps_the_weights():
     """Failure handling at network level, forced from the host: the SECOND recurrent layer's recursions get a spin
     limit of zero, the first layer's stay as they are.  Every kernel still ends normally; the failure is reported by
