@@ -14,8 +14,10 @@
 // adds two, so the result is closer to a 64-bit product than before: 2-norm error 4.9e-7 against 5.7e-7 at k = 1024, 1.2e-6
 // against 1.4e-6 at k = 6000, 1.6e-7 against 2.0e-7 at k = 128.  Values that are infinite, or round to an infinite bf16
 // value, leave infinity minus infinity in their parts; a sum that is not finite is formed again in plain fp32.
-//   1024 x 12000 x 1024: 283 -> 167 us (150 TFLOP/s), 512 x 6000 x 512: 40 -> 30 us, 1024 x 6000 x 512: 74 -> 55 us,
-//   1024 x 32000 x 128: 108 -> 72 us, 425 x 12000 x 1024: 141 -> 100 us.
+//   1024 x 12000 x 1024: 283 -> 157 us (160 TFLOP/s), 512 x 6000 x 512: 40 -> 30 us, 1024 x 6000 x 512: 74 -> 57 us,
+//   1024 x 32000 x 128: 108 -> 73 us, 425 x 12000 x 1024: 141 -> 97 us, 300 x 10000 x 425: 47 -> 35 us.
+// Operands whose lines are no multiple of four long are read in vectors of four as well (FastStage); with one float per
+// lane and load the last two sizes took 100 and 43 us.
 // What bounds it now, at the first size per SIMD: 69 us of matrix instructions, 38 us of conversions, 51 us of LDS traffic,
 // which overlap only in part.  Measured and not taken: the conversion of the next tile between the matrix instructions of
 // this one, with two LDS buffers and one or two tiles of loads in flight (245 us: one wave per SIMD issues a vector
@@ -58,8 +60,7 @@ inline int pick_vec(const GemmArgs &a, bool for_a) {
 // Tile edge.  128 x 128 tiles convert and read half as much per matrix instruction, but three of them fill a compute unit, so a
 // launch needs some 600 of them, and a run over k long enough that filling and draining the pipeline does not show
 // (64 / 128, us: 1024 x 12000 x 1024 with 752 large tiles 200 / 165; 1024 x 6000 x 512 with 376 of them 54 / 56; 512 x
-// 6000 x 512 with 188 30 / 51; 1024 x 32000 x 128 with 2000 71 / 103).  They exist for operands with 16-byte vectors only: with narrower
-// ones the loader's registers spill (425 x 12000 x 1024: 100 / 396).
+// 6000 x 512 with 188 30 / 51; 1024 x 32000 x 128 with 2000 71 / 103).
 inline long large_tiles(const GemmArgs &a) { return (long)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.nprob; }
 
 // The weight gradient of one dense layer of 64 large tiles or more (1024 x 1024 weights) also takes the large tile, and as
@@ -72,9 +73,9 @@ inline bool wide_gradient(const GemmArgs &a) {
     return a.nprob == 1 && !a.masked && !a.a_kcontig && !a.b_kcontig && large_tiles(a) >= 64 && large_tiles(a) <= kWideGradientGroups / 2;
 }
 
-int pick_tile(const GemmArgs &a, int va, int vb) {
+int pick_tile(const GemmArgs &a) {
     static const int forced = [] { const char *e = std::getenv("CNT_GEMM_TILE"); return e ? std::atoi(e) : 0; }();
-    if (va != 4 || vb != 4 || a.masked || a.epilogue == EPI_FAN) return 64;
+    if (a.masked || a.epilogue == EPI_FAN) return 64;
     if (forced == 64 || forced == 128) return forced;
     const long t128 = large_tiles(a) * a.splitk;
     if (wide_gradient(a) && t128 >= kWideGradientGroups / 2) return 128;
@@ -239,7 +240,7 @@ void gemm_plan(GemmArgs &args, hipStream_t stream) {
     const int target = forced_target > 0 ? forced_target : ((long)args.m * args.n <= 16384 ? 1024 : tiles >= 64 ? 768 : 512);
     const long kt = ((long)args.k + BK - 1) / BK * args.nseg;
     long s = (target + tiles - 1) / tiles;
-    if (forced_target == 0 && wide_gradient(args) && pick_vec(args, true) == 4 && pick_vec(args, false) == 4)
+    if (forced_target == 0 && wide_gradient(args))
         s = kWideGradientGroups / large_tiles(args);
     s = std::min(s, std::max(1L, kt / 8));
     s = std::max(1L, s);
@@ -295,27 +296,31 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
     CNT_REQUIRE(args.masked || (reachable(args.m, args.lda, args.a_kcontig) && reachable(args.n, args.ldb, args.b_kcontig)),
                 "gemm: operands of 4 GiB and more are not supported (%d x %d x %d, lda %d, ldb %d)", args.m, args.n, args.k,
                 args.lda, args.ldb);
-    const int va = pick_vec(args, true), vb = pick_vec(args, false);
+    int va = pick_vec(args, true), vb = pick_vec(args, false);
+    const bool aligned = va == 4 && vb == 4;
+    if (!args.masked && args.epilogue != EPI_FAN) {  // the unmasked loader goes by the length of the lines alone
+        va = (args.a_kcontig ? args.k : args.m) % 4 == 0 ? 4 : 1;
+        vb = (args.b_kcontig ? args.k : args.n) % 4 == 0 ? 4 : 1;
+    }
     gemm_plan(args, stream);
     if (args.epilogue != EPI_PARTIAL) args.rowsum = 0;
-    const int tile = pick_tile(args, va, vb);
+    const int tile = pick_tile(args);
     static const bool use_lines = [] { const char *e = std::getenv("CNT_GEMM_K_ORDER"); return !e || std::atoi(e) != 0; }();
     if (!use_lines) args.k_order = nullptr;
     // a list of k lines is used where the kernel that reads through it exists, and ignored otherwise (the lines it leaves
     // out are zero)
-    if (args.k_order && !(args.k_count && !args.masked && !args.a_kcontig && !args.b_kcontig && va == 4 && vb == 4 &&
+    if (args.k_order && !(args.k_count && !args.masked && !args.a_kcontig && !args.b_kcontig && aligned &&
                           args.epilogue != EPI_FAN && args.k < (1 << 24) && args.lda < (1 << 22) && args.ldb < (1 << 22)))
         args.k_order = nullptr;
     const int tiles = ((args.m + tile - 1) / tile) * ((args.n + tile - 1) / tile);
     dim3 grid(tiles, args.splitk, args.nprob);
-    // XCD-aware placement (gemm_kernel.hpp) for launches of several problems: measured with FETCH_SIZE on MI355X it
-    // cuts what the L2s fetch 2.2-2.6x for the WaveNet stack's batched weight gradients (a convolution's two taps and
-    // a stack's conditioning projections share an operand) and ends that pass 0.5% sooner.  For one problem per launch
-    // it cuts the fetches 2-4x as well (the acoustic model's weight gradients: 270 -> 68 MB) and the products run 1%
-    // faster, but that model's pass came out 0.7% slower in every run, so single problems keep the launch order
-    // (CNT_GEMM_XCD_MAP=2 maps them too, 0 maps nothing).
-    static const int xcd_map = [] { const char *e = std::getenv("CNT_GEMM_XCD_MAP"); return e ? std::atoi(e) : 1; }();
-    args.xcd_map = (xcd_map == 2 || (xcd_map == 1 && args.nprob > 1)) && (long)tiles * args.splitk * args.nprob >= 16 ? 1 : 0;
+    // XCD-aware placement (gemm_kernel.hpp): measured with FETCH_SIZE on MI355X it cuts what the L2s fetch 2.2-2.6x for the
+    // WaveNet stack's batched weight gradients (a convolution's two taps and a stack's conditioning projections share an
+    // operand) and 2-4x for single problems (the acoustic model's weight gradients: 270 -> 68 MB).  Since the products run on the
+    // bf16 instructions they feel it: the feed-forward model's pass takes 2283 us with single problems mapped, 2363 without, the
+    // models with recurrent layers 0.1-0.5% less.
+    static const bool xcd_map = [] { const char *e = std::getenv("CNT_GEMM_XCD_MAP"); return !e || std::atoi(e) != 0; }();
+    args.xcd_map = xcd_map && (long)tiles * args.splitk * args.nprob >= 16 ? 1 : 0;
     ProfileScope prof(stream, args.label ? args.label : "gemm");
     std::unique_lock<std::mutex> split_lock(g_split_mu, std::defer_lock);
     // a product and its reduction stay adjacent on the stream

@@ -244,70 +244,70 @@ struct TileStage {
     }
 };
 
-// The unmasked loader.  What a thread loads differs from tile to tile only by the tile's k
-// offset, so everything per thread is computed once: `voff`, the byte offset of its vector inside the operand at k = 0
-// (row clamped into the matrix), as a 32-bit offset beside a 64-bit base that is uniform over the workgroup -- the
-// address form that costs no vector arithmetic per load -- and which of its vectors lie inside the matrix.  A tile
-// needs masking only at the matrix edge or in the last, partly filled k tile of an operand pair; both are uniform over
-// the workgroup (`special`), every other tile is stored as it arrived.
-template <int VEC, bool KCONTIG, int ROWS>
+// The unmasked loader, in vectors of four floats at any float's address (the hardware loads 16 bytes from a multiple of 4; a
+// vector that is not aligned costs at most a second cache line, where one float per lane costs four times the instructions).
+// What a thread loads differs from tile to tile only by the tile's k offset, so everything per thread is computed once:
+// `voff`, the byte offset of its vector inside the operand at k = 0 (row clamped into the matrix), as a 32-bit offset beside
+// a 64-bit base that is uniform over the workgroup -- the address form that costs no vector arithmetic per load.  A vector may
+// reach beyond its own line only where it still ends inside the operand: rows outside the matrix reach only sums that are not
+// stored, and the tiles where a vector could leave the operand or hold k values beyond its end take a path of their own
+// (uniform over the workgroup), one float at a time unless the lines are a multiple of four long.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+// WHOLE: the lines are a multiple of four long, so that no vector crosses the end of one.
+template <bool WHOLE, bool KCONTIG, int ROWS>
 struct FastStage {
-    typedef TileLayout<VEC, KCONTIG, ROWS> L;
+    typedef TileLayout<4, KCONTIG, ROWS> L;
     static constexpr int NLOAD = L::NLOAD;
-    typedef typename VecT<VEC>::type vec_t;
-    vec_t r[NLOAD];
-    unsigned voff[NLOAD];    // byte offsets at k = 0
-    unsigned koff[NLOAD];    // what has to be taken off voff to reach k position 0 of the tile (used in a k tail only)
-    int kpos[NLOAD];         // first k of the vector inside the tile
-    int k_valid;             // uniform: k values of the tile in registers that lie inside the operand pair
+    float4 r[NLOAD];
+    unsigned voff[NLOAD];
+    int ld, row0, rows_total;  // uniform
 
-    __device__ __forceinline__ void init(int ld, int row0, int rows_total, int tid) {
-        if (KCONTIG) {
-            const int kq = L::first_k(tid);
+    __device__ __forceinline__ void init(int ld_, int row0_, int rows_total_, int tid) {
+        ld = ld_; row0 = row0_; rows_total = rows_total_;
 #pragma unroll
-            for (int p = 0; p < NLOAD; ++p) {
-                const int row = row0 + L::row(tid, p);
-                voff[p] = (unsigned)(((size_t)min(row, rows_total - 1) * ld + kq) * sizeof(float));
-                koff[p] = (unsigned)(kq * sizeof(float));
-                kpos[p] = kq;
-            }
-        } else {
-            const int rq = L::first_row(tid), kk = L::first_k(tid);
-#pragma unroll
-            for (int p = 0; p < NLOAD; ++p) {
-                const int k = kk + p;
-                const int rc = (row0 + rq) < rows_total ? row0 + rq : 0;
-                voff[p] = (unsigned)(((size_t)k * ld + rc) * sizeof(float));
-                koff[p] = (unsigned)((size_t)k * ld * sizeof(float));
-                kpos[p] = k;
-            }
+        for (int p = 0; p < NLOAD; ++p) {
+            const int row = row0 + L::row(tid, p), k = kpos(tid, p);
+            const int rc = KCONTIG ? min(row, rows_total - 1) : row < rows_total ? row : 0;
+            voff[p] = (unsigned)((KCONTIG ? (size_t)rc * ld + k : (size_t)k * ld + rc) * sizeof(float));
         }
     }
-    // base = the operand at the tile's first k (uniform), kv = valid k values of the tile
-    __device__ __forceinline__ void load(const float *__restrict__ base, int kv) {
-        k_valid = kv;
+    static __device__ __forceinline__ int kpos(int tid, int p) { return L::first_k(tid) + (KCONTIG ? 0 : p); }
+    // base = the operand at the tile's first k, left = k values from there to the operand's end (both uniform)
+    __device__ __forceinline__ void load(const float *__restrict__ base, int left, int tid) {
         const char *b = reinterpret_cast<const char *>(base);
-        if (kv >= BK) {
+        // (row-contiguous: a vector that crosses ends at most three floats behind its line, hence three lines behind at most)
+        if (left >= (KCONTIG || WHOLE ? BK : BK + 3)) {
 #pragma unroll
-            for (int p = 0; p < NLOAD; ++p) r[p] = *reinterpret_cast<const vec_t *>(b + voff[p]);
+            for (int p = 0; p < NLOAD; ++p) {
+                const f32x4u v = *reinterpret_cast<const f32x4u *>(b + voff[p]);
+                r[p] = float4{v[0], v[1], v[2], v[3]};
+            }
+        } else if (WHOLE) {
+#pragma unroll
+            for (int p = 0; p < NLOAD; ++p) {
+                const int k = kpos(tid, p);
+                const unsigned back = (unsigned)(k * (KCONTIG ? 1 : ld)) * (unsigned)sizeof(float);  // to k position 0
+                const f32x4u v = *reinterpret_cast<const f32x4u *>(b + (k < left ? voff[p] : voff[p] - back));
+                r[p] = k < left ? float4{v[0], v[1], v[2], v[3]} : float4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
         } else {
-            // partly filled tile: a vector beyond the operand's k extent is read from k position 0 instead (in bounds)
-            // and dropped at the store
+            int line = ld;
+            asm volatile("" : "+s"(line));  // the addresses below are formed here, not kept in registers through the loop
 #pragma unroll
-            for (int p = 0; p < NLOAD; ++p)
-                r[p] = *reinterpret_cast<const vec_t *>(b + (kpos[p] < kv ? voff[p] : voff[p] - koff[p]));
+            for (int p = 0; p < NLOAD; ++p) {
+                float e[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int k = kpos(tid, p) + (KCONTIG ? q : 0), kc = k < left ? k : 0;
+                    const int row = min(row0 + L::row(tid, p) + (KCONTIG ? 0 : q), rows_total - 1);
+                    const float v = base[KCONTIG ? (size_t)row * line + kc : (size_t)kc * line + row];
+                    e[q] = k < left ? v : 0.0f;
+                }
+                r[p] = float4{e[0], e[1], e[2], e[3]};
+            }
         }
     }
-    __device__ __forceinline__ void store(uint4 *__restrict__ lds, int tid) const {
-        if (k_valid < BK) {
-            vec_t v[NLOAD];
-#pragma unroll
-            for (int p = 0; p < NLOAD; ++p) v[p] = kpos[p] < k_valid ? r[p] : vec_t{};
-            L::put(lds, tid, v);
-        } else {
-            L::put(lds, tid, r);
-        }
-    }
+    __device__ __forceinline__ void store(uint4 *__restrict__ lds, int tid) const { L::put(lds, tid, r); }
 };
 
 // The unmasked loader for row-contiguous operands whose k lines are picked through a list (16-byte vectors only): tile k
@@ -373,6 +373,8 @@ __device__ __forceinline__ float plain_element(const GemmArgs &args, const GemmP
     return sum;
 }
 
+// VA, VB: vector widths of the masked loader, 16-byte alignment included; unmasked: 4 where the operand's lines are a
+// multiple of four long, at any alignment, else 1.
 // MASKED selects the time-shifted, padding-masked B loader at compile time: its per-element predication is a lot
 // of code, which inside the plain kernels would
 // push their hot loop out of the instruction cache.
@@ -382,12 +384,12 @@ __device__ __forceinline__ float plain_element(const GemmArgs &args, const GemmP
 // The workgroups a compute unit is to hold (by registers; LDS allows as many) are what hides one's loads and conversions
 // behind another's matrix instructions.
 template <int VA, bool AK, int VB, bool BK_, bool MASKED, int TILE, bool FAN = false, bool GATHER = false>
-__global__ __launch_bounds__(NTHREADS, TILE == 128 ? 3 : VA == 1 || VB == 1 ? 4 : 5) void gemm_split_kernel(const GemmArgs args) {
+__global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 ? 3 : 2) : VA * VB == 16 ? 5 : 4) void gemm_split_kernel(const GemmArgs args) {
     constexpr int BM = TILE, BN = TILE;
     constexpr int WT = TILE / 2;   // edge of a wave's block (waves are arranged 2 x 2)
     constexpr int NB = WT / 32;    // 32 x 32 MFMA tiles per wave and dimension
-    typedef TileLayout<VA, AK, TILE> LA;
-    typedef TileLayout<VB, BK_, TILE> LB;
+    typedef TileLayout<MASKED ? VA : 4, AK, TILE> LA;
+    typedef TileLayout<MASKED ? VB : 4, BK_, TILE> LB;
     __shared__ uint4 lds[LA::UNITS + LB::UNITS];
     uint4 *const lds_a = lds, *const lds_b = lds + LA::UNITS;
 
@@ -552,17 +554,16 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? 3 : VA == 1 || VB == 1 ? 4 
     } else {
         // the tile cursor: operand pair `seg`, k tile `kin` inside it; the operands' base pointers are looked up only
         // when the pair changes
-        FastStage<VA, AK, TILE> sa;
-        FastStage<VB, BK_, TILE> sb;
+        FastStage<VA == 4, AK, TILE> sa;
+        FastStage<VB == 4, BK_, TILE> sb;
         sa.init(args.lda, m0, args.m, tid);
         sb.init(args.ldb, n0, args.n, tid);
         int seg = it_begin / kt_per_seg, kin = it_begin % kt_per_seg, left = it_end - it_begin - 1;
         const float *pa = pb.A[seg], *pbb = pb.B[seg];
         const size_t ka = AK ? 1 : (size_t)args.lda, kb = BK_ ? 1 : (size_t)args.ldb;  // floats per k step
-        auto fetch_next = [&](FastStage<VA, AK, TILE> &qa, FastStage<VB, BK_, TILE> &qb) __attribute__((always_inline)) {
-            const int kv = min(BK, args.k - kin * BK);
-            qa.load(pa + (size_t)kin * BK * ka, kv);
-            qb.load(pbb + (size_t)kin * BK * kb, kv);
+        auto fetch_next = [&](FastStage<VA == 4, AK, TILE> &qa, FastStage<VB == 4, BK_, TILE> &qb) __attribute__((always_inline)) {
+            qa.load(pa + (size_t)kin * BK * ka, args.k - kin * BK, tid);
+            qb.load(pbb + (size_t)kin * BK * kb, args.k - kin * BK, tid);
             if (left > 0) {
                 --left;
                 if (++kin == kt_per_seg) {
@@ -733,13 +734,9 @@ void launch_t(const GemmArgs &a, dim3 grid, hipStream_t s, int tile) {
         }
     } else if (a.masked) {
         hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, true, 64>), grid, dim3(NTHREADS), 0, s, a);
-    } else {
-        if constexpr (VA == 4 && VB == 4)
-            if (tile == 128) {
-                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128>), grid, dim3(NTHREADS), 0, s, a);
-                return;
-            }
-        hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64>), grid, dim3(NTHREADS), 0, s, a);
+    } else if constexpr (VA != 2 && VB != 2) {
+        if (tile == 128) hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128>), grid, dim3(NTHREADS), 0, s, a);
+        else hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64>), grid, dim3(NTHREADS), 0, s, a);
     }
 }
 template <int VA, bool AK, int VB>

@@ -528,14 +528,19 @@ def _product(m, n, k, tA, tB, A, B):
     (63, 65, 31, False, False), (64, 64, 32, True, False), (66, 130, 33, False, True), (132, 68, 36, True, False),
     (257, 129, 97, False, False), (130, 66, 34, False, True), (1, 1, 1, False, False), (4, 1000, 100, False, True),
     (3100, 3076, 516, True, False), (3076, 3100, 540, False, True),
+    # lines of no multiple of four: vectors that cross the end of a line, last lines and last tiles float by float
+    (3, 2, 200, False, True), (1, 1, 70, False, True), (2, 1, 35, False, False), (61, 187, 425, True, False), (425, 64, 131, False, True),
+    (131, 66, 34, False, True), (129, 255, 99, False, False), (3101, 3077, 517, True, False), (3077, 3101, 541, False, True),
+    (3102, 3079, 515, False, False),
 ])
 def test_matrix_product_is_as_exact_as_fp32_sums(m, n, k, tA, tB):
     """The operands are multiplied as three bf16 parts each: what the six part products leave out is below 2^-25 of
     |a||b| per term, and every sum is fp32, so the bound of a plain fp32 product holds: (k + 2) * 2^-24 * |A||B|."""
     import torch
     g = torch.Generator(device="cuda").manual_seed(m + 7 * n + 31 * k)
-    A = torch.randn(m * k, device="cuda", generator=g) * torch.exp2(
-        torch.randint(-20, 20, (m * k,), device="cuda", generator=g).float())
+    A = torch.randn(m * k + 1, device="cuda", generator=g) * torch.exp2(
+        torch.randint(-20, 20, (m * k + 1,), device="cuda", generator=g).float())
+    A = A[1:] if k % 2 else A[:-1]  # odd cases: an operand aligned to 4 bytes only
     B = torch.randn(n * k, device="cuda", generator=g)
     C, A64, B64 = _product(m, n, k, tA, tB, A, B)
     bound = (k + 2) * 2.0 ** -24 * (A64.abs() @ B64.abs())
