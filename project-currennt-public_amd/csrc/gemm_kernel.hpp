@@ -308,6 +308,13 @@ struct FastStage {
         }
     }
     __device__ __forceinline__ void store(uint4 *__restrict__ lds, int tid) const { L::put(lds, tid, r); }
+    // adds the tile in registers to the sums of the thread's four rows (row-contiguous operands)
+    __device__ __forceinline__ void add_rows(float (&sum)[4]) const {
+#pragma unroll
+        for (int p = 0; p < NLOAD; ++p) {
+            sum[0] += r[p].x; sum[1] += r[p].y; sum[2] += r[p].z; sum[3] += r[p].w;
+        }
+    }
 };
 
 // The unmasked loader for row-contiguous operands whose k lines are picked through a list (16-byte vectors only): tile k
@@ -344,6 +351,13 @@ struct GatherStage {
             L::put(lds, tid, v);
         } else {
             L::put(lds, tid, r);
+        }
+    }
+    __device__ __forceinline__ void add_rows(float (&sum)[4]) const {
+#pragma unroll
+        for (int p = 0; p < NLOAD; ++p) {
+            const float4 v = kk + p < k_valid ? r[p] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+            sum[0] += v.x; sum[1] += v.y; sum[2] += v.z; sum[3] += v.w;
         }
     }
 };
@@ -450,12 +464,11 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 ? 3 : 2) : V
 
     const char *mask_pat = MASKED ? args.pat : nullptr;
 
-    // sum of the B operand over this split's k range, per row (dense bias gradient); the waves that keep it run a loop
-    // of their own, and only the operand kinds of a weight gradient have one
-    const bool rowsum = !AK && !BK_ && !MASKED && args.rowsum != 0 && wm == 0 && m0 == 0;
-    float rs[NB];
-#pragma unroll
-    for (int j = 0; j < NB; ++j) rs[j] = 0.0f;
+    // sum of the B operand over this split's k range, per row (dense bias gradient), by the workgroups of the first row of
+    // tiles: taken from the fp32 values on their way to LDS, because an infinite value cannot be put together again from its
+    // parts.  Those workgroups run a loop of their own, and only the operand kinds of a weight gradient have one.
+    const bool rowsum = !AK && !BK_ && !MASKED && args.rowsum != 0 && m0 == 0;
+    float rs[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // the rows of one of the thread's vectors, over the k positions it loads
 
     const int frag_row = lane & 31;
     const int half = lane >> 5;
@@ -466,6 +479,7 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 ? 3 : 2) : V
     auto loop = [&](auto &ra, auto &rb, auto &fetch_next, auto sums) __attribute__((always_inline)) {
         fetch_next(ra, rb);
         for (int it = it_begin; it < it_end; ++it) {
+            if constexpr (decltype(sums)::value) rb.add_rows(rs);
             ra.store(lds_a, tid);
             rb.store(lds_b, tid);
             fetch_next(ra, rb);
@@ -486,12 +500,6 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 ? 3 : 2) : V
 #pragma unroll
                         for (int j = 0; j < NB; ++j)
                             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j][QB[t]], fa[i][QA[t]], acc[i][j], 0, 0, 0);
-                if constexpr (decltype(sums)::value) {
-#pragma unroll
-                    for (int j = 0; j < NB; ++j)
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) rs[j] += ((float)fb[j][2][e] + (float)fb[j][1][e]) + (float)fb[j][0][e];
-                }
             }
             lds_only_barrier();
         }
@@ -623,14 +631,21 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 ? 3 : 2) : V
                 }
             }
         }
-        if (rowsum) {
-            float *__restrict__ R = args.partial + (size_t)split_id * args.partial_stride +
-                                    (size_t)args.nprob * args.m * args.n + (size_t)prob_id * args.n;
+        if constexpr (!AK && !BK_ && !MASKED) {
+            if (!rowsum) return;
+            // the threads that loaded different k positions of the same rows add up through LDS, in a fixed order
+            constexpr int PARTS = BK / LB::NLOAD;
+            static_assert(PARTS * BN * sizeof(float) <= sizeof(lds), "the row sums fit the tile's buffer");
+            float *const sums = reinterpret_cast<float *>(lds);
+            __syncthreads();
+            *reinterpret_cast<float4 *>(sums + LB::first_k(tid) / LB::NLOAD * BN + LB::first_row(tid)) = float4{rs[0], rs[1], rs[2], rs[3]};
+            __syncthreads();
+            if (tid < BN && n0 + tid < args.n) {
+                float s = 0.0f;
 #pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                const float s = rs[j] + __shfl_xor(rs[j], 32);
-                const int n = n0 + wn * WT + j * 32 + frag_row;
-                if (half == 0 && n < args.n) R[n] = s;
+                for (int q = 0; q < PARTS; ++q) s += sums[q * BN + tid];
+                args.partial[(size_t)split_id * args.partial_stride + (size_t)args.nprob * args.m * args.n +
+                             (size_t)prob_id * args.n + n0 + tid] = s;
             }
         }
         return;

@@ -569,3 +569,29 @@ def test_matrix_product_of_infinite_huge_and_missing_values(m, n, k, tA, tB):
     finite = want.isfinite()
     scale = (k + 2) * 2.0 ** -24 * (torch.nan_to_num(A64, 0.0, 0.0, 0.0).abs() @ torch.nan_to_num(B64).abs())
     assert bool(((C - want).abs() <= scale)[finite].all())
+
+
+@pytest.mark.parametrize("static", [False, True])
+@pytest.mark.parametrize("P,D,N,bias", [(64, 128, 3000, 0.5), (30, 61, 997, 1.0), (256, 132, 2049, 0.25)])
+def test_bias_gradient_of_infinite_huge_and_missing_errors(P, D, N, bias, static):
+    """The bias gradients that a weight gradient's launch sums along are fp32 sums of the errors as they are: an infinite
+    error gives an infinite sum, one that rounds to an infinite bf16 value a finite one.  Bound of the finite sums: N terms,
+    each rounded once per addition, and the product with the bias value."""
+    import torch
+    capi = PC.pkg().capi
+    g = torch.Generator(device="cuda").manual_seed(P + D)
+    x, err = torch.randn(N, P, device="cuda", generator=g), torch.randn(N, D, device="cuda", generator=g)
+    err[N - 1, 1] = 3.402823e38
+    err[3, 2], err[N // 2, 2] = -3.4e38, 3.4e38
+    err[0, 5], err[7, D - 1] = float("inf"), -float("inf")
+    err[9, 8], err[10, 8] = float("inf"), -float("inf")
+    err[N // 3, 11] = float("nan")
+    dW = torch.full((P * D + D,), 3.0, device="cuda")
+    (capi.dense_backward_weights_static if static else capi.dense_backward_weights)(P, D, N, bias, x, err, dW)
+    got, want = dW[P * D:].double(), bias * err.double().sum(0)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isposinf(), want.isposinf()) and torch.equal(got.isneginf(), want.isneginf())
+    finite = want.isfinite()
+    assert int((~finite).sum()) == 4
+    bound = (N + 2) * 2.0 ** -24 * bias * err.double().abs().sum(0)
+    assert bool(((got - want).abs() <= bound)[finite].all())
