@@ -13,7 +13,7 @@
 // |a||b|, less than the rounding of one fp32 product.  An instruction adds sixteen products before it rounds, where the fp32 one
 // adds two, so the result is closer to a 64-bit product than before: 2-norm error 4.9e-7 against 5.7e-7 at k = 1024, 1.2e-6
 // against 1.4e-6 at k = 6000, 1.6e-7 against 2.0e-7 at k = 128.  Values that are infinite, or round to an infinite bf16
-// value, leave infinity minus infinity in their parts; a sum that is not finite is formed again in plain fp32.
+// value, leave infinity minus infinity in their parts; a block of sums of which one is not finite is formed again on the fp32 instructions.
 //   1024 x 12000 x 1024: 283 -> 157 us (160 TFLOP/s), 512 x 6000 x 512: 40 -> 30 us, 1024 x 6000 x 512: 74 -> 57 us,
 //   1024 x 32000 x 128: 108 -> 73 us, 425 x 12000 x 1024: 141 -> 97 us, 300 x 10000 x 425: 47 -> 35 us.
 // Operands whose lines are no multiple of four long are read in vectors of four as well (FastStage); with one float per

@@ -362,29 +362,52 @@ struct GatherStage {
     }
 };
 
-// One element of the product over the k tiles [it_begin, it_end) in plain fp32, for the few that the split product cannot
-// form: an operand that is infinite or rounds to an infinite bf16 value leaves infinity minus infinity in its parts.
+// 32 x 32 sums of the product over the k tiles [it_begin, it_end), by one wave on the fp32 matrix instructions and straight
+// from memory, where the split product left sums that are not finite (an operand that is infinite or rounds to an infinite
+// bf16 value has infinity minus infinity in its parts).  Infinities and NaN come out as fp32 arithmetic has them.  A pass of a network
+// that has diverged is full of NaN, which stay what they are: the walk along k ends when all sums are.  1024 x 6000 x 1024,
+// usually 107 us: 107 us with NaN throughout, 756 with one at the end of every sum; one thread per sum took 11 400.
 template <bool AK, bool BK_, bool MASKED, bool GATHER>
-__device__ __forceinline__ float plain_element(const GemmArgs &args, const GemmProblem &pb, int m, int n, int it_begin,
-                                                         int it_end, int kt_per_seg, int k_extent, int k_lo) {
-    float sum = 0.0f;
+__device__ __forceinline__ f32x16 plain_sums(const GemmArgs &args, const GemmProblem &pb, int m0, int n0, int lane, int it_begin,
+                                             int it_end, int kt_per_seg, int k_extent, int k_lo) {
+    constexpr int AHEAD = 4;  // matrix instructions whose operands are in flight together
+    const int half = lane >> 5;
+    const int m = min(m0 + (lane & 31), args.m - 1), n = min(n0 + (lane & 31), args.n - 1);  // past an edge: sums that are not stored
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll 1
     for (int it = it_begin; it < it_end; ++it) {
         const int seg = it / kt_per_seg, k0 = (it % kt_per_seg) * BK, k1 = min(k0 + BK, k_extent);
-        for (int kk = k0; kk < k1; ++kk) {
-            const int k = GATHER ? args.k_order[k_lo + kk] + pb.k_shift : kk;
-            int bk = k, bn = n;
-            bool keep = true;
-            if (MASKED && args.pat) {
-                const int u = args.b_time_on_k ? k : n, src = u + pb.b_shift[seg];
-                keep = args.pat[u] != 0 && src >= 0 && src < args.n_slots && args.pat[src] != 0;
-                if (args.b_time_on_k) bk = src; else bn = src;
+#pragma unroll 1
+        for (int kk = k0; kk < k1; kk += 2 * AHEAD) {
+            float a[AHEAD], b[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                const int at = kk + 2 * u + half;
+                const bool on = at < k1;  // a lane without a k position takes the tile's first one, times zero
+                const int k = GATHER ? args.k_order[k_lo + (on ? at : k0)] + pb.k_shift : on ? at : k0;
+                int bk = k, bn = n;
+                bool keep = on;
+                if (MASKED && args.pat) {
+                    const int slot = args.b_time_on_k ? k : n, from = slot + pb.b_shift[seg], src = min(max(from, 0), args.n_slots - 1);
+                    keep = on && args.pat[slot] != 0 && src == from && args.pat[src] != 0;
+                    if (args.b_time_on_k) bk = src; else bn = src;
+                }
+                const float x = pb.A[seg][AK ? (size_t)m * args.lda + k : (size_t)k * args.lda + m];
+                const float y = pb.B[seg][BK_ ? (size_t)bn * args.ldb + bk : (size_t)bk * args.ldb + bn];
+                a[u] = on ? x : 0.0f;
+                b[u] = keep ? y : 0.0f;
             }
-            const float a = pb.A[seg][AK ? (size_t)m * args.lda + k : (size_t)k * args.lda + m];
-            const float b = keep ? pb.B[seg][BK_ ? (size_t)bn * args.ldb + bk : (size_t)bk * args.ldb + bn] : 0.0f;
-            sum = __builtin_fmaf(a, b, sum);
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(b[u], a[u], acc, 0, 0, 0);
         }
+        bool open = false;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) open = open || acc[r] == acc[r];
+        if (__builtin_amdgcn_ballot_w64(open) == 0) break;
     }
-    return sum;
+    return acc;
 }
 
 // VA, VB: vector widths of the masked loader, 16-byte alignment included; unmasked: 4 where the operand's lines are a
@@ -396,9 +419,11 @@ __device__ __forceinline__ float plain_element(const GemmArgs &args, const GemmP
 // the shapes of the error products that use it) so that its registers and code stay out of every other product.
 // GATHER: the k lines of both (row-contiguous, 16-byte aligned) operands are those a list names (GemmArgs::k_order).
 // The workgroups a compute unit is to hold (by registers; LDS allows as many) are what hides one's loads and conversions
-// behind another's matrix instructions.
+// behind another's matrix instructions.  128 x 128 tiles of two row-contiguous operands take 55 KB each, so two: where three were
+// asked for, the compiler held operands in accumulator registers and a small change made it miss two as well (the feed-forward
+// model 2213 -> 2293 us per pass).
 template <int VA, bool AK, int VB, bool BK_, bool MASKED, int TILE, bool FAN = false, bool GATHER = false>
-__global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 ? 3 : 2) : VA * VB == 16 ? 5 : 4) void gemm_split_kernel(const GemmArgs args) {
+__global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK_) ? 3 : 2) : VA * VB == 16 ? 5 : 4) void gemm_split_kernel(const GemmArgs args) {
     constexpr int BM = TILE, BN = TILE;
     constexpr int WT = TILE / 2;   // edge of a wave's block (waves are arranged 2 x 2)
     constexpr int NB = WT / 32;    // 32 x 32 MFMA tiles per wave and dimension
@@ -583,34 +608,18 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 ? 3 : 2) : V
         run(sa, sb, fetch_next);
     }
 
-    // what came out infinite or not a number is formed again (plain_element)
-    bool finite = true;
+    // what came out infinite or not a number is formed again (plain_sums)
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
-        for (int j = 0; j < NB; ++j)
+        for (int j = 0; j < NB; ++j) {
+            bool finite = true;
 #pragma unroll
             for (int r = 0; r < 16; ++r) finite = finite && __builtin_fabsf(acc[i][j][r]) <= lim::kMax;
-    if (__builtin_expect(!finite, 0)) {
-        // through LDS, where a rolled loop can index a thread's sums: this code is cold and should take no registers
-        static_assert(NB * 16 * NTHREADS * sizeof(float) <= sizeof(lds), "a row of accumulators fits the tile's buffer");
-        float *mine = reinterpret_cast<float *>(lds) + tid;
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-#pragma unroll
-            for (int e = 0; e < NB * 16; ++e) mine[e * NTHREADS] = acc[i][e / 16][e % 16];
-            const int m = m0 + wm * WT + i * 32 + frag_row;
-#pragma unroll 1
-            for (int e = 0; e < NB * 16; ++e) {
-                const int r = e % 16, n = n0 + wn * WT + (e / 16) * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-                if (!(__builtin_fabsf(mine[e * NTHREADS]) <= lim::kMax) && m < args.m && n < args.n)
-                    mine[e * NTHREADS] =
-                        plain_element<AK, BK_, MASKED, GATHER>(args, pb, m, n, it_begin, it_end, kt_per_seg, k_extent, k_lo);
-            }
-#pragma unroll
-            for (int e = 0; e < NB * 16; ++e) acc[i][e / 16][e % 16] = mine[e * NTHREADS];
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!finite) != 0, 0))
+                acc[i][j] = plain_sums<AK, BK_, MASKED, GATHER>(args, pb, m0 + wm * WT + 32 * i, n0 + wn * WT + 32 * j, lane, it_begin,
+                                                                it_end, kt_per_seg, k_extent, k_lo);
         }
-    }
 
     // epilogue: lane%32 runs along m (contiguous), the 16 accumulators along n
     float *__restrict__ C = pb.C;

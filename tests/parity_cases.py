@@ -57,7 +57,7 @@ def lstm_inputs(P, L, bidir, S, T, lengths, seed, wscale=0.1, escale=0.1):
 
 
 def run_lstm_case(P, L, bidir, lengths, seed, wscale=0.1, escale=0.1, bias=1.0, repeat_backward=False,
-                  tol=1e-4, verbose=False):
+                  tol=1e-4, verbose=False, huge=False):
     import torch
 
     capi = pkg().capi
@@ -66,6 +66,8 @@ def run_lstm_case(P, L, bidir, lengths, seed, wscale=0.1, escale=0.1, bias=1.0, 
     H = L // nd
     N = T * S
     W, x, outerr = lstm_inputs(P, L, bidir, S, T, lengths, seed, wscale, escale)
+    if huge:  # one input that rounds to an infinite bf16 value
+        x.reshape(T, S, P)[T // 4, 0, 3] = 3.402823e38
     pat = make_pat_types(lengths, T)
 
     # ---- oracle
@@ -408,7 +410,7 @@ def run_sigmoid_case(lengths, K, extra, continuous, seed, with_softmax=False):
     return worst
 
 
-def run_cnn_case(P, half_width, interval, lengths, causal, out_tanh, seed, bias=1.0, maxT=None):
+def run_cnn_case(P, half_width, interval, lengths, causal, out_tanh, seed, bias=1.0, maxT=None, huge=False):
     """1-D convolution layer forward + backward against the oracle (which scatters into a real column buffer)."""
     import torch
 
@@ -424,6 +426,9 @@ def run_cnn_case(P, half_width, interval, lengths, causal, out_tanh, seed, bias=
     W = rng.uniform(-0.1, 0.1, P * Lw + D).astype(np.float32)
     x = rng.standard_normal((T, S, P)).astype(np.float32)
     err = rng.standard_normal((T, S, D)).astype(np.float32)
+    if huge:  # inputs that round to an infinite bf16 value; their products with weights and errors stay finite
+        x[T // 3, 0, P - 1], x[0, S - 1, 0] = 3.402823e38, -3.402823e38
+        err *= 0.01
     pat = make_pat_types(lengths, T)
     stale = rng.standard_normal(D * N).astype(np.float32)  # outputs keep their old content on padding slots
     con = np.zeros(Lw * N, dtype=np.float32)

@@ -571,6 +571,56 @@ def test_matrix_product_of_infinite_huge_and_missing_values(m, n, k, tA, tB):
     assert bool(((C - want).abs() <= scale)[finite].all())
 
 
+# every orientation, row of tiles and vector width; k a multiple of the staged depth, one more, and one tile only
+@pytest.mark.parametrize("m,n,k,tA,tB", [(33, 64, 32, True, False), (64, 31, 65, False, True), (130, 96, 96, False, False),
+                                         (61, 67, 7, True, False), (3077, 3101, 513, False, True), (3100, 3076, 544, True, False)])
+def test_matrix_product_next_to_infinite_and_missing_values(m, n, k, tA, tB):
+    """The sums around one that is not finite are formed again with it: they keep the bound of fp32 sums, whichever the
+    operands' orientation, and so do those of the rows and columns at the edges."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    A, B = torch.randn(m * k, device="cuda", generator=g), torch.randn(n * k, device="cuda", generator=g)
+    (A.view(m, k) if tA else A.view(k, m).t())[m - 1, k - 1] = float("nan")
+    (B.view(k, n) if tB else B.view(n, k).t())[0, n - 1] = float("inf")
+    C, A64, B64 = _product(m, n, k, tA, tB, A, B)
+    assert bool(C[m - 1].isnan().all()) and bool((~C[:m - 1, n - 1].isfinite()).all())
+    A64, B64 = torch.nan_to_num(A64, 0.0), torch.nan_to_num(B64, posinf=0.0)
+    bound = (k + 2) * 2.0 ** -24 * (A64.abs() @ B64.abs())
+    assert bool(((C - A64 @ B64).abs() <= bound)[:m - 1, :n - 1].all())
+
+
+@pytest.mark.parametrize("everywhere,times", [(True, 4), (False, 20)])
+def test_products_full_of_missing_values_stay_in_the_range_of_others(everywhere, times):
+    """A pass of a network that has diverged is full of NaN; it takes about as long as another, and some times as long, not
+    a hundred, where each sum meets its only NaN at the end (1.0 and 7 measured)."""
+    import torch
+    m, n, k = 1024, 6000, 1024
+    A, B = torch.randn(m * k, device="cuda"), torch.randn(n * k, device="cuda")
+    C = torch.empty(m * n, device="cuda")
+
+    def best():
+        spans = []
+        for _ in range(4):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            PC.pkg().capi.matrix_product(C, m, n, k, A, True, B, False, False)
+            end.record()
+            torch.cuda.synchronize()
+            spans.append(begin.elapsed_time(end))
+        return min(spans)
+
+    usual = best()
+    A.view(m, k)[:, 0 if everywhere else k - 1:] = float("nan")
+    missing = best()
+    print("usual %.3f ms, NaN %.3f ms" % (usual, missing), flush=True)
+    assert bool(C.isnan().all()) and missing < times * usual
+
+
+def test_lstm_with_a_huge_input_and_much_padding():
+    """The product over the listed slots of a fraction (much padding, enough slots) with a value that has no finite parts."""
+    assert PC.run_lstm_case(60, 64, True, [260, 100] * 4, seed=6, huge=True) < TOL
+
+
 @pytest.mark.parametrize("static", [False, True])
 @pytest.mark.parametrize("P,D,N,bias", [(64, 128, 3000, 0.5), (30, 61, 997, 1.0), (256, 132, 2049, 0.25)])
 def test_bias_gradient_of_infinite_huge_and_missing_errors(P, D, N, bias, static):

@@ -25,6 +25,14 @@ def test_cnn_layer(P, hw, it, lengths, causal, tanh):
     assert PC.run_cnn_case(P, hw, it, lengths, causal, tanh, seed=P + len(hw)) < TOL
 
 
+@pytest.mark.parametrize("P,hw,it,lengths,causal", [
+    (5, [1] * 6, [4] * 6, [17, 9, 14], 1), (64, [1] * 128, [2] * 128, [150, 120], 1), (6, [0] * 30, [1] * 30, [200, 90], 0),
+])
+def test_cnn_layer_of_huge_inputs(P, hw, it, lengths, causal):
+    """Masked products (taps that read other slots, slots that do not count) of values that have no finite bf16 parts."""
+    assert PC.run_cnn_case(P, hw, it, lengths, causal, 0, seed=P, huge=True) < TOL
+
+
 def test_cnn_layer_short_fraction_clears_tail():
     print("cnn short fraction", flush=True)
     assert PC.run_cnn_case(6, [1] * 4, [2] * 4, [9, 5], 1, 1, seed=9, bias=0.5, maxT=15) < TOL
