@@ -7,15 +7,19 @@
 // long-K weight-gradient shapes, and a fused bias + activation epilogue for the dense forward.
 //
 // Arithmetic: the fp32 matrix instructions end at 157 TFLOP/s and reached 88 here, with the matrix units 56% busy.  Every
-// operand value is therefore split into three bf16 parts, x = h + m + l exactly (round to nearest, so m <= 2^-9 |x| and
-// l <= 2^-18 |x|), and a product is the sum of the six part products h*h, h*m, m*h, m*m, h*l, l*h, which the bf16
+// operand value is therefore split into three bf16 parts, 2^16 x = h + m + l (round to nearest, so m <= 2^-9 of it and
+// l <= 2^-18), and a product is the sum of the six part products h*h, h*m, m*h, m*m, h*l, l*h, which the bf16
 // instructions form exactly and add in fp32, the small ones first.  What is left out (m*l, l*m, l*l) is below 2^-25 of
 // |a||b|, less than the rounding of one fp32 product.  An instruction adds sixteen products before it rounds, where the fp32 one
 // adds two, so the result is closer to a 64-bit product than before: 2-norm error 4.9e-7 against 5.7e-7 at k = 1024, 1.2e-6
-// against 1.4e-6 at k = 6000, 1.6e-7 against 2.0e-7 at k = 128.  Values that are infinite, or round to an infinite bf16
-// value, leave infinity minus infinity in their parts; a block of sums of which one is not finite is formed again on the fp32 instructions.
-//   1024 x 12000 x 1024: 283 -> 157 us (160 TFLOP/s), 512 x 6000 x 512: 40 -> 30 us, 1024 x 6000 x 512: 74 -> 57 us,
-//   1024 x 32000 x 128: 108 -> 73 us, 425 x 12000 x 1024: 141 -> 97 us, 300 x 10000 x 425: 47 -> 35 us.
+// against 1.4e-6 at k = 6000, 1.6e-7 against 2.0e-7 at k = 128.
+// Range: the split is exact for every fp32 value below 2^112, subnormal ones included, which is what the factor 2^16 is for
+// (without it values below 2^-110 lose their low parts, and products of values around 2^-126 were off by 2^-9); it costs a
+// multiplication per operand value and load, 1-3% of a product's time.  Operands from 2^112 on, infinite ones and sums
+// from 2^96 on leave infinities or infinity minus infinity behind; a block of sums of which one is not finite is formed again on
+// the fp32 instructions (plain_sums).
+//   1024 x 12000 x 1024: 283 -> 140 us (180 TFLOP/s), 512 x 6000 x 512: 40 -> 29 us, 1024 x 6000 x 512: 74 -> 51 us,
+//   1024 x 32000 x 128: 108 -> 73 us, 425 x 12000 x 1024: 141 -> 96 us, 300 x 10000 x 425: 47 -> 34 us.
 // Operands whose lines are no multiple of four long are read in vectors of four as well (FastStage); with one float per
 // lane and load the last two sizes took 100 and 43 us.
 // What bounds it now, at the first size per SIMD: 69 us of matrix instructions, 38 us of conversions, 51 us of LDS traffic,

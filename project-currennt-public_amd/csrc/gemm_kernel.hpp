@@ -33,12 +33,17 @@ struct VecT<2> { typedef float2 type; };
 template <>
 struct VecT<4> { typedef float4 type; };
 
-// Two fp32 values as three bf16 pairs (the lower half of a word belongs to x0): x = h + m + l exactly, each part the
-// nearest bf16 value to what the parts before it leave (8 + 8 + 8 bits of significand hold the 24 of x).
+// Two fp32 values as three bf16 pairs (the lower half of a word belongs to x0): kSplitScale * x = h + m + l exactly, each part
+// the nearest bf16 value to what the parts before it leave (8 + 8 + 8 bits of significand hold the 24 of x).  bf16 ends at
+// 2^-133, fp32 at 2^-149: without the factor the low parts of values below 2^-110 are cut off, and one near 2^-126 keeps eight
+// bits.  With it the parts of every fp32 value below 2^112 are exact, and sums up to 2^96 come out finite; those above are
+// formed again (plain_sums).
+constexpr float kSplitScale = 65536.0f;
 __device__ __forceinline__ unsigned nearest_bf16(float x0, float x1) {
     return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x0, x1}), bf16x2));
 }
 __device__ __forceinline__ void split_pair(float x0, float x1, unsigned (&part)[3]) {
+    x0 *= kSplitScale; x1 *= kSplitScale;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
         part[q] = nearest_bf16(x0, x1);
@@ -616,6 +621,8 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
             bool finite = true;
 #pragma unroll
             for (int r = 0; r < 16; ++r) finite = finite && __builtin_fabsf(acc[i][j][r]) <= lim::kMax;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] *= 1.0f / (kSplitScale * kSplitScale);
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(!finite) != 0, 0))
                 acc[i][j] = plain_sums<AK, BK_, MASKED, GATHER>(args, pb, m0 + wm * WT + 32 * i, n0 + wn * WT + 32 * j, lane, it_begin,
                                                                 it_end, kt_per_seg, k_extent, k_lo);

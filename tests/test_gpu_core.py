@@ -621,6 +621,22 @@ def test_lstm_with_a_huge_input_and_much_padding():
     assert PC.run_lstm_case(60, 64, True, [260, 100] * 4, seed=6, huge=True) < TOL
 
 
+@pytest.mark.parametrize("ea,eb", [(-108, 0), (-118, 40), (-126, 40), (-140, 60), (30, -126), (-66, -66), (-115, 110), (95, 0), (110, -20),
+                                   (50, 46), (50, 50)])
+@pytest.mark.parametrize("m,n,k,tA,tB", [(130, 66, 300, True, False), (67, 129, 65, False, True)])
+def test_matrix_product_over_the_range_of_fp32(m, n, k, tA, tB, ea, eb):
+    """Operands whose parts would fall below the smallest bf16 value, subnormal ones, and sums around the limit above which
+    they are formed again: the bound of fp32 sums holds, plus half of the smallest fp32 value for the rounding of a subnormal
+    result and as much for every term."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(k)
+    A = (torch.randn(m * k, device="cuda", generator=g).double() * 2.0 ** ea).float()
+    B = (torch.randn(n * k, device="cuda", generator=g).double() * 2.0 ** eb).float()
+    C, A64, B64 = _product(m, n, k, tA, tB, A, B)
+    bound = (k + 2) * 2.0 ** -24 * (A64.abs() @ B64.abs()) + (k + 1) * 2.0 ** -150
+    assert bool(((C - A64 @ B64).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("static", [False, True])
 @pytest.mark.parametrize("P,D,N,bias", [(64, 128, 3000, 0.5), (30, 61, 997, 1.0), (256, 132, 2049, 0.25)])
 def test_bias_gradient_of_infinite_huge_and_missing_errors(P, D, N, bias, static):
