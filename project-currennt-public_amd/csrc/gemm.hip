@@ -280,6 +280,7 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
                 args.nseg, kGemmMaxSeg);
     CNT_REQUIRE(args.nprob >= 1 && args.nprob <= kGemmMaxProb, "gemm: %d problems, supported 1..%d",
                 args.nprob, kGemmMaxProb);
+    CNT_REQUIRE(!args.a_kcontig || args.b_kcontig, "gemm: a k-contiguous A with a row-contiguous B is not supported");
     CNT_REQUIRE(args.splitk >= 0 && (args.splitk == 1 || args.epilogue == EPI_ATOMIC || args.epilogue == EPI_PARTIAL),
                 "gemm: split-K needs the atomic epilogue");
     CNT_REQUIRE(args.epilogue != EPI_STORE_DELTA || (args.splitk == 1 && args.prob[0].aux_in != nullptr),

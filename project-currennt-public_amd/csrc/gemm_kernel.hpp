@@ -165,6 +165,12 @@ struct TileStage {
     __device__ __forceinline__ void load(const float *__restrict__ base, int ld, int row0, int k0,
                                          int rows_total, int k_total, int tid, const char *__restrict__ pat = nullptr,
                                          int shift = 0, int n_slots = 0, bool time_on_k = false) {
+        // Addresses are formed here, tile by tile, where keeping them through the loop would push the data or the pattern bytes out
+        // of the registers (the kernels for sizes that are no multiple of four spilled 2 to 27 of them): 63 -> 126 channels over 2 x 8000
+        // slots 22.1 -> 19.4 us forward, 31 -> 62 over 16 000 14.3 -> 12.5, 63 -> 128 over 2 x 16 000 30.4 -> 26.0.  A bound of three
+        // workgroups per compute unit instead of four gave the first two and took 28.0 instead of 22.1 for 62 -> 124 over 2 x 16 000.
+        if (KCONTIG && VEC < 4 && pat) asm volatile("" : "+s"(ld));
+        if (!KCONTIG && pat) asm volatile("" : "+s"(row0));
         if (KCONTIG) {
             const int kq = L::first_k(tid);
 #pragma unroll
@@ -773,7 +779,7 @@ void launch_t(const GemmArgs &a, dim3 grid, hipStream_t s, int tile) {
 template <int VA, bool AK, int VB>
 void launch_b(const GemmArgs &a, dim3 grid, hipStream_t s, bool bk, int tile) {
     if (bk) launch_t<VA, AK, VB, true>(a, grid, s, tile);
-    else launch_t<VA, AK, VB, false>(a, grid, s, tile);
+    else if constexpr (!AK) launch_t<VA, AK, VB, false>(a, grid, s, tile);  // (no product has a k-contiguous A and a row-contiguous B)
 }
 template <int VA, bool AK>
 void launch_vb(const GemmArgs &a, dim3 grid, hipStream_t s, int vb, bool bk, int tile) {
