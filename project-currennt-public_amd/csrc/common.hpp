@@ -53,40 +53,38 @@ constexpr float kMinLarg = 1.1754944e-038f;
 constexpr float kMinLogExp = -69.0776f;
 }  // namespace lim
 
-// 1 / (1 + exp(m)), m * log2(e) given as the sum of m * hi and m * lo: exp2 of the hardware over [-1/2, 1/2], the integer
+// 1 / (1 + exp(m)), m * log2(e) given as the sum of m * hi and m * lo (argument reduction by log2(e) as a float and its
+// remainder, one Newton step for the quotient): exp2 of the hardware over [-1/2, 1/2], the integer
 // part (the low bits of t, which has 1.5 * 2^23 added) put into the exponent, and a reciprocal with one Newton step that
-// also takes in what 1 + e rounds away: fourteen instructions with the clamp.  expf and an fp32 quotient take about forty
-// (denormal results, exact rounding).  Against double precision over every fifth float between 3e-8 and 87 of both signs: largest
-// error 2.62 ulp (expf and quotient: 2.62), root mean square 0.34 (0.56); of tanh_act 0.94e-7 absolute (1.79e-7).  Without the
-// rest of the sum the largest error was 0.03 ulp more than the quotient's, and no pass was faster.  The callers clamp m * log2(e) to
+// also takes in what 1 + e rounds away (REST): fourteen instructions with the clamp, eleven without REST.  expf and an fp32
+// quotient take about forty (denormal results, exact rounding).  Against double precision over every float between 3e-8 and 87 of
+// both signs: largest error 2.62 ulp with REST and without it (expf and quotient: 2.62), root mean square 0.34 and 0.56 (0.56); of
+// the tanh functions 0.97e-7 and 1.79e-7 absolute (1.79e-7).  The callers clamp m * log2(e) to
 // [-126, 128), which needs no branch and no select: a NaN becomes the lower limit, which gives 1 as it always did.
 // Results below 1.2e-38 are zero.
+template <bool REST>
 __device__ __forceinline__ float logistic_of_negative(float m, float hi, float lo) {
     const float t = __builtin_fmaf(m, hi, 12582912.0f);
     const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(m, lo, __builtin_fmaf(m, hi, -(t - 12582912.0f))));
     const float e = __uint_as_float(__float_as_uint(p) + (__float_as_uint(t) << 23));
     const float d = 1.0f + e, rest = e - (d - 1.0f);  // 1 + e = d + rest
-    const float y = __builtin_amdgcn_rcpf(d);
-    return __builtin_fmaf(__builtin_fmaf(-rest, y, __builtin_fmaf(-d, y, 1.0f)), y, y);
+    const float y = __builtin_amdgcn_rcpf(d), left = __builtin_fmaf(-d, y, 1.0f);
+    return __builtin_fmaf(REST ? __builtin_fmaf(-rest, y, left) : left, y, y);
 }
+template <bool REST = true>
 __device__ __forceinline__ float logistic(float x) {
-    return logistic_of_negative(__builtin_amdgcn_fmed3f(-x, -87.3f, 88.72283f), 1.44269504088896341f, 1.92596303e-8f);
+    return logistic_of_negative<REST>(__builtin_amdgcn_fmed3f(-x, -87.3f, 88.72283f), 1.44269504088896341f, 1.92596303e-8f);
 }
-// The same functions from the hardware's exp2 and reciprocal alone, for the forward recursion, where the five of them per cell
-// and time step sit on the critical path of every step.  Not bit-identical to the functions above: exp2 and rcp are
-// good to 1 ulp each, but the argument -1.4427 * x is rounded to fp32 before the exponential, which alone is a
-// relative error of |x| * 6e-8 in exp(-x).  The result stays within 4e-6 absolute of the exact logistic function
-// (8e-6 for tanh) over the whole unclamped range, which tests/test_gpu_core.py checks against the CPU functions.
-__device__ __forceinline__ float logistic_quick(float x) {
-    float y = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * x));
-    y = x > -lim::kExpLimit ? y : 0.0f;
-    return x < lim::kExpLimit ? y : 1.0f;
-}
-__device__ __forceinline__ float tanh_quick(float x) { return 2.0f * logistic_quick(2.0f * x) - 1.0f; }
-__device__ __forceinline__ float logistic_deriv(float y) { return y * (1.0f - y); }
+template <bool REST = true>
 __device__ __forceinline__ float tanh_act(float x) {
-    return 2.0f * logistic_of_negative(__builtin_amdgcn_fmed3f(-x, -43.65f, 44.361415f), 2.88539008177792681f, 3.85192606e-8f) - 1.0f;
+    return 2.0f * logistic_of_negative<REST>(__builtin_amdgcn_fmed3f(-x, -43.65f, 44.361415f), 2.88539008177792681f, 3.85192606e-8f) - 1.0f;
 }
+// The same functions in the form of eleven instructions, for the forward recursion, where the five of them per cell and time step
+// sit on the critical path of every step: an utterance of 800 steps through two layers of 512 cells 2074 us (2115 with REST), a
+// pass of the acoustic model 3790 us (3787).
+__device__ __forceinline__ float logistic_quick(float x) { return logistic<false>(x); }
+__device__ __forceinline__ float tanh_quick(float x) { return tanh_act<false>(x); }
+__device__ __forceinline__ float logistic_deriv(float y) { return y * (1.0f - y); }
 __device__ __forceinline__ float tanh_deriv(float y) { return 1.0f - y * y; }
 __device__ __forceinline__ float clip1(float e) { return e < -1.0f ? -1.0f : (e > 1.0f ? 1.0f : e); }
 __device__ __forceinline__ float safe_exp(float x) {
