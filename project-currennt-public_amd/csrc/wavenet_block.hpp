@@ -163,6 +163,8 @@ __global__ __launch_bounds__(R * 4, 2) void wavenet_block_forward_kernel(const B
     // ---- convolution, conditioning projection and gate, one step of sixteen samples after the other.  The gate of a
     // step is evaluated between the matrix instructions of the next one's convolution: seven vector instructions fit
     // into the 32 cycles that one of those takes.
+    // (without conditioning features `cond` has no words: what is read, and not used, then comes from the block's input)
+    const f32x4 *const features = cj > 0 ? cond : now;
     f32x4 c0, c1, t0, t1;  // convolution and conditioning sums of the step, both halves
     auto gate = [&](int s, f32x4 p, f32x4 q, f32x4 tp, f32x4 tq) {
         const unsigned at = 4 * ((16 * s + col) * 2 * R + own);
@@ -205,7 +207,7 @@ __global__ __launch_bounds__(R * 4, 2) void wavenet_block_forward_kernel(const B
 #pragma unroll
             for (int j = 0; j < RJ; ++j) b[tap][j] = (tap == 0 ? earlier : now)[(4 * j + quarter) * ROW + 16 * s + col];
 #pragma unroll
-        for (int j = 0; j < CJ; ++j) x[j] = cond[(4 * min(j, max(cj - 1, 0)) + quarter) * ROW + 16 * s + col];
+        for (int j = 0; j < CJ; ++j) x[j] = features[(4 * min(j, max(cj - 1, 0)) + quarter) * ROW + 16 * s + col];
         c0 = f32x4{0, 0, 0, 0};
         c1 = f32x4{0, 0, 0, 0};
 #pragma unroll

@@ -483,10 +483,11 @@ class _CondOracleBackend(OM.OracleBackend):
 
 
 # one launch per residual block: tiles of 16, 32 and 64 samples with a ragged last one, conditioning rows that end inside
-# a 16-byte piece or start off a 16-byte boundary, fewer skip than residual channels, the widest conditioning
+# a 16-byte piece or start off a 16-byte boundary, fewer skip than residual channels, the widest conditioning, none
 @pytest.mark.parametrize("cnn_tanh,R,K,C,lengths", [
     (1, 32, 32, 4, [1]), (1, 64, 32, 7, [40, 33, 1]), (0, 48, 96, 45, [70, 51]), (1, 48, 256, 112, [17]), (1, 64, 80, 81, [2050, 1999]),
     (1, 32, 64, 20, [12300, 12295]), (1, 64, 128, 100, [8200, 7000, 8199]),
+    (1, 32, 32, 0, [40, 33]), (0, 48, 16, 0, [16]), (1, 64, 128, 0, [2200, 2001]),
 ])
 def test_wavenet_block_forward_edges(cnn_tanh, R, K, C, lengths):
     import torch
@@ -495,13 +496,15 @@ def test_wavenet_block_forward_edges(cnn_tanh, R, K, C, lengths):
     capi, networks = PC.pkg().capi, PC.networks()
     O.use_all_cores()
     nb, Q, S, T = 2, 32, len(lengths), max(lengths)
-    pat, _, ctx, target, N = WD.make(lengths, Q, C, upsample=5, seed=7)
+    pat, _, ctx, target, N = WD.make(lengths, Q, C or 4, upsample=5, seed=7)
     onehot = np.zeros((N, Q), np.float32)  # the feedback layer's: also in the first padding slot behind a sequence
     follows = np.flatnonzero(pat[: N - S] != 0)
     onehot[follows + S, np.asarray(target).reshape(-1)[follows].astype(int)] = 1
-    ref = networks.WaveNet(OM.OracleBackend(), nb, S, T, Q=Q, R=R, K=K, C=C, cnn_tanh=cnn_tanh, dilation_cycle=10)
+    ref = networks.WaveNet(OM.OracleBackend(), nb, S, T, Q=Q, R=R, K=K, C=C or 4, cnn_tanh=cnn_tanh, dilation_cycle=10)
     W = WD.init_weights({k: len(ref.buf[k]["W"]) for k in ref.weight_names()}, seed=3)
     for k, w in W.items():
+        if not C and k.startswith("wav"):
+            w[:] = 0  # a layer without conditioning features is one whose features count nothing
         ref.buf[k]["W"][:] = w
     ref.set_inputs(pat, onehot.reshape(-1), ctx, target)
     ref.forward()
@@ -510,7 +513,8 @@ def test_wavenet_block_forward_edges(cnn_tanh, R, K, C, lengths):
         if L["weight_count"]:
             L["weights"].copy_(torch.from_numpy(W[L["name"]]))
     ctx_d = PC.dev(ctx)
-    net.set_context(ctx_d)
+    if C:
+        net.set_context(ctx_d)
     net.load_sequences(PC.dev(pat), T, min(lengths), torch.zeros(N, dtype=torch.float32, device="cuda"), PC.dev(target))
     for layer in net.layers:
         if layer["type"] == "cnn":
