@@ -25,14 +25,15 @@
 #include <cerrno>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <limits>
 #include <memory>
 #include <mutex>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include <fcntl.h>
@@ -243,7 +244,8 @@ void swapped_copy(unsigned *dst, const unsigned *src, size_t n) {
 
 // Threads that help the caller through a list of independent pieces of work; they are started by the first list and joined
 // with the pool.  The caller works through the list itself and waits only for helpers that have taken a piece, so a list
-// also ends where no helper is left (a forked child) or none could be started.
+// also ends where no helper is left (a forked child) or none could be started.  A piece that throws, on whichever thread, ends
+// the list; the caller gets the exception when no helper is at work any more.
 class Helpers {
     std::mutex m, busy;
     std::condition_variable wake, idle;
@@ -255,9 +257,16 @@ class Helpers {
     int active = 0;
     bool stop = false;
     pid_t owner = 0;
+    std::exception_ptr failed;
 
-    static void work(const std::function<void(size_t)> &f, std::atomic<size_t> &next, size_t count) {
-        for (size_t i; (i = next.fetch_add(1, std::memory_order_relaxed)) < count;) f(i);
+    void work(const std::function<void(size_t)> &f, size_t n) noexcept {
+        try {
+            for (size_t i; (i = next.fetch_add(1, std::memory_order_relaxed)) < n;) f(i);
+        } catch (...) {
+            next.store(n, std::memory_order_relaxed);  // (a counter past n ends the others' loops as well)
+            std::lock_guard<std::mutex> lock(m);
+            if (!failed) failed = std::current_exception();
+        }
     }
     void help() {
         unsigned seen = 0;
@@ -270,7 +279,7 @@ class Helpers {
             const size_t n = count;
             ++active;
             lock.unlock();
-            work(f, next, n);
+            work(f, n);
             lock.lock();
             if (--active == 0) idle.notify_one();
         }
@@ -293,7 +302,7 @@ public:
             owner = getpid();
             try {
                 for (int k = helpers_wanted(); k > 0; --k) threads.emplace_back([this] { help(); });
-            } catch (const std::system_error &) {
+            } catch (const std::exception &) {
             }  // fewer helpers then
         }
         {
@@ -301,10 +310,11 @@ public:
             next = 0; count = n; job = &f; ++generation;
         }
         wake.notify_all();
-        work(f, next, n);
+        work(f, n);
         std::unique_lock<std::mutex> lock(m);
         job = nullptr;
         idle.wait(lock, [&] { return active == 0; });
+        if (failed) std::rethrow_exception(std::exchange(failed, nullptr));
     }
     // false in a forked child, which has the objects but not the threads: nothing there may be waited for or destroyed
     bool owned() const { return owner == 0 || owner == getpid(); }
@@ -350,20 +360,34 @@ int dataset_error(cnt_dataset *d, const std::string &what) {
     return CNT_ERR_ARG;
 }
 
+// what an exception becomes at the C interface; in the handlers of the calls that allocate
+int exception_error(const char *call) noexcept {
+    try {
+        throw;
+    } catch (const std::bad_alloc &) {
+        cnt::set_error("%s: out of host memory", call);
+    } catch (const std::exception &e) {
+        cnt::set_error("%s: %s", call, e.what());
+    } catch (...) {
+        cnt::set_error("%s: unknown error", call);
+    }
+    return CNT_ERR_ARG;
+}
+
 }  // namespace
 
 extern "C" {
 
-int cnt_dataset_open(const char *nc_path, const cnt_dataset_desc *desc, cnt_dataset **out) {
+int cnt_dataset_open(const char *nc_path, const cnt_dataset_desc *desc, cnt_dataset **out) try {
     using namespace cnt;
     CNT_REQUIRE(nc_path && desc && out, "dataset_open: null argument");
     CNT_REQUIRE(desc->parallel_sequences >= 1, "dataset_open: parallel_sequences must be positive");
     // the reference's check (data_sets/DataSet.cpp:1322-1323)
     CNT_REQUIRE(desc->fraction > 0 && desc->fraction <= 1, "Invalid fraction");
-    cnt_dataset *d = new (std::nothrow) cnt_dataset();
-    CNT_REQUIRE(d != nullptr, "dataset_open: out of host memory");
+    std::unique_ptr<cnt_dataset> owned(new cnt_dataset());
+    cnt_dataset *const d = owned.get();
     d->desc = *desc;
-    auto bail = [&](const std::string &m) { const int s = dataset_error(d, m); delete d; return s; };
+    auto bail = [&](const std::string &m) { return dataset_error(d, m); };
     if (!d->file.open(nc_path)) return bail("dataset_open");
     long max_tag, in_size, n_seq, n_steps = 0, labels = 0, out_size = 0;
     if (!d->file.dimension("maxSeqTagLength", max_tag)) return bail("Cannot get dimension 'maxSeqTagLength'");
@@ -424,8 +448,10 @@ int cnt_dataset_open(const char *nc_path, const cnt_dataset_desc *desc, cnt_data
     if (desc->training_mode)
         std::stable_sort(d->sequences.begin(), d->sequences.end(),
                          [](const Sequence &a, const Sequence &b) { return a.length < b.length; });
-    *out = d;
+    *out = owned.release();
     return CNT_OK;
+} catch (...) {
+    return exception_error("dataset_open");
 }
 
 // DataSet::_shuffleSequences / _shuffleFractions (data_sets/DataSet.cpp:491-514), run by the reference at the start of
@@ -435,7 +461,7 @@ int cnt_dataset_open(const char *nc_path, const cnt_dataset_desc *desc, cnt_data
 // of libstdc++ runs -- element i changes places with a uniformly drawn element of 0..i -- on one Mersenne twister per
 // data set that the first call seeds (the reference seeds one per process from --random_seed and draws through
 // boost::uniform_int, so the permutations themselves are not the reference's).
-int cnt_dataset_shuffle(cnt_dataset *d, int shuffle_sequences, int shuffle_fractions, unsigned seed) {
+int cnt_dataset_shuffle(cnt_dataset *d, int shuffle_sequences, int shuffle_fractions, unsigned seed) try {
     using namespace cnt;
     CNT_REQUIRE(d, "dataset_shuffle: null handle");
     if (!d->shuffle_seeded) {
@@ -463,11 +489,14 @@ int cnt_dataset_shuffle(cnt_dataset *d, int shuffle_sequences, int shuffle_fract
             groups.back().push_back(d->sequences[i]);
         }
         shuffle(groups);
-        d->sequences.clear();
-        for (const auto &g : groups)
-            for (const auto &q : g) d->sequences.push_back(q);
+        std::vector<Sequence> order;
+        order.reserve(d->sequences.size());
+        for (const auto &g : groups) order.insert(order.end(), g.begin(), g.end());
+        d->sequences.swap(order);
     }
     return CNT_OK;
+} catch (...) {
+    return exception_error("dataset_shuffle");
 }
 
 int cnt_dataset_close(cnt_dataset *d) {
@@ -519,7 +548,7 @@ int cnt_dataset_fraction_shape(cnt_dataset *d, int first_seq, int *num_seqs, int
 }
 
 int cnt_dataset_fraction_fill(cnt_dataset *d, int first_seq, char *patTypes, float *inputs, float *targets,
-                              int *target_classes) {
+                              int *target_classes) try {
     using namespace cnt;
     int n, T;
     CNT_TRY(cnt_dataset_fraction_shape(d, first_seq, &n, &T, nullptr, nullptr));
@@ -592,6 +621,8 @@ int cnt_dataset_fraction_fill(cnt_dataset *d, int first_seq, char *patTypes, flo
             patTypes[(size_t)t * S + i] = t == 0 ? 1 : (t == s.length - 1 ? 3 : 2);  // FIRST, LAST, NORMAL
     }
     return CNT_OK;
+} catch (...) {
+    return exception_error("dataset_fraction");
 }
 
 }  // extern "C"

@@ -262,3 +262,66 @@ def test_fractions_in_blocks(tmp_path, lengths, P, Q, classes, S):
     assert os.waitpid(pid, 0)[1] == 0
     assert same()
     ds.close()
+
+
+_FAILING_NEW = r"""
+#include <cstdlib>
+#include <new>
+static size_t limit = 0;
+extern "C" void refuse_allocations_from(size_t bytes) { limit = bytes; }
+void *operator new(size_t n) {
+    if (limit && n >= limit) throw std::bad_alloc();
+    if (void *p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+"""
+
+_REFUSED = r"""
+import ctypes, sys
+sys.path.insert(0, sys.argv[1])
+from __graft_entry__ import load_package
+capi = load_package().capi
+refuse = ctypes.CDLL(sys.argv[2]).refuse_allocations_from
+refuse.argtypes = [ctypes.c_size_t]
+ds = capi.Dataset(sys.argv[3], int(sys.argv[4]), True, 0, 1.0)
+for limit in (60000, 1):
+    refuse(limit)
+    try:
+        ds.fraction(0)
+        text = "filled"
+    except RuntimeError as e:
+        text = str(e)
+    refuse(0)
+    assert "out of host memory" in text, text
+refuse(1)
+try:
+    capi.Dataset(sys.argv[3], int(sys.argv[4]))
+    text = "opened"
+except RuntimeError as e:
+    text = str(e)
+refuse(0)
+assert "out of host memory" in text, text
+first, again = ds.fraction(0), ds.fraction(0)
+assert (first["inputs"] == again["inputs"]).all() and first["inputs"].any()
+ds.close()
+print("survived")
+"""
+
+
+@pytest.mark.parametrize("lengths,P", [([30, 20], 600), ([900, 512, 300, 130], 200)])
+def test_refused_allocations_are_errors(tmp_path, lengths, P):
+    """A failing allocation inside a fraction, on the calling thread (small fractions) or on the helper threads as well (large
+    ones), is an error of that call: the process goes on and the data set stays usable."""
+    import subprocess
+    import sys
+
+    source, lib = tmp_path / "refuse.cpp", tmp_path / "librefuse.so"
+    source.write_text(_FAILING_NEW)
+    subprocess.check_call(["g++", "-O1", "-shared", "-fPIC", "-o", str(lib), str(source)])
+    p = str(tmp_path / "data.nc")
+    write_nc(p, lengths, P, 3, 2, seed=4)
+    r = subprocess.run([sys.executable, "-c", _REFUSED, ROOT, str(lib), p, str(len(lengths))], capture_output=True, text=True,
+                       env=dict(os.environ, LD_PRELOAD=" ".join([str(lib)] + os.environ.get("LD_PRELOAD", "").split())))
+    assert r.returncode == 0 and "survived" in r.stdout, (r.returncode, r.stdout, r.stderr)
