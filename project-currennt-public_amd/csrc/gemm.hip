@@ -67,14 +67,23 @@ inline int pick_vec(const GemmArgs &a, bool for_a) {
 // 6000 x 512 with 188 30 / 51; 1024 x 32000 x 128 with 2000 71 / 103).
 inline long large_tiles(const GemmArgs &a) { return (long)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.nprob; }
 
-// The weight gradient of one dense layer of 64 large tiles or more (1024 x 1024 weights) also takes the large tile, and as
-// many splits of k as make two workgroups per compute unit (the parts of two row-contiguous operands take 55 KB of LDS, so more do not
-// fit): the feed-forward model of five such layers 2320 -> 2224 us per pass, 768 workgroups 2230.  The gradients of a
+// The weight gradient of one dense layer of 64 to 256 large tiles (1024 x 1024 weights and more) also takes the large tile, and
+// as many splits of k as make two workgroups per compute unit (the parts of two row-contiguous operands take 55 KB of LDS, so more
+// do not fit), as long as a split has at least 768 values of k: below that, filling and draining the pipeline and the atomic sums
+// of the tiles outweigh what the large tile saves, and three times as many small workgroups share them better.  64 / 128, us,
+// with the clear and the column sum behind it: 1024 x 1024 over 2000 / 5000 / 8000 / 12 000 slots (250 / 625 / 1000 / 1500 per
+// split) 43 / 58, 88 / 89, 134 / 121, 193 / 162; 1300 x 1300 over 3000 / 4000 (750 / 1000) 98 / 101, 125 / 120; 2048 x 2048 over
+// 1000 / 3000 (500 / 1500) 73 / 79, 187 / 159.  (Below 64 tiles the line is further up, 896 x 896 over 2000 / 6000 / 12 000
+// 41 / 57, 92 / 86, 173 / 136, and layers of 32 tiles gain nothing; they keep the small tile.)  The feed-forward model of five
+// such layers: 2320 -> 2224 us per pass, with 768 workgroups 2230.  The gradients of a
 // recurrent layer, several problems per launch, run beside the recursion of the layer below and leave it less LDS and
 // issue slots then: with them on the large tile the acoustic model's pass takes 3787 instead of 3767 us.
 constexpr long kWideGradientGroups = 512;
+constexpr long kWideGradientSplit = 768;
 inline bool wide_gradient(const GemmArgs &a) {
-    return a.nprob == 1 && !a.masked && !a.a_kcontig && !a.b_kcontig && large_tiles(a) >= 64 && large_tiles(a) <= kWideGradientGroups / 2;
+    const long tiles = large_tiles(a);
+    return a.nprob == 1 && !a.masked && !a.a_kcontig && !a.b_kcontig && tiles >= 64 && tiles <= kWideGradientGroups / 2 &&
+           (long)a.k * a.nseg * tiles >= kWideGradientSplit * kWideGradientGroups;
 }
 
 int pick_tile(const GemmArgs &a) {

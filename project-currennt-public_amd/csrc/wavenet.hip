@@ -938,10 +938,13 @@ extern "C++" int cnt::wavenet_block_forward(hipStream_t stream, const cnt_cnn *c
                           (const void *)a.gated, (const void *)a.out, (const void *)a.sum, (const void *)a.skip})
         CNT_REQUIRE((reinterpret_cast<uintptr_t>(p) & 15) == 0, "wavenet_block_forward: buffers must be 16-byte aligned");
     // Samples per workgroup (16, 32 or 64): the more, the fewer times a block's weights are read, the fewer, the more
-    // workgroups share the chip.  Measured with 80 conditioning features (us at 16 / 32 / 64 samples): 64 channels, 4 000
-    // samples 10.3 / 13.9 / 21.1, 16 000 samples 27.4 / 21.5 / 22.1, 24 000 samples 38.3 / 32.9 / 34.5, 32 000 samples
-    // 50.8 / 41.0 / 35.4; 32 channels (60 features), 4 000 samples 6.9 / 9.5 / 15.3, 24 000 samples 15.6 / 15.9 / 24.3,
-    // 32 000 samples 23.7 / 17.7 / 24.6.
+    // workgroups share the chip, and a launch's time steps up where they start to share a compute unit.  us at 16 / 32 / 64
+    // samples per workgroup: 64 channels (80 conditioning features), 4096 samples 13.1 / 17.1 / 24.2, 5000 samples 17.5 / 17.1 /
+    // 24.3, 8192 samples 18.6 / 17.7 / 24.8, 12 000 samples 24.7 / 24.5 / 25.5, 16 000 samples 31.8 / 26.0 / 27.1, 24 000 samples
+    // 44.4 / 39.6 / 40.3, 28 000 samples 50.3 / 44.9 / 41.5; 48 channels (80 features), 8192 samples 14.5 / 15.1 / 21.8, 12 000
+    // samples 18.1 / 20.9 / 22.0, 16 000 samples 23.1 / 21.9 / 22.7, 24 000 samples 32.2 / 32.6 / 33.8, 28 000 samples 36.6 / 37.9 /
+    // 34.6; 32 channels (60 features), 4096 samples 9.5 / 12.1 / 18.0, 24 000 samples 18.5 / 19.0 / 27.4, 28 000 samples 23.2 /
+    // 20.3 / 27.8.
     const int st = N <= 4096 || (R < 64 && N <= 24576) ? 1 : R == 32 || N <= 24576 ? 2 : 4;
     const block_fwd_kernel_t kernel = pick_block_forward_kernel(R, st);
     const int lds = 16 * block_forward_lds_words(R, st, C);

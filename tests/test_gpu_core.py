@@ -656,6 +656,19 @@ def test_matrix_product_over_the_range_of_fp32(m, n, k, tA, tB, ea, eb):
     assert bool(((C - A64 @ B64).abs() <= bound).all())
 
 
+# both sides of the lines at which a dense layer's weight gradient changes its tile: 64 large tiles, 768 slots per split of k
+@pytest.mark.parametrize("P,D,N", [(1000, 1021, 6143), (1000, 1021, 6144), (896, 1024, 7100), (1700, 2048, 1600)])
+def test_wide_weight_gradient_on_both_tiles(P, D, N):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x, err = torch.randn(N, P, device="cuda", generator=g), torch.randn(N, D, device="cuda", generator=g)
+    dW = torch.full((P * D + D,), 3.0, device="cuda")
+    PC.pkg().capi.dense_backward_weights(P, D, N, 1.0, x, err, dW)
+    want, size = err.double().t() @ x.double(), err.double().abs().t() @ x.double().abs()
+    assert bool(((dW[:P * D].view(D, P) - want).abs() <= (N + 2) * 2.0 ** -24 * size).all())
+    assert bool(((dW[P * D:] - err.double().sum(0)).abs() <= (N + 2) * 2.0 ** -24 * err.double().abs().sum(0)).all())
+
+
 @pytest.mark.parametrize("static", [False, True])
 @pytest.mark.parametrize("P,D,N,bias", [(64, 128, 3000, 0.5), (30, 61, 997, 1.0), (256, 132, 2049, 0.25)])
 def test_bias_gradient_of_infinite_huge_and_missing_errors(P, D, N, bias, static):
