@@ -374,9 +374,9 @@ struct GatherStage {
 };
 
 // 32 x 32 sums of the product over the k tiles [it_begin, it_end), by one wave on the fp32 matrix instructions and straight
-// from memory, where the split product left sums that are not finite (an operand that is infinite or rounds to an infinite
-// bf16 value has infinity minus infinity in its parts).  Infinities and NaN come out as fp32 arithmetic has them.  A pass of a network
-// that has diverged is full of NaN, which stay what they are: the walk along k ends when all sums are.  1024 x 6000 x 1024,
+// from memory, where the split product left sums that are not finite: scaled, an operand from 2^112 on is infinite and has
+// infinity minus infinity in its parts, and a sum from 2^96 on overflows.  Infinities and NaN come out as fp32 arithmetic has them.
+// A pass of a network that has diverged is full of NaN, which stay what they are: the walk along k ends when all sums are.  1024 x 6000 x 1024,
 // usually 107 us: 107 us with NaN throughout, 756 with one at the end of every sum; one thread per sum took 11 400.
 template <bool AK, bool BK_, bool MASKED, bool GATHER>
 __device__ __forceinline__ f32x16 plain_sums(const GemmArgs &args, const GemmProblem &pb, int m0, int n0, int lane, int it_begin,
