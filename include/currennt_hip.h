@@ -141,7 +141,7 @@ typedef struct {
  * CNT_LSTM_LOCAL_JB=8|16 (cells per workgroup of a team), CNT_LSTM_SLOTS=<n> (workgroups of a recursion a compute unit may
  * take), CNT_LSTM_SOLO=<cells> (largest layer run by one workgroup per job), CNT_LSTM_WARM=1 (a
  * full-bandwidth read of the states into the memory-side cache in front of the backward recursion),
- * CNT_LSTM_MEM_DELAY=<units of 64 clocks> (how long the backward recursion's memory wave sleeps after a step's barrier),
+ * CNT_LSTM_MEM_DELAY=<units of 64 clocks> (how long the backward recursion's store wave sleeps after a step's barrier),
  * CNT_LSTM_STEPWISE=1. */
 int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out);
 int cnt_lstm_destroy(cnt_lstm *h);

@@ -17,7 +17,7 @@
 // loads that bypass the non-coherent caches, and handed back as empty after use; four slots rotate.  Every
 // poll loop is bounded: when the bound is hit the workgroup raises a device flag and every workgroup drains
 // out.  Inside a workgroup, waves specialise (polling waves that never store, product / cell waves that never
-// wait for a store, one memory wave for all ordinary loads and stores), see the kernels' comments.
+// wait for a store, a load and a store wave for all ordinary loads and stores), see the kernels' comments.
 //
 // The dense work that does not sit on the recursion is batched over all time steps on the MFMA
 // GEMM: input projections (8 problems, one launch), the error to the preceding layer
@@ -59,10 +59,9 @@ struct ChainParams {
     float *herr_out;      // backward, unidirectional: where the summed error is written back
     unsigned spin_limit;
     int *abort_flag;
-    long long *phase_ticks;  // optional diagnostic: per workgroup accumulated phase durations (100 MHz ticks)
     int poll_delay, poll_gap;  // s_sleep units before the first poll of a step / between polls
-    int mem_delay;             // XCD-local backward recursion: s_sleep units before the memory wave's work of a step
-    int poll_delay_fwd;
+    int mem_delay;             // XCD-local backward recursion: s_sleep units before the store wave's work of a step
+    int poll_delay_fwd, mem_delay_fwd;  // forward: the same, and before the load wave's
     int *latch;  // host-visible mark "a recursion of this handle gave up" (pinned host memory), never cleared by kernels
     int *veto;   // optional device flag shared by a network's handles, set together with the latch
     // XCD-local backward recursion: jobs = (direction, group of sequences), see lstm_local.hpp
@@ -113,7 +112,14 @@ __device__ __forceinline__ void lds_barrier() {
 // ---------------------------------------------------------------------------------------------------
 constexpr unsigned kEmpty = 0xFFFFFFFFu;
 constexpr int kMailSlots = 4;
-constexpr int kForwardPause = 18;  // pause before the first poll of a forward step, units of 64 clocks
+// Pauses of the XCD-local recursions, units of 64 clocks: before the first poll of a step (a pause that ends after the words have
+// arrived costs a poll round less, one that ends too late its own length), and before the store wave's work of a backward and the
+// load wave's of a forward step, which then stay out of the first poll's way.  Measured on MI355X, us per step.  Backward, first
+// poll after 1 / 3 / 5 / 7 / 9 units: 256 cells 8 jobs of 2-3 sequences 0.90 / 0.87 / 0.91 / 0.97 / 1.00, jobs of one 0.75 / 0.77 /
+// 0.80 / 0.84 / 0.89; stores after 0 / 4 / 8 units 0.90 / 0.87 / 0.88.  Forward, 8 / 9 / 10 / 11 / 12 / 13 / 14 / 16 units: 1.05 / 1.04 /
+// 1.03 / 1.00 / 1.00 / 1.01 / 1.03 / 1.07 and 0.88 / 0.88 / 0.87 / 0.86 / 0.87 / 0.89 / 0.92 / 0.98; loads after 0 / 4 units 0.99 / 0.98.
+// Sizes of 128 to 512 cells and 1 to 16 jobs have their best values within one unit of these.
+constexpr int kBackwardPause = 3, kStorePause = 4, kForwardPause = 11, kLoadPause = 4;
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima) as a builtin, so that the compiler's own wait
@@ -377,9 +383,7 @@ struct cnt_lstm {
     int *abort_flag;
     int device;
     unsigned spin_limit;
-    long long *phase_ticks;  // diagnostic buffer, allocated when CNT_LSTM_TIMING is set
     int poll_gap;
-    int last_was_forward;  // which recursion the diagnostic buffer describes
     int bmail_dirty;       // the backward mailbox may hold words that are not empty
     int flmail_dirty;      // the same for the XCD-local forward recursion's mailbox
     cnt::SlotOrder slot_order;  // the loaded fraction's slots, valid ones first (set by the owner of the pattern types, or null)
@@ -394,19 +398,19 @@ struct cnt_lstm {
     int njobs, groups;
     int launch_jobs;       // jobs of one launch: as many as complete teams fit the compute units at once
     int local_jb, team;    // cells per workgroup and workgroups of a team
+    int local_nsq;         // sequences a job's kernels move and multiply: 1, 2 or 4
     int ctl_teams;
     unsigned *ctl;
     float *lmail;
     size_t lmail_words;
     float *flmail;         // XCD-local forward recursion: one mailbox per job
     size_t flmail_words;
-    int last_blocks;       // workgroups of the last recursion launch
     int warm;  // read the recursion's inputs once before the XCD-local backward recursion (off; CNT_LSTM_WARM=1: on)
     int spread_lds_most;
     int spread_lds;  // dynamic LDS the XCD-local recursion asks for so that a compute unit takes one of its workgroups
     int poll_delay_local;  // pause before the first poll of a step in the XCD-local recursion, units of 64 clocks
-    int mem_delay_local;   // pause of that recursion's memory wave after the step barrier, same units
-    int poll_delay_fwd_local;  // the same for the XCD-local forward recursion
+    int mem_delay_local;   // pause of that recursion's store wave after the step barrier, same units
+    int poll_delay_fwd_local, mem_delay_fwd_local;  // XCD-local forward recursion: pauses before the first poll and the loads of a step
     // set by every recursion launch: the failure latch is taken only once the launch that may have set it has ended
     // (the device's recursion-order event, see launch_in_order), so that no workgroup of that launch can set it (or the
     // veto) again after the report
@@ -451,8 +455,8 @@ void fill_chain_params(const cnt_lstm *h, const float *weights, ChainParams &p) 
     p.ctl = h->ctl;
     p.lmail = h->lmail;
     p.flmail = h->flmail;
-    p.phase_ticks = h->phase_ticks;
     p.poll_delay = h->poll_delay_local; p.poll_gap = h->poll_gap; p.poll_delay_fwd = h->poll_delay_fwd_local;
+    p.mem_delay_fwd = h->mem_delay_fwd_local;
     p.mem_delay = h->mem_delay_local;
 }
 
@@ -497,33 +501,47 @@ int warm_backward_inputs(const cnt_lstm *h, hipStream_t stream, const ChainParam
     return CNT_OK;
 }
 
-template <int PW, int JB>
+template <int PW, int JB, int NSQ>
 chain_kernel_t local_pair(bool fwd) {
-    return fwd ? (chain_kernel_t)lstm_forward_local<PW, JB> : (chain_kernel_t)lstm_backward_local<PW, JB>;
+    return fwd ? (chain_kernel_t)lstm_forward_local<PW, JB, NSQ> : (chain_kernel_t)lstm_backward_local<PW, JB, NSQ>;
+}
+template <int PW, int JB>
+chain_kernel_t local_pair(bool fwd, int nsq) {
+    return nsq == 1 ? local_pair<PW, JB, 1>(fwd) : nsq == 2 ? local_pair<PW, JB, 2>(fwd) : local_pair<PW, JB, 4>(fwd);
 }
 
 // Cells per workgroup of a layer with H cells per direction and `jobs` jobs; 0: no XCD-local kernel.  A team should fit
 // the 32 compute units of an XCD one workgroup each, and two teams where there are more jobs than XCDs: 16 cells of 8
 // per workgroup for up to 128 cells, 32 of 8 up to 256 cells -- or 16 of 16 when there are more than eight jobs --, 32
-// of 16 up to 512.  Measured, us per step forward / backward, MI355X: 128 cells 8 jobs 1.15 / 1.16 with 4 cells per
-// workgroup, 1.20 / 1.16 with 8, 16 jobs 1.29 / 1.33 and 1.21 / 1.17; 256 cells 8 jobs 1.28 / 1.28 with 8 and 1.45 / 1.49
-// with 16, 16 jobs 1.72 / 1.66 (two workgroups per compute unit) and 1.48 / 1.52.
+// of 16 up to 512.  Measured, us per step forward / backward, MI355X: 256 cells 8 jobs 0.99 / 0.87 with 8 and 1.09 / 1.03
+// with 16 cells per workgroup, 16 jobs 1.33 / 1.33 (two workgroups per compute unit) and 1.19 / 1.14; 200 cells 0.95 / 0.85 and
+// 1.08 / 1.01, 1.23 / 1.16 and 1.14 / 1.05.
 int local_cells(int H, int jobs) {
     if (const char *e = std::getenv("CNT_LSTM_LOCAL_JB")) return std::atoi(e);
     return H > 512 ? 0 : H <= 128 ? 8 : H <= 256 ? (jobs <= kLocalXcds ? 8 : 16) : 16;
 }
 
-chain_kernel_t pick_local_kernel(bool fwd, int H, int JB) {
+// Sequences the kernels of a job move: the smallest that holds the largest job.  Jobs of one or two sequences are rare where
+// layers of up to 256 cells take 16 cells per workgroup (more than eight jobs): no kernels of their own.
+int local_sequences(int H, int JB, int most) { return most > 2 || (JB == 16 && H <= 256) ? 4 : most; }
+
+chain_kernel_t pick_local_kernel(bool fwd, int H, int JB, int nsq) {
     const int PW = (H + 63) / 64;
-    if (JB == 8) return PW == 2 ? local_pair<2, 8>(fwd) : PW == 3 ? local_pair<3, 8>(fwd) : PW == 4 ? local_pair<4, 8>(fwd) : nullptr;
+    if (JB == 8) {
+        switch (PW) {
+            case 2: return local_pair<2, 8>(fwd, nsq);
+            case 3: return local_pair<3, 8>(fwd, nsq);
+            case 4: return local_pair<4, 8>(fwd, nsq);
+        }
+    }
     if (JB == 16) {
         switch (PW) {
-            case 3: return local_pair<3, 16>(fwd);
-            case 4: return local_pair<4, 16>(fwd);
-            case 5: return local_pair<5, 16>(fwd);
-            case 6: return local_pair<6, 16>(fwd);
-            case 7: return local_pair<7, 16>(fwd);
-            case 8: return local_pair<8, 16>(fwd);
+            case 3: return local_pair<3, 16, 4>(fwd);
+            case 4: return local_pair<4, 16, 4>(fwd);
+            case 5: return local_pair<5, 16>(fwd, nsq);
+            case 6: return local_pair<6, 16>(fwd, nsq);
+            case 7: return local_pair<7, 16>(fwd, nsq);
+            case 8: return local_pair<8, 16>(fwd, nsq);
         }
     }
     return nullptr;
@@ -610,7 +628,7 @@ int launch_chain(cnt_lstm *h, hipStream_t stream, bool fwd, ChainParams &p) {
         CNT_HIP(hipGetLastError());
         return CNT_OK;
     }
-    chain_kernel_t k = pick_local_kernel(fwd, h->H, h->local_jb);
+    chain_kernel_t k = pick_local_kernel(fwd, h->H, h->local_jb, h->local_nsq);
     CNT_REQUIRE(k != nullptr, "lstm: no recursion kernel for H=%d JB=%d", h->H, h->local_jb);
     // heals the handle after a launch that gave up, zeroes the placement counters; in front of the backward recursion it
     // can be part of the cache-warming launch
@@ -634,14 +652,12 @@ int launch_chain(cnt_lstm *h, hipStream_t stream, bool fwd, ChainParams &p) {
     if (dirty) CNT_TRY(fill_words(stream, reinterpret_cast<unsigned *>(fwd ? h->flmail : h->lmail),
                                   fwd ? h->flmail_words : h->lmail_words, kEmpty));
     dirty = 0;
-    h->last_was_forward = fwd ? 1 : 0;
     if (!fwd && h->warm && !resumes) {
         GuardParams none = {};
         none.abort_flag = h->abort_flag;  // with nothing to zero or refill the body only reads the flag
         CNT_TRY(warm_backward_inputs(h, stream, p, guard_rides ? g : none));
     }
     ProfileScope prof(stream, fwd ? "lstm_forward_chain" : "lstm_backward_chain");
-    h->last_blocks = local_blocks(h);
     // One workgroup per compute unit while the teams of an XCD fit its 32 compute units.  A team's workgroups take a step
     // in lock-step, and two of them on one compute unit share its four matrix pipes and its path to the L2 at exactly
     // the same moments: the dispatcher, left to itself, puts the 32 workgroups of a 256-cell team on 16-17 compute units,
@@ -655,7 +671,7 @@ int launch_chain(cnt_lstm *h, hipStream_t stream, bool fwd, ChainParams &p) {
         p.job0 = (unsigned)job0;
         p.njobs = std::min(h->launch_jobs, h->njobs - job0);
         CNT_TRY(launch_in_order(h, stream, [&] {
-            hipLaunchKernelGGL(k, dim3(h->last_blocks), dim3(local_threads((h->H + 63) / 64)), (size_t)h->spread_lds, stream, p);
+            hipLaunchKernelGGL(k, dim3(local_blocks(h)), dim3(local_threads((h->H + 63) / 64, h->local_jb, h->local_nsq)), (size_t)h->spread_lds, stream, p);
         }));
     }
     return CNT_OK;
@@ -669,8 +685,8 @@ void local_placement(cnt_lstm *h, int lds_per_cu, int cus_per_xcd) {
     int most = kLocalSlots;
     for (int fwd = 0; fwd < 2; ++fwd) {
         int fit = 0;
-        const void *k = reinterpret_cast<const void *>(pick_local_kernel(fwd != 0, h->H, h->local_jb));
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k, local_threads((h->H + 63) / 64), 0) != hipSuccess) {
+        const void *k = reinterpret_cast<const void *>(pick_local_kernel(fwd != 0, h->H, h->local_jb, h->local_nsq));
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k, local_threads((h->H + 63) / 64, h->local_jb, h->local_nsq), 0) != hipSuccess) {
             (void)hipGetLastError();
             fit = 1;
         }
@@ -785,7 +801,8 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     // one-workgroup kernels gain nothing from smaller jobs)
     const int groups = std::max((desc->S + kLocalSeqs - 1) / kLocalSeqs, solo ? 1 : std::min(kLocalXcds / ndir, desc->S));
     const int local_jb = local_cells(H, ndir * groups);
-    const bool stepwise = (!solo && pick_local_kernel(true, H, local_jb) == nullptr) || std::getenv("CNT_LSTM_STEPWISE") != nullptr;
+    const int local_nsq = local_sequences(H, local_jb, (desc->S + groups - 1) / groups);
+    const bool stepwise = (!solo && pick_local_kernel(true, H, local_jb, local_nsq) == nullptr) || std::getenv("CNT_LSTM_STEPWISE") != nullptr;
 
     cnt_lstm *h = new (std::nothrow) cnt_lstm();
     CNT_REQUIRE(h != nullptr, "lstm_create: out of host memory");
@@ -795,31 +812,17 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     h->solo = solo && !stepwise ? 1 : 0;
     h->local = !solo && !stepwise ? 1 : 0;
     h->local_jb = local_jb;
+    h->local_nsq = local_nsq;
     h->bmail_dirty = 1;
     h->flmail_dirty = 1;
     h->spin_limit = 1u << 22;
     if (const char *e = std::getenv("CNT_LSTM_SPIN_LIMIT")) h->spin_limit = (unsigned)std::strtoul(e, nullptr, 10);
-    // XCD-local recursion: product (about 0.3 us) and one hop through the L2 (about 0.45 us) pass between a step's
-    // barrier and the arrival of the next partial errors
-    // (fitted on the benchmark models with one workgroup of a team per compute unit: the acoustic model's pass takes
-    // 2.41 / 2.38 / 2.35 / 2.39 / 2.47 / 2.50 ms at 8 / 9 / 10 / 11 / 12 / 13 units, the single 256-cell layer 0.355 /
-    // 0.353 / 0.361 ms at 9 / 10 / 11: a pause that ends after the words have arrived costs a whole poll round less,
-    // one that ends too late costs its own length)
-    h->poll_delay_local = 10;
-    // The memory wave's loads and stores of a step are issued once the first poll is expected back: pause of the poll
-    // plus one poll round (four 16-byte loads per lane at 256 cells, two or one below).  Measured on MI355X: acoustic
-    // model 2.39 / 2.53 / 2.52 / 2.36 / 2.31 / 2.32 / 2.34 / 2.36 ms at 0 / 12 / 14 / 16 / 17 / 18 / 19 / 24 units (a wave that
-    // wakes while the poll is in flight is the worst case); a 128- or 64-cell BLSTM layer alone 716 / 661 / 695 / 722 us
-    // and 688 / 641 / 678 / 713 us at 0 / 15 / 17 / 19 units.  With the mailbox hand-back stores in this wave as well the
-    // landscape moves by one unit (2.51 / 2.35 / 2.28 / 2.30 / 2.31 / 2.34 ms at 16 / 17 / 18 / 19 / 20 / 21).  The value kept
-    // is one unit behind the best one: the step in front of the best value is a cliff, the step behind it costs 0.2 %.
-    // (128- and 64-cell layers alone, hand-back stores included: 679 / 647 / 657 / 676 us and 683 / 648 / 662 / 672 us at
-    // 14 / 15 / 16 / 17 units.)
-    h->mem_delay_local = h->poll_delay_local + (H >= 256 ? 9 : 6);
+    h->poll_delay_local = kBackwardPause;
+    h->mem_delay_local = kStorePause;
     if (const char *e = std::getenv("CNT_LSTM_MEM_DELAY")) h->mem_delay_local = std::atoi(e);
     // The full-bandwidth read of the recursion's inputs in front of it (warm_cache) was worth 0.15 ms per model pass
-    // while the memory wave's loads were issued in front of the polls; with that wave's pause it costs more than it
-    // gains (2.290 -> 2.282 ms without it, 0.355 -> 0.352 ms for the single layer).  CNT_LSTM_WARM=1 turns it on.
+    // while loads were issued in front of the polls in every step; now it costs more than it gains.  CNT_LSTM_WARM=1 turns
+    // it on.
     h->make_order = true;
     if (const char *e = std::getenv("CNT_LSTM_SKIP_PADDING")) h->make_order = std::atoi(e) != 0;
     h->warm = 0;
@@ -835,10 +838,8 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
         }
     }
     if (const char *e = std::getenv("CNT_LSTM_POLL_DELAY")) h->poll_delay_local = std::atoi(e);
-    // the same pause for the forward recursion.  Measured at 14 / 16 / 18 / 20 / 22 / 24 units: 256 cells 1.32 / 1.33 / 1.29 /
-    // 1.29 / 1.31 / 1.36 us per step, two teams per XCD 1.36 / 1.34 / 1.32 / 1.35 / 1.41 / 1.46, 150 cells 1.22 / 1.21 / 1.21 /
-    // 1.22 / 1.28 / 1.33, 128 cells 1.19 / 1.19 / 1.18 / 1.21 / 1.27 / 1.32
     h->poll_delay_fwd_local = kForwardPause;
+    h->mem_delay_fwd_local = kLoadPause;
     if (const char *e = std::getenv("CNT_LSTM_POLL_DELAY_FWD")) h->poll_delay_fwd_local = std::atoi(e);
     if (const char *e = std::getenv("CNT_LSTM_POLL_GAP")) h->poll_gap = std::atoi(e);
     hipError_t err = hipGetDevice(&h->device);
@@ -853,7 +854,7 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     h->njobs = ndir * groups;
     if (h->local) {
         h->team = (H + h->local_jb - 1) / h->local_jb;
-        h->lmail_words = h->flmail_words = (size_t)h->njobs * local_job_words(h->team, h->local_jb);
+        h->lmail_words = h->flmail_words = (size_t)h->njobs * local_job_words(h->team, h->local_jb, h->local_nsq);
         local_placement(h, per_cu, cus / kLocalXcds);
         h->ctl_teams = local_blocks(h) / h->team + 1;
         if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void **>(&h->lmail), h->lmail_words * sizeof(float));
@@ -861,9 +862,6 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
         if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void **>(&h->ctl), ctl_words(h->ctl_teams) * sizeof(unsigned));
         if (err == hipSuccess) err = hipMemset(h->ctl, 0, ctl_words(h->ctl_teams) * sizeof(unsigned));
     }
-    if (err == hipSuccess && std::getenv("CNT_LSTM_TIMING"))
-        err = hipMalloc(reinterpret_cast<void **>(&h->phase_ticks), 8 * 512 * 6 * sizeof(long long));
-    if (err == hipSuccess && h->phase_ticks) err = hipMemset(h->phase_ticks, 0, 8 * 512 * 6 * sizeof(long long));
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void **>(&h->own_order), ((size_t)h->desc.maxT * h->desc.S + 4) * sizeof(int));
     if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void **>(&h->abort_flag), sizeof(int));
     if (err == hipSuccess) err = hipMemset(h->abort_flag, 0, sizeof(int));
@@ -889,7 +887,6 @@ int cnt_lstm_destroy(cnt_lstm *h) {
             if (h->state[dir][w]) (void)hipFree(h->state[dir][w]);
     }
     if (h->abort_flag) (void)hipFree(h->abort_flag);
-    if (h->phase_ticks) (void)hipFree(h->phase_ticks);
     if (h->lmail) (void)hipFree(h->lmail);
     if (h->flmail) (void)hipFree(h->flmail);
     if (h->ctl) (void)hipFree(h->ctl);
@@ -950,8 +947,8 @@ int cnt_lstm_set_wait_bounds(cnt_lstm *h, unsigned spin_limit, int poll_delay_ba
     CNT_REQUIRE(poll_delay_backward >= 0 && poll_delay_backward <= 4096 && poll_delay_forward >= 0 &&
                 poll_delay_forward <= 4096, "lstm_set_wait_bounds: poll delays must be within 0..4096");
     h->spin_limit = spin_limit;
-    h->poll_delay_local = poll_delay_backward < 10 ? poll_delay_backward : 10;
-    if (poll_delay_backward < 10) h->mem_delay_local = poll_delay_backward;
+    h->poll_delay_local = std::min(poll_delay_backward, kBackwardPause);
+    h->mem_delay_local = std::min(poll_delay_backward, kStorePause);
     h->poll_delay_fwd_local = std::min(poll_delay_forward, kForwardPause);
     return CNT_OK;
 }
@@ -1017,43 +1014,6 @@ int cnt_lstm_check(cnt_lstm *h, void *stream) {
     using namespace cnt;
     CNT_REQUIRE(h, "lstm_check: null handle");
     CNT_HIP(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
-    if (h->phase_ticks && h->local) {
-        // diagnostic: mean phase durations of the last recursion over the workgroups that took part
-        const int blocks = std::min(h->last_blocks, (int)kTraceBlocks);
-        const bool local = h->local && !h->last_was_forward;
-        const int stride = local ? 8 : 6;
-        std::vector<long long> t((size_t)blocks * stride);
-        CNT_HIP(hipMemcpy(t.data(), h->phase_ticks, t.size() * sizeof(long long), hipMemcpyDeviceToHost));
-        double m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        int active = 0;
-        for (int b = 0; b < blocks; ++b) {
-            if (t[(size_t)b * stride + 3] == 0) continue;
-            ++active;
-            for (int q = 0; q < stride; ++q) m[q] += (double)t[(size_t)b * stride + q];
-        }
-        if (local && std::getenv("CNT_LSTM_TRACE")) {
-            std::vector<long long> tr((size_t)blocks * kTraceStride);
-            CNT_HIP(hipMemcpy(tr.data(), h->phase_ticks + kTraceBase, tr.size() * sizeof(long long), hipMemcpyDeviceToHost));
-            for (int b = 0; b < blocks; ++b) {
-                if (t[(size_t)b * stride + 3] == 0) continue;
-                const long long *r = &tr[(size_t)b * kTraceStride];
-                std::fprintf(stderr, "trace block %d job %lld member %lld xcd %lld hwid %lld:", b, r[0], r[1], r[2], r[3]);
-                for (int q = 0; q < 5 * kTraceSteps; ++q) std::fprintf(stderr, " %lld", r[4 + q]);
-                std::fprintf(stderr, "\n");
-            }
-        }
-        CNT_HIP(hipMemset(h->phase_ticks, 0, 8 * 512 * 6 * sizeof(long long)));
-        const double us = active ? 0.01 / active / h->T : 0.0;
-        if (h->last_was_forward)
-            std::fprintf(stderr, "lstm forward per step [us]: gather waves pause+poll %.3f product %.3f barrier %.3f loop %.3f "
-                         "poll rounds %.2f (T=%d, %d workgroups)\n", m[1] * us, (m[0] - m[1] - m[2]) * us, m[2] * us, m[3] * us,
-                         active ? m[4] / active / h->T : 0.0, h->T, active);
-        else
-            std::fprintf(stderr, "lstm backward per step [us]: cell wave wait+poll %.3f (lane 0's polls %.3f in %.2f rounds) "
-                         "update+barrier %.3f loop %.3f | product waves busy %.3f | memory wave busy %.3f (T=%d, %d workgroups)\n",
-                         m[0] * us, m[6] * us, active ? m[4] / active / h->T : 0.0, m[1] * us, m[3] * us, m[2] * us, m[5] * us,
-                         h->T, active);
-    }
     if (lstm_take_failure(h)) {
         set_error("%s", kGaveUp);
         return CNT_ERR_DEVICE;

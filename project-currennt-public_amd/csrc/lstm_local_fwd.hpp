@@ -11,41 +11,48 @@
 // written yet, four slots; a receiver hands the words of a slot back as empty in the step after it has read them.
 //
 // Waves and roles, one LDS-only barrier per step, every LDS buffer twice (step parity):
-//   gather waves (H/64)  each takes 64 source cells for all of the workgroup's (gate, cell) rows: polls its quarter of
-//                        the block (one 16-byte vector per lane), passes the words through its own corner of LDS into
-//                        B operands of v_mfma_f32_4x4x1 (blocks = four rows x one residue of the cell index), leaves
+//   gather waves (H/64)  each takes 64 source cells for all of the workgroup's (cell, gate) rows: polls its quarter of
+//                        the block, one 16-byte vector per lane, which is the A operand of the step's recurrent product as
+//                        it stands (lane = 4 * source cells / 4 + sequence; local_product broadcasts the blocks), leaves
 //                        its share of the recurrent sums in LDS.  They issue no stores.
-//   cell wave (1)        after the barrier: pre-activations = input projection + recurrent sums, gates, cell state,
-//                        h[t]; publishes h[t] to every member's block and empties the block it read.
-//   memory wave (1)      input projections two steps ahead; gate activations, cell states and outputs of the finished
-//                        step to the state arrays.
+//   cell waves (CW)      after the barrier: lane = one gate of one (cell, sequence) element.  Pre-activation = input
+//                        projection + recurrent sums, first pass of the gate function (the four lanes of an element
+//                        evaluate the gates side by side; tanh and logistic differ in constants only), cell state in every
+//                        lane, second pass: tanh(c) and the output gate side by side.  The row of sixteen lanes holds four
+//                        neighbouring cells of a sequence: h[t] is broadcast inside the row and published to every member's
+//                        block as it stands.
+//   load wave (1)        input projections of several steps at a time.
+//   store wave (1)       gate activations, cell states and outputs of finished steps to the state arrays, 64 lanes' worth at a
+//                        time; empties the block that was read.
+// What bounds a step: the chain sums -> gates -> c -> h -> LDS -> store -> L2 -> poll -> 4 * JB matrix instructions -> LDS.  With one
+// cell wave that computed all gates of an element in one lane (five gate functions, two of them side by side at best, twenty LDS
+// reads), gather waves that passed the words through LDS into B operands, messages of four sequences throughout and one wave for all
+// loads and stores, a step took, us on MI355X (input products included): 256 cells, 8 jobs of 2-3 sequences 1.34, 2 jobs of one
+// 1.29, 16 jobs of four 1.43; 128 cells, 8 jobs of two 1.22; 512 cells, 6 jobs of one 1.97.  Now 0.99, 0.85, 1.18, 0.89 and 1.34.
+// Publishing without LDS, by a broadcast inside the row of sixteen lanes, saves a round trip of 0.03 but stores pieces of 16
+// bytes: 1.05 instead of 1.00.
 
-// PW = ceil(cells per direction / 64) gather waves, JB cells per workgroup
-template <int PW, int JB>
-__global__ __launch_bounds__(local_threads(PW)) void lstm_forward_local(const ChainParams p) {
+// PW = ceil(cells per direction / 64) gather waves, JB cells per workgroup, NSQ sequences per job
+template <int PW, int JB, int NSQ>
+__global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local(const ChainParams p) {
+    using Shape = LocalShape<JB, NSQ>;
     const int H = p.H, G = p.team;       // G = ceil(H / JB) workgroups; the last one may own fewer than JB cells
-    constexpr int NSQ = kLocalSeqs;
-    constexpr int ROWS = 4 * JB;         // (gate, cell) rows of this workgroup: row = gate * JB + cell
-    constexpr int NQ = PW;               // 16-byte vectors per lane that hand a block back; the last may lie past its end
-    constexpr int EL = NSQ * JB;         // (sequence, cell) elements: e = sequence * JB + cell
-    constexpr int PAIR = NSQ * JB;       // words one sender leaves in one receiver's block
-    constexpr int CH = PAIR / 4;         // 16-byte chunks of those
-    constexpr int RPS = 64 / CH;         // receivers served by one publishing store
-    constexpr int PUB = (64 * PW / JB + RPS - 1) / RPS;  // publishing stores per lane; the last may lie past the team
-    const unsigned RECV = (unsigned)(G * PAIR);  // words of a receiver's block
-    const int vectors = G * JB;          // 16-byte vectors of a receiver's block
-    static_assert(EL <= 64, "local forward geometry");
-    enum { R_NI = 0, R_IG, R_FG, R_OG, R_C, R_H, NRES };
+    constexpr int EL = Shape::EL, VEC = Shape::VEC, VPW = Shape::VPW, CW = Shape::CW;
+    constexpr int STEPS = Shape::STEPS, BATCH = Shape::BATCH, SETS = Shape::SETS, RING = 2 * BATCH;
+    constexpr int TEAM = (64 * PW + JB - 1) / JB;  // G at most
+    constexpr int ROWS = 4 * JB;         // (cell, gate) rows of this workgroup: row = cell * 4 + gate
+    constexpr int PUB = (TEAM * VPW + 63) / 64;  // publishing stores per lane; the last may lie past the team
+    constexpr int NQ = (TEAM * VEC + 63) / 64;  // vectors per lane that hand a block back
+    const unsigned RECV = (unsigned)(G * EL);   // words of a receiver's block
+    const int vectors = G * VEC;                // 16-byte vectors of a receiver's block
 
-    __shared__ float red[2][PW][ROWS][NSQ];   // recurrent sums of the step, one share per gather wave
-    // a gather wave's 64 source cells per sequence, in cell order; the pitch keeps the four sequences' 16-byte reads
-    // off each other's banks
-    __shared__ __attribute__((aligned(16))) float hstage[PW][NSQ][64 + 4];
-    __shared__ float pre[2][4][64];       // input projections of the step
-    __shared__ int pre_dummy[2][64];
-    __shared__ float res[2][NRES][64];    // results of the step
-    __shared__ int res_flags[2][64];      // bit 0: gate activations to store, bit 1: cell state to store
-    __shared__ __attribute__((aligned(16))) float hpub[NSQ][JB];
+    // element = (group of four cells * NSQ + sequence) * 4 + cell of the group, as in the messages
+    __shared__ __attribute__((aligned(16))) float red[2][PW][ROWS][NSQ];  // recurrent sums of the step, one share per gather wave
+    __shared__ __attribute__((aligned(16))) float pre[RING][EL][4];    // input projections of the step
+    __shared__ int pre_dummy[RING][EL];
+    __shared__ __attribute__((aligned(16))) float res_gate[2][EL][4];     // results of the step
+    __shared__ __attribute__((aligned(16))) float res[2][EL][4];          // cell state, output, not 0: padding slot
+    __shared__ __attribute__((aligned(16))) float hpub[CW][VPW][4];
     __shared__ int wait_failed;
     __shared__ int role_sh;
 
@@ -64,197 +71,221 @@ __global__ __launch_bounds__(local_threads(PW)) void lstm_forward_local(const Ch
     const int S = p.S, T = p.T;
     const int j0 = me * JB;
     const int n = S * H;
-    float *const mailbox = p.flmail + (size_t)job * local_job_words(G, JB);
+    float *const mailbox = p.flmail + (size_t)job * local_job_words(G, JB, NSQ);
     const unsigned slot_words = (unsigned)G * RECV;
     const __amdgpu_buffer_rsrc_t mail =
-        __builtin_amdgcn_make_buffer_rsrc(mailbox, 0, (int)(local_job_words(G, JB) * sizeof(float)), 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(mailbox, 0, (int)(local_job_words(G, JB, NSQ) * sizeof(float)), 0x00020000);
     auto slot_of = [&](int step) { return dir ? (T - 1 - step) : step; };
+    auto given_up = [&]() { return *(__attribute__((address_space(3))) volatile int *)&wait_failed; };
 
-    if (wave == PW + 1) {
-        // ------------------------------------------------------------------ memory wave
+    // the load and the store wave: lane = (step of an access, sequence, cell)
+    const int cs = lane % EL / JB, cj = lane % JB;
+    const bool valid = cs < nseq && j0 + cj < H;
+    const int ahead = lane / EL;
+
+    if (wave == PW + CW) {
+        // ------------------------------------------------------------------ load wave
         struct StepIn { float a[4]; char pat; };
-        const int cs = lane / JB, cj = lane % JB;
-        const bool valid = lane < EL && cs < nseq && j0 + cj < H;
-        const int s = seq0 + cs;
-        auto load_step = [&](int step, StepIn &v) {
-            v = StepIn{{0, 0, 0, 0}, 1};
-            if (!valid || step >= T) return;
-            const int t = slot_of(step);
-            const size_t gi = (size_t)t * n + (size_t)s * H + j0 + cj;
-            v.a[0] = D.ni[gi]; v.a[1] = D.ig[gi]; v.a[2] = D.fg[gi]; v.a[3] = D.og[gi];
-            v.pat = p.pat[t * S + s];
-        };
-        auto put_pre = [&](int step, const StepIn &v) {
-            const int t = slot_of(step);
+        const int s = seq0 + cs, el = (cj / 4 * NSQ + cs) * 4 + cj % 4;
+        auto load_batch = [&](int first, StepIn (&in)[SETS]) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) pre[step & 1][g][lane] = v.a[g];
-            pre_dummy[step & 1][lane] = ((t >= p.Tmin) && (v.pat == 0)) ? 1 : 0;
-        };
-        auto store_results = [&](int step) {
-            if (!valid) return;
-            const int t = slot_of(step), b = step & 1;
-            const size_t gi = (size_t)t * n + (size_t)s * H + j0 + cj;
-            const int flags = res_flags[b][lane];
-            if (flags & 1) {
-                D.ni[gi] = res[b][R_NI][lane]; D.ig[gi] = res[b][R_IG][lane];
-                D.fg[gi] = res[b][R_FG][lane]; D.og[gi] = res[b][R_OG][lane];
+            for (int i = 0; i < SETS; ++i) {
+                StepIn &v = in[i];
+                v = StepIn{{0, 0, 0, 0}, 1};
+                const int step = first + i * STEPS + ahead;
+                if (!valid || step >= T) continue;
+                const int t = slot_of(step);
+                const size_t gi = (size_t)t * n + (size_t)s * H + j0 + cj;
+                v.a[0] = D.ni[gi]; v.a[1] = D.ig[gi]; v.a[2] = D.fg[gi]; v.a[3] = D.og[gi];
+                v.pat = p.pat[t * S + s];
             }
-            if (flags & 2) D.c[gi] = res[b][R_C][lane];
-            const float hval = res[b][R_H][lane];
-            D.h[gi] = hval;
-            if (p.out) p.out[((size_t)t * S + s) * p.L + dir * H + j0 + cj] = hval;
         };
-        auto run_step = [&](const int step, StepIn &far, const StepIn &near) __attribute__((always_inline)) -> bool {
-            lds_barrier();  // results of step-1 and the recurrent sums of this step are in LDS
-            if (wait_failed) return false;
-            wait_all_vmem();  // whatever is still in flight was issued a step ago
-            load_step(step + 2, far);
-            if (step + 1 < T) put_pre(step + 1, near);
-            if (step > 0) store_results(step - 1);
-            return true;
+        auto put_batch = [&](int first, const StepIn (&in)[SETS]) {
+#pragma unroll
+            for (int i = 0; i < SETS; ++i) {
+                const int step = first + i * STEPS + ahead;
+                if (step >= T) continue;
+                *reinterpret_cast<f32x4 *>(pre[step % RING][el]) = f32x4{in[i].a[0], in[i].a[1], in[i].a[2], in[i].a[3]};
+                pre_dummy[step % RING][el] = slot_of(step) >= p.Tmin && in[i].pat == 0 ? 1 : 0;
+            }
         };
-        StepIn in_a, in_b;
-        load_step(0, in_a);
-        load_step(1, in_b);
-        put_pre(0, in_a);
+        StepIn in[SETS];
+        load_batch(0, in);
+        wait_all_vmem();
+        put_batch(0, in);
         lds_barrier();  // start of the recursion
-        for (int step = 0; step < T; step += 2) {
-            if (!run_step(step, in_a, in_b)) return;
-            if (step + 1 < T && !run_step(step + 1, in_b, in_a)) return;
+        for (int step = 0; step < T; ++step) {
+            lds_barrier();
+            if (given_up()) return;
+            const int phase = step % BATCH, next = step - phase + BATCH;
+            if (phase == 0) {
+                for (int d = 0; d < p.mem_delay_fwd; ++d) __builtin_amdgcn_s_sleep(1);
+                load_batch(next, in);
+            } else if (phase == BATCH / 2) {
+                wait_all_vmem();  // requested two steps ago or more
+                put_batch(next, in);
+            }
         }
-        lds_barrier();  // results of the last step
-        if (wait_failed) return;
-        store_results(T - 1);
         return;
     }
 
-    if (wave == PW) {
-        // ------------------------------------------------------------------ cell wave
-        const int cs = lane / JB, cj = lane % JB;
-        const bool cell_lane = lane < EL;
-        const bool cell_valid = cell_lane && cs < nseq && j0 + cj < H;
-        float b_ni = 0, b_ig = 0, b_fg = 0, b_og = 0, p_ig = 0, p_fg = 0, p_og = 0;
-        if (cell_valid) {
-            b_ni = p.bias * D.b[0][j0 + cj]; b_ig = p.bias * D.b[1][j0 + cj];
-            b_fg = p.bias * D.b[2][j0 + cj]; b_og = p.bias * D.b[3][j0 + cj];
-            p_ig = D.peep[0][j0 + cj]; p_fg = D.peep[1][j0 + cj]; p_og = D.peep[2][j0 + cj];
-        }
-        // publishing role: lane l writes chunk l % CH (cells 4*half .. + 3 of one sequence) into the blocks of the
-        // receivers l / CH + (64 / CH) * i
-        const int ch = lane % CH, ch_half = ch / NSQ, ch_seq = ch % NSQ;
-        const unsigned pub_off = (((unsigned)(lane / CH)) * RECV + (unsigned)me * PAIR + (unsigned)ch * 4u) * 4u;
-        const unsigned pub_stride = (unsigned)RPS * RECV * 4u;
-        const int pub_last = G - (PUB - 1) * RPS;   // receivers of the last store
-        const unsigned reset_off = ((unsigned)me * RECV + (unsigned)lane * 4u) * 4u;
-        float c_prev = 0.0f;
-        wait_all_vmem();
+    if (wave == PW + CW + 1) {
+        // ------------------------------------------------------------------ store wave
+        const int s = seq0 + cs, el = (cj / 4 * NSQ + cs) * 4 + cj % 4;
+        f32x4 g = {0, 0, 0, 0}, r = {0, 0, 0, 0};
         lds_barrier();  // start of the recursion
+        lds_barrier();  // the first step's sums
         for (int step = 0; step < T; ++step) {
-            const bool first = (step == 0);
-            const int b = step & 1;
-            lds_barrier();
-            if (wait_failed) return;
-            // stores of the previous step (publication, reset) are complete before this step publishes
-            wait_all_vmem();
-            float hval = 0.0f;
-            if (cell_lane) {
-                float a_ni = pre[b][0][lane], a_ig = pre[b][1][lane], a_fg = pre[b][2][lane], a_og = pre[b][3][lane];
-                if (!first) {
-#pragma unroll
-                    for (int w = 0; w < PW; ++w) {
-                        a_ni += red[b][w][0 * JB + cj][cs]; a_ig += red[b][w][1 * JB + cj][cs];
-                        a_fg += red[b][w][2 * JB + cj][cs]; a_og += red[b][w][3 * JB + cj][cs];
-                    }
+            const int b = step & 1, held = step % STEPS;
+            lds_barrier();  // results of this step are in LDS
+            if (given_up()) return;
+            if (ahead == held) {
+                g = *reinterpret_cast<const f32x4 *>(res_gate[b][el]);
+                r = *reinterpret_cast<const f32x4 *>(res[b][el]);
+            }
+            wait_all_vmem();  // the stores of the step before are done
+            if ((held == STEPS - 1 || step == T - 1) && valid && ahead <= held) {
+                // An access stores as many steps as it has lanes for.  A padding slot keeps its summed pre-activations, and its
+                // cell state unless the direction is the time-reversed one (the reference clears it there).
+                const int mine = step - held + ahead, t = slot_of(mine);
+                const bool pad = r[2] != 0.0f;
+                const size_t gi = (size_t)t * n + (size_t)s * H + j0 + cj;
+                if (!pad || mine > 0) {
+                    D.ni[gi] = g[0]; D.ig[gi] = g[1]; D.fg[gi] = g[2]; D.og[gi] = g[3];
                 }
-                int flags;
-                if (pre_dummy[b][lane]) {
-                    // the reference leaves the summed pre-activations in place on padding slots, clears the cell only
-                    // in the time-reversed direction and emits a zero output
-                    res[b][R_NI][lane] = a_ni; res[b][R_IG][lane] = a_ig; res[b][R_FG][lane] = a_fg; res[b][R_OG][lane] = a_og;
-                    res[b][R_C][lane] = 0.0f;
-                    flags = (first ? 0 : 1) | (dir ? 2 : 0);
-                    if (dir) c_prev = 0.0f;
-                } else {
-                    float x_ni = a_ni + b_ni, x_ig = a_ig + b_ig, x_fg = a_fg + b_fg, x_og = a_og + b_og;
-                    if (!first) { x_ig += c_prev * p_ig; x_fg += c_prev * p_fg; }
-                    const float ni = tanh_quick(x_ni), ig = logistic_quick(x_ig), fg = logistic_quick(x_fg);
-                    float c = ni * ig;
-                    if (!first) c += c_prev * fg;
-                    x_og += c * p_og;
-                    const float og = logistic_quick(x_og);
-                    hval = tanh_quick(c) * og;
-                    res[b][R_NI][lane] = ni; res[b][R_IG][lane] = ig; res[b][R_FG][lane] = fg; res[b][R_OG][lane] = og;
-                    res[b][R_C][lane] = c;
-                    flags = 3;
-                    c_prev = c;
-                }
-                if (!cell_valid) hval = 0.0f;
-                res[b][R_H][lane] = hval;
-                res_flags[b][lane] = flags;
-                hpub[cs][cj] = hval;
+                if (!pad || dir) D.c[gi] = r[0];
+                D.h[gi] = r[1];
+                if (p.out) p.out[((size_t)t * S + s) * p.L + dir * H + j0 + cj] = r[1];
             }
             if (step + 1 < T) {
-                // the wave's own LDS writes above are visible to all of its lanes
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                u32x4 v = *reinterpret_cast<const u32x4 *>(&hpub[ch_seq][4 * ch_half]);
-                v.x = v.x == kEmpty ? 0x7FC00000u : v.x; v.y = v.y == kEmpty ? 0x7FC00000u : v.y;
-                v.z = v.z == kEmpty ? 0x7FC00000u : v.z; v.w = v.w == kEmpty ? 0x7FC00000u : v.w;
-#pragma unroll
-                for (int i = 0; i < PUB; ++i)
-                    if (i + 1 < PUB || lane / CH < pub_last)
-                        __builtin_amdgcn_raw_buffer_store_b128(v, mail, (int)((unsigned)(step % kMailSlots) * slot_words * 4u + pub_off + (unsigned)i * pub_stride), 0, 0);
-            }
-            if (step > 0) {
-                // the words the gather waves read for this step are empty again
+                // the words the gather waves have read for the next step are empty again
                 const u32x4 empty = {kEmpty, kEmpty, kEmpty, kEmpty};
 #pragma unroll
                 for (int q = 0; q < NQ; ++q)
-                    if (q + 1 < NQ || lane < vectors - 64 * (NQ - 1))
-                        __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)((step - 1) % kMailSlots) * slot_words * 4u + reset_off + (unsigned)q * 1024u), 0, 0);
+                    if (q * 64 + lane < vectors)
+                        __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)(step % kMailSlots) * slot_words * 4u +
+                                                               ((unsigned)me * RECV + (unsigned)(q * 64 + lane) * 4u) * 4u), 0, 0);
             }
+        }
+        return;
+    }
+
+    if (wave >= PW) {
+        // ------------------------------------------------------------------ cell waves
+        const int cw = wave - PW;
+        const int row = lane >> 4, q = cw * VPW + row % VPW;  // vector of the message: four cells of a sequence
+        const int el = 4 * q + (lane >> 2 & 3), gate = lane & 3;
+        const int cell = q / NSQ * 4 + (lane >> 2 & 3), seq = q % NSQ;
+        const bool cell_valid = seq < nseq && j0 + cell < H;
+        float bias = 0, peep = 0, p_og = 0;
+        if (cell_valid) {
+            bias = p.bias * D.b[gate][j0 + cell];
+            if (gate == 1 || gate == 2) peep = D.peep[gate - 1][j0 + cell];
+            p_og = D.peep[2][j0 + cell];
+        }
+        const bool peeps = gate == 1 || gate == 2, is_tanh = gate == 0;
+        // tanh_quick for the lanes of the cell input, logistic_quick for the others
+        const float lo = is_tanh ? -43.65f : -87.3f, hi = is_tanh ? 44.361415f : 88.72283f;
+        const float log2e = is_tanh ? 2.88539008177792681f : 1.44269504088896341f;
+        const float log2e_rest = is_tanh ? 3.85192606e-8f : 1.92596303e-8f;
+        const float times = is_tanh ? 2.0f : 1.0f, plus = is_tanh ? -1.0f : 0.0f;
+        auto gate_fn = [&](float x) __attribute__((always_inline)) {
+            return __builtin_fmaf(times, logistic_of_negative<false>(__builtin_amdgcn_fmed3f(-x, lo, hi), log2e, log2e_rest), plus);
+        };
+        auto of_gate = [](float v, auto g) __attribute__((always_inline)) {
+            constexpr int k = decltype(g)::value;
+            return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), k * 0x55, 0xF, 0xF, true));
+        };
+        const std::integral_constant<int, 0> c0; const std::integral_constant<int, 1> c1;
+        const std::integral_constant<int, 2> c2; const std::integral_constant<int, 3> c3;
+        // publishing role: vector lane % VPW of the wave's goes into the blocks of the receivers lane / VPW + 64 / VPW * i
+        const int first_receiver = lane / VPW;
+        const unsigned pub_off = ((unsigned)first_receiver * RECV + (unsigned)me * EL + (unsigned)(cw * VPW + lane % VPW) * 4u) * 4u;
+        const unsigned pub_stride = (unsigned)(64 / VPW) * RECV * 4u;
+        float *const my_h = &hpub[cw][row % VPW][lane >> 2 & 3];
+        const float *const sent = hpub[cw][lane % VPW];
+        const float *const my_red = &red[0][0][cell * 4 + gate][seq];
+        float c_prev = 0.0f, start = bias;
+        wait_all_vmem();
+        lds_barrier();  // start of the recursion
+        for (int step = 0; step < T; ++step) {
+            const int b = step & 1;
+            lds_barrier();
+            // (looked at at the end of the step: what a step that failed publishes no longer matters)
+            const int failed = given_up();
+            float a = pre[step % RING][el][gate];
+            int padding = pre_dummy[step % RING][el];
+            asm volatile("" : "+v"(padding));  // read here, with the sums: the compiler would read it between the gates and wait there
+            const bool dummy = padding != 0;
+            if (step > 0) {
+                float share[PW];
+#pragma unroll
+                for (int w = 0; w < PW; ++w) share[w] = my_red[(size_t)(b * PW + w) * ROWS * NSQ];
+#pragma unroll
+                for (int w = 0; w + 1 < PW; w += 2) share[w / 2] = share[w] + share[w + 1];
+                if (PW % 2) share[PW / 2] = share[PW - 1];
+#pragma unroll
+                for (int w = 0; w < (PW + 1) / 2; ++w) a += share[w];
+            }
+            const float x0 = a + start, v1 = gate_fn(x0);
+            float c = of_gate(v1, c0) * of_gate(v1, c1) + c_prev * of_gate(v1, c2);
+            // second pass: tanh(c) in the lanes of the cell input, the output gate in its own
+            const float v2 = gate_fn(is_tanh ? c : x0 + c * p_og);
+            float hval = of_gate(v2, c0) * of_gate(v2, c3);
+            hval = dummy || !cell_valid ? 0.0f : hval;
+            // the publication of the previous step is complete before this step publishes
+            wait_all_vmem();
+            if (step + 1 < T) {
+                // through LDS, so that neighbouring lanes hold what goes into one receiver's block
+                *my_h = __builtin_bit_cast(float, publishable(hval));
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                const u32x4 v = *reinterpret_cast<const u32x4 *>(sent);
+#pragma unroll
+                for (int i = 0; i < PUB; ++i)
+                    if (first_receiver + 64 / VPW * i < G)
+                        __builtin_amdgcn_raw_buffer_store_b128(v, mail, (int)((unsigned)(step % kMailSlots) * slot_words * 4u + pub_off + (unsigned)i * pub_stride), 0, 0);
+            }
+            c = dummy ? 0.0f : c;
+            if (row < VPW) {
+                // on a padding slot the reference leaves the summed pre-activations in place, clears the cell only in the
+                // time-reversed direction and emits a zero output
+                res_gate[b][el][gate] = dummy ? a : gate == 3 ? v2 : v1;
+                if (gate < 3) res[b][el][gate] = gate == 0 ? c : gate == 1 ? hval : dummy ? 1.0f : 0.0f;
+            }
+            c_prev = dummy && !dir ? c_prev : c;
+            start = peeps ? bias + c_prev * peep : bias;
+            if (failed) return;
         }
         lds_barrier();  // results of the last step are in LDS
         return;
     }
 
     // ---------------------------------------------------------------------- gather waves
-    // Wave pw takes the source cells 64*pw .. 64*pw + 63 for ALL of the workgroup's rows.  MFMA blocks: block = kq * RG + rg
-    // multiplies the four rows 4*rg .. + 3 with the kq-th run of NI source cells (cell = NI * kq + i in instruction i), so
-    // the sum over a block's cells happens inside the accumulator and only the KQ runs meet across lanes afterwards.  A
-    // lane's polled vector (four neighbouring cells of one sequence) goes to LDS as it is, and a lane's B operands are
-    // NI neighbouring cells of its sequence: 16-byte LDS accesses on both sides.
+    // Wave pw takes the source cells 64*pw .. 64*pw + 63 for ALL of the workgroup's rows; with 32 rows each half of the wave
+    // takes 32 of them, and the two halves' sums meet at the end.
     const int pw = wave;
-    constexpr int RG = ROWS / 4;         // groups of four rows
-    constexpr int KQ = 16 / RG;          // residues of the source cell index dealt to the blocks
-    constexpr int NI = 64 / KQ;          // MFMA instructions per step
-    static_assert(RG * KQ == 16 && (KQ == 1 || KQ == 2 || KQ == 4), "blocks of the recurrent product");
-    const int blk = lane >> 2, sub = lane & 3;  // A operand: row sub of the block; B operand and accumulator: sequence sub
-    const int rg = blk % RG, kq = blk / RG;
-    float wreg[NI];
+    constexpr int HALVES = 64 / ROWS;    // parts of the wave with source cells of their own
+    constexpr int BLOCKS = 16 / HALVES;  // blocks of the A operand (four source cells each) of a part
+    float wreg[4 * BLOCKS];
     {
-        const int o = rg * 4 + sub, g = o / JB, jj = o % JB;
+        const int o = lane % ROWS, g = o % 4, jj = o / 4;
         const float *wg = D.w_int + (size_t)g * p.L * H + (size_t)(j0 + jj) * H;
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int from = 64 * pw + NI * kq + i;
+        for (int i = 0; i < 4 * BLOCKS; ++i) {
+            const int from = 64 * pw + 4 * BLOCKS * (lane / ROWS) + i;
             wreg[i] = from < H && j0 + jj < H ? wg[from] : 0.0f;
         }
     }
-    // the wave's own staging buffer: [sequence][cell], written as the words arrive, read back as B operands
-    float (*hb)[64 + 4] = hstage[pw];
-    // a lane past the end of the block polls its wave's first vector instead and stages zeros
-    const bool inside = 64 * pw + lane < vectors;
-    const unsigned poll_off = ((unsigned)me * RECV + (unsigned)(64 * pw + (inside ? lane : 0)) * 4u) * 4u;
-    long long ph0 = 0, ph1 = 0, ph2 = 0, ph3 = 0, poll_rounds = 0;
-    const bool timing = p.phase_ticks != nullptr && blockIdx.x < kTraceBlocks;
-    const long long tk_begin = timing ? wall_clock64() : 0;
+    // a lane past the end of the block polls the block's first vector instead and multiplies zeros
+    const int my_vec = (16 * pw + (lane >> 2)) * NSQ + (lane & 3) % NSQ;
+    const bool inside = my_vec < vectors;
+    const unsigned poll_off = ((unsigned)me * RECV + (unsigned)(inside ? my_vec : 0) * 4u) * 4u;
     wait_all_vmem();
     lds_barrier();  // start of the recursion
     lds_barrier();  // step 0 has nothing to gather
 
     for (int step = 1; step < T; ++step) {
-        const long long tk0 = timing ? wall_clock64() : 0;
         const float *slot = mailbox + (size_t)((step - 1) % kMailSlots) * slot_words;
         bool ok = true;
         u32x4 w[1];
@@ -263,7 +294,6 @@ __global__ __launch_bounds__(local_threads(PW)) void lstm_forward_local(const Ch
         for (;;) {
             poll_load<1>(slot, poll_off, 0u, poll_off, w);
             const unsigned worst = max(max(w[0].x, w[0].y), max(w[0].z, w[0].w));
-            if (timing) ++poll_rounds;
             if (worst != kEmpty) break;
             if (++spins > p.spin_limit) { ok = false; break; }
             if ((spins & 255u) == 0u &&
@@ -273,56 +303,27 @@ __global__ __launch_bounds__(local_threads(PW)) void lstm_forward_local(const Ch
             }
             for (int d = 0; d < p.poll_gap; ++d) __builtin_amdgcn_s_sleep(1);
         }
-        if (timing) ph1 += wall_clock64() - tk0;
-        // this lane's vector: sequence sub, source cells 4*blk .. + 3 of the wave's 64
         if (!inside) w[0] = u32x4{0, 0, 0, 0};
-        *reinterpret_cast<f32x4 *>(&hb[sub][4 * blk]) = __builtin_bit_cast(f32x4, w[0]);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        f32x4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
+        f32x4 sum = local_product<JB == 8 ? 3 : 4, 4 * BLOCKS>(__builtin_bit_cast(f32x4, w[0]), wreg, std::make_integer_sequence<int, BLOCKS>{});
+        // register = sequence; where the wave's halves meet, the lower one ends up with the first half of the sequences
+        float *const out = &red[step & 1][pw][lane % ROWS][0];
+        if constexpr (HALVES == 1) {
 #pragma unroll
-        for (int i4 = 0; i4 < NI; i4 += 4) {
-            const f32x4 hv = *reinterpret_cast<const f32x4 *>(&hb[sub][NI * kq + i4]);
-            acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(wreg[i4 + 0], hv[0], acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(wreg[i4 + 1], hv[1], acc1, 0, 0, 0);
-            acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(wreg[i4 + 2], hv[2], acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(wreg[i4 + 3], hv[3], acc1, 0, 0, 0);
-        }
-        f32x4 sum = acc0 + acc1;
-        // the residues sit in lane bits 4 and 5 (KQ = 4), in lane bit 5 (KQ = 2), or there is only one (KQ = 1)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            float v = sum[r];
-            if (KQ == 4) {
-                const unsigned u = __builtin_bit_cast(unsigned, v);
-                const auto x = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-                v = __builtin_bit_cast(float, (unsigned)x[0]) + __builtin_bit_cast(float, (unsigned)x[1]);
-            }
-            if (KQ >= 2) {
-                const unsigned u = __builtin_bit_cast(unsigned, v);
-                const auto x = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-                v = __builtin_bit_cast(float, (unsigned)x[0]) + __builtin_bit_cast(float, (unsigned)x[1]);
-            }
-            sum[r] = v;
-        }
-        if (kq == 0) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) red[step & 1][pw][rg * 4 + r][sub] = sum[r];
+            for (int r = 0; r < NSQ; ++r) out[r] = sum[r];
+        } else if constexpr (NSQ == 4) {
+            const float lower = sum_halves(sum[0], sum[2]), upper = sum_halves(sum[1], sum[3]);
+            out[lane / ROWS * 2] = lower; out[lane / ROWS * 2 + 1] = upper;
+        } else if constexpr (NSQ == 2) {
+            out[lane / ROWS] = sum_halves(sum[0], sum[1]);
+        } else {
+            out[0] = sum_halves(sum[0], sum[0]);
         }
         if (__builtin_amdgcn_ballot_w64(!ok) != 0) wait_failed = 1;
-        const long long tk2 = timing ? wall_clock64() : 0;
         lds_barrier();
-        if (timing) ph2 += wall_clock64() - tk2;
-        if (wait_failed) {
+        if (given_up()) {
             if (tid == 0) raise_abort(p);
             return;
         }
-        if (timing) ph0 += wall_clock64() - tk0;
     }
     lds_barrier();  // results of the last step
-    if (timing) ph3 = wall_clock64() - tk_begin;
-    if (timing && tid == 0) {
-        long long *o = p.phase_ticks + (size_t)blockIdx.x * 6;
-        o[0] = ph0; o[1] = ph1; o[2] = ph2; o[3] = ph3; o[4] = poll_rounds;
-    }
 }

@@ -532,6 +532,27 @@ def test_lstm_recursion_geometries(L, bidir, lengths):
     assert PC.run_lstm_two_recursions(19, L, bidir, lengths, seed=L + len(lengths)) < TOL
 
 
+@pytest.mark.parametrize("T", [1, 2, 3, 5, 8, 9, 17])
+@pytest.mark.parametrize("L,bidir,S", [
+    (256, True, 3), (300, True, 4), (70, False, 1),       # jobs of one sequence, 8 cells per workgroup
+    (400, True, 7), (130, False, 9),                      # of one and two
+    (512, True, 9), (200, False, 21),                     # of two and three
+    (300, False, 5), (258, False, 11), (480, False, 30),  # 16 cells per workgroup: one, one and two, three and four
+])
+def test_lstm_job_sizes_and_batches_of_steps(L, bidir, S, T):
+    """Kernels for jobs of one, two and up to four sequences, at step counts around the batches in which their inputs are
+    requested (four or eight steps) and their results stored (one to eight): ragged lengths, both directions."""
+    print("lstm jobs", L, bidir, S, T, flush=True)
+    lengths = [max(1, T - 3 * i % 4) for i in range(S)]
+    assert PC.run_lstm_two_recursions(19, L, bidir, lengths, seed=L + S + T) < TOL
+
+
+@pytest.mark.parametrize("L,bidir,S,T,cuts", [(512, True, 3, 26, [3, 8, 17]), (256, True, 8, 14, [1, 2, 7]), (400, False, 20, 11, [2, 6])])
+def test_lstm_recursion_resumes_between_batches_of_steps(L, bidir, S, T, cuts):
+    """Cuts inside the batches of steps whose inputs are requested and results stored together."""
+    test_lstm_recursion_in_several_launches_is_the_same_recursion(L, bidir, S, T, cuts)
+
+
 def _product(m, n, k, tA, tB, A, B):
     import torch
     C = torch.empty(m * n, device="cuda")
