@@ -217,6 +217,10 @@ struct GemmArgs {
 // EPI_ATOMIC product to EPI_PARTIAL.  A caller that needs to know whether C must be cleared first calls this
 // before gemm_launch and looks at args.epilogue; gemm_launch calls it for everyone else.
 void gemm_plan(GemmArgs &args, hipStream_t stream);
+// The kernel for products that are too small for the tiled one (gemm_direct.hip): whether these arguments take it (masked
+// products never do), and its launch
+bool direct_product(const GemmArgs &args);
+void gemm_direct_launch(const GemmArgs &args, hipStream_t stream);
 // whether a product with these operands can take the EPI_FAN epilogue (operand kinds, alignment)
 bool gemm_fan_supported(const GemmArgs &args);
 int gemm_launch(hipStream_t stream, const GemmArgs &args);

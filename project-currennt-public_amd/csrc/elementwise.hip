@@ -357,7 +357,7 @@ extern "C++" int cnt::dense_backward_weights_batch(hipStream_t stream, int P, in
     ga.overwrite_ok = 1;
     ga.rowsum = 1;
     gemm_plan(ga, stream);
-    if (ga.epilogue == EPI_PARTIAL) return gemm_launch(stream, ga);
+    if (ga.epilogue != EPI_ATOMIC) return gemm_launch(stream, ga);
     for (int z = 0; z < count; ++z) CNT_TRY(fill_zero(stream, weight_updates[z], (size_t)P * D + D));
     CNT_TRY(gemm_launch(stream, ga));
     for (int z = 0; z < count; ++z)

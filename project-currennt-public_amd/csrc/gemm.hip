@@ -237,6 +237,13 @@ int gemm_scratch_buffers() {
 
 void gemm_plan(GemmArgs &args, hipStream_t stream) {
     if (args.splitk != 0) return;
+    if (direct_product(args)) {
+        // one workgroup sums over all of k: nothing to add to, and the row sums come along
+        args.splitk = 1;
+        if (args.epilogue == EPI_ATOMIC && args.overwrite_ok) args.epilogue = EPI_STORE;
+        else args.rowsum = 0;
+        return;
+    }
     // Long-K products with a small output (weight gradients): cut K so that the launch has about
     // `target` workgroups of 64 x 64 tiles, but leave every workgroup at least eight k-iterations -- each
     // one ends with an atomic add (or a store) of its whole tile, and those, not the products, dominate short
@@ -317,10 +324,16 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
         vb = (args.b_kcontig ? args.k : args.n) % 4 == 0 ? 4 : 1;
     }
     gemm_plan(args, stream);
-    if (args.epilogue != EPI_PARTIAL) args.rowsum = 0;
-    const int tile = pick_tile(args);
     static const bool use_lines = [] { const char *e = std::getenv("CNT_GEMM_K_ORDER"); return !e || std::atoi(e) != 0; }();
     if (!use_lines) args.k_order = nullptr;
+    if (args.splitk == 1 && args.epilogue != EPI_PARTIAL && direct_product(args)) {
+        ProfileScope prof(stream, args.label ? args.label : "gemm");
+        gemm_direct_launch(args, stream);
+        CNT_HIP(hipGetLastError());
+        return CNT_OK;
+    }
+    if (args.epilogue != EPI_PARTIAL) args.rowsum = 0;
+    const int tile = pick_tile(args);
     // a list of k lines is used where the kernel that reads through it exists, and ignored otherwise (the lines it leaves
     // out are zero)
     if (args.k_order && !(args.k_count && !args.masked && !args.a_kcontig && !args.b_kcontig && aligned &&
@@ -374,6 +387,11 @@ int gemm_dense_weights_static(hipStream_t stream, int P, int D, int N, float bia
     ga.prob[0].rowsum_scale = bias;
     ga.label = "gemm:dense_dW_static";
     ga.rowsum = 1;
+    if (direct_product(ga)) {
+        ga.splitk = 1;
+        ga.epilogue = EPI_STORE;
+        return gemm_launch(stream, ga);
+    }
     // as many splits as the usual plan takes, as far as their partial products fit into the array
     GemmArgs probe = ga;
     probe.epilogue = EPI_ATOMIC; probe.splitk = 0; probe.overwrite_ok = 0;

@@ -587,6 +587,46 @@ def test_matrix_product_is_as_exact_as_fp32_sums(m, n, k, tA, tB):
     assert bool(((C - A64 @ B64).abs() <= bound).all())
 
 
+# products of few blocks: eight waves share k in steps of sixteen; blocks and k around 32, 16 and 128, fewer rows than a vector,
+# the last sizes before the tiled kernel takes over (640 blocks) and the first behind them
+@pytest.mark.parametrize("tA,tB", [(True, False), (False, False), (False, True)])
+@pytest.mark.parametrize("m,n,k", [
+    (32, 32, 16), (33, 31, 15), (31, 35, 17), (34, 66, 127), (65, 32, 128), (5, 97, 129), (4, 4, 257), (36, 29, 143), (3, 70, 300), (70, 2, 33),
+    (640, 1024, 40), (641, 1023, 41), (640, 1025, 24), (96, 100, 2100),
+])
+def test_matrix_product_of_few_blocks(m, n, k, tA, tB):
+    """Bound of an fp32 product in any order of its sums, as above; infinite and missing values in two rows give what a sum of
+    single terms gives."""
+    import torch
+    test_matrix_product_is_as_exact_as_fp32_sums(m, n, k, tA, tB)
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    A, B = torch.randn(m * k, device="cuda", generator=g), torch.randn(n * k, device="cuda", generator=g)
+    row = (lambda i, q: i * k + q) if tA else (lambda i, q: q * m + i)
+    A[row(0, k - 1)], A[row(m - 1, k // 2)] = float("inf"), float("nan")
+    C, A64, B64 = _product(m, n, k, tA, tB, A, B)
+    assert bool(C[m - 1].isnan().all())
+    assert torch.equal(C[0].isposinf(), B64[k - 1] > 0) and torch.equal(C[0].isneginf(), B64[k - 1] < 0)
+    bound = (k + 2) * 2.0 ** -24 * (A64.abs() @ B64.abs())
+    assert bool(((C - A64 @ B64).abs() <= bound)[1:m - 1].all())
+
+
+@pytest.mark.parametrize("static", [False, True])
+@pytest.mark.parametrize("P,D,N", [(32, 32, 16), (20, 33, 120), (37, 35, 130), (5, 4, 7), (3, 60, 200), (60, 2, 200), (256, 2048, 100), (288, 2048, 100),
+                                   (100, 90, 2048), (100, 90, 2049)])
+def test_weight_gradient_of_few_blocks(P, D, N, static):
+    """Both sides of the line between the kernel that sums over all slots in one workgroup, bias gradient included, and
+    the one that cuts them (512 blocks, 2048 slots); rows at the edge of a block whose vectors overlap."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(P + D + N)
+    x, err = torch.randn(N, P, device="cuda", generator=g), torch.randn(N, D, device="cuda", generator=g)
+    dW = torch.full((P * D + D,), 3.0, device="cuda")
+    capi = PC.pkg().capi
+    (capi.dense_backward_weights_static if static else capi.dense_backward_weights)(P, D, N, 0.5, x, err, dW)
+    want, size = err.double().t() @ x.double(), err.double().abs().t() @ x.double().abs()
+    assert bool(((dW[:P * D].view(D, P) - want).abs() <= (N + 2) * 2.0 ** -24 * size).all())
+    assert bool(((dW[P * D:] - 0.5 * err.double().sum(0)).abs() <= (N + 2) * 2.0 ** -24 * 0.5 * err.double().abs().sum(0)).all())
+
+
 @pytest.mark.parametrize("m,n,k,tA,tB", [(70, 66, 37, True, False), (3100, 3076, 516, False, False)])
 def test_matrix_product_of_infinite_huge_and_missing_values(m, n, k, tA, tB):
     """Values that have no finite bf16 parts give what fp32 arithmetic gives."""
