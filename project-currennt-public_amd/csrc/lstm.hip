@@ -547,16 +547,17 @@ chain_kernel_t pick_local_kernel(bool fwd, int H, int JB, int nsq) {
     return nullptr;
 }
 
-template <int NW>
+template <int NW, int CELLS>
 chain_kernel_t solo_pair(bool fwd) {
-    return fwd ? (chain_kernel_t)lstm_forward_solo<NW> : (chain_kernel_t)lstm_backward_solo<NW>;
+    return fwd ? (chain_kernel_t)lstm_forward_solo<NW, CELLS> : (chain_kernel_t)lstm_backward_solo<NW, CELLS>;
 }
 chain_kernel_t pick_solo_kernel(bool fwd, int H) {
+    const bool aligned = H % 4 == 0;
     switch ((H + 15) / 16) {
-        case 1: return solo_pair<1>(fwd);
-        case 2: return solo_pair<2>(fwd);
-        case 3: return solo_pair<3>(fwd);
-        case 4: return solo_pair<4>(fwd);
+        case 1: return H < 4 ? solo_pair<1, kSingle>(fwd) : aligned ? solo_pair<1, kAligned>(fwd) : solo_pair<1, kOverlapping>(fwd);
+        case 2: return aligned ? solo_pair<2, kAligned>(fwd) : solo_pair<2, kOverlapping>(fwd);
+        case 3: return aligned ? solo_pair<3, kAligned>(fwd) : solo_pair<3, kOverlapping>(fwd);
+        case 4: return aligned ? solo_pair<4, kAligned>(fwd) : solo_pair<4, kOverlapping>(fwd);
     }
     return nullptr;
 }

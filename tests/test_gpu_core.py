@@ -547,6 +547,15 @@ def test_lstm_job_sizes_and_batches_of_steps(L, bidir, S, T):
     assert PC.run_lstm_two_recursions(19, L, bidir, lengths, seed=L + S + T) < TOL
 
 
+@pytest.mark.parametrize("H", [1, 3, 4, 5, 18, 31, 47, 50, 61])
+@pytest.mark.parametrize("bidir,lengths", [(True, [9, 4, 6]), (False, [1]), (True, [5, 5, 2, 5, 3]), (False, [13, 2])])
+def test_lstm_small_layers_move_their_cells_in_vectors(H, bidir, lengths):
+    """One-workgroup recursions whose cells are no multiple of four: the last vector overlaps the one before it, below four
+    cells there are no vectors."""
+    print("lstm small", H, bidir, lengths, flush=True)
+    assert PC.run_lstm_two_recursions(11, H * (2 if bidir else 1), bidir, lengths, seed=H + len(lengths)) < TOL
+
+
 @pytest.mark.parametrize("L,bidir,S,T,cuts", [(512, True, 3, 26, [3, 8, 17]), (256, True, 8, 14, [1, 2, 7]), (400, False, 20, 11, [2, 6])])
 def test_lstm_recursion_resumes_between_batches_of_steps(L, bidir, S, T, cuts):
     """Cuts inside the batches of steps whose inputs are requested and results stored together."""
