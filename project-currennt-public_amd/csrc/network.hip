@@ -229,6 +229,8 @@ struct NetLayer {
     const float **in_ptrs = nullptr;         // skip layers: device tables
     float **tgt_ptrs = nullptr;
     int *tgt_is_skip = nullptr;
+    int side = -1;                           // skip layers: index of the side buffer in cnt_network::sides
+    std::vector<int> side_targets;           // skip layers: side buffers this layer's step adds to
     bool ptrs_aligned = false;               // every buffer the skip kernels touch for this layer is 16-byte aligned
     long weight_count() const { return n_in + n_bias + n_int; }
 };
@@ -296,6 +298,34 @@ __global__ void feedback_kernel(size_t count, int dim_out, int d1, int prev_tota
             v = (cls == d - d1) ? 1.0f : 0.0f;
         }
         out[i] = v;
+    }
+}
+
+// The same with 16-byte stores (dim_out a multiple of four, `out` 16-byte aligned).  Bound by the stores, so a thread
+// should cost little else: 2^lanes_log2 neighbouring lanes take one slot, its class is read once and no index is
+// divided.  32 000 slots of 1024 dimensions (131 MB): 19-28 us, 82 us for the kernel above with its element per thread,
+// which is left for the other sizes.
+__global__ __launch_bounds__(256) void feedback_vec4_kernel(int N, int dim_out, int d1, int prev_total, int prev_start, int S,
+                                                            int target_dim, int target_start, int lanes_log2,
+                                                            const char *__restrict__ pat, const float *__restrict__ prev_out,
+                                                            const float *__restrict__ targets, float *__restrict__ out) {
+    const int lane = threadIdx.x & ((1 << lanes_log2) - 1), per_block = 256 >> lanes_log2;
+    for (int slot = blockIdx.x * per_block + (threadIdx.x >> lanes_log2); slot < N; slot += gridDim.x * per_block) {
+        const int before = max(slot - S, 0);
+        const int cls = (int)targets[(size_t)before * target_dim + target_start];
+        const int one = slot >= S && pat[before] != 0 ? cls : -1;  // -1: no class
+        const float *from = prev_out + (size_t)slot * prev_total + prev_start;
+        float4 *to = reinterpret_cast<float4 *>(out + (size_t)slot * dim_out);
+        for (int d = 4 * lane; d < dim_out; d += 4 << lanes_log2) {
+            float4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+            float *e = reinterpret_cast<float *>(&v);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (d + q < d1) e[q] = from[d + q];
+                else if (d + q - d1 == one) e[q] = 1.0f;
+            }
+            to[d / 4] = v;
+        }
     }
 }
 
@@ -459,8 +489,13 @@ struct cnt_network {
     const char *pat = nullptr;
     long n_weights = 0;
     float *weights = nullptr, *updates = nullptr;
-    float *skip_errors = nullptr;  // err and eskip of every skip layer, one allocation
-    size_t skip_error_count = 0;
+    // err and eskip of every skip layer, one allocation: first the `skip_always` floats that a forward pass always clears,
+    // then the side buffers, of which it clears those that a backward pass has added to since they were allocated as
+    // zeros, then the errors that the layer behind writes over in every pass
+    float *skip_errors = nullptr;
+    size_t skip_always = 0;
+    struct SideBuffer { size_t end; bool touched; };  // the first begins at skip_always, the others where one ends
+    std::vector<SideBuffer> sides;
     const float *ctx = nullptr;    // conditioning features of the wavnetc layers, C x (maxT*S)
     // conditioning sub-network: the layer flagged "wavenetConditionInputLayer" feeds the wavnetc layers
     int flagged = -1, first_wavnetc = -1;
@@ -880,7 +915,14 @@ int finish_build(cnt_network *net, const json::Value *weights) {
         return !(nx.kind == K_FEEDBACK && nx.fb_end == nx.fb_start);
     };
     std::vector<char> shares(n_layers, 0);  // skip layer that shares its linker's sum
-    size_t skip_total = 0;
+    // the layer behind writes all of a skip layer's errors before anything adds to them or reads them
+    auto written_over = [&](int i) {
+        if (i == net->flagged || i + 1 >= n_layers) return false;
+        const NetLayer &nx = net->layers[(size_t)i + 1];
+        return (nx.kind == K_DENSE || nx.kind == K_LSTM || nx.kind == K_CNN || nx.kind == K_WAVNETC) &&
+               nx.res == net->layers[(size_t)i].res;
+    };
+    size_t skip_always = 0, skip_side = 0, skip_over = 0;
     for (int i = 0; i < n_layers; ++i) {
         NetLayer &L = net->layers[(size_t)i];
         if (!is_skip_kind(L.kind)) continue;
@@ -888,21 +930,26 @@ int finish_build(cnt_network *net, const json::Value *weights) {
         if (L.kind == K_SKIPCAT) links[i] = std::max(links[i], 2);  // always keeps both buffers
         shares[i] = (is_sum_skip(L.kind) && !followed_by_writer(i) && links[i] == 1) ? 1 : 0;
         L.needs_sum = !shares[i] && links[i] > 0;
-        if (!shares[i]) skip_total += (size_t)L.size * lslots * (links[i] > 0 ? 2 : 1);
+        if (shares[i]) continue;
+        (written_over(i) ? skip_over : skip_always) += (size_t)L.size * lslots;
+        if (links[i] > 0) skip_side += (size_t)L.size * lslots;
     }
-    net->skip_error_count = skip_total;
-    if (skip_total) {
-        CNT_TRY(device_alloc(net, (void **)&net->skip_errors, skip_total * sizeof(float), true));
-        size_t at = 0;
+    net->skip_always = skip_always;
+    if (skip_always + skip_side + skip_over) {
+        CNT_TRY(device_alloc(net, (void **)&net->skip_errors, (skip_always + skip_side + skip_over) * sizeof(float), true));
+        size_t at = 0, side_at = skip_always, over_at = skip_always + skip_side;
         for (int i = 0; i < n_layers; ++i) {
             NetLayer &L = net->layers[(size_t)i];
             if (!is_skip_kind(L.kind) || shares[i]) continue;
             const size_t lslots = (size_t)net->S * L.maxTr;
-            L.err = net->skip_errors + at;
-            at += (size_t)L.size * lslots;
+            size_t &err_at = written_over(i) ? over_at : at;
+            L.err = net->skip_errors + err_at;
+            err_at += (size_t)L.size * lslots;
             if (links[i] > 0) {
-                L.eskip = net->skip_errors + at;
-                at += (size_t)L.size * lslots;
+                L.eskip = net->skip_errors + side_at;
+                side_at += (size_t)L.size * lslots;
+                L.side = (int)net->sides.size();
+                net->sides.push_back({side_at, false});
             }
         }
     }
@@ -919,6 +966,10 @@ int finish_build(cnt_network *net, const json::Value *weights) {
     std::vector<int> owner(n_layers, -1);
     for (int i = n_layers - 1; i >= 0; --i)
         if (is_skip_kind(net->layers[(size_t)i].kind)) owner[i] = shares[i] ? owner[linker[i]] : i;
+    for (auto &L : net->layers)
+        if (L.kind == K_SKIPCAT)
+            for (int x : L.pre)
+                if (net->layers[(size_t)x].side >= 0) L.side_targets.push_back(net->layers[(size_t)x].side);
     std::vector<std::vector<float *>> tgt(n_layers);
     std::vector<std::vector<int>> flag(n_layers);
     for (int i = n_layers - 1; i >= 0; --i) {
@@ -939,6 +990,7 @@ int finish_build(cnt_network *net, const json::Value *weights) {
             if (t) {
                 tgt[(size_t)owner[i]].push_back(t);
                 flag[(size_t)owner[i]].push_back(skip);
+                if (skip) net->layers[(size_t)owner[i]].side_targets.push_back(src.side);
             }
         }
     }
@@ -1280,8 +1332,28 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
     CNT_REQUIRE(net && net->T > 0, "network_forward: no fraction loaded");
     CNT_TRY(report_failure(net, static_cast<hipStream_t>(stream_)));
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    // what the skip layers' forward passes clear (layers/SkipAddLayer.cu:195-205)
-    if (net->skip_error_count) CNT_TRY(fill_zero(stream, net->skip_errors, net->skip_error_count));
+    // What the skip layers' forward passes clear (layers/SkipAddLayer.cu:195-205), as far as it matters: not the errors
+    // that the layer behind writes over, and of the side buffers only those that a backward pass has added to -- in a
+    // stack of WaveNet blocks, where the block launches hand the sums on, none (30 blocks of 64 channels on 32 000
+    // samples: 500 MB less to write per pass, 184 us).  A pass under capture may be replayed after backward passes that
+    // are not known yet, so it clears all side buffers.
+    bool all = false;
+    if (!net->sides.empty()) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        all = hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
+    }
+    size_t lo = 0, hi = net->skip_always, at = hi;  // [lo, hi): the run to clear that has not ended yet
+    for (const auto &side : net->sides) {
+        if (all || side.touched) {
+            if (at != hi) {
+                if (hi > lo) CNT_TRY(fill_zero(stream, net->skip_errors + lo, hi - lo));
+                lo = at;
+            }
+            hi = side.end;
+        }
+        at = side.end;
+    }
+    if (hi > lo) CNT_TRY(fill_zero(stream, net->skip_errors + lo, hi - lo));
     static const bool fuse_blocks = [] { const char *e = std::getenv("CNT_NET_FUSE_BLOCKS"); return !e || std::atoi(e) != 0; }();
     // a WaveNet residual block seen from its convolution layer i: [cnn 2R (i)][wavnetc R][dense R, identity]
     // [skipadd of the block's input and that layer][skipini, shares the sum][dense K, identity]
@@ -1381,9 +1453,17 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
             case K_FEEDBACK: {
                 const NetLayer &post = net->layers.back();
                 ProfileScope prof(stream, "feedback");
-                hipLaunchKernelGGL(feedback_kernel, dim3(blocks_for(count)), dim3(256), 0, stream, count, L.size,
-                                   L.fb_end - L.fb_start, prev.size, L.fb_start, net->S, post.size, net->mdn_target_start,
-                                   L.pat, prev.out, post.out, L.out);
+                if (L.size % 4 == 0 && (reinterpret_cast<uintptr_t>(L.out) & 15) == 0) {
+                    int lanes_log2 = 0;
+                    while (lanes_log2 < 6 && (4 << lanes_log2) < L.size) ++lanes_log2;
+                    hipLaunchKernelGGL(feedback_vec4_kernel, dim3(blocks_for((size_t)N << lanes_log2)), dim3(256), 0, stream, N,
+                                       L.size, L.fb_end - L.fb_start, prev.size, L.fb_start, net->S, post.size,
+                                       net->mdn_target_start, lanes_log2, L.pat, prev.out, post.out, L.out);
+                } else {
+                    hipLaunchKernelGGL(feedback_kernel, dim3(blocks_for(count)), dim3(256), 0, stream, count, L.size,
+                                       L.fb_end - L.fb_start, prev.size, L.fb_start, net->S, post.size, net->mdn_target_start,
+                                       L.pat, prev.out, post.out, L.out);
+                }
                 CNT_HIP(hipGetLastError());
                 break;
             }
@@ -1612,6 +1692,10 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
             for (ShapeGroup &c : groups) CNT_TRY(hand_over_group(c));
         return CNT_OK;
     };
+    // the side buffers that a launch of skip layer `from` adds to: the next forward pass clears them
+    auto adds_to_side = [&](const NetLayer &from) {
+        for (int k : from.side_targets) net->sides[(size_t)k].touched = true;
+    };
     for (size_t i = net->layers.size() - 1; i >= 1; --i) {
         NetLayer &L = net->layers[i];
         NetLayer &prev = net->layers[i - 1];
@@ -1685,6 +1769,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                             direct_from[i - 8] = prev_err;
                         }
                         const bool fan_live = block_fan.n > 0 || block_fan.from_skip;
+                        if (block_fan.n > 0) adds_to_side(prev);
                         CNT_TRY(wavenet_block_errors(stream, prev.size, L.size, N, L.pat, W, net->weights + out.w_off, L.err,
                                                      prev_err, fan_live ? &block_fan : nullptr, wav.core,
                                                      wav.ctx_dim > 0 ? wav.cth : nullptr, cnn.delta_fused ? cnn.out : nullptr,
@@ -1698,6 +1783,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                     }
                     static const bool early = [] { const char *e = std::getenv("CNT_NET_EARLY_WEIGHTS"); return !e || std::atoi(e) != 0; }();
                     if (errors_done[i]) goto weight_half_of_layer;
+                    if (wanted) adds_to_side(prev);
                     if (L.kind == K_DENSE && early && net->overlap && prev_err && (double)prev.size * L.size * N >= 4e8) {
                         // a large dense layer: deltas first, then its weight half starts on a side stream next to the
                         // product for the preceding layer's errors instead of after it
@@ -1789,6 +1875,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                 if (!L.needs_sum && L.live_targets == 0) break;
                 if (fan_done[i]) break;  // done in the epilogue of the following layer's product
                 ProfileScope prof(stream, "skip_fan");
+                adds_to_side(L);
                 const float *from_skip = L.needs_sum ? L.eskip : static_cast<const float *>(nullptr);
                 if (L.ptrs_aligned && count % 4 == 0)
                     hipLaunchKernelGGL(skip_fan_kernel<float4>, dim3(blocks_for(count / 4)), dim3(256), 0, stream, count / 4,
@@ -1801,6 +1888,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
             }
             case K_SKIPCAT: {
                 // SkipCatLayer::computeBackwardPass (layers/SkipCatLayer.cu:340-397)
+                adds_to_side(L);
                 hipLaunchKernelGGL(add_inplace_kernel, dim3(blocks_for(count)), dim3(256), 0, stream, count, L.err, L.eskip);
                 CNT_HIP(hipGetLastError());
                 int at = 0;

@@ -38,6 +38,15 @@ def test_softmax_unit(lengths, K, extra):
     assert PC.run_softmax_case(lengths, K, extra, seed=K) < TOL
 
 
+# a frame in registers: one quad, every lane's last quad, one more or less than a lane holds, the largest (1024) and the
+# first size past it; four leading columns move the unit's first column, two take it off 16 bytes
+@pytest.mark.parametrize("lengths,K,extra", [([3, 1], 4, 0), ([5, 2, 4], 252, 4), ([9, 9], 256, 0), ([6, 2], 260, 4), ([7], 512, 2),
+                                             ([4, 3], 516, 0), ([5, 1], 1020, 4), ([2, 2], 1028, 0)])
+def test_softmax_unit_sizes_in_registers(lengths, K, extra):
+    print("mdn softmax sizes", lengths, K, extra, flush=True)
+    assert PC.run_softmax_case(lengths, K, extra, seed=K) < TOL
+
+
 def test_unsupported_units_are_rejected():
     capi = PC.pkg().capi
     with pytest.raises(RuntimeError):

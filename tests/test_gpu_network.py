@@ -411,6 +411,37 @@ def test_wavenet_network_file_against_oracle_graph(nb, cnn_tanh, R, K, Q, C, len
     net.close()
 
 
+# slots of one lane, of a few, of a wave and of more than one store per lane; the columns taken from the layer before end
+# inside a group of four; sizes that are no multiple of four
+@pytest.mark.parametrize("P,lo,hi,Q,lengths", [(3, 0, 3, 1, [4, 2]), (3, 1, 3, 6, [1]), (5, 0, 5, 30, [9, 4, 7]), (6, 2, 5, 253, [31, 30]),
+                                               (4, 0, 0, 1024, [700, 650]), (7, 0, 7, 26, [40])])
+def test_feedback_of_the_true_class(P, lo, hi, Q, lengths):
+    import torch
+
+    S, T = len(lengths), max(lengths)
+    N, D = S * T, hi - lo + Q
+    doc = {"layers": [{"size": P, "name": "input", "type": "input"},
+                      {"size": P, "name": "below", "type": "feedforward_tanh", "bias": 1.0},
+                      {"size": D, "name": "fb", "type": "feedback", "bias": 1.0, "previousDimStart": lo, "previousDimEnd": hi},
+                      {"size": Q, "name": "out", "type": "feedforward_identity", "bias": 1.0},
+                      {"size": 1, "name": "post", "type": "mdn"}]}
+    net = PC.pkg().capi.Network(json.dumps(doc), S, T, mdn_config=[1, 0, Q, 0, 1, -1])
+    net.randomize(3, 0.3)
+    rng = np.random.default_rng(P + Q)
+    pat = make_pat_types(lengths, T)
+    cls = rng.integers(0, Q, N)
+    net.load_sequences(PC.dev(pat), T, min(lengths), PC.dev(rng.standard_normal(P * N).astype(np.float32)), PC.dev(cls.astype(np.float32)))
+    net.forward()
+    torch.cuda.synchronize()
+    want = np.zeros((N, D), np.float32)
+    want[:, : hi - lo] = net.layer("below")["outputs"].cpu().numpy()[: N * P].reshape(N, P)[:, lo:hi]
+    for n in range(S, N):
+        if pat[n - S]:
+            want[n, hi - lo + cls[n - S]] = 1.0
+    assert np.array_equal(net.layer("fb")["outputs"].cpu().numpy()[: N * D].reshape(N, D), want)
+    net.close()
+
+
 def test_network_file_rejections():
     capi = PC.pkg().capi
 
