@@ -1327,6 +1327,44 @@ int cnt_network_load_sequences(cnt_network *net, void *stream_, int T, int Tmin,
     return CNT_OK;
 }
 
+}  // extern "C"
+
+namespace cnt {
+namespace {
+
+bool fuse_blocks() {
+    static const bool on = [] { const char *e = std::getenv("CNT_NET_FUSE_BLOCKS"); return !e || std::atoi(e) != 0; }();
+    return on;
+}
+
+// WaveNet residual block seen from its skip 1x1 layer i: [cnn 2R][wavnetc R][dense R, identity][skipadd, shares
+// the following sum][skipini][dense K, identity (i)]
+bool block_errors_at(const cnt_network *net, size_t i) {
+    if (!fuse_blocks() || i < 5) return false;
+    const NetLayer &sk = net->layers[i], &ini = net->layers[i - 1], &add = net->layers[i - 2], &out = net->layers[i - 3];
+    const NetLayer &wav = net->layers[i - 4], &cnn = net->layers[i - 5];
+    const int R = ini.size;
+    auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    return sk.kind == K_DENSE && sk.act == ACT_IDENTITY && ini.kind == K_SKIPINI && ini.err && ini.err == ini.total &&
+           is_sum_skip(add.kind) && add.total == ini.total && !add.needs_sum && add.live_targets == 0 && add.size == R &&
+           out.kind == K_DENSE && out.act == ACT_IDENTITY && out.err == ini.total && out.size == R &&
+           wav.kind == K_WAVNETC && wav.size == R && wav.core && (wav.ctx_dim == 0 || wav.cth) &&
+           cnn.kind == K_CNN && cnn.size == 2 * R && cnn.err &&
+           sk.N == ini.N && sk.N == out.N && sk.N == wav.N && sk.N == cnn.N &&
+           wavenet_block_errors_supported(R, sk.size) && aligned(sk.err) && aligned(ini.total) && aligned(ini.eskip) &&
+           aligned(wav.core) && aligned(wav.cth) && aligned(cnn.out) && aligned(cnn.err) &&
+           aligned(net->weights + sk.w_off) && aligned(net->weights + out.w_off);
+}
+
+// That launch adds the gate's pre-activations up from the convolution's outputs and the conditioning part, both of which
+// it reads for their derivatives: the forward pass then need not leave them behind.
+bool block_sums_core(const NetLayer &cnn, const NetLayer &wav) { return cnn.delta_fused && wav.ctx_dim > 0; }
+
+}  // namespace
+}  // namespace cnt
+
+extern "C" {
+
 int cnt_network_forward(cnt_network *net, void *stream_) {
     using namespace cnt;
     CNT_REQUIRE(net && net->T > 0, "network_forward: no fraction loaded");
@@ -1354,11 +1392,10 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
         at = side.end;
     }
     if (hi > lo) CNT_TRY(fill_zero(stream, net->skip_errors + lo, hi - lo));
-    static const bool fuse_blocks = [] { const char *e = std::getenv("CNT_NET_FUSE_BLOCKS"); return !e || std::atoi(e) != 0; }();
     // a WaveNet residual block seen from its convolution layer i: [cnn 2R (i)][wavnetc R][dense R, identity]
     // [skipadd of the block's input and that layer][skipini, shares the sum][dense K, identity]
     auto block_at = [&](size_t i) {
-        if (!fuse_blocks || i < 1 || i + 5 >= net->layers.size()) return false;
+        if (!fuse_blocks() || i < 1 || i + 5 >= net->layers.size()) return false;
         const NetLayer &in = net->layers[i - 1], &cnn = net->layers[i], &wav = net->layers[i + 1], &out = net->layers[i + 2];
         const NetLayer &add = net->layers[i + 3], &ini = net->layers[i + 4], &sk = net->layers[i + 5];
         const int R = in.size;
@@ -1436,8 +1473,9 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
                 if (block_at(i)) {
                     const NetLayer &wav = net->layers[i + 1], &out = net->layers[i + 2], &sk = net->layers[i + 5];
                     CNT_TRY(conditioning(i + 1));
+                    float *core = block_errors_at(net, i + 5) && block_sums_core(L, wav) ? nullptr : wav.core;
                     const BlockForward block = {prev.out, net->ctx, W, net->weights + wav.w_off, net->weights + out.w_off,
-                                                net->weights + sk.w_off, out.bias, sk.bias, L.out, wav.core, wav.cth, wav.out,
+                                                net->weights + sk.w_off, out.bias, sk.bias, L.out, core, wav.cth, wav.out,
                                                 out.out, net->layers[i + 3].out, sk.out};
                     CNT_TRY(wavenet_block_forward(stream, L.cnn, prev.size, sk.size, wav.ctx_dim, N, L.pat, block));
                     i += 5;
@@ -1542,28 +1580,10 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                (int)below != net->flagged && !is_skip_kind(net->layers[below + 1].kind);
     };
     for (auto &L : net->layers) L.colsum_rows = 0;
-    static const bool fuse_blocks = [] { const char *e = std::getenv("CNT_NET_FUSE_BLOCKS"); return !e || std::atoi(e) != 0; }();
-    // WaveNet residual block seen from its skip 1x1 layer i: [cnn 2R][wavnetc R][dense R, identity][skipadd, shares
-    // the following sum][skipini][dense K, identity (i)]
     std::vector<int> fold_from(net->layers.size(), -1);  // skip 1x1 layer -> convolution layer folded into its launch
     std::vector<const float *> direct_from(net->layers.size(), nullptr);  // skip 1x1 layer -> the block above's sum
     static const bool direct_sums = [] { const char *e = std::getenv("CNT_NET_DIRECT_SUMS"); return !e || std::atoi(e) != 0; }();
-    auto block_at = [&](size_t i) {
-        if (!fuse_blocks || i < 5) return false;
-        const NetLayer &sk = net->layers[i], &ini = net->layers[i - 1], &add = net->layers[i - 2], &out = net->layers[i - 3];
-        const NetLayer &wav = net->layers[i - 4], &cnn = net->layers[i - 5];
-        const int R = ini.size;
-        auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-        return sk.kind == K_DENSE && sk.act == ACT_IDENTITY && ini.kind == K_SKIPINI && ini.err && ini.err == ini.total &&
-               is_sum_skip(add.kind) && add.total == ini.total && !add.needs_sum && add.live_targets == 0 && add.size == R &&
-               out.kind == K_DENSE && out.act == ACT_IDENTITY && out.err == ini.total && out.size == R &&
-               wav.kind == K_WAVNETC && wav.size == R && wav.core && (wav.ctx_dim == 0 || wav.cth) &&
-               cnn.kind == K_CNN && cnn.size == 2 * R && cnn.err &&
-               sk.N == ini.N && sk.N == out.N && sk.N == wav.N && sk.N == cnn.N &&
-               wavenet_block_errors_supported(R, sk.size) && aligned(sk.err) && aligned(ini.total) && aligned(ini.eskip) &&
-               aligned(wav.core) && aligned(wav.cth) && aligned(cnn.out) && aligned(cnn.err) &&
-               aligned(net->weights + sk.w_off) && aligned(net->weights + out.w_off);
-    };
+    auto block_at = [&](size_t i) { return block_errors_at(net, i); };
     auto fold_at = [&](size_t i) {
         if (i < 8) return false;
         const NetLayer &C = net->layers[i], &closing = net->layers[i - 1], &sk = net->layers[i - 3];
@@ -1771,7 +1791,8 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                         const bool fan_live = block_fan.n > 0 || block_fan.from_skip;
                         if (block_fan.n > 0) adds_to_side(prev);
                         CNT_TRY(wavenet_block_errors(stream, prev.size, L.size, N, L.pat, W, net->weights + out.w_off, L.err,
-                                                     prev_err, fan_live ? &block_fan : nullptr, wav.core,
+                                                     prev_err, fan_live ? &block_fan : nullptr,
+                                                     block_sums_core(cnn, wav) ? nullptr : wav.core,
                                                      wav.ctx_dim > 0 ? wav.cth : nullptr, cnn.delta_fused ? cnn.out : nullptr,
                                                      cnn.err, fold ? fold->cnn : nullptr,
                                                      fold ? net->weights + fold->w_off : nullptr, fold ? fold->err : nullptr,

@@ -192,7 +192,7 @@ struct BlockErrArgs {
     int fan_n;
     float *const *fan_targets;
     const int *fan_is_skip;
-    const float *pre;        // 2R x N: pre-activations of the gated unit
+    const float *pre;        // 2R x N: pre-activations of the gated unit (null: the sum of conv_tanh and ctx_tanh)
     const float *conv_tanh;  // 2R x N or null: outputs of a convolution layer with tanh output
     float *ctx_tanh;         // 2R x N or null: tanh of the conditioning part, overwritten with its gradient
     float *deltas;           // 2R x N: errors (or deltas) of the convolution layer
@@ -206,7 +206,9 @@ struct BlockErrArgs {
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
-template <int R, int K, bool CONV>
+// SUM: the gate's pre-activations are formed again from the convolution's outputs and the conditioning part, which the
+// launch reads anyway; `pre` is not read then.
+template <int R, int K, bool CONV, bool SUM>
 __global__ __launch_bounds__(CONV ? 512 : 256, (CONV || K > 128) ? 1 : 2) void wavenet_block_errors_kernel(const BlockErrArgs a) {
     static_assert(R % 16 == 0 && K % 16 == 0 && R <= 128, "block geometry");
     constexpr int NT = CONV ? 512 : 256;  // the folded convolution's weights take 2 x 2R x R words of LDS more
@@ -290,16 +292,29 @@ __global__ __launch_bounds__(CONV ? 512 : 256, (CONV || K > 128) ? 1 : 2) void w
             }
         }
     }
-    // the gate's pre-activations and the first target's old values are requested before the products start
-    float4 p1[RT], p2[RT], old0[RT];
+    // the gate's operands and the first target's old values are requested before the products start, those of a launch that
+    // needs the registers for both taps behind the first tap's products
+    float4 p1[RT], p2[RT], old0[RT], y1[SUM ? RT : 1], y2[SUM ? RT : 1], c1[SUM ? RT : 1], c2[SUM ? RT : 1];
     const bool add_first = ok && a.fan_n > 0 && a.fan_is_skip[0] != 0;
+    auto request_gate = [&] {
 #pragma unroll
-    for (int t = 0; t < RT; ++t) {
-        const size_t at = n * 2 * R + 16 * t + 4 * quarter;
-        p1[t] = *reinterpret_cast<const float4 *>(a.pre + at);
-        p2[t] = *reinterpret_cast<const float4 *>(a.pre + at + R);
-        if (add_first) old0[t] = *reinterpret_cast<const float4 *>(a.fan_targets[0] + n * R + 16 * t + 4 * quarter);
-    }
+        for (int t = 0; t < RT; ++t) {
+            const size_t at = n * 2 * R + 16 * t + 4 * quarter;
+            if (SUM) {
+                y1[SUM ? t : 0] = *reinterpret_cast<const float4 *>(a.conv_tanh + at);
+                y2[SUM ? t : 0] = *reinterpret_cast<const float4 *>(a.conv_tanh + at + R);
+                c1[SUM ? t : 0] = *reinterpret_cast<const float4 *>(a.ctx_tanh + at);
+                c2[SUM ? t : 0] = *reinterpret_cast<const float4 *>(a.ctx_tanh + at + R);
+            } else {
+                p1[t] = *reinterpret_cast<const float4 *>(a.pre + at);
+                p2[t] = *reinterpret_cast<const float4 *>(a.pre + at + R);
+            }
+        }
+    };
+    if (!(SUM && CONV)) request_gate();
+    if (add_first)
+#pragma unroll
+        for (int t = 0; t < RT; ++t) old0[t] = *reinterpret_cast<const float4 *>(a.fan_targets[0] + n * R + 16 * t + 4 * quarter);
     __syncthreads();
 
     f32x4v e[RT];
@@ -327,6 +342,7 @@ __global__ __launch_bounds__(CONV ? 512 : 256, (CONV || K > 128) ? 1 : 2) void w
         e[t] = acc0 + acc1;
     }
     if (CONV) {
+        if (SUM) request_gate();
         __syncthreads();  // every wave is done with the first tap's weights
 #pragma unroll
         for (int q = 0; q < FC; ++q)
@@ -397,6 +413,11 @@ __global__ __launch_bounds__(CONV ? 512 : 256, (CONV || K > 128) ? 1 : 2) void w
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
         const size_t at = n * 2 * R + 16 * t + 4 * quarter;
+        if (SUM) {
+            const int z = SUM ? t : 0;
+            p1[t] = float4{y1[z].x + c1[z].x, y1[z].y + c1[z].y, y1[z].z + c1[z].z, y1[z].w + c1[z].w};
+            p2[t] = float4{y2[z].x + c2[z].x, y2[z].y + c2[z].y, y2[z].z + c2[z].z, y2[z].w + c2[z].w};
+        }
         const float *a1 = reinterpret_cast<const float *>(&p1[t]), *a2 = reinterpret_cast<const float *>(&p2[t]);
         float g1[4], g2[4];
 #pragma unroll
@@ -408,11 +429,11 @@ __global__ __launch_bounds__(CONV ? 512 : 256, (CONV || K > 128) ? 1 : 2) void w
             g2[q] = live ? th * (sg * (1.0f - sg)) * ev : 0.0f;
         }
         float4 o1 = {g1[0], g1[1], g1[2], g1[3]}, o2 = {g2[0], g2[1], g2[2], g2[3]};
-        if (a.conv_tanh) {
-            const float4 y1 = *reinterpret_cast<const float4 *>(a.conv_tanh + at);
-            const float4 y2 = *reinterpret_cast<const float4 *>(a.conv_tanh + at + R);
-            o1 = float4{tanh_deriv(y1.x) * g1[0], tanh_deriv(y1.y) * g1[1], tanh_deriv(y1.z) * g1[2], tanh_deriv(y1.w) * g1[3]};
-            o2 = float4{tanh_deriv(y2.x) * g2[0], tanh_deriv(y2.y) * g2[1], tanh_deriv(y2.z) * g2[2], tanh_deriv(y2.w) * g2[3]};
+        if (SUM || a.conv_tanh) {
+            const float4 v1 = SUM ? y1[SUM ? t : 0] : *reinterpret_cast<const float4 *>(a.conv_tanh + at);
+            const float4 v2 = SUM ? y2[SUM ? t : 0] : *reinterpret_cast<const float4 *>(a.conv_tanh + at + R);
+            o1 = float4{tanh_deriv(v1.x) * g1[0], tanh_deriv(v1.y) * g1[1], tanh_deriv(v1.z) * g1[2], tanh_deriv(v1.w) * g1[3]};
+            o2 = float4{tanh_deriv(v2.x) * g2[0], tanh_deriv(v2.y) * g2[1], tanh_deriv(v2.z) * g2[2], tanh_deriv(v2.w) * g2[3]};
         }
         if (ok) {
             *reinterpret_cast<float4 *>(a.deltas + at) = o1;
@@ -420,11 +441,11 @@ __global__ __launch_bounds__(CONV ? 512 : 256, (CONV || K > 128) ? 1 : 2) void w
         }
         cs1[t] = ok ? o1 : float4{0.0f, 0.0f, 0.0f, 0.0f};
         cs2[t] = ok ? o2 : float4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (a.ctx_tanh) {
-            const float4 c1 = *reinterpret_cast<const float4 *>(a.ctx_tanh + at);
-            const float4 c2 = *reinterpret_cast<const float4 *>(a.ctx_tanh + at + R);
-            const float4 q1 = {tanh_deriv(c1.x) * g1[0], tanh_deriv(c1.y) * g1[1], tanh_deriv(c1.z) * g1[2], tanh_deriv(c1.w) * g1[3]};
-            const float4 q2 = {tanh_deriv(c2.x) * g2[0], tanh_deriv(c2.y) * g2[1], tanh_deriv(c2.z) * g2[2], tanh_deriv(c2.w) * g2[3]};
+        if (SUM || a.ctx_tanh) {
+            const float4 v1 = SUM ? c1[SUM ? t : 0] : *reinterpret_cast<const float4 *>(a.ctx_tanh + at);
+            const float4 v2 = SUM ? c2[SUM ? t : 0] : *reinterpret_cast<const float4 *>(a.ctx_tanh + at + R);
+            const float4 q1 = {tanh_deriv(v1.x) * g1[0], tanh_deriv(v1.y) * g1[1], tanh_deriv(v1.z) * g1[2], tanh_deriv(v1.w) * g1[3]};
+            const float4 q2 = {tanh_deriv(v2.x) * g2[0], tanh_deriv(v2.y) * g2[1], tanh_deriv(v2.z) * g2[2], tanh_deriv(v2.w) * g2[3]};
             if (ok) {
                 *reinterpret_cast<float4 *>(a.ctx_tanh + at) = q1;
                 *reinterpret_cast<float4 *>(a.ctx_tanh + at + R) = q2;
@@ -503,9 +524,14 @@ __global__ void fill_zero_list_kernel(const FillList f) {
 }
 
 typedef void (*block_err_kernel_t)(const BlockErrArgs);
-block_err_kernel_t pick_block_errors_kernel(int R, int K, bool conv) {
+template <int R, int K>
+block_err_kernel_t block_errors_of(bool conv, bool sum) {
+    return conv ? (sum ? wavenet_block_errors_kernel<R, K, true, true> : wavenet_block_errors_kernel<R, K, true, false>)
+                : (sum ? wavenet_block_errors_kernel<R, K, false, true> : wavenet_block_errors_kernel<R, K, false, false>);
+}
+block_err_kernel_t pick_block_errors_kernel(int R, int K, bool conv, bool sum) {
 #define CNT_BLOCK_KERNEL(r, k) \
-    if (R == r && K == k) return conv ? wavenet_block_errors_kernel<r, k, true> : wavenet_block_errors_kernel<r, k, false>;
+    if (R == r && K == k) return block_errors_of<r, k>(conv, sum);
     CNT_BLOCK_KERNEL(64, 128)
     CNT_BLOCK_KERNEL(64, 256)
     CNT_BLOCK_KERNEL(64, 64)
@@ -919,7 +945,7 @@ extern "C++" bool cnt::wavenet_block_forward_supported(const cnt_cnn *cnn, int R
 extern "C++" int cnt::wavenet_block_forward(hipStream_t stream, const cnt_cnn *cnn, int R, int K, int C, int N,
                                             const char *patTypes, const BlockForward &b) {
     CNT_REQUIRE(wavenet_block_forward_supported(cnn, R, K, C), "wavenet_block_forward: no kernel for this block");
-    CNT_REQUIRE(N > 0 && patTypes && b.x && b.conv_weights && b.out_weights && b.skip_weights && b.conv && b.core && b.gated &&
+    CNT_REQUIRE(N > 0 && patTypes && b.x && b.conv_weights && b.out_weights && b.skip_weights && b.conv && b.gated &&
                 b.out && b.sum && b.skip && (C == 0 || (b.ctx && b.ctx_weights && b.ctx_tanh)),
                 "wavenet_block_forward: null argument");
     const cnt_cnn_group &g = cnn->groups[0];
@@ -956,7 +982,7 @@ extern "C++" int cnt::wavenet_block_forward(hipStream_t stream, const cnt_cnn *c
     return CNT_OK;
 }
 
-extern "C++" bool cnt::wavenet_block_errors_supported(int R, int K) { return pick_block_errors_kernel(R, K, false) != nullptr; }
+extern "C++" bool cnt::wavenet_block_errors_supported(int R, int K) { return pick_block_errors_kernel(R, K, false, false) != nullptr; }
 
 extern "C++" int cnt::wavenet_block_rows(int N, bool fold) { return fold ? (N + 127) / 128 : (N + 63) / 64; }
 
@@ -971,9 +997,10 @@ extern "C++" int cnt::wavenet_block_errors(hipStream_t stream, int R, int K, int
                                            float *total, const FanOut *fan, const float *core_buf, float *ctx_tanh,
                                            const float *conv_tanh_outputs, float *conv_errors, const cnt_cnn *fold,
                                            const float *fold_weights, const float *fold_deltas, float *colsum_partial) {
-    block_err_kernel_t k = pick_block_errors_kernel(R, K, fold != nullptr);
+    block_err_kernel_t k = pick_block_errors_kernel(R, K, fold != nullptr, core_buf == nullptr);
     CNT_REQUIRE(k != nullptr, "wavenet_block_errors: no kernel for %d residual and %d skip channels", R, K);
-    CNT_REQUIRE(N > 0 && patTypes && skip_weights && out_weights && skip_errors && total && core_buf && conv_errors,
+    CNT_REQUIRE(N > 0 && patTypes && skip_weights && out_weights && skip_errors && total && (core_buf || (ctx_tanh && conv_tanh_outputs)) &&
+                conv_errors,
                 "wavenet_block_errors: null argument");
     BlockErrArgs a = {};
     a.N = N; a.pat = patTypes; a.w_skip = skip_weights; a.w_out = out_weights; a.e_skip = skip_errors;

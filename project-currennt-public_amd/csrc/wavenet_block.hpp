@@ -23,7 +23,7 @@ struct BlockFwdArgs {
     const float *skip_w, *skip_bias;  // [K][R]
     float conv_scale, out_scale, skip_scale;  // factors of the bias vectors
     int conv_tanh;
-    float *conv, *core, *ctx_tanh, *gated, *out, *sum, *skip;
+    float *conv, *core, *ctx_tanh, *gated, *out, *sum, *skip;  // core: null where the backward pass forms it again
 };
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -157,8 +157,8 @@ __global__ __launch_bounds__(R * 4, 2) void wavenet_block_forward_kernel(const B
     auto put = [](__amdgpu_buffer_rsrc_t to, unsigned offset, const f32x4 &v) {
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), to, offset, 0, 2);  // non-temporal: read in another pass
     };
-    const auto to_conv = rows_of(a.conv, 2 * R), to_core = rows_of(a.core, 2 * R), to_gated = rows_of(a.gated, R);
-    const auto to_ctx = a.ctx_tanh ? rows_of(a.ctx_tanh, 2 * R) : __builtin_amdgcn_make_buffer_rsrc(a.core, 0, 0, 0x00020000);
+    const auto to_conv = rows_of(a.conv, 2 * R), to_gated = rows_of(a.gated, R), nowhere = __builtin_amdgcn_make_buffer_rsrc(a.conv, 0, 0, 0x00020000);
+    const auto to_core = a.core ? rows_of(a.core, 2 * R) : nowhere, to_ctx = a.ctx_tanh ? rows_of(a.ctx_tanh, 2 * R) : nowhere;
 
     // ---- convolution, conditioning projection and gate, one step of sixteen samples after the other.  The gate of a
     // step is evaluated between the matrix instructions of the next one's convolution: seven vector instructions fit
