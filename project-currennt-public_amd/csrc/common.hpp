@@ -193,8 +193,8 @@ struct GemmArgs {
     // Split-K products with a small output (EPI_ATOMIC, splitk = 0): `overwrite_ok` allows gemm_plan to choose
     // EPI_PARTIAL, which overwrites C instead of adding to a cleared C.  With `rowsum` (one operand pair, unmasked)
     // the same pass also sums every problem's B operand over k into that problem's rowsum_out -- the bias gradient
-    // of a dense layer, for which the atomic path needs a separate column-sum launch.  gemm_plan clears `rowsum`
-    // where it does not choose EPI_PARTIAL.
+    // of a dense layer; with EPI_ATOMIC it adds to what the caller has cleared.  gemm_plan clears `rowsum` where the
+    // product cannot bring it along (operands that are not row-contiguous, several pairs).
     int overwrite_ok;
     int rowsum;
     int fan_n;                   // EPI_FAN: device tables of fan_n targets and their flags

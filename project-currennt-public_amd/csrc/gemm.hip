@@ -71,7 +71,7 @@ inline long large_tiles(const GemmArgs &a) { return (long)((a.m + 127) / 128) * 
 // as many splits of k as make two workgroups per compute unit (the parts of two row-contiguous operands take 55 KB of LDS, so more
 // do not fit), as long as a split has at least 768 values of k: below that, filling and draining the pipeline and the atomic sums
 // of the tiles outweigh what the large tile saves, and three times as many small workgroups share them better.  64 / 128, us,
-// with the clear and the column sum behind it: 1024 x 1024 over 2000 / 5000 / 8000 / 12 000 slots (250 / 625 / 1000 / 1500 per
+// with the clear and a column sum behind it, which the product brings along by now: 1024 x 1024 over 2000 / 5000 / 8000 / 12 000 slots (250 / 625 / 1000 / 1500 per
 // split) 43 / 58, 88 / 89, 134 / 121, 193 / 162; 1300 x 1300 over 3000 / 4000 (750 / 1000) 98 / 101, 125 / 120; 2048 x 2048 over
 // 1000 / 3000 (500 / 1500) 73 / 79, 187 / 159.  (Below 64 tiles the line is further up, 896 x 896 over 2000 / 6000 / 12 000
 // 41 / 57, 92 / 86, 173 / 136, and layers of 32 tiles gain nothing; they keep the small tile.)  The feed-forward model of five
@@ -283,7 +283,7 @@ void gemm_plan(GemmArgs &args, hipStream_t stream) {
     if (partial) {
         args.epilogue = EPI_PARTIAL;
         args.partial_stride = stride;
-    } else {
+    } else if (!rowsum_ok || args.epilogue != EPI_ATOMIC || args.a_kcontig || args.b_kcontig) {
         args.rowsum = 0;  // the caller sums the rows itself
     }
 }
@@ -332,7 +332,7 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
         CNT_HIP(hipGetLastError());
         return CNT_OK;
     }
-    if (args.epilogue != EPI_PARTIAL) args.rowsum = 0;
+    if (args.epilogue != EPI_PARTIAL && args.epilogue != EPI_ATOMIC) args.rowsum = 0;
     const int tile = pick_tile(args);
     // a list of k lines is used where the kernel that reads through it exists, and ignored otherwise (the lines it leaves
     // out are zero)

@@ -264,6 +264,21 @@ struct TileStage {
 // stored, and the tiles where a vector could leave the operand or hold k values beyond its end take a path of their own
 // (uniform over the workgroup), one float at a time unless the lines are a multiple of four long.
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+// adds a thread's share of a tile, NLOAD k positions of four rows, to its sums of those rows: the positions among themselves
+// first, so that a sum's chain of additions has one link per tile
+template <int NLOAD>
+__device__ __forceinline__ void add_tile_rows(float (&sum)[4], const float4 (&r)[NLOAD]) {
+    float4 v = r[0];
+    if constexpr (NLOAD == 4) {
+        v.x = (r[0].x + r[1].x) + (r[2].x + r[3].x); v.y = (r[0].y + r[1].y) + (r[2].y + r[3].y);
+        v.z = (r[0].z + r[1].z) + (r[2].z + r[3].z); v.w = (r[0].w + r[1].w) + (r[2].w + r[3].w);
+    } else {
+#pragma unroll
+        for (int p = 1; p < NLOAD; ++p) { v.x += r[p].x; v.y += r[p].y; v.z += r[p].z; v.w += r[p].w; }
+    }
+    sum[0] += v.x; sum[1] += v.y; sum[2] += v.z; sum[3] += v.w;
+}
+
 // WHOLE: the lines are a multiple of four long, so that no vector crosses the end of one.
 template <bool WHOLE, bool KCONTIG, int ROWS>
 struct FastStage {
@@ -320,12 +335,7 @@ struct FastStage {
     }
     __device__ __forceinline__ void store(uint4 *__restrict__ lds, int tid) const { L::put(lds, tid, r); }
     // adds the tile in registers to the sums of the thread's four rows (row-contiguous operands)
-    __device__ __forceinline__ void add_rows(float (&sum)[4]) const {
-#pragma unroll
-        for (int p = 0; p < NLOAD; ++p) {
-            sum[0] += r[p].x; sum[1] += r[p].y; sum[2] += r[p].z; sum[3] += r[p].w;
-        }
-    }
+    __device__ __forceinline__ void add_rows(float (&sum)[4]) const { add_tile_rows<NLOAD>(sum, r); }
 };
 
 // The unmasked loader for row-contiguous operands whose k lines are picked through a list (16-byte vectors only): tile k
@@ -365,11 +375,10 @@ struct GatherStage {
         }
     }
     __device__ __forceinline__ void add_rows(float (&sum)[4]) const {
+        float4 v[NLOAD];
 #pragma unroll
-        for (int p = 0; p < NLOAD; ++p) {
-            const float4 v = kk + p < k_valid ? r[p] : float4{0.0f, 0.0f, 0.0f, 0.0f};
-            sum[0] += v.x; sum[1] += v.y; sum[2] += v.z; sum[3] += v.w;
-        }
+        for (int p = 0; p < NLOAD; ++p) v[p] = kk + p < k_valid ? r[p] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+        add_tile_rows<NLOAD>(sum, v);
     }
 };
 
@@ -636,6 +645,27 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
 
     // epilogue: lane%32 runs along m (contiguous), the 16 accumulators along n
     float *__restrict__ C = pb.C;
+    if constexpr (!AK && !BK_ && !MASKED) {
+        if (rowsum) {
+            // the threads that loaded different k positions of the same rows add up through LDS, in a fixed order
+            constexpr int PARTS = BK / LB::NLOAD;
+            static_assert(PARTS * BN * sizeof(float) <= sizeof(lds), "the row sums fit the tile's buffer");
+            float *const sums = reinterpret_cast<float *>(lds);
+            __syncthreads();
+            *reinterpret_cast<float4 *>(sums + LB::first_k(tid) / LB::NLOAD * BN + LB::first_row(tid)) = float4{rs[0], rs[1], rs[2], rs[3]};
+            __syncthreads();
+            if (tid < BN && n0 + tid < args.n) {
+                float s = 0.0f;
+#pragma unroll
+                for (int q = 0; q < PARTS; ++q) s += sums[q * BN + tid];
+                if (args.epilogue == EPI_PARTIAL)
+                    args.partial[(size_t)split_id * args.partial_stride + (size_t)args.nprob * args.m * args.n +
+                                 (size_t)prob_id * args.n + n0 + tid] = s;
+                else
+                    atomicAdd(pb.rowsum_out + n0 + tid, pb.rowsum_scale * s);
+            }
+        }
+    }
     if (args.epilogue == EPI_PARTIAL) {
         // this split's partial product, m x n column-major without padding, after those of the problems before it
         float *__restrict__ P = args.partial + (size_t)split_id * args.partial_stride +
@@ -651,23 +681,6 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
                     const int n = n0 + wn * WT + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
                     if (n < args.n) P[(size_t)n * args.m + m] = acc[i][j][r];
                 }
-            }
-        }
-        if constexpr (!AK && !BK_ && !MASKED) {
-            if (!rowsum) return;
-            // the threads that loaded different k positions of the same rows add up through LDS, in a fixed order
-            constexpr int PARTS = BK / LB::NLOAD;
-            static_assert(PARTS * BN * sizeof(float) <= sizeof(lds), "the row sums fit the tile's buffer");
-            float *const sums = reinterpret_cast<float *>(lds);
-            __syncthreads();
-            *reinterpret_cast<float4 *>(sums + LB::first_k(tid) / LB::NLOAD * BN + LB::first_row(tid)) = float4{rs[0], rs[1], rs[2], rs[3]};
-            __syncthreads();
-            if (tid < BN && n0 + tid < args.n) {
-                float s = 0.0f;
-#pragma unroll
-                for (int q = 0; q < PARTS; ++q) s += sums[q * BN + tid];
-                args.partial[(size_t)split_id * args.partial_stride + (size_t)args.nprob * args.m * args.n +
-                             (size_t)prob_id * args.n + n0 + tid] = s;
             }
         }
         return;

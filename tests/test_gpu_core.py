@@ -636,6 +636,23 @@ def test_weight_gradient_of_few_blocks(P, D, N, static):
     assert bool(((dW[P * D:] - 0.5 * err.double().sum(0)).abs() <= (N + 2) * 2.0 ** -24 * 0.5 * err.double().abs().sum(0)).all())
 
 
+@pytest.mark.parametrize("P,D,N", [(1024, 1024, 6200), (512, 514, 2501), (401, 600, 3001), (260, 4100, 2600), (4100, 64, 2066)])
+def test_bias_gradient_beside_atomic_sums(P, D, N):
+    """Weight gradients whose splits add to a cleared output bring the bias gradient along: large and small tiles, rows that end
+    inside a tile, operands whose rows are no multiple of four long, a last split of another length, one infinite delta."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(P + D + N)
+    x, err = torch.randn(N, P, device="cuda", generator=g), torch.randn(N, D, device="cuda", generator=g)
+    err[N - 1, D - 1] = float("inf")
+    dW = torch.full((P * D + D,), 3.0, device="cuda")
+    PC.pkg().capi.dense_backward_weights(P, D, N, 0.5, x, err, dW)
+    size = err.double().abs().sum(0)
+    assert torch.isposinf(dW[-1])
+    assert bool(((dW[P * D:] - 0.5 * err.double().sum(0)).abs()[:-1] <= (N + 2) * 2.0 ** -24 * 0.5 * size[:-1]).all())
+    want = err.double().t() @ x.double()
+    assert bool(((dW[:P * D].view(D, P) - want).abs() <= (N + 2) * 2.0 ** -24 * (err.double().abs().t() @ x.double().abs()))[:-1].all())
+
+
 @pytest.mark.parametrize("m,n,k,tA,tB", [(70, 66, 37, True, False), (3100, 3076, 516, False, False)])
 def test_matrix_product_of_infinite_huge_and_missing_values(m, n, k, tA, tB):
     """Values that have no finite bf16 parts give what fp32 arithmetic gives."""
