@@ -7,23 +7,30 @@
 // runs about a dozen launches and three cuFFT calls per resolution and waveform, with every intermediate
 // (framed signals, spectra, per-bin differences, framed gradients) in device memory.
 //
-// Here a frame stays in one workgroup's LDS end to end, all resolutions of a call are one launch, and nothing
+// Here a frame stays in one workgroup's registers and LDS end to end, all resolutions of a call are one launch, and nothing
 // but the waveforms and the gradient touches HBM:
 //   frame + window source and target  ->  ONE complex FFT of z = source + i*target in LDS (both real
 //   spectra are recovered from Z[b] and Z[N-b])  ->  per-bin distance, loss partial and gradient spectrum,
 //   written back as its Hermitian extension  ->  inverse FFT in LDS  ->  windowed overlap-add straight into
 //   the per-sample gradient with float atomics.
-// A workgroup makes several such passes (short transforms more than long ones, so that the workgroups of all
-// resolutions carry similar work), loads its twiddles once, fetches the next pass's samples while it computes,
-// and adds its loss partial to the per-waveform sums once at its end.
+// A workgroup of 256 threads holds 2048 points, one frame of 2048 or as many shorter ones as that makes, eight points per
+// thread in registers; frames of up to 512 points lie inside one wave and need no barrier.  It adds its loss partial to the
+// per-waveform sums once at its end.
+// What bounds it is the chain of a frame: loads, LOGN/2 - 1 exchanges through LDS, the bins, the exchanges back, the atomics.
+// Eight waveforms of 16 000 samples at 2048 / 512 / 128 points: 23 us with four points per butterfly read from and written to
+// LDS, a barrier per radix-4 step, tables in LDS and two or three passes of a workgroup; 16 us now (16 points per thread, four
+// stages per exchange: 19 us; three stages of eight: 15 us, but its rounding differs and the log distance's gradient, which
+// divides by amplitudes close to zero, moves by 5e-5).  The registers decide: 119 of them let four workgroups share a compute
+// unit, with a loop over several frames per workgroup (145, three workgroups) the same call takes 24.5 instead of 18.7 us.
 // The forward transform is decimation-in-frequency (natural order in, bit-reversed out), the per-bin stage
 // addresses bins through the bit-reversal, and the inverse is decimation-in-time (bit-reversed in, natural
 // out), so no reordering pass exists; two butterfly stages share a barrier as one radix-4 butterfly.  Twiddles
-// (one run per stage, so that a stage reads consecutive LDS words) and the window (with the reference's
+// (one run per stage, so that a wave reads consecutive words) and the window (with the reference's
 // constant 3.141215) are tabulated in double on the host.  Transform conventions are cuFFT's: unnormalised,
 // N/2+1 bins, the imaginary parts of the DC and Nyquist bins do not enter the inverse.
 #include "common.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -34,6 +41,7 @@ namespace {
 
 constexpr int kMaxRes = 3;
 constexpr int kMaxWavesPerLaunch = 32;
+constexpr int kMaxThreads = 512;  // eight points per thread: a workgroup holds a frame of 4096
 
 struct DftParams {
     // per resolution: log2 of the fft length, frame length, frame shift, blocks along x that carry frames
@@ -132,174 +140,225 @@ __device__ inline void bin_phase(float sx, float sy, float tx, float ty, float &
 
 constexpr int kMaxLogN = 12;
 
-// One block = passes of FPB frames of resolution `res` of one waveform.  lds: max(1024, N) + N complex words.
+// ---- the transform: radix 4, eight points per thread ----
+// In-place decimation in frequency over T = N/8 threads.  Stage s, from LOGN - 1 down, combines points 2^s apart; the stages s and
+// s - 1 are one radix-4 butterfly on the points base + {0, q, 2q, 3q}, q = 2^(s-1).  In a pass a thread takes the butterflies t
+// and t + T, in the first one, q = N/4, that is the points t + j*T, which is how the samples arrive; in the last one it takes the
+// points 8t + r, in three stages for odd LOGN, in two for even.  A pass leaves its results where it took its points, so one
+// exchange through LDS lies between two passes.  Point p is then bin bitrev(p).  The inverse walks the same stages backwards
+// with conjugated twiddles and ends with the samples t + j*T.
+struct Twiddles4 {
+    float2 w1, w2;  // of the butterfly's first stage (its second pair takes -i times that) and of its second
+};
+// Which products are rounded is written out: a spectrum's small amplitudes, by which some distances divide, are what their
+// rounding leaves, and the log distance's gradient moves by up to 5e-5 with it.
+__device__ __forceinline__ float2 turned(float2 a, float2 w) {  // a * w
+    return make_float2(__builtin_fmaf(a.x, w.x, -(a.y * w.y)), __builtin_fmaf(a.y, w.x, a.x * w.y));
+}
+__device__ __forceinline__ float2 turned_back(float2 a, float2 w) {  // a * conj(w)
+    return make_float2(__builtin_fmaf(a.x, w.x, a.y * w.y), __builtin_fmaf(a.y, w.x, -(a.x * w.y)));
+}
+// what enters and leaves a butterfly is rounded, whatever the compiler could join across it
+__device__ __forceinline__ void settle(float2 &x) { asm volatile("" : "+v"(x.x), "+v"(x.y)); }
+
+__device__ __forceinline__ void butterfly4(float2 &x0, float2 &x1, float2 &x2, float2 &x3, const Twiddles4 &w) {
+    const float2 w1 = w.w1, w2 = w.w2;
+    const float2 y0 = make_float2(x0.x + x2.x, x0.y + x2.y), d02 = make_float2(x0.x - x2.x, x0.y - x2.y);
+    const float2 y1 = make_float2(x1.x + x3.x, x1.y + x3.y), d13 = make_float2(x1.y - x3.y, x3.x - x1.x);
+    const float2 y2 = turned(d02, w1), y3 = turned(d13, w1);
+    const float2 e01 = make_float2(y0.x - y1.x, y0.y - y1.y), e23 = make_float2(y2.x - y3.x, y2.y - y3.y);
+    x0 = make_float2(y0.x + y1.x, y0.y + y1.y);
+    x1 = turned(e01, w2);
+    x2 = make_float2(y2.x + y3.x, y2.y + y3.y);
+    x3 = make_float2(__builtin_fmaf(e23.x, w2.x, -(e23.y * w2.y)), __builtin_fmaf(e23.x, w2.y, e23.y * w2.x));
+    settle(x0); settle(x1); settle(x2); settle(x3);
+}
+__device__ __forceinline__ void inverse_butterfly4(float2 &x0, float2 &x1, float2 &x2, float2 &x3, const Twiddles4 &w) {
+    const float2 w1 = w.w1, w2 = w.w2;
+    const float2 v1 = turned_back(x1, w2), v3 = turned_back(x3, w2);
+    const float2 y0 = make_float2(x0.x + v1.x, x0.y + v1.y), y1 = make_float2(x0.x - v1.x, x0.y - v1.y);
+    const float2 y2 = make_float2(x2.x + v3.x, x2.y + v3.y), y3 = make_float2(x2.x - v3.x, x2.y - v3.y);
+    const float2 u2 = turned_back(y2, w1), t3 = turned_back(y3, w1);
+    const float2 u3 = make_float2(-t3.y, t3.x);  // conj(-i * w1) = i * conj(w1)
+    x0 = make_float2(y0.x + u2.x, y0.y + u2.y);
+    x1 = make_float2(y1.x + u3.x, y1.y + u3.y);
+    x2 = make_float2(y0.x - u2.x, y0.y - u2.y);
+    x3 = make_float2(y1.x - u3.x, y1.y - u3.y);
+    settle(x0); settle(x1); settle(x2); settle(x3);
+}
+__device__ __forceinline__ void butterfly2(float2 &a, float2 &b) {
+    const float2 d = make_float2(a.x - b.x, a.y - b.y);
+    a = make_float2(a.x + b.x, a.y + b.y);
+    b = d;
+    settle(a); settle(b);
+}
+
+// One block = passes of FPB frames of resolution `res` of one waveform.  lds: 9 complex words per thread.
 template <int LOGN, int DIS>
 __device__ __forceinline__ void dft_frames(const DftParams &p, const int res, float2 *__restrict__ lds,
-                                           float (*err_part)[4]) {
-    constexpr int N = 1 << LOGN;
-    float2 *__restrict__ zbuf = lds;                      // frame storage: FPB * N = max(1024, N) complex words
-    float2 *__restrict__ tw = lds + (N > 1024 ? N : 1024);  // N twiddles
-    constexpr int HALF = N / 2;
-    constexpr int QUARTER = N / 4;
-    constexpr int TPF = QUARTER < 256 ? QUARTER : 256;  // threads per frame: one per radix-4 butterfly up to N = 1024
-    constexpr int FPB = 256 / TPF;                      // frames per block
-    static_assert(FPB * N <= (N > 1024 ? N : 1024), "frame storage: max(1024, N) complex words");
-
-    constexpr int EPT = N / TPF;  // samples per thread and frame
-
-    const int tid = threadIdx.x;
-    const int fl = tid / TPF, ft = tid % TPF;  // frame slot in the block, thread within the frame
-    float2 *zf = zbuf + fl * N;                // this frame's storage
+                                           float (*err_part)[kMaxThreads / 64]) {
+    constexpr int N = 1 << LOGN, HALF = N / 2, TPF = N / 8;
+    constexpr bool ODD = LOGN & 1;
+    constexpr int PASSES = LOGN / 2;  // the last one included
+    const int tid = threadIdx.x, fpb = blockDim.x / TPF;
+    const int fl = tid / TPF, t = tid % TPF;  // frame slot in the block, thread within the frame
+    float2 *const zf = lds + fl * (N + N / 8);  // this frame's storage; a word of padding every eight
     const int Nw = p.Nw[res], Hs = p.Hs[res];
-    const float *__restrict__ win = p.window[res];
     const int wave_id = blockIdx.y;
     const int length = p.lengths[wave_id];
     const int Kvalid = frame_count(length, Nw, Hs);
-    const int kstep = p.nblocks[res] * FPB;  // frames between two passes of this block
-    const float *src = p.source + (size_t)wave_id * p.max_length;
-    const float *tgt = p.target + (size_t)wave_id * p.max_length;
+    const float *__restrict__ win = p.window[res];
+    const float *__restrict__ src = p.source + (size_t)wave_id * p.max_length;
+    const float *__restrict__ tgt = p.target + (size_t)wave_id * p.max_length;
     float *g = p.grad + (size_t)wave_id * p.max_length;
     const bool phase = p.zeta > 0.0f;
     const float inv = 1.0f / (float)((HALF + 1) * Kvalid);
     const float scale = phase ? inv : p.gamma * inv;
     float err = 0.0f, err_ph = 0.0f;
 
-    // windowed samples of frame k, source in x and target in y; zero outside the window, the waveform and Kvalid
-    auto fetch = [&](const int k, float2 (&v)[EPT]) {
-#pragma unroll
-        for (int e = 0; e < EPT; ++e) {
-            const int j = ft + e * TPF, pos = k * Hs + j;
-            v[e] = make_float2(0.0f, 0.0f);
-            if (k < Kvalid && j < Nw && pos < length) {
-                const float w = win[j];
-                v[e] = make_float2(src[pos] * w, tgt[pos] * w);
-            }
+    if ((int)blockIdx.x * fpb >= Kvalid) return;  // the same for every thread
+    const int k = blockIdx.x * fpb + fl;
+    const bool active = k < Kvalid;
+    const int start = active ? k * Hs : 0;
+
+    // frames of up to 64 threads lie inside one wave, whose LDS accesses run in order
+    auto exchange = [] {
+        if (TPF > 64) {
+            __syncthreads();
+        } else {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
         }
     };
-
-    int k0 = blockIdx.x * FPB;  // first frame of the pass; the same for every thread, so the barriers are uniform
-    if (k0 >= Kvalid) return;
-    for (int i = tid; i < N; i += 256) tw[i] = p.twiddle[res][i];
-    float2 cur[EPT];
-    fetch(k0 + fl, cur);
-    for (; k0 < Kvalid; k0 += kstep) {
-        const int k = k0 + fl;
-        const bool active = k < Kvalid;
+    auto at = [](int pos) { return pos + (pos >> 3); };
+    // windowed samples, source in x and target in y; zero outside the window, the waveform and Kvalid
+    float2 v[8];  // point m of the pass's butterfly b in v[2m + b]
+    float w[8];
 #pragma unroll
-        for (int e = 0; e < EPT; ++e) zf[ft + e * TPF] = cur[e];
-        __syncthreads();
-        // the next pass's samples travel while this pass computes
-        if (k0 + kstep < Kvalid) fetch(k + kstep, cur);
+    for (int e = 0; e < 8; ++e) {
+        const int j = t + e * TPF, pos = start + j, from = min(max(pos, 0), length - 1);
+        w[e] = win[min(j, Nw - 1)];
+        const float s = src[from] * w[e], r = tgt[from] * w[e];
+        v[e] = active && j < Nw && pos < length ? make_float2(s, r) : make_float2(0.0f, 0.0f);
+    }
+    // The table holds exp(-2 pi i k / 2^(s+1)) at 2^s + k for stage s.  A thread's two butterflies share their twiddles but in the
+    // first pass; those of the last pass are the same for all threads.
+    const float2 *__restrict__ table = p.twiddle[res];
+    Twiddles4 tw[PASSES - 1];
+    const Twiddles4 tw_second = {table[N / 2 + TPF + t], table[N / 4 + TPF + t]};
+#pragma unroll
+    for (int c = 0; c + 1 < PASSES; ++c) {
+        const int q = N / 4 >> 2 * c, j = t & (q - 1);
+        tw[c] = {table[2 * q + j], table[q + j]};
+    }
+    const Twiddles4 last0 = ODD ? Twiddles4{table[4], table[2]} : Twiddles4{table[2], table[1]}, last1 = {table[5], table[3]};
+    // the place of point m of butterfly b (0: t, 1: t + T) of pass c; in the last pass of the point 8t + r, r = 2m + b
+    auto place = [&](int c, int b, int m) {
+        if (c == PASSES - 1) return 9 * t + 2 * m + b;
+        const int q = N / 4 >> 2 * c, i = t + b * TPF;
+        return at(i / q * 4 * q + i % q + m * q);
+    };
+    // The thread that holds the bins N - b of this thread's bins b = bitrev(8t + r), r even, in register 7 - r.  Thread 0, whose
+    // bins are the multiples of N/8, holds its own: bin 0 (register 0) and N/2 (1) pair with themselves, register 4 with
+    // 7, 2 with 3, 6 with 5.
+    constexpr int TLOG = LOGN - 3;
+    const unsigned bin_t = __brev((unsigned)t) >> (32 - TLOG);
+    const int partner = (int)(__brev((TPF - bin_t) & (TPF - 1)) >> (32 - TLOG));
+    auto mirror = [&](int r) { return t == 0 ? (r == 4 ? 7 : r == 2 ? 3 : r == 6 ? 5 : 1) : 9 * partner + 7 - r; };
 
-        // forward: decimation in frequency, two stages (s, s - 1) per barrier as one radix-4 butterfly on the words
-        // base + {0, q, 2q, 3q}, q = 2^(s-1); the twiddle of the second pair of stage s is -i times the first's
-#pragma unroll 1
-        for (int s = LOGN - 1; s >= 1; s -= 2) {
-            const int q = 1 << (s - 1);
-            for (int i = ft; i < QUARTER; i += TPF) {
-                const int j = i & (q - 1);
-                const int base = ((i >> (s - 1)) << (s + 1)) + j;
-                const float2 x0 = zf[base], x1 = zf[base + q], x2 = zf[base + 2 * q], x3 = zf[base + 3 * q];
-                const float2 w1 = tw[2 * q + j], w2 = tw[q + j];
-                const float2 y0 = make_float2(x0.x + x2.x, x0.y + x2.y), d02 = make_float2(x0.x - x2.x, x0.y - x2.y);
-                const float2 y1 = make_float2(x1.x + x3.x, x1.y + x3.y), d13 = make_float2(x1.y - x3.y, x3.x - x1.x);
-                const float2 y2 = make_float2(d02.x * w1.x - d02.y * w1.y, d02.x * w1.y + d02.y * w1.x);
-                const float2 y3 = make_float2(d13.x * w1.x - d13.y * w1.y, d13.x * w1.y + d13.y * w1.x);
-                const float2 e01 = make_float2(y0.x - y1.x, y0.y - y1.y), e23 = make_float2(y2.x - y3.x, y2.y - y3.y);
-                zf[base] = make_float2(y0.x + y1.x, y0.y + y1.y);
-                zf[base + q] = make_float2(e01.x * w2.x - e01.y * w2.y, e01.x * w2.y + e01.y * w2.x);
-                zf[base + 2 * q] = make_float2(y2.x + y3.x, y2.y + y3.y);
-                zf[base + 3 * q] = make_float2(e23.x * w2.x - e23.y * w2.y, e23.x * w2.y + e23.y * w2.x);
-            }
-            __syncthreads();
-        }
-        if (LOGN & 1) {  // the last stage on its own: neighbours, twiddle 1
-            for (int i = ft; i < HALF; i += TPF) {
-                const float2 u = zf[2 * i], v = zf[2 * i + 1];
-                zf[2 * i] = make_float2(u.x + v.x, u.y + v.y);
-                zf[2 * i + 1] = make_float2(u.x - v.x, u.y - v.y);
-            }
-            __syncthreads();
-        }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) settle(v[e]);
+    // from the places of one pass to those of another
+    auto move = [&](int from, int to) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) zf[place(from, e & 1, e >> 1)] = v[e];
+        exchange();
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = zf[place(to, e & 1, e >> 1)];
+    };
+#pragma unroll
+    for (int c = 0; c + 1 < PASSES; ++c) {
+        butterfly4(v[0], v[2], v[4], v[6], tw[c]);
+        butterfly4(v[1], v[3], v[5], v[7], c == 0 ? tw_second : tw[c]);
+        move(c, c + 1);
+    }
+    if (ODD) {
+        butterfly4(v[0], v[2], v[4], v[6], last0);
+        butterfly4(v[1], v[3], v[5], v[7], last1);
+#pragma unroll
+        for (int r = 0; r < 8; r += 2) butterfly2(v[r], v[r + 1]);
+    } else {
+        butterfly4(v[0], v[1], v[2], v[3], last0);
+        butterfly4(v[4], v[5], v[6], v[7], last0);
+    }
 
-        // per-bin stage on the pairs (b, N-b); bin b lives at position bitrev(b)
-        // With the phase term both gradient spectra are weighted here and share the inverse transform (the
-        // reference runs a second framing / FFT / inverse FFT / overlap-add for it,
-        // layers/DFTErrorPostoutputLayer.cu:1246-1295).
-        // Stored position q holds bin bitrev(q).  Thread index t walks the even positions 2t (bins below N/2) and
-        // pairs each with the position of bin N - b, which for a wave's consecutive t are consecutive words too;
-        // walking the bins in natural order instead puts a wave's reads into two LDS banks.  Bins 0 (position 0)
-        // and N/2 (position 1) pair with themselves.
-        auto bin = [&](const int pb, const int pnb) {
-            const float2 zb = zf[pb], zn = zf[pnb];
-            // S = (Z[b] + conj(Z[N-b])) / 2,  T = (Z[b] - conj(Z[N-b])) / (2i)
-            const float sx = 0.5f * (zb.x + zn.x), sy = 0.5f * (zb.y - zn.y);
-            const float tx = 0.5f * (zb.y + zn.y), ty = -0.5f * (zb.x - zn.x);
-            float e, gx, gy;
-            bin_distance<DIS>(sx, sy, tx, ty, p.log_floor, e, gx, gy);
-            if (active) err += e;
-            if (phase) {
-                float pe, px, py;
-                bin_phase(sx, sy, tx, ty, pe, px, py);
-                if (active) err_ph += pe;
-                gx = p.gamma * gx + p.zeta * px;
-                gy = p.gamma * gy + p.zeta * py;
-            }
-            if (pb == pnb) {
-                zf[pb] = make_float2(gx, 0.0f);
-            } else {
-                zf[pb] = make_float2(gx, gy);
-                zf[pnb] = make_float2(gx, -gy);
-            }
-        };
-        for (int t = ft; t < HALF; t += TPF) {
-            const int b = (int)(__brev((unsigned)(2 * t)) >> (32 - LOGN));
-            const int pnb = (int)(__brev((unsigned)((N - b) & (N - 1))) >> (32 - LOGN));
-            bin(2 * t, pnb);
+    // Per-bin stage on the pairs (b, N - b).  The bins below N/2 are this thread's even registers, their partners another
+    // thread's odd ones: those are put into LDS, and what the pair leaves there is taken back.
+    // With the phase term both gradient spectra are weighted here and share the inverse transform (the
+    // reference runs a second framing / FFT / inverse FFT / overlap-add for it,
+    // layers/DFTErrorPostoutputLayer.cu:1246-1295).
+    auto bin = [&](const float2 zb, const float2 zn) {
+        // S = (Z[b] + conj(Z[N-b])) / 2,  T = (Z[b] - conj(Z[N-b])) / (2i)
+        const float sx = 0.5f * (zb.x + zn.x), sy = 0.5f * (zb.y - zn.y);
+        const float tx = 0.5f * (zb.y + zn.y), ty = -0.5f * (zb.x - zn.x);
+        float e, gx, gy;
+        bin_distance<DIS>(sx, sy, tx, ty, p.log_floor, e, gx, gy);
+        if (active) err += e;
+        if (phase) {
+            float pe, px, py;
+            bin_phase(sx, sy, tx, ty, pe, px, py);
+            if (active) err_ph += pe;
+            gx = p.gamma * gx + p.zeta * px;
+            gy = p.gamma * gy + p.zeta * py;
         }
-        if (ft == 0) bin(1, 1);
-        __syncthreads();
+        return make_float2(gx, gy);
+    };
+#pragma unroll
+    for (int r = 1; r < 8; r += 2) zf[9 * t + r] = v[r];
+    exchange();
+    float2 zn[4];
+#pragma unroll
+    for (int r = 0; r < 8; r += 2) zn[r / 2] = zf[mirror(r)];
+    if (t == 0) {
+        zn[0] = v[0];
+        v[1] = make_float2(bin(v[1], v[1]).x, 0.0f);
+    }
+#pragma unroll
+    for (int r = 0; r < 8; r += 2) {
+        v[r] = bin(v[r], zn[r / 2]);
+        settle(v[r]);
+        if (t == 0 && r == 0) v[0].y = 0.0f;
+        else zf[mirror(r)] = make_float2(v[r].x, -v[r].y);
+    }
+    exchange();
+#pragma unroll
+    for (int r = 1; r < 8; r += 2)
+        if (t != 0 || r != 1) v[r] = zf[9 * t + r];
 
-        // inverse: decimation in time with conjugated twiddles, unnormalised; stages (s - 1, s) per barrier
-        if (LOGN & 1) {
-            for (int i = ft; i < HALF; i += TPF) {
-                const float2 u = zf[2 * i], v = zf[2 * i + 1];
-                zf[2 * i] = make_float2(u.x + v.x, u.y + v.y);
-                zf[2 * i + 1] = make_float2(u.x - v.x, u.y - v.y);
-            }
-            __syncthreads();
-        }
-#pragma unroll 1
-        for (int s = 1 + (LOGN & 1); s < LOGN; s += 2) {
-            const int q = 1 << (s - 1);
-            for (int i = ft; i < QUARTER; i += TPF) {
-                const int j = i & (q - 1);
-                const int base = ((i >> (s - 1)) << (s + 1)) + j;
-                const float2 x0 = zf[base], x1 = zf[base + q], x2 = zf[base + 2 * q], x3 = zf[base + 3 * q];
-                const float2 w1 = tw[2 * q + j], w2 = tw[q + j];
-                const float2 v1 = make_float2(x1.x * w2.x + x1.y * w2.y, x1.y * w2.x - x1.x * w2.y);
-                const float2 v3 = make_float2(x3.x * w2.x + x3.y * w2.y, x3.y * w2.x - x3.x * w2.y);
-                const float2 y0 = make_float2(x0.x + v1.x, x0.y + v1.y), y1 = make_float2(x0.x - v1.x, x0.y - v1.y);
-                const float2 y2 = make_float2(x2.x + v3.x, x2.y + v3.y), y3 = make_float2(x2.x - v3.x, x2.y - v3.y);
-                const float2 u2 = make_float2(y2.x * w1.x + y2.y * w1.y, y2.y * w1.x - y2.x * w1.y);
-                const float2 t3 = make_float2(y3.x * w1.x + y3.y * w1.y, y3.y * w1.x - y3.x * w1.y);
-                const float2 u3 = make_float2(-t3.y, t3.x);  // conj(-i * w1) = i * conj(w1)
-                zf[base] = make_float2(y0.x + u2.x, y0.y + u2.y);
-                zf[base + q] = make_float2(y1.x + u3.x, y1.y + u3.y);
-                zf[base + 2 * q] = make_float2(y0.x - u2.x, y0.y - u2.y);
-                zf[base + 3 * q] = make_float2(y1.x - u3.x, y1.y - u3.y);
-            }
-            __syncthreads();
-        }
+    // inverse, unnormalised
+    if (ODD) {
+#pragma unroll
+        for (int r = 0; r < 8; r += 2) butterfly2(v[r], v[r + 1]);
+        inverse_butterfly4(v[0], v[2], v[4], v[6], last0);
+        inverse_butterfly4(v[1], v[3], v[5], v[7], last1);
+    } else {
+        inverse_butterfly4(v[0], v[1], v[2], v[3], last0);
+        inverse_butterfly4(v[4], v[5], v[6], v[7], last0);
+    }
+#pragma unroll
+    for (int c = PASSES - 2; c >= 0; --c) {
+        move(c + 1, c);
+        inverse_butterfly4(v[0], v[2], v[4], v[6], tw[c]);
+        inverse_butterfly4(v[1], v[3], v[5], v[7], c == 0 ? tw_second : tw[c]);
+    }
 
-        // windowed overlap-add; frames at or beyond Kvalid contribute nothing
-        if (active) {
-            for (int j = ft; j < Nw; j += TPF) {
-                const int pos = k * Hs + j;
-                if (pos < length) atomicAdd(&g[pos], scale * zf[j].x * win[j]);
-            }
+    // windowed overlap-add; frames at or beyond Kvalid contribute nothing
+    if (active) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int j = t + e * TPF, pos = start + j;
+            if (j < Nw && pos < length) atomicAdd(&g[pos], scale * v[e].x * w[e]);
         }
-        __syncthreads();  // the next pass overwrites the frame storage
     }
 
     for (int o = 32; o > 0; o >>= 1) {
@@ -312,7 +371,9 @@ __device__ __forceinline__ void dft_frames(const DftParams &p, const int res, fl
     }
     __syncthreads();
     if (tid < 2 && (tid == 0 || phase)) {
-        const float e = (err_part[tid][0] + err_part[tid][1] + err_part[tid][2] + err_part[tid][3]) * inv;
+        float e = 0.0f;
+        for (int q = 0; q < (int)blockDim.x / 64; ++q) e += err_part[tid][q];
+        e *= inv;
         if (e != 0.0f) atomicAdd(&p.errors[tid * p.n_waves * p.n_res + wave_id * p.n_res + res], e);
     }
 }
@@ -320,10 +381,10 @@ __device__ __forceinline__ void dft_frames(const DftParams &p, const int res, fl
 // All resolutions of a call in one launch: blockIdx.z selects the resolution, blockIdx.x the group of frames
 // (blocks beyond a resolution's last frame leave at once), blockIdx.y the waveform.
 template <int DIS>
-__global__ __launch_bounds__(256) void dft_loss_kernel(const DftParams p) {
+__global__ __launch_bounds__(kMaxThreads) void dft_loss_kernel(const DftParams p) {
     // sized by the launch for the call's longest transform; every instantiation places its tables at fixed offsets
     extern __shared__ __attribute__((aligned(16))) float2 dft_lds[];
-    __shared__ float err_part[2][4];
+    __shared__ float err_part[2][kMaxThreads / 64];
     const int res = blockIdx.z;
     if ((int)blockIdx.x >= p.nblocks[res]) return;
     switch (p.logn[res]) {
@@ -436,11 +497,6 @@ int cnt_dft_create(const cnt_dft_desc *desc, cnt_dft **out) {
     }
     if (err == hipSuccess)
         err = hipMalloc(reinterpret_cast<void **>(&h->grad), (size_t)desc->max_waves * desc->max_length * sizeof(float));
-    // a 4096-point transform takes 64 KB of LDS for its frame and twiddles, beyond what a launch may ask for unannounced
-    for (int r = 0; r < desc->n_res && err == hipSuccess; ++r)
-        if (desc->fft_length[r] > 2048)
-            err = hipFuncSetAttribute(reinterpret_cast<const void *>(pick_dft_kernel(desc->spec_dis_type)),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 4096 * (int)sizeof(float2));
     if (err != hipSuccess) {
         set_error("dft_create: %s", hipGetErrorString(err));
         cnt_dft_destroy(h);
@@ -488,34 +544,18 @@ int cnt_dft_forward(cnt_dft *h, void *stream_, int n_waves, const int *lengths, 
     DftParams p;
     fill_params(h, p);
     p.source = source; p.target = target; p.errors = errors_dev;
-    // A block of a short transform makes several passes over its waveform's frames, so that the blocks of all
-    // resolutions carry about the work of one pass of the longest transform (work per pass: N * log2 N per frame,
-    // 256 / (N/4) frames per pass below N = 1024).
-    const long max_passes = 8;
-    int gx = 1;
-    long work_max = 1;
-    size_t lds_bytes = 0;
+    // a workgroup transforms eight points per thread, whatever the transforms' length
+    int threads = 256, gx = 1;
+    for (int r = 0; r < h->desc.n_res; ++r) threads = p.logn[r] > 11 ? kMaxThreads : threads;
     for (int r = 0; r < h->desc.n_res; ++r) {
-        const long n = h->desc.fft_length[r];
-        const long w = (n < 1024 ? 1024 : n) * p.logn[r];
-        work_max = w > work_max ? w : work_max;
-        const size_t b = (size_t)((n < 1024 ? 1024 : n) + n) * sizeof(float2);
-        lds_bytes = b > lds_bytes ? b : lds_bytes;
+        const int fpb = threads * 8 >> p.logn[r];
+        p.nblocks[r] = (frame_count(max_len, p.Nw[r], p.Hs[r]) + fpb - 1) / fpb;
+        gx = std::max(gx, p.nblocks[r]);
     }
-    for (int r = 0; r < h->desc.n_res; ++r) {
-        const long n = h->desc.fft_length[r];
-        const int quarter = (int)(n / 4);
-        const int fpb = quarter < 256 ? 256 / quarter : 1;
-        const int kmax = frame_count(max_len, p.Nw[r], p.Hs[r]);
-        long passes = work_max / ((n < 1024 ? 1024 : n) * p.logn[r]);
-        passes = passes < 1 ? 1 : passes > max_passes ? max_passes : passes;
-        const int groups = (kmax + fpb - 1) / fpb;
-        p.nblocks[r] = (int)((groups + passes - 1) / passes);
-        gx = p.nblocks[r] > gx ? p.nblocks[r] : gx;
-    }
+    const size_t lds_bytes = (size_t)threads * 9 * sizeof(float2);
     {
         ProfileScope prof(stream, "dft_loss");
-        hipLaunchKernelGGL(pick_dft_kernel(h->desc.spec_dis_type), dim3(gx, n_waves, h->desc.n_res), dim3(256), lds_bytes, stream,
+        hipLaunchKernelGGL(pick_dft_kernel(h->desc.spec_dis_type), dim3(gx, n_waves, h->desc.n_res), dim3(threads), lds_bytes, stream,
                            p);
         CNT_HIP(hipGetLastError());
     }

@@ -24,6 +24,19 @@ def test_dft_loss(res, max_len, lengths):
     assert PC.run_dft_case(res, max_len, lengths, seed=len(res) + max_len, gamma=0.8) < TOL
 
 
+# every transform length alone, with the complex spectral distance, which is linear in the spectra: a last workgroup that is
+# partly filled, windows that end inside a thread's points, one frame (and a frame shift whose multiples leave 32 bits).  The
+# bound is two transforms of log2 N stages, each rounding to 2^-24, the few frames that add to a sample, and what the oracle
+# loses where it adds up to 2 distances per sample one after the other in fp32 (a random walk of that many roundings).
+@pytest.mark.parametrize("logn", range(5, 13))
+@pytest.mark.parametrize("shrink,shift,samples", [(0, 3, 9000), (5, 2, 4103), (0, 1 << 30, 4096)])
+def test_dft_every_length(logn, shrink, shift, samples):
+    n = 1 << logn
+    hop = n // shift if shift < 10 else shift
+    print("dft length", n, shrink, hop, samples, flush=True)
+    assert PC.run_dft_case([(n, n - shrink, hop)], samples, [samples, samples - 1], seed=logn, dis_type=4) < (2 * logn + 8 + (2 * samples) ** 0.5) * 2.0 ** -24
+
+
 def test_dft_loss_config5_full_size():
     """benchmark config 5 at its size: 8 waveforms x 16000 samples (two of them shorter), the three resolutions."""
     print("dft config 5 full size", flush=True)
