@@ -335,13 +335,17 @@ int fill_zero(hipStream_t stream, float *p, size_t count);
 // two buffers in one launch
 int fill_zero_pair(hipStream_t stream, float *p, size_t count, float *q, size_t count_q);
 // What a network does on the device when a fraction is loaded, as ONE launch: up to kLoadClears buffers zeroed (the
-// recurrent layers' stored output-gate deltas) and, when `order` is given, the fraction's slot order built (as
-// slot_order_build does).
-constexpr int kLoadClears = 8;
+// recurrent layers' stored output-gate deltas), up to two copied (inputs and targets, from memory of this device) and, when
+// `order` is given, the fraction's slot order built (as slot_order_build does).
+constexpr int kLoadClears = 8, kLoadCopies = 2;
 struct LoadClears {
     float *ptr[kLoadClears];
     unsigned long long count[kLoadClears];  // floats, multiples of four, 16-byte aligned buffers
     int n;
+    const float *from[kLoadCopies];
+    float *to[kLoadCopies];
+    unsigned long long copy_count[kLoadCopies];  // floats
+    int copies;
 };
 int load_clear_and_order(hipStream_t stream, const LoadClears &clears, const char *pat, int n_slots, int slots_per_step,
                          int *order, int *count);

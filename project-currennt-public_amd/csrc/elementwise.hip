@@ -178,7 +178,8 @@ __global__ __launch_bounds__(kOrderThreads) void slot_order_kernel(const char *_
     slot_order_block(pat, n, per_step, order, count);
 }
 
-// workgroup 0 builds the slot order (when there is one to build), the others zero the listed buffers with 16-byte stores
+// workgroup 0 builds the slot order (when there is one to build), the others zero the listed buffers with 16-byte stores and
+// make the copies, 16 bytes at a time where both ends are aligned
 __global__ __launch_bounds__(kOrderThreads) void load_clear_and_order_kernel(const LoadClears c, const char *__restrict__ pat,
                                                                              int n, int per_step, int *__restrict__ order,
                                                                              int *__restrict__ count) {
@@ -193,6 +194,13 @@ __global__ __launch_bounds__(kOrderThreads) void load_clear_and_order_kernel(con
         const size_t n4 = c.count[b] / 4;
         for (size_t i = first; i < n4; i += stride) p[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
+    for (int b = 0; b < c.copies; ++b) {
+        const float *from = c.from[b];
+        float *to = c.to[b];
+        const size_t n4 = ((reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(to)) & 15) == 0 ? c.copy_count[b] / 4 : 0;
+        for (size_t i = first; i < n4; i += stride) reinterpret_cast<float4 *>(to)[i] = reinterpret_cast<const float4 *>(from)[i];
+        for (size_t i = 4 * n4 + first; i < c.copy_count[b]; i += stride) to[i] = from[i];
+    }
 }
 
 }  // namespace
@@ -201,11 +209,13 @@ int load_clear_and_order(hipStream_t stream, const LoadClears &clears, const cha
                          int *order, int *count) {
     CNT_REQUIRE(clears.n >= 0 && clears.n <= kLoadClears, "load_clear_and_order: %d buffers", clears.n);
     CNT_REQUIRE(!order || (pat && count && n_slots > 0 && slots_per_step > 0), "load_clear_and_order: bad slot order argument");
-    if (clears.n == 0 && !order) return CNT_OK;
+    CNT_REQUIRE(clears.copies >= 0 && clears.copies <= kLoadCopies, "load_clear_and_order: %d copies", clears.copies);
+    if (clears.n == 0 && clears.copies == 0 && !order) return CNT_OK;
     size_t floats = 0;
     for (int b = 0; b < clears.n; ++b) floats += clears.count[b];
-    const unsigned fill_blocks = clears.n ? (unsigned)std::min<size_t>((floats / 4 + kOrderThreads - 1) / kOrderThreads, 1024) : 0;
-    hipLaunchKernelGGL(load_clear_and_order_kernel, dim3(1 + fill_blocks), dim3(kOrderThreads), 0, stream, clears, pat, n_slots,
+    for (int b = 0; b < clears.copies; ++b) floats += clears.copy_count[b];
+    const unsigned others = (unsigned)std::min<size_t>((floats / 4 + kOrderThreads - 1) / kOrderThreads, 1024);
+    hipLaunchKernelGGL(load_clear_and_order_kernel, dim3(1 + std::max(others, clears.n + clears.copies ? 1u : 0u)), dim3(kOrderThreads), 0, stream, clears, pat, n_slots,
                        slots_per_step, order, count);
     CNT_HIP(hipGetLastError());
     return CNT_OK;

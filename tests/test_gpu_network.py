@@ -411,6 +411,29 @@ def test_wavenet_network_file_against_oracle_graph(nb, cnn_tanh, R, K, Q, C, len
     net.close()
 
 
+# inputs and targets that start on and off a 16-byte boundary, counts that are no multiple of four, with and without a slot order
+# and recurrent layers' clears beside the copies
+@pytest.mark.parametrize("shift", [0, 1, 2])
+@pytest.mark.parametrize("P,D,lengths,recurrent", [(1, 3, [1], False), (3, 5, [7, 4], True), (37, 2, [300, 299, 151], True), (382, 187, [600] * 10, False)])
+def test_inputs_and_targets_of_any_alignment(shift, P, D, lengths, recurrent):
+    import torch
+
+    S, T = len(lengths), max(lengths)
+    N = S * T
+    mid = [{"size": 32, "name": "l", "type": "lstm", "bias": 1.0}] if recurrent else []
+    net = PC.pkg().capi.Network(json.dumps({"layers": [{"size": P, "name": "input", "type": "input"}] + mid + [
+        {"size": D, "name": "o", "type": "feedforward_identity", "bias": 1.0}, {"size": D, "name": "post", "type": "sse"}]}), S, T + 3)
+    x, y = torch.randn(P * N + shift, device="cuda")[shift:], torch.randn(D * N + shift, device="cuda")[shift:]
+    net.layers[0]["outputs"].fill_(9.0)
+    net.layers[-1]["outputs"].fill_(9.0)
+    net.load_sequences(PC.dev(make_pat_types(lengths, T)), T, min(lengths), x, y)
+    torch.cuda.synchronize()
+    for layer, given in ((net.layers[0], x), (net.layers[-1], y)):
+        assert torch.equal(layer["outputs"][: given.numel()], given)
+        assert bool((layer["outputs"][given.numel():] == 9.0).all())
+    net.close()
+
+
 # slots of one lane, of a few, of a wave and of more than one store per lane; the columns taken from the layer before end
 # inside a group of four; sizes that are no multiple of four
 @pytest.mark.parametrize("P,lo,hi,Q,lengths", [(3, 0, 3, 1, [4, 2]), (3, 1, 3, 6, [1]), (5, 0, 5, 30, [9, 4, 7]), (6, 2, 5, 253, [31, 30]),
