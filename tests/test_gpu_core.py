@@ -85,6 +85,15 @@ def test_lstm(P, L, bidir, lengths):
     assert PC.run_lstm_case(P, L, bidir, lengths, seed=len(lengths) + L) < TOL
 
 
+# the sums over the patterns with two cells and one cell per thread: a workgroup's cells and one more, chunks that end inside
+# a row of workgroups' patterns
+@pytest.mark.parametrize("P,L,bidir,lengths", [(3, 2, True, [5, 2]), (4, 500, True, [9, 8]), (5, 258, False, [17, 3]), (5, 257, False, [16]),
+                                               (6, 30, True, [2100, 1999]), (3, 7, False, [700] * 6)])
+def test_lstm_bias_and_peephole_gradients(P, L, bidir, lengths):
+    print("lstm bias and peepholes", P, L, bidir, lengths, flush=True)
+    assert PC.run_lstm_case(P, L, bidir, lengths, seed=L) < TOL
+
+
 def test_lstm_clip_and_repeat_backward():
     """Large errors activate the [-1,1] clip; a second backward without load_sequences adds the stored
     output-gate deltas, as in the reference."""
