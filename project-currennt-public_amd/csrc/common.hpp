@@ -354,6 +354,9 @@ int load_clear_and_order(hipStream_t stream, const LoadClears &clears, const cha
 int lstm_load_sequences_collect(cnt_lstm *h, hipStream_t stream, const char *patTypes, int curMaxT, int curMinT,
                                 LoadClears &clears);
 int fill_words(hipStream_t stream, unsigned *p, size_t count, unsigned word);
+// cnt_sse_error and cnt_sse_backward in one launch; sum: 64 words of the caller's that are zero between calls
+int sse_error_backward(hipStream_t stream, int D, int N, const char *patTypes, const float *y, const float *target, float *err,
+                       float *result_dev, float *sum);
 // out[d] += scale * sum over the N columns of a D x N column-major matrix (out pre-zeroed by the caller)
 int column_sum(hipStream_t stream, const float *v, int D, int N, float scale, float *out);
 

@@ -215,7 +215,8 @@ struct NetLayer {
     std::vector<int> cat_lo, cat_hi;         // skipcat: dimension range taken from each source
     const float *ext_data = nullptr;         // externalloader: [frame][sequence][dimension], set by the caller
     const float *ext_mean_std = nullptr;
-    bool mdn_errors_done = false;            // mdn: calculate_error has already written the preceding layer's errors
+    bool post_errors_done = false;           // sse, mdn: calculate_error has already written the preceding layer's errors
+    float *loss_sum = nullptr;               // sse: see sse_error_backward
     int ext_frames = 0, index_load_method = 0;
     int cnn_tanh = 0;                        // cnn: "tanhoutput"
     bool delta_fused = false;                // cnn followed by a wavnetc layer: that layer writes this layer's delta
@@ -1061,6 +1062,7 @@ int finish_build(cnt_network *net, const json::Value *weights) {
     {
         const char *e = std::getenv("CNT_NET_SKIP_PADDING");
         net->skip_padding = !e || std::atoi(e) != 0;
+        if (net->layers.back().kind == K_SSE) CNT_TRY(device_alloc(net, (void **)&net->layers.back().loss_sum, 64 * sizeof(float), true));
         CNT_TRY(device_alloc(net, (void **)&net->order, ((size_t)net->S * net->maxT + 4) * sizeof(int), true));
         net->order_count = net->order + (size_t)net->S * net->maxT;
     }
@@ -1285,6 +1287,7 @@ int cnt_network_load_sequences(cnt_network *net, void *stream_, int T, int Tmin,
     CNT_REQUIRE(T >= 1 && T <= net->maxT && Tmin >= 1 && Tmin <= T, "network_load_sequences: lengths %d / %d outside "
                 "1..%d", T, Tmin, net->maxT);
     hipStream_t stream = static_cast<hipStream_t>(stream_);
+    net->layers.back().post_errors_done = false;
     net->T = T;
     net->Tmin = Tmin;
     net->pat = patTypes;
@@ -1363,6 +1366,11 @@ bool fuse_blocks() {
     return on;
 }
 
+bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
+}
+
 // WaveNet residual block seen from its skip 1x1 layer i: [cnn 2R][wavnetc R][dense R, identity][skipadd, shares
 // the following sum][skipini][dense K, identity (i)]
 bool block_errors_at(const cnt_network *net, size_t i) {
@@ -1401,11 +1409,8 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
     // stack of WaveNet blocks, where the block launches hand the sums on, none (30 blocks of 64 channels on 32 000
     // samples: 500 MB less to write per pass, 184 us).  A pass under capture may be replayed after backward passes that
     // are not known yet, so it clears all side buffers.
-    bool all = false;
-    if (!net->sides.empty()) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        all = hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
-    }
+    const bool all = !net->sides.empty() && capturing(stream);
+    net->layers.back().post_errors_done = false;  // errors written for other outputs do not count
     size_t lo = 0, hi = net->skip_always, at = hi;  // [lo, hi): the run to clear that has not ended yet
     for (const auto &side : net->sides) {
         if (all || side.touched) {
@@ -1533,7 +1538,7 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
             }
             case K_MDN:
                 CNT_TRY(cnt_mdn_forward(L.mdn, stream, prev.out));
-                L.mdn_errors_done = false;  // new parameters: errors written for the old ones do not count
+                L.post_errors_done = false;  // new parameters: errors written for the old ones do not count
                 break;
             case K_GATED:
                 CNT_TRY(cnt_gatedact_forward(stream, L.size, N, L.pat, prev.out, L.out));
@@ -1557,7 +1562,13 @@ int cnt_network_calculate_error(cnt_network *net, void *stream_, float *loss_dev
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     NetLayer &post = net->layers.back();
     const NetLayer &last = net->layers[net->layers.size() - 2];
-    if (post.kind == K_SSE) return cnt_sse_error(stream, post.size, post.N, post.pat, last.out, post.out, loss_dev);
+    if (post.kind == K_SSE) {
+        // (as with a mixture layer below: both passes read outputs and targets)
+        if (!last.err) return cnt_sse_error(stream, post.size, post.N, post.pat, last.out, post.out, loss_dev);
+        CNT_TRY(sse_error_backward(stream, post.size, post.N, post.pat, last.out, post.out, last.err, loss_dev, post.loss_sum));
+        post.post_errors_done = true;
+        return CNT_OK;
+    }
     if (post.kind == K_DFT) {
         // DFTPostoutputLayer::calculateError (layers/DFTErrorPostoutputLayer.cu:2105-2150): the plain sum of the
         // distances of every resolution
@@ -1570,7 +1581,7 @@ int cnt_network_calculate_error(cnt_network *net, void *stream_, float *loss_dev
     // The preceding layer's error buffer has no other writer between the forward pass and the backward pass.
     if (last.err) {
         CNT_TRY(cnt_mdn_error_backward(post.mdn, stream, post.out, loss_dev, last.err));
-        post.mdn_errors_done = true;
+        post.post_errors_done = true;
         return CNT_OK;
     }
     return cnt_mdn_calculate_error(post.mdn, stream, post.out, loss_dev);
@@ -1754,11 +1765,17 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         const size_t count = (size_t)L.size * N;
         switch (L.kind) {
             case K_SSE:
+                // already written by cnt_network_calculate_error of this fraction's forward pass (a captured pass may be replayed
+                // without it)
+                if (L.post_errors_done) {
+                    L.post_errors_done = false;  // a layer below turns them into its deltas in place
+                    if (!capturing(stream)) break;
+                }
                 CNT_TRY(cnt_sse_backward(stream, L.size, N, L.pat, prev.out, L.out, prev.err));
                 break;
             case K_MDN:
                 // already written by cnt_network_calculate_error of this fraction's forward pass
-                if (L.mdn_errors_done) L.mdn_errors_done = false;
+                if (L.post_errors_done) L.post_errors_done = false;
                 else CNT_TRY(cnt_mdn_backward(L.mdn, stream, L.out, prev.err));
                 break;
             case K_DFT:

@@ -434,6 +434,36 @@ def test_inputs_and_targets_of_any_alignment(shift, P, D, lengths, recurrent):
     net.close()
 
 
+# slots of one lane, of a part of a wave, of a wave and more; one workgroup, several, and more slots than they take at a time
+@pytest.mark.parametrize("D,lengths", [(1, [1]), (3, [700, 650]), (16, [40, 3]), (64, [5]), (65, [300, 299]), (187, [600] * 9 + [20])])
+def test_squared_error_with_its_gradient(D, lengths):
+    import torch
+
+    S, T = len(lengths), max(lengths)
+    N = S * T
+    net = PC.pkg().capi.Network(json.dumps({"layers": [{"size": 2, "name": "input", "type": "input"},
+                                                       {"size": D, "name": "o", "type": "feedforward_identity", "bias": 1.0},
+                                                       {"size": D, "name": "post", "type": "sse"}]}), S, T)
+    net.randomize(3, 0.3)
+    pat = make_pat_types(lengths, T)
+    x, t = torch.randn(2 * N, device="cuda"), torch.randn(D * N, device="cuda")
+    net.load_sequences(PC.dev(pat), T, min(lengths), x, t)
+    valid = PC.dev(pat).view(N, 1) != 0
+    for repeat in range(3):
+        net.forward()
+        for _ in range(2):
+            loss = float(net.calculate_error().item())
+        if repeat == 1:
+            net.backward()  # uses the errors up
+        net.backward()
+        torch.cuda.synchronize()
+        want = torch.where(valid, net.layer("o")["outputs"][: N * D].view(N, D) - t.view(N, D), 0.0)
+        assert torch.equal(net.layer("o")["errors"][: N * D].view(N, D), want)
+        exact = 0.5 * float((want.double() ** 2).sum())
+        assert abs(loss - exact) <= (N * D / 256 + 300) * 2.0 ** -24 * exact  # a thread's chain, waves, workgroups
+    net.close()
+
+
 # slots of one lane, of a few, of a wave and of more than one store per lane; the columns taken from the layer before end
 # inside a group of four; sizes that are no multiple of four
 @pytest.mark.parametrize("P,lo,hi,Q,lengths", [(3, 0, 3, 1, [4, 2]), (3, 1, 3, 6, [1]), (5, 0, 5, 30, [9, 4, 7]), (6, 2, 5, 253, [31, 30]),
