@@ -65,6 +65,10 @@ inline int pick_vec(const GemmArgs &a, bool for_a) {
 // launch needs some 600 of them, and a run over k long enough that filling and draining the pipeline does not show
 // (64 / 128, us: 1024 x 12000 x 1024 with 752 large tiles 200 / 165; 1024 x 6000 x 512 with 376 of them 54 / 56; 512 x
 // 6000 x 512 with 188 30 / 51; 1024 x 32000 x 128 with 2000 71 / 103).
+// Between 256 and 511 values of k it is the last generation that decides: large tiles pay where they fill what the chip holds of
+// them at a time (768) to at least nine tenths.  64 / 128, us, for 1024 rows and a k-contiguous A: k = 256, 752 tiles (0.98) 54 /
+// 49, 704 (0.92) 1.05 times as fast, 1360 (0.89) 1.02, 2000 (0.87) 0.97, 640 (0.83) 1.04, 1040 (0.68) 0.87; k = 448, 752 tiles 86 /
+// 72, 1360 1.09 times, 1040 0.98; a row-contiguous A within 3% of that; 1936 x 6000 x 256 59 / 50; k = 192 no gain anywhere.
 inline long large_tiles(const GemmArgs &a) { return (long)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.nprob; }
 
 // The weight gradient of one dense layer of 64 to 256 large tiles (1024 x 1024 weights and more) also takes the large tile, and
@@ -92,7 +96,9 @@ int pick_tile(const GemmArgs &a) {
     if (forced == 64 || forced == 128) return forced;
     const long t128 = large_tiles(a) * a.splitk;
     if (wide_gradient(a) && t128 >= kWideGradientGroups / 2) return 128;
-    return t128 >= 600 && (long)a.k * a.nseg / a.splitk >= 512 ? 128 : 64;
+    const long run = (long)a.k * a.nseg / a.splitk;
+    const bool quads = (a.a_kcontig ? a.k : a.m) % 4 == 0 && a.b_kcontig && a.k % 4 == 0;  // 768 at a time
+    return t128 >= 600 && (run >= 512 || (run >= 256 && quads && 10 * t128 >= 9 * ((t128 + 767) / 768 * 768))) ? 128 : 64;
 }
 
 // ----- split-K through partial products ---------------------------------------------------------------------

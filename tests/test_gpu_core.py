@@ -628,6 +628,17 @@ def test_matrix_product_of_few_blocks(m, n, k, tA, tB):
     assert bool(((C - A64 @ B64).abs() <= bound)[1:m - 1].all())
 
 
+@pytest.mark.parametrize("m,n,k,tA,tB", [(1024, 11900, 256, True, False), (1024, 11900, 256, False, False), (1012, 12001, 300, True, False),
+                                         (1936, 5999, 508, False, False), (1024, 11000, 252, True, False)])
+def test_matrix_product_of_short_runs_and_full_generations(m, n, k, tA, tB):
+    """Both sides of the line between the tile sizes for 256 to 511 values of k; rows and columns that end inside a tile."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    A, B = torch.randn(m * k, device="cuda", generator=g), torch.randn(n * k, device="cuda", generator=g)
+    C, A64, B64 = _product(m, n, k, tA, tB, A, B)
+    assert bool(((C - A64 @ B64).abs() <= (k + 2) * 2.0 ** -24 * (A64.abs() @ B64.abs())).all())
+
+
 @pytest.mark.parametrize("static", [False, True])
 @pytest.mark.parametrize("P,D,N", [(32, 32, 16), (20, 33, 120), (37, 35, 130), (5, 4, 7), (3, 60, 200), (60, 2, 200), (256, 2048, 100), (288, 2048, 100),
                                    (100, 90, 2048), (100, 90, 2049)])
