@@ -68,7 +68,11 @@ inline int pick_vec(const GemmArgs &a, bool for_a) {
 // Between 256 and 511 values of k it is the last generation that decides: large tiles pay where they fill what the chip holds of
 // them at a time (768) to at least nine tenths.  64 / 128, us, for 1024 rows and a k-contiguous A: k = 256, 752 tiles (0.98) 54 /
 // 49, 704 (0.92) 1.05 times as fast, 1360 (0.89) 1.02, 2000 (0.87) 0.97, 640 (0.83) 1.04, 1040 (0.68) 0.87; k = 448, 752 tiles 86 /
-// 72, 1360 1.09 times, 1040 0.98; a row-contiguous A within 3% of that; 1936 x 6000 x 256 59 / 50; k = 192 no gain anywhere.
+// 72, 1360 1.09 times, 1040 0.98; a row-contiguous A within 3% of that; 1936 x 6000 x 256 59 / 50; k = 192 no gain anywhere.  From
+// 768 values on they pay from 336 tiles on (300 / 336 / 376 / 480 / 560 tiles, times as fast: k = 768 0.84 / 1.00 / 1.01 / 1.17 /
+// 1.03, k = 2048 0.94 / 1.11 / 1.11 / 1.28 / 1.10; 1024 x 6144 x 2048 170 / 132 us), and with 512 to 767 values they lose 1 to 10 % where
+// they begin a second generation that stays a quarter full or less (800 / 896 / 960 / 1040 tiles of k = 512 0.90 / 0.93 / 0.98 /
+// 1.06).
 inline long large_tiles(const GemmArgs &a) { return (long)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.nprob; }
 
 // The weight gradient of one dense layer of 64 to 256 large tiles (1024 x 1024 weights and more) also takes the large tile, and
@@ -98,7 +102,10 @@ int pick_tile(const GemmArgs &a) {
     if (wide_gradient(a) && t128 >= kWideGradientGroups / 2) return 128;
     const long run = (long)a.k * a.nseg / a.splitk;
     const bool quads = (a.a_kcontig ? a.k : a.m) % 4 == 0 && a.b_kcontig && a.k % 4 == 0;  // 768 at a time
-    return t128 >= 600 && (run >= 512 || (run >= 256 && quads && 10 * t128 >= 9 * ((t128 + 767) / 768 * 768))) ? 128 : 64;
+    if (!quads) return t128 >= 600 && run >= 512 ? 128 : 64;
+    if (run >= 768) return t128 >= 336 ? 128 : 64;
+    if (run >= 512) return t128 >= 600 && (t128 <= 768 || t128 > 960) ? 128 : 64;
+    return t128 >= 600 && run >= 256 && 10 * t128 >= 9 * ((t128 + 767) / 768 * 768) ? 128 : 64;
 }
 
 // ----- split-K through partial products ---------------------------------------------------------------------
