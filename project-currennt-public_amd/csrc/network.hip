@@ -1368,7 +1368,9 @@ bool fuse_blocks() {
 
 bool capturing(hipStream_t stream) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) == hipSuccess) return capture != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
 }
 
 // WaveNet residual block seen from its skip 1x1 layer i: [cnn 2R][wavnetc R][dense R, identity][skipadd, shares
