@@ -2063,9 +2063,13 @@ int cnt_network_update(cnt_network *net, void *stream_, int option, float learni
         CNT_REQUIRE(net->stats_option < 0, "network_update: the optimizer option changed from %d to %d", net->stats_option,
                     option);
         // optimizers/Optimizer.cu:427-447: AdaGrad statistics start at 1e-6, Adam's (m, v) pairs at 0
-        std::vector<float> init(adam ? 2 * n : n, adam ? 0.0f : 1e-6f);
-        CNT_TRY(device_alloc(net, (void **)&net->stats, init.size() * sizeof(float), false));
-        CNT_HIP(hipMemcpy(net->stats, init.data(), init.size() * sizeof(float), hipMemcpyHostToDevice));
+        // (filled on the device: 42 MB for the feed-forward model's five million weights took 5 ms from the host)
+        const float start = adam ? 0.0f : 1e-6f;
+        unsigned word;
+        std::memcpy(&word, &start, sizeof(word));
+        const size_t count = adam ? 2 * n : n;
+        CNT_TRY(device_alloc(net, (void **)&net->stats, count * sizeof(float), false));
+        CNT_TRY(fill_words(static_cast<hipStream_t>(stream_), reinterpret_cast<unsigned *>(net->stats), count, word));
         net->stats_option = option;
     }
     if (adam) {
