@@ -306,7 +306,7 @@ int wavenet_block_errors(hipStream_t stream, int R, int K, int N, const char *pa
                          const float *core_buf, float *ctx_tanh, const float *conv_tanh_outputs, float *conv_errors,
                          const cnt_cnn *fold, const float *fold_weights, const float *fold_deltas, float *colsum_partial);
 // workgroups of that launch = rows of `colsum_partial` ([rows][2R]: per-workgroup sums of conv_errors over the samples)
-int wavenet_block_rows(int N, bool fold);
+int wavenet_block_rows(int R, int N, bool fold);
 int wavnetc_context_grad(hipStream_t stream, int D, int C, int N, const float *weights, const float *ctx_tanh,
                          float *ctx_grad);
 int cnn_backward_errors_fan(cnt_cnn *h, hipStream_t stream, const char *patTypes, int curT, const float *weights,

@@ -1842,7 +1842,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                                                      cnn.err, fold ? fold->cnn : nullptr,
                                                      fold ? net->weights + fold->w_off : nullptr, fold ? fold->err : nullptr,
                                                      cnn.colsum));
-                        if (cnn.colsum) net->layers[i - 5].colsum_rows = wavenet_block_rows(N, fold != nullptr);
+                        if (cnn.colsum) net->layers[i - 5].colsum_rows = wavenet_block_rows(prev.size, N, fold != nullptr);
                         fan_done[i - 1] = 1;
                         errors_done[i - 3] = errors_done[i - 4] = 1;
                         goto weight_half_of_layer;

@@ -208,10 +208,9 @@ typedef float f32x4v __attribute__((ext_vector_type(4)));
 
 // SUM: the gate's pre-activations are formed again from the convolution's outputs and the conditioning part, which the
 // launch reads anyway; `pre` is not read then.
-template <int R, int K, bool CONV, bool SUM>
-__global__ __launch_bounds__(CONV ? 512 : 256, (CONV || K > 128) ? 1 : 2) void wavenet_block_errors_kernel(const BlockErrArgs a) {
+template <int R, int K, bool CONV, bool SUM, int NT>
+__global__ __launch_bounds__(NT, (CONV || K > 128) ? 1 : 2) void wavenet_block_errors_kernel(const BlockErrArgs a) {
     static_assert(R % 16 == 0 && K % 16 == 0 && R <= 128, "block geometry");
-    constexpr int NT = CONV ? 512 : 256;  // the folded convolution's weights take 2 x 2R x R words of LDS more
     constexpr int RT = R / 16;  // channel tiles
     constexpr int KJ = K / 16, RJ = R / 16, CJ = 2 * R / 16;
     // A operands: [tile][j][lane = 16*quarter + channel in tile][i] = W[16j + 4*quarter + i][16*tile + channel]
@@ -534,13 +533,15 @@ __global__ void fill_zero_list_kernel(const FillList f) {
 
 typedef void (*block_err_kernel_t)(const BlockErrArgs);
 template <int R, int K>
-block_err_kernel_t block_errors_of(bool conv, bool sum) {
-    return conv ? (sum ? wavenet_block_errors_kernel<R, K, true, true> : wavenet_block_errors_kernel<R, K, true, false>)
-                : (sum ? wavenet_block_errors_kernel<R, K, false, true> : wavenet_block_errors_kernel<R, K, false, false>);
+block_err_kernel_t block_errors_of(bool conv, bool sum, int threads) {
+    if constexpr (R > 32)
+        if (threads == 512) return sum ? wavenet_block_errors_kernel<R, K, true, true, 512> : wavenet_block_errors_kernel<R, K, true, false, 512>;
+    return conv ? (sum ? wavenet_block_errors_kernel<R, K, true, true, 256> : wavenet_block_errors_kernel<R, K, true, false, 256>)
+                : (sum ? wavenet_block_errors_kernel<R, K, false, true, 256> : wavenet_block_errors_kernel<R, K, false, false, 256>);
 }
-block_err_kernel_t pick_block_errors_kernel(int R, int K, bool conv, bool sum) {
+block_err_kernel_t pick_block_errors_kernel(int R, int K, bool conv, bool sum, int threads) {
 #define CNT_BLOCK_KERNEL(r, k) \
-    if (R == r && K == k) return block_errors_of<r, k>(conv, sum);
+    if (R == r && K == k) return block_errors_of<r, k>(conv, sum, threads);
     CNT_BLOCK_KERNEL(64, 128)
     CNT_BLOCK_KERNEL(64, 256)
     CNT_BLOCK_KERNEL(64, 64)
@@ -1000,9 +1001,20 @@ extern "C++" int cnt::wavenet_block_forward(hipStream_t stream, const cnt_cnn *c
     return CNT_OK;
 }
 
-extern "C++" bool cnt::wavenet_block_errors_supported(int R, int K) { return pick_block_errors_kernel(R, K, false, false) != nullptr; }
+extern "C++" bool cnt::wavenet_block_errors_supported(int R, int K) { return pick_block_errors_kernel(R, K, false, false, 256) != nullptr; }
 
-extern "C++" int cnt::wavenet_block_rows(int N, bool fold) { return fold ? (N + 127) / 128 : (N + 63) / 64; }
+// Threads of a workgroup, four samples' worth of a wave each: 64 samples per workgroup put a short waveform on twice as many
+// compute units and wait for half as many waves at a barrier, 128 read a block's weights half as often.  With a folded convolution
+// of 64 channels (80 KB of weights, one workgroup per compute unit) the smaller ones win as long as they are all resident at
+// once.  us per launch, products beside them, 256 / 512 threads: 64 channels, 2000 samples 24 / 33, 8000 25 / 34, 16 000 29 / 36,
+// 18 000 47 / 38, 32 000 58 / 47, 48 000 82 / 81; 32 channels, 2000 13.4 / 16.9, 16 000 15.4 / 18.3, 18 000 to 32 000 the same, 48 000
+// 29 / 37.
+static int block_errors_threads(int R, int N, bool fold) { return fold && R > 32 && N > 64 * 256 ? 512 : 256; }
+
+extern "C++" int cnt::wavenet_block_rows(int R, int N, bool fold) {
+    const int samples = block_errors_threads(R, N, fold) / 4;
+    return (N + samples - 1) / samples;
+}
 
 extern "C++" bool cnt::cnn_foldable(const cnt_cnn *h, int R) {
     // one run of filters, causal, two live taps, R inputs and 2R filters
@@ -1015,7 +1027,8 @@ extern "C++" int cnt::wavenet_block_errors(hipStream_t stream, int R, int K, int
                                            float *total, const FanOut *fan, const float *core_buf, float *ctx_tanh,
                                            const float *conv_tanh_outputs, float *conv_errors, const cnt_cnn *fold,
                                            const float *fold_weights, const float *fold_deltas, float *colsum_partial) {
-    block_err_kernel_t k = pick_block_errors_kernel(R, K, fold != nullptr, core_buf == nullptr);
+    const int threads = block_errors_threads(R, N, fold != nullptr);
+    block_err_kernel_t k = pick_block_errors_kernel(R, K, fold != nullptr, core_buf == nullptr, threads);
     CNT_REQUIRE(k != nullptr, "wavenet_block_errors: no kernel for %d residual and %d skip channels", R, K);
     CNT_REQUIRE(N > 0 && patTypes && skip_weights && out_weights && skip_errors && total && (core_buf || (ctx_tanh && conv_tanh_outputs)) &&
                 conv_errors,
@@ -1044,7 +1057,7 @@ extern "C++" int cnt::wavenet_block_errors(hipStream_t stream, int R, int K, int
                 aligned(a.from_skip) && aligned(core_buf) && aligned(ctx_tanh) && aligned(conv_tanh_outputs) &&
                 aligned(conv_errors), "wavenet_block_errors: buffers must be 16-byte aligned");
     ProfileScope prof(stream, fold ? "wavenet_block_errors+cnn" : "wavenet_block_errors");
-    hipLaunchKernelGGL(k, dim3(wavenet_block_rows(N, fold != nullptr)), dim3(fold ? 512 : 256), 0, stream, a);
+    hipLaunchKernelGGL(k, dim3(wavenet_block_rows(R, N, fold != nullptr)), dim3(threads), 0, stream, a);
     CNT_HIP(hipGetLastError());
     return CNT_OK;
 }

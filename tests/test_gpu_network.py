@@ -411,6 +411,13 @@ def test_wavenet_network_file_against_oracle_graph(nb, cnn_tanh, R, K, Q, C, len
     net.close()
 
 
+# block launches of 64 and of 128 samples per workgroup: a part of one workgroup, one and a sample more, and both sides of the line
+# between them at 64 channels (16 384 samples); 32 channels behind that line
+@pytest.mark.parametrize("R,K,lengths", [(64, 64, [1]), (64, 128, [64]), (32, 64, [65]), (64, 64, [8192, 8101]), (64, 64, [8193, 8050]), (32, 32, [8193, 8192])])
+def test_wavenet_block_errors_of_both_workgroup_sizes(R, K, lengths):
+    test_wavenet_network_file_against_oracle_graph(2, 1, R, K, 16, 4, lengths, 2, 5)
+
+
 # inputs and targets that start on and off a 16-byte boundary, counts that are no multiple of four, with and without a slot order
 # and recurrent layers' clears beside the copies
 @pytest.mark.parametrize("shift", [0, 1, 2])
