@@ -79,8 +79,8 @@ inline long large_tiles(const GemmArgs &a) { return (long)((a.m + 127) / 128) * 
 // as many splits of k as make two workgroups per compute unit (the parts of two row-contiguous operands take 55 KB of LDS, so more
 // do not fit), as long as a split has at least 768 values of k: below that, filling and draining the pipeline and the atomic sums
 // of the tiles outweigh what the large tile saves, and three times as many small workgroups share them better.  64 / 128, us,
-// with the clear and a column sum behind it, which the product brings along by now: 1024 x 1024 over 2000 / 5000 / 8000 / 12 000 slots (250 / 625 / 1000 / 1500 per
-// split) 43 / 58, 88 / 89, 134 / 121, 193 / 162; 1300 x 1300 over 3000 / 4000 (750 / 1000) 98 / 101, 125 / 120; 2048 x 2048 over
+// with the clear and a column sum behind it, which the product brings along by now: 1024 x 1024 over 2000 / 5000 / 8000 /
+// 12 000 slots (250 / 625 / 1000 / 1500 per split) 43 / 58, 88 / 89, 134 / 121, 193 / 162; 1300 x 1300 over 3000 / 4000 (750 / 1000) 98 / 101, 125 / 120; 2048 x 2048 over
 // 1000 / 3000 (500 / 1500) 73 / 79, 187 / 159.  (Below 64 tiles the line is further up, 896 x 896 over 2000 / 6000 / 12 000
 // 41 / 57, 92 / 86, 173 / 136, and layers of 32 tiles gain nothing; they keep the small tile.)  The feed-forward model of five
 // such layers: 2320 -> 2224 us per pass, with 768 workgroups 2230.  The gradients of a

@@ -12,9 +12,10 @@
 // A block of the matrix instruction holds four cells of one gate for the four sequences; lane swaps afterwards transpose
 // the gates into registers (forward) or add the gates' shares (backward) and leave each lane with its own element.
 // Two more waves do all global accesses: one requests a step's inputs kSoloAhead steps ahead and hands them over through LDS,
-// the other stores the step before's results.  They take four neighbouring cells per lane in one access, so that an array takes one access per step instead of one per cell wave: an access occupies the compute
-// unit's address path for sixteen clocks whatever its width, and twelve to fourteen of each of four waves, issued between
-// the LDS reads and the matrix instructions, held those up by 700 clocks a step (64 / 48 / 32 / 16 cells, us per step forward 0.77 /
+// the other stores the step before's results.  They take four neighbouring cells per lane in one access, so that an array
+// takes one access per step instead of one per cell wave: an access occupies the compute unit's address path for sixteen
+// clocks whatever its width, and twelve to fourteen of each of four waves, issued between the LDS reads and the matrix
+// instructions, held those up by 700 clocks a step (64 / 48 / 32 / 16 cells, us per step forward 0.77 /
 // 0.65 / 0.54 / 0.44, backward 0.74 / 0.63 / 0.52 / 0.40; now 0.60 / 0.53 / 0.47 / 0.37 and 0.65 / 0.50 / 0.50 / 0.35).
 // Global accesses are buffer accesses whose range check drops what a lane or a step has no part in: every step issues
 // the same number of loads and stores and no branch, so that the compiler's wait for the loads of a step does not wait for
