@@ -224,7 +224,8 @@ int cnt_lstm_check(cnt_lstm *h, void *stream);
  * > 0 = number of Gaussians (layers/MDNLayer.hpp:35-36).  Other unit types and tied variances are rejected.
  * cnt_mdn_calculate_error adds up the units' errors as the reference does: the mixture and softmax units
  * contribute their summed negative log-likelihood, a sigmoid unit its cross entropy divided by the number
- * of non-padding frames (layers/MDNUnit.cu:3821). */
+ * of non-padding frames (layers/MDNUnit.cu:3821).  The sum over frames is formed in 64 bits in an accumulator of the
+ * handle: the same bits in every call, and calls on one handle belong on one stream (or in order). */
 typedef struct cnt_mdn cnt_mdn;
 
 typedef struct {

@@ -44,6 +44,51 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+__device__ __forceinline__ double wave_sum(double v) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+}
+
+// Sum of the errors of a call, over the workgroups of all its units' launches.  It is formed in 64 bits: workgroups add in the
+// order they finish in, and in 32 bits the last digits follow that order (the error of 31 000 frames, 2.2e5, came out
+// up to 0.27 apart between two passes over the same probabilities).  The values added have 24 digits each, so their 64-bit sum
+// is exact, or as good as, in any order.
+// The workgroup that finishes last hands the sum to the caller and leaves accumulator and ticket counter at zero for the next
+// call, so that no launch has to clear the caller's result first.
+struct LossSum {
+    double *acc;
+    unsigned *ticket;     // workgroups that have added so far
+    unsigned workgroups;  // of the call
+    float *result;
+};
+
+// by one thread of a workgroup, once
+__device__ __forceinline__ void add_loss(const LossSum &s, double v) {
+    // No fence (a device-scope fence writes the L2 back, which costs more than the kernel): the ticket is taken
+    // only after the add has returned its old value, i.e. has been performed where every XCD's atomics meet.
+    const double before = __hip_atomic_fetch_add(s.acc, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned one = 1u;
+    asm volatile("" : "+v"(one) : "v"(before));  // the ticket's operand depends on the returned value
+    if (__hip_atomic_fetch_add(s.ticket, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == s.workgroups - 1u) {
+        *s.result = (float)__hip_atomic_exchange(s.acc, 0.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(s.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// every wave's value to the call's sum; all threads of the workgroup take part
+template <int WAVES>
+__device__ __forceinline__ void add_block_loss(const LossSum &s, double wave_total) {
+    __shared__ double block_sum[WAVES];
+    if ((threadIdx.x & 63) == 0) block_sum[threadIdx.x >> 6] = wave_total;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double v = 0.0;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) v += block_sum[w];
+        add_loss(s, v);
+    }
+}
+
 // offset = (min + max) / 2 with the reference's start values, exp((x - offset)/T), normalise.
 // `in` points at the K inputs of the frame, `out` at its K outputs.
 __device__ __forceinline__ void softmax_frame(const float *__restrict__ in, float *__restrict__ out, int K,
@@ -91,15 +136,15 @@ __global__ void sigmoid_forward_kernel(UnitGeom g, const char *__restrict__ pat,
 // sums[0] += binary cross entropy of the valid frames, sums[1] += number of valid frames
 __global__ void sigmoid_error_kernel(UnitGeom g, int continuous, const char *__restrict__ pat,
                                      const float *__restrict__ target, const float *__restrict__ prob,
-                                     float *__restrict__ sums) {
+                                     double *__restrict__ sums) {
     const size_t n = (size_t)g.F * g.M;
-    float v = 0.0f, cnt = 0.0f;
+    double v = 0.0, cnt = 0.0;
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     for (; i < n; i += (size_t)gridDim.x * blockDim.x) {
         const size_t f = i / g.M;
         const int k = (int)(i % g.M);
         if (pat[f] == 0) continue;
-        if (k == 0) cnt += 1.0f;
+        if (k == 0) cnt += 1.0;
         const float p = prob[i], pr = (float)(1.0 - p);
         const float d = target[f * g.Lt + g.startDOut + k];
         if (continuous) {
@@ -113,14 +158,14 @@ __global__ void sigmoid_error_kernel(UnitGeom g, int continuous, const char *__r
     v = wave_sum(v);
     cnt = wave_sum(cnt);
     if ((threadIdx.x & 63) == 0) {
-        if (v != 0.0f) atomicAdd(sums, v);
-        if (cnt != 0.0f) atomicAdd(sums + 1, cnt);
+        if (v != 0.0) atomicAdd(sums, v);
+        if (cnt != 0.0) atomicAdd(sums + 1, cnt);
     }
 }
 
 // the unit's error is the summed cross entropy divided by the number of valid frames (MDNUnit.cu:3821)
-__global__ void sigmoid_error_finish_kernel(const float *__restrict__ sums, float *__restrict__ result) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *result += sums[0] / sums[1];
+__global__ void sigmoid_error_finish_kernel(const double *__restrict__ sums, LossSum loss) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) add_loss(loss, sums[0] / sums[1]);
 }
 
 __global__ void sigmoid_backward_kernel(UnitGeom g, int continuous, const char *__restrict__ pat,
@@ -213,8 +258,10 @@ __global__ __launch_bounds__(64 * kFramesPerBlock) void softmax_forward_vec4_ker
     }
 }
 
-__global__ void softmax_error_kernel(UnitGeom g, const char *__restrict__ pat, const float *__restrict__ target,
-                                     const float *__restrict__ prob, float *__restrict__ result) {
+constexpr int kSoftmaxErrWaves = 4;
+__global__ __launch_bounds__(64 * kSoftmaxErrWaves) void softmax_error_kernel(UnitGeom g, const char *__restrict__ pat,
+                                                                              const float *__restrict__ target,
+                                                                              const float *__restrict__ prob, LossSum loss) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     float v = 0.0f;
     if (f < g.F && pat[f] != 0) {
@@ -224,8 +271,7 @@ __global__ void softmax_error_kernel(UnitGeom g, const char *__restrict__ pat, c
         if (idx < g.capacity && idx >= 0) p = fmaxf(lim::kMin, prob[idx]);
         v = -logf(p);
     }
-    v = wave_sum(v);
-    if ((threadIdx.x & 63) == 0 && v != 0.0f) atomicAdd(result, v);
+    add_block_loss<kSoftmaxErrWaves>(loss, wave_sum((double)v));
 }
 
 __global__ void softmax_backward_kernel(UnitGeom g, const char *__restrict__ pat, const float *__restrict__ target,
@@ -296,41 +342,41 @@ __global__ void mixture_forward_kernel(UnitGeom g, const char *__restrict__ pat,
     }
 }
 
-// tmp = [F*M per-mixture log-likelihoods | F log-sums]; result accumulates -sum of log-sums
-__global__ void mixture_error_kernel(UnitGeom g, const char *__restrict__ pat, const float *__restrict__ target,
-                                     const float *__restrict__ para, float *__restrict__ tmp,
-                                     float *__restrict__ result) {
+// tmp = [F*M per-mixture log-likelihoods | F log-sums]; the call's sum takes the negative log-sums
+__global__ __launch_bounds__(64 * kFramesPerBlock) void mixture_error_kernel(UnitGeom g, const char *__restrict__ pat,
+                                                                             const float *__restrict__ target,
+                                                                             const float *__restrict__ para,
+                                                                             float *__restrict__ tmp, LossSum loss) {
     const int lane = threadIdx.x & 63;
     const int f = blockIdx.x * kFramesPerBlock + (threadIdx.x >> 6);
-    if (f >= g.F) return;
     const int M = g.M, D = g.D;
-    if (pat[f] == 0) {
+    double wave_total = 0.0;
+    if (f < g.F && pat[f] == 0) {
         for (int m = lane; m < M; m += 64) tmp[(size_t)f * M + m] = 0.0f;  // distance pass writes 0, the rest skips
-        return;
-    }
-    const float *t = target + (size_t)f * g.Lt + g.startDOut;
-    const float *mean = para + (size_t)g.F * M + (size_t)f * M * D;
-    const float *sd = para + (size_t)g.F * M * (1 + D) + (size_t)f * M * D;
-    const float gauss_const = (float)(D * log(2 * 3.141215) / 2.0);  // the reference's own value of pi
-    float lsum = lim::kLogZero;
-    for (int m = 0; m < M; ++m) {
-        float dist = 0.0f, logsd = 0.0f;
-        for (int d = lane; d < D; d += 64) {
-            const float s = sd[m * D + d], diff = t[d] - mean[m * D + d];
-            dist += diff * diff / (s * s) * 0.5f;
-            logsd += safe_log(s);
+    } else if (f < g.F) {
+        const float *t = target + (size_t)f * g.Lt + g.startDOut;
+        const float *mean = para + (size_t)g.F * M + (size_t)f * M * D;
+        const float *sd = para + (size_t)g.F * M * (1 + D) + (size_t)f * M * D;
+        const float gauss_const = (float)(D * log(2 * 3.141215) / 2.0);  // the reference's own value of pi
+        float lsum = lim::kLogZero;
+        for (int m = 0; m < M; ++m) {
+            float dist = 0.0f, logsd = 0.0f;
+            for (int d = lane; d < D; d += 64) {
+                const float s = sd[m * D + d], diff = t[d] - mean[m * D + d];
+                dist += diff * diff / (s * s) * 0.5f;
+                logsd += safe_log(s);
+            }
+            dist = wave_sum(dist);
+            logsd = wave_sum(logsd);
+            float lp = logf(para[(size_t)f * M + m]) - dist - gauss_const - logsd;
+            if (lp < lim::kLSmall) lp = lim::kLSmall;
+            lsum = log_add(lsum, lp);
+            if (lane == 0) tmp[(size_t)f * M + m] = lp;
         }
-        dist = wave_sum(dist);
-        logsd = wave_sum(logsd);
-        float lp = logf(para[(size_t)f * M + m]) - dist - gauss_const - logsd;
-        if (lp < lim::kLSmall) lp = lim::kLSmall;
-        lsum = log_add(lsum, lp);
-        if (lane == 0) tmp[(size_t)f * M + m] = lp;
+        if (lane == 0) tmp[(size_t)g.F * M + f] = lsum;
+        wave_total = -(double)lsum;
     }
-    if (lane == 0) {
-        tmp[(size_t)g.F * M + f] = lsum;
-        atomicAdd(result, -lsum);
-    }
+    add_block_loss<kFramesPerBlock>(loss, wave_total);
 }
 
 // The same error pass for units whose data can be moved 16 bytes at a time (the condition of the VEC4 backward
@@ -340,21 +386,20 @@ __global__ void mixture_error_kernel(UnitGeom g, const char *__restrict__ pat, c
 // The log-sum over the components is max + log(sum exp(. - max)) over the wave (the reference's running log_add in
 // another order: terms below e^-69 of the largest drop out either way).  A wave takes one frame (a frame is one chain
 // of loads, reductions and transcendentals; two frames in turn per wave are 1-2 % slower), and the eight
-// waves of a workgroup add their frames' log-sums in LDS, so the single result word receives one atomic per 8
+// waves of a workgroup add their frames' log-sums in LDS, so the call's sum receives one atomic per 8
 // frames -- 6000 atomics on one address, which serialise, were what the first kernel's time went to.
 constexpr int kErrFramesPerWave = 1;
 constexpr int kErrWaves = 8;
 __global__ __launch_bounds__(64 * kErrWaves) void mixture_error_vec_kernel(UnitGeom g, const char *__restrict__ pat,
                                                                 const float *__restrict__ target,
                                                                 const float *__restrict__ para, float *__restrict__ tmp,
-                                                                float *__restrict__ result) {
+                                                                LossSum loss) {
     __shared__ float lp_sh[kErrWaves][64];
-    __shared__ float block_sum[kErrWaves];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int M = g.M, D = g.D, MD = M * D, DV = D / 4;
     const int p = lane & 3, ml = lane >> 2;  // lane (ml, p): component ml of the pass, quarter p
     const float gauss_const = (float)(D * log(2 * 3.141215) / 2.0);  // the reference's own value of pi
-    float wave_total = 0.0f;
+    double wave_total = 0.0;
     for (int i = 0; i < kErrFramesPerWave; ++i) {
         const int f = (blockIdx.x * kErrWaves + wave) * kErrFramesPerWave + i;
         if (f >= g.F) break;
@@ -418,14 +463,7 @@ __global__ __launch_bounds__(64 * kErrWaves) void mixture_error_vec_kernel(UnitG
             wave_total -= lsum;
         }
     }
-    if (lane == 0) block_sum[wave] = wave_total;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float v = 0.0f;
-#pragma unroll
-        for (int w = 0; w < kErrWaves; w += 2) v += block_sum[w] + block_sum[w + 1];
-        if (v != 0.0f) atomicAdd(result, v);
-    }
+    add_block_loss<kErrWaves>(loss, wave_total);
 }
 
 // VEC4: the mean / std part moves 16 bytes per lane (D, M, Lp, Lt and both start columns multiples of four and all
@@ -509,18 +547,13 @@ __global__ __launch_bounds__(64 * kFusedWaves) void mixture_error_backward_kerne
                                                                                  const float *__restrict__ target,
                                                                                  const float *__restrict__ para,
                                                                                  float *__restrict__ tmp,
-                                                                                 float *__restrict__ result,
-                                                                                 float *__restrict__ errors,
-                                                                                 float *__restrict__ loss_acc,
-                                                                                 unsigned *__restrict__ loss_ticket,
-                                                                                 unsigned total_workgroups) {
-    __shared__ float block_sum[kFusedWaves];
+                                                                                 float *__restrict__ errors, LossSum loss) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int M = g.M, D = g.D, MD = M * D, DV = D / 4, Lp = g.Lp;
     const int p = lane & 3, m = lane >> 2;
     const int unit_cols = M + 2 * MD;
     const int f = blockIdx.x * kFusedWaves + wave;
-    float wave_total = 0.0f;
+    double wave_total = 0.0;
     if (f < g.F) {
         float *e = errors + (size_t)f * Lp + g.startD;
         if (pat[f] == 0) {
@@ -597,25 +630,7 @@ __global__ __launch_bounds__(64 * kFusedWaves) void mixture_error_backward_kerne
             }
         }
     }
-    if (lane == 0) block_sum[wave] = wave_total;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float v = 0.0f;
-#pragma unroll
-        for (int w = 0; w < kFusedWaves; w += 2) v += block_sum[w] + block_sum[w + 1];
-        // The workgroups of a call (of all its units' launches) add into an accumulator of the handle; the one that
-        // finishes last hands the sum to the caller and leaves accumulator and ticket counter at zero for the next
-        // call, so that no launch has to clear the caller's result first.
-        // No fence (a device-scope fence writes the L2 back, which costs more than the kernel): the ticket is taken
-        // only after the add has returned its old value, i.e. has been performed where every XCD's atomics meet.
-        const float before = __hip_atomic_fetch_add(loss_acc, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        unsigned one = 1u;
-        asm volatile("" : "+v"(one) : "v"(before));  // the ticket's operand depends on the returned value
-        if (__hip_atomic_fetch_add(loss_ticket, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total_workgroups - 1u) {
-            *result = __hip_atomic_exchange(loss_acc, 0.0f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(loss_ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
+    add_block_loss<kFusedWaves>(loss, wave_total);
 }
 
 }  // namespace
@@ -639,7 +654,7 @@ struct cnt_mdn {
     const char *pat;
     int T;
     bool covers_all_columns;
-    float *loss_acc;         // cnt_mdn_error_backward: the call's running sum (device), zero between calls
+    double *loss_acc;        // running sum of a call's errors (device), zero between calls
     unsigned *loss_ticket;   // and the count of workgroups that have added to it
 };
 
@@ -686,7 +701,7 @@ int cnt_mdn_create(const cnt_mdn_desc *desc, const float *config, int config_len
         } else if (ok && u.type == 0) {
             u.M = cols; u.D = 1;
             u.para_capacity = maxF * u.M;
-            u.tmp_capacity = 2;  // cross-entropy sum and frame count
+            u.tmp_capacity = 4;  // cross-entropy sum and frame count, 64 bits each
             ok = (dims == cols);
         } else if (ok && u.type > 0) {
             u.M = u.type; u.D = dims;
@@ -807,39 +822,51 @@ int cnt_mdn_forward(cnt_mdn *h, void *stream_, const float *nn_outputs) {
     return CNT_OK;
 }
 
+// the mixture units whose error kernel moves 16 bytes at a time, and workgroups of a unit's error launch
+static bool mixture_error_vec(const cnt::UnitGeom &g, const cnt_mdn_unit &u, const float *targets) {
+    auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    return g.D % 4 == 0 && g.M % 4 == 0 && g.M <= 64 && g.Lt % 4 == 0 && g.startDOut % 4 == 0 && aligned(targets) &&
+           aligned(u.para);
+}
+static unsigned error_workgroups(const cnt::UnitGeom &g, const cnt_mdn_unit &u, const float *targets) {
+    using namespace cnt;
+    if (u.type == 0) return 1;  // the launch that forms the unit's mean
+    const int frames = u.type == -1                       ? 64 * kSoftmaxErrWaves
+                       : mixture_error_vec(g, u, targets) ? kErrWaves * kErrFramesPerWave
+                                                          : kFramesPerBlock;
+    return (unsigned)((g.F + frames - 1) / frames);
+}
+
 int cnt_mdn_calculate_error(cnt_mdn *h, void *stream_, const float *targets, float *result_dev) {
     using namespace cnt;
     CNT_REQUIRE(h && targets && result_dev, "mdn_calculate_error: null argument");
     CNT_REQUIRE(h->T > 0, "mdn_calculate_error: load_sequences has not been called");
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    CNT_TRY(fill_zero(stream, result_dev, 1));
+    if (h->units.empty()) return fill_zero(stream, result_dev, 1);
+    LossSum loss = {h->loss_acc, h->loss_ticket, 0, result_dev};
+    for (auto &u : h->units) loss.workgroups += error_workgroups(unit_geom(h, u), u, targets);
     for (auto &u : h->units) {
         const UnitGeom g = unit_geom(h, u);
+        const dim3 grid(error_workgroups(g, u, targets));
         if (u.type == 0) {
             ProfileScope prof(stream, "mdn_sigmoid_error");
             const size_t n = (size_t)g.F * g.M;
-            CNT_TRY(fill_zero(stream, u.tmp, 2));
+            CNT_TRY(fill_zero(stream, u.tmp, 4));
+            double *sums = reinterpret_cast<double *>(u.tmp);
             hipLaunchKernelGGL(sigmoid_error_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 1024)), dim3(256), 0,
-                               stream, g, h->desc.sigmoid_continuous, h->pat, targets, u.para, u.tmp);
-            hipLaunchKernelGGL(sigmoid_error_finish_kernel, dim3(1), dim3(64), 0, stream, u.tmp, result_dev);
+                               stream, g, h->desc.sigmoid_continuous, h->pat, targets, u.para, sums);
+            hipLaunchKernelGGL(sigmoid_error_finish_kernel, grid, dim3(64), 0, stream, sums, loss);
         } else if (u.type == -1) {
             ProfileScope prof(stream, "mdn_softmax_error");
-            hipLaunchKernelGGL(softmax_error_kernel, dim3((g.F + 255) / 256), dim3(256), 0, stream, g, h->pat, targets,
-                               u.para, result_dev);
+            hipLaunchKernelGGL(softmax_error_kernel, grid, dim3(64 * kSoftmaxErrWaves), 0, stream, g, h->pat, targets, u.para, loss);
         } else {
             ProfileScope prof(stream, "mdn_mixture_error");
-            auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-            const bool vec4 = g.D % 4 == 0 && g.M % 4 == 0 && g.M <= 64 && g.Lt % 4 == 0 && g.startDOut % 4 == 0 &&
-                              aligned(targets) && aligned(u.para);
-            if (vec4) {
-                const int per_block = kErrWaves * kErrFramesPerWave;
-                hipLaunchKernelGGL(mixture_error_vec_kernel, dim3((g.F + per_block - 1) / per_block), dim3(64 * kErrWaves), 0, stream, g,
-                                   h->pat, targets, u.para, u.tmp, result_dev);
-            } else {
-                const dim3 grid((g.F + kFramesPerBlock - 1) / kFramesPerBlock), block(64 * kFramesPerBlock);
-                hipLaunchKernelGGL(mixture_error_kernel, grid, block, 0, stream, g, h->pat, targets, u.para, u.tmp,
-                                   result_dev);
-            }
+            if (mixture_error_vec(g, u, targets))
+                hipLaunchKernelGGL(mixture_error_vec_kernel, grid, dim3(64 * kErrWaves), 0, stream, g, h->pat, targets, u.para,
+                                   u.tmp, loss);
+            else
+                hipLaunchKernelGGL(mixture_error_kernel, grid, dim3(64 * kFramesPerBlock), 0, stream, g, h->pat, targets, u.para,
+                                   u.tmp, loss);
         }
         CNT_HIP(hipGetLastError());
     }
@@ -872,13 +899,13 @@ int cnt_mdn_error_backward(cnt_mdn *h, void *stream_, const float *targets, floa
     const size_t cap = (size_t)h->desc.maxT * h->desc.S * h->desc.Lp;
     if (!h->covers_all_columns) CNT_TRY(fill_zero(stream, prev_errors, used));
     if (cap > used) CNT_TRY(fill_zero(stream, prev_errors + used, cap - used));
-    unsigned total = 0;
-    for (auto &u : h->units) total += (unsigned)((unit_geom(h, u).F + kFusedWaves - 1) / kFusedWaves);
+    LossSum loss = {h->loss_acc, h->loss_ticket, 0, result_dev};
+    for (auto &u : h->units) loss.workgroups += (unsigned)((unit_geom(h, u).F + kFusedWaves - 1) / kFusedWaves);
     for (auto &u : h->units) {
         const UnitGeom g = unit_geom(h, u);
         ProfileScope prof(stream, "mdn_mixture_error_backward");
         hipLaunchKernelGGL(mixture_error_backward_kernel, dim3((g.F + kFusedWaves - 1) / kFusedWaves), dim3(64 * kFusedWaves), 0,
-                           stream, g, h->pat, targets, u.para, u.tmp, result_dev, prev_errors, h->loss_acc, h->loss_ticket, total);
+                           stream, g, h->pat, targets, u.para, u.tmp, prev_errors, loss);
         CNT_HIP(hipGetLastError());
     }
     return CNT_OK;

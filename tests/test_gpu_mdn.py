@@ -1,6 +1,7 @@
 """GPU parity (through the C ABI) of the mixture-density layer: flat softmax unit and untied-variance
 mixture unit, forward parameters, negative log-likelihood and gradients; 1e-4 L2-normalised per tensor,
 zero patterns (padding frames, the reference's index collision) exact."""
+import numpy as np
 import pytest
 
 import parity_cases as PC
@@ -64,3 +65,58 @@ def test_unsupported_units_are_rejected():
 def test_sigmoid_unit(lengths, K, extra, continuous, with_softmax):
     print("mdn sigmoid case", lengths, K, extra, continuous, with_softmax, flush=True)
     assert PC.run_sigmoid_case(lengths, K, extra, continuous, seed=K + extra, with_softmax=with_softmax) < TOL
+
+
+@pytest.mark.parametrize("kind,lengths", [("softmax", [1]), ("softmax", [16000, 15000]), ("mixture", [16000, 15000]),
+                                          ("mixture_odd", [1500, 1200, 40]), ("sigmoid", [9000, 8000]), ("both", [600, 411])])
+def test_error_is_the_sum_over_frames_whatever_their_order(kind, lengths):
+    """The error of a call against the 64-bit sum of what the frames contribute, formed from the unit's own buffers, and the
+    same bits in every call.  Bounds: a mixture frame's log-sum is stored, so only the result is rounded (2^-24); -log of a
+    probability is good to 2 units in its last place (2^-22 of the sum, whose terms have one sign), plus that rounding."""
+    import torch
+
+    print("mdn error sums", kind, lengths, flush=True)
+    capi = PC.pkg().capi
+    S, T = len(lengths), max(lengths)
+    N = S * T
+    pat = PC.make_pat_types(lengths, T)
+    valid = pat != 0
+    rng = np.random.default_rng(N)
+    K, M, D = 60, {"mixture": 4, "mixture_odd": 3}.get(kind, 0), 8
+    config, Lp, Lt = {"softmax": ([1, 0, K, 0, 1, -1], K, 1), "sigmoid": ([1, 0, K, 0, K, 0], K, K),
+                      "both": ([2, 0, K, 0, 1, -1, K, K + 5, 1, 6, 0], K + 5, 6)}.get(
+                          kind, ([1, 0, M * (1 + 2 * D), 0, D, M], M * (1 + 2 * D), D))
+    x = rng.standard_normal((N, Lp)).astype(np.float32)
+    tgt = rng.standard_normal((N, Lt)).astype(np.float32)
+    if kind in ("softmax", "both"):
+        tgt[:, 0] = rng.integers(0, K, size=N)
+    layer = capi.Mdn(Lp, Lt, S, T, config)
+    pd, xd, td = PC.dev(pat), PC.dev(x.reshape(-1)), PC.dev(tgt.reshape(-1))
+    layer.load_sequences(pd, T)
+    layer.forward(xd)
+    results = torch.zeros(12, device="cuda")
+    errors = torch.zeros(N * Lp, device="cuda")
+    for i in range(12):
+        if i % 4 == 3:
+            layer.error_backward(td, results[i:i + 1], errors)
+        else:
+            layer.calculate_error(td, results[i:i + 1])
+    torch.cuda.synchronize()
+    got = results.cpu().numpy()
+    want, bound = 0.0, 0.0
+    if kind in ("softmax", "both"):
+        p = layer.unit_buffer(0, 0).cpu().numpy().reshape(N, K)[np.arange(N), tgt[:, 0].astype(np.int64)].astype(np.float64)
+        want += -np.log(p[valid]).sum()
+        bound += want * 2.0 ** -22
+    if kind in ("sigmoid", "both"):
+        k = Lt - (kind == "both")
+        p = layer.unit_buffer(int(kind == "both"), 0).cpu().numpy().reshape(N, k)
+        b = np.where(tgt[:, Lt - k:] > 0, p, np.float32(1) - p).astype(np.float64)
+        mean = -np.log(b[valid]).sum() / valid.sum()
+        want += mean
+        bound += mean * 2.0 ** -22
+    if M:
+        want = -layer.unit_buffer(0, 1).cpu().numpy()[N * M:][valid].astype(np.float64).sum()
+    layer.close()
+    assert len(set(got.tobytes()[4 * i:4 * i + 4] for i in range(12))) == 1, got
+    assert abs(float(got[0]) - want) <= bound + abs(want) * 2.0 ** -24

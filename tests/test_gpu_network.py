@@ -812,7 +812,10 @@ def test_full_size_wavenet_sequencer_matches_layer_by_layer_walk():
     """benchmark configs[3] at its real size (30 blocks, 2 x 16000 samples, 1024 classes): the sequencer (shared sums,
     aliased buffers, fan-in / fan-out tables, side streams, fused delta) against the plain layer-by-layer walk over
     the same kernels, which the shortened-stack tests tie to the oracle.  Loss equal to 1e-6, every weight gradient
-    to the tolerance of the split-K atomics' summation order."""
+    to the tolerance of the split-K atomics' summation order.  What each frame contributes is compared by itself (the last
+    product adds 128 terms below one: 128 * 2^-24 per logit, twice that in the log-probability), and each pass's loss with the
+    64-bit sum of its own frames (2^-20 per frame for exponential, sum and quotient of a probability at exponents of a few
+    units, 2^-22 of the value for its logarithm), so that a frame computed wrongly is not taken for rounding."""
     import torch
 
     print("full-size wavenet sequencer vs walk", flush=True)
@@ -842,6 +845,16 @@ def test_full_size_wavenet_sequencer_matches_layer_by_layer_walk():
     net.backward()
     torch.cuda.synchronize()
     ref_loss = float(walk.loss.item())
+
+    def by_frame(logits):
+        v = torch.log_softmax(logits[: N * Q].view(N, Q).double(), 1)
+        return -v[torch.arange(N, device="cuda"), tgt_d.long()][pat_d != 0]
+
+    frames, ref_frames = by_frame(net.layer("output")["outputs"]), by_frame(walk.buf["output"]["out"])
+    assert float((frames - ref_frames).abs().max()) <= 2 * 128 * 2.0 ** -24
+    for total, each in ((loss, frames), (ref_loss, ref_frames)):
+        exact = float(each.sum())
+        assert abs(total - exact) <= len(each) * 2.0 ** -20 + exact * 2.0 ** -22
     assert abs(loss - ref_loss) <= 1e-6 * abs(ref_loss)
     for L in net.layers:
         if L["weight_count"]:
