@@ -469,8 +469,11 @@ int cnt_network_calculate_error(cnt_network *net, void *stream, float *loss_dev)
 /* NeuralNetwork::computeBackwardPass (NeuralNetwork.cpp:2744-2800, :2864-2895): layers in reverse order.  The
  * layers' weight gradients run on streams of the network's own (same priority as any other stream), ordered after
  * the error computations they depend on; small layers of one shape share a launch.  On return the caller's stream
- * has been made to wait for those streams, so weight updates are complete in stream order.  One call per forward
- * pass: the gradient of a wavnetc layer's conditioning part takes the place of its values. */
+ * has been made to wait for those streams, so weight updates are complete in stream order.  A second call
+ * after one forward pass gives the same gradients again, with two exceptions, as in the reference: where layers are linked by
+ * skip connections whose errors are summed in buffers that the forward pass clears, these sums go on, and a wavnetc layer whose
+ * convolution has no tanh output, or whose sizes have no kernel for a whole block, has by then replaced the values of its
+ * conditioning part with their gradient (see cnt_wavnetc_backward). */
 int cnt_network_backward(cnt_network *net, void *stream);
 /* cnt_lstm_check for every LSTM layer (all of them are looked at; the first failure is returned).  Failure contract
  * of the network: a pass in which a recursion gave up cannot reach the weights -- the failed launch sets a device

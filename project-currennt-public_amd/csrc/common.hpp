@@ -299,11 +299,12 @@ int wavenet_block_forward(hipStream_t stream, const cnt_cnn *cnn, int R, int K, 
 // layer behind the gated unit, the gated unit): see wavenet_block_errors_kernel.
 bool wavenet_block_errors_supported(int R, int K);
 // `fold` (optional): the convolution layer above the block, whose error product (two live taps) is added to the
-// block's summed errors inside the same launch instead of being written to the closing skip layer first
+// block's summed errors inside the same launch instead of being written to the closing skip layer first.
+// ctx_grad receives the gradient of the conditioning part: ctx_tanh itself (if core_buf is given) or a buffer of its own
 bool cnn_foldable(const cnt_cnn *h, int R);
 int wavenet_block_errors(hipStream_t stream, int R, int K, int N, const char *patTypes, const float *skip_weights,
                          const float *out_weights, const float *skip_errors, float *total, const FanOut *fan,
-                         const float *core_buf, float *ctx_tanh, const float *conv_tanh_outputs, float *conv_errors,
+                         const float *core_buf, const float *ctx_tanh, float *ctx_grad, const float *conv_tanh_outputs, float *conv_errors,
                          const cnt_cnn *fold, const float *fold_weights, const float *fold_deltas, float *colsum_partial);
 // workgroups of that launch = rows of `colsum_partial` ([rows][2R]: per-workgroup sums of conv_errors over the samples)
 int wavenet_block_rows(int R, int N, bool fold);

@@ -203,7 +203,9 @@ struct NetLayer {
     float *dft_errors = nullptr;             // dft: per-resolution distances written by the forward pass
     int dft_error_count = 0;
     float dft_beta = 0.0f;                   // dft: weight of the waveform MSE gradient
-    float *core = nullptr, *cth = nullptr;  // wavnetc
+    // wavnetc: pre-activations, tanh of the conditioning part, and where the backward pass has left that part's gradient: in the
+    // place of its values, or of the pre-activations if these are not kept (block_sums_core)
+    float *core = nullptr, *cth = nullptr, *cgrad = nullptr;
     int ctx_dim = 0;
     int fb_start = 0, fb_end = 0;            // feedback: dimensions taken from the preceding layer
     // time base: a layer with "resolution" r has one slot per r time steps (layers/Layer.cu:254-305)
@@ -1641,7 +1643,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         }
         if (L.kind == K_LSTM) return cnt_lstm_backward_weights(L.lstm, ws, prev.out, dW);
         if (L.kind == K_CNN) return cnt_cnn_backward_weights(L.cnn, ws, L.pat, L.T, prev.out, L.err, dW);
-        return cnt_wavnetc_backward_weights(ws, L.size, L.ctx_dim, L.N, net->ctx, L.cth, dW);
+        return cnt_wavnetc_backward_weights(ws, L.size, L.ctx_dim, L.N, net->ctx, L.cgrad, dW);
     };
     // Large layers' weight halves go round-robin over all side streams, the collected small ones over the first two:
     // measured on MI355X, a third stream gains 1% on the acoustic model (its last recurrent layer's and the dense
@@ -1713,7 +1715,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
             NetLayer &prev = net->layers[g.layers[(size_t)z] - 1];
             dW[z] = net->updates + L.w_off;
             bias[z] = L.bias;
-            in0[z] = g.kind == K_WAVNETC ? L.cth : prev.out;
+            in0[z] = g.kind == K_WAVNETC ? L.cgrad : prev.out;
             in1[z] = L.err;
             cnn[z] = L.cnn;
             colsum[z] = L.colsum; colsum_rows[z] = L.colsum_rows;
@@ -1818,7 +1820,10 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                         fan_done[i - 1] = 1;
                         goto weight_half_of_layer;
                     } else if (block_at(i)) {
-                        const NetLayer &out = net->layers[i - 3], &wav = net->layers[i - 4], &cnn = net->layers[i - 5];
+                        const NetLayer &out = net->layers[i - 3], &cnn = net->layers[i - 5];
+                        NetLayer &wav = net->layers[i - 4];
+                        const bool sums_core = block_sums_core(cnn, wav);
+                        wav.cgrad = sums_core ? wav.core : wav.cth;
                         const NetLayer *fold = fold_from[i] >= 0 ? &net->layers[(size_t)fold_from[i]] : nullptr;
                         FanOut block_fan = fan;
                         // with a folded convolution, what the later block handed to the closing skipadd layer comes in
@@ -1837,8 +1842,8 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                         if (block_fan.n > 0) adds_to_side(prev);
                         CNT_TRY(wavenet_block_errors(stream, prev.size, L.size, N, L.pat, W, net->weights + out.w_off, L.err,
                                                      prev_err, fan_live ? &block_fan : nullptr,
-                                                     block_sums_core(cnn, wav) ? nullptr : wav.core,
-                                                     wav.ctx_dim > 0 ? wav.cth : nullptr, cnn.delta_fused ? cnn.out : nullptr,
+                                                     sums_core ? nullptr : wav.core, wav.ctx_dim > 0 ? wav.cth : nullptr,
+                                                     wav.ctx_dim > 0 ? wav.cgrad : nullptr, cnn.delta_fused ? cnn.out : nullptr,
                                                      cnn.err, fold ? fold->cnn : nullptr,
                                                      fold ? net->weights + fold->w_off : nullptr, fold ? fold->err : nullptr,
                                                      cnn.colsum));
@@ -1900,8 +1905,9 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                 } else {
                     if (errors_done[i]) {
                         if (L.ctx_dim > 0 && net->flagged >= 0)
-                            CNT_TRY(wavnetc_context_grad(stream, L.size, L.ctx_dim, N, W, L.cth, net->ctx_grad));
+                            CNT_TRY(wavnetc_context_grad(stream, L.size, L.ctx_dim, N, W, L.cgrad, net->ctx_grad));
                     } else {
+                        L.cgrad = L.cth;
                         CNT_TRY(cnt_wavnetc_backward_errors(stream, L.size, L.ctx_dim, N, L.pat, W, L.core, L.cth, L.err,
                                                             prev.err, net->flagged >= 0 ? net->ctx_grad : nullptr,
                                                             prev.delta_fused ? prev.out : nullptr));

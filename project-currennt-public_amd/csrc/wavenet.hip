@@ -194,7 +194,8 @@ struct BlockErrArgs {
     const int *fan_is_skip;
     const float *pre;        // 2R x N: pre-activations of the gated unit (null: the sum of conv_tanh and ctx_tanh)
     const float *conv_tanh;  // 2R x N or null: outputs of a convolution layer with tanh output
-    float *ctx_tanh;         // 2R x N or null: tanh of the conditioning part, overwritten with its gradient
+    const float *ctx_tanh;   // 2R x N or null: tanh of the conditioning part
+    float *ctx_grad;         // 2R x N: the gradient of that part (may be ctx_tanh)
     float *deltas;           // 2R x N: errors (or deltas) of the convolution layer
     // folded convolution (two live taps, R inputs, 2R filters) whose errors go to the block's closing skip layer:
     const float *conv_w[2];      // weight of (filter 0, tap q); filter d at + d*conv_ld, input channel p at + p
@@ -207,7 +208,8 @@ struct BlockErrArgs {
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
 // SUM: the gate's pre-activations are formed again from the convolution's outputs and the conditioning part, which the
-// launch reads anyway; `pre` is not read then.
+// launch reads anyway; `pre` is not read then.  Both have to be there for a second backward pass as well, so the gradient of the
+// conditioning part goes to another place than its values.
 template <int R, int K, bool CONV, bool SUM, int NT>
 __global__ __launch_bounds__(NT, (CONV || K > 128) ? 1 : 2) void wavenet_block_errors_kernel(const BlockErrArgs a) {
     static_assert(R % 16 == 0 && K % 16 == 0 && R <= 128, "block geometry");
@@ -447,8 +449,8 @@ __global__ __launch_bounds__(NT, (CONV || K > 128) ? 1 : 2) void wavenet_block_e
             const float4 q1 = {tanh_deriv(v1.x) * g1[0], tanh_deriv(v1.y) * g1[1], tanh_deriv(v1.z) * g1[2], tanh_deriv(v1.w) * g1[3]};
             const float4 q2 = {tanh_deriv(v2.x) * g2[0], tanh_deriv(v2.y) * g2[1], tanh_deriv(v2.z) * g2[2], tanh_deriv(v2.w) * g2[3]};
             if (ok) {
-                *reinterpret_cast<float4 *>(a.ctx_tanh + at) = q1;
-                *reinterpret_cast<float4 *>(a.ctx_tanh + at + R) = q2;
+                *reinterpret_cast<float4 *>(a.ctx_grad + at) = q1;
+                *reinterpret_cast<float4 *>(a.ctx_grad + at + R) = q2;
             }
         }
     }
@@ -1024,20 +1026,20 @@ extern "C++" bool cnt::cnn_foldable(const cnt_cnn *h, int R) {
 
 extern "C++" int cnt::wavenet_block_errors(hipStream_t stream, int R, int K, int N, const char *patTypes,
                                            const float *skip_weights, const float *out_weights, const float *skip_errors,
-                                           float *total, const FanOut *fan, const float *core_buf, float *ctx_tanh,
-                                           const float *conv_tanh_outputs, float *conv_errors, const cnt_cnn *fold,
+                                           float *total, const FanOut *fan, const float *core_buf, const float *ctx_tanh,
+                                           float *ctx_grad, const float *conv_tanh_outputs, float *conv_errors, const cnt_cnn *fold,
                                            const float *fold_weights, const float *fold_deltas, float *colsum_partial) {
     const int threads = block_errors_threads(R, N, fold != nullptr);
     block_err_kernel_t k = pick_block_errors_kernel(R, K, fold != nullptr, core_buf == nullptr, threads);
     CNT_REQUIRE(k != nullptr, "wavenet_block_errors: no kernel for %d residual and %d skip channels", R, K);
     CNT_REQUIRE(N > 0 && patTypes && skip_weights && out_weights && skip_errors && total && (core_buf || (ctx_tanh && conv_tanh_outputs)) &&
-                conv_errors,
+                conv_errors && (!ctx_tanh || ctx_grad) && (core_buf || ctx_grad != ctx_tanh),
                 "wavenet_block_errors: null argument");
     BlockErrArgs a = {};
     a.N = N; a.pat = patTypes; a.w_skip = skip_weights; a.w_out = out_weights; a.e_skip = skip_errors;
     a.total = total;
     if (fan) { a.from_skip = fan->from_skip; a.fan_n = fan->n; a.fan_targets = fan->targets; a.fan_is_skip = fan->is_skip; }
-    a.pre = core_buf; a.conv_tanh = conv_tanh_outputs; a.ctx_tanh = ctx_tanh; a.deltas = conv_errors;
+    a.pre = core_buf; a.conv_tanh = conv_tanh_outputs; a.ctx_tanh = ctx_tanh; a.ctx_grad = ctx_grad; a.deltas = conv_errors;
     a.colsum = colsum_partial;
     auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     if (fold) {
@@ -1054,8 +1056,8 @@ extern "C++" int cnt::wavenet_block_errors(hipStream_t stream, int R, int K, int
         a.conv_deltas = fold_deltas;
     }
     CNT_REQUIRE(aligned(skip_weights) && aligned(out_weights) && aligned(skip_errors) && aligned(total) &&
-                aligned(a.from_skip) && aligned(core_buf) && aligned(ctx_tanh) && aligned(conv_tanh_outputs) &&
-                aligned(conv_errors), "wavenet_block_errors: buffers must be 16-byte aligned");
+                aligned(a.from_skip) && aligned(core_buf) && aligned(ctx_tanh) && aligned(ctx_grad) &&
+                aligned(conv_tanh_outputs) && aligned(conv_errors), "wavenet_block_errors: buffers must be 16-byte aligned");
     ProfileScope prof(stream, fold ? "wavenet_block_errors+cnn" : "wavenet_block_errors");
     hipLaunchKernelGGL(k, dim3(wavenet_block_rows(R, N, fold != nullptr)), dim3(threads), 0, stream, a);
     CNT_HIP(hipGetLastError());

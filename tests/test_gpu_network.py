@@ -625,6 +625,39 @@ def test_wavenet_block_forward_edges(cnn_tanh, R, K, C, lengths):
     net.close()
 
 
+# block launches that form the gate's pre-activations again (tanh convolution), ones that read them, ones without conditioning
+# features.  Not compared: the layer below the blocks, whose errors go through a sum that only a forward pass clears, and the
+# conditioning part of layers whose pre-activations are kept: its gradient takes the place of its values.
+@pytest.mark.parametrize("cnn_tanh,R,K,C,lengths,conditioning_again", [
+    (1, 32, 64, 20, [120, 90], True), (1, 64, 128, 81, [700, 333], True), (1, 64, 256, 7, [16500], True), (0, 32, 64, 20, [120, 90], False),
+    (1, 64, 64, 0, [70, 52], True),
+])
+def test_second_backward_pass_of_a_wavenet_stack(cnn_tanh, R, K, C, lengths, conditioning_again):
+    import torch
+
+    print("wavenet second backward pass", cnn_tanh, R, K, C, lengths, flush=True)
+    capi = PC.pkg().capi
+    nb, Q, S, T = 3, 32, len(lengths), max(lengths)
+    pat, _, ctx, target, N = WD.make(lengths, Q, C or 4, upsample=5, seed=7)
+    net = capi.Network(json.dumps(PC.pkg().specs.wavenet_network_doc(nb, Q, R, K, C, cnn_tanh, 3)), S, T, mdn_config=[1, 0, Q, 0, 1, -1])
+    net.randomize(11, 0.2)
+    ctx_d = PC.dev(ctx)
+    if C:
+        net.set_context(ctx_d)
+    net.load_sequences(PC.dev(pat), T, min(lengths), torch.zeros(N, dtype=torch.float32, device="cuda"), PC.dev(target))
+    net.forward()
+    net.calculate_error()
+    net.backward()
+    first = {L["name"]: L["updates"].cpu().numpy() for L in net.layers if L["weight_count"]}
+    assert all(np.abs(v).max() > 0 for v in first.values())
+    net.backward()
+    for L in net.layers:
+        if L["weight_count"] and L["name"] != "emb" and (conditioning_again or L["type"] != "wavnetc"):
+            # the same products; only the order of their atomic sums may differ
+            assert PC.relerr(L["updates"].cpu().numpy(), first[L["name"]]) < 1e-5, L["name"]
+    net.close()
+
+
 @pytest.mark.parametrize("context_mv", [False, True])
 def test_wavenet_with_frame_rate_conditioning_network(context_mv, tmp_path):
     """The reference example's layout in full: externalloader -> skipini -> blstm -> cnn -> skipcat at one slot per
