@@ -464,7 +464,10 @@ int cnt_network_load_sequences(cnt_network *net, void *stream, int T, int Tmin, 
                                const float *inputs, const float *targets);
 /* NeuralNetwork::computeForwardPass in training mode (NeuralNetwork.cpp:1419-1471, :1734-1760). */
 int cnt_network_forward(cnt_network *net, void *stream);
-/* NeuralNetwork::calculateError (NeuralNetwork.cpp:2897-2990): the post-output layer's error into *loss_dev. */
+/* NeuralNetwork::calculateError (NeuralNetwork.cpp:2897-2990): the post-output layer's error into *loss_dev.  With an mdn
+ * layer the call also writes the output errors of the layer below (cnt_mdn_error_backward: the gradient takes what the
+ * error pass leaves in the units, in the reference as well), and the next cnt_network_backward starts from them: targets or
+ * outputs changed in between do not count, and a call after the backward pass replaces the deltas it has left there. */
 int cnt_network_calculate_error(cnt_network *net, void *stream, float *loss_dev);
 /* NeuralNetwork::computeBackwardPass (NeuralNetwork.cpp:2744-2800, :2864-2895): layers in reverse order.  The
  * layers' weight gradients run on streams of the network's own (same priority as any other stream), ordered after

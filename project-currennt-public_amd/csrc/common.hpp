@@ -118,6 +118,52 @@ __device__ __forceinline__ float act_deriv(int act, float y) {
     }
 }
 
+// ----- sum of a call's errors ---------------------------------------------------------------------
+__device__ __forceinline__ double wave_sum_64(double v) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+}
+
+// Sum of the errors of a call, over the workgroups of all its units' launches.  It is formed in 64 bits: workgroups add in the
+// order they finish in, and in 32 bits the last digits follow that order (the error of 31 000 frames, 2.2e5, came out
+// up to 0.27 apart between two passes over the same probabilities).  The values added have 24 digits each, so their 64-bit sum
+// is exact, or as good as, in any order.
+// The workgroup that finishes last hands the sum to the caller and leaves accumulator and ticket counter at zero for the next
+// call, so that no launch has to clear the caller's result first.
+struct LossSum {
+    double *acc;
+    unsigned *ticket;     // workgroups that have added so far
+    unsigned workgroups;  // of the call
+    float *result;
+};
+
+// by one thread of a workgroup, once
+__device__ __forceinline__ void add_loss(const LossSum &s, double v) {
+    // No fence (a device-scope fence writes the L2 back, which costs more than the kernel): the ticket is taken
+    // only after the add has returned its old value, i.e. has been performed where every XCD's atomics meet.
+    const double before = __hip_atomic_fetch_add(s.acc, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned one = 1u;
+    asm volatile("" : "+v"(one) : "v"(before));  // the ticket's operand depends on the returned value
+    if (__hip_atomic_fetch_add(s.ticket, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == s.workgroups - 1u) {
+        *s.result = (float)__hip_atomic_exchange(s.acc, 0.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(s.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// every wave's value to the call's sum; all threads of the workgroup take part
+template <int WAVES>
+__device__ __forceinline__ void add_block_loss(const LossSum &s, double wave_total) {
+    __shared__ double block_sum[WAVES];
+    if ((threadIdx.x & 63) == 0) block_sum[threadIdx.x >> 6] = wave_total;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double v = 0.0;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) v += block_sum[w];
+        add_loss(s, v);
+    }
+}
+
 // ----- optional per-kernel timing (capi.hip) -------------------------------------------------------
 // When enabled through cnt_profile_enable, every ProfileScope brackets the launches made inside it
 // with a pair of HIP events on the launch stream; cnt_profile_get sums them per label.
@@ -355,9 +401,9 @@ int load_clear_and_order(hipStream_t stream, const LoadClears &clears, const cha
 int lstm_load_sequences_collect(cnt_lstm *h, hipStream_t stream, const char *patTypes, int curMaxT, int curMinT,
                                 LoadClears &clears);
 int fill_words(hipStream_t stream, unsigned *p, size_t count, unsigned word);
-// cnt_sse_error and cnt_sse_backward in one launch; sum: 64 words of the caller's that are zero between calls
-int sse_error_backward(hipStream_t stream, int D, int N, const char *patTypes, const float *y, const float *target, float *err,
-                       float *result_dev, float *sum);
+// cnt_sse_error in one launch, summed in 64 bits; sum: 64 words of the caller's that are zero between calls
+int sse_error_once(hipStream_t stream, int D, int N, const char *patTypes, const float *y, const float *target, float *result_dev,
+                   float *sum);
 // out[d] += scale * sum over the N columns of a D x N column-major matrix (out pre-zeroed by the caller)
 int column_sum(hipStream_t stream, const float *v, int D, int N, float scale, float *out);
 

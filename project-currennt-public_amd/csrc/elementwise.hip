@@ -101,44 +101,25 @@ __global__ void sse_error_kernel(int D, size_t count, const char *__restrict__ p
     if (threadIdx.x == 0) atomicAdd(result, 0.5f * (part[0] + part[1] + part[2] + part[3]));
 }
 
-// Both in one pass over outputs and targets, for a caller that always runs both.  2^lanes_log2 neighbouring lanes take a slot, so no
-// index is divided; nothing waits for the pattern type.  The sum goes through an accumulator that the caller keeps at zero
-// between calls: the workgroup that adds last hands it to *result (its ticket is taken after its add has returned, so all adds
-// have been made) and clears it, and no launch has to clear *result first.  187 outputs at 12 000 slots: clear, error and
-// gradient launch took 5 + 21 + 5 us, this one 13.
+// The same in one launch, for a caller that keeps an accumulator: no launch clears *result first.  2^lanes_log2 neighbouring lanes
+// take a slot, so no index is divided; nothing waits for the pattern type.
 constexpr int kSseThreads = 1024;
-__global__ __launch_bounds__(kSseThreads) void sse_error_backward_kernel(int D, int N, int lanes_log2, const char *__restrict__ pat,
-                                                                         const float *__restrict__ y, const float *__restrict__ tgt,
-                                                                         float *__restrict__ err, float *__restrict__ result,
-                                                                         float *__restrict__ sum, unsigned *__restrict__ ticket) {
-    __shared__ float part[kSseThreads / 64];
+__global__ __launch_bounds__(kSseThreads) void sse_error_once_kernel(int D, int N, int lanes_log2, const char *__restrict__ pat,
+                                                                     const float *__restrict__ y, const float *__restrict__ tgt,
+                                                                     LossSum loss) {
     const int lane = threadIdx.x & ((1 << lanes_log2) - 1), slots = kSseThreads >> lanes_log2;
-    float acc = 0.0f;
+    double acc = 0.0;
     for (int slot = blockIdx.x * slots + (threadIdx.x >> lanes_log2); slot < N; slot += gridDim.x * slots) {
         const bool valid = pat[slot] != 0;
         const size_t row = (size_t)slot * D;
 #pragma unroll 4
         for (int d = lane; d < D; d += 1 << lanes_log2) {
             const float diff = y[row + d] - tgt[row + d];
-            const float e = valid ? diff : 0.0f;
-            err[row + d] = e;
+            const double e = valid ? diff : 0.0f;
             acc += e * e;
         }
     }
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float v = 0.0f;
-        for (int w = 0; w < kSseThreads / 64; ++w) v += part[w];
-        const float before = __hip_atomic_fetch_add(sum, 0.5f * v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        unsigned one = 1u;
-        asm volatile("" : "+v"(one) : "v"(before));  // the ticket's operand depends on the returned value
-        if (__hip_atomic_fetch_add(ticket, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u) {
-            *result = __hip_atomic_exchange(sum, 0.0f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
+    add_block_loss<kSseThreads / 64>(loss, wave_sum_64(0.5 * acc));
 }
 
 inline int stream_blocks(size_t count) {
@@ -453,13 +434,15 @@ int cnt_sse_backward(void *stream_, int D, int N, const char *patTypes, const fl
     return CNT_OK;
 }
 
-extern "C++" int cnt::sse_error_backward(hipStream_t stream, int D, int N, const char *patTypes, const float *y, const float *target,
-                                         float *err, float *result_dev, float *sum) {
+extern "C++" int cnt::sse_error_once(hipStream_t stream, int D, int N, const char *patTypes, const float *y, const float *target,
+                                     float *result_dev, float *sum) {
     int lanes_log2 = 0;
     while (lanes_log2 < 6 && (1 << lanes_log2) < D) ++lanes_log2;
     const int slots = kSseThreads >> lanes_log2;
-    hipLaunchKernelGGL(sse_error_backward_kernel, dim3((unsigned)std::min(256L, ((long)N + slots - 1) / slots)), dim3(kSseThreads), 0,
-                       stream, D, N, lanes_log2, patTypes, y, target, err, result_dev, sum, reinterpret_cast<unsigned *>(sum + 32));
+    const unsigned workgroups = (unsigned)std::min(256L, ((long)N + slots - 1) / slots);
+    const LossSum loss = {reinterpret_cast<double *>(sum), reinterpret_cast<unsigned *>(sum + 32), workgroups, result_dev};
+    hipLaunchKernelGGL(sse_error_once_kernel, dim3(workgroups), dim3(kSseThreads), 0, stream, D, N, lanes_log2, patTypes, y, target,
+                       loss);
     CNT_HIP(hipGetLastError());
     return CNT_OK;
 }

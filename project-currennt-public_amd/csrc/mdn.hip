@@ -44,51 +44,6 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-
-// Sum of the errors of a call, over the workgroups of all its units' launches.  It is formed in 64 bits: workgroups add in the
-// order they finish in, and in 32 bits the last digits follow that order (the error of 31 000 frames, 2.2e5, came out
-// up to 0.27 apart between two passes over the same probabilities).  The values added have 24 digits each, so their 64-bit sum
-// is exact, or as good as, in any order.
-// The workgroup that finishes last hands the sum to the caller and leaves accumulator and ticket counter at zero for the next
-// call, so that no launch has to clear the caller's result first.
-struct LossSum {
-    double *acc;
-    unsigned *ticket;     // workgroups that have added so far
-    unsigned workgroups;  // of the call
-    float *result;
-};
-
-// by one thread of a workgroup, once
-__device__ __forceinline__ void add_loss(const LossSum &s, double v) {
-    // No fence (a device-scope fence writes the L2 back, which costs more than the kernel): the ticket is taken
-    // only after the add has returned its old value, i.e. has been performed where every XCD's atomics meet.
-    const double before = __hip_atomic_fetch_add(s.acc, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    unsigned one = 1u;
-    asm volatile("" : "+v"(one) : "v"(before));  // the ticket's operand depends on the returned value
-    if (__hip_atomic_fetch_add(s.ticket, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == s.workgroups - 1u) {
-        *s.result = (float)__hip_atomic_exchange(s.acc, 0.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(s.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-
-// every wave's value to the call's sum; all threads of the workgroup take part
-template <int WAVES>
-__device__ __forceinline__ void add_block_loss(const LossSum &s, double wave_total) {
-    __shared__ double block_sum[WAVES];
-    if ((threadIdx.x & 63) == 0) block_sum[threadIdx.x >> 6] = wave_total;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double v = 0.0;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) v += block_sum[w];
-        add_loss(s, v);
-    }
-}
-
 // offset = (min + max) / 2 with the reference's start values, exp((x - offset)/T), normalise.
 // `in` points at the K inputs of the frame, `out` at its K outputs.
 __device__ __forceinline__ void softmax_frame(const float *__restrict__ in, float *__restrict__ out, int K,
@@ -155,8 +110,8 @@ __global__ void sigmoid_error_kernel(UnitGeom g, int continuous, const char *__r
             v += -logf(fmaxf(lim::kMin, b));
         }
     }
-    v = wave_sum(v);
-    cnt = wave_sum(cnt);
+    v = wave_sum_64(v);
+    cnt = wave_sum_64(cnt);
     if ((threadIdx.x & 63) == 0) {
         if (v != 0.0) atomicAdd(sums, v);
         if (cnt != 0.0) atomicAdd(sums + 1, cnt);
@@ -271,7 +226,7 @@ __global__ __launch_bounds__(64 * kSoftmaxErrWaves) void softmax_error_kernel(Un
         if (idx < g.capacity && idx >= 0) p = fmaxf(lim::kMin, prob[idx]);
         v = -logf(p);
     }
-    add_block_loss<kSoftmaxErrWaves>(loss, wave_sum((double)v));
+    add_block_loss<kSoftmaxErrWaves>(loss, wave_sum_64((double)v));
 }
 
 __global__ void softmax_backward_kernel(UnitGeom g, const char *__restrict__ pat, const float *__restrict__ target,

@@ -217,8 +217,8 @@ struct NetLayer {
     std::vector<int> cat_lo, cat_hi;         // skipcat: dimension range taken from each source
     const float *ext_data = nullptr;         // externalloader: [frame][sequence][dimension], set by the caller
     const float *ext_mean_std = nullptr;
-    bool post_errors_done = false;           // sse, mdn: calculate_error has already written the preceding layer's errors
-    float *loss_sum = nullptr;               // sse: see sse_error_backward
+    bool mdn_errors_done = false;            // mdn: calculate_error has already written the preceding layer's errors
+    float *loss_sum = nullptr;               // sse: see sse_error_once
     int ext_frames = 0, index_load_method = 0;
     int cnn_tanh = 0;                        // cnn: "tanhoutput"
     bool delta_fused = false;                // cnn followed by a wavnetc layer: that layer writes this layer's delta
@@ -1289,7 +1289,7 @@ int cnt_network_load_sequences(cnt_network *net, void *stream_, int T, int Tmin,
     CNT_REQUIRE(T >= 1 && T <= net->maxT && Tmin >= 1 && Tmin <= T, "network_load_sequences: lengths %d / %d outside "
                 "1..%d", T, Tmin, net->maxT);
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    net->layers.back().post_errors_done = false;
+    net->layers.back().mdn_errors_done = false;
     net->T = T;
     net->Tmin = Tmin;
     net->pat = patTypes;
@@ -1414,7 +1414,6 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
     // samples: 500 MB less to write per pass, 184 us).  A pass under capture may be replayed after backward passes that
     // are not known yet, so it clears all side buffers.
     const bool all = !net->sides.empty() && capturing(stream);
-    net->layers.back().post_errors_done = false;  // errors written for other outputs do not count
     size_t lo = 0, hi = net->skip_always, at = hi;  // [lo, hi): the run to clear that has not ended yet
     for (const auto &side : net->sides) {
         if (all || side.touched) {
@@ -1542,7 +1541,7 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
             }
             case K_MDN:
                 CNT_TRY(cnt_mdn_forward(L.mdn, stream, prev.out));
-                L.post_errors_done = false;  // new parameters: errors written for the old ones do not count
+                L.mdn_errors_done = false;  // new parameters: errors written for the old ones do not count
                 break;
             case K_GATED:
                 CNT_TRY(cnt_gatedact_forward(stream, L.size, N, L.pat, prev.out, L.out));
@@ -1566,13 +1565,7 @@ int cnt_network_calculate_error(cnt_network *net, void *stream_, float *loss_dev
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     NetLayer &post = net->layers.back();
     const NetLayer &last = net->layers[net->layers.size() - 2];
-    if (post.kind == K_SSE) {
-        // (as with a mixture layer below: both passes read outputs and targets)
-        if (!last.err) return cnt_sse_error(stream, post.size, post.N, post.pat, last.out, post.out, loss_dev);
-        CNT_TRY(sse_error_backward(stream, post.size, post.N, post.pat, last.out, post.out, last.err, loss_dev, post.loss_sum));
-        post.post_errors_done = true;
-        return CNT_OK;
-    }
+    if (post.kind == K_SSE) return sse_error_once(stream, post.size, post.N, post.pat, last.out, post.out, loss_dev, post.loss_sum);
     if (post.kind == K_DFT) {
         // DFTPostoutputLayer::calculateError (layers/DFTErrorPostoutputLayer.cu:2105-2150): the plain sum of the
         // distances of every resolution
@@ -1585,7 +1578,7 @@ int cnt_network_calculate_error(cnt_network *net, void *stream_, float *loss_dev
     // The preceding layer's error buffer has no other writer between the forward pass and the backward pass.
     if (last.err) {
         CNT_TRY(cnt_mdn_error_backward(post.mdn, stream, post.out, loss_dev, last.err));
-        post.post_errors_done = true;
+        post.mdn_errors_done = true;
         return CNT_OK;
     }
     return cnt_mdn_calculate_error(post.mdn, stream, post.out, loss_dev);
@@ -1769,17 +1762,11 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         const size_t count = (size_t)L.size * N;
         switch (L.kind) {
             case K_SSE:
-                // already written by cnt_network_calculate_error of this fraction's forward pass (a captured pass may be replayed
-                // without it)
-                if (L.post_errors_done) {
-                    L.post_errors_done = false;  // a layer below turns them into its deltas in place
-                    if (!capturing(stream)) break;
-                }
                 CNT_TRY(cnt_sse_backward(stream, L.size, N, L.pat, prev.out, L.out, prev.err));
                 break;
             case K_MDN:
                 // already written by cnt_network_calculate_error of this fraction's forward pass
-                if (L.post_errors_done) L.post_errors_done = false;
+                if (L.mdn_errors_done) L.mdn_errors_done = false;
                 else CNT_TRY(cnt_mdn_backward(L.mdn, stream, L.out, prev.err));
                 break;
             case K_DFT:

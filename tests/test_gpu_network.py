@@ -461,13 +461,47 @@ def test_squared_error_with_its_gradient(D, lengths):
         for _ in range(2):
             loss = float(net.calculate_error().item())
         if repeat == 1:
-            net.backward()  # uses the errors up
+            net.backward()  # a layer turns the errors into its deltas in place; the second pass forms them again
         net.backward()
         torch.cuda.synchronize()
         want = torch.where(valid, net.layer("o")["outputs"][: N * D].view(N, D) - t.view(N, D), 0.0)
         assert torch.equal(net.layer("o")["errors"][: N * D].view(N, D), want)
         exact = 0.5 * float((want.double() ** 2).sum())
         assert abs(loss - exact) <= (N * D / 256 + 300) * 2.0 ** -24 * exact  # a thread's chain, waves, workgroups
+    net.close()
+
+
+@pytest.mark.parametrize("act,D,lengths", [("identity", 3, [70, 65]), ("tanh", 187, [300, 299])])
+def test_squared_error_leaves_the_errors_alone(act, D, lengths):
+    """The error of a fraction can be asked for at any time: the gradient comes from the outputs and targets that are there when
+    the backward pass runs, and the deltas a backward pass has left stay."""
+    import torch
+
+    S, T = len(lengths), max(lengths)
+    N = S * T
+    net = PC.pkg().capi.Network(json.dumps({"layers": [{"size": 5, "name": "input", "type": "input"},
+                                                       {"size": D, "name": "o", "type": "feedforward_" + act, "bias": 1.0},
+                                                       {"size": D, "name": "post", "type": "sse"}]}), S, T)
+    net.randomize(3, 0.3)
+    pat = make_pat_types(lengths, T)
+    valid = PC.dev(pat).view(N, 1) != 0
+    net.load_sequences(PC.dev(pat), T, min(lengths), torch.randn(5 * N, device="cuda"), torch.randn(D * N, device="cuda"))
+    net.forward()
+    net.calculate_error()
+    o, tgt = net.layer("o"), net.layers[-1]["outputs"]
+    tgt.mul_(0.5).add_(1.0)
+    o["outputs"].mul_(0.75)
+    net.backward()
+    y = o["outputs"].view(N, D)
+    want = torch.where(valid, y - tgt.view(N, D), 0.0)
+    if act == "tanh":
+        want = (1.0 - y * y) * want
+    deltas = o["errors"].clone()
+    assert float((deltas.view(N, D) - want).abs().max()) <= 4e-7 * float(want.abs().max())
+    loss = float(net.calculate_error().item())
+    assert torch.equal(o["errors"], deltas)
+    exact = 0.5 * float((torch.where(valid, y - tgt.view(N, D), 0.0).double() ** 2).sum())
+    assert abs(loss - exact) <= 1.001 * 2.0 ** -24 * exact  # summed in 64 bits, rounded once
     net.close()
 
 
