@@ -1375,6 +1375,20 @@ bool capturing(hipStream_t stream) {
     return true;
 }
 
+// Fills memory that a call has just allocated and that keeps its content from then on.  Under capture the fill must not become
+// part of the graph, whose replays would start over from it: it runs on a stream of its own and is awaited.
+int fill_once(hipStream_t stream, unsigned *p, size_t count, unsigned word) {
+    if (!capturing(stream)) return fill_words(stream, p, count, word);
+    hipStream_t own = nullptr;
+    CNT_HIP(hipStreamCreateWithFlags(&own, hipStreamNonBlocking));
+    const int status = fill_words(own, p, count, word);
+    const hipError_t done = hipStreamSynchronize(own);
+    (void)hipStreamDestroy(own);
+    CNT_TRY(status);
+    CNT_HIP(done);
+    return CNT_OK;
+}
+
 // WaveNet residual block seen from its skip 1x1 layer i: [cnn 2R][wavnetc R][dense R, identity][skipadd, shares
 // the following sum][skipini][dense K, identity (i)]
 bool block_errors_at(const cnt_network *net, size_t i) {
@@ -2047,32 +2061,30 @@ int cnt_network_update(cnt_network *net, void *stream_, int option, float learni
     // call into the network reports it.
     CNT_TRY(report_failure(net, static_cast<hipStream_t>(stream_)));
     const size_t n = (size_t)net->n_weights;
+    // what the first update allocates is filled on the device: 42 MB of Adam's state for the feed-forward model's five
+    // million weights took 5 ms from the host
+    auto state = [&](float **p, size_t count, float start) -> int {
+        unsigned word;
+        std::memcpy(&word, &start, sizeof(word));
+        CNT_TRY(device_alloc(net, (void **)p, count * sizeof(float), false));
+        return fill_once(static_cast<hipStream_t>(stream_), reinterpret_cast<unsigned *>(*p), count, word);
+    };
     if (!net->cur_updates) {
-        CNT_TRY(device_alloc(net, (void **)&net->cur_updates, n * sizeof(float), true));
-        CNT_TRY(device_alloc(net, (void **)&net->deltas, n * sizeof(float), true));
+        CNT_TRY(state(&net->cur_updates, n, 0.0f));
+        CNT_TRY(state(&net->deltas, n, 0.0f));
     }
     const bool adagrad = option == 1 || option == 3, adam = option == 5;
     if ((adagrad || adam) && net->stats_option != option) {
         CNT_REQUIRE(net->stats_option < 0, "network_update: the optimizer option changed from %d to %d", net->stats_option,
                     option);
         // optimizers/Optimizer.cu:427-447: AdaGrad statistics start at 1e-6, Adam's (m, v) pairs at 0
-        // (filled on the device: 42 MB for the feed-forward model's five million weights took 5 ms from the host)
-        const float start = adam ? 0.0f : 1e-6f;
-        unsigned word;
-        std::memcpy(&word, &start, sizeof(word));
-        const size_t count = adam ? 2 * n : n;
-        CNT_TRY(device_alloc(net, (void **)&net->stats, count * sizeof(float), false));
-        CNT_TRY(fill_words(static_cast<hipStream_t>(stream_), reinterpret_cast<unsigned *>(net->stats), count, word));
+        CNT_TRY(state(&net->stats, adam ? 2 * n : n, adam ? 0.0f : 1e-6f));
         net->stats_option = option;
     }
     if (adam) {
         // beta1^t and beta2^t live in device memory and advance under the same flag as the step itself, so that a step
         // the device-side veto skips leaves them untouched as well
-        if (!net->adam_accum) {
-            const float ones[2] = {1.0f, 1.0f};
-            CNT_TRY(device_alloc(net, (void **)&net->adam_accum, sizeof(ones), false));
-            CNT_HIP(hipMemcpy(net->adam_accum, ones, sizeof(ones), hipMemcpyHostToDevice));
-        }
+        if (!net->adam_accum) CNT_TRY(state(&net->adam_accum, 2, 1.0f));
         CNT_TRY(opt_adam_advance(static_cast<hipStream_t>(stream_), net->adam_accum, net->veto));
     }
     const float *accum_dev = adam ? net->adam_accum : nullptr;

@@ -659,6 +659,49 @@ def test_wavenet_block_forward_edges(cnn_tanh, R, K, C, lengths):
     net.close()
 
 
+@pytest.mark.parametrize("option,rate,sgd_before", [(1, 1e-2, True), (1, 1e-2, False), (5, 1e-3, True), (5, 1e-3, False)])
+def test_first_optimizer_step_under_capture(option, rate, sgd_before):
+    """AdaGrad's and Adam's state is set up by the first update.  Where that one is captured, the replays go on from the state
+    as eager updates do, instead of starting over with each.  The step rounds every operation on its own: equal bits.
+    (Plain steps may come before, they keep no statistics.)"""
+    import torch
+
+    print("first update captured", option, sgd_before, flush=True)
+    capi = PC.pkg().capi
+    S, T, lengths = 2, 9, [9, 7]
+    doc = json.dumps({"layers": [{"size": 5, "name": "input", "type": "input"},
+                                 {"size": 3, "name": "o", "type": "feedforward_tanh", "bias": 1.0},
+                                 {"size": 3, "name": "post", "type": "sse"}]})
+    pat, x, t = PC.dev(make_pat_types(lengths, T)), torch.randn(5 * S * T, device="cuda"), torch.randn(3 * S * T, device="cuda")
+    nets = [capi.Network(doc, S, T) for _ in range(2)]
+    for net in nets:
+        net.randomize(3, 0.3)
+        net.load_sequences(pat, T, min(lengths), x, t)
+        net.forward()
+        net.backward()
+    graphed, eager = nets
+    graphed.updates.copy_(eager.updates)
+    if sgd_before:
+        for net in nets:
+            net.update(0, 1e-2, 0.0, 1.0)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, capture_error_mode="relaxed"):
+        graphed.update(option, rate, 0.0, float(sum(lengths)))
+    torch.cuda.synchronize()
+    assert torch.equal(graphed.weights, eager.weights)  # nothing has run yet
+    for step in range(4):
+        gradient = torch.randn_like(eager.updates) * (step + 1)
+        for net in nets:
+            net.updates.copy_(gradient)
+        graph.replay()
+        eager.update(option, rate, 0.0, float(sum(lengths)))
+        torch.cuda.synchronize()
+        assert torch.equal(graphed.weights, eager.weights), step
+    for net in nets:
+        net.close()
+
+
 # block launches that form the gate's pre-activations again (tanh convolution), ones that read them, ones without conditioning
 # features.  Not compared: the layer below the blocks, whose errors go through a sum that only a forward pass clears, and the
 # conditioning part of layers whose pre-activations are kept: its gradient takes the place of its values.
