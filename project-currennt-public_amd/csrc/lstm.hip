@@ -76,6 +76,7 @@ struct ChainParams {
     // at a later step takes what the step before it left: the carried cell-state terms from the state arrays, the
     // partial errors from the mailbox (which nothing may touch in between).
     int step_begin, step_end;
+    long long *clocks;  // of the kernels with CLOCKS
 };
 
 // A workgroup that gives up: every workgroup of the launch sees the device flag and drains; the host sees the latch
@@ -371,6 +372,7 @@ struct cnt_lstm {
     size_t lmail_words;
     float *flmail;         // XCD-local forward recursion: one mailbox per job
     size_t flmail_words;
+    long long *clocks;     // CNT_LSTM_TIMING: kClockWords of the forward and of the backward recursion
     int warm;  // read the recursion's inputs once before the XCD-local backward recursion (off; CNT_LSTM_WARM=1: on)
     int spread_lds_most;
     int spread_lds;  // dynamic LDS the XCD-local recursion asks for so that a compute unit takes one of its workgroups
@@ -468,12 +470,15 @@ int warm_backward_inputs(const cnt_lstm *h, hipStream_t stream, const ChainParam
 }
 
 template <int PW, int JB, int NSQ>
-chain_kernel_t local_pair(bool fwd) {
-    return fwd ? (chain_kernel_t)lstm_forward_local<PW, JB, NSQ> : (chain_kernel_t)lstm_backward_local<PW, JB, NSQ>;
+chain_kernel_t local_pair(bool fwd, bool clocks) {
+    if (clocks) return fwd ? (chain_kernel_t)lstm_forward_local<PW, JB, NSQ, true> : (chain_kernel_t)lstm_backward_local<PW, JB, NSQ, true>;
+    return fwd ? (chain_kernel_t)lstm_forward_local<PW, JB, NSQ, false> : (chain_kernel_t)lstm_backward_local<PW, JB, NSQ, false>;
 }
 template <int PW, int JB>
-chain_kernel_t local_pair(bool fwd, int nsq) {
-    return nsq == 1 ? local_pair<PW, JB, 1>(fwd) : nsq == 2 ? local_pair<PW, JB, 2>(fwd) : local_pair<PW, JB, 4>(fwd);
+chain_kernel_t local_pair(bool fwd, int nsq, bool clocks) {
+    return nsq == 1   ? local_pair<PW, JB, 1>(fwd, clocks)
+           : nsq == 2 ? local_pair<PW, JB, 2>(fwd, clocks)
+                      : local_pair<PW, JB, 4>(fwd, clocks);
 }
 
 // Cells per workgroup of a layer with H cells per direction and `jobs` jobs; 0: no XCD-local kernel.  A team should fit
@@ -491,23 +496,23 @@ int local_cells(int H, int jobs) {
 // layers of up to 256 cells take 16 cells per workgroup (more than eight jobs): no kernels of their own.
 int local_sequences(int H, int JB, int most) { return most > 2 || (JB == 16 && H <= 256) ? 4 : most; }
 
-chain_kernel_t pick_local_kernel(bool fwd, int H, int JB, int nsq) {
+chain_kernel_t pick_local_kernel(bool fwd, int H, int JB, int nsq, bool clocks) {
     const int PW = (H + 63) / 64;
     if (JB == 8) {
         switch (PW) {
-            case 2: return local_pair<2, 8>(fwd, nsq);
-            case 3: return local_pair<3, 8>(fwd, nsq);
-            case 4: return local_pair<4, 8>(fwd, nsq);
+            case 2: return local_pair<2, 8>(fwd, nsq, clocks);
+            case 3: return local_pair<3, 8>(fwd, nsq, clocks);
+            case 4: return local_pair<4, 8>(fwd, nsq, clocks);
         }
     }
     if (JB == 16) {
         switch (PW) {
-            case 3: return local_pair<3, 16, 4>(fwd);
-            case 4: return local_pair<4, 16, 4>(fwd);
-            case 5: return local_pair<5, 16>(fwd, nsq);
-            case 6: return local_pair<6, 16>(fwd, nsq);
-            case 7: return local_pair<7, 16>(fwd, nsq);
-            case 8: return local_pair<8, 16>(fwd, nsq);
+            case 3: return local_pair<3, 16, 4>(fwd, clocks);
+            case 4: return local_pair<4, 16, 4>(fwd, clocks);
+            case 5: return local_pair<5, 16>(fwd, nsq, clocks);
+            case 6: return local_pair<6, 16>(fwd, nsq, clocks);
+            case 7: return local_pair<7, 16>(fwd, nsq, clocks);
+            case 8: return local_pair<8, 16>(fwd, nsq, clocks);
         }
     }
     return nullptr;
@@ -595,7 +600,7 @@ int launch_chain(cnt_lstm *h, hipStream_t stream, bool fwd, ChainParams &p) {
         CNT_HIP(hipGetLastError());
         return CNT_OK;
     }
-    chain_kernel_t k = pick_local_kernel(fwd, h->H, h->local_jb, h->local_nsq);
+    chain_kernel_t k = pick_local_kernel(fwd, h->H, h->local_jb, h->local_nsq, h->clocks != nullptr);
     CNT_REQUIRE(k != nullptr, "lstm: no recursion kernel for H=%d JB=%d", h->H, h->local_jb);
     // heals the handle after a launch that gave up, zeroes the placement counters; in front of the backward recursion it
     // can be part of the cache-warming launch
@@ -633,6 +638,7 @@ int launch_chain(cnt_lstm *h, hipStream_t stream, bool fwd, ChainParams &p) {
     // more than half of a compute unit's LDS (unused dynamic shared memory), which still leaves room for two workgroups
     // of a matrix product beside it.  CNT_LSTM_SPREAD_LDS sets the request in bytes (0: none).
     CNT_TRY(set_spread_lds(h, reinterpret_cast<const void *>(k)));
+    p.clocks = h->clocks ? h->clocks + (fwd ? 0 : kClockWords) : nullptr;
     for (int job0 = 0; job0 < h->njobs; job0 += h->launch_jobs) {
         if (job0) CNT_TRY(guard());
         p.job0 = (unsigned)job0;
@@ -652,7 +658,7 @@ void local_placement(cnt_lstm *h, int lds_per_cu, int cus_per_xcd) {
     int most = kLocalSlots;
     for (int fwd = 0; fwd < 2; ++fwd) {
         int fit = 0;
-        const void *k = reinterpret_cast<const void *>(pick_local_kernel(fwd != 0, h->H, h->local_jb, h->local_nsq));
+        const void *k = reinterpret_cast<const void *>(pick_local_kernel(fwd != 0, h->H, h->local_jb, h->local_nsq, h->clocks != nullptr));
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k, local_threads((h->H + 63) / 64, h->local_jb, h->local_nsq), 0) != hipSuccess) {
             (void)hipGetLastError();
             fit = 1;
@@ -769,7 +775,7 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     const int groups = std::max((desc->S + kLocalSeqs - 1) / kLocalSeqs, solo ? 1 : std::min(kLocalXcds / ndir, desc->S));
     const int local_jb = local_cells(H, ndir * groups);
     const int local_nsq = local_sequences(H, local_jb, (desc->S + groups - 1) / groups);
-    const bool stepwise = (!solo && pick_local_kernel(true, H, local_jb, local_nsq) == nullptr) || std::getenv("CNT_LSTM_STEPWISE") != nullptr;
+    const bool stepwise = (!solo && pick_local_kernel(true, H, local_jb, local_nsq, false) == nullptr) || std::getenv("CNT_LSTM_STEPWISE") != nullptr;
 
     cnt_lstm *h = new (std::nothrow) cnt_lstm();
     CNT_REQUIRE(h != nullptr, "lstm_create: out of host memory");
@@ -822,6 +828,10 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     if (h->local) {
         h->team = (H + h->local_jb - 1) / h->local_jb;
         h->lmail_words = h->flmail_words = (size_t)h->njobs * local_job_words(h->team, h->local_jb, h->local_nsq);
+        if (err == hipSuccess && std::getenv("CNT_LSTM_TIMING")) {
+            err = hipMalloc(reinterpret_cast<void **>(&h->clocks), 2 * kClockWords * sizeof(long long));
+            if (err == hipSuccess) err = hipMemset(h->clocks, 0, 2 * kClockWords * sizeof(long long));
+        }
         local_placement(h, per_cu, cus / kLocalXcds);
         h->ctl_teams = local_blocks(h) / h->team + 1;
         if (err == hipSuccess) err = hipMalloc(reinterpret_cast<void **>(&h->lmail), h->lmail_words * sizeof(float));
@@ -857,6 +867,7 @@ int cnt_lstm_destroy(cnt_lstm *h) {
     if (h->lmail) (void)hipFree(h->lmail);
     if (h->flmail) (void)hipFree(h->flmail);
     if (h->ctl) (void)hipFree(h->ctl);
+    if (h->clocks) (void)hipFree(h->clocks);
     if (h->own_order) (void)hipFree(h->own_order);
     if (h->latch_host) (void)hipHostFree(h->latch_host);
     delete h;
@@ -977,10 +988,43 @@ extern "C++" int cnt::lstm_take_failure(cnt_lstm *h) {
         }                                       \
     } while (0)
 
+// CNT_LSTM_TIMING: means over the workgroups of the handle's last recursion in either direction of time, to stderr; then the
+// counts start over.  CNT_LSTM_TRACE: the points of the steps, too.
+static int print_clocks(cnt_lstm *h) {
+    using namespace cnt;
+    std::vector<long long> all(2 * kClockWords);
+    CNT_HIP(hipMemcpy(all.data(), h->clocks, all.size() * sizeof(long long), hipMemcpyDeviceToHost));
+    CNT_HIP(hipMemset(h->clocks, 0, all.size() * sizeof(long long)));
+    for (int backward = 0; backward < 2; ++backward) {
+        const long long *counts = all.data() + (backward ? kClockWords : 0), *traces = counts + (size_t)kClockBlocks * kClockCounts;
+        double m[kClockCounts] = {};
+        int active = 0;
+        for (unsigned b = 0; b < kClockBlocks; ++b) {
+            const long long *c = counts + (size_t)b * kClockCounts, *t = traces + (size_t)b * kTraceWords;
+            if (c[CLK_LOOP] == 0) continue;
+            ++active;
+            for (int q = 0; q < kClockCounts; ++q) m[q] += (double)c[q];
+            if (!std::getenv("CNT_LSTM_TRACE")) continue;
+            std::fprintf(stderr, "trace %s block %u job %lld member %lld xcd %lld:", backward ? "backward" : "forward", b, t[0], t[1], t[2]);
+            for (int q = 4; q < kTraceWords; ++q) std::fprintf(stderr, " %lld", t[q]);
+            std::fprintf(stderr, "\n");
+        }
+        if (!active) continue;
+        const double us = 0.01 / active / h->T;
+        std::fprintf(stderr, "lstm %s per step [us]: %s wave pause+poll %.3f (%.2f rounds) %s %.3f barrier %.3f loop %.3f | load wave busy "
+                     "%.3f store wave %.3f %s wave %.3f (T=%d, %d workgroups)\n", backward ? "backward" : "forward",
+                     backward ? "cell" : "gather", m[CLK_WAIT] * us, m[CLK_ROUNDS] / active / h->T, backward ? "update" : "product",
+                     m[CLK_REST] * us, m[CLK_BARRIER] * us, m[CLK_LOOP] * us, m[CLK_LOAD] * us, m[CLK_STORE] * us,
+                     backward ? "product" : "cell", m[CLK_OTHER] * us, h->T, active);
+    }
+    return CNT_OK;
+}
+
 int cnt_lstm_check(cnt_lstm *h, void *stream) {
     using namespace cnt;
     CNT_REQUIRE(h, "lstm_check: null handle");
     CNT_HIP(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
+    if (h->clocks) CNT_TRY(print_clocks(h));
     if (lstm_take_failure(h)) {
         set_error("%s", kGaveUp);
         return CNT_ERR_DEVICE;

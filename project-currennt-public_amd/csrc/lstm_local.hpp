@@ -174,8 +174,54 @@ __device__ __forceinline__ f32x4 local_product(const f32x4 &a, const float (&wre
     return acc0 + acc1;
 }
 
+// Diagnostic clocks (CNT_LSTM_TIMING, CNT_LSTM_TRACE): every kernel of the two recursions exists a second time, with CLOCKS, in
+// which the workgroups add up what their waves spend in the parts of a step and, for some steps in the middle, note when
+// they pass five points of it, on the 100 MHz clock that all compute units share.  The kernels without are free of all of
+// it: a branch on the chain of a step costs some of what it would measure.
+constexpr unsigned kClockBlocks = 512;  // workgroups that record
+enum { CLK_WAIT, CLK_REST, CLK_BARRIER, CLK_LOOP, CLK_ROUNDS, CLK_LOAD, CLK_STORE, CLK_OTHER, kClockCounts };
+constexpr int kTraceFirst = 100, kTraceSteps = 4, kTracePoints = 5, kTraceWords = 4 + kTraceSteps * kTracePoints;
+constexpr size_t kClockWords = (size_t)kClockBlocks * (kClockCounts + kTraceWords);  // of one direction of time
+template <bool CLOCKS>
+__device__ __forceinline__ long long clock_now() {
+    if constexpr (CLOCKS) return wall_clock64();
+    return 0;
+}
+template <bool CLOCKS>
+__device__ __forceinline__ void clock_add(long long &sum, long long since) {
+    if constexpr (CLOCKS) sum += wall_clock64() - since;
+}
+// by one lane of the wave that counted
+template <bool CLOCKS>
+__device__ __forceinline__ void clock_store(const ChainParams &p, int what, long long v) {
+    if constexpr (CLOCKS)
+        if (blockIdx.x < kClockBlocks) p.clocks[(size_t)blockIdx.x * kClockCounts + what] = v;
+}
+template <bool CLOCKS>
+__device__ __forceinline__ long long *clock_trace(const ChainParams &p) {
+    if constexpr (CLOCKS)
+        if (blockIdx.x < kClockBlocks) return p.clocks + (size_t)kClockBlocks * kClockCounts + (size_t)blockIdx.x * kTraceWords;
+    return nullptr;
+}
+template <bool CLOCKS>
+__device__ __forceinline__ void clock_point(const ChainParams &p, int step, int point) {
+    if constexpr (CLOCKS) {
+        long long *const trace = clock_trace<true>(p);
+        if (trace && step >= kTraceFirst && step < kTraceFirst + kTraceSteps)
+            trace[4 + kTracePoints * (step - kTraceFirst) + point] = wall_clock64();
+    }
+}
+template <bool CLOCKS>
+__device__ __forceinline__ void clock_where(const ChainParams &p, int job, int member) {
+    if constexpr (CLOCKS)
+        if (long long *const trace = clock_trace<true>(p)) {
+            trace[0] = job; trace[1] = member;
+            trace[2] = __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15u;  // XCC_ID, bits 3:0
+        }
+}
+
 // PW = ceil(cells per direction / 64) product waves, JB cells per workgroup, NSQ sequences per job
-template <int PW, int JB, int NSQ>
+template <int PW, int JB, int NSQ, bool CLOCKS>
 __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_local(const ChainParams p) {
     using Shape = LocalShape<JB, NSQ>;
     const int H = p.H, G = p.team;    // G = ceil(H / JB) workgroups; the last one may own fewer than JB cells
@@ -269,10 +315,12 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
         load_batch(sb, in);
         wait_all_vmem();
         put_batch(sb, in);
+        long long busy = 0;
         lds_barrier();  // start of the recursion
         for (int step = sb; step < p.step_end; ++step) {
             lds_barrier();
             if (given_up()) return;
+            const long long since = clock_now<CLOCKS>();
             const int phase = (step - sb) % BATCH, next = step - phase + BATCH;
             if (phase == 0) {
                 load_batch(next, in);
@@ -280,7 +328,9 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
                 wait_all_vmem();  // requested two steps ago or more
                 put_batch(next, in);
             }
+            clock_add<CLOCKS>(busy, since);
         }
+        if (lane == 0) clock_store<CLOCKS>(p, CLK_LOAD, busy);
         return;
     }
 
@@ -289,11 +339,13 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
         const int s = seq0 + ej, el = ec * NSQ + ej;
         f32x4 d = {0, 0, 0, 0};
         float e = 0, ce = 0;
+        long long busy = 0;
         lds_barrier();  // start of the recursion
         for (int step = p.step_begin; step < p.step_end; ++step) {
             const int b = step & 1, held = (step - p.step_begin) % STEPS;
             lds_barrier();  // results of this step are in LDS
             if (given_up()) return;
+            const long long since = clock_now<CLOCKS>();
             if (ahead == held) {
                 d = *reinterpret_cast<const f32x4 *>(&dl[b][ej][4 * ec]);
                 e = res[b][el][0]; ce = res[b][el][1];
@@ -319,7 +371,9 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
                         __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)((step - 1) % kMailSlots) * slot_words * 4u +
                                                                ((unsigned)me * RECV + (unsigned)(q * 64 + lane) * 4u) * 4u), 0, 0);
             }
+            clock_add<CLOCKS>(busy, since);
         }
+        if (lane == 0) clock_store<CLOCKS>(p, CLK_STORE, busy);
         return;
     }
 
@@ -336,10 +390,13 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
         const float *const mine = &dl[0][(lane & 3) % NSQ][4 * ((lane >> 2) % JB)];
         const unsigned pub_off = ((unsigned)(h / JB) * RECV + (unsigned)me * EL + (unsigned)(h % JB) * NSQ) * 4u;
         const bool publishes = h < G * JB;
+        long long busy = 0;
         wait_all_vmem();
         lds_barrier();  // start of the recursion
         for (int step = p.step_begin; step < p.step_end; ++step) {
             lds_barrier();  // the deltas of this step are in LDS
+            const long long since = clock_now<CLOCKS>();
+            if (tid == 0) clock_point<CLOCKS>(p, step, 3);
             // looked at only at the end of the step: the read is in flight behind the barrier together with the
             // deltas', and what a failed step publishes no longer matters
             const f32x4 a = *reinterpret_cast<const f32x4 *>(mine + (step & 1) * NSQ * DP);
@@ -352,8 +409,11 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
                 if (publishes)
                     mail_store(v, mail, (unsigned)(step % kMailSlots) * slot_words * 4u + pub_off, std::integral_constant<int, NSQ>{});
             }
+            clock_add<CLOCKS>(busy, since);
+            if (tid == 0) clock_point<CLOCKS>(p, step, 4);
             if (failed) return;
         }
+        if (tid == 0) clock_store<CLOCKS>(p, CLK_OTHER, busy);
         return;
     }
 
@@ -383,12 +443,17 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
         fg_later = D.fg[gi]; cerr_later = D.cerr[gi];
         if (peeps) own_later = gate == 1 ? D.dig[gi] : D.dfg[gi];
     }
+    long long waited = 0, rest = 0, barrier = 0, rounds = 0;
+    const bool records = CLOCKS && cw == 0 && lane == 0;
     wait_all_vmem();  // peepholes are in registers before the recursion starts
     lds_barrier();    // start of the recursion: coefficients of steps 0 and 1 are in LDS
+    const long long begin = clock_now<CLOCKS>();
 
     for (int step = p.step_begin; step < p.step_end; ++step) {
         const bool first = (step == 0), last = (step == T - 1);
         const int b = step & 1, r = (step - p.step_begin) % RING;
+        const long long since = clock_now<CLOCKS>();
+        if (records) clock_point<CLOCKS>(p, step, 0);
         // this step's coefficients: in LDS since before the previous barrier, fetched while the poll is in flight
         const f32x4 k = *reinterpret_cast<const f32x4 *>(coef[r][el]);
         const float k_own = coef_own[r][el][gate], fg = coef_fg[r][el][0], dummy = coef_fg[r][el][1];
@@ -407,6 +472,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
             for (int d = 0; d < p.poll_delay; ++d) __builtin_amdgcn_s_sleep(1);
             for (;;) {
                 poll_load<NL>(slot, poll_off, poll_stride, poll_off_last, w);
+                if constexpr (CLOCKS) ++rounds;
                 unsigned worst = 0;
 #pragma unroll
                 for (int i = 0; i < NL; ++i) worst = max(max(worst, w[i].x), max(max(w[i].y, w[i].z), w[i].w));
@@ -419,6 +485,8 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
                 }
                 for (int d = 0; d < p.poll_gap; ++d) __builtin_amdgcn_s_sleep(1);
             }
+            clock_add<CLOCKS>(waited, since);
+            if (records) clock_point<CLOCKS>(p, step, 1);
             f32x4 sum = __builtin_bit_cast(f32x4, w[NL - 1]);
 #pragma unroll
             for (int r = 0; r < 4; ++r) sum[r] = last_counts ? sum[r] : 0.0f;
@@ -442,7 +510,19 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
             wait_failed = 1;
             if (lane == 0) raise_abort(p);
         }
+        if (records) clock_point<CLOCKS>(p, step, 2);
+        const long long at_barrier = clock_now<CLOCKS>();
         lds_barrier();
+        clock_add<CLOCKS>(barrier, at_barrier);
+        clock_add<CLOCKS>(rest, since);  // the whole step: what was waited is taken off below
         if (given_up()) return;
+    }
+    if (records) {
+        clock_store<CLOCKS>(p, CLK_WAIT, waited);
+        clock_store<CLOCKS>(p, CLK_REST, rest - waited - barrier);
+        clock_store<CLOCKS>(p, CLK_BARRIER, barrier);
+        clock_store<CLOCKS>(p, CLK_ROUNDS, rounds);
+        clock_store<CLOCKS>(p, CLK_LOOP, clock_now<CLOCKS>() - begin);
+        clock_where<CLOCKS>(p, job, me);
     }
 }

@@ -33,7 +33,7 @@
 // bytes: 1.05 instead of 1.00.
 
 // PW = ceil(cells per direction / 64) gather waves, JB cells per workgroup, NSQ sequences per job
-template <int PW, int JB, int NSQ>
+template <int PW, int JB, int NSQ, bool CLOCKS>
 __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local(const ChainParams p) {
     using Shape = LocalShape<JB, NSQ>;
     const int H = p.H, G = p.team;       // G = ceil(H / JB) workgroups; the last one may own fewer than JB cells
@@ -113,10 +113,12 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
         load_batch(0, in);
         wait_all_vmem();
         put_batch(0, in);
+        long long busy = 0;
         lds_barrier();  // start of the recursion
         for (int step = 0; step < T; ++step) {
             lds_barrier();
             if (given_up()) return;
+            const long long since = clock_now<CLOCKS>();
             const int phase = step % BATCH, next = step - phase + BATCH;
             if (phase == 0) {
                 for (int d = 0; d < p.mem_delay_fwd; ++d) __builtin_amdgcn_s_sleep(1);
@@ -125,7 +127,9 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
                 wait_all_vmem();  // requested two steps ago or more
                 put_batch(next, in);
             }
+            clock_add<CLOCKS>(busy, since);
         }
+        if (lane == 0) clock_store<CLOCKS>(p, CLK_LOAD, busy);
         return;
     }
 
@@ -133,12 +137,14 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
         // ------------------------------------------------------------------ store wave
         const int s = seq0 + cs, el = (cj / 4 * NSQ + cs) * 4 + cj % 4;
         f32x4 g = {0, 0, 0, 0}, r = {0, 0, 0, 0};
+        long long busy = 0;
         lds_barrier();  // start of the recursion
         lds_barrier();  // the first step's sums
         for (int step = 0; step < T; ++step) {
             const int b = step & 1, held = step % STEPS;
             lds_barrier();  // results of this step are in LDS
             if (given_up()) return;
+            const long long since = clock_now<CLOCKS>();
             if (ahead == held) {
                 g = *reinterpret_cast<const f32x4 *>(res_gate[b][el]);
                 r = *reinterpret_cast<const f32x4 *>(res[b][el]);
@@ -166,7 +172,9 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
                         __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)(step % kMailSlots) * slot_words * 4u +
                                                                ((unsigned)me * RECV + (unsigned)(q * 64 + lane) * 4u) * 4u), 0, 0);
             }
+            clock_add<CLOCKS>(busy, since);
         }
+        if (lane == 0) clock_store<CLOCKS>(p, CLK_STORE, busy);
         return;
     }
 
@@ -206,11 +214,15 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
         const float *const sent = hpub[cw][lane % VPW];
         const float *const my_red = &red[0][0][cell * 4 + gate][seq];
         float c_prev = 0.0f, start = bias;
+        long long busy = 0;
+        const bool records = CLOCKS && cw == 0 && lane == 0;
         wait_all_vmem();
         lds_barrier();  // start of the recursion
         for (int step = 0; step < T; ++step) {
             const int b = step & 1;
             lds_barrier();
+            const long long since = clock_now<CLOCKS>();
+            if (records) clock_point<CLOCKS>(p, step, 3);
             // (looked at at the end of the step: what a step that failed publishes no longer matters)
             const int failed = given_up();
             float a = pre[step % RING][el][gate];
@@ -255,9 +267,12 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
             }
             c_prev = dummy && !dir ? c_prev : c;
             start = peeps ? bias + c_prev * peep : bias;
+            clock_add<CLOCKS>(busy, since);
+            if (records) clock_point<CLOCKS>(p, step, 4);
             if (failed) return;
         }
         lds_barrier();  // results of the last step are in LDS
+        if (records) clock_store<CLOCKS>(p, CLK_OTHER, busy);
         return;
     }
 
@@ -281,11 +296,16 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
     const int my_vec = (16 * pw + (lane >> 2)) * NSQ + (lane & 3) % NSQ;
     const bool inside = my_vec < vectors;
     const unsigned poll_off = ((unsigned)me * RECV + (unsigned)(inside ? my_vec : 0) * 4u) * 4u;
+    long long waited = 0, rest = 0, barrier = 0, rounds = 0;
+    const bool records = CLOCKS && tid == 0;
     wait_all_vmem();
     lds_barrier();  // start of the recursion
+    const long long begin = clock_now<CLOCKS>();
     lds_barrier();  // step 0 has nothing to gather
 
     for (int step = 1; step < T; ++step) {
+        const long long since = clock_now<CLOCKS>();
+        if (records) clock_point<CLOCKS>(p, step, 0);
         const float *slot = mailbox + (size_t)((step - 1) % kMailSlots) * slot_words;
         bool ok = true;
         u32x4 w[1];
@@ -293,6 +313,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
         for (int d = 0; d < p.poll_delay_fwd; ++d) __builtin_amdgcn_s_sleep(1);
         for (;;) {
             poll_load<1>(slot, poll_off, 0u, poll_off, w);
+            if constexpr (CLOCKS) ++rounds;
             const unsigned worst = max(max(w[0].x, w[0].y), max(w[0].z, w[0].w));
             if (worst != kEmpty) break;
             if (++spins > p.spin_limit) { ok = false; break; }
@@ -303,6 +324,8 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
             }
             for (int d = 0; d < p.poll_gap; ++d) __builtin_amdgcn_s_sleep(1);
         }
+        clock_add<CLOCKS>(waited, since);
+        if (records) clock_point<CLOCKS>(p, step, 1);
         if (!inside) w[0] = u32x4{0, 0, 0, 0};
         f32x4 sum = local_product<JB == 8 ? 3 : 4, 4 * BLOCKS>(__builtin_bit_cast(f32x4, w[0]), wreg, std::make_integer_sequence<int, BLOCKS>{});
         // register = sequence; where the wave's halves meet, the lower one ends up with the first half of the sequences
@@ -319,11 +342,23 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
             out[0] = sum_halves(sum[0], sum[0]);
         }
         if (__builtin_amdgcn_ballot_w64(!ok) != 0) wait_failed = 1;
+        if (records) clock_point<CLOCKS>(p, step, 2);
+        const long long at_barrier = clock_now<CLOCKS>();
         lds_barrier();
+        clock_add<CLOCKS>(barrier, at_barrier);
+        clock_add<CLOCKS>(rest, since);  // the whole step: what was waited is taken off below
         if (given_up()) {
             if (tid == 0) raise_abort(p);
             return;
         }
     }
     lds_barrier();  // results of the last step
+    if (records) {
+        clock_store<CLOCKS>(p, CLK_WAIT, waited);
+        clock_store<CLOCKS>(p, CLK_REST, rest - waited - barrier);
+        clock_store<CLOCKS>(p, CLK_BARRIER, barrier);
+        clock_store<CLOCKS>(p, CLK_ROUNDS, rounds);
+        clock_store<CLOCKS>(p, CLK_LOOP, clock_now<CLOCKS>() - begin);
+        clock_where<CLOCKS>(p, job, me);
+    }
 }

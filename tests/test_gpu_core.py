@@ -1,6 +1,8 @@
 """GPU parity tests (through the C ABI) for the matrix product seam, dense / SSE layers and the LSTM.
 Tolerance: 1e-4 on the L2-normalised difference per tensor (fp32, different summation order);
 masking and indexing are asserted bit-exactly inside parity_cases."""
+import re
+
 import pytest
 
 import parity_cases as PC
@@ -447,6 +449,28 @@ def test_lstm_step_by_step_recursion_equals_the_persistent_kernels(monkeypatch):
     monkeypatch.setenv("CNT_LSTM_STEPWISE", "1")
     assert PC.run_lstm_case(24, 128, True, [10, 6, 10], seed=5, wscale=0.5, escale=20.0, repeat_backward=True) < TOL
     assert PC.run_lstm_case(30, 256, False, [12, 12, 7], seed=6) < TOL
+
+
+@pytest.mark.parametrize("L,bidir,lengths", [(256, True, [110, 104, 90]), (256, False, [107]), (600, True, [104] * 34), (1024, True, [106, 105])])
+def test_lstm_recursion_clocks(L, bidir, lengths, monkeypatch, capfd):
+    """CNT_LSTM_TIMING / CNT_LSTM_TRACE: the recursion kernels with clocks compute the same, and cnt_lstm_check prints what the
+    parts of a step took and when every workgroup of a team passed the points of the traced steps."""
+    print("lstm recursion clocks", L, bidir, lengths, flush=True)
+    monkeypatch.setenv("CNT_LSTM_TIMING", "1")
+    monkeypatch.setenv("CNT_LSTM_TRACE", "1")
+    assert PC.run_lstm_two_recursions(16, L, bidir, lengths, seed=4) < TOL
+    lines = capfd.readouterr().err.splitlines()
+    for kind in ("forward", "backward"):
+        mean, = [line for line in lines if line.startswith("lstm %s per step" % kind)]
+        part = {k: float(re.search(k + r" ([0-9.]+)", mean).group(1)) for k in (r"pause\+poll", "barrier", "loop")}
+        assert 0 < part[r"pause\+poll"] < part["loop"] and 0 < part["barrier"] < part["loop"], mean
+        traces = [line for line in lines if line.startswith("trace %s block" % kind)]
+        assert len(traces) == int(re.search(r"(\d+) workgroups", mean).group(1)) > 0
+        for line in traces:
+            points = [int(v) for v in line.split(":")[1].split()]
+            assert len(points) == 20
+            for i in range(0, 20, 5):
+                assert 0 < points[i] <= points[i + 1] <= points[i + 2] and 0 < points[i + 3] <= points[i + 4], line
 
 
 def test_lstm_config2_layer_full_length_two_recursions():
