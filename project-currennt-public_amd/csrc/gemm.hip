@@ -68,11 +68,18 @@ inline int pick_vec(const GemmArgs &a, bool for_a) {
 // Between 256 and 511 values of k it is the last generation that decides: large tiles pay where they fill what the chip holds of
 // them at a time (768) to at least nine tenths.  64 / 128, us, for 1024 rows and a k-contiguous A: k = 256, 752 tiles (0.98) 54 /
 // 49, 704 (0.92) 1.05 times as fast, 1360 (0.89) 1.02, 2000 (0.87) 0.97, 640 (0.83) 1.04, 1040 (0.68) 0.87; k = 448, 752 tiles 86 /
-// 72, 1360 1.09 times, 1040 0.98; a row-contiguous A within 3% of that; 1936 x 6000 x 256 59 / 50; k = 192 no gain anywhere.  From
-// 768 values on they pay from 336 tiles on (300 / 336 / 376 / 480 / 560 tiles, times as fast: k = 768 0.84 / 1.00 / 1.01 / 1.17 /
-// 1.03, k = 2048 0.94 / 1.11 / 1.11 / 1.28 / 1.10; 1024 x 6144 x 2048 170 / 132 us), and with 512 to 767 values they lose 1 to 10 % where
-// they begin a second generation that stays a quarter full or less (800 / 896 / 960 / 1040 tiles of k = 512 0.90 / 0.93 / 0.98 /
-// 1.06).
+// 72, 1360 1.09 times, 1040 0.98; a row-contiguous A within 3% of that; 1936 x 6000 x 256 59 / 50; k = 192 no gain anywhere.
+// The other lines lie where a generation ends, too: the 256 compute units hold 768 large and 1280 small tiles at a time, five
+// per compute unit.  From 768 values on the large tile pays as soon as the small ones begin a second generation: 320 large tiles are
+// 1280 small ones.  Times as fast with 304 / 320 / 336 / 400 / 480 / 560 / 768 / 800 / 1040 large tiles (least and most over 512,
+// 1024 and 2048 rows and both orders of A): k = 768 0.84-0.87 / 0.86-0.89 / 1.00-1.04 / 1.08-1.13 / 1.16-1.19 / 1.04 / 1.23-1.25 /
+// 0.97-0.99 / 1.10-1.12, k = 1024 0.87-0.92 / 0.89-0.94 / 1.04-1.08 / 1.12-1.18 / 1.20-1.24 / 1.05-1.07 / 1.26-1.28 / 1.00 / 1.11-1.15,
+// k = 3072 0.95-1.01 / 0.96-1.02 / 1.12-1.18 / 1.22-1.28 / 1.28-1.34 / 1.12 / 1.32-1.35 / 1.06 / 1.17-1.20.
+// With 512 to 767 values it needs 600 (560: 0.99-1.05, 600: 1.05-1.12, 768: 1.17-1.25), and a second generation of its own that is
+// hardly begun costs more than it gains: 800 / 864 / 896 / 960 / 1040 tiles at k = 512 0.90 / 0.92 / 0.93 / 0.96-0.99 /
+// 1.03-1.07, k = 600 0.93 / 0.96 / 0.97 / 1.00-1.02 / 1.06-1.11, k = 640 0.93 / 0.98 / 1.00 / 1.03 / 1.07-1.12, k = 736
+// 0.96 / 1.00-1.03 / 1.02-1.04 / 1.06-1.08 / 1.09-1.12.  The line at 960 is right for k up to 600; it gives away up to 7 % of
+// the 860 to 960 tiles at longer k.
 inline long large_tiles(const GemmArgs &a) { return (long)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.nprob; }
 
 // The weight gradient of one dense layer of 64 to 256 large tiles (1024 x 1024 weights and more) also takes the large tile, and
