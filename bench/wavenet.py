@@ -70,15 +70,15 @@ def run(args, pkg):
     roof = {"bound": "hbm", "kernel": dom, "traffic": None, "peak": PEAK_HBM_GBS, "unit": "GB/s"}
     if dom == "wavenet_block_errors+cnn" and (R, K, N) == (64, 128, 32000):
         # two rocprofv3 --pmc runs (FETCH_SIZE x 2.00 by a copy of known size, WRITE_SIZE x 1.00) of this workload:
-        # 105.8 MB read + 54.8 MB written per launch of wavenet_block_errors_kernel<64, 128, true>
-        roof["traffic"] = 160.6e6
+        # 82.0 MB read + 44.6 MB written per launch of wavenet_block_errors_kernel<64, 128, true, true, 512>
+        roof["traffic"] = 126.6e6
         roof["traffic_source"] = "profiles/wavenet_c4_backward_kernel_stats.md"
     if dom == "wavenet_block_errors+cnn":
         # one residual block's error path: reads the skip errors (K), what the later block handed on (R), the deltas of
-        # the convolution above (2R, both taps from the same array), the gate pre-activations, the convolution's tanh
-        # outputs and the conditioning tanh (2R each); writes the block's summed errors (R, which the earlier block's
+        # the convolution above (2R, both taps from the same array), the convolution's tanh outputs and the conditioning
+        # tanh (2R each); writes the block's summed errors (R, which the earlier block's
         # launch reads where they stand), the convolution deltas and the conditioning gradient (2R each)
-        nbytes = ((K + R + 4 * 2 * R) + (R + 2 * 2 * R)) * 4.0 * N
+        nbytes = ((K + R + 3 * 2 * R) + (R + 2 * 2 * R)) * 4.0 * N
     elif dom == "gemm:cnn_dW":
         # per launch: read x (R) and the deltas (2R) for each of the two live taps, write nothing of size N
         nbytes = 2 * (R + 2 * R) * 4.0 * N

@@ -92,11 +92,11 @@ def lstm_c1(args, pkg):
     hop_us = capi.probe_hop_latency(same_xcd=True, with_compute=True, rounds=2000)
     roof = {"bound": "mfma", "achieved": ach, "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s", "frac": ach / PEAK_FP32_MFMA_TFLOPS,
             # two rocprofv3 --pmc runs of this workload (FETCH_SIZE x 2.00 by a copy of known size, WRITE_SIZE x 1.00):
-            # 12.2 MB read + 7.0 MB written per launch of lstm_backward_local<4, 8>; algorithmic 12.5 MB
+            # 10.6 MB read + 5.5 MB written per launch of lstm_backward_local<4, 8, 1, false>; algorithmic 12.5 MB
             "traffic": 16.1e6, "traffic_source": "profiles/lstm_c1_backward_kernel_stats.md",
             "kernel": dom, "us_per_step": us_per_step, "latency_floor_us_per_step": hop_us,
             "frac_of_latency_floor": hop_us / us_per_step,
-            "note": "latency-bound recursion (T sequential steps, one job of four sequences on one XCD): `frac` is against the "
+            "note": "latency-bound recursion (T sequential steps, four jobs of one sequence, each on one XCD): `frac` is against the "
                     "fp32 MFMA peak, `frac_of_latency_floor` against one measured hop inside an XCD plus a step's arithmetic"}
     extra = {"roofline": roof, "kernels": kernels}
     if not args.no_cpu:
@@ -209,9 +209,9 @@ def dft_c5(args, pkg):
     nbytes = 12.0 * W * n  # per launch (all three resolutions in it): read source + target once, write the gradient once
     ach = nbytes / (kernels[dom]["avg_ms"] * 1e-3) / 1e9
     # traffic: two rocprofv3 --pmc runs of this workload (FETCH_SIZE x 2.00 by a copy of known size, WRITE_SIZE x 1.00):
-    # dft_loss_kernel 6.3 MB read (every sample is part of four frames per resolution) + 6.3 MB written (overlap-add)
+    # dft_loss_kernel 5.4 MB read (every sample is part of four frames per resolution) + 6.3 MB written (overlap-add)
     roof = {"bound": "hbm", "achieved": ach, "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": ach / PEAK_HBM_GBS,
-            "traffic": 12.6e6 if (W, n) == (8, 16000) else None, "traffic_source": "profiles/dft_c5_backward_kernel_stats.md",
+            "traffic": 11.7e6 if (W, n) == (8, 16000) else None, "traffic_source": "profiles/dft_c5_backward_kernel_stats.md",
             "kernel": dom, "note": "1.5 MB of samples and gradients, 0.17 GFLOP: launch- and latency-bound, far from either roof"}
     extra = {"roofline": roof, "kernels": kernels}
     if not args.no_cpu:

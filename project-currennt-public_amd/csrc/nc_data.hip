@@ -562,8 +562,10 @@ int cnt_dataset_fraction_fill(cnt_dataset *d, int first_seq, char *patTypes, flo
     // no row.  (Reading a sequence whole, swapping it in place and copying its rows over a cleared fraction moves every
     // byte five times.)  From two megabytes on several threads share the blocks; below, waking them takes what they save.
     // 10 sequences of 300 to 600 rows of 382 inputs and 187 targets, 13.7 MB, into fresh pages: 907 -> 491 us with eight
-    // threads, what is left is mostly the kernel's zeroing of the pages; 8 x 48 rows of 432 + 4 values, 0.7 MB, by the
-    // caller alone: 54 -> 32 us.
+    // threads; 8 x 48 rows of 432 + 4 values, 0.7 MB, by the caller alone: 54 -> 32 us.  Of the 491, some 350 are the kernel's
+    // faults and zeroing of the pages: into arrays that are there the call takes 120 to 150 us.  (Bare loops of eight threads
+    // there: reading the rows from the file cache 31 us, with a copy to pages that are there 52, to fresh ones 404, touching
+    // fresh pages alone 438.)
     struct Block { long long at; float *out; int col, t0, t1, rows, width; };  // rows of t0 .. t1 from the file, the rest zeros
     std::vector<Block> blocks;
     auto add = [&](const char *name, int width, float *out) {
