@@ -125,8 +125,8 @@ __device__ __forceinline__ double wave_sum_64(double v) {
 }
 
 // Sum of the errors of a call, over the workgroups of all its units' launches.  It is formed in 64 bits: workgroups add in the
-// order they finish in, and in 32 bits the last digits follow that order (the error of 31 000 frames, 2.2e5, came out
-// up to 0.27 apart between two passes over the same probabilities).  The values added have 24 digits each, so their 64-bit sum
+// order they finish in, and in 32 bits the last digits follow that order (over the same probabilities the error of 31 000 frames,
+// 2.2e5, came out up to 0.36 apart).  The values added have 24 binary digits each, so their 64-bit sum
 // is exact, or as good as, in any order.
 // The workgroup that finishes last hands the sum to the caller and leaves accumulator and ticket counter at zero for the next
 // call, so that no launch has to clear the caller's result first.
