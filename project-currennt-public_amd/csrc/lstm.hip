@@ -64,7 +64,7 @@ struct ChainParams {
     int poll_delay_fwd, mem_delay_fwd;  // forward: the same, and before the load wave's
     int *latch;  // host-visible mark "a recursion of this handle gave up" (pinned host memory), never cleared by kernels
     int *veto;   // optional device flag shared by a network's handles, set together with the latch
-    // XCD-local backward recursion: jobs = (direction, group of sequences), see lstm_local.hpp
+    // XCD-local recursions: jobs = (direction, group of sequences), see lstm_local.hpp
     unsigned job0;      // first job of this launch
     int njobs, groups;  // jobs of this launch; groups of sequences per direction
     int team;           // workgroups of a job's team
@@ -365,7 +365,7 @@ struct cnt_lstm {
     int njobs, groups;
     int launch_jobs;       // jobs of one launch: as many as complete teams fit the compute units at once
     int local_jb, team;    // cells per workgroup and workgroups of a team
-    int local_nsq;         // sequences a job's kernels move and multiply: 1, 2 or 4
+    int local_most;        // sequences of a job at most: 1 or 4
     int ctl_teams;
     unsigned *ctl;
     float *lmail;
@@ -469,16 +469,14 @@ int warm_backward_inputs(const cnt_lstm *h, hipStream_t stream, const ChainParam
     return CNT_OK;
 }
 
-template <int PW, int JB, int NSQ>
+template <int PW, int JB, int MOST>
 chain_kernel_t local_pair(bool fwd, bool clocks) {
-    if (clocks) return fwd ? (chain_kernel_t)lstm_forward_local<PW, JB, NSQ, true> : (chain_kernel_t)lstm_backward_local<PW, JB, NSQ, true>;
-    return fwd ? (chain_kernel_t)lstm_forward_local<PW, JB, NSQ, false> : (chain_kernel_t)lstm_backward_local<PW, JB, NSQ, false>;
+    if (clocks) return fwd ? (chain_kernel_t)lstm_forward_local<PW, JB, MOST, true> : (chain_kernel_t)lstm_backward_local<PW, JB, MOST, true>;
+    return fwd ? (chain_kernel_t)lstm_forward_local<PW, JB, MOST, false> : (chain_kernel_t)lstm_backward_local<PW, JB, MOST, false>;
 }
 template <int PW, int JB>
-chain_kernel_t local_pair(bool fwd, int nsq, bool clocks) {
-    return nsq == 1   ? local_pair<PW, JB, 1>(fwd, clocks)
-           : nsq == 2 ? local_pair<PW, JB, 2>(fwd, clocks)
-                      : local_pair<PW, JB, 4>(fwd, clocks);
+chain_kernel_t local_pair(bool fwd, int most, bool clocks) {
+    return most == 1 ? local_pair<PW, JB, 1>(fwd, clocks) : local_pair<PW, JB, kLocalSeqs>(fwd, clocks);
 }
 
 // Cells per workgroup of a layer with H cells per direction and `jobs` jobs; 0: no XCD-local kernel.  A team should fit
@@ -492,27 +490,32 @@ int local_cells(int H, int jobs) {
     return H > 512 ? 0 : H <= 128 ? 8 : H <= 256 ? (jobs <= kLocalXcds ? 8 : 16) : 16;
 }
 
-// Sequences the kernels of a job move: the smallest that holds the largest job.  Jobs of one or two sequences are rare where
-// layers of up to 256 cells take 16 cells per workgroup (more than eight jobs): no kernels of their own.
-int local_sequences(int H, int JB, int most) { return most > 2 || (JB == 16 && H <= 256) ? 4 : most; }
+// Groups of sequences per direction.  A job of fewer sequences takes shorter steps, so as many as complete teams fit the compute
+// units one workgroup each; at least what four sequences per job need.
+int local_groups(int H, int JB, int S, int ndir, int cus_per_xcd) {
+    const int least = (S + kLocalSeqs - 1) / kLocalSeqs;
+    if (JB <= 0) return least;
+    const int resident = kLocalXcds * std::max(1, cus_per_xcd / ((H + JB - 1) / JB));
+    return std::max(least, std::min(resident / ndir, S));
+}
 
-chain_kernel_t pick_local_kernel(bool fwd, int H, int JB, int nsq, bool clocks) {
+chain_kernel_t pick_local_kernel(bool fwd, int H, int JB, int most, bool clocks) {
     const int PW = (H + 63) / 64;
     if (JB == 8) {
         switch (PW) {
-            case 2: return local_pair<2, 8>(fwd, nsq, clocks);
-            case 3: return local_pair<3, 8>(fwd, nsq, clocks);
-            case 4: return local_pair<4, 8>(fwd, nsq, clocks);
+            case 2: return local_pair<2, 8>(fwd, most, clocks);
+            case 3: return local_pair<3, 8>(fwd, most, clocks);
+            case 4: return local_pair<4, 8>(fwd, most, clocks);
         }
     }
     if (JB == 16) {
         switch (PW) {
-            case 3: return local_pair<3, 16, 4>(fwd, clocks);
-            case 4: return local_pair<4, 16, 4>(fwd, clocks);
-            case 5: return local_pair<5, 16>(fwd, nsq, clocks);
-            case 6: return local_pair<6, 16>(fwd, nsq, clocks);
-            case 7: return local_pair<7, 16>(fwd, nsq, clocks);
-            case 8: return local_pair<8, 16>(fwd, nsq, clocks);
+            case 3: return local_pair<3, 16, kLocalSeqs>(fwd, clocks);  // (layers of up to 256 cells come here with more than eight jobs)
+            case 4: return local_pair<4, 16, kLocalSeqs>(fwd, clocks);
+            case 5: return local_pair<5, 16>(fwd, most, clocks);
+            case 6: return local_pair<6, 16>(fwd, most, clocks);
+            case 7: return local_pair<7, 16>(fwd, most, clocks);
+            case 8: return local_pair<8, 16>(fwd, most, clocks);
         }
     }
     return nullptr;
@@ -600,7 +603,7 @@ int launch_chain(cnt_lstm *h, hipStream_t stream, bool fwd, ChainParams &p) {
         CNT_HIP(hipGetLastError());
         return CNT_OK;
     }
-    chain_kernel_t k = pick_local_kernel(fwd, h->H, h->local_jb, h->local_nsq, h->clocks != nullptr);
+    chain_kernel_t k = pick_local_kernel(fwd, h->H, h->local_jb, h->local_most, h->clocks != nullptr);
     CNT_REQUIRE(k != nullptr, "lstm: no recursion kernel for H=%d JB=%d", h->H, h->local_jb);
     // heals the handle after a launch that gave up, zeroes the placement counters; in front of the backward recursion it
     // can be part of the cache-warming launch
@@ -644,7 +647,7 @@ int launch_chain(cnt_lstm *h, hipStream_t stream, bool fwd, ChainParams &p) {
         p.job0 = (unsigned)job0;
         p.njobs = std::min(h->launch_jobs, h->njobs - job0);
         CNT_TRY(launch_in_order(h, stream, [&] {
-            hipLaunchKernelGGL(k, dim3(local_blocks(h)), dim3(local_threads((h->H + 63) / 64, h->local_jb, h->local_nsq)), (size_t)h->spread_lds, stream, p);
+            hipLaunchKernelGGL(k, dim3(local_blocks(h)), dim3(local_threads((h->H + 63) / 64, h->local_jb, h->local_most)), (size_t)h->spread_lds, stream, p);
         }));
     }
     return CNT_OK;
@@ -658,8 +661,8 @@ void local_placement(cnt_lstm *h, int lds_per_cu, int cus_per_xcd) {
     int most = kLocalSlots;
     for (int fwd = 0; fwd < 2; ++fwd) {
         int fit = 0;
-        const void *k = reinterpret_cast<const void *>(pick_local_kernel(fwd != 0, h->H, h->local_jb, h->local_nsq, h->clocks != nullptr));
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k, local_threads((h->H + 63) / 64, h->local_jb, h->local_nsq), 0) != hipSuccess) {
+        const void *k = reinterpret_cast<const void *>(pick_local_kernel(fwd != 0, h->H, h->local_jb, h->local_most, h->clocks != nullptr));
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k, local_threads((h->H + 63) / 64, h->local_jb, h->local_most), 0) != hipSuccess) {
             (void)hipGetLastError();
             fit = 1;
         }
@@ -770,12 +773,22 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     if (const char *e = std::getenv("CNT_LSTM_SOLO")) solo_cells = std::min(std::atoi(e), kSoloCells);
     // (the one-workgroup kernels address their arrays by 31-bit byte offsets)
     const bool solo = H <= solo_cells && (size_t)desc->L * desc->maxT * desc->S < ((size_t)1 << 29) - 16;
-    // jobs of one direction and at most four sequences, spread over the XCDs while there are fewer jobs than XCDs (the
-    // one-workgroup kernels gain nothing from smaller jobs)
-    const int groups = std::max((desc->S + kLocalSeqs - 1) / kLocalSeqs, solo ? 1 : std::min(kLocalXcds / ndir, desc->S));
-    const int local_jb = local_cells(H, ndir * groups);
-    const int local_nsq = local_sequences(H, local_jb, (desc->S + groups - 1) / groups);
-    const bool stepwise = (!solo && pick_local_kernel(true, H, local_jb, local_nsq, false) == nullptr) || std::getenv("CNT_LSTM_STEPWISE") != nullptr;
+    int per_cu = 0, cus = 0;  // LDS of a compute unit, compute units
+    {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&per_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+            (void)hipGetLastError();
+            per_cu = cus = 0;
+        }
+    }
+    // jobs of one direction and at most four sequences (the one-workgroup kernels gain nothing from smaller jobs)
+    const int least = (desc->S + kLocalSeqs - 1) / kLocalSeqs;
+    const int local_jb = local_cells(H, ndir * least);
+    const int groups = solo ? least : local_groups(H, local_jb, desc->S, ndir, cus / kLocalXcds);
+    const int local_most = groups >= desc->S ? 1 : kLocalSeqs;
+    const bool stepwise = (!solo && pick_local_kernel(true, H, local_jb, local_most, false) == nullptr) || std::getenv("CNT_LSTM_STEPWISE") != nullptr;
 
     cnt_lstm *h = new (std::nothrow) cnt_lstm();
     CNT_REQUIRE(h != nullptr, "lstm_create: out of host memory");
@@ -785,7 +798,7 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     h->solo = solo && !stepwise ? 1 : 0;
     h->local = !solo && !stepwise ? 1 : 0;
     h->local_jb = local_jb;
-    h->local_nsq = local_nsq;
+    h->local_most = local_most;
     h->bmail_dirty = 1;
     h->flmail_dirty = 1;
     h->spin_limit = 1u << 22;
@@ -800,16 +813,6 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     if (const char *e = std::getenv("CNT_LSTM_SKIP_PADDING")) h->make_order = std::atoi(e) != 0;
     h->warm = 0;
     if (const char *e = std::getenv("CNT_LSTM_WARM")) h->warm = std::atoi(e) != 0;
-    int per_cu = 0, cus = 0;  // LDS of a compute unit, compute units
-    {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&per_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-            (void)hipGetLastError();
-            per_cu = cus = 0;
-        }
-    }
     if (const char *e = std::getenv("CNT_LSTM_POLL_DELAY")) h->poll_delay_local = std::atoi(e);
     h->poll_delay_fwd_local = kForwardPause;
     h->mem_delay_fwd_local = kLoadPause;
@@ -827,7 +830,7 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     h->njobs = ndir * groups;
     if (h->local) {
         h->team = (H + h->local_jb - 1) / h->local_jb;
-        h->lmail_words = h->flmail_words = (size_t)h->njobs * local_job_words(h->team, h->local_jb, h->local_nsq);
+        h->lmail_words = h->flmail_words = (size_t)h->njobs * local_job_words(h->team, h->local_jb, h->local_most);
         if (err == hipSuccess && std::getenv("CNT_LSTM_TIMING")) {
             err = hipMalloc(reinterpret_cast<void **>(&h->clocks), 2 * kClockWords * sizeof(long long));
             if (err == hipSuccess) err = hipMemset(h->clocks, 0, 2 * kClockWords * sizeof(long long));

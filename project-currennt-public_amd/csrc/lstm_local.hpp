@@ -17,8 +17,8 @@
 // waited for -- with 19-workgroup teams, one workgroup per compute unit and a second team left half resident, the
 // remaining workgroups were never dispatched and the launch gave up.
 //
-// A job moves and multiplies NSQ sequences (1, 2 or 4: the smallest that holds the launch's largest job), so a fraction of one
-// or two sequences per job exchanges a quarter or half of the words.
+// A job moves and multiplies NSQ sequences (1, 2 or 4: the smallest that holds its own), so one of one or two sequences
+// exchanges a quarter or half of the words.  Which sequences share a job, and which steps it leaves out: local_setup.
 //
 // Per workgroup (cells j0 .. j0+JB-1 of the job's direction, all T steps): the recurrent weights that read this
 // workgroup's gate deltas, W[h][k] for every cell h of the direction and k = (own cell, gate), live in registers
@@ -72,13 +72,13 @@ struct LocalShape {
 constexpr int local_threads(int PW, int JB, int NSQ) { return (PW + (JB * NSQ + 15) / 16 + 2) * 64; }
 constexpr size_t local_job_words(int G, int JB, int NSQ) { return (size_t)kMailSlots * G * G * NSQ * JB; }
 
-// Job -> direction and sequences: the sequences are dealt to the groups as evenly as possible, in order.
-struct LocalJob { int dir, seq0, nseq; };
-__device__ __forceinline__ LocalJob local_job(const ChainParams &p, int job) {
-    const int dir = job / p.groups, q = job % p.groups;
-    const int each = p.S / p.groups, more = p.S % p.groups;
-    return LocalJob{dir, q * each + min(q, more), each + (q < more ? 1 : 0)};
-}
+// What a job does: its direction, its sequences (order[0 .. nseq)), and the launch's steps that it has to take,
+// [begin, end) -- on the others all its sequences are padding (fill_padding).
+struct LocalJob {
+    int dir, nseq;
+    const int *order;
+    int first, last, begin, end;  // first and last: of the pass, which may lie outside the launch's range
+};
 
 // The placement counters carry nothing but their own values (everything else a workgroup reads was written by earlier
 // launches), so every access to them is a relaxed device-scope atomic: acquire or release at that scope would write
@@ -129,6 +129,144 @@ __device__ int local_claim_role(const ChainParams &p, int G) {
     return (int)((p.job0 + job - 1u) * 64u + member);
 }
 
+// How the sequences of a direction are dealt to its groups.  A recursion lasts as long as its longest job, and a step of a job is
+// shorter the fewer sequences it has (kStepCost), so the longest sequences get jobs of their own and the shortest ones share:
+// sorted by length, cut so that the largest product of a job's longest sequence and its step is smallest (greedily for a
+// bound, the bound by bisection).  A job then leaves out the steps on which all of its sequences are padding.  The lengths come
+// from the pattern types, so every launch of a pass, and every workgroup of a launch, finds the same cut.  The acoustic model's
+// pass (ten sequences of 300 to 600 steps, two layers of 256 cells in two directions) 2930 us dealt evenly and in order, 2750 so;
+// 150 and 200 cells with twenty sequences of 211 to 500 steps 2455 and 2305.
+// Step of a job of 1 to 4 sequences, of 128 (us per step, forward / backward, 256 cells: 0.867 / 0.777, 0.910 / 0.838, 0.987 / 0.869,
+// 0.999 / 0.873; other sizes in about the same proportions).
+template <bool FWD>
+__device__ __forceinline__ int step_cost(int sequences) {
+    constexpr int cost[5] = {0, FWD ? 111 : 114, FWD ? 117 : 123, FWD ? 126 : 127, 128};
+    return cost[sequences];
+}
+constexpr int kPlannedSeqs = 64;  // more parallel sequences are dealt evenly and in order, and take every step
+struct LocalPlan {
+    int role;
+    int length[kPlannedSeqs];  // steps until the last one that is no padding; then the same, longest first
+    int order[kPlannedSeqs];
+    int start[kPlannedSeqs + 1];  // first position in `order` of every group
+};
+
+// Called by all threads; wave 0 claims the role while the others look at the pattern types.
+template <int MOST, bool FWD>
+__device__ __forceinline__ LocalJob local_setup(const ChainParams &p, LocalPlan &plan, int &job, int &me) {
+    const int tid = threadIdx.x, lane = tid & 63, S = p.S, T = p.T, Tmin = min(p.Tmin, T);
+    const bool planned = S <= kPlannedSeqs;
+    if (tid < kPlannedSeqs) plan.length[tid] = Tmin;
+    __syncthreads();
+    if (tid == 0) {
+        plan.role = local_claim_role(p, p.team);
+    } else if (tid >= 64 && planned && Tmin < T) {
+        const int threads = blockDim.x - 64, rows = threads / S, s = (tid - 64) % S, row = (tid - 64) / S;
+        if (row < rows) {
+            int length = 0;
+#pragma unroll 4
+            for (int t = Tmin + row; t < T; t += rows) length = p.pat[(size_t)t * S + s] != 0 ? t + 1 : length;
+            atomicMax(&plan.length[s], length);
+        }
+    }
+    __syncthreads();
+    LocalJob part = {0, 0, plan.order, 0, 0, 0, 0};
+    if (plan.role < 0) return part;
+    const int role = __builtin_amdgcn_readfirstlane(plan.role);
+    job = role >> 6; me = role & 63;
+    part.dir = job / p.groups;
+    const int group = job % p.groups;
+    int longest = T;
+    if (!planned) {
+        const int each = S / p.groups, more = S % p.groups;
+        part.nseq = each + (group < more ? 1 : 0);
+        // (jobs of more than kPlannedSeqs sequences in all still hold at most MOST each)
+        if (tid < part.nseq) plan.order[tid] = group * each + min(group, more) + tid;
+    } else {
+        if (tid < 64) {
+            const int mine = lane < S ? plan.length[lane] : -1;
+            int rank = 0;
+            for (int s = 0; s < S; ++s) {
+                const int other = __builtin_amdgcn_readlane(mine, s);
+                rank += other > mine || (other == mine && s < lane) ? 1 : 0;
+            }
+            if (lane < S) { plan.order[rank] = lane; plan.length[rank] = mine; }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const int sorted = lane < S ? plan.length[lane] : 0;
+            auto most_within = [&](int bound) {  // sequences of a job that starts with this lane's
+                int n = 0;
+#pragma unroll
+                for (int q = 1; q <= MOST; ++q) n = sorted * step_cost<FWD>(q) <= bound ? q : n;
+                return n;
+            };
+            auto cut = [&](int bound, bool keep) {
+                const int n = most_within(bound);
+                int at = 0, g = 0;
+                for (; at < S && g < p.groups; ++g) {
+                    const int take = __builtin_amdgcn_readlane(n, at);
+                    if (take == 0) break;
+                    if (keep && lane == 0) plan.start[g] = at;
+                    at = min(at + take, S);
+                }
+                if (keep)
+                    for (; g <= p.groups; ++g)
+                        if (lane == 0) plan.start[g] = S;
+                return at >= S;
+            };
+            const int top = __builtin_amdgcn_readlane(sorted, 0);
+            int low = top * step_cost<FWD>(1) - 1, high = top * step_cost<FWD>(MOST);  // `high` always suffices
+            // (four in every job: nothing to choose)
+            for (int q = 0; q < 10 && high - low > 1 && p.groups * MOST > S; ++q) {
+                const int mid = (low + high) / 2;
+                if (cut(mid, false)) high = mid;
+                else low = mid;
+            }
+            cut(high, true);
+        }
+        __syncthreads();
+        const int from = __builtin_amdgcn_readfirstlane(plan.start[group]);
+        part.nseq = __builtin_amdgcn_readfirstlane(plan.start[group + 1]) - from;
+        part.order = plan.order + from;
+        longest = part.nseq > 0 ? max(__builtin_amdgcn_readfirstlane(plan.length[from]), 1) : 0;
+    }
+    __syncthreads();
+    // Steps of the pass: those on which a sequence is no padding, and where time runs forward one more, the first slot behind the
+    // sequences, which still sees what the last one hands on.
+    const bool forward_in_time = FWD ? part.dir == 0 : part.dir != 0;
+    part.first = forward_in_time ? 0 : T - longest;
+    part.last = (forward_in_time ? min(T, longest + 1) : T) - 1;
+    part.begin = max(part.first, p.step_begin);
+    part.end = min(part.last + 1, p.step_end);
+    return part;
+}
+
+// The launch's steps that the job leaves out: what a padding slot gets there.  me = the workgroup's place in its team.
+template <int JB, bool FWD>
+__device__ __forceinline__ void fill_padding(const ChainParams &p, const LocalJob &part, int me) {
+    const DirPtrs &D = p.d[part.dir];
+    const int H = p.H, S = p.S, j0 = me * JB, per_step = part.nseq * JB;
+    // before the job's steps or behind them
+    const int b0 = p.step_begin, e0 = min(p.step_end, max(part.begin, b0)), b1 = max(part.end, e0), e1 = max(p.step_end, b1);
+    const int before = e0 - b0, count = (before + (e1 - b1)) * per_step;
+    const bool forward_in_time = FWD ? part.dir == 0 : part.dir != 0;
+    for (int i = threadIdx.x; i < count; i += blockDim.x) {
+        const int q = i / per_step, r = i % per_step, c = j0 + r % JB;
+        if (c >= H) continue;
+        const int step = q < before ? b0 + q : b1 + q - before, t = forward_in_time ? step : p.T - 1 - step;
+        const size_t slot = (size_t)t * S + part.order[r / JB], gi = slot * H + c, oi = slot * p.L + part.dir * H + c;
+        if (FWD) {
+            if (part.dir) D.c[gi] = 0.0f;
+            D.h[gi] = 0.0f;
+            if (p.out) p.out[oi] = 0.0f;
+        } else {
+            D.dni[gi] = 0.0f; D.dig[gi] = 0.0f; D.dfg[gi] = 0.0f; D.dog[gi] = 0.0f; D.cerr[gi] = 0.0f;
+            // (a layer of one direction keeps the summed errors where the output errors stand: nothing is added here)
+            if (!p.herr_out) D.herr[gi] = p.outerr[oi];
+        }
+    }
+}
+
 // v + (v rotated by N lanes within its row of sixteen).  Rotations by 8, 4, ... in this order add up what the lanes of a row
 // that are N apart hold, with the same rounding in every one of them (each pair adds the same two values).
 template <int N>
@@ -175,12 +313,12 @@ __device__ __forceinline__ f32x4 local_product(const f32x4 &a, const float (&wre
 }
 
 // Diagnostic clocks (CNT_LSTM_TIMING, CNT_LSTM_TRACE): every kernel of the two recursions exists a second time, with CLOCKS, in
-// which the workgroups add up what their waves spend in the parts of a step and, for some steps in the middle, note when
+// which the workgroups add up what their waves spend in the parts of a step and, for some steps of the job, counted from its first, note when
 // they pass five points of it, on the 100 MHz clock that all compute units share.  The kernels without are free of all of
 // it: a branch on the chain of a step costs some of what it would measure.
 constexpr unsigned kClockBlocks = 512;  // workgroups that record
 enum { CLK_WAIT, CLK_REST, CLK_BARRIER, CLK_LOOP, CLK_ROUNDS, CLK_LOAD, CLK_STORE, CLK_OTHER, kClockCounts };
-constexpr int kTraceFirst = 100, kTraceSteps = 4, kTracePoints = 5, kTraceWords = 4 + kTraceSteps * kTracePoints;
+constexpr int kTraceFirst = 64, kTraceSteps = 4, kTracePoints = 5, kTraceWords = 4 + kTraceSteps * kTracePoints;
 constexpr size_t kClockWords = (size_t)kClockBlocks * (kClockCounts + kTraceWords);  // of one direction of time
 template <bool CLOCKS>
 __device__ __forceinline__ long long clock_now() {
@@ -220,9 +358,25 @@ __device__ __forceinline__ void clock_where(const ChainParams &p, int job, int m
         }
 }
 
-// PW = ceil(cells per direction / 64) product waves, JB cells per workgroup, NSQ sequences per job
+// LDS of a job
+template <int JB, int NSQ>
+struct BackwardShared {
+    using Shape = LocalShape<JB, NSQ>;
+    static constexpr int EL = Shape::EL, RING = 2 * Shape::BATCH;
+    static constexpr int DP = 4 * JB + 16;  // pitch of a sequence's deltas: the four sequences' rows on different banks
+    __attribute__((aligned(16))) float dl[2][NSQ][DP];      // [sequence][cell][gate]
+    // element = cell * NSQ + sequence, as in the messages
+    __attribute__((aligned(16))) float coef[RING][EL][4];      // of e in d_og and in the cell error, stored d_og, e
+    __attribute__((aligned(16))) float coef_own[RING][EL][4];  // of the cell error in d_ni, d_ig, d_fg
+    __attribute__((aligned(16))) float coef_fg[RING][EL][2];   // forget gate activation, 1: padding slot
+    __attribute__((aligned(16))) float res[2][EL][2];       // summed output error, cell error
+    int wait_failed;
+};
+
+// One job by one workgroup of its team.  PW = ceil(cells per direction / 64) product waves, JB cells per workgroup, a job of up to
+// NSQ sequences
 template <int PW, int JB, int NSQ, bool CLOCKS>
-__global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_local(const ChainParams p) {
+__device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJob &part, int job, int me, unsigned mail_words, BackwardShared<JB, NSQ> &sh) {
     using Shape = LocalShape<JB, NSQ>;
     const int H = p.H, G = p.team;    // G = ceil(H / JB) workgroups; the last one may own fewer than JB cells
     constexpr int EL = Shape::EL, VEC = Shape::VEC, VPW = Shape::VPW, CW = Shape::CW;
@@ -231,59 +385,51 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
     constexpr int SPW = 64 / VPW;     // senders side by side in a polling wave
     constexpr int NL = (TEAM + SPW - 1) / SPW;  // 16-byte loads per polling lane; the last one may lie past the last sender
     constexpr int KW = 4 * JB;        // k extent of the product: (own cell, gate)
-    constexpr int DP = KW + 16;       // pitch of a sequence's deltas in LDS: the four sequences' rows on different banks
+    constexpr int DP = BackwardShared<JB, NSQ>::DP;
     constexpr int NQ = (TEAM * VEC + 63) / 64;  // vectors per lane that hand a step's words back
     const unsigned RECV = (unsigned)(G * EL);   // words one receiver gets per step
-
-    __shared__ __attribute__((aligned(16))) float dl[2][NSQ][DP];      // [sequence][cell][gate]
-    // element = cell * NSQ + sequence, as in the messages
-    __shared__ __attribute__((aligned(16))) float coef[RING][EL][4];      // of e in d_og and in the cell error, stored d_og, e
-    __shared__ __attribute__((aligned(16))) float coef_own[RING][EL][4];  // of the cell error in d_ni, d_ig, d_fg
-    __shared__ __attribute__((aligned(16))) float coef_fg[RING][EL][2];   // forget gate activation, 1: padding slot
-    __shared__ __attribute__((aligned(16))) float res[2][EL][2];       // summed output error, cell error
-    __shared__ int wait_failed;
-    __shared__ int role_sh;
+    auto &dl = sh.dl;
+    auto &coef = sh.coef;
+    auto &coef_own = sh.coef_own;
+    auto &coef_fg = sh.coef_fg;
+    auto &res = sh.res;
+    int &wait_failed = sh.wait_failed;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) {
-        wait_failed = 0;
-        role_sh = local_claim_role(p, G);
-    }
-    __syncthreads();
-    const int role = role_sh;
-    if (role < 0) return;
-    const int job = role >> 6, me = role & 63;
-    const LocalJob part = local_job(p, job);
-    const int dir = part.dir, seq0 = part.seq0, nseq = part.nseq;
+    if (wave >= PW + CW + 2) return;  // (of a launch whose largest jobs need more waves)
+    const int nseq = part.nseq, begin_step = part.begin, end_step = part.end;
+    int dir = part.dir;
+    asm volatile("" : "+s"(dir));  // the direction's pointers are read here, not in front of the choice of the kernel's three jobs
     const DirPtrs &D = p.d[dir];
     const int S = p.S, T = p.T;
     const int j0 = me * JB;
     const int n = S * H;
-    float *const mailbox = p.lmail + (size_t)job * local_job_words(G, JB, NSQ);
+    float *const mailbox = p.lmail + (size_t)job * mail_words;
     const unsigned slot_words = (unsigned)G * RECV;
     const __amdgpu_buffer_rsrc_t mail =
         __builtin_amdgcn_make_buffer_rsrc(mailbox, 0, (int)(local_job_words(G, JB, NSQ) * sizeof(float)), 0x00020000);
+    const int last_step = part.last;  // of the pass: its partial errors go nowhere
     auto slot_of = [&](int step) { return dir ? step : (T - 1 - step); };
     // read through the LDS address space: a volatile read through a generic pointer becomes a flat load, which takes the
     // vector-memory path
     auto given_up = [&]() { return *(__attribute__((address_space(3))) volatile int *)&wait_failed; };
 
     // the load and the store wave: lane = (step of an access, sequence, cell)
-    const int ej = lane % EL / JB, ec = lane % JB;  // sequence seq0 + ej, cell j0 + ec
+    const int ej = lane % EL / JB, ec = lane % JB;  // the job's sequence ej, cell j0 + ec
     const bool valid = ej < nseq && j0 + ec < H;
     const int ahead = lane / EL;
 
     if (wave == PW + CW) {
         // ------------------------------------------------------------------ load wave
         struct StepIn { float e, ni, ig, fg, og, dog_old, c, c_earlier; char pat; };
-        const int s = seq0 + ej, el = ec * NSQ + ej;
+        const int s = part.order[min(ej, nseq - 1)], el = ec * NSQ + ej;
         auto load_batch = [&](int first, StepIn (&in)[SETS]) {
 #pragma unroll
             for (int i = 0; i < SETS; ++i) {
                 StepIn &v = in[i];
                 v = StepIn{0, 0, 0, 0, 0, 0, 0, 0, 1};
                 const int step = first + i * STEPS + ahead;
-                if (!valid || step >= T) continue;
+                if (!valid || step >= end_step) continue;
                 const int t = slot_of(step);
                 const size_t gi = (size_t)t * n + (size_t)s * H + j0 + ec;
                 v.e = p.outerr[((size_t)t * S + s) * p.L + dir * H + j0 + ec];
@@ -299,8 +445,8 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
             for (int i = 0; i < SETS; ++i) {
                 const StepIn &x = in[i];
                 const int step = first + i * STEPS + ahead;
-                if (step >= T) continue;
-                const int t = slot_of(step), b = (step - p.step_begin) % RING;
+                if (step >= end_step) continue;
+                const int t = slot_of(step), b = (int)((unsigned)(step - begin_step) % RING);
                 const float tc = tanh_act(x.c);
                 // d_og = first * e + stored d_og, cell error = second * e + ...
                 *reinterpret_cast<f32x4 *>(coef[b][el]) = f32x4{logistic_deriv(x.og) * tc, x.og * tanh_deriv(tc), x.dog_old, x.e};
@@ -311,17 +457,17 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
             }
         };
         StepIn in[SETS];
-        const int sb = p.step_begin;
+        const int sb = begin_step;
         load_batch(sb, in);
         wait_all_vmem();
         put_batch(sb, in);
         long long busy = 0;
         lds_barrier();  // start of the recursion
-        for (int step = sb; step < p.step_end; ++step) {
+        for (int step = sb; step < end_step; ++step) {
             lds_barrier();
             if (given_up()) return;
             const long long since = clock_now<CLOCKS>();
-            const int phase = (step - sb) % BATCH, next = step - phase + BATCH;
+            const int phase = (int)((unsigned)(step - sb) % BATCH), next = step - phase + BATCH;
             if (phase == 0) {
                 load_batch(next, in);
             } else if (phase == BATCH / 2) {
@@ -336,13 +482,13 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
 
     if (wave == PW + CW + 1) {
         // ------------------------------------------------------------------ store wave
-        const int s = seq0 + ej, el = ec * NSQ + ej;
+        const int s = part.order[min(ej, nseq - 1)], el = ec * NSQ + ej;
         f32x4 d = {0, 0, 0, 0};
         float e = 0, ce = 0;
         long long busy = 0;
         lds_barrier();  // start of the recursion
-        for (int step = p.step_begin; step < p.step_end; ++step) {
-            const int b = step & 1, held = (step - p.step_begin) % STEPS;
+        for (int step = begin_step; step < end_step; ++step) {
+            const int b = step & 1, held = (int)((unsigned)(step - begin_step) % STEPS);
             lds_barrier();  // results of this step are in LDS
             if (given_up()) return;
             const long long since = clock_now<CLOCKS>();
@@ -352,7 +498,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
             }
             for (int i = 0; i < p.mem_delay; ++i) __builtin_amdgcn_s_sleep(1);
             wait_all_vmem();  // the stores of the step before are done
-            if ((held == STEPS - 1 || step == p.step_end - 1) && valid && ahead <= held) {
+            if ((held == STEPS - 1 || step == end_step - 1) && valid && ahead <= held) {
                 // an access stores as many steps as it has lanes for
                 const size_t gi = (size_t)slot_of(step - held + ahead) * n + (size_t)s * H + j0 + ec;
                 D.dni[gi] = d[0]; D.dig[gi] = d[1]; D.dfg[gi] = d[2]; D.dog[gi] = d[3];
@@ -360,7 +506,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
                 if (p.herr_out) p.herr_out[gi] = e;
                 else D.herr[gi] = e;
             }
-            if (step > 0) {
+            if (step > part.first) {
                 // The words the cell waves consumed in this step (before the barrier) are empty again.  The slot is used
                 // again three steps from now, so this hand-back can wait for this wave's turn instead of sitting in
                 // front of the next poll in the compute unit's queue.
@@ -368,7 +514,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
 #pragma unroll
                 for (int q = 0; q < NQ; ++q)
                     if (q * 64 + lane < G * VEC)
-                        __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)((step - 1) % kMailSlots) * slot_words * 4u +
+                        __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)(step - 1) % kMailSlots * slot_words * 4u +
                                                                ((unsigned)me * RECV + (unsigned)(q * 64 + lane) * 4u) * 4u), 0, 0);
             }
             clock_add<CLOCKS>(busy, since);
@@ -393,24 +539,24 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
         long long busy = 0;
         wait_all_vmem();
         lds_barrier();  // start of the recursion
-        for (int step = p.step_begin; step < p.step_end; ++step) {
+        for (int step = begin_step; step < end_step; ++step) {
             lds_barrier();  // the deltas of this step are in LDS
             const long long since = clock_now<CLOCKS>();
-            if (tid == 0) clock_point<CLOCKS>(p, step, 3);
+            if (tid == 0) clock_point<CLOCKS>(p, step - begin_step, 3);
             // looked at only at the end of the step: the read is in flight behind the barrier together with the
             // deltas', and what a failed step publishes no longer matters
             const f32x4 a = *reinterpret_cast<const f32x4 *>(mine + (step & 1) * NSQ * DP);
             const int failed = given_up();
             // everything this wave stored in the previous step has reached the L2 before it publishes again
             wait_all_vmem();
-            if (step < T - 1) {
+            if (step < last_step) {
                 const f32x4 sum = local_product<JB == 8 ? 3 : 4, KW>(a, wreg, std::make_integer_sequence<int, JB>{});
                 const u32x4 v = {publishable(sum[0]), publishable(sum[1]), publishable(sum[2]), publishable(sum[3])};
                 if (publishes)
-                    mail_store(v, mail, (unsigned)(step % kMailSlots) * slot_words * 4u + pub_off, std::integral_constant<int, NSQ>{});
+                    mail_store(v, mail, (unsigned)step % kMailSlots * slot_words * 4u + pub_off, std::integral_constant<int, NSQ>{});
             }
             clock_add<CLOCKS>(busy, since);
-            if (tid == 0) clock_point<CLOCKS>(p, step, 4);
+            if (tid == 0) clock_point<CLOCKS>(p, step - begin_step, 4);
             if (failed) return;
         }
         if (tid == 0) clock_store<CLOCKS>(p, CLK_OTHER, busy);
@@ -437,9 +583,9 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
     }
     const bool peeps = gate == 1 || gate == 2;
     float fg_later = 0, cerr_later = 0, own_later = 0;
-    if (p.step_begin > 0 && real_cell && cj < nseq) {
+    if (begin_step > part.first && real_cell && cj < nseq) {
         // a launch that starts in the middle: what the step before carried over stands in the state arrays
-        const size_t gi = (size_t)slot_of(p.step_begin - 1) * n + (size_t)(seq0 + cj) * H + j0 + cc;
+        const size_t gi = (size_t)slot_of(begin_step - 1) * n + (size_t)part.order[cj] * H + j0 + cc;
         fg_later = D.fg[gi]; cerr_later = D.cerr[gi];
         if (peeps) own_later = gate == 1 ? D.dig[gi] : D.dfg[gi];
     }
@@ -449,11 +595,11 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
     lds_barrier();    // start of the recursion: coefficients of steps 0 and 1 are in LDS
     const long long begin = clock_now<CLOCKS>();
 
-    for (int step = p.step_begin; step < p.step_end; ++step) {
-        const bool first = (step == 0), last = (step == T - 1);
-        const int b = step & 1, r = (step - p.step_begin) % RING;
+    for (int step = begin_step; step < end_step; ++step) {
+        const bool first = (step == part.first), last = (step == T - 1);
+        const int b = step & 1, r = (int)((unsigned)(step - begin_step) % RING);
         const long long since = clock_now<CLOCKS>();
-        if (records) clock_point<CLOCKS>(p, step, 0);
+        if (records) clock_point<CLOCKS>(p, step - begin_step, 0);
         // this step's coefficients: in LDS since before the previous barrier, fetched while the poll is in flight
         const f32x4 k = *reinterpret_cast<const f32x4 *>(coef[r][el]);
         const float k_own = coef_own[r][el][gate], fg = coef_fg[r][el][0], dummy = coef_fg[r][el][1];
@@ -466,7 +612,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
 
         bool ok = true;
         if (!first) {
-            const float *slot = mailbox + (size_t)((step - 1) % kMailSlots) * slot_words;
+            const float *slot = mailbox + (size_t)((unsigned)(step - 1) % kMailSlots) * slot_words;
             u32x4 w[NL];
             unsigned spins = 0;
             for (int d = 0; d < p.poll_delay; ++d) __builtin_amdgcn_s_sleep(1);
@@ -486,7 +632,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
                 for (int d = 0; d < p.poll_gap; ++d) __builtin_amdgcn_s_sleep(1);
             }
             clock_add<CLOCKS>(waited, since);
-            if (records) clock_point<CLOCKS>(p, step, 1);
+            if (records) clock_point<CLOCKS>(p, step - begin_step, 1);
             f32x4 sum = __builtin_bit_cast(f32x4, w[NL - 1]);
 #pragma unroll
             for (int r = 0; r < 4; ++r) sum[r] = last_counts ? sum[r] : 0.0f;
@@ -510,7 +656,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
             wait_failed = 1;
             if (lane == 0) raise_abort(p);
         }
-        if (records) clock_point<CLOCKS>(p, step, 2);
+        if (records) clock_point<CLOCKS>(p, step - begin_step, 2);
         const long long at_barrier = clock_now<CLOCKS>();
         lds_barrier();
         clock_add<CLOCKS>(barrier, at_barrier);
@@ -525,4 +671,20 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_backward_loca
         clock_store<CLOCKS>(p, CLK_LOOP, clock_now<CLOCKS>() - begin);
         clock_where<CLOCKS>(p, job, me);
     }
+}
+
+template <int PW, int JB, int MOST, bool CLOCKS>
+__global__ __launch_bounds__(local_threads(PW, JB, MOST)) void lstm_backward_local(const ChainParams p) {
+    __shared__ LocalPlan plan;
+    __shared__ union Shared { BackwardShared<JB, 1> one; BackwardShared<JB, MOST < 2 ? 1 : 2> two; BackwardShared<JB, MOST> most; } sh;
+    int job = 0, me = 0;
+    const LocalJob part = local_setup<MOST, false>(p, plan, job, me);
+    if (part.nseq == 0) return;
+    fill_padding<JB, false>(p, part, me);
+    if (part.begin >= part.end) return;
+    const unsigned mail_words = (unsigned)local_job_words(p.team, JB, MOST);
+    if (threadIdx.x == 0) (part.nseq == 1 ? sh.one.wait_failed : part.nseq == 2 ? sh.two.wait_failed : sh.most.wait_failed) = 0;
+    if (MOST == 1 || part.nseq == 1) backward_job<PW, JB, 1, CLOCKS>(p, part, job, me, mail_words, sh.one);
+    else if (part.nseq == 2) backward_job<PW, JB, MOST < 2 ? 1 : 2, CLOCKS>(p, part, job, me, mail_words, sh.two);
+    else backward_job<PW, JB, MOST, CLOCKS>(p, part, job, me, mail_words, sh.most);
 }

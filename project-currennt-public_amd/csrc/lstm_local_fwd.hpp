@@ -32,9 +32,25 @@
 // Publishing without LDS, by a broadcast inside the row of sixteen lanes, saves a round trip of 0.03 but stores pieces of 16
 // bytes: 1.05 instead of 1.00.
 
-// PW = ceil(cells per direction / 64) gather waves, JB cells per workgroup, NSQ sequences per job
+// LDS of a job
+template <int PW, int JB, int NSQ>
+struct ForwardShared {
+    using Shape = LocalShape<JB, NSQ>;
+    static constexpr int EL = Shape::EL, RING = 2 * Shape::BATCH, ROWS = 4 * JB;
+    // element = (group of four cells * NSQ + sequence) * 4 + cell of the group, as in the messages
+    __attribute__((aligned(16))) float red[2][PW][ROWS][NSQ];  // recurrent sums of the step, one share per gather wave
+    __attribute__((aligned(16))) float pre[RING][EL][4];    // input projections of the step
+    int pre_dummy[RING][EL];
+    __attribute__((aligned(16))) float res_gate[2][EL][4];     // results of the step
+    __attribute__((aligned(16))) float res[2][EL][4];          // cell state, output, not 0: padding slot
+    __attribute__((aligned(16))) float hpub[Shape::CW][Shape::VPW][4];
+    int wait_failed;
+};
+
+// One job by one workgroup of its team.  PW = ceil(cells per direction / 64) gather waves, JB cells per workgroup, a job of up to
+// NSQ sequences
 template <int PW, int JB, int NSQ, bool CLOCKS>
-__global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local(const ChainParams p) {
+__device__ __forceinline__ void forward_job(const ChainParams &p, const LocalJob &part, int job, int me, unsigned mail_words, ForwardShared<PW, JB, NSQ> &sh) {
     using Shape = LocalShape<JB, NSQ>;
     const int H = p.H, G = p.team;       // G = ceil(H / JB) workgroups; the last one may own fewer than JB cells
     constexpr int EL = Shape::EL, VEC = Shape::VEC, VPW = Shape::VPW, CW = Shape::CW;
@@ -45,33 +61,24 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
     constexpr int NQ = (TEAM * VEC + 63) / 64;  // vectors per lane that hand a block back
     const unsigned RECV = (unsigned)(G * EL);   // words of a receiver's block
     const int vectors = G * VEC;                // 16-byte vectors of a receiver's block
-
-    // element = (group of four cells * NSQ + sequence) * 4 + cell of the group, as in the messages
-    __shared__ __attribute__((aligned(16))) float red[2][PW][ROWS][NSQ];  // recurrent sums of the step, one share per gather wave
-    __shared__ __attribute__((aligned(16))) float pre[RING][EL][4];    // input projections of the step
-    __shared__ int pre_dummy[RING][EL];
-    __shared__ __attribute__((aligned(16))) float res_gate[2][EL][4];     // results of the step
-    __shared__ __attribute__((aligned(16))) float res[2][EL][4];          // cell state, output, not 0: padding slot
-    __shared__ __attribute__((aligned(16))) float hpub[CW][VPW][4];
-    __shared__ int wait_failed;
-    __shared__ int role_sh;
+    auto &red = sh.red;
+    auto &pre = sh.pre;
+    auto &pre_dummy = sh.pre_dummy;
+    auto &res_gate = sh.res_gate;
+    auto &res = sh.res;
+    auto &hpub = sh.hpub;
+    int &wait_failed = sh.wait_failed;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) {
-        wait_failed = 0;
-        role_sh = local_claim_role(p, G);
-    }
-    __syncthreads();
-    const int role = role_sh;
-    if (role < 0) return;
-    const int job = role >> 6, me = role & 63;
-    const LocalJob part = local_job(p, job);
-    const int dir = part.dir, seq0 = part.seq0, nseq = part.nseq;
+    if (wave >= PW + CW + 2) return;  // (of a launch whose largest jobs need more waves)
+    const int nseq = part.nseq, begin_step = part.begin, end_step = part.end;
+    int dir = part.dir;
+    asm volatile("" : "+s"(dir));  // the direction's pointers are read here, not in front of the choice of the kernel's three jobs
     const DirPtrs &D = p.d[dir];
     const int S = p.S, T = p.T;
     const int j0 = me * JB;
     const int n = S * H;
-    float *const mailbox = p.flmail + (size_t)job * local_job_words(G, JB, NSQ);
+    float *const mailbox = p.flmail + (size_t)job * mail_words;
     const unsigned slot_words = (unsigned)G * RECV;
     const __amdgpu_buffer_rsrc_t mail =
         __builtin_amdgcn_make_buffer_rsrc(mailbox, 0, (int)(local_job_words(G, JB, NSQ) * sizeof(float)), 0x00020000);
@@ -86,14 +93,14 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
     if (wave == PW + CW) {
         // ------------------------------------------------------------------ load wave
         struct StepIn { float a[4]; char pat; };
-        const int s = seq0 + cs, el = (cj / 4 * NSQ + cs) * 4 + cj % 4;
+        const int s = part.order[min(cs, nseq - 1)], el = (cj / 4 * NSQ + cs) * 4 + cj % 4;
         auto load_batch = [&](int first, StepIn (&in)[SETS]) {
 #pragma unroll
             for (int i = 0; i < SETS; ++i) {
                 StepIn &v = in[i];
                 v = StepIn{{0, 0, 0, 0}, 1};
                 const int step = first + i * STEPS + ahead;
-                if (!valid || step >= T) continue;
+                if (!valid || step >= end_step) continue;
                 const int t = slot_of(step);
                 const size_t gi = (size_t)t * n + (size_t)s * H + j0 + cj;
                 v.a[0] = D.ni[gi]; v.a[1] = D.ig[gi]; v.a[2] = D.fg[gi]; v.a[3] = D.og[gi];
@@ -104,22 +111,22 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
 #pragma unroll
             for (int i = 0; i < SETS; ++i) {
                 const int step = first + i * STEPS + ahead;
-                if (step >= T) continue;
-                *reinterpret_cast<f32x4 *>(pre[step % RING][el]) = f32x4{in[i].a[0], in[i].a[1], in[i].a[2], in[i].a[3]};
-                pre_dummy[step % RING][el] = slot_of(step) >= p.Tmin && in[i].pat == 0 ? 1 : 0;
+                if (step >= end_step) continue;
+                *reinterpret_cast<f32x4 *>(pre[(unsigned)step % RING][el]) = f32x4{in[i].a[0], in[i].a[1], in[i].a[2], in[i].a[3]};
+                pre_dummy[(unsigned)step % RING][el] = slot_of(step) >= p.Tmin && in[i].pat == 0 ? 1 : 0;
             }
         };
         StepIn in[SETS];
-        load_batch(0, in);
+        load_batch(begin_step, in);
         wait_all_vmem();
-        put_batch(0, in);
+        put_batch(begin_step, in);
         long long busy = 0;
         lds_barrier();  // start of the recursion
-        for (int step = 0; step < T; ++step) {
+        for (int step = begin_step; step < end_step; ++step) {
             lds_barrier();
             if (given_up()) return;
             const long long since = clock_now<CLOCKS>();
-            const int phase = step % BATCH, next = step - phase + BATCH;
+            const int phase = (int)((unsigned)(step - begin_step) % BATCH), next = step - phase + BATCH;
             if (phase == 0) {
                 for (int d = 0; d < p.mem_delay_fwd; ++d) __builtin_amdgcn_s_sleep(1);
                 load_batch(next, in);
@@ -135,13 +142,13 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
 
     if (wave == PW + CW + 1) {
         // ------------------------------------------------------------------ store wave
-        const int s = seq0 + cs, el = (cj / 4 * NSQ + cs) * 4 + cj % 4;
+        const int s = part.order[min(cs, nseq - 1)], el = (cj / 4 * NSQ + cs) * 4 + cj % 4;
         f32x4 g = {0, 0, 0, 0}, r = {0, 0, 0, 0};
         long long busy = 0;
         lds_barrier();  // start of the recursion
         lds_barrier();  // the first step's sums
-        for (int step = 0; step < T; ++step) {
-            const int b = step & 1, held = step % STEPS;
+        for (int step = begin_step; step < end_step; ++step) {
+            const int b = step & 1, held = (int)((unsigned)(step - begin_step) % STEPS);
             lds_barrier();  // results of this step are in LDS
             if (given_up()) return;
             const long long since = clock_now<CLOCKS>();
@@ -150,7 +157,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
                 r = *reinterpret_cast<const f32x4 *>(res[b][el]);
             }
             wait_all_vmem();  // the stores of the step before are done
-            if ((held == STEPS - 1 || step == T - 1) && valid && ahead <= held) {
+            if ((held == STEPS - 1 || step == end_step - 1) && valid && ahead <= held) {
                 // An access stores as many steps as it has lanes for.  A padding slot keeps its summed pre-activations, and its
                 // cell state unless the direction is the time-reversed one (the reference clears it there).
                 const int mine = step - held + ahead, t = slot_of(mine);
@@ -163,13 +170,13 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
                 D.h[gi] = r[1];
                 if (p.out) p.out[((size_t)t * S + s) * p.L + dir * H + j0 + cj] = r[1];
             }
-            if (step + 1 < T) {
+            if (step + 1 < end_step) {
                 // the words the gather waves have read for the next step are empty again
                 const u32x4 empty = {kEmpty, kEmpty, kEmpty, kEmpty};
 #pragma unroll
                 for (int q = 0; q < NQ; ++q)
                     if (q * 64 + lane < vectors)
-                        __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)(step % kMailSlots) * slot_words * 4u +
+                        __builtin_amdgcn_raw_buffer_store_b128(empty, mail, (int)((unsigned)step % kMailSlots * slot_words * 4u +
                                                                ((unsigned)me * RECV + (unsigned)(q * 64 + lane) * 4u) * 4u), 0, 0);
             }
             clock_add<CLOCKS>(busy, since);
@@ -214,31 +221,31 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
         const float *const sent = hpub[cw][lane % VPW];
         const float *const my_red = &red[0][0][cell * 4 + gate][seq];
         float c_prev = 0.0f, start = bias;
+        // the first step has no recurrent sums
+        for (int i = 64 * cw + lane; i < PW * ROWS * NSQ; i += 64 * CW) (&red[begin_step & 1][0][0][0])[i] = 0.0f;
         long long busy = 0;
         const bool records = CLOCKS && cw == 0 && lane == 0;
         wait_all_vmem();
         lds_barrier();  // start of the recursion
-        for (int step = 0; step < T; ++step) {
+        for (int step = begin_step; step < end_step; ++step) {
             const int b = step & 1;
             lds_barrier();
             const long long since = clock_now<CLOCKS>();
-            if (records) clock_point<CLOCKS>(p, step, 3);
+            if (records) clock_point<CLOCKS>(p, step - begin_step, 3);
             // (looked at at the end of the step: what a step that failed publishes no longer matters)
             const int failed = given_up();
-            float a = pre[step % RING][el][gate];
-            int padding = pre_dummy[step % RING][el];
-            asm volatile("" : "+v"(padding));  // read here, with the sums: the compiler would read it between the gates and wait there
+            float a = pre[(unsigned)step % RING][el][gate];
+            int padding = pre_dummy[(unsigned)step % RING][el];
+            float share[PW];
+#pragma unroll
+            for (int w = 0; w < PW; ++w) share[w] = my_red[(size_t)(b * PW + w) * ROWS * NSQ];
+#pragma unroll
+            for (int w = 0; w + 1 < PW; w += 2) share[w / 2] = share[w] + share[w + 1];
+            if (PW % 2) share[PW / 2] = share[PW - 1];
+#pragma unroll
+            for (int w = 0; w < (PW + 1) / 2; ++w) a += share[w];
+            asm volatile("" : "+v"(padding));  // read above, with the sums: the compiler would read it between the gates and wait there
             const bool dummy = padding != 0;
-            if (step > 0) {
-                float share[PW];
-#pragma unroll
-                for (int w = 0; w < PW; ++w) share[w] = my_red[(size_t)(b * PW + w) * ROWS * NSQ];
-#pragma unroll
-                for (int w = 0; w + 1 < PW; w += 2) share[w / 2] = share[w] + share[w + 1];
-                if (PW % 2) share[PW / 2] = share[PW - 1];
-#pragma unroll
-                for (int w = 0; w < (PW + 1) / 2; ++w) a += share[w];
-            }
             const float x0 = a + start, v1 = gate_fn(x0);
             float c = of_gate(v1, c0) * of_gate(v1, c1) + c_prev * of_gate(v1, c2);
             // second pass: tanh(c) in the lanes of the cell input, the output gate in its own
@@ -247,7 +254,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
             hval = dummy || !cell_valid ? 0.0f : hval;
             // the publication of the previous step is complete before this step publishes
             wait_all_vmem();
-            if (step + 1 < T) {
+            if (step + 1 < end_step) {
                 // through LDS, so that neighbouring lanes hold what goes into one receiver's block
                 *my_h = __builtin_bit_cast(float, publishable(hval));
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -256,7 +263,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
 #pragma unroll
                 for (int i = 0; i < PUB; ++i)
                     if (first_receiver + 64 / VPW * i < G)
-                        __builtin_amdgcn_raw_buffer_store_b128(v, mail, (int)((unsigned)(step % kMailSlots) * slot_words * 4u + pub_off + (unsigned)i * pub_stride), 0, 0);
+                        __builtin_amdgcn_raw_buffer_store_b128(v, mail, (int)((unsigned)step % kMailSlots * slot_words * 4u + pub_off + (unsigned)i * pub_stride), 0, 0);
             }
             c = dummy ? 0.0f : c;
             if (row < VPW) {
@@ -268,7 +275,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
             c_prev = dummy && !dir ? c_prev : c;
             start = peeps ? bias + c_prev * peep : bias;
             clock_add<CLOCKS>(busy, since);
-            if (records) clock_point<CLOCKS>(p, step, 4);
+            if (records) clock_point<CLOCKS>(p, step - begin_step, 4);
             if (failed) return;
         }
         lds_barrier();  // results of the last step are in LDS
@@ -301,12 +308,12 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
     wait_all_vmem();
     lds_barrier();  // start of the recursion
     const long long begin = clock_now<CLOCKS>();
-    lds_barrier();  // step 0 has nothing to gather
+    lds_barrier();  // the first step has nothing to gather
 
-    for (int step = 1; step < T; ++step) {
+    for (int step = begin_step + 1; step < end_step; ++step) {
         const long long since = clock_now<CLOCKS>();
-        if (records) clock_point<CLOCKS>(p, step, 0);
-        const float *slot = mailbox + (size_t)((step - 1) % kMailSlots) * slot_words;
+        if (records) clock_point<CLOCKS>(p, step - begin_step, 0);
+        const float *slot = mailbox + (size_t)((unsigned)(step - 1) % kMailSlots) * slot_words;
         bool ok = true;
         u32x4 w[1];
         unsigned spins = 0;
@@ -325,7 +332,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
             for (int d = 0; d < p.poll_gap; ++d) __builtin_amdgcn_s_sleep(1);
         }
         clock_add<CLOCKS>(waited, since);
-        if (records) clock_point<CLOCKS>(p, step, 1);
+        if (records) clock_point<CLOCKS>(p, step - begin_step, 1);
         if (!inside) w[0] = u32x4{0, 0, 0, 0};
         f32x4 sum = local_product<JB == 8 ? 3 : 4, 4 * BLOCKS>(__builtin_bit_cast(f32x4, w[0]), wreg, std::make_integer_sequence<int, BLOCKS>{});
         // register = sequence; where the wave's halves meet, the lower one ends up with the first half of the sequences
@@ -342,7 +349,7 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
             out[0] = sum_halves(sum[0], sum[0]);
         }
         if (__builtin_amdgcn_ballot_w64(!ok) != 0) wait_failed = 1;
-        if (records) clock_point<CLOCKS>(p, step, 2);
+        if (records) clock_point<CLOCKS>(p, step - begin_step, 2);
         const long long at_barrier = clock_now<CLOCKS>();
         lds_barrier();
         clock_add<CLOCKS>(barrier, at_barrier);
@@ -361,4 +368,20 @@ __global__ __launch_bounds__(local_threads(PW, JB, NSQ)) void lstm_forward_local
         clock_store<CLOCKS>(p, CLK_LOOP, clock_now<CLOCKS>() - begin);
         clock_where<CLOCKS>(p, job, me);
     }
+}
+
+template <int PW, int JB, int MOST, bool CLOCKS>
+__global__ __launch_bounds__(local_threads(PW, JB, MOST)) void lstm_forward_local(const ChainParams p) {
+    __shared__ LocalPlan plan;
+    __shared__ union Shared { ForwardShared<PW, JB, 1> one; ForwardShared<PW, JB, MOST < 2 ? 1 : 2> two; ForwardShared<PW, JB, MOST> most; } sh;
+    int job = 0, me = 0;
+    const LocalJob part = local_setup<MOST, true>(p, plan, job, me);
+    if (part.nseq == 0) return;
+    fill_padding<JB, true>(p, part, me);
+    if (part.begin >= part.end) return;
+    const unsigned mail_words = (unsigned)local_job_words(p.team, JB, MOST);
+    if (threadIdx.x == 0) (part.nseq == 1 ? sh.one.wait_failed : part.nseq == 2 ? sh.two.wait_failed : sh.most.wait_failed) = 0;
+    if (MOST == 1 || part.nseq == 1) forward_job<PW, JB, 1, CLOCKS>(p, part, job, me, mail_words, sh.one);
+    else if (part.nseq == 2) forward_job<PW, JB, MOST < 2 ? 1 : 2, CLOCKS>(p, part, job, me, mail_words, sh.two);
+    else forward_job<PW, JB, MOST, CLOCKS>(p, part, job, me, mail_words, sh.most);
 }

@@ -24,6 +24,13 @@
 constexpr int kSoloCells = 64;
 constexpr int kSoloAhead = 4;   // even: the step parity of every unrolled step is a constant
 constexpr int solo_threads(int NW) { return (NW + 2) * 64; }
+// The sequences are dealt to the groups as evenly as possible, in order.
+struct SoloJob { int dir, seq0, nseq; };
+__device__ __forceinline__ SoloJob solo_job(const ChainParams &p, int job) {
+    const int dir = job / p.groups, q = job % p.groups;
+    const int each = p.S / p.groups, more = p.S % p.groups;
+    return SoloJob{dir, q * each + min(q, more), each + (q < more ? 1 : 0)};
+}
 constexpr unsigned kSoloNowhere = 0x7FFFFFFCu;  // an offset past every array: loads give zero, stores go nowhere
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t solo_array(const void *base, size_t bytes) {
@@ -118,7 +125,7 @@ __global__ __launch_bounds__(solo_threads(NW)) __attribute__((amdgpu_waves_per_e
     __shared__ unsigned pads[2][kLocalSeqs];
 
     const int H = p.H, S = p.S, T = p.T;
-    const LocalJob part = local_job(p, blockIdx.x);
+    const SoloJob part = solo_job(p, blockIdx.x);
     const int dir = part.dir;
     const DirPtrs &D = p.d[dir];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -292,7 +299,7 @@ __global__ __launch_bounds__(solo_threads(NW)) __attribute__((amdgpu_waves_per_e
     __shared__ unsigned pads[2][kLocalSeqs];
 
     const int H = p.H, S = p.S, T = p.T;
-    const LocalJob part = local_job(p, blockIdx.x);
+    const SoloJob part = solo_job(p, blockIdx.x);
     const int dir = part.dir;
     const DirPtrs &D = p.d[dir];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;

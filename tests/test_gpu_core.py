@@ -1,6 +1,7 @@
 """GPU parity tests (through the C ABI) for the matrix product seam, dense / SSE layers and the LSTM.
 Tolerance: 1e-4 on the L2-normalised difference per tensor (fp32, different summation order);
 masking and indexing are asserted bit-exactly inside parity_cases."""
+import os
 import re
 
 import pytest
@@ -449,6 +450,55 @@ def test_lstm_step_by_step_recursion_equals_the_persistent_kernels(monkeypatch):
     monkeypatch.setenv("CNT_LSTM_STEPWISE", "1")
     assert PC.run_lstm_case(24, 128, True, [10, 6, 10], seed=5, wscale=0.5, escale=20.0, repeat_backward=True) < TOL
     assert PC.run_lstm_case(30, 256, False, [12, 12, 7], seed=6) < TOL
+
+
+@pytest.mark.parametrize("L,bidir,lengths", [
+    (512, True, [30, 17, 40, 38, 25, 40, 9, 33, 28, 36]),        # a job for the longest, others share
+    (256, True, [5, 40, 2, 40, 0, 31, 1, 22, 17, 12]),           # an empty sequence, two teams of an XCD
+    (300, True, [40 - 2 * (i % 15) for i in range(20)]),         # sixteen cells per workgroup
+    (200, False, [7] * 30 + [40, 39]),                           # two long sequences among many short ones
+    (130, False, [3 + (7 * i) % 38 for i in range(64)]),         # as many as are planned, several launches
+    (130, False, [3 + (7 * i) % 38 for i in range(65)]),         # one more: dealt evenly
+    (512, False, [12, 40, 33]), (512, True, [21, 20, 20, 20, 20, 20, 20, 20] * 2), (600, True, [20, 5, 20, 11, 3] * 4),
+])
+def test_lstm_sequences_dealt_by_length(L, bidir, lengths):
+    """Jobs hold sequences by length and leave out the steps on which all of theirs are padding: every state array, also on the
+    padding slots that a longer fraction has used before, is what the step-by-step schedule leaves."""
+    import torch
+
+    print("lstm dealt by length", L, bidir, lengths, flush=True)
+    capi = PC.pkg().capi
+    P, S, T = 16, len(lengths), 40
+    fractions = []
+    for k, ends in enumerate(([T] * S, lengths)):
+        W, x, outerr = PC.lstm_inputs(P, L, bidir, S, T, ends, 5 + k)
+        pat = PC.make_pat_types(ends, T).reshape(T, S)
+        pat[:, [s for s in range(S) if ends[s] == 0]] = 0
+        fractions.append((PC.dev(W), PC.dev(x), PC.dev(outerr), PC.dev(pat.reshape(-1)), min(ends)))
+    got = []
+    for stepwise in (False, True):
+        if stepwise:
+            os.environ["CNT_LSTM_STEPWISE"] = "1"
+        try:
+            layer = capi.Lstm(P, L, bidir, S, T)
+        finally:
+            os.environ.pop("CNT_LSTM_STEPWISE", None)
+        out, ex = torch.zeros(L * T * S, device="cuda"), torch.zeros(P * T * S, device="cuda")
+        dW = torch.zeros_like(fractions[0][0])
+        for W, x, outerr, pat, shortest in fractions:
+            err = outerr.clone()
+            layer.load_sequences(pat, T, shortest)
+            layer.forward(W, x, out)
+            layer.backward(W, x, out, err, ex, dW)
+            layer.check()
+        r = {"out": out, "err": err, "ex": ex, "dW": dW}
+        for d in range(2 if bidir else 1):
+            for k in ("ni", "ig", "fg", "og", "c", "h", "dni", "dig", "dfg", "dog", "cerr") + (("herr",) if bidir else ()):
+                r["%s%d" % (k, d)] = layer.state(d, k)
+        got.append({k: v.cpu().numpy() for k, v in r.items()})
+        layer.close()
+    for k in got[0]:
+        assert PC.relerr(got[0][k], got[1][k]) < TOL, k
 
 
 @pytest.mark.parametrize("L,bidir,lengths", [(256, True, [110, 104, 90]), (256, False, [107]), (600, True, [104] * 34), (1024, True, [106, 105])])
