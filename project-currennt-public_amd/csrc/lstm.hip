@@ -59,9 +59,9 @@ struct ChainParams {
     float *herr_out;      // backward, unidirectional: where the summed error is written back
     unsigned spin_limit;
     int *abort_flag;
-    int poll_delay, poll_gap;  // s_sleep units before the first poll of a step / between polls
+    int poll_delay, poll_limit, poll_gap;  // s_sleep units before the first poll of a step (-1: as the job's size wants it) and at most / between polls
     int mem_delay;             // XCD-local backward recursion: s_sleep units before the store wave's work of a step
-    int poll_delay_fwd, mem_delay_fwd;  // forward: the same, and before the load wave's
+    int poll_delay_fwd, poll_limit_fwd, mem_delay_fwd;  // forward: the same, and before the load wave's
     int *latch;  // host-visible mark "a recursion of this handle gave up" (pinned host memory), never cleared by kernels
     int *veto;   // optional device flag shared by a network's handles, set together with the latch
     // XCD-local recursions: jobs = (direction, group of sequences), see lstm_local.hpp
@@ -115,12 +115,16 @@ constexpr unsigned kEmpty = 0xFFFFFFFFu;
 constexpr int kMailSlots = 4;
 // Pauses of the XCD-local recursions, units of 64 clocks: before the first poll of a step (a pause that ends after the words have
 // arrived costs a poll round less, one that ends too late its own length), and before the store wave's work of a backward and the
-// load wave's of a forward step, which then stay out of the first poll's way.  Measured on MI355X, us per step.  Backward, first
-// poll after 1 / 3 / 5 / 7 / 9 units: 256 cells 8 jobs of 2-3 sequences 0.90 / 0.87 / 0.91 / 0.97 / 1.00, jobs of one 0.75 / 0.77 /
-// 0.80 / 0.84 / 0.89; stores after 0 / 4 / 8 units 0.90 / 0.87 / 0.88.  Forward, 8 / 9 / 10 / 11 / 12 / 13 / 14 / 16 units: 1.05 / 1.04 /
-// 1.03 / 1.00 / 1.00 / 1.01 / 1.03 / 1.07 and 0.88 / 0.88 / 0.87 / 0.86 / 0.87 / 0.89 / 0.92 / 0.98; loads after 0 / 4 units 0.99 / 0.98.
-// Sizes of 128 to 512 cells and 1 to 16 jobs have their best values within one unit of these.
-constexpr int kBackwardPause = 3, kStorePause = 4, kForwardPause = 11, kLoadPause = 4;
+// load wave's of a forward step, which then stay out of the first poll's way.  Measured on MI355X, us per step.  Forward, 8 / 9 / 10 /
+// 11 / 12 units: 256 cells 8 jobs of one sequence 0.785 / 0.769 / 0.776 / 0.798 / 0.832, of two 0.84 / 0.83 / 0.83 / 0.85 / 0.86, of three
+// 0.93 / 0.91 / 0.92 / 0.92 / 0.92, 16 jobs of four (16 cells per workgroup) 1.14 / 1.14 / 1.13 / 1.12 / 1.12, 150 cells 0.96 / 0.93 /
+// 0.96 / 0.98 / 1.00, 512 cells jobs of four 1.62 / 1.60 / 1.58 / 1.55 / 1.55.  Backward, 1 / 2 / 3 / 4 / 5 units: 0.68 / 0.67 / 0.70 / 0.75 / 0.76,
+// 0.76 / 0.75 / 0.75 / 0.77 / 0.79, 0.84 / 0.83 / 0.81 / 0.82 / 0.86, 1.14 / 1.13 / 1.08 / 1.07 / 1.08, 0.85 / 0.86 / 0.86 / 0.89 / 0.90, 1.49 / 1.49 /
+// 1.48 / 1.43 / 1.42.  Stores after 0 / 2 / 4 / 6 units: within 2 % of each other.
+// EL = words of a message, cells per workgroup times sequences of the job.
+constexpr int kStorePause = 4, kLoadPause = 4;
+constexpr int backward_pause(int EL) { return EL <= 8 ? 2 : EL <= 32 ? 3 : 4; }
+constexpr int forward_pause(int EL) { return EL <= 32 ? 9 : 11; }
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima) as a builtin, so that the compiler's own wait
@@ -143,6 +147,14 @@ __device__ __forceinline__ void poll_load(const float *base, unsigned byte_off, 
     wait_all_vmem();
 #pragma unroll
     for (int q = 0; q < N; ++q) asm volatile("" : "+v"(w[q]));  // consumers stay behind the wait
+}
+
+// After a poll that found a word empty: has this wave polled long enough, or another workgroup given up?  Uniform over the wave, as
+// is the poll loop's way out: with every lane leaving for itself the masks of the loop were some twenty scalar instructions on
+// the chain of a step.
+__device__ __forceinline__ bool poll_gives_up(const ChainParams &p, unsigned spins) {
+    if (spins > p.spin_limit) return true;
+    return (spins & 255u) == 0u && __builtin_amdgcn_readfirstlane(__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
 }
 
 #include "lstm_local.hpp"
@@ -376,9 +388,9 @@ struct cnt_lstm {
     int warm;  // read the recursion's inputs once before the XCD-local backward recursion (off; CNT_LSTM_WARM=1: on)
     int spread_lds_most;
     int spread_lds;  // dynamic LDS the XCD-local recursion asks for so that a compute unit takes one of its workgroups
-    int poll_delay_local;  // pause before the first poll of a step in the XCD-local recursion, units of 64 clocks
+    int poll_delay_local, poll_limit_local;  // pause before the first poll of a step in the XCD-local recursion, units of 64 clocks (-1: the job's), and its limit
     int mem_delay_local;   // pause of that recursion's store wave after the step barrier, same units
-    int poll_delay_fwd_local, mem_delay_fwd_local;  // XCD-local forward recursion: pauses before the first poll and the loads of a step
+    int poll_delay_fwd_local, poll_limit_fwd_local, mem_delay_fwd_local;  // XCD-local forward recursion: the same, and before the loads of a step
     // set by every recursion launch: the failure latch is taken only once the launch that may have set it has ended
     // (the device's recursion-order event, see launch_in_order), so that no workgroup of that launch can set it (or the
     // veto) again after the report
@@ -423,6 +435,7 @@ void fill_chain_params(const cnt_lstm *h, const float *weights, ChainParams &p) 
     p.ctl = h->ctl;
     p.lmail = h->lmail;
     p.flmail = h->flmail;
+    p.poll_limit = h->poll_limit_local; p.poll_limit_fwd = h->poll_limit_fwd_local;
     p.poll_delay = h->poll_delay_local; p.poll_gap = h->poll_gap; p.poll_delay_fwd = h->poll_delay_fwd_local;
     p.mem_delay_fwd = h->mem_delay_fwd_local;
     p.mem_delay = h->mem_delay_local;
@@ -803,7 +816,8 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     h->flmail_dirty = 1;
     h->spin_limit = 1u << 22;
     if (const char *e = std::getenv("CNT_LSTM_SPIN_LIMIT")) h->spin_limit = (unsigned)std::strtoul(e, nullptr, 10);
-    h->poll_delay_local = kBackwardPause;
+    h->poll_delay_local = h->poll_delay_fwd_local = -1;
+    h->poll_limit_local = h->poll_limit_fwd_local = 1 << 20;
     h->mem_delay_local = kStorePause;
     if (const char *e = std::getenv("CNT_LSTM_MEM_DELAY")) h->mem_delay_local = std::atoi(e);
     // The full-bandwidth read of the recursion's inputs in front of it (warm_cache) was worth 0.15 ms per model pass
@@ -814,7 +828,6 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     h->warm = 0;
     if (const char *e = std::getenv("CNT_LSTM_WARM")) h->warm = std::atoi(e) != 0;
     if (const char *e = std::getenv("CNT_LSTM_POLL_DELAY")) h->poll_delay_local = std::atoi(e);
-    h->poll_delay_fwd_local = kForwardPause;
     h->mem_delay_fwd_local = kLoadPause;
     if (const char *e = std::getenv("CNT_LSTM_POLL_DELAY_FWD")) h->poll_delay_fwd_local = std::atoi(e);
     if (const char *e = std::getenv("CNT_LSTM_POLL_GAP")) h->poll_gap = std::atoi(e);
@@ -928,9 +941,9 @@ int cnt_lstm_set_wait_bounds(cnt_lstm *h, unsigned spin_limit, int poll_delay_ba
     CNT_REQUIRE(poll_delay_backward >= 0 && poll_delay_backward <= 4096 && poll_delay_forward >= 0 &&
                 poll_delay_forward <= 4096, "lstm_set_wait_bounds: poll delays must be within 0..4096");
     h->spin_limit = spin_limit;
-    h->poll_delay_local = std::min(poll_delay_backward, kBackwardPause);
+    h->poll_limit_local = poll_delay_backward;
     h->mem_delay_local = std::min(poll_delay_backward, kStorePause);
-    h->poll_delay_fwd_local = std::min(poll_delay_forward, kForwardPause);
+    h->poll_limit_fwd_local = poll_delay_forward;
     return CNT_OK;
 }
 

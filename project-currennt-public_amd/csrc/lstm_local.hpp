@@ -42,8 +42,9 @@
 // chain are what counts.  With one cell wave, all gates of an element in one lane, a sum of 32 lane swaps, a product whose B
 // operand was read from LDS once per four instructions, messages of four sequences throughout and one wave for all loads and
 // stores (whose pause then set the step's length) a step took, us on MI355X: 256 cells, 8 jobs of 2-3 sequences 1.25, 2 jobs of
-// one 1.24, 16 jobs of four 1.73; 128 cells, 8 jobs of two 1.24; 512 cells, 6 jobs of one 1.85.  Now 0.87, 0.78, 1.15, 0.83 and
-// 1.22.  (A hop inside an XCD with nothing but a
+// one 1.24, 16 jobs of four 1.73; 128 cells, 8 jobs of two 1.24; 512 cells, 6 jobs of one 1.85.  Then 0.87, 0.78, 1.15, 0.83 and
+// 1.22; now, with a branch of the whole wave out of the poll loop and what does not wait for the poll worked out in front of it,
+// 0.81, 0.69, 1.05, 0.69 and 1.11.  (A hop inside an XCD with nothing but a
 // poll and a store at its ends takes 0.25, one of a 4 KB message 0.45.)
 //
 // Mailbox of a job: plain 4-byte words [slot][receiver][sender][cell of the receiver][sequence], kEmpty = not
@@ -571,6 +572,7 @@ __device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJo
     constexpr unsigned poll_stride = (unsigned)SPW * EL * 4u;
     // lanes past the last sender poll their first vector once more and leave it out of the sum
     const bool last_counts = lane / VPW + SPW * (NL - 1) < G;
+    const int pause = min(p.poll_limit, p.poll_delay >= 0 ? p.poll_delay : backward_pause(EL));
     const unsigned poll_off_last = last_counts ? poll_off + (unsigned)(NL - 1) * poll_stride
                                                : ((unsigned)me * RECV + (unsigned)(vec * 4)) * 4u;
     // cell-update role: after the sum a lane holds word lane / 16 of its vector; of the copies in the row each takes a gate
@@ -609,24 +611,24 @@ __device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJo
         carry = first ? 0.0f : fg_later * cerr_later + carry;
         const bool no_delta = dummy != 0.0f || (last && gate == 2);
         float e = k[3];
-
-        bool ok = true;
+        // what does not wait for the poll is worked out while it is in flight (the compiler would move it behind)
+        unsigned to_dl = (unsigned)((b * NSQ + cj) * DP + 4 * cc + gate), to_res = (unsigned)((b * EL + el) * 2 + gate);
+        asm volatile("" : "+v"(carry), "+v"(to_dl), "+v"(to_res));
         if (!first) {
             const float *slot = mailbox + (size_t)((unsigned)(step - 1) % kMailSlots) * slot_words;
             u32x4 w[NL];
             unsigned spins = 0;
-            for (int d = 0; d < p.poll_delay; ++d) __builtin_amdgcn_s_sleep(1);
+            for (int d = 0; d < pause; ++d) __builtin_amdgcn_s_sleep(1);
             for (;;) {
                 poll_load<NL>(slot, poll_off, poll_stride, poll_off_last, w);
                 if constexpr (CLOCKS) ++rounds;
                 unsigned worst = 0;
 #pragma unroll
                 for (int i = 0; i < NL; ++i) worst = max(max(worst, w[i].x), max(max(w[i].y, w[i].z), w[i].w));
-                if (worst != kEmpty) break;
-                if (++spins > p.spin_limit) { ok = false; break; }
-                if ((spins & 255u) == 0u &&
-                    __hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-                    ok = false;
+                if (__builtin_amdgcn_ballot_w64(worst == kEmpty) == 0) break;
+                if (poll_gives_up(p, ++spins)) {
+                    wait_failed = 1;
+                    if (lane == 0) raise_abort(p);
                     break;
                 }
                 for (int d = 0; d < p.poll_gap; ++d) __builtin_amdgcn_s_sleep(1);
@@ -646,16 +648,13 @@ __device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJo
         const float d_og = k[0] * e + k[2];
         float ce = k[1] * e + p_og * d_og;
         ce += carry;
-        float own = clip1(gate == 3 ? d_og : k_own * ce);
-        own = no_delta ? 0.0f : own;
+        float own = gate == 3 ? d_og : k_own * ce;
+        const float clipped = __builtin_amdgcn_fmed3f(own, -1.0f, 1.0f);  // clip1, with the test for NaN beside it
+        own = no_delta ? 0.0f : own == own ? clipped : own;
         ce = dummy != 0.0f ? 0.0f : ce;
-        dl[b][cj][4 * cc + gate] = own;
-        if (gate < 2) res[b][el][gate] = gate ? ce : e;
+        (&dl[0][0][0])[to_dl] = own;
+        if (gate < 2) (&res[0][0][0])[to_res] = gate ? ce : e;
         fg_later = fg; cerr_later = ce; own_later = own;
-        if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
-            wait_failed = 1;
-            if (lane == 0) raise_abort(p);
-        }
         if (records) clock_point<CLOCKS>(p, step - begin_step, 2);
         const long long at_barrier = clock_now<CLOCKS>();
         lds_barrier();

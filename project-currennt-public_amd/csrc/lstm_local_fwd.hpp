@@ -28,7 +28,8 @@
 // cell wave that computed all gates of an element in one lane (five gate functions, two of them side by side at best, twenty LDS
 // reads), gather waves that passed the words through LDS into B operands, messages of four sequences throughout and one wave for all
 // loads and stores, a step took, us on MI355X (input products included): 256 cells, 8 jobs of 2-3 sequences 1.34, 2 jobs of one
-// 1.29, 16 jobs of four 1.43; 128 cells, 8 jobs of two 1.22; 512 cells, 6 jobs of one 1.97.  Now 0.99, 0.85, 1.18, 0.89 and 1.34.
+// 1.29, 16 jobs of four 1.43; 128 cells, 8 jobs of two 1.22; 512 cells, 6 jobs of one 1.97.  Then 0.99, 0.85, 1.18, 0.89 and 1.34;
+// now, with a branch of the whole wave out of the poll loop and pauses of a job's own, 0.92, 0.77, 1.14, 0.75 and 1.26.
 // Publishing without LDS, by a broadcast inside the row of sixteen lanes, saves a round trip of 0.03 but stores pieces of 16
 // bytes: 1.05 instead of 1.00.
 
@@ -302,6 +303,7 @@ __device__ __forceinline__ void forward_job(const ChainParams &p, const LocalJob
     // a lane past the end of the block polls the block's first vector instead and multiplies zeros
     const int my_vec = (16 * pw + (lane >> 2)) * NSQ + (lane & 3) % NSQ;
     const bool inside = my_vec < vectors;
+    const int pause = min(p.poll_limit_fwd, p.poll_delay_fwd >= 0 ? p.poll_delay_fwd : forward_pause(EL));
     const unsigned poll_off = ((unsigned)me * RECV + (unsigned)(inside ? my_vec : 0) * 4u) * 4u;
     long long waited = 0, rest = 0, barrier = 0, rounds = 0;
     const bool records = CLOCKS && tid == 0;
@@ -314,21 +316,15 @@ __device__ __forceinline__ void forward_job(const ChainParams &p, const LocalJob
         const long long since = clock_now<CLOCKS>();
         if (records) clock_point<CLOCKS>(p, step - begin_step, 0);
         const float *slot = mailbox + (size_t)((unsigned)(step - 1) % kMailSlots) * slot_words;
-        bool ok = true;
         u32x4 w[1];
         unsigned spins = 0;
-        for (int d = 0; d < p.poll_delay_fwd; ++d) __builtin_amdgcn_s_sleep(1);
+        for (int d = 0; d < pause; ++d) __builtin_amdgcn_s_sleep(1);
         for (;;) {
             poll_load<1>(slot, poll_off, 0u, poll_off, w);
             if constexpr (CLOCKS) ++rounds;
             const unsigned worst = max(max(w[0].x, w[0].y), max(w[0].z, w[0].w));
-            if (worst != kEmpty) break;
-            if (++spins > p.spin_limit) { ok = false; break; }
-            if ((spins & 255u) == 0u &&
-                __hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-                ok = false;
-                break;
-            }
+            if (__builtin_amdgcn_ballot_w64(worst == kEmpty) == 0) break;
+            if (poll_gives_up(p, ++spins)) { wait_failed = 1; break; }
             for (int d = 0; d < p.poll_gap; ++d) __builtin_amdgcn_s_sleep(1);
         }
         clock_add<CLOCKS>(waited, since);
@@ -348,7 +344,6 @@ __device__ __forceinline__ void forward_job(const ChainParams &p, const LocalJob
         } else {
             out[0] = sum_halves(sum[0], sum[0]);
         }
-        if (__builtin_amdgcn_ballot_w64(!ok) != 0) wait_failed = 1;
         if (records) clock_point<CLOCKS>(p, step - begin_step, 2);
         const long long at_barrier = clock_now<CLOCKS>();
         lds_barrier();
