@@ -360,6 +360,28 @@ int cnn_backward_errors_fan(cnt_cnn *h, hipStream_t stream, const char *patTypes
                             const float *outputs, float *output_errors, float *prev_errors, int delta_applied,
                             const FanOut *fan, bool *fused);
 
+// Weight gradients of up to kBlockGradients such blocks in one launch (wavenet_weights.hip): the convolution (two live taps of a
+// window of three), the conditioning projection, the 1x1 layer behind the gate and the skip 1x1 layer, with the bias gradients.
+constexpr int kBlockGradients = 8;
+struct BlockGradients {
+    const float *x, *gated, *sum;                                // inputs of the convolution and of the two 1x1 layers
+    const float *deltas, *ctx_grad, *out_errors, *skip_errors;   // what their outputs receive, in that order
+    float *conv, *conv_bias, *ctx, *out, *out_bias, *skip, *skip_bias;  // the weight updates
+    float conv_scale, out_scale, skip_scale;                     // factors of the bias gradients
+    int shift;                                                   // the earlier tap reads slot n - shift
+};
+bool wavenet_block_weights_supported(int R, int K, int C, long N);
+size_t wavenet_block_weights_scratch();  // floats; one launch at a time
+int wavenet_block_weights(hipStream_t stream, int R, int K, int C, int N, int count, const BlockGradients *blocks, const float *ctx,
+                          const char *patTypes, float *scratch);
+// the shift, the bias gradient's place behind the weights and its factor, of a layer that cnn_foldable accepts
+struct CnnTaps {
+    int shift;
+    size_t bias_at;
+    float bias;
+};
+CnnTaps cnn_taps(const cnt_cnn *h);
+
 // ----- weight-gradient halves of several layers of one shape in one launch --------------------------
 // For the network sequencer: `count` (<= kGemmMaxProb) dense layers with the same P, D, N, or wavnetc layers with the
 // same D, C, N and one context buffer, as the problems of one product.  Same results as `count` calls of

@@ -518,6 +518,7 @@ struct cnt_network {
     // optimizer state (allocated by the first update)
     float *cur_updates = nullptr, *deltas = nullptr, *stats = nullptr;
     int stats_option = -1;
+    float *block_sums = nullptr;  // of wavenet_block_weights, whose launches go to the first side stream one after the other
     float *adam_accum = nullptr;  // beta1^t, beta2^t of Adam's bias correction (device)
     int mdn_target_start = 0, mdn_classes = 0;
     // set on the device by an LSTM recursion that gives up; the optimizer step looks at it and leaves the weights alone
@@ -1059,6 +1060,10 @@ int finish_build(cnt_network *net, const json::Value *weights) {
         const size_t rows = ((size_t)net->S * C.maxTr + 63) / 64;
         CNT_TRY(device_alloc(net, (void **)&C.colsum, rows * C.size * sizeof(float), false));
     }
+    for (size_t i = 5; i < net->layers.size() && !net->block_sums; ++i)
+        if (net->layers[i].kind == K_DENSE && net->layers[i - 4].kind == K_WAVNETC &&
+            wavenet_block_weights_supported(net->layers[i - 4].size, net->layers[i].size, net->layers[i - 4].ctx_dim, 1))
+            CNT_TRY(device_alloc(net, (void **)&net->block_sums, wavenet_block_weights_scratch() * sizeof(float), false));
     // the slots of a fraction with the valid ones first: the weight gradients of the dense and recurrent layers sum over
     // those only (CNT_NET_SKIP_PADDING=0: over all slots)
     {
@@ -1412,6 +1417,13 @@ bool block_errors_at(const cnt_network *net, size_t i) {
 // it reads for their derivatives: the forward pass then need not leave them behind.
 bool block_sums_core(const NetLayer &cnn, const NetLayer &wav) { return cnn.delta_fused && wav.ctx_dim > 0; }
 
+// whether the weight gradients of the block that block_errors_at describes go into the blocks' common launches
+bool block_weights_at(const cnt_network *net, size_t i) {
+    const NetLayer &sk = net->layers[i], &ini = net->layers[i - 1], &wav = net->layers[i - 4], &cnn = net->layers[i - 5];
+    return net->block_sums && wavenet_block_weights_supported(ini.size, sk.size, wav.ctx_dim, sk.N) && cnn_foldable(cnn.cnn, ini.size) &&
+           (cnn.delta_fused || !cnn.cnn_tanh);
+}
+
 }  // namespace
 }  // namespace cnt
 
@@ -1760,6 +1772,47 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
             for (ShapeGroup &c : groups) CNT_TRY(hand_over_group(c));
         return CNT_OK;
     };
+    // Weight gradients of residual blocks, eight blocks to a launch
+    std::vector<char> weights_done(net->layers.size(), 0);
+    std::vector<size_t> blocks;  // their skip 1x1 layers
+    auto hand_over_blocks = [&]() -> int {
+        if (blocks.empty()) return CNT_OK;
+        hipStream_t ws = stream;
+        if (net->overlap) {
+            ws = net->side[0];
+            CNT_HIP(hipEventRecord(net->ev_main, stream));
+            CNT_HIP(hipStreamWaitEvent(ws, net->ev_main, 0));
+            side_used[0] = true;
+        }
+        BlockGradients g[kBlockGradients];
+        const NetLayer &first = net->layers[blocks[0]];
+        for (size_t z = 0; z < blocks.size(); ++z) {
+            const size_t i = blocks[z];
+            const NetLayer &sk = net->layers[i], &out = net->layers[i - 3], &wav = net->layers[i - 4], &cnn = net->layers[i - 5];
+            const int R = wav.size;
+            const CnnTaps taps = cnn_taps(cnn.cnn);
+            float *const u = net->updates;
+            g[z] = {net->layers[i - 6].out, wav.out, net->layers[i - 1].out, cnn.err, wav.cgrad, out.err, sk.err,
+                    u + cnn.w_off, u + cnn.w_off + taps.bias_at, u + wav.w_off, u + out.w_off, u + out.w_off + (size_t)R * R,
+                    u + sk.w_off, u + sk.w_off + (size_t)R * sk.size, taps.bias, out.bias, sk.bias, taps.shift};
+        }
+        const int count = (int)blocks.size();
+        blocks.clear();
+        return wavenet_block_weights(ws, net->layers[(size_t)(&first - net->layers.data()) - 1].size, first.size,
+                                     net->layers[(size_t)(&first - net->layers.data()) - 4].ctx_dim, first.N, count, g, net->ctx,
+                                     first.pat, net->block_sums);
+    };
+    auto join_blocks = [&](size_t i) -> int {
+        if (!blocks.empty()) {
+            const size_t o = blocks[0];
+            if (net->layers[o].size != net->layers[i].size || net->layers[o - 1].size != net->layers[i - 1].size ||
+                net->layers[o].N != net->layers[i].N || net->layers[o].pat != net->layers[i].pat)
+                CNT_TRY(hand_over_blocks());
+        }
+        blocks.push_back(i);
+        for (size_t k : {i, i - 3, i - 4, i - 5}) weights_done[k] = 1;
+        return blocks.size() == kBlockGradients ? hand_over_blocks() : CNT_OK;
+    };
     // the side buffers that a launch of skip layer `from` adds to: the next forward pass clears them
     auto adds_to_side = [&](const NetLayer &from) {
         for (int k : from.side_targets) net->sides[(size_t)k].touched = true;
@@ -1840,6 +1893,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                             direct_from[i - 8] = prev_err;
                         }
                         const bool fan_live = block_fan.n > 0 || block_fan.from_skip;
+                        const bool together = block_weights_at(net, i);
                         if (block_fan.n > 0) adds_to_side(prev);
                         CNT_TRY(wavenet_block_errors(stream, prev.size, L.size, N, L.pat, W, net->weights + out.w_off, L.err,
                                                      prev_err, fan_live ? &block_fan : nullptr,
@@ -1847,8 +1901,9 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                                                      wav.ctx_dim > 0 ? wav.cgrad : nullptr, cnn.delta_fused ? cnn.out : nullptr,
                                                      cnn.err, fold ? fold->cnn : nullptr,
                                                      fold ? net->weights + fold->w_off : nullptr, fold ? fold->err : nullptr,
-                                                     cnn.colsum));
-                        if (cnn.colsum) net->layers[i - 5].colsum_rows = wavenet_block_rows(prev.size, N, fold != nullptr);
+                                                     together ? nullptr : cnn.colsum));
+                        if (together) CNT_TRY(join_blocks(i));
+                        else if (cnn.colsum) net->layers[i - 5].colsum_rows = wavenet_block_rows(prev.size, N, fold != nullptr);
                         fan_done[i - 1] = 1;
                         errors_done[i - 3] = errors_done[i - 4] = 1;
                         goto weight_half_of_layer;
@@ -1922,7 +1977,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                     }
                 }
             weight_half_of_layer:
-                if (L.kind == K_WAVNETC && L.ctx_dim == 0) break;
+                if (weights_done[i] || (L.kind == K_WAVNETC && L.ctx_dim == 0)) break;
                 if (!net->overlap) {
                     CNT_TRY(weight_half(i, stream));
                     break;
@@ -1995,6 +2050,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                 break;
         }
     }
+    CNT_TRY(hand_over_blocks());
     CNT_TRY(hand_over(false));
     for (ShapeGroup &g : groups) CNT_TRY(hand_over_group(g));
     for (int k = 0; k < net->n_side; ++k) {

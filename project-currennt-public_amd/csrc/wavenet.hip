@@ -1024,6 +1024,10 @@ extern "C++" bool cnt::cnn_foldable(const cnt_cnn *h, int R) {
            h->groups[0].d1 == h->desc.D && h->desc.P == R && h->desc.D == 2 * R;
 }
 
+extern "C++" cnt::CnnTaps cnt::cnn_taps(const cnt_cnn *h) {
+    return {h->groups[0].dil * h->desc.S, (size_t)h->desc.P * h->Lw, h->desc.bias};
+}
+
 extern "C++" int cnt::wavenet_block_errors(hipStream_t stream, int R, int K, int N, const char *patTypes,
                                            const float *skip_weights, const float *out_weights, const float *skip_errors,
                                            float *total, const FanOut *fan, const float *core_buf, const float *ctx_tanh,
