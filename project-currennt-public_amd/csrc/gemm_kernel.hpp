@@ -726,6 +726,8 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
         }
         return;
     }
+    const float *const old = args.epilogue == EPI_STORE_DELTA || args.epilogue == EPI_CONTEXT ? pb.aux_in
+                                        : args.epilogue == EPI_ADD ? C : nullptr;
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
         const int m = m0 + wm * WT + i * 32 + frag_row;
@@ -735,6 +737,17 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
             bterm = args.bias_scale * pb.bias_vec[m];
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
+            // What the sums meet in memory is requested for sixteen of them at a time: the compiler cannot know that it does not
+            // overlap the output and would wait for one load per sum (a dense layer's deltas in the epilogue of the product above
+            // it: the feed-forward model's pass, four such products, 2260 -> 2183 us).
+            float met[16];
+            if (old) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int n = min(n0 + wn * WT + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3), args.n - 1);
+                    met[r] = old[(size_t)n * args.ldc + m];
+                }
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int n = n0 + wn * WT + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
@@ -744,8 +757,8 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
                 const float v = acc[i][j][r];
                 switch (args.epilogue) {
                     case EPI_STORE: *dst = v; break;
-                    case EPI_STORE_DELTA: *dst = v * act_deriv(args.act, pb.aux_in[idx]); break;
-                    case EPI_ADD: *dst = *dst + v; break;
+                    case EPI_STORE_DELTA: *dst = v * act_deriv(args.act, met[r]); break;
+                    case EPI_ADD: *dst = met[r] + v; break;
                     case EPI_ATOMIC: atomicAdd(dst, v); break;
 
                     case EPI_BIAS_ACT: *dst = act_fn(args.act, v + bterm); break;
@@ -756,7 +769,7 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
                         const bool valid = args.pat[n] != 0;
                         const float th = valid ? tanh_act(v) : 0.0f;
                         if (pb.aux_out) pb.aux_out[idx] = th;
-                        *dst = valid ? pb.aux_in[idx] + th : 0.0f;
+                        *dst = valid ? met[r] + th : 0.0f;
                     } break;
                 }
             }
