@@ -22,15 +22,20 @@
 //   1024 x 32000 x 128: 108 -> 73 us, 425 x 12000 x 1024: 141 -> 96 us, 300 x 10000 x 425: 47 -> 34 us.
 // Operands whose lines are no multiple of four long are read in vectors of four as well (FastStage); with one float per
 // lane and load the last two sizes took 100 and 43 us.
-// What bounds it now, at the first size per SIMD: 69 us of matrix instructions, 38 us of conversions, 51 us of LDS traffic,
-// which overlap only in part.  Measured and not taken: the conversion of the next tile between the matrix instructions of
+// What bounds it now: the matrix instructions under the card's power limit.  With random operands one takes 20 to 24 ns of a SIMD
+// (15 with zeros), which is 105 us of the first size's 138; leaving out five of the six part products gives 80 us, the
+// conversions 130, the loads 122.  With 64 x 64 tiles (512 x 9600 x 1024, 77 us: 48, 68, 60) the loads through the L2s and the
+// conversions weigh twice as much.  Measured and not taken: the conversion of the next tile between the matrix instructions of
 // this one, with two LDS buffers and one or two tiles of loads in flight (245 us: one wave per SIMD issues a vector
-// instruction every eight clocks, not four); 128 x 64 tiles (182 us).
+// instruction every eight clocks, not four); 128 x 64 tiles (182 us); 256 x 192 tiles of eight waves, half of them converting
+// in turn (162 us); LDS stores without bank conflicts (a third of the LDS clocks less, no difference); instructions of
+// 16 x 16 x 32, which alone run a third faster (150 us: twice as many of them hold the vector instructions up).
 //
 // Tiling: T x T x 32 per workgroup with T = 128 or 64, four 64-lane waves in a 2 x 2 arrangement, each wave
 // owning a T/2 x T/2 block as tiles of v_mfma_f32_32x32x16_bf16.  The parts lie in LDS in the order the instruction takes
 // them (TileLayout); 50 KB (T = 128) and 26 KB (T = 64) per workgroup leave room for three and five of them per compute unit, whose
-// phases overlap.  Two workgroups of T = 128 instead of three: 197 us at the first size above.
+// phases overlap.  Two workgroups of T = 128 instead of three: 197 us at the first size above.  A launch of few large tiles
+// takes eight waves for each of them, 2 x 4 of 64 x 32 (same sums, bit for bit; eight_waves below).
 // The MFMA operands are swapped (the B tile feeds the instruction's A port) so that lane%32 walks
 // along the column-major output's contiguous dimension and every store is a 128-byte segment.
 #include "gemm_kernel.hpp"
@@ -61,25 +66,37 @@ inline int pick_vec(const GemmArgs &a, bool for_a) {
     return v;
 }
 
-// Tile edge.  128 x 128 tiles convert and read half as much per matrix instruction, but three of them fill a compute unit, so a
-// launch needs some 600 of them, and a run over k long enough that filling and draining the pipeline does not show
-// (64 / 128, us: 1024 x 12000 x 1024 with 752 large tiles 200 / 165; 1024 x 6000 x 512 with 376 of them 54 / 56; 512 x
-// 6000 x 512 with 188 30 / 51; 1024 x 32000 x 128 with 2000 71 / 103).
-// Between 256 and 511 values of k it is the last generation that decides: large tiles pay where they fill what the chip holds of
-// them at a time (768) to at least nine tenths.  64 / 128, us, for 1024 rows and a k-contiguous A: k = 256, 752 tiles (0.98) 54 /
-// 49, 704 (0.92) 1.05 times as fast, 1360 (0.89) 1.02, 2000 (0.87) 0.97, 640 (0.83) 1.04, 1040 (0.68) 0.87; k = 448, 752 tiles 86 /
-// 72, 1360 1.09 times, 1040 0.98; a row-contiguous A within 3% of that; 1936 x 6000 x 256 59 / 50; k = 192 no gain anywhere.
-// The other lines lie where a generation ends, too: the 256 compute units hold 768 large and 1280 small tiles at a time, five
-// per compute unit.  From 768 values on the large tile pays as soon as the small ones begin a second generation: 320 large tiles are
-// 1280 small ones.  Times as fast with 304 / 320 / 336 / 400 / 480 / 560 / 768 / 800 / 1040 large tiles (least and most over 512,
-// 1024 and 2048 rows and both orders of A): k = 768 0.84-0.87 / 0.86-0.89 / 1.00-1.04 / 1.08-1.13 / 1.16-1.19 / 1.04 / 1.23-1.25 /
-// 0.97-0.99 / 1.10-1.12, k = 1024 0.87-0.92 / 0.89-0.94 / 1.04-1.08 / 1.12-1.18 / 1.20-1.24 / 1.05-1.07 / 1.26-1.28 / 1.00 / 1.11-1.15,
-// k = 3072 0.95-1.01 / 0.96-1.02 / 1.12-1.18 / 1.22-1.28 / 1.28-1.34 / 1.12 / 1.32-1.35 / 1.06 / 1.17-1.20.
-// With 512 to 767 values it needs 600 (560: 0.99-1.05, 600: 1.05-1.12, 768: 1.17-1.25), and a second generation of its own that is
-// hardly begun costs more than it gains: 800 / 864 / 896 / 960 / 1040 tiles at k = 512 0.90 / 0.92 / 0.93 / 0.96-0.99 /
-// 1.03-1.07, k = 600 0.93 / 0.96 / 0.97 / 1.00-1.02 / 1.06-1.11, k = 640 0.93 / 0.98 / 1.00 / 1.03 / 1.07-1.12, k = 736
-// 0.96 / 1.00-1.03 / 1.02-1.04 / 1.06-1.08 / 1.09-1.12.  The line at 960 is right for k up to 600; it gives away up to 7 % of
-// the 860 to 960 tiles at longer k.
+// Tile edge, and the waves of a workgroup.  128 x 128 tiles convert and read half as much per matrix instruction as 64 x 64 ones.
+// On four waves three of them fill a compute unit, and a launch needs some 600 of them to hide a tile's chain of load, conversion,
+// barrier and products behind the others'.  On eight waves (kEightWaves) the chain is half as long, so that ONE per compute unit
+// is worth having: a launch then takes as long as its busiest compute unit, and what decides is how full the last level of
+// one tile per compute unit is.  Times as fast on eight waves as the better of 64 x 64 and 128 x 128 on four (1024 rows, both
+// operands k-contiguous; a row-contiguous A and operands of odd length within 5 % of it or better):
+//   tiles     192  208  256  264  320  336  400  512  520  640  680  768  800  960 1024 1040 1200 1280 1536 2048
+//   level     .75  .81   1   .52  .62  .66  .78   1   .68  .83  .89   1   .78  .94   1   .81  .94   1    1    1
+//   k = 384   .93 1.07 1.08  .87  .90 1.03 1.13 1.19  .94 1.03 1.05 1.07 1.05 1.16 1.21 1.05 1.18 1.21 1.10 1.17
+//   512       .94 1.11 1.09  .88  .92 1.05 1.09 1.19  .96 1.01 1.01 1.05 1.06 1.19 1.19 1.02 1.04 1.14 1.05 1.06
+//   768       .97 1.15 1.16  .90  .92 1.06 1.07 1.10  .94  .99  .98 1.00 1.08 1.13 1.10  .96 1.00 1.08  .98  .99
+//   1024      .98 1.18 1.14  .91  .94 1.02 1.01 1.05  .93  .96  .97  .98 1.08 1.09 1.06  .95  .98 1.00  .98  .97
+//   2048     1.02 1.21 1.22  .93  .95  .96  .98 1.00  .92  .94  .94  .96 1.05 1.06 1.03  .95
+// (512 x 8192 x 2048, 256 tiles: 123 us with 64 x 64, 128 on four waves, 103 on eight.)  From 768 values on, three levels and more
+// than four are better off on four waves (a generation of those is 768), and the lines below give away at most 5 %.  Below 384
+// values the launch is its stores: back to back eight waves gain up to 15 % there, too, but inside a pass, with operands that have
+// left the caches, 1024 x 32000 x 128 takes 99 instead of 79 us, 1936 x 6000 x 256 61 instead of 53, 1024 x 12000 x 187 101 instead of
+// 94 (x 425: 100 either way, 2048 x 9600 x 512 123 instead of 125 to 156).
+inline bool eight_waves(long tiles, long run) {
+    const long levels = (tiles + 255) / 256, percent = 100 * tiles / (256 * levels);
+    if (run >= 1536) return levels == 1 ? percent >= 80 : levels == 4;
+    if (run >= 768) return levels == 1 ? percent >= 80 : levels == 2 ? percent >= 65 : levels == 4;
+    return run >= 384 && (levels == 2 ? percent >= 65 : levels == 3 ? percent >= 77 : levels == 4 || percent >= 80);
+}
+// Elsewhere, 64 x 64 or 128 x 128 on four waves.  Between 256 and 383 values the large tile pays where it fills the last generation
+// of 768 to nine tenths: 64 / 128, us, for 1024 rows and a k-contiguous A: 752 tiles (0.98) 54 / 49, 704 (0.92) 1.05 times as fast,
+// 1360 (0.89) 1.02, 2000 (0.87) 0.97, 640 (0.83) 1.04, 1040 (0.68) 0.87; k = 192 no gain anywhere.  With 768 values and more: the
+// large tile from 336 tiles on, where the small ones begin a second generation (1280 of them at a time); times as fast with 304 / 320 / 336 / 400 / 600 / 768 / 800 / 1040 large tiles
+// (least and most over 512, 1024 and 2048 rows and both orders of A): k = 768 0.84-0.87 / 0.86-0.89 / 1.00-1.04 / 1.08-1.13 / 1.04 /
+// 1.23-1.25 / 0.97-0.99 / 1.10-1.12, k = 3072 0.95-1.01 / 0.96-1.02 / 1.12-1.18 / 1.22-1.28 / 1.12 / 1.32-1.35 / 1.06 / 1.17-1.20.  Lines
+// of odd length (loads of single values at the edges): from 600 tiles and 512 values on.
 inline long large_tiles(const GemmArgs &a) { return (long)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.nprob; }
 
 // The weight gradient of one dense layer of 64 to 256 large tiles (1024 x 1024 weights and more) also takes the large tile, and
@@ -90,9 +107,7 @@ inline long large_tiles(const GemmArgs &a) { return (long)((a.m + 127) / 128) * 
 // 12 000 slots (250 / 625 / 1000 / 1500 per split) 43 / 58, 88 / 89, 134 / 121, 193 / 162; 1300 x 1300 over 3000 / 4000 (750 / 1000) 98 / 101, 125 / 120; 2048 x 2048 over
 // 1000 / 3000 (500 / 1500) 73 / 79, 187 / 159.  (Below 64 tiles the line is further up, 896 x 896 over 2000 / 6000 / 12 000
 // 41 / 57, 92 / 86, 173 / 136, and layers of 32 tiles gain nothing; they keep the small tile.)  The feed-forward model of five
-// such layers: 2320 -> 2224 us per pass, with 768 workgroups 2230.  The gradients of a
-// recurrent layer, several problems per launch, run beside the recursion of the layer below and leave it less LDS and
-// issue slots then: with them on the large tile the acoustic model's pass takes 3787 instead of 3767 us.
+// such layers: 2320 -> 2224 us per pass, with 768 workgroups 2230; on eight waves 2228 -> 2152.
 constexpr long kWideGradientGroups = 512;
 constexpr long kWideGradientSplit = 768;
 inline bool wide_gradient(const GemmArgs &a) {
@@ -101,17 +116,35 @@ inline bool wide_gradient(const GemmArgs &a) {
            (long)a.k * a.nseg * tiles >= kWideGradientSplit * kWideGradientGroups;
 }
 
+// The gradients of a recurrent layer, several problems per launch, on eight waves and one tile per compute unit: at least 32 large
+// tiles that the outputs fill, cut into as many splits as make 256 workgroups, of at least 704 values of k.  64 x 64 tiles cut to
+// 768 workgroups / 192, 256, 384, 512 workgroups of eight waves, us per pass: 32 sequences 2463 / 2410, 2373, 2357, 2376; the
+// acoustic model, where they run beside the recursion of the layer below, 2587 / 2582, 2569, 2620, 2599.  A layer of 2 x 256 cells
+// by itself over 2048 / 3200 / 6400 / 9600 slots (512, 800, 1600 and 2400 per split of the input weights) 454 / 464, 626 / 620, 837 /
+// 817, 1189 / 1161, of 2 x 512 cells over 2048 / 9600 757 / 743, 3008 / 2886.  (300 and 200 cells leave a quarter of the large
+// tiles' rows empty: 2264 -> 2315 with them.)
+constexpr long kLevelGradientGroups = 256;
+constexpr long kLevelGradientSplit = 704;
+inline bool level_gradient(const GemmArgs &a) {
+    const long tiles = large_tiles(a);
+    return a.nprob > 1 && !a.masked && !a.a_kcontig && !a.b_kcontig && tiles >= 32 && tiles <= kLevelGradientGroups &&
+           20L * a.m * a.n * a.nprob >= 19L * 16384 * tiles && (long)a.k * a.nseg * tiles >= kLevelGradientSplit * kLevelGradientGroups;
+}
+
 int pick_tile(const GemmArgs &a) {
     static const int forced = [] { const char *e = std::getenv("CNT_GEMM_TILE"); return e ? std::atoi(e) : 0; }();
     if (a.masked || a.epilogue == EPI_FAN) return 64;
-    if (forced == 64 || forced == 128) return forced;
+    if (forced == 64 || forced == 128 || forced == kEightWaves) return forced;
     const long t128 = large_tiles(a) * a.splitk;
-    if (wide_gradient(a) && t128 >= kWideGradientGroups / 2) return 128;
+    if ((wide_gradient(a) && t128 >= kWideGradientGroups / 2) || (level_gradient(a) && t128 >= kLevelGradientGroups / 2)) return kEightWaves;
     const long run = (long)a.k * a.nseg / a.splitk;
-    const bool quads = (a.a_kcontig ? a.k : a.m) % 4 == 0 && a.b_kcontig && a.k % 4 == 0;  // 768 at a time
+    const long t64 = (long)((a.m + 63) / 64) * ((a.n + 63) / 64) * a.nprob * a.splitk;
+    // (outputs that leave more than a twelfth of the large tiles' rows and columns empty stay on the small ones: 300 x 10 000 x 425
+    // and the like, 2207 -> 2276 us per pass with them on the large ones)
+    if ((a.a_kcontig || a.b_kcontig) && 12 * t64 >= 11 * 4 * t128 && eight_waves(t128, run)) return kEightWaves;
+    const bool quads = (a.a_kcontig ? a.k : a.m) % 4 == 0 && a.b_kcontig && a.k % 4 == 0;
     if (!quads) return t128 >= 600 && run >= 512 ? 128 : 64;
     if (run >= 768) return t128 >= 336 ? 128 : 64;
-    if (run >= 512) return t128 >= 600 && (t128 <= 768 || t128 > 960) ? 128 : 64;
     return t128 >= 600 && run >= 256 && 10 * t128 >= 9 * ((t128 + 767) / 768 * 768) ? 128 : 64;
 }
 
@@ -282,6 +315,8 @@ void gemm_plan(GemmArgs &args, hipStream_t stream) {
     long s = (target + tiles - 1) / tiles;
     if (forced_target == 0 && wide_gradient(args))
         s = kWideGradientGroups / large_tiles(args);
+    else if (forced_target == 0 && level_gradient(args))
+        s = kLevelGradientGroups / large_tiles(args);
     s = std::min(s, std::max(1L, kt / 8));
     s = std::max(1L, s);
     // no empty split: every split of the partial-product path has to write its share
@@ -354,12 +389,13 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
     }
     if (args.epilogue != EPI_PARTIAL && args.epilogue != EPI_ATOMIC) args.rowsum = 0;
     const int tile = pick_tile(args);
+    const int edge = tile == kEightWaves ? 128 : tile;
     // a list of k lines is used where the kernel that reads through it exists, and ignored otherwise (the lines it leaves
     // out are zero)
     if (args.k_order && !(args.k_count && !args.masked && !args.a_kcontig && !args.b_kcontig && aligned &&
                           args.epilogue != EPI_FAN && args.k < (1 << 24) && args.lda < (1 << 22) && args.ldb < (1 << 22)))
         args.k_order = nullptr;
-    const int tiles = ((args.m + tile - 1) / tile) * ((args.n + tile - 1) / tile);
+    const int tiles = ((args.m + edge - 1) / edge) * ((args.n + edge - 1) / edge);
     dim3 grid(tiles, args.splitk, args.nprob);
     // XCD-aware placement (gemm_kernel.hpp): measured with FETCH_SIZE on MI355X it cuts what the L2s fetch 2.2-2.6x for the
     // WaveNet stack's batched weight gradients (a convolution's two taps and a stack's conditioning projections share an

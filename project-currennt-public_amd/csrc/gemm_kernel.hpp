@@ -11,6 +11,7 @@ namespace {
 
 constexpr int BK = 32;  // k depth of a staged tile: two matrix instructions deep
 constexpr int NTHREADS = 256;
+constexpr int kEightWaves = 129;  // "tile" of a launch: 128 x 128, on eight waves
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -57,9 +58,9 @@ __device__ __forceinline__ void split_pair(float x0, float x1, unsigned (&part)[
 // takes: eight consecutive k of one row.  Units are ordered [part][k / 8][position of the row]; the position of a row is the
 // row itself where a thread loads along k, and r * GROUP + t for row VEC * t + r where it loads VEC rows at once, so that in
 // both cases the lanes of one store, and those of one read, fall on distinct banks (the pads of GROUP and LINE see to it).
-template <int VEC, bool KCONTIG, int ROWS>
+template <int VEC, bool KCONTIG, int ROWS, int NT = NTHREADS>
 struct TileLayout {
-    static constexpr int NLOAD = (ROWS * BK) / (NTHREADS * VEC);  // vectors per thread
+    static constexpr int NLOAD = (ROWS * BK) / (NT * VEC);  // vectors per thread
     static_assert(NLOAD >= 1, "tile too small for this vector width");
     static constexpr int GROUP = ROWS / VEC + (VEC == 4 ? 4 : VEC == 2 ? 8 : 0);
     static constexpr int LINE = KCONTIG ? ROWS + 4 : VEC * GROUP;  // units per k / 8
@@ -69,7 +70,7 @@ struct TileLayout {
 
     // k-contiguous: the thread's vectors start at k position first_k of the rows row(p); row-contiguous: they hold the VEC
     // rows from first_row on, of the NLOAD consecutive k positions from first_k on
-    static constexpr int TPR = BK / VEC, RPP = NTHREADS / TPR;
+    static constexpr int TPR = BK / VEC, RPP = NT / TPR;
     static constexpr int TPK = ROWS / VEC;
     static __device__ __forceinline__ int column(int tid) {  // t above
         if (TPK == 32) return (tid & 15) | ((tid & 32) >> 1);  // sixteen lanes along the rows, two halves of a unit
@@ -280,9 +281,9 @@ __device__ __forceinline__ void add_tile_rows(float (&sum)[4], const float4 (&r)
 }
 
 // WHOLE: the lines are a multiple of four long, so that no vector crosses the end of one.
-template <bool WHOLE, bool KCONTIG, int ROWS>
+template <bool WHOLE, bool KCONTIG, int ROWS, int NT>
 struct FastStage {
-    typedef TileLayout<4, KCONTIG, ROWS> L;
+    typedef TileLayout<4, KCONTIG, ROWS, NT> L;
     static constexpr int NLOAD = L::NLOAD;
     float4 r[NLOAD];
     unsigned voff[NLOAD];
@@ -341,9 +342,9 @@ struct FastStage {
 // The unmasked loader for row-contiguous operands whose k lines are picked through a list (16-byte vectors only): tile k
 // line j is line idx[j] of the operand.  The indices of a tile are loaded one iteration ahead by the kernel (both operands
 // share them) and handed to load(); everything else is FastStage.
-template <int ROWS>
+template <int ROWS, int NT>
 struct GatherStage {
-    typedef TileLayout<4, false, ROWS> L;
+    typedef TileLayout<4, false, ROWS, NT> L;
     static constexpr int NLOAD = L::NLOAD;
     float4 r[NLOAD];
     unsigned roff;   // byte offset of the thread's four rows inside a k line (clamped into the matrix)
@@ -442,13 +443,15 @@ __device__ __forceinline__ f32x16 plain_sums(const GemmArgs &args, const GemmPro
 // behind another's matrix instructions.  128 x 128 tiles of two row-contiguous operands take 55 KB each, so two: where three were
 // asked for, the compiler held operands in accumulator registers and a small change made it miss two as well (the feed-forward
 // model 2213 -> 2293 us per pass).
-template <int VA, bool AK, int VB, bool BK_, bool MASKED, int TILE, bool FAN = false, bool GATHER = false>
-__global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK_) ? 3 : 2) : VA * VB == 16 ? 5 : 4) void gemm_split_kernel(const GemmArgs args) {
+template <int VA, bool AK, int VB, bool BK_, bool MASKED, int TILE, bool FAN = false, bool GATHER = false, int WAVES = 4>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (VA * VB == 16 && (AK || BK_) ? 3 : 2) : VA * VB == 16 ? 5 : 4) void gemm_split_kernel(const GemmArgs args) {
     constexpr int BM = TILE, BN = TILE;
-    constexpr int WT = TILE / 2;   // edge of a wave's block (waves are arranged 2 x 2)
-    constexpr int NB = WT / 32;    // 32 x 32 MFMA tiles per wave and dimension
-    typedef TileLayout<MASKED ? VA : 4, AK, TILE> LA;
-    typedef TileLayout<MASKED ? VB : 4, BK_, TILE> LB;
+    constexpr int NT = 64 * WAVES;
+    static_assert(WAVES == 4 || !MASKED, "the masked loader is for four waves");
+    constexpr int WM = TILE / 2, WN = 2 * TILE / WAVES;  // a wave's block (waves are arranged 2 x 2 or 2 x 4)
+    constexpr int NBM = WM / 32, NBN = WN / 32;          // 32 x 32 MFMA tiles per wave and dimension
+    typedef TileLayout<MASKED ? VA : 4, AK, TILE, NT> LA;
+    typedef TileLayout<MASKED ? VB : 4, BK_, TILE, NT> LB;
     __shared__ uint4 lds[LA::UNITS + LB::UNITS];
     uint4 *const lds_a = lds, *const lds_b = lds + LA::UNITS;
 
@@ -499,11 +502,11 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
     // (a split left without k lines by a short list still has its partial product to write)
     if (it_begin >= it_end && !(GATHER && args.epilogue == EPI_PARTIAL)) return;
 
-    f32x16 acc[NB][NB];
+    f32x16 acc[NBM][NBN];
 #pragma unroll
-    for (int i = 0; i < NB; ++i)
+    for (int i = 0; i < NBM; ++i)
 #pragma unroll
-        for (int j = 0; j < NB; ++j)
+        for (int j = 0; j < NBN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
@@ -531,19 +534,19 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
             lds_only_barrier();
 #pragma unroll
             for (int s = 0; s < BK / 16; ++s) {
-                bf16x8 fa[NB][3], fb[NB][3];
+                bf16x8 fa[NBM][3], fb[NBN][3];
 #pragma unroll
-                for (int i = 0; i < NB; ++i) LA::fragment(lds_a, wm * WT + i * 32 + frag_row, 2 * s + half, fa[i]);
+                for (int i = 0; i < NBM; ++i) LA::fragment(lds_a, wm * WM + i * 32 + frag_row, 2 * s + half, fa[i]);
 #pragma unroll
-                for (int j = 0; j < NB; ++j) LB::fragment(lds_b, wn * WT + j * 32 + frag_row, 2 * s + half, fb[j]);
+                for (int j = 0; j < NBN; ++j) LB::fragment(lds_b, wn * WN + j * 32 + frag_row, 2 * s + half, fb[j]);
                 // h*l, l*h, m*m, h*m, m*h, h*h: the small terms first
                 constexpr int QA[6] = {0, 2, 1, 0, 1, 0}, QB[6] = {2, 0, 1, 1, 0, 0};
 #pragma unroll
                 for (int t = 0; t < 6; ++t)
 #pragma unroll
-                    for (int i = 0; i < NB; ++i)
+                    for (int i = 0; i < NBM; ++i)
 #pragma unroll
-                        for (int j = 0; j < NB; ++j)
+                        for (int j = 0; j < NBN; ++j)
                             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j][QB[t]], fa[i][QA[t]], acc[i][j], 0, 0, 0);
             }
             lds_only_barrier();
@@ -560,10 +563,10 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
     };
     if constexpr (GATHER) {
         static_assert(VA == 4 && VB == 4 && !AK && !BK_ && !MASKED, "the gathering loader is for two row-contiguous operands");
-        GatherStage<TILE> ga, gb;
+        GatherStage<TILE, NT> ga, gb;
         ga.init(m0, args.m, tid);
         gb.init(n0, args.n, tid);
-        constexpr int NL = GatherStage<TILE>::NLOAD;
+        constexpr int NL = GatherStage<TILE, NT>::NLOAD;
         const int *__restrict__ order = args.k_order + k_lo;
         const int k_shift = pb.k_shift;
         const unsigned a_line = (unsigned)(args.lda * sizeof(float)), b_line = (unsigned)(args.ldb * sizeof(float));
@@ -576,7 +579,7 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
             for (int p = 0; p < NL; ++p) idx[p] = order[max(min(tile * BK + ga.kk + p, k_extent - 1), 0)] + k_shift;
         };
         lines_of(kin);
-        auto fetch_next = [&](GatherStage<TILE> &qa, GatherStage<TILE> &qb) __attribute__((always_inline)) {
+        auto fetch_next = [&](GatherStage<TILE, NT> &qa, GatherStage<TILE, NT> &qb) __attribute__((always_inline)) {
             const int kv = min(BK, k_extent - kin * BK);
             qa.load(pa, a_line, idx, kv);
             qb.load(pbb, b_line, idx, kv);
@@ -607,14 +610,14 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
     } else {
         // the tile cursor: operand pair `seg`, k tile `kin` inside it; the operands' base pointers are looked up only
         // when the pair changes
-        FastStage<VA == 4, AK, TILE> sa;
-        FastStage<VB == 4, BK_, TILE> sb;
+        FastStage<VA == 4, AK, TILE, NT> sa;
+        FastStage<VB == 4, BK_, TILE, NT> sb;
         sa.init(args.lda, m0, args.m, tid);
         sb.init(args.ldb, n0, args.n, tid);
         int seg = it_begin / kt_per_seg, kin = it_begin % kt_per_seg, left = it_end - it_begin - 1;
         const float *pa = pb.A[seg], *pbb = pb.B[seg];
         const size_t ka = AK ? 1 : (size_t)args.lda, kb = BK_ ? 1 : (size_t)args.ldb;  // floats per k step
-        auto fetch_next = [&](FastStage<VA == 4, AK, TILE> &qa, FastStage<VB == 4, BK_, TILE> &qb) __attribute__((always_inline)) {
+        auto fetch_next = [&](FastStage<VA == 4, AK, TILE, NT> &qa, FastStage<VB == 4, BK_, TILE, NT> &qb) __attribute__((always_inline)) {
             qa.load(pa + (size_t)kin * BK * ka, args.k - kin * BK, tid);
             qb.load(pbb + (size_t)kin * BK * kb, args.k - kin * BK, tid);
             if (left > 0) {
@@ -630,16 +633,16 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
 
     // what came out infinite or not a number is formed again (plain_sums)
 #pragma unroll
-    for (int i = 0; i < NB; ++i)
+    for (int i = 0; i < NBM; ++i)
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
+        for (int j = 0; j < NBN; ++j) {
             bool finite = true;
 #pragma unroll
             for (int r = 0; r < 16; ++r) finite = finite && __builtin_fabsf(acc[i][j][r]) <= lim::kMax;
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] *= 1.0f / (kSplitScale * kSplitScale);
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(!finite) != 0, 0))
-                acc[i][j] = plain_sums<AK, BK_, MASKED, GATHER>(args, pb, m0 + wm * WT + 32 * i, n0 + wn * WT + 32 * j, lane, it_begin,
+                acc[i][j] = plain_sums<AK, BK_, MASKED, GATHER>(args, pb, m0 + wm * WM + 32 * i, n0 + wn * WN + 32 * j, lane, it_begin,
                                                                 it_end, kt_per_seg, k_extent, k_lo);
         }
 
@@ -671,14 +674,14 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
         float *__restrict__ P = args.partial + (size_t)split_id * args.partial_stride +
                                 (size_t)prob_id * args.m * args.n;
 #pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            const int m = m0 + wm * WT + i * 32 + frag_row;
+        for (int i = 0; i < NBM; ++i) {
+            const int m = m0 + wm * WM + i * 32 + frag_row;
             if (m >= args.m) continue;
 #pragma unroll
-            for (int j = 0; j < NB; ++j) {
+            for (int j = 0; j < NBN; ++j) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int n = n0 + wn * WT + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+                    const int n = n0 + wn * WN + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
                     if (n < args.n) P[(size_t)n * args.m + m] = acc[i][j][r];
                 }
             }
@@ -689,16 +692,16 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
         // All loads of a 32 x 32 tile's sixteen values per lane are issued before anything is stored: the compiler
         // cannot know that the buffers do not overlap and would otherwise wait for memory once per value.
 #pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            const int m = m0 + wm * WT + i * 32 + frag_row;
+        for (int i = 0; i < NBM; ++i) {
+            const int m = m0 + wm * WM + i * 32 + frag_row;
 #pragma unroll
-            for (int j = 0; j < NB; ++j) {
+            for (int j = 0; j < NBN; ++j) {
                 size_t idx[16];
                 bool ok[16];
                 float e[16], old[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int n = n0 + wn * WT + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+                    const int n = n0 + wn * WN + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
                     ok[r] = m < args.m && n < args.n;
                     idx[r] = ok[r] ? (size_t)n * args.ldc + m : 0;
                     old[r] = (ok[r] && pb.aux_in) ? pb.aux_in[idx[r]] : 0.0f;
@@ -729,14 +732,14 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
     const float *const old = args.epilogue == EPI_STORE_DELTA || args.epilogue == EPI_CONTEXT ? pb.aux_in
                                         : args.epilogue == EPI_ADD ? C : nullptr;
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-        const int m = m0 + wm * WT + i * 32 + frag_row;
+    for (int i = 0; i < NBM; ++i) {
+        const int m = m0 + wm * WM + i * 32 + frag_row;
         if (m >= args.m) continue;
         float bterm = 0.0f;
         if (args.epilogue == EPI_BIAS_ACT || args.epilogue == EPI_BIAS_ACT_SKIP)
             bterm = args.bias_scale * pb.bias_vec[m];
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
+        for (int j = 0; j < NBN; ++j) {
             // What the sums meet in memory is requested for sixteen of them at a time: the compiler cannot know that it does not
             // overlap the output and would wait for one load per sum (a dense layer's deltas in the epilogue of the product above
             // it: the feed-forward model's pass, four such products, 2260 -> 2183 us).
@@ -744,13 +747,13 @@ __global__ __launch_bounds__(NTHREADS, TILE == 128 ? (VA * VB == 16 && (AK || BK
             if (old) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int n = min(n0 + wn * WT + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3), args.n - 1);
+                    const int n = min(n0 + wn * WN + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3), args.n - 1);
                     met[r] = old[(size_t)n * args.ldc + m];
                 }
             }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int n = n0 + wn * WT + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+                const int n = n0 + wn * WN + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
                 if (n >= args.n) continue;
                 const size_t idx = (size_t)n * args.ldc + m;
                 float *dst = C + idx;
@@ -790,7 +793,9 @@ void launch_t(const GemmArgs &a, dim3 grid, hipStream_t s, int tile) {
         }
     } else if (a.k_order) {
         if constexpr (VA == 4 && !AK && VB == 4 && !BK_) {
-            if (tile == 128)
+            if (tile == kEightWaves)
+                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128, false, true, 8>), grid, dim3(2 * NTHREADS), 0, s, a);
+            else if (tile == 128)
                 hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128, false, true>), grid, dim3(NTHREADS), 0, s, a);
             else
                 hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64, false, true>), grid, dim3(NTHREADS), 0, s, a);
@@ -798,7 +803,9 @@ void launch_t(const GemmArgs &a, dim3 grid, hipStream_t s, int tile) {
     } else if (a.masked) {
         hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, true, 64>), grid, dim3(NTHREADS), 0, s, a);
     } else if constexpr (VA != 2 && VB != 2) {
-        if (tile == 128) hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128>), grid, dim3(NTHREADS), 0, s, a);
+        if (tile == kEightWaves)
+            hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128, false, false, 8>), grid, dim3(2 * NTHREADS), 0, s, a);
+        else if (tile == 128) hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128>), grid, dim3(NTHREADS), 0, s, a);
         else hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64>), grid, dim3(NTHREADS), 0, s, a);
     }
 }

@@ -22,6 +22,42 @@ def test_matrix_product(m, n, k, tA, tB, acc):
     assert PC.run_gemm_case(m, n, k, tA, tB, acc, seed=m + n + k) < TOL
 
 
+# Launches whose last level of large tiles is full enough for eight waves per tile: 212 to 256 tiles, two levels, four levels; edges
+# and ends of k that are no multiple of the tile, of four, of a vector.  Tolerance: k products of six parts each in steps of sixteen,
+# 6 k / 16 roundings of 2^-24 of the sum so far: sqrt(6 * 2050 / 16) * 2^-24 = 1.7e-6.
+@pytest.mark.parametrize("m,n,k,tA,tB,acc", [
+    (1000, 3460, 385, 0, 0, 0), (1000, 3460, 388, 1, 0, 1), (2040, 1793, 384, 1, 0, 0), (128, 27300, 420, 0, 0, 0), (1020, 6100, 900, 1, 0, 0),
+    (1018, 6101, 769, 0, 0, 1), (1024, 15900, 387, 1, 0, 0), (1021, 3300, 2050, 0, 0, 0),
+])
+def test_matrix_product_on_eight_waves(m, n, k, tA, tB, acc):
+    import torch
+
+    print("gemm case on eight waves", m, n, k, tA, tB, acc, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    A, B, C = (torch.randn(c, device="cuda", generator=gen) for c in (m * k, k * n, m * n))
+    want = B.double().reshape(n, k) @ (A.double().reshape(m, k).T if tA else A.double().reshape(k, m)).contiguous()
+    if acc:
+        want += C.double().reshape(n, m)
+    PC.pkg().capi.matrix_product(C, m, n, k, A, tA, B, tB, acc)
+    assert ((C.double().reshape(n, m) - want).norm() / want.norm()).item() < 2e-6
+
+
+# The weight gradients that take eight waves: one wide dense layer (with its bias gradient), tiles at the output's edges, slots that
+# are no multiple of the tile.  Tolerance as above: at most 1600 slots per split, 1.5e-6.
+@pytest.mark.parametrize("P,D,N", [(1024, 1024, 6200), (1000, 1022, 6401), (1300, 900, 6163)])
+def test_wide_dense_gradient_on_eight_waves(P, D, N):
+    import torch
+
+    print("wide dense gradient", P, D, N, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(P + D + N)
+    x, e = torch.randn(N * P, device="cuda", generator=gen), torch.randn(N * D, device="cuda", generator=gen)
+    W, y = torch.zeros(P * D + D, device="cuda"), torch.zeros(N * D, device="cuda")
+    updates, below = torch.full((P * D + D,), 3.0, device="cuda"), torch.zeros(N * P, device="cuda")
+    want = torch.cat([(e.double().reshape(N, D).T.contiguous() @ x.double().reshape(N, P)).reshape(-1), 0.5 * e.double().reshape(N, D).sum(0)])
+    PC.pkg().capi.dense_backward(P, D, N, 0, 0.5, W, x, y, e, below, updates)
+    assert ((updates.double() - want).norm() / want.norm()).item() < 3e-6
+
+
 def test_matrix_product_rejects_double_transpose():
     import torch
 
