@@ -1651,6 +1651,9 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         return C.fold_ok && block_at(i - 3) && C.N == sk.N && closing.N == sk.N && cnn_foldable(C.cnn, closing.size) &&
                (C.delta_fused || !C.cnn_tanh) && aligned(net->weights + C.w_off) && aligned(C.err) && aligned(closing.eskip);
     };
+    std::vector<char> in_block(net->layers.size(), 0);  // weight gradients in the blocks' common launches
+    for (size_t i = 5; i < net->layers.size(); ++i)
+        if (block_at(i) && block_weights_at(net, i)) in_block[i] = in_block[i - 3] = in_block[i - 4] = in_block[i - 5] = 1;
     std::vector<size_t> pending;
     auto weight_half = [&](size_t i, hipStream_t ws) -> int {
         NetLayer &L = net->layers[i];
@@ -1764,7 +1767,15 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
             g = &groups.back();
         }
         g->layers.push_back(i);
-        if ((int)g->layers.size() >= g->cap) CNT_TRY(hand_over_group(*g));
+        // no layer further down will join: nothing to wait for (a short waveform's output layers, three launches of 17 us, used
+        // to run behind the error chain instead of beside it)
+        bool more = false;
+        for (size_t j = i - 1; j >= 1 && !more; --j) {
+            const NetLayer &o = net->layers[j];
+            more = !in_block[j] && o.kind == L.kind && o.N == L.N && o.size == L.size &&
+                   (L.kind == K_DENSE ? net->layers[j - 1].size == a : L.kind == K_CNN || o.ctx_dim == b);
+        }
+        if (!more || (int)g->layers.size() >= g->cap) CNT_TRY(hand_over_group(*g));
         // a network of many small layers that do not share shapes: do not let all of them wait for the pass's end
         size_t waiting = 0;
         for (const ShapeGroup &c : groups) waiting += c.layers.size();
@@ -1773,7 +1784,6 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         return CNT_OK;
     };
     // Weight gradients of residual blocks, eight blocks to a launch
-    std::vector<char> weights_done(net->layers.size(), 0);
     std::vector<size_t> blocks;  // their skip 1x1 layers
     auto hand_over_blocks = [&]() -> int {
         if (blocks.empty()) return CNT_OK;
@@ -1810,7 +1820,6 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                 CNT_TRY(hand_over_blocks());
         }
         blocks.push_back(i);
-        for (size_t k : {i, i - 3, i - 4, i - 5}) weights_done[k] = 1;
         return blocks.size() == kBlockGradients ? hand_over_blocks() : CNT_OK;
     };
     // the side buffers that a launch of skip layer `from` adds to: the next forward pass clears them
@@ -1893,7 +1902,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                             direct_from[i - 8] = prev_err;
                         }
                         const bool fan_live = block_fan.n > 0 || block_fan.from_skip;
-                        const bool together = block_weights_at(net, i);
+                        const bool together = in_block[i] != 0;
                         if (block_fan.n > 0) adds_to_side(prev);
                         CNT_TRY(wavenet_block_errors(stream, prev.size, L.size, N, L.pat, W, net->weights + out.w_off, L.err,
                                                      prev_err, fan_live ? &block_fan : nullptr,
@@ -1977,7 +1986,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                     }
                 }
             weight_half_of_layer:
-                if (weights_done[i] || (L.kind == K_WAVNETC && L.ctx_dim == 0)) break;
+                if (in_block[i] || (L.kind == K_WAVNETC && L.ctx_dim == 0)) break;
                 if (!net->overlap) {
                     CNT_TRY(weight_half(i, stream));
                     break;
