@@ -93,7 +93,8 @@ inline bool eight_waves(long tiles, long run) {
 // Elsewhere, 64 x 64 or 128 x 128 on four waves.  Between 256 and 383 values the large tile pays where it fills the last generation
 // of 768 to nine tenths: 64 / 128, us, for 1024 rows and a k-contiguous A: 752 tiles (0.98) 54 / 49, 704 (0.92) 1.05 times as fast,
 // 1360 (0.89) 1.02, 2000 (0.87) 0.97, 640 (0.83) 1.04, 1040 (0.68) 0.87; k = 192 no gain anywhere.  With 768 values and more: the
-// large tile from 336 tiles on, where the small ones begin a second generation (1280 of them at a time); times as fast with 304 / 320 / 336 / 400 / 600 / 768 / 800 / 1040 large tiles
+// large tile from 336 tiles on, where the small ones begin a second generation (1280 of them at a time); times as fast with 304 /
+// 320 / 336 / 400 / 600 / 768 / 800 / 1040 large tiles
 // (least and most over 512, 1024 and 2048 rows and both orders of A): k = 768 0.84-0.87 / 0.86-0.89 / 1.00-1.04 / 1.08-1.13 / 1.04 /
 // 1.23-1.25 / 0.97-0.99 / 1.10-1.12, k = 3072 0.95-1.01 / 0.96-1.02 / 1.12-1.18 / 1.22-1.28 / 1.12 / 1.32-1.35 / 1.06 / 1.17-1.20.  Lines
 // of odd length (loads of single values at the edges): from 600 tiles and 512 values on.

@@ -410,7 +410,8 @@ __global__ __launch_bounds__(256) void wavenet_block_weights_sum_kernel(const Ta
 
 bool wavenet_block_weights_supported(int R, int K, int C, long N) {
     // (32-bit byte offsets, one window of shifts ahead of the first slot and a few tiles behind the last)
-    return (N + 8 * kTallDepth) * std::max({2 * R, K, C}) * (long)sizeof(float) < (1L << 30) && R >= 4 && R <= 64 && R % 4 == 0 && K >= 4 && K <= 256 && K % 4 == 0 && C >= 4 && C <= 128;
+    return (N + 8 * kTallDepth) * std::max({2 * R, K, C}) * (long)sizeof(float) < (1L << 30) && R >= 4 && R <= 64 && R % 4 == 0 &&
+           K >= 4 && K <= 256 && K % 4 == 0 && C >= 4 && C <= 128;
 }
 
 size_t wavenet_block_weights_scratch() { return (size_t)kTallWorkgroups * (kTallBlocks * 1024 + 256); }

@@ -15,14 +15,14 @@ pytestmark = pytest.mark.gpu
 TOL = 2e-6
 
 
-def gradient_errors(capi, specs, blocks, R, K, C, lengths, seed=1, spike=None):
-    """2-norm errors of every gradient of every block, and the gradients themselves"""
+def passed_network(capi, specs, blocks, R, K, C, lengths, seed=1, spike=None, overlap=True):
+    """A stack after one forward and one backward pass, its conditioning features and the mask of its valid slots"""
     import torch
 
     S, T = len(lengths), max(lengths)
     N, Q = S * T, 16
     gen = torch.Generator(device="cuda").manual_seed(seed)
-    net = capi.Network(json.dumps(specs.wavenet_network_doc(blocks, Q, R, K, C, 0, 4)), S, T, mdn_config=[1, 0, Q, 0, 1, -1])
+    net = capi.Network(json.dumps(specs.wavenet_network_doc(blocks, Q, R, K, C, 0, 4)), S, T, mdn_config=[1, 0, Q, 0, 1, -1], overlap=overlap)
     net.weights.copy_(torch.empty(net.n_weights, device="cuda").uniform_(-0.1, 0.1, generator=gen))
     t = torch.arange(T, device="cuda")[:, None]
     valid = t < torch.tensor(lengths, device="cuda")
@@ -37,7 +37,16 @@ def gradient_errors(capi, specs, blocks, R, K, C, lengths, seed=1, spike=None):
     net.forward()
     net.backward()
     torch.cuda.synchronize()
+    return net, ctx, valid
 
+
+def gradient_errors(capi, specs, blocks, R, K, C, lengths, seed=1, spike=None, overlap=True):
+    """2-norm errors of every gradient of every block, and the gradients themselves"""
+    import torch
+
+    net, ctx, valid = passed_network(capi, specs, blocks, R, K, C, lengths, seed, spike, overlap)
+    S, T = len(lengths), max(lengths)
+    N = S * T
     live = valid.reshape(-1, 1)
     of = lambda name, what: net.layer(name)[what].reshape(N, -1).double()  # noqa: E731
     errors, got = {}, {}
@@ -90,9 +99,32 @@ def test_block_weight_gradients(blocks, R, K, C, lengths):
     assert all(bool((first[n] == again[n]).all()) for n in first)  # the order of all additions is fixed
 
 
-def test_block_weight_gradients_of_the_largest_values():
+@pytest.mark.parametrize("overlap", [True, False])
+def test_block_weight_gradients_of_the_largest_values(overlap):
     """A conditioning feature of 3e38: its split has an infinite part, its gate is flat, so that the gradients stay what they are."""
     pkg = PC.pkg()
-    errors, got = gradient_errors(pkg.capi, pkg.specs, 2, 64, 128, 80, [200, 170], spike=(77, 41, 3e38))
+    errors, got = gradient_errors(pkg.capi, pkg.specs, 2, 64, 128, 80, [200, 170], spike=(77, 41, 3e38), overlap=overlap)
     assert all(np.isfinite(v.cpu().numpy()).all() for v in got.values())
     assert max(errors.values()) < TOL, errors
+
+
+def test_block_weight_gradients_under_capture():
+    """A forward and a backward pass recorded once: every replay gives the eager passes' gradients, bit for bit."""
+    import torch
+
+    pkg = PC.pkg()
+    net, ctx, _ = passed_network(pkg.capi, pkg.specs, 9, 64, 128, 20, [300, 211])
+    want = net.updates.clone()
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+        net.forward(stream=stream)
+        net.backward(stream=stream)
+    for _ in range(3):
+        net.updates.fill_(5.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool((net.updates == want).all())
+    net.close()
