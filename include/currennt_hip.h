@@ -77,15 +77,14 @@ int cnt_dense_backward(void *stream, int P, int D, int N, int act, float bias, c
  * half (delta in place, prev_err) is what the next layer's backward waits for; the weight half
  * (weight_updates from x and the deltas) has no consumer before the optimizer.  The reference has no such
  * split; calling both in this order on one stream is cnt_dense_backward.
- * Device memory: the weight half of a narrow layer over a long input (P*D up to 64 K floats, N in the thousands)
- * sums split partial products through a scratch buffer of 16 MB per stream, which the library allocates the first
- * time such a product runs on a stream and keeps; the same holds for cnt_cnn_backward_weights and
- * cnt_wavnetc_backward_weights.  Apart from that, only the *_create calls allocate. */
+ * Device memory: a weight half whose sum over the slots is cut into parts adds the parts up through a scratch buffer of 36 MB per
+ * stream, which the library allocates the first time such a product runs on a stream and keeps; the same holds for
+ * cnt_cnn_backward_weights and cnt_wavnetc_backward_weights.  Apart from that, only the *_create calls allocate. */
 int cnt_dense_backward_errors(void *stream, int P, int D, int N, int act, const float *weights, const float *y,
                               float *err, float *prev_err);
 int cnt_dense_backward_weights(void *stream, int P, int D, int N, float bias, const float *x, const float *err,
                                float *weight_updates);
-/* The scratch buffer of `stream` for those split products (16 MB of device memory), allocated now instead of
+/* The scratch buffer of `stream` for those split products (36 MB of device memory), allocated now instead of
  * inside the first product that wants it, and freed again (the stream must be idle).  No counterpart in the
  * reference, whose cuBLAS handle owns its workspace.  A product that finds no buffer and cannot get one (out of
  * memory, a stream under capture) adds its splits atomically instead. */

@@ -236,8 +236,8 @@ struct GemmArgs {
     const char *pat;  // masked mode and the *_SKIP / CONTEXT epilogues
     GemmProblem prob[kGemmMaxProb];
     const char *label;  // name under which the launch is timed when profiling is on (may be NULL)
-    // Split-K products with a small output (EPI_ATOMIC, splitk = 0): `overwrite_ok` allows gemm_plan to choose
-    // EPI_PARTIAL, which overwrites C instead of adding to a cleared C.  With `rowsum` (one operand pair, unmasked)
+    // Split-K products (EPI_ATOMIC, splitk = 0): `overwrite_ok` allows gemm_plan to choose EPI_PARTIAL, or EPI_STORE for a single
+    // split, which overwrite C instead of adding to a cleared C.  With `rowsum` (one operand pair, unmasked)
     // the same pass also sums every problem's B operand over k into that problem's rowsum_out -- the bias gradient
     // of a dense layer; with EPI_ATOMIC it adds to what the caller has cleared.  gemm_plan clears `rowsum` where the
     // product cannot bring it along (operands that are not row-contiguous, several pairs).
@@ -247,7 +247,7 @@ struct GemmArgs {
     float *const *fan_targets;
     const int *fan_is_skip;
     float *partial;        // scratch of splitk * partial_stride floats: the stream's buffer (set by gemm_plan) or the caller's
-    size_t partial_stride;  // floats per split: nprob * m * n (+ nprob * n with rowsum)
+    size_t partial_stride;  // floats per split: nprob * m * n (+ nprob * n with rowsum), rounded up to a multiple of four
     int xcd_map;            // set by gemm_launch: workgroups pick their tile by XCD (gemm_kernel.hpp)
     // A product over the slots of a fraction (weight gradients) that leaves the padding slots out (both in device memory,
     // or both NULL): only the k lines k_order[lo .. lo + n) of the operands are read, the others being all zero in at least
@@ -259,8 +259,8 @@ struct GemmArgs {
     const int *k_count;
 };
 
-// Resolves splitk = 0 (chosen by the launcher) and, where the arguments allow it and it pays, switches an
-// EPI_ATOMIC product to EPI_PARTIAL.  A caller that needs to know whether C must be cleared first calls this
+// Resolves splitk = 0 (chosen by the launcher) and, where the arguments allow it, switches an
+// EPI_ATOMIC product to EPI_PARTIAL or EPI_STORE.  A caller that needs to know whether C must be cleared first calls this
 // before gemm_launch and looks at args.epilogue; gemm_launch calls it for everyone else.
 void gemm_plan(GemmArgs &args, hipStream_t stream);
 // The kernel for products that are too small for the tiled one (gemm_direct.hip): whether these arguments take it (masked
@@ -398,6 +398,9 @@ bool cnn_batch_compatible(const cnt_cnn *a, const cnt_cnn *b);
 int cnn_backward_weights_batch(cnt_cnn *const *h, int count, hipStream_t stream, const char *patTypes, int curT,
                                const float *const *x, const float *const *output_errors, float *const *weight_updates,
                                const float *const *colsum_partial = nullptr, const int *colsum_rows = nullptr);
+
+// whether the stream is being captured; a stream that cannot be asked (the null stream beside a capture) counts as captured
+bool capturing(hipStream_t stream);
 
 // ----- small streaming kernels (elementwise.hip) ----------------------------------------------------
 int fill_zero(hipStream_t stream, float *p, size_t count);

@@ -383,9 +383,10 @@ extern "C++" int cnt::dense_backward_weights_batch(hipStream_t stream, int P, in
         ga.k_count = order->count;
     }
     ga.label = "gemm:dense_dW";
-    // narrow layers: the launcher sums partial products instead of adding atomically, which overwrites the weight part.  The
-    // bias part (row sums of the errors) comes along either way: a column sum behind the atomic product cost 11 us at
-    // 256 x 1936 over 6000 slots (the model with that mixture layer 211 -> 201 us) and 34 us at 1024 x 1024 over 12 000.
+    // The launcher sums partial products in a fixed order, which overwrites the updates; it adds atomically, to updates that are cleared
+    // here, only where it has no scratch (gemm.hip).  The bias part (row sums of the errors) comes along either way: a column sum behind
+    // the atomic product cost 11 us at 256 x 1936 over 6000 slots (the model with that mixture layer 211 -> 201 us) and 34 us at
+    // 1024 x 1024 over 12 000.
     ga.overwrite_ok = 1;
     ga.rowsum = 1;
     gemm_plan(ga, stream);

@@ -150,14 +150,18 @@ int pick_tile(const GemmArgs &a) {
 }
 
 // ----- split-K through partial products ---------------------------------------------------------------------
-// Weight gradients of narrow layers over long inputs (a 64 x 128 output summed over 32 000 slots) need a few
-// hundred splits to fill the machine, and with the atomic epilogue every output element then receives a few
-// hundred atomic adds; atomics to one address serialise, and they, not the loads, set the run time of such a
-// launch.  Here every split stores its partial product with plain stores into a scratch buffer and a second,
-// small kernel sums the splits into C.  That also replaces the clearing launch in front of the atomic path and,
-// for dense layers, the separate column sum for the bias gradient (the splits carry the row sums of B along).
-constexpr size_t kSplitScratchFloats = (size_t)4 << 20;  // 16 MB per (device, stream)
-constexpr long kPartialMaxOutput = 128 << 10;            // floats of output (all problems) up to which it pays
+// Weight gradients sum over all slots of a fraction, so their products are cut along k, and the splits' sums have to meet.  Every
+// split stores its partial product with plain stores into a scratch buffer and a second, small kernel adds the splits up in a fixed
+// order, the row sums of B (a dense layer's bias gradient) with them.  Nothing has to be cleared and nothing is added atomically.
+// Outputs of a few hundred splits (64 x 128 summed over 32 000 slots) would be bound by their atomic additions.  Wide outputs of a
+// few splits take as long either way (five 1024 x 1024 layers over 10 000 slots: pass 2104 us with a clear and atomic additions,
+// 2112 so, of 33 MB of partial products a layer; the model with mixture outputs 191 and 189), but a clear in front of atomic
+// additions has once been seen to take a split's additions with it: on one run the bias gradient of a 1024 x 1028 layer came out
+// without its first split's share.  Nothing in the launches' order explains it, so weight gradients of dense, convolution and
+// conditioning layers no longer rest on it, and they are the same bits in every call.
+constexpr size_t kSplitScratchFloats = (size_t)9 << 20;  // 36 MB per (device, stream): kWideGradientGroups large tiles, and their row sums
+constexpr long kManySplits = 8;                          // from here on, and up to kFewOutputs sums, eight threads share a sum's splits
+constexpr long kFewOutputs = 128 << 10;
 
 struct SplitScratch {
     int device;
@@ -260,6 +264,53 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs args)
     }
 }
 
+// Outputs large enough to fill the chip with a thread per four neighbouring sums, or with few splits: a thread adds up all splits of
+// its sums, eight loads in flight.
+constexpr int kReduceThreads = 256;
+__global__ __launch_bounds__(kReduceThreads) void splitk_reduce_quads_kernel(const GemmArgs args) {
+    const size_t mn = (size_t)args.m * args.n;
+    const size_t products = mn * args.nprob;
+    const size_t total = products + (args.rowsum ? (size_t)args.n * args.nprob : 0);
+    const size_t e = 4 * ((size_t)blockIdx.x * kReduceThreads + threadIdx.x);
+    if (e >= total) return;
+    const float4 *__restrict__ p = reinterpret_cast<const float4 *>(args.partial + e);
+    const size_t st = args.partial_stride / 4;  // (a multiple of four floats, so that every split's quads are aligned)
+    const auto add = [](const float4 &x, const float4 &y) { return float4{x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w}; };
+    float4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    int s = 0;
+    for (; s + 8 <= args.splitk; s += 8) {
+        float4 x[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) x[q] = p[(size_t)(s + q) * st];
+        v = add(v, add(add(add(x[0], x[1]), add(x[2], x[3])), add(add(x[4], x[5]), add(x[6], x[7]))));
+    }
+    for (; s + 2 <= args.splitk; s += 2) {
+        const float4 x = p[(size_t)s * st], y = p[(size_t)(s + 1) * st];
+        v = add(v, add(x, y));
+    }
+    if (s < args.splitk) v = add(v, p[(size_t)s * st]);
+    const size_t z = e / mn, r = e - z * mn;
+    if (e + 4 <= products && r + 4 <= mn && args.ldc == args.m) {
+        float *const to = args.prob[z].C + r;
+        if ((reinterpret_cast<uintptr_t>(to) & 15) == 0) {
+            *reinterpret_cast<float4 *>(to) = v;
+            return;
+        }
+    }
+    const float x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const size_t at = e + i;
+        if (at < products) {
+            const size_t zi = at / mn, ri = at % mn;
+            args.prob[zi].C[(ri / args.m) * args.ldc + ri % args.m] = x[i];
+        } else if (at < total) {
+            const size_t zi = (at - products) / args.n, j = (at - products) % args.n;
+            args.prob[zi].rowsum_out[j] = args.prob[zi].rowsum_scale * x[i];
+        }
+    }
+}
+
 }  // namespace
 
 bool gemm_fan_supported(const GemmArgs &a) {
@@ -289,6 +340,13 @@ int gemm_scratch_buffers() {
     return (int)g_split_scratch.size();
 }
 
+namespace {
+// floats of a split's partial products and row sums, a multiple of four
+size_t partial_stride(const GemmArgs &a) {
+    return ((size_t)a.m * a.n * a.nprob + (a.rowsum ? (size_t)a.n * a.nprob : 0) + 3) / 4 * 4;
+}
+}  // namespace
+
 void gemm_plan(GemmArgs &args, hipStream_t stream) {
     if (args.splitk != 0) return;
     if (direct_product(args)) {
@@ -304,8 +362,8 @@ void gemm_plan(GemmArgs &args, hipStream_t stream) {
     // ranges.
     // Outputs of one or two tiles per problem (the WaveNet layers' 64 x 64 ... 80 x 128 weights) take twice the
     // workgroups: measured on MI355X next to the error chain of the same pass, 1024 workgroups end the stack's backward
-    // pass 4% sooner than 512, and 1536 or more (where the partial products no longer fit the scratch buffer and the
-    // launch adds atomically) 4-8% later; the acoustic model's wide outputs are best at 768 (2.249 / 2.232 / 2.219 / 2.246 /
+    // pass 4% sooner than 512, and 1536 or more (whose partial products did not fit the scratch buffer of then, so that the
+    // launch added atomically) 4-8% later; the acoustic model's wide outputs are best at 768 (2.249 / 2.232 / 2.219 / 2.246 /
     // 2.243 ms at 512 / 640 / 768 / 896 / 1024 with the loader of constant offsets; they were best at 512 before it).
     static const int forced_target = [] { const char *e = std::getenv("CNT_GEMM_SPLIT_TARGET"); return e ? std::atoi(e) : 0; }();
     const long tiles = (long)((args.m + 63) / 64) * ((args.n + 63) / 64) * args.nprob;
@@ -320,20 +378,25 @@ void gemm_plan(GemmArgs &args, hipStream_t stream) {
         s = kLevelGradientGroups / large_tiles(args);
     s = std::min(s, std::max(1L, kt / 8));
     s = std::max(1L, s);
+    static const bool partial_on = [] { const char *e = std::getenv("CNT_GEMM_PARTIAL"); return !e || std::atoi(e) != 0; }();
+    const size_t stride = partial_stride(args);
+    const bool rowsum_ok = !args.rowsum || (args.nseg == 1 && !args.masked);
+    bool partial = partial_on && args.epilogue == EPI_ATOMIC && args.overwrite_ok && rowsum_ok;
+    if (partial) s = std::max(1L, std::min(s, (long)(kSplitScratchFloats / stride)));
     // no empty split: every split of the partial-product path has to write its share
     while (s > 1 && (s - 1) * ((kt + s - 1) / s) >= kt) --s;
     args.splitk = (int)s;
-    static const bool partial_on = [] { const char *e = std::getenv("CNT_GEMM_PARTIAL"); return !e || std::atoi(e) != 0; }();
-    const long out = (long)args.m * args.n * args.nprob;
-    const size_t stride = (size_t)out + (args.rowsum ? (size_t)args.n * args.nprob : 0);
-    const bool rowsum_ok = !args.rowsum || (args.nseg == 1 && !args.masked);
-    bool partial = partial_on && args.epilogue == EPI_ATOMIC && args.overwrite_ok && rowsum_ok && s >= 8 &&
-                   out <= kPartialMaxOutput && stride * (size_t)s <= kSplitScratchFloats;
+    const bool sums_with_store = !args.rowsum || (!args.a_kcontig && !args.b_kcontig);
+    if (partial && s == 1 && sums_with_store) {
+        args.epilogue = EPI_STORE;
+        return;
+    }
     if (partial && !args.partial) {
-        // the stream's scratch buffer: reserved by its owner, else allocated on first use; without one (allocation
-        // refused) the product adds atomically
+        // the stream's scratch buffer: reserved by its owner, else allocated on first use; without one (allocation refused, a
+        // stream under capture, whose graph may outlive a buffer that nobody has reserved) the product adds atomically
         std::lock_guard<std::mutex> lock(g_split_mu);
-        args.partial = split_scratch(stream);
+        args.partial = split_scratch_find(stream);
+        if (!args.partial && !capturing(stream)) args.partial = split_scratch(stream);
         partial = args.partial != nullptr;
     }
     if (partial) {
@@ -388,7 +451,7 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
         CNT_HIP(hipGetLastError());
         return CNT_OK;
     }
-    if (args.epilogue != EPI_PARTIAL && args.epilogue != EPI_ATOMIC) args.rowsum = 0;
+    if (args.epilogue != EPI_PARTIAL && args.epilogue != EPI_ATOMIC && args.epilogue != EPI_STORE) args.rowsum = 0;
     const int tile = pick_tile(args);
     const int edge = tile == kEightWaves ? 128 : tile;
     // a list of k lines is used where the kernel that reads through it exists, and ignored otherwise (the lines it leaves
@@ -416,8 +479,12 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
     CNT_HIP(hipGetLastError());
     if (args.epilogue == EPI_PARTIAL) {
         const size_t total = args.partial_stride;
-        hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((total + kReduceOutputs - 1) / kReduceOutputs)), dim3(256),
-                           0, stream, args);
+        if (args.splitk >= kManySplits && total <= (size_t)kFewOutputs)
+            hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((total + kReduceOutputs - 1) / kReduceOutputs)), dim3(256), 0,
+                               stream, args);
+        else
+            hipLaunchKernelGGL(splitk_reduce_quads_kernel, dim3((unsigned)((total / 4 + kReduceThreads - 1) / kReduceThreads)),
+                               dim3(kReduceThreads), 0, stream, args);
         CNT_HIP(hipGetLastError());
     }
     return CNT_OK;
@@ -427,10 +494,10 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
 // split-K product whose partial products go through the code object's own scratch array: no allocation at all.
 int gemm_dense_weights_static(hipStream_t stream, int P, int D, int N, float bias, const float *x, const float *err,
                               float *weight_updates) {
-    const size_t stride = (size_t)P * D + D;
+    const size_t sums = (size_t)P * D + D, stride = (sums + 3) / 4 * 4;
     CNT_REQUIRE(stride <= kStaticScratchFloats,
                 "dense_backward_weights_static: %d x %d weights + %d biases = %zu floats exceed the static scratch of %zu "
-                "floats; use cnt_dense_backward_weights", P, D, D, stride, kStaticScratchFloats);
+                "floats; use cnt_dense_backward_weights", P, D, D, sums, kStaticScratchFloats);
     float *buf = static_scratch();
     if (!buf) return CNT_ERR_HIP;
     GemmArgs ga = {};

@@ -494,13 +494,13 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (VA * VB
         else if (pb.k_trim == 2) k_extent -= args.k_count[2];
         k_extent = max(k_extent, 0);
     }
-    const int kt_per_seg = (k_extent + BK - 1) / BK;
-    const int total_it = kt_per_seg * args.nseg;
+    const int kt_per_seg = max((k_extent + BK - 1) / BK, 1);  // (1 where the list is empty: no k tile, and nothing divided by zero)
+    const int total_it = k_extent > 0 ? kt_per_seg * args.nseg : 0;
     const int per_split = (total_it + args.splitk - 1) / args.splitk;
     const int it_begin = split_id * per_split;
     const int it_end = min(total_it, it_begin + per_split);
-    // (a split left without k lines by a short list still has its partial product to write)
-    if (it_begin >= it_end && !(GATHER && args.epilogue == EPI_PARTIAL)) return;
+    // (a split left without k lines by a short list still has its zeros to write)
+    if (it_begin >= it_end && !(GATHER && args.epilogue != EPI_ATOMIC)) return;
 
     f32x16 acc[NBM][NBN];
 #pragma unroll
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (VA * VB
         const int *__restrict__ order = args.k_order + k_lo;
         const int k_shift = pb.k_shift;
         const unsigned a_line = (unsigned)(args.lda * sizeof(float)), b_line = (unsigned)(args.ldb * sizeof(float));
-        int seg = it_begin / kt_per_seg, kin = it_begin % kt_per_seg, left = it_end - it_begin - 1;
+        int seg = min(it_begin / kt_per_seg, args.nseg - 1), kin = it_begin % kt_per_seg, left = it_end - it_begin - 1;
         const float *pa = pb.A[seg], *pbb = pb.B[seg];
         // the k lines of the cursor's tile, loaded while the tile before it is being requested
         int idx[NL];
@@ -664,6 +664,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (VA * VB
                 if (args.epilogue == EPI_PARTIAL)
                     args.partial[(size_t)split_id * args.partial_stride + (size_t)args.nprob * args.m * args.n +
                                  (size_t)prob_id * args.n + n0 + tid] = s;
+                else if (args.epilogue == EPI_STORE)
+                    pb.rowsum_out[n0 + tid] = pb.rowsum_scale * s;
                 else
                     atomicAdd(pb.rowsum_out + n0 + tid, pb.rowsum_scale * s);
             }

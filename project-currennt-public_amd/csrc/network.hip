@@ -1366,18 +1366,19 @@ int cnt_network_load_sequences(cnt_network *net, void *stream_, int T, int Tmin,
 }  // extern "C"
 
 namespace cnt {
-namespace {
-
-bool fuse_blocks() {
-    static const bool on = [] { const char *e = std::getenv("CNT_NET_FUSE_BLOCKS"); return !e || std::atoi(e) != 0; }();
-    return on;
-}
 
 bool capturing(hipStream_t stream) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &capture) == hipSuccess) return capture != hipStreamCaptureStatusNone;
     (void)hipGetLastError();
     return true;
+}
+
+namespace {
+
+bool fuse_blocks() {
+    static const bool on = [] { const char *e = std::getenv("CNT_NET_FUSE_BLOCKS"); return !e || std::atoi(e) != 0; }();
+    return on;
 }
 
 // Fills memory that a call has just allocated and that keeps its content from then on.  Under capture the fill must not become

@@ -785,6 +785,58 @@ def test_bias_gradient_beside_atomic_sums(P, D, N):
     assert bool(((dW[:P * D].view(D, P) - want).abs() <= (N + 2) * 2.0 ** -24 * (err.double().abs().t() @ x.double().abs()))[:-1].all())
 
 
+# three, eight and twelve splits of 64 x 64 and 128 x 128 tiles; sums and bias gradients that end inside a quad; few outputs with few
+# splits; one split, which stores; a row of large tiles
+@pytest.mark.parametrize("P,D,N", [(1024, 1028, 653), (1024, 1024, 6200), (512, 514, 2501), (401, 603, 3001), (1026, 7, 1200), (37, 1, 2300),
+                                   (2048, 3072, 70), (2049, 3071, 300), (128, 8192, 9000)])
+def test_weight_gradient_is_the_same_in_every_call(P, D, N):
+    """The splits of a weight gradient meet in a fixed order: the same bits whatever the updates held before, within the bound
+    of fp32 sums in any order."""
+    import torch
+    print("weight gradient repeated", P, D, N, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(P + D + N)
+    x, err = torch.randn(N, P, device="cuda", generator=g), torch.randn(N, D, device="cuda", generator=g)
+    first = None
+    for before in (3.0, float("nan"), -1e30, 0.0):
+        dW = torch.full((P * D + D + 4,), before, device="cuda")
+        PC.pkg().capi.dense_backward_weights(P, D, N, 0.5, x, err, dW)
+        assert bool((dW[P * D + D:] == before).all()) or before != before and bool(dW[P * D + D:].isnan().all())
+        dW = dW[:P * D + D]
+        assert first is None or torch.equal(first, dW)
+        first = dW
+    want, size = err.double().t() @ x.double(), err.double().abs().t() @ x.double().abs()
+    assert bool(((first[:P * D].view(D, P) - want).abs() <= (N + 2) * 2.0 ** -24 * size).all())
+    assert bool(((first[P * D:] - 0.5 * err.double().sum(0)).abs() <= (N + 2) * 2.0 ** -24 * 0.5 * err.double().abs().sum(0)).all())
+
+
+@pytest.mark.parametrize("reserved", [True, False])
+def test_weight_gradient_under_capture(reserved):
+    """A captured product uses the stream's scratch where its owner has reserved one, and allocates none where not."""
+    import torch
+    P, D, N = 1024, 1028, 1300
+    capi = PC.pkg().capi
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x, err, dW = torch.randn(N, P, device="cuda", generator=g), torch.randn(N, D, device="cuda", generator=g), torch.zeros(P * D + D, device="cuda")
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    if reserved:
+        capi.gemm_reserve(stream)
+    held = capi.lib().cnt_gemm_scratch_buffers()
+    capi.dense_backward_weights(P, D, 8, 0.5, x, err, dW)  # (the code is loaded outside the capture)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+        capi.dense_backward_weights(P, D, N, 0.5, x, err, dW, stream=stream)
+    assert capi.lib().cnt_gemm_scratch_buffers() == held
+    want, size = err.double().t() @ x.double(), err.double().abs().t() @ x.double().abs()
+    for _ in range(3):
+        dW.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool(((dW[:P * D].view(D, P) - want).abs() <= (N + 2) * 2.0 ** -24 * size).all())
+        assert bool(((dW[P * D:] - 0.5 * err.double().sum(0)).abs() <= (N + 2) * 2.0 ** -24 * 0.5 * err.double().abs().sum(0)).all())
+    del graph
+    capi.gemm_release(stream)
+
+
 @pytest.mark.parametrize("m,n,k,tA,tB", [(70, 66, 37, True, False), (3100, 3076, 516, False, False)])
 def test_matrix_product_of_infinite_huge_and_missing_values(m, n, k, tA, tB):
     """Values that have no finite bf16 parts give what fp32 arithmetic gives."""

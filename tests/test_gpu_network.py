@@ -194,6 +194,31 @@ def test_weight_gradients_of_wide_dense_layers(lengths):
     net.close()
 
 
+@pytest.mark.parametrize("T", [40, 700])
+def test_weight_gradients_of_a_fraction_without_a_valid_slot(T):
+    """Every weight gradient over an empty list of slots is zero, whatever the updates held: one split, several, narrow and wide."""
+    import torch
+
+    print("network case: no valid slot", T, flush=True)
+    capi = PC.pkg().capi
+    P, Q, S = 20, 8, 3
+    layers = [{"size": P, "name": "input", "type": "input"}, {"name": "ff1", "type": "feedforward_tanh", "size": 64, "bias": 1.0},
+              {"name": "ff2", "type": "feedforward_logistic", "size": 512, "bias": 0.5},
+              {"name": "ff3", "type": "feedforward_tanh", "size": 512, "bias": 0.5},
+              {"name": "out", "type": "feedforward_identity", "size": Q, "bias": 1.0}, {"name": "postoutput", "type": "sse", "size": Q}]
+    net = capi.Network(json.dumps({"layers": layers}), S, T)
+    net.randomize(3, 0.1)
+    x, tgt = torch.randn(T * S * P, device="cuda"), torch.randn(T * S * Q, device="cuda")
+    for pat, zero in ((make_pat_types([T] * S, T), False), (np.zeros(T * S, dtype=np.int8), True)):
+        net.load_sequences(PC.dev(pat), T, 1 if zero else T, x, tgt)
+        net.updates.fill_(5.0)
+        net.forward()
+        net.backward()
+        torch.cuda.synchronize()
+        assert bool((net.updates == 0).all()) == zero
+    net.close()
+
+
 def test_network_reports_a_later_lstm_layer_that_gave_up_and_keeps_the_weights():
     """Failure handling at network level, forced from the host: the SECOND recurrent layer's recursions get a spin
     limit of zero, the first layer's stay as they are.  Every kernel still ends normally; the failure is reported by
