@@ -512,6 +512,12 @@ int local_groups(int H, int JB, int S, int ndir, int cus_per_xcd) {
     return std::max(least, std::min(resident / ndir, S));
 }
 
+// Sequences of a job at most, by which mailboxes, launches and kernels go alike: one where every sequence has a job of its own and
+// kernels for that exist.  (Layers of 129 to 256 cells take 16 cells per workgroup with more than eight jobs of four, so there are none
+// for them; CNT_LSTM_LOCAL_JB takes fewer jobs there.)
+constexpr int local_most(int H, int JB, int groups, int S) { return groups < S || (JB == 16 && H <= 256) ? kLocalSeqs : 1; }
+
+// nullptr: no such kernel
 chain_kernel_t pick_local_kernel(bool fwd, int H, int JB, int most, bool clocks) {
     const int PW = (H + 63) / 64;
     if (JB == 8) {
@@ -523,8 +529,8 @@ chain_kernel_t pick_local_kernel(bool fwd, int H, int JB, int most, bool clocks)
     }
     if (JB == 16) {
         switch (PW) {
-            case 3: return local_pair<3, 16, kLocalSeqs>(fwd, clocks);  // (layers of up to 256 cells come here with more than eight jobs)
-            case 4: return local_pair<4, 16, kLocalSeqs>(fwd, clocks);
+            case 3: return most == kLocalSeqs ? local_pair<3, 16, kLocalSeqs>(fwd, clocks) : nullptr;
+            case 4: return most == kLocalSeqs ? local_pair<4, 16, kLocalSeqs>(fwd, clocks) : nullptr;
             case 5: return local_pair<5, 16>(fwd, most, clocks);
             case 6: return local_pair<6, 16>(fwd, most, clocks);
             case 7: return local_pair<7, 16>(fwd, most, clocks);
@@ -800,8 +806,8 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     const int least = (desc->S + kLocalSeqs - 1) / kLocalSeqs;
     const int local_jb = local_cells(H, ndir * least);
     const int groups = solo ? least : local_groups(H, local_jb, desc->S, ndir, cus / kLocalXcds);
-    const int local_most = groups >= desc->S ? 1 : kLocalSeqs;
-    const bool stepwise = (!solo && pick_local_kernel(true, H, local_jb, local_most, false) == nullptr) || std::getenv("CNT_LSTM_STEPWISE") != nullptr;
+    const int most = local_most(H, local_jb, groups, desc->S);
+    const bool stepwise = (!solo && pick_local_kernel(true, H, local_jb, most, false) == nullptr) || std::getenv("CNT_LSTM_STEPWISE") != nullptr;
 
     cnt_lstm *h = new (std::nothrow) cnt_lstm();
     CNT_REQUIRE(h != nullptr, "lstm_create: out of host memory");
@@ -811,7 +817,7 @@ int cnt_lstm_create(const cnt_lstm_desc *desc, cnt_lstm **out) {
     h->solo = solo && !stepwise ? 1 : 0;
     h->local = !solo && !stepwise ? 1 : 0;
     h->local_jb = local_jb;
-    h->local_most = local_most;
+    h->local_most = most;
     h->bmail_dirty = 1;
     h->flmail_dirty = 1;
     h->spin_limit = 1u << 22;

@@ -537,6 +537,19 @@ def test_lstm_sequences_dealt_by_length(L, bidir, lengths):
         assert PC.relerr(got[0][k], got[1][k]) < TOL, k
 
 
+@pytest.mark.parametrize("cells", [8, 16])
+@pytest.mark.parametrize("L,bidir,lengths", [
+    (512, True, [21]), (512, True, [21, 9]), (200, False, [17]), (258, True, [13, 12, 5]),  # a job per sequence
+    (512, True, [20, 20, 11, 7, 3] * 4), (150, False, [15] * 9), (300, False, [12, 8]), (100, False, [9, 4]),
+])
+def test_lstm_cells_per_workgroup_by_the_environment(L, bidir, lengths, cells, monkeypatch):
+    """CNT_LSTM_LOCAL_JB: mailboxes, launch and kernel go by the same number of sequences per job, also where a layer would not take
+    that many cells per workgroup by itself; sizes without such a kernel go step by step."""
+    print("lstm cells per workgroup", cells, L, bidir, lengths, flush=True)
+    monkeypatch.setenv("CNT_LSTM_LOCAL_JB", str(cells))
+    assert PC.run_lstm_two_recursions(21, L, bidir, lengths, seed=cells + L) < TOL
+
+
 @pytest.mark.parametrize("L,bidir,lengths", [(256, True, [110, 104, 90]), (256, False, [107]), (600, True, [104] * 34), (1024, True, [106, 105])])
 def test_lstm_recursion_clocks(L, bidir, lengths, monkeypatch, capfd):
     """CNT_LSTM_TIMING / CNT_LSTM_TRACE: the recursion kernels with clocks compute the same, and cnt_lstm_check prints what the
