@@ -140,10 +140,14 @@ __device__ int local_claim_role(const ChainParams &p, int G) {
 // Step of a job of 1 to 4 sequences, of 128 (us per step, forward / backward, 256 cells: 0.867 / 0.777, 0.910 / 0.838, 0.987 / 0.869,
 // 0.999 / 0.873; other sizes in about the same proportions).
 template <bool FWD>
-__device__ __forceinline__ int step_cost(int sequences) {
+__host__ __device__ constexpr int step_cost(int sequences) {
     constexpr int cost[5] = {0, FWD ? 111 : 114, FWD ? 117 : 123, FWD ? 126 : 127, 128};
     return cost[sequences];
 }
+// in 64 bits: 2^24 steps and more of 128 are no 32-bit number
+template <bool FWD>
+__host__ __device__ constexpr long long job_cost(int steps, int sequences) { return (long long)steps * step_cost<FWD>(sequences); }
+static_assert(job_cost<true>(0x7FFFFFFF, 4) == 0x7FFFFFFFLL * 128 && job_cost<false>(0x7FFFFFFF, 1) > 0x7FFFFFFFLL, "no wrap at any length");
 constexpr int kPlannedSeqs = 64;  // more parallel sequences are dealt evenly and in order, and take every step
 struct LocalPlan {
     int role;
@@ -195,13 +199,16 @@ __device__ __forceinline__ LocalJob local_setup(const ChainParams &p, LocalPlan 
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             const int sorted = lane < S ? plan.length[lane] : 0;
-            auto most_within = [&](int bound) {  // sequences of a job that starts with this lane's
+            long long cost[MOST];  // of a job of this lane's sequence and the q behind it
+#pragma unroll
+            for (int q = 0; q < MOST; ++q) cost[q] = job_cost<FWD>(sorted, q + 1);
+            auto most_within = [&](long long bound) {  // sequences of a job that starts with this lane's
                 int n = 0;
 #pragma unroll
-                for (int q = 1; q <= MOST; ++q) n = sorted * step_cost<FWD>(q) <= bound ? q : n;
+                for (int q = 0; q < MOST; ++q) n = cost[q] <= bound ? q + 1 : n;
                 return n;
             };
-            auto cut = [&](int bound, bool keep) {
+            auto cut = [&](long long bound, bool keep) {
                 const int n = most_within(bound);
                 int at = 0, g = 0;
                 for (; at < S && g < p.groups; ++g) {
@@ -216,10 +223,10 @@ __device__ __forceinline__ LocalJob local_setup(const ChainParams &p, LocalPlan 
                 return at >= S;
             };
             const int top = __builtin_amdgcn_readlane(sorted, 0);
-            int low = top * step_cost<FWD>(1) - 1, high = top * step_cost<FWD>(MOST);  // `high` always suffices
+            long long low = job_cost<FWD>(top, 1) - 1, high = job_cost<FWD>(top, MOST);  // `high` always suffices
             // (four in every job: nothing to choose)
             for (int q = 0; q < 10 && high - low > 1 && p.groups * MOST > S; ++q) {
-                const int mid = (low + high) / 2;
+                const long long mid = (low + high) / 2;
                 if (cut(mid, false)) high = mid;
                 else low = mid;
             }
@@ -249,11 +256,12 @@ __device__ __forceinline__ void fill_padding(const ChainParams &p, const LocalJo
     const int H = p.H, S = p.S, j0 = me * JB, per_step = part.nseq * JB;
     // before the job's steps or behind them
     const int b0 = p.step_begin, e0 = min(p.step_end, max(part.begin, b0)), b1 = max(part.end, e0), e1 = max(p.step_end, b1);
-    const int before = e0 - b0, count = (before + (e1 - b1)) * per_step;
+    const int before = e0 - b0, steps = before + (e1 - b1);
     const bool forward_in_time = FWD ? part.dir == 0 : part.dir != 0;
-    for (int i = threadIdx.x; i < count; i += blockDim.x) {
-        const int q = i / per_step, r = i % per_step, c = j0 + r % JB;
-        if (c >= H) continue;
+    // as many steps side by side as the workgroup has threads for
+    const int rows = (int)blockDim.x / per_step, r = (int)threadIdx.x % per_step, c = j0 + r % JB, first = (int)threadIdx.x / per_step;
+    if (first >= rows || c >= H) return;
+    for (int q = first; q < steps; q += rows) {
         const int step = q < before ? b0 + q : b1 + q - before, t = forward_in_time ? step : p.T - 1 - step;
         const size_t slot = (size_t)t * S + part.order[r / JB], gi = slot * H + c, oi = slot * p.L + part.dir * H + c;
         if (FWD) {
