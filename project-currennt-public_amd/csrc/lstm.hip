@@ -1032,12 +1032,12 @@ static int print_clocks(cnt_lstm *h) {
             std::fprintf(stderr, "\n");
         }
         if (!active) continue;
-        const double us = 0.01 / active / h->T;
+        const double steps = std::max(m[CLK_STEPS], 1.0), us = 0.01 / steps;  // a job leaves out steps on which all its sequences are padding
         std::fprintf(stderr, "lstm %s per step [us]: %s wave pause+poll %.3f (%.2f rounds) %s %.3f barrier %.3f loop %.3f | load wave busy "
-                     "%.3f store wave %.3f %s wave %.3f (T=%d, %d workgroups)\n", backward ? "backward" : "forward",
-                     backward ? "cell" : "gather", m[CLK_WAIT] * us, m[CLK_ROUNDS] / active / h->T, backward ? "update" : "product",
+                     "%.3f store wave %.3f %s wave %.3f (T=%d, %.1f steps of a job, %d workgroups)\n", backward ? "backward" : "forward",
+                     backward ? "cell" : "gather", m[CLK_WAIT] * us, m[CLK_ROUNDS] / steps, backward ? "update" : "product",
                      m[CLK_REST] * us, m[CLK_BARRIER] * us, m[CLK_LOOP] * us, m[CLK_LOAD] * us, m[CLK_STORE] * us,
-                     backward ? "product" : "cell", m[CLK_OTHER] * us, h->T, active);
+                     backward ? "product" : "cell", m[CLK_OTHER] * us, h->T, steps / active, active);
     }
     return CNT_OK;
 }

@@ -326,7 +326,7 @@ __device__ __forceinline__ f32x4 local_product(const f32x4 &a, const float (&wre
 // they pass five points of it, on the 100 MHz clock that all compute units share.  The kernels without are free of all of
 // it: a branch on the chain of a step costs some of what it would measure.
 constexpr unsigned kClockBlocks = 512;  // workgroups that record
-enum { CLK_WAIT, CLK_REST, CLK_BARRIER, CLK_LOOP, CLK_ROUNDS, CLK_LOAD, CLK_STORE, CLK_OTHER, kClockCounts };
+enum { CLK_WAIT, CLK_REST, CLK_BARRIER, CLK_LOOP, CLK_ROUNDS, CLK_LOAD, CLK_STORE, CLK_OTHER, CLK_STEPS, kClockCounts };
 constexpr int kTraceFirst = 64, kTraceSteps = 4, kTracePoints = 5, kTraceWords = 4 + kTraceSteps * kTracePoints;
 constexpr size_t kClockWords = (size_t)kClockBlocks * (kClockCounts + kTraceWords);  // of one direction of time
 template <bool CLOCKS>
@@ -675,6 +675,7 @@ __device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJo
         clock_store<CLOCKS>(p, CLK_REST, rest - waited - barrier);
         clock_store<CLOCKS>(p, CLK_BARRIER, barrier);
         clock_store<CLOCKS>(p, CLK_ROUNDS, rounds);
+        clock_store<CLOCKS>(p, CLK_STEPS, end_step - begin_step);
         clock_store<CLOCKS>(p, CLK_LOOP, clock_now<CLOCKS>() - begin);
         clock_where<CLOCKS>(p, job, me);
     }

@@ -360,6 +360,7 @@ __device__ __forceinline__ void forward_job(const ChainParams &p, const LocalJob
         clock_store<CLOCKS>(p, CLK_REST, rest - waited - barrier);
         clock_store<CLOCKS>(p, CLK_BARRIER, barrier);
         clock_store<CLOCKS>(p, CLK_ROUNDS, rounds);
+        clock_store<CLOCKS>(p, CLK_STEPS, end_step - begin_step);
         clock_store<CLOCKS>(p, CLK_LOOP, clock_now<CLOCKS>() - begin);
         clock_where<CLOCKS>(p, job, me);
     }

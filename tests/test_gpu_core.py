@@ -572,6 +572,22 @@ def test_lstm_recursion_clocks(L, bidir, lengths, monkeypatch, capfd):
                 assert 0 < points[i] <= points[i + 1] <= points[i + 2] and 0 < points[i + 3] <= points[i + 4], line
 
 
+@pytest.mark.parametrize("bidir", [False, True])
+def test_lstm_recursion_clocks_count_a_jobs_own_steps(bidir, monkeypatch, capfd):
+    """Per-step times are sums over the steps that the jobs took: as many as their sequences are long (where time runs forward one
+    more, the slot behind the sequence), not as the fraction is."""
+    print("lstm recursion clocks, own steps", bidir, flush=True)
+    monkeypatch.setenv("CNT_LSTM_TIMING", "1")
+    lengths, L = [107, 30, 64], 512 if bidir else 256
+    assert PC.run_lstm_two_recursions(16, L, bidir, lengths, seed=6) < TOL
+    lines = capfd.readouterr().err.splitlines()
+    mean = {kind: [line for line in lines if line.startswith("lstm %s per step" % kind)][0] for kind in ("forward", "backward")}
+    taken = {kind: float(re.search(r"([0-9.]+) steps of a job", line).group(1)) for kind, line in mean.items()}
+    alone, behind = sum(lengths) / 3, sum(min(n + 1, 107) for n in lengths) / 3
+    want = {"forward": (alone + behind) / 2 if bidir else behind, "backward": (alone + behind) / 2 if bidir else alone}
+    assert all(abs(taken[k] - want[k]) < 0.051 for k in want), (taken, want)
+
+
 def test_lstm_config2_layer_full_length_two_recursions():
     """A BLSTM layer of benchmark config 2 at its full size (512 inputs, 256 cells per direction, T=600, S=10,
     lengths drawn from 300..600): the persistent recursion kernels against the step-by-step schedule.  The CPU
