@@ -1062,6 +1062,7 @@ int finish_build(cnt_network *net, const json::Value *weights) {
     }
     for (size_t i = 5; i < net->layers.size() && !net->block_sums; ++i)
         if (net->layers[i].kind == K_DENSE && net->layers[i - 4].kind == K_WAVNETC &&
+            wavenet_block_errors_supported(net->layers[i - 4].size, net->layers[i].size) &&
             wavenet_block_weights_supported(net->layers[i - 4].size, net->layers[i].size, net->layers[i - 4].ctx_dim, 1))
             CNT_TRY(device_alloc(net, (void **)&net->block_sums, wavenet_block_weights_scratch() * sizeof(float), false));
     // the slots of a fraction with the valid ones first: the weight gradients of the dense and recurrent layers sum over

@@ -128,3 +128,23 @@ def test_block_weight_gradients_under_capture():
         torch.cuda.synchronize()
         assert bool((net.updates == want).all())
     net.close()
+
+
+@pytest.mark.parametrize("R,K,scratch", [(64, 128, True), (48, 96, False), (64, 32, False), (32, 256, False)])
+def test_scratch_of_the_common_launches_only_where_they_are_made(R, K, scratch):
+    """A stack whose block sizes have no launch for the errors sums its weight gradients without the blocks' scratch (34 MB)."""
+    import torch
+
+    pkg = PC.pkg()
+
+    def taken(C):
+        doc = json.dumps(pkg.specs.wavenet_network_doc(1, 16, R, K, C, 0, 4))
+        pkg.capi.Network(doc, 1, 64, mdn_config=[1, 0, 16, 0, 1, -1]).close()
+        before = torch.cuda.mem_get_info()[0]
+        net = pkg.capi.Network(doc, 1, 64, mdn_config=[1, 0, 16, 0, 1, -1])
+        after = torch.cuda.mem_get_info()[0]
+        net.close()
+        return before - after
+
+    # (beside the same stack without conditioning features, which never has it)
+    assert (taken(20) - taken(0) >= 32 << 20) == scratch
