@@ -141,8 +141,15 @@ int pick_tile(const GemmArgs &a) {
     const long run = (long)a.k * a.nseg / a.splitk;
     const long t64 = (long)((a.m + 63) / 64) * ((a.n + 63) / 64) * a.nprob * a.splitk;
     // (outputs that leave more than a twelfth of the large tiles' rows and columns empty stay on the small ones: 300 x 10 000 x 425
-    // and the like, 2207 -> 2276 us per pass with them on the large ones)
-    if ((a.a_kcontig || a.b_kcontig) && 12 * t64 >= 11 * 4 * t128 && eight_waves(t128, run)) return kEightWaves;
+    // and the like, 2207 -> 2276 us per pass with them on the large ones.  Up to an eighth empty, 600 tiles and more of 512 to 767
+    // values are better off on the large ones, us with 64 x 64 / 128 on four waves / on eight: 430 rows, k = 640, 608 tiles 89 / 85 / 87,
+    // 680 94 / 86 / 88, 760 103 / 90 / 90, 980 129 / 133 / 116, 1100 145 / 141 / 142, 1300 165 / 164 / 168, 1400 181 / 168 / 170; k = 760, 680 tiles
+    // 115 / 104 / 105, 1100 179 / 167 / 171; 550 rows the same within 1 %; 300 rows, a sixth empty, k = 512 to 760, 609 to 1300 tiles 67 to 194 /
+    // 71 to 196 / 72 to 201.)
+    const bool filled = 12 * t64 >= 11 * 4 * t128;
+    if ((a.a_kcontig || a.b_kcontig) && filled && eight_waves(t128, run)) return kEightWaves;
+    if ((a.a_kcontig || a.b_kcontig) && !filled && 8 * t64 >= 7 * 4 * t128 && t128 >= 600 && run >= 512 && run < 768)
+        return t128 > 768 && t128 <= 1024 ? kEightWaves : 128;
     const bool quads = (a.a_kcontig ? a.k : a.m) % 4 == 0 && a.b_kcontig && a.k % 4 == 0;
     if (!quads) return t128 >= 600 && run >= 512 ? 128 : 64;
     if (run >= 768) return t128 >= 336 ? 128 : 64;

@@ -769,7 +769,9 @@ def test_matrix_product_of_few_blocks(m, n, k, tA, tB):
 
 @pytest.mark.parametrize("m,n,k,tA,tB", [(1024, 11900, 256, True, False), (1024, 11900, 256, False, False), (1012, 12001, 300, True, False),
                                          (1936, 5999, 508, False, False), (1024, 11000, 252, True, False),
-                                         (1024, 5370, 768, True, False), (1020, 5110, 768, False, False), (1024, 12700, 516, False, False)])
+                                         (1024, 5370, 768, True, False), (1020, 5110, 768, False, False), (1024, 12700, 516, False, False),
+                                         # an eighth and a sixth of the large tiles' rows empty
+                                         (430, 21700, 640, True, False), (432, 31350, 512, False, False), (300, 28900, 640, True, False)])
 def test_matrix_product_of_short_runs_and_full_generations(m, n, k, tA, tB):
     """Both sides of the lines between the tile sizes by length of run and number of tiles; rows and columns that end inside a
     tile."""
