@@ -16,6 +16,9 @@
 // compiler then waits for every load in flight (40 us per block), which is why the kinds of segments are loops of their own.
 // Two workgroups per compute unit (128 registers) rather than one, so that one's barriers fall into the other's work.
 //
+// Padding counts like any slot (the 1x1 products of before left it out): still the faster way where nearly half of a fraction is padding,
+// 30 blocks over 2 x 16 000 slots with a sequence of 1000 3622 -> 3528 us per pass before the shares were dealt as they are now.
+//
 // Sums: a run of kTallRun tiles is added up by the matrix instructions, then joins the sums of earlier runs, then come the splits.
 // 2-norm error against 64 bits, before / now, for the convolution, the projection, the 1x1 and the skip layer: 1.6 / 1.0, 4.0 /
 // 2.3, 1.4 / 1.2, 1.1 / 0.9e-7 (32 000 slots); 1.8 / 1.3, 2.4 / 1.7, 1.7 / 1.2, 1.7 / 1.2e-7 (2001).  Without runs the 1x1 layers
@@ -40,6 +43,7 @@ constexpr int kTallRun = 8;         // tiles added up before the sum joins the s
 constexpr int kTallWorkgroups = 512;
 constexpr int kTallBlocks = 16;      // 32 x 32 blocks of sums of a workgroup
 constexpr int kTallMaxJobs = 5;
+constexpr int kTallTileCost = 8;     // of a tile of any size, see wavenet_block_weights
 
 struct TallArgs {
     BlockGradients block[kBlockGradients];
@@ -432,14 +436,18 @@ int wavenet_block_weights(hipStream_t stream, int R, int K, int C, int N, int co
     a.partial = scratch;
     a.rows = scratch + (size_t)kTallWorkgroups * kTallBlocks * 1024;
     // The launch is one generation, two workgroups per compute unit; a block's share is dealt to its jobs by what a tile of theirs
-    // takes: 16 rows to convert weigh about as much as a block of sums to multiply.
+    // takes: 16 rows to convert weigh about as much as a block of sums to multiply, and a tile's barriers and the wait for its loads
+    // about eight times that.  Pass without this constant / with 3 / 5 / 8, us: 20 blocks of 32 and 32 channels, 80 features, 24 000
+    // slots 1088 / 1015 / 1011 / 994 (the tiled products took 1060 to 1075 there), 32 and 64 channels, 50 features 1073 / - / - / 1033, 64 and
+    // 256 channels 2270 / 2263 / 2270 / 2266, 30 blocks of 64 and 128 over 32 000 3407 / 3352 / 3334 / 3328; with 16 to 30 the wide ones lose
+    // 1 to 2 % again.
     const int per_block = kTallWorkgroups / count;
     const auto blocks_of = [](int rows) { return (rows + 31) / 32; };
     int cost[kTallMaxJobs], total = 0;
     for (int j = 0; j < a.jobs; ++j) {
         const int skip = std::min(K - 128 * (j - 3), 128);
         const int m = j == 0 ? 2 * R : j == 1 ? C : R, n = j < 2 ? 2 * R : j == 2 ? R : skip;
-        cost[j] = (m + n + 15) / 16 + (j == 0 ? 2 * blocks_of(R) : blocks_of(m)) * blocks_of(n);
+        cost[j] = kTallTileCost + (m + n + 15) / 16 + (j == 0 ? 2 * blocks_of(R) : blocks_of(m)) * blocks_of(n);
         total += cost[j];
     }
     const int tiles = (N + kTallDepth - 1) / kTallDepth;

@@ -1,9 +1,9 @@
 """Weight gradients of a WaveNet stack's residual blocks, all blocks of a launch together (csrc/wavenet_weights.hip), against 64-bit
 products of the network's own inputs and errors.
 
-Tolerance: a gradient is a sum over the slots, in runs of at most 256 slots (16 tiles of six instructions: 96 roundings of at most
-2^-24 of the sum so far, sqrt(96) * 2^-24 = 6e-7 if they are independent) that are added up in at most a few dozen additions more;
-2e-6 of the result's 2-norm holds that three times over."""
+Tolerance: a gradient is a sum over the slots, in runs of 128 slots (8 tiles of six instructions: 48 roundings of at most
+2^-24 of the sum so far) that are added up in at most some forty additions more; sqrt(48 + 40) * 2^-24 = 5.6e-7 of the result's
+2-norm if they are independent.  Measured: 0.6 to 1.7e-7."""
 import json
 
 import numpy as np
@@ -12,7 +12,7 @@ import pytest
 import parity_cases as PC
 
 pytestmark = pytest.mark.gpu
-TOL = 2e-6
+TOL = 5.6e-7
 
 
 def passed_network(capi, specs, blocks, R, K, C, lengths, seed=1, spike=None, overlap=True):
