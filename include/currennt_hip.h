@@ -79,7 +79,7 @@ int cnt_dense_backward(void *stream, int P, int D, int N, int act, float bias, c
  * split; calling both in this order on one stream is cnt_dense_backward.
  * Device memory: a weight half whose sum over the slots is cut into parts adds the parts up through a scratch buffer of 36 MB per
  * stream, which the library allocates the first time such a product runs on a stream and keeps; the same holds for
- * cnt_cnn_backward_weights and cnt_wavnetc_backward_weights.  Apart from that, only the *_create calls allocate. */
+ * cnt_cnn_backward_weights, cnt_wavnetc_backward_weights and cnt_lstm_backward_weights.  Apart from that, only the *_create calls allocate. */
 int cnt_dense_backward_errors(void *stream, int P, int D, int N, int act, const float *weights, const float *y,
                               float *err, float *prev_err);
 int cnt_dense_backward_weights(void *stream, int P, int D, int N, float bias, const float *x, const float *err,

@@ -7,6 +7,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <functional>
 
 #include "../../include/currennt_hip.h"
 
@@ -275,6 +276,36 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args);
 void gemm_release_stream(hipStream_t stream);
 // Allocates the split-K scratch buffer of `stream` now instead of inside the first product that wants it.
 int gemm_reserve_stream(hipStream_t stream);
+// Sum over `count` parts, `stride` floats apart, of output e < total, by a workgroup of 256 for 32 consecutive outputs: the parts are
+// dealt to eight groups of 32 threads whose sums meet in LDS, four loads in flight per thread.  The first 32 threads have the sums.
+constexpr int kPartOutputs = 32;
+__device__ __forceinline__ float sum_of_parts(const float *__restrict__ parts, size_t e, size_t total, int count, size_t stride) {
+    constexpr int G = 256 / kPartOutputs;
+    __shared__ float part[G][kPartOutputs];
+    const int tx = threadIdx.x % kPartOutputs, g = threadIdx.x / kPartOutputs;
+    float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+    if (e < total) {
+        const float *__restrict__ p = parts + e;
+        int s = g;
+        for (; s + 3 * G < count; s += 4 * G) {
+            const float x0 = p[(size_t)s * stride], x1 = p[(size_t)(s + G) * stride];
+            const float x2 = p[(size_t)(s + 2 * G) * stride], x3 = p[(size_t)(s + 3 * G) * stride];
+            a0 += x0; a1 += x1; a2 += x2; a3 += x3;
+        }
+        for (; s < count; s += G) a0 += p[(size_t)s * stride];
+    }
+    part[g][tx] = (a0 + a1) + (a2 + a3);
+    __syncthreads();
+    float v = 0.0f;
+    if (g == 0)
+#pragma unroll
+        for (int q = 0; q < G; ++q) v += part[q][tx];
+    return v;
+}
+// Launches by other files whose parts meet in the stream's split-K scratch: calls `enqueue` with the buffer, and no product of the
+// stream comes between what it launches.  false: no buffer of that size (as for gemm_plan), nothing was called.
+constexpr size_t kSplitScratchFloats = (size_t)9 << 20;  // 36 MB per (device, stream)
+bool with_split_scratch(hipStream_t stream, size_t floats, const std::function<void(float *)> &enqueue);
 // number of split-K scratch buffers the library holds at the moment (one per stream that has needed or reserved one)
 int gemm_scratch_buffers();
 // cnt_dense_backward_weights with the partial products in a scratch array that is part of the code object
@@ -429,7 +460,9 @@ int fill_words(hipStream_t stream, unsigned *p, size_t count, unsigned word);
 // cnt_sse_error in one launch, summed in 64 bits; sum: 64 words of the caller's that are zero between calls
 int sse_error_once(hipStream_t stream, int D, int N, const char *patTypes, const float *y, const float *target, float *result_dev,
                    float *sum);
-// out[d] += scale * sum over the N columns of a D x N column-major matrix (out pre-zeroed by the caller)
+// out[d] += scale * sum over the N columns of a D x N column-major matrix (out pre-zeroed by the caller), and the same with `=`, through
+// the stream's scratch where it has one
 int column_sum(hipStream_t stream, const float *v, int D, int N, float scale, float *out);
+int column_sum_store(hipStream_t stream, const float *v, int D, int N, float scale, float *out);
 
 }  // namespace cnt

@@ -50,10 +50,12 @@ __global__ void dense_delta_kernel(float *__restrict__ err, const float *__restr
     for (size_t i = 4 * n4 + first; i < count; i += stride) err[i] = act_deriv(act, y[i]) * err[i];
 }
 
-// out[d] += scale * sum_i v[d + i*D]; out is zeroed by the caller.  A block is 64 rows x 4 column lanes (one
+// scale * sum_i v[d + i*D].  A block is 64 rows x 4 column lanes (one
 // wave per lane, 256-byte row segments); every lane strides over the columns with eight loads in flight, the
-// four partial sums meet in LDS and leave as one atomic per row and block.  The number of blocks is kept near
+// four partial sums meet in LDS and leave as one value per row and block: PARTS, to the block's row of `out`; otherwise as an
+// atomic addition to out[d], zeroed by the caller.  The number of blocks is kept near
 // 512: atomics to one address serialise, and with thousands of blocks they, not the reads, set the run time.
+template <bool PARTS>
 __global__ __launch_bounds__(256) void column_sum_kernel(const float *__restrict__ v, int D, int N, float scale,
                                                          float *__restrict__ out) {
     __shared__ float part[4][64];
@@ -74,7 +76,17 @@ __global__ __launch_bounds__(256) void column_sum_kernel(const float *__restrict
     }
     part[ty][tx] = (a0 + a1) + (a2 + a3);
     __syncthreads();
-    if (ty == 0 && d < D) atomicAdd(out + d, (part[0][tx] + part[1][tx]) + (part[2][tx] + part[3][tx]));
+    const float sum = (part[0][tx] + part[1][tx]) + (part[2][tx] + part[3][tx]);
+    if (ty == 0 && d < D) {
+        if (PARTS) out[(size_t)blockIdx.y * D + d] = sum;
+        else atomicAdd(out + d, sum);
+    }
+}
+
+__global__ __launch_bounds__(256) void sum_parts_kernel(const float *__restrict__ parts, int count, int total, float *__restrict__ out) {
+    const size_t e = (size_t)blockIdx.x * kPartOutputs + threadIdx.x % kPartOutputs;
+    const float v = sum_of_parts(parts, e, total, count, total);
+    if (threadIdx.x < kPartOutputs && e < (size_t)total) out[e] = v;
 }
 
 __global__ void sse_backward_kernel(int D, size_t count, const char *__restrict__ pat, const float *__restrict__ y,
@@ -272,14 +284,36 @@ int fill_words(hipStream_t stream, unsigned *p, size_t count, unsigned word) {
     return CNT_OK;
 }
 
-int column_sum(hipStream_t stream, const float *v, int D, int N, float scale, float *out) {
+namespace {
+dim3 column_sum_grid(int D, int N) {
     const int gx = (D + 63) / 64;
     int gy = (N + 31) / 32;  // at least eight columns per lane
     gy = std::min(gy, std::max(1, 512 / gx));
-    gy = std::max(gy, 1);
-    hipLaunchKernelGGL(column_sum_kernel, dim3(gx, gy), dim3(64, 4), 0, stream, v, D, N, scale, out);
+    return dim3(gx, std::max(gy, 1));
+}
+}  // namespace
+
+int column_sum(hipStream_t stream, const float *v, int D, int N, float scale, float *out) {
+    hipLaunchKernelGGL(column_sum_kernel<false>, column_sum_grid(D, N), dim3(64, 4), 0, stream, v, D, N, scale, out);
     CNT_HIP(hipGetLastError());
     return CNT_OK;
+}
+
+int column_sum_store(hipStream_t stream, const float *v, int D, int N, float scale, float *out) {
+    const dim3 grid = column_sum_grid(D, N);
+    if (grid.y == 1) {
+        hipLaunchKernelGGL(column_sum_kernel<true>, grid, dim3(64, 4), 0, stream, v, D, N, scale, out);
+        CNT_HIP(hipGetLastError());
+        return CNT_OK;
+    }
+    const bool stored = with_split_scratch(stream, (size_t)grid.y * D, [&](float *parts) {
+        hipLaunchKernelGGL(column_sum_kernel<true>, grid, dim3(64, 4), 0, stream, v, D, N, scale, parts);
+        hipLaunchKernelGGL(sum_parts_kernel, dim3((D + kPartOutputs - 1) / kPartOutputs), dim3(256), 0, stream, parts, (int)grid.y, D, out);
+    });
+    CNT_HIP(hipGetLastError());
+    if (stored) return CNT_OK;
+    CNT_TRY(fill_zero(stream, out, (size_t)D));
+    return column_sum(stream, v, D, N, scale, out);
 }
 
 }  // namespace cnt

@@ -161,12 +161,12 @@ int pick_tile(const GemmArgs &a) {
 // split stores its partial product with plain stores into a scratch buffer and a second, small kernel adds the splits up in a fixed
 // order, the row sums of B (a dense layer's bias gradient) with them.  Nothing has to be cleared and nothing is added atomically.
 // Outputs of a few hundred splits (64 x 128 summed over 32 000 slots) would be bound by their atomic additions.  Wide outputs of a
-// few splits take as long either way (five 1024 x 1024 layers over 10 000 slots: pass 2104 us with a clear and atomic additions,
-// 2112 so, of 33 MB of partial products a layer; the model with mixture outputs 191 and 189), but a clear in front of atomic
-// additions has once been seen to take a split's additions with it: on one run the bias gradient of a 1024 x 1028 layer came out
-// without its first split's share.  Nothing in the launches' order explains it, so weight gradients of dense, convolution and
-// conditioning layers no longer rest on it, and they are the same bits in every call.
-constexpr size_t kSplitScratchFloats = (size_t)9 << 20;  // 36 MB per (device, stream): kWideGradientGroups large tiles, and their row sums
+// few splits take as long either way (five 1024 x 1024 layers over 10 000 slots: pass 2143 us with clears and atomic additions,
+// 2152 so, of 33 MB of partial products a layer; the acoustic model 2615 and 2574, 32 sequences 2446 and 2469), but a clear in front of
+// atomic additions has once been seen to take a split's additions with it: on one run the bias gradient of a 1024 x 1028 layer came
+// out without its first split's share.  Nothing in the launches' order explains it, so no layer's weight gradient rests on it any
+// more, and all of them are the same bits in every call.
+// (kSplitScratchFloats holds kWideGradientGroups large tiles and their row sums)
 constexpr long kManySplits = 8;                          // from here on, and up to kFewOutputs sums, eight threads share a sum's splits
 constexpr long kFewOutputs = 128 << 10;
 
@@ -232,35 +232,13 @@ float *static_scratch() {
     return g_static_ptr[dev];
 }
 
-// 32 consecutive outputs per block, the splits dealt to eight groups of 32 threads whose sums meet in LDS; four
-// loads in flight per thread
-constexpr int kReduceOutputs = 32;
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs args) {
-    constexpr int G = 256 / kReduceOutputs;
-    __shared__ float part[G][kReduceOutputs];
-    const int tx = threadIdx.x % kReduceOutputs, g = threadIdx.x / kReduceOutputs;
     const size_t mn = (size_t)args.m * args.n;
     const size_t products = mn * args.nprob;
     const size_t total = products + (args.rowsum ? (size_t)args.n * args.nprob : 0);
-    const size_t e = (size_t)blockIdx.x * kReduceOutputs + tx;
-    float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
-    if (e < total) {
-        const float *__restrict__ p = args.partial + e;
-        const size_t st = args.partial_stride;
-        int s = g;
-        for (; s + 3 * G < args.splitk; s += 4 * G) {
-            const float x0 = p[(size_t)s * st], x1 = p[(size_t)(s + G) * st];
-            const float x2 = p[(size_t)(s + 2 * G) * st], x3 = p[(size_t)(s + 3 * G) * st];
-            a0 += x0; a1 += x1; a2 += x2; a3 += x3;
-        }
-        for (; s < args.splitk; s += G) a0 += p[(size_t)s * st];
-    }
-    part[g][tx] = (a0 + a1) + (a2 + a3);
-    __syncthreads();
-    if (g == 0 && e < total) {
-        float v = 0.0f;
-#pragma unroll
-        for (int q = 0; q < G; ++q) v += part[q][tx];
+    const size_t e = (size_t)blockIdx.x * kPartOutputs + threadIdx.x % kPartOutputs;
+    const float v = sum_of_parts(args.partial, e, total, args.splitk, args.partial_stride);
+    if (threadIdx.x < kPartOutputs && e < total) {
         if (e < products) {
             const size_t z = e / mn, r = e % mn;
             args.prob[z].C[(r / args.m) * args.ldc + r % args.m] = v;
@@ -340,6 +318,15 @@ int gemm_reserve_stream(hipStream_t stream) {
     std::lock_guard<std::mutex> lock(g_split_mu);
     CNT_REQUIRE(split_scratch(stream) != nullptr, "gemm: no memory for the split-K scratch buffer");
     return CNT_OK;
+}
+
+bool with_split_scratch(hipStream_t stream, size_t floats, const std::function<void(float *)> &enqueue) {
+    if (floats > kSplitScratchFloats) return false;
+    std::lock_guard<std::mutex> lock(g_split_mu);
+    float *buf = split_scratch_find(stream);
+    if (!buf && !capturing(stream)) buf = split_scratch(stream);
+    if (buf) enqueue(buf);
+    return buf != nullptr;
 }
 
 int gemm_scratch_buffers() {
@@ -487,7 +474,7 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
     if (args.epilogue == EPI_PARTIAL) {
         const size_t total = args.partial_stride;
         if (args.splitk >= kManySplits && total <= (size_t)kFewOutputs)
-            hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((total + kReduceOutputs - 1) / kReduceOutputs)), dim3(256), 0,
+            hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((total + kPartOutputs - 1) / kPartOutputs)), dim3(256), 0,
                                stream, args);
         else
             hipLaunchKernelGGL(splitk_reduce_quads_kernel, dim3((unsigned)((total / 4 + kReduceThreads - 1) / kReduceThreads)),

@@ -188,8 +188,8 @@ __global__ __launch_bounds__(1024) void chain_guard(const GuardParams g) { guard
 // Bias and peephole gradients: per (direction, gate, cell) sums over all patterns
 // (LstmLayer.cu:524-541, 574-610, 625-646).  A thread owns V neighbouring cells (4, 2 or 1, what divides the cell count per
 // direction: 16-byte loads where it can be), a wave walks whole rows of the state arrays, a workgroup's waves share a chunk of
-// patterns and add up in LDS first, so that a gradient element takes one global atomic per chunk -- atomics to one address
-// serialise, and with a short chunk they, not the loads, set the kernel's time.  blockIdx.z is the direction.
+// patterns and add up in LDS.  The chunks' sums meet in the stream's scratch in a fixed order (lstm_small_grads_sum); without one they
+// are added atomically to gradients that the caller has cleared.  blockIdx.z is the direction.
 // 150 cells in two directions over 10 000 patterns: 24 + 29 us with a thread per cell, a chunk of 32 patterns and a launch per
 // direction, 23 us now.
 // ---------------------------------------------------------------------------------------------------
@@ -199,55 +199,72 @@ struct SmallGradDirs {
     const float *dni[2], *dig[2], *dfg[2], *dog[2], *c[2];
     float *g_bias;  // + g*L + dir*H + u
     float *g_peep;  // + k*L + dir*H + u
+    float *parts;   // [chunk][direction][4 biases, 3 peepholes][cell]
 };
+constexpr int kSmallSums = 7;  // per cell: four biases, three peepholes
 
 template <int V>
 __global__ __launch_bounds__(256) void lstm_small_grads(const SmallGradDirs p) {
     typedef float cells __attribute__((ext_vector_type(V)));
-    __shared__ float acc[7][256];
+    __shared__ cells acc[kSmallSums][256];  // [row of patterns walked side by side][group of cells]
     const int dir = blockIdx.z;
     const int groups = p.H / V;
     const int gpb = min(groups, 256 / V);  // groups of cells per workgroup
     const int rows = 256 / gpb;            // pattern rows walked side by side
     const int tid = threadIdx.x;
-    for (int k = 0; k < 7; ++k) acc[k][tid] = 0.0f;
-    __syncthreads();
     const int gl = tid % gpb, r = tid / gpb;
     const int q = blockIdx.x * gpb + gl;
-    if (r < rows && q < groups) {
-        const int i0 = blockIdx.y * p.chunk, i1 = min(p.N, i0 + p.chunk);
-        const int S = p.S;
-        const cells *dni = reinterpret_cast<const cells *>(p.dni[dir]), *dig = reinterpret_cast<const cells *>(p.dig[dir]);
-        const cells *dfg = reinterpret_cast<const cells *>(p.dfg[dir]), *dog = reinterpret_cast<const cells *>(p.dog[dir]);
-        const cells *c = reinterpret_cast<const cells *>(p.c[dir]);
+    if (r < rows) {
         cells b0 = {}, b1 = b0, b2 = b0, b3 = b0, q_ig = b0, q_fg = b0, q_og = b0;
+        if (q < groups) {
+            const int i0 = blockIdx.y * p.chunk, i1 = min(p.N, i0 + p.chunk);
+            const int S = p.S;
+            const cells *dni = reinterpret_cast<const cells *>(p.dni[dir]), *dig = reinterpret_cast<const cells *>(p.dig[dir]);
+            const cells *dfg = reinterpret_cast<const cells *>(p.dfg[dir]), *dog = reinterpret_cast<const cells *>(p.dog[dir]);
+            const cells *c = reinterpret_cast<const cells *>(p.c[dir]);
 #pragma unroll 4
-        for (int i = i0 + r; i < i1; i += rows) {
-            const size_t o = (size_t)i * groups + q;
-            const cells d_ni = dni[o], d_ig = dig[o], d_fg = dfg[o], d_og = dog[o];
-            b0 += d_ni; b1 += d_ig; b2 += d_fg; b3 += d_og;
-            q_og += c[o] * d_og;
-            // input/forget peepholes look at the cell state one step earlier in processing order
-            const int ie = dir ? i + S : i - S;
-            if (ie >= 0 && ie < p.N) {
-                const cells ce = c[(size_t)ie * groups + q];
-                q_ig += ce * d_ig;
-                q_fg += ce * d_fg;
+            for (int i = i0 + r; i < i1; i += rows) {
+                const size_t o = (size_t)i * groups + q;
+                const cells d_ni = dni[o], d_ig = dig[o], d_fg = dfg[o], d_og = dog[o];
+                b0 += d_ni; b1 += d_ig; b2 += d_fg; b3 += d_og;
+                q_og += c[o] * d_og;
+                // input/forget peepholes look at the cell state one step earlier in processing order
+                const int ie = dir ? i + S : i - S;
+                if (ie >= 0 && ie < p.N) {
+                    const cells ce = c[(size_t)ie * groups + q];
+                    q_ig += ce * d_ig;
+                    q_fg += ce * d_fg;
+                }
             }
         }
-        const cells v[7] = {b0 * p.bias, b1 * p.bias, b2 * p.bias, b3 * p.bias, q_ig, q_fg, q_og};
+        const cells v[kSmallSums] = {b0 * p.bias, b1 * p.bias, b2 * p.bias, b3 * p.bias, q_ig, q_fg, q_og};
 #pragma unroll
-        for (int k = 0; k < 7; ++k)
-#pragma unroll
-            for (int e = 0; e < V; ++e) atomicAdd(&acc[k][V * gl + e], v[k][e]);
+        for (int k = 0; k < kSmallSums; ++k) acc[k][tid] = v[k];
     }
     __syncthreads();
-    const int u = blockIdx.x * gpb * V + tid;
-    if (tid < V * gpb && u < p.H) {
-        float *gb = p.g_bias + dir * p.H + u, *gp = p.g_peep + dir * p.H + u;
-        for (int k = 0; k < 4; ++k) atomicAdd(gb + k * p.L, acc[k][tid]);
-        for (int k = 0; k < 3; ++k) atomicAdd(gp + k * p.L, acc[4 + k][tid]);
+    const int mine = V * gpb, u0 = blockIdx.x * mine;
+    for (int i = tid; i < kSmallSums * mine; i += 256) {
+        const int k = i / mine, j = i % mine, u = u0 + j;
+        if (u >= p.H) continue;
+        const float *const sums = reinterpret_cast<const float *>(acc[k]) + j;
+        float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+        int row = 0;
+        for (; row + 4 <= rows; row += 4) {
+            s0 += sums[row * mine]; s1 += sums[(row + 1) * mine]; s2 += sums[(row + 2) * mine]; s3 += sums[(row + 3) * mine];
+        }
+        for (; row < rows; ++row) s0 += sums[row * mine];
+        const float s = (s0 + s1) + (s2 + s3);
+        if (p.parts) p.parts[(((size_t)blockIdx.y * gridDim.z + dir) * kSmallSums + k) * p.H + u] = s;
+        else atomicAdd((k < 4 ? p.g_bias + (size_t)k * p.L : p.g_peep + (size_t)(k - 4) * p.L) + dir * p.H + u, s);
     }
+}
+
+__global__ __launch_bounds__(256) void lstm_small_grads_sum(const SmallGradDirs p, int ndir, int chunks) {
+    const size_t total = (size_t)ndir * kSmallSums * p.H, e = (size_t)blockIdx.x * kPartOutputs + threadIdx.x % kPartOutputs;
+    const float v = sum_of_parts(p.parts, e, total, chunks, total);
+    if (threadIdx.x >= kPartOutputs || e >= total) return;
+    const int u = (int)(e % p.H), k = (int)(e / p.H % kSmallSums), dir = (int)(e / p.H / kSmallSums);
+    (k < 4 ? p.g_bias + (size_t)k * p.L : p.g_peep + (size_t)(k - 4) * p.L)[dir * p.H + u] = v;
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -1222,12 +1239,6 @@ extern "C++" int cnt::lstm_backward_weights_parts(cnt_lstm *h, hipStream_t strea
     const size_t nW = weight_count(P, L, d.bidir);
     const size_t off_bias = (size_t)4 * P * L, off_int = off_bias + (size_t)4 * L;
     const size_t off_peep = off_int + (size_t)4 * L * H;
-    if ((parts & 3) == 3) {
-        CNT_TRY(fill_zero(stream, weight_updates, nW));
-    } else {
-        if (parts & 1) CNT_TRY(fill_zero(stream, weight_updates, off_bias));
-        if (parts & 2) CNT_TRY(fill_zero(stream, weight_updates + off_bias, nW - off_bias));
-    }
     if (parts & 1) {
         // input weights: dW_in[g,dir] (P x H) = x (P x N) * delta^T
         GemmArgs ga = {};
@@ -1250,6 +1261,9 @@ extern "C++" int cnt::lstm_backward_weights_parts(cnt_lstm *h, hipStream_t strea
             ga.k_count = h->slot_order.count;
         }
         ga.label = "gemm:lstm_dW_input";
+        ga.overwrite_ok = 1;  // the problems cover all input weights
+        gemm_plan(ga, stream);
+        if (ga.epilogue == EPI_ATOMIC) CNT_TRY(fill_zero(stream, weight_updates, off_bias));
         CNT_TRY(gemm_launch(stream, ga));
     }
     if (!(parts & 2)) return CNT_OK;
@@ -1281,10 +1295,15 @@ extern "C++" int cnt::lstm_backward_weights_parts(cnt_lstm *h, hipStream_t strea
             ga.k_count = h->slot_order.count;
         }
         ga.label = "gemm:lstm_dW_internal";
+        ga.overwrite_ok = 1;  // the problems cover all recurrent weights
+        gemm_plan(ga, stream);
+        if (ga.epilogue == EPI_ATOMIC) CNT_TRY(fill_zero(stream, weight_updates + off_int, off_peep - off_int));
         CNT_TRY(gemm_launch(stream, ga));
+    } else {
+        CNT_TRY(fill_zero(stream, weight_updates + off_int, off_peep - off_int));
     }
     SmallGradDirs sp;
-    sp.H = H; sp.L = L; sp.S = S; sp.N = N; sp.bias = d.bias;
+    sp.H = H; sp.L = L; sp.S = S; sp.N = N; sp.bias = d.bias; sp.parts = nullptr;
     sp.chunk = N >= 4096 ? 64 : 16;  // a short fraction still fills some tens of workgroups
     for (int dir = 0; dir < 2; ++dir) {
         const int sd = dir < h->ndir ? dir : 0;
@@ -1294,13 +1313,26 @@ extern "C++" int cnt::lstm_backward_weights_parts(cnt_lstm *h, hipStream_t strea
     sp.g_bias = weight_updates + off_bias;
     sp.g_peep = weight_updates + off_peep;
     const int V = H % 4 == 0 ? 4 : H % 2 == 0 ? 2 : 1, groups = H / V, gpb = std::min(groups, 256 / V);
-    dim3 grid((groups + gpb - 1) / gpb, (N + sp.chunk - 1) / sp.chunk, h->ndir);
+    // (very long fractions: as many chunks as the scratch holds sums of)
+    const size_t sums = (size_t)h->ndir * kSmallSums * H, most = std::max<size_t>(kSplitScratchFloats / sums, 1);
+    sp.chunk = std::max(sp.chunk, (int)((N + most - 1) / most));
+    const dim3 grid((groups + gpb - 1) / gpb, (N + sp.chunk - 1) / sp.chunk, h->ndir);
+    const auto small = V == 4 ? lstm_small_grads<4> : V == 2 ? lstm_small_grads<2> : lstm_small_grads<1>;
     ProfileScope prof(stream, "lstm_small_grads");
-    hipLaunchKernelGGL(V == 4 ? lstm_small_grads<4> : V == 2 ? lstm_small_grads<2> : lstm_small_grads<1>, grid, dim3(256), 0, stream, sp);
+    const bool stored = with_split_scratch(stream, sums * grid.y, [&](float *buf) {
+        sp.parts = buf;
+        hipLaunchKernelGGL(small, grid, dim3(256), 0, stream, sp);
+        hipLaunchKernelGGL(lstm_small_grads_sum, dim3((unsigned)((sums + kPartOutputs - 1) / kPartOutputs)), dim3(256), 0, stream, sp,
+                           h->ndir, (int)grid.y);
+    });
+    if (!stored) {
+        sp.parts = nullptr;
+        CNT_TRY(fill_zero_pair(stream, weight_updates + off_bias, off_int - off_bias, weight_updates + off_peep, nW - off_peep));
+        hipLaunchKernelGGL(small, grid, dim3(256), 0, stream, sp);
+    }
     CNT_HIP(hipGetLastError());
     return CNT_OK;
 }
-
 
 int cnt_lstm_backward(cnt_lstm *h, void *stream, const float *weights, const float *x, const float *outputs,
                       float *output_errors, float *prev_errors, float *weight_updates) {

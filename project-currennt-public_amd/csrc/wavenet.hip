@@ -793,7 +793,7 @@ extern "C++" int cnt::cnn_backward_weights_batch(cnt_cnn *const *h, int count, h
         size_t most = 0;
         for (int z = 0; z < count; ++z) {
             fl.ptr[z] = weight_updates[z];
-            fl.count[z] = (size_t)P * h[z]->Lw + D;
+            fl.count[z] = (size_t)P * h[z]->Lw;  // (the products write the live taps over, the rest stays)
             most = std::max(most, (size_t)fl.count[z]);
         }
         fl.n = count;
@@ -837,7 +837,7 @@ extern "C++" int cnt::cnn_backward_weights_batch(cnt_cnn *const *h, int count, h
             sums.rows[at] = colsum_rows[z];
             sums.scale[at] = h[z]->desc.bias;
         } else {
-            CNT_TRY(column_sum(stream, output_errors[z], D, N, h[z]->desc.bias, bias_grad));
+            CNT_TRY(column_sum_store(stream, output_errors[z], D, N, h[z]->desc.bias, bias_grad));
         }
     }
     if (sums.n > 0) {
@@ -856,7 +856,7 @@ int cnt_cnn_backward_weights(cnt_cnn *h, void *stream_, const char *patTypes, in
     const cnt_cnn_desc &d = h->desc;
     const int P = d.P, D = d.D, S = d.S, N = curT * S;
 
-    CNT_TRY(fill_zero(stream, weight_updates, (size_t)P * h->Lw + D));
+    CNT_TRY(fill_zero(stream, weight_updates, (size_t)P * h->Lw));
     for (const cnt_cnn_group &g : h->groups) {
         GemmArgs ga = {};
         ga.m = P; ga.n = g.d1 - g.d0; ga.k = N;
@@ -880,7 +880,7 @@ int cnt_cnn_backward_weights(cnt_cnn *h, void *stream_, const char *patTypes, in
         CNT_TRY(gemm_launch(stream, ga));
     }
     // bias gradient over every slot, padding included, as the reference's ones-vector product does
-    return column_sum(stream, output_errors, D, N, d.bias, weight_updates + (size_t)P * h->Lw);
+    return column_sum_store(stream, output_errors, D, N, d.bias, weight_updates + (size_t)P * h->Lw);
 }
 
 int cnt_cnn_backward(cnt_cnn *h, void *stream, const char *patTypes, int curT, const float *weights, const float *x,

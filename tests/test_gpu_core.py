@@ -801,7 +801,7 @@ def test_weight_gradient_of_few_blocks(P, D, N, static):
 
 @pytest.mark.parametrize("P,D,N", [(1024, 1024, 6200), (512, 514, 2501), (401, 600, 3001), (260, 4100, 2600), (4100, 64, 2066)])
 def test_bias_gradient_beside_atomic_sums(P, D, N):
-    """Weight gradients whose splits add to a cleared output bring the bias gradient along: large and small tiles, rows that end
+    """Weight gradients of several splits bring the bias gradient along: large and small tiles, rows that end
     inside a tile, operands whose rows are no multiple of four long, a last split of another length, one infinite delta."""
     import torch
     g = torch.Generator(device="cuda").manual_seed(P + D + N)
@@ -840,6 +840,56 @@ def test_weight_gradient_is_the_same_in_every_call(P, D, N):
     assert bool(((first[P * D:] - 0.5 * err.double().sum(0)).abs() <= (N + 2) * 2.0 ** -24 * 0.5 * err.double().abs().sum(0)).all())
 
 
+# one, two and four cells per thread of the bias and peephole sums, groups of cells that leave threads idle, one time step (no recurrent
+# gradient), chunks of 16 and 64 patterns, large and small tiles, inputs of odd length
+@pytest.mark.parametrize("P,L,bidir,lengths", [
+    (30, 256, True, [40, 33, 7]), (17, 7, False, [19, 4]), (33, 300, False, [120, 90, 61, 120]), (512, 512, True, [260] * 16),
+    (20, 12, True, [1, 1, 1]), (16, 130, True, [9]), (70, 1040, True, [30, 8]), (8, 2, True, [5, 3]),
+])
+def test_recurrent_weight_gradients_are_the_same_in_every_call(P, L, bidir, lengths):
+    """All four sections of a recurrent layer's weight gradient against 64-bit sums of the layer's own states, the same bits whatever
+    the updates held before."""
+    import torch
+    print("recurrent weight gradients", P, L, bidir, lengths, flush=True)
+    S, T = len(lengths), max(lengths)
+    N, H, dirs, bias = S * T, L // (2 if bidir else 1), 2 if bidir else 1, 0.75
+    W, x, outerr = PC.lstm_inputs(P, L, bidir, S, T, lengths, 7)
+    layer = PC.pkg().capi.Lstm(P, L, bidir, S, T, bias)
+    Wd, xd, err = PC.dev(W), PC.dev(x), PC.dev(outerr)
+    layer.load_sequences(PC.dev(PC.make_pat_types(lengths, T)), T, min(lengths))
+    out, dW = torch.zeros(L * N, device="cuda"), torch.zeros(len(W), device="cuda")
+    layer.forward(Wd, xd, out)
+    layer.backward_errors(Wd, err, None)
+    first = None
+    for before in (3.0, float("nan"), 0.0):
+        dW.fill_(before)
+        layer.backward_weights(xd, dW)
+        assert first is None or torch.equal(first, dW)
+        first = dW.clone()
+    layer.check()
+    X = xd.view(N, P).double()
+    want, size = torch.zeros(len(W), device="cuda").double(), torch.zeros(len(W), device="cuda").double()
+    rec, peep = 4 * P * L + 4 * L, 4 * P * L + 4 * L + 4 * L * H
+
+    def put(at, a, b):
+        want[at:at + a.shape[1] * b.shape[1]] = (a.t() @ b).reshape(-1)
+        size[at:at + a.shape[1] * b.shape[1]] = (a.abs().t() @ b.abs()).reshape(-1)
+
+    for d in range(dirs):
+        delta = [layer.state(d, k).view(N, H).double() for k in ("dni", "dig", "dfg", "dog")]
+        h, c = layer.state(d, "h").view(N, H).double(), layer.state(d, "c").view(N, H).double()
+        now, earlier = (slice(0, N - S), slice(S, N)) if d else (slice(S, N), slice(0, N - S))
+        for g in range(4):
+            put(g * P * L + d * P * H, delta[g], X)
+            put(4 * P * L + g * L + d * H, delta[g], torch.full((N, 1), bias, device="cuda").double())
+            put(rec + g * L * H + d * H * H, delta[g][now], h[earlier])
+        for k, (a, b) in enumerate(((delta[1][now], c[earlier]), (delta[2][now], c[earlier]), (delta[3], c))):
+            want[peep + k * L + d * H:peep + k * L + d * H + H] = (a * b).sum(0)
+            size[peep + k * L + d * H:peep + k * L + d * H + H] = (a * b).abs().sum(0)
+    layer.close()
+    assert bool(((first - want).abs() <= (N + 2) * 2.0 ** -24 * size).all())
+
+
 @pytest.mark.parametrize("reserved", [True, False])
 def test_weight_gradient_under_capture(reserved):
     """A captured product uses the stream's scratch where its owner has reserved one, and allocates none where not."""
@@ -866,6 +916,40 @@ def test_weight_gradient_under_capture(reserved):
         assert bool(((dW[P * D:] - 0.5 * err.double().sum(0)).abs() <= (N + 2) * 2.0 ** -24 * 0.5 * err.double().abs().sum(0)).all())
     del graph
     capi.gemm_release(stream)
+
+
+@pytest.mark.parametrize("reserved", [True, False])
+def test_recurrent_weight_gradients_under_capture(reserved):
+    """The same on a stream with and without scratch: replays give what an eager call gives, the latter through atomic additions."""
+    import torch
+    P, L, lengths = 33, 260, [90, 71, 90]
+    S, T = len(lengths), max(lengths)
+    W, x, outerr = PC.lstm_inputs(P, L, True, S, T, lengths, 9)
+    capi = PC.pkg().capi
+    layer = capi.Lstm(P, L, True, S, T)
+    Wd, xd, err = PC.dev(W), PC.dev(x), PC.dev(outerr)
+    out, dW = torch.zeros(L * S * T, device="cuda"), torch.zeros(len(W), device="cuda")
+    layer.load_sequences(PC.dev(PC.make_pat_types(lengths, T)), T, min(lengths))
+    layer.forward(Wd, xd, out)
+    layer.backward_errors(Wd, err, None)
+    layer.backward_weights(xd, dW)
+    torch.cuda.synchronize()
+    want, stream, graph = dW.clone(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    if reserved:
+        capi.gemm_reserve(stream)
+    held = capi.lib().cnt_gemm_scratch_buffers()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+        layer.backward_weights(xd, dW, stream=stream)
+    assert capi.lib().cnt_gemm_scratch_buffers() == held
+    for _ in range(3):
+        dW.fill_(7.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(dW, want) if reserved else PC.relerr(dW.cpu().numpy(), want.cpu().numpy()) < 1e-6
+    del graph
+    capi.gemm_release(stream)
+    layer.close()
 
 
 @pytest.mark.parametrize("m,n,k,tA,tB", [(70, 66, 37, True, False), (3100, 3076, 516, False, False)])
