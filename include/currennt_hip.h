@@ -51,6 +51,10 @@ int cnt_probe_hop_message(void *stream, int kilobytes, int rounds, float *hop_us
  * +-88.72); 2, 3: the same two from the hardware's exp2 and reciprocal, which only the forward LSTM recursion uses
  * (within 4e-6 / 8e-6 absolute of the former, not bit-identical). */
 int cnt_probe_activation(void *stream, int which, long n, const float *x, float *out);
+/* Test hook: what the launcher chooses for `problems` products of m x n x k (k-contiguous operands or not; weight_gradient: cut
+ * along k) with 16-byte aligned operands.  plan[0]: edge of an output tile (32, 64 or 128), plan[1]: waves of a workgroup,
+ * plan[2]: splits of k.  Needs no device. */
+int cnt_probe_gemm_plan(int m, int n, int k, int problems, int a_kcontig, int b_kcontig, int weight_gradient, int *plan);
 
 /* ---- helpers::Matrix product seam -------------------------------------------------------------
  * Replaces helpers::Matrix<Gpu>::assignProduct / addProduct (helpers/Matrix.cu:353-377, which call

@@ -71,6 +71,7 @@ _SIGNATURES = {
     "cnt_probe_hop_latency": (I, [VP, I, I, I, C.POINTER(F)]),
     "cnt_probe_hop_message": (I, [VP, I, I, C.POINTER(F)]),
     "cnt_probe_activation": (I, [VP, I, C.c_long, VP, VP]),
+    "cnt_probe_gemm_plan": (I, [I, I, I, I, I, I, I, C.POINTER(I)]),
     "cnt_gemm_reserve": (I, [VP]),
     "cnt_gemm_release": (I, [VP]),
     "cnt_gemm_scratch_buffers": (I, []),
@@ -253,6 +254,13 @@ def probe_hop_message(kilobytes=4, rounds=2000, stream=None):
 
 def probe_activation(which, x, out, stream=None):
     check(lib().cnt_probe_activation(stream_ptr(stream), int(which), x.numel(), ptr(x), ptr(out)))
+
+
+def probe_gemm_plan(m, n, k, problems=1, a_kcontig=False, b_kcontig=False, weight_gradient=False):
+    """(edge of an output tile, waves of a workgroup, splits of k) of a product (see cnt_probe_gemm_plan)."""
+    out = (C.c_int * 3)()
+    check(lib().cnt_probe_gemm_plan(m, n, k, problems, int(a_kcontig), int(b_kcontig), int(weight_gradient), out))
+    return tuple(out)
 
 
 def gemm_reserve(stream=None):

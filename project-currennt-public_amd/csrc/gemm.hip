@@ -122,8 +122,11 @@ inline bool wide_gradient(const GemmArgs &a) {
 // 768 workgroups / 192, 256, 384, 512 workgroups of eight waves, us per pass: 32 sequences 2463 / 2410, 2373, 2357, 2376; the
 // acoustic model, where they run beside the recursion of the layer below, 2587 / 2582, 2569, 2620, 2599.  A layer of 2 x 256 cells
 // by itself over 2048 / 3200 / 6400 / 9600 slots (512, 800, 1600 and 2400 per split of the input weights) 454 / 464, 626 / 620, 837 /
-// 817, 1189 / 1161, of 2 x 512 cells over 2048 / 9600 757 / 743, 3008 / 2886.  (300 and 200 cells leave a quarter of the large
-// tiles' rows empty: 2264 -> 2315 with them.)
+// 817, 1189 / 1161, of 2 x 512 cells over 2048 / 9600 757 / 743, 3008 / 2886.  Around the line,
+// 2 x 256 cells over 2048 / 2304 / 2560 / 2752 / 3008 / 3200 / 3840 slots (512 to 960 per split) 613 / 611, 667 / 670, 720 / 724, 763 / 766,
+// 815 / 817, 855 / 855, 990 / 986; 2 x 512 over 1536 / 2048 / 2560 / 3200 (768 to 1600) 784 / 776, 963 / 943, 1190 / 1157, 1435 / 1397: what
+// lies on the wrong side of it is 0.5 %.  (300 and 200 cells leave a quarter of the large tiles' rows empty: 2264 -> 2315 with
+// them.)
 constexpr long kLevelGradientGroups = 256;
 constexpr long kLevelGradientSplit = 704;
 inline bool level_gradient(const GemmArgs &a) {
@@ -177,6 +180,12 @@ struct SplitScratch {
 };
 std::mutex g_split_mu;  // held while a product and its reduction are enqueued, so that they stay adjacent
 std::vector<SplitScratch> g_split_scratch;
+
+// CNT_GEMM_PARTIAL=0: no scratch, everything adds atomically
+bool partial_on() {
+    static const bool on = [] { const char *e = std::getenv("CNT_GEMM_PARTIAL"); return !e || std::atoi(e) != 0; }();
+    return on;
+}
 
 // One scratch buffer per stream: launches on a stream execute in order, so the next product on the same stream
 // cannot overwrite partial sums that a reduction has yet to read.  Kept until gemm_release_stream.
@@ -321,7 +330,7 @@ int gemm_reserve_stream(hipStream_t stream) {
 }
 
 bool with_split_scratch(hipStream_t stream, size_t floats, const std::function<void(float *)> &enqueue) {
-    if (floats > kSplitScratchFloats) return false;
+    if (!partial_on() || floats > kSplitScratchFloats) return false;
     std::lock_guard<std::mutex> lock(g_split_mu);
     float *buf = split_scratch_find(stream);
     if (!buf && !capturing(stream)) buf = split_scratch(stream);
@@ -372,10 +381,9 @@ void gemm_plan(GemmArgs &args, hipStream_t stream) {
         s = kLevelGradientGroups / large_tiles(args);
     s = std::min(s, std::max(1L, kt / 8));
     s = std::max(1L, s);
-    static const bool partial_on = [] { const char *e = std::getenv("CNT_GEMM_PARTIAL"); return !e || std::atoi(e) != 0; }();
     const size_t stride = partial_stride(args);
     const bool rowsum_ok = !args.rowsum || (args.nseg == 1 && !args.masked);
-    bool partial = partial_on && args.epilogue == EPI_ATOMIC && args.overwrite_ok && rowsum_ok;
+    bool partial = partial_on() && args.epilogue == EPI_ATOMIC && args.overwrite_ok && rowsum_ok;
     if (partial) s = std::max(1L, std::min(s, (long)(kSplitScratchFloats / stride)));
     // no empty split: every split of the partial-product path has to write its share
     while (s > 1 && (s - 1) * ((kt + s - 1) / s) >= kt) --s;
@@ -545,3 +553,27 @@ int gemm_simple(hipStream_t stream, float *C, int m, int n, int k, const float *
 }
 
 }  // namespace cnt
+
+extern "C" int cnt_probe_gemm_plan(int m, int n, int k, int problems, int a_kcontig, int b_kcontig, int weight_gradient, int *plan) {
+    using namespace cnt;
+    CNT_REQUIRE(plan && m > 0 && n > 0 && k > 0 && problems >= 1 && problems <= kGemmMaxProb && (!a_kcontig || b_kcontig),
+                "probe_gemm_plan: bad argument");
+    GemmArgs a = {};
+    a.m = m; a.n = n; a.k = k;
+    a.a_kcontig = a_kcontig != 0; a.lda = a_kcontig ? k : m;
+    a.b_kcontig = b_kcontig != 0; a.ldb = b_kcontig ? k : n;
+    a.ldc = m;
+    a.nseg = 1; a.nprob = problems;
+    a.epilogue = weight_gradient ? EPI_ATOMIC : EPI_STORE;
+    a.splitk = weight_gradient ? 0 : 1;
+    a.overwrite_ok = 1;
+    float nothing = 0.0f;
+    a.partial = &nothing;  // (a plan is made for the stream's scratch; none is asked for here)
+    gemm_plan(a, nullptr);
+    const bool direct = a.splitk == 1 && a.epilogue != EPI_PARTIAL && direct_product(a);
+    const int tile = direct ? 32 : pick_tile(a);
+    plan[0] = tile == kEightWaves ? 128 : tile;
+    plan[1] = direct || tile == kEightWaves ? 8 : 4;
+    plan[2] = a.splitk;
+    return CNT_OK;
+}

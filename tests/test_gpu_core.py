@@ -33,6 +33,7 @@ def test_matrix_product_on_eight_waves(m, n, k, tA, tB, acc):
     import torch
 
     print("gemm case on eight waves", m, n, k, tA, tB, acc, flush=True)
+    assert PC.pkg().capi.probe_gemm_plan(m, n, k, 1, tA, not tB)[:2] == (128, 8)
     gen = torch.Generator(device="cuda").manual_seed(m + n + k)
     A, B, C = (torch.randn(c, device="cuda", generator=gen) for c in (m * k, k * n, m * n))
     want = B.double().reshape(n, k) @ (A.double().reshape(m, k).T if tA else A.double().reshape(k, m)).contiguous()
@@ -49,6 +50,7 @@ def test_wide_dense_gradient_on_eight_waves(P, D, N):
     import torch
 
     print("wide dense gradient", P, D, N, flush=True)
+    assert PC.pkg().capi.probe_gemm_plan(P, D, N, weight_gradient=True)[:2] == (128, 8)
     gen = torch.Generator(device="cuda").manual_seed(P + D + N)
     x, e = torch.randn(N * P, device="cuda", generator=gen), torch.randn(N * D, device="cuda", generator=gen)
     W, y = torch.zeros(P * D + D, device="cuda"), torch.zeros(N * D, device="cuda")
@@ -719,8 +721,9 @@ def _product(m, n, k, tA, tB, A, B):
     return C.view(n, m).t().double(), A64, B64
 
 
-# sizes around the two tiles' edges, k around the staged depth, every vector width and both orientations; the last two take
-# the 128 x 128 tile (600 tiles and k >= 512)
+# sizes around the two tiles' edges, k around the staged depth, every vector width and both orientations; with 3000 rows and more
+# 128 x 128 tiles, on eight waves where one operand is k-contiguous and k below 768, on four waves otherwise
+# (test_gemm_plans.py)
 @pytest.mark.parametrize("m,n,k,tA,tB", [
     (63, 65, 31, False, False), (64, 64, 32, True, False), (66, 130, 33, False, True), (132, 68, 36, True, False),
     (257, 129, 97, False, False), (130, 66, 34, False, True), (1, 1, 1, False, False), (4, 1000, 100, False, True),
@@ -728,7 +731,7 @@ def _product(m, n, k, tA, tB, A, B):
     # lines of no multiple of four: vectors that cross the end of a line, last lines and last tiles float by float
     (3, 2, 200, False, True), (1, 1, 70, False, True), (2, 1, 35, False, False), (61, 187, 425, True, False), (425, 64, 131, False, True),
     (131, 66, 34, False, True), (129, 255, 99, False, False), (3101, 3077, 517, True, False), (3077, 3101, 541, False, True),
-    (3102, 3079, 515, False, False),
+    (3102, 3079, 515, False, False), (3101, 3077, 801, True, False), (3102, 3079, 770, False, False), (3100, 3076, 800, False, False),
 ])
 def test_matrix_product_is_as_exact_as_fp32_sums(m, n, k, tA, tB):
     """The operands are multiplied as three bf16 parts each: what the six part products leave out is below 2^-25 of
@@ -770,11 +773,12 @@ def test_matrix_product_of_few_blocks(m, n, k, tA, tB):
 @pytest.mark.parametrize("m,n,k,tA,tB", [(1024, 11900, 256, True, False), (1024, 11900, 256, False, False), (1012, 12001, 300, True, False),
                                          (1936, 5999, 508, False, False), (1024, 11000, 252, True, False),
                                          (1024, 5370, 768, True, False), (1020, 5110, 768, False, False), (1024, 12700, 516, False, False),
+                                         (1020, 9000, 800, False, False), (1024, 5370, 900, False, False),
                                          # an eighth and a sixth of the large tiles' rows empty
                                          (430, 21700, 640, True, False), (432, 31350, 512, False, False), (300, 28900, 640, True, False)])
 def test_matrix_product_of_short_runs_and_full_generations(m, n, k, tA, tB):
-    """Both sides of the lines between the tile sizes by length of run and number of tiles; rows and columns that end inside a
-    tile."""
+    """Both sides of the lines between the tile sizes, and between four and eight waves, by length of run and number of tiles; rows
+    and columns that end inside a tile (test_gemm_plans.py has what each case takes)."""
     import torch
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
     A, B = torch.randn(m * k, device="cuda", generator=g), torch.randn(n * k, device="cuda", generator=g)
@@ -816,9 +820,9 @@ def test_bias_gradient_beside_atomic_sums(P, D, N):
     assert bool(((dW[:P * D].view(D, P) - want).abs() <= (N + 2) * 2.0 ** -24 * (err.double().abs().t() @ x.double().abs()))[:-1].all())
 
 
-# three, eight and twelve splits of 64 x 64 and 128 x 128 tiles; sums and bias gradients that end inside a quad; few outputs with few
-# splits; one split, which stores; a row of large tiles
-@pytest.mark.parametrize("P,D,N", [(1024, 1028, 653), (1024, 1024, 6200), (512, 514, 2501), (401, 603, 3001), (1026, 7, 1200), (37, 1, 2300),
+# two to eleven splits of 64 x 64 and 128 x 128 tiles; sums and bias gradients that end inside a quad; few outputs; one split, which
+# stores, and one workgroup per block of the output; a row of large tiles
+@pytest.mark.parametrize("P,D,N", [(1024, 1028, 653), (1024, 1028, 1200), (1024, 1024, 6200), (512, 514, 2501), (401, 603, 3001), (1026, 7, 1200), (37, 1, 2300),
                                    (2048, 3072, 70), (2049, 3071, 300), (128, 8192, 9000)])
 def test_weight_gradient_is_the_same_in_every_call(P, D, N):
     """The splits of a weight gradient meet in a fixed order: the same bits whatever the updates held before, within the bound

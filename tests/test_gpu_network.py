@@ -154,7 +154,7 @@ def test_weight_gradients_of_a_fraction_that_is_mostly_padding():
 
 @pytest.mark.parametrize("lengths", [(400, 250, 3), (353, 352, 352)])
 def test_weight_gradients_of_wide_dense_layers(lengths):
-    """1024 x 1028 weights take the large tile, with the fraction's valid slots or all of them as the inner dimension."""
+    """1024 x 1028 weights in three splits of 64 x 64 tiles, with the fraction's valid slots or all of them as the inner dimension."""
     import torch
 
     print("network case: wide dense layers", lengths, flush=True)
@@ -191,6 +191,44 @@ def test_weight_gradients_of_wide_dense_layers(lengths):
     torch.cuda.synchronize()
     for L, g in zip([L for L in net.layers if L["weight_count"]], grads):
         assert PC.relerr(L["updates"].cpu().numpy(), g) < TOL, L["name"]
+    net.close()
+
+
+@pytest.mark.parametrize("lengths", [(2000, 1900, 1801), (2000, 30, 1), (2000, 2000, 2000)])
+def test_weight_gradients_of_large_tiles_over_listed_slots(lengths):
+    """1024 x 1028 weights over 6000 slots on eight waves, bias gradient included, through the list of valid slots: a last tile and a
+    last split that are not full, splits that the list leaves empty, no padding at all.  Against 64-bit sums of the network's own
+    inputs and deltas, within the bound of fp32 sums in any order; the same bits in a second pass."""
+    import torch
+
+    print("network case: large tiles over listed slots", lengths, flush=True)
+    capi = PC.pkg().capi
+    P, Q, S, T, bias = 20, 8, 3, lengths[0], 0.5
+    N = S * T
+    assert capi.probe_gemm_plan(1024, 1028, N, weight_gradient=True)[:2] == (128, 8)
+    layers = [{"size": P, "name": "input", "type": "input"}, {"name": "ff1", "type": "feedforward_tanh", "size": 1024, "bias": 1.0},
+              {"name": "ff2", "type": "feedforward_logistic", "size": 1028, "bias": bias},
+              {"name": "out", "type": "feedforward_identity", "size": Q, "bias": 1.0}, {"name": "postoutput", "type": "sse", "size": Q}]
+    net = capi.Network(json.dumps({"layers": layers}), S, T)
+    net.randomize(3, 0.1)
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    pat = PC.dev(make_pat_types(list(lengths), T))
+    live = (pat != 0).view(N, 1)
+    x, tgt = torch.randn(N, P, device="cuda", generator=gen) * live, torch.randn(N, Q, device="cuda", generator=gen) * live
+    got = []
+    for _ in range(2):
+        net.load_sequences(pat, T, min(lengths), x.reshape(-1), tgt.reshape(-1))
+        net.updates.fill_(float("nan"))
+        net.forward()
+        net.backward()
+        torch.cuda.synchronize()
+        got.append(net.layer("ff2")["updates"].clone())
+    assert torch.equal(got[0], got[1])
+    below, delta = net.layer("ff1")["outputs"].view(N, 1024).double() * live, net.layer("ff2")["errors"].view(N, 1028).double()
+    assert not bool((delta * ~live).any())
+    want = torch.cat([(delta.t() @ below).reshape(-1), bias * delta.sum(0)])
+    size = torch.cat([(delta.abs().t() @ below.abs()).reshape(-1), bias * delta.abs().sum(0)])
+    assert bool(((got[0] - want).abs() <= (N + 2) * 2.0 ** -24 * size).all())
     net.close()
 
 
