@@ -137,10 +137,11 @@ __device__ int local_claim_role(const ChainParams &p, int G) {
 // from the pattern types, so every launch of a pass, and every workgroup of a launch, finds the same cut.  The acoustic model's
 // pass (ten sequences of 300 to 600 steps, two layers of 256 cells in two directions) 2930 us dealt evenly and in order, 2750 so;
 // 150 and 200 cells with twenty sequences of 211 to 500 steps 2455 and 2305.
-// Step of a job of 1 to 4 sequences, of 128.  Measured, us per step, forward / backward: 256 cells, 8 per workgroup, 0.72 / 0.63, 0.75 / 0.67,
-// 0.82 / 0.71, 0.84 / 0.73, which is 110 / 110, 114 / 117, 125 / 124 and 128; 150 cells, 8 per workgroup, 0.69 / 0.65, 0.72 / 0.67, 0.77 / 0.71, 0.77 /
-// 0.72.  With 16 cells per workgroup small jobs are cheaper than this says: 512 cells 1.06 / 0.97, 1.15 / 1.08, 1.31 / 1.31, 1.40 / 1.35
-// (97 / 92, 105 / 102, 120 / 124), 300 cells 1.01 / 0.95, 1.02 / 1.02, 1.11 / 1.09, 1.14 / 1.22; one table for all sizes all the same.
+// Step of a job of 1 to 4 sequences, of 128.  Measured, us per step, forward / backward: 256 cells, 8 per workgroup, 0.72 / 0.63, 0.75 /
+// 0.67, 0.82 / 0.71, 0.84 / 0.73, which is 110 / 110, 114 / 117, 125 / 124 and 128; 150 cells, 8 per workgroup, 0.69 / 0.65, 0.72 / 0.67,
+// 0.77 / 0.71, 0.77 / 0.72.  With 16 cells per workgroup small jobs are cheaper than this says: 512 cells 1.06 / 0.97, 1.15 / 1.08, 1.31 /
+// 1.31, 1.40 / 1.35 (97 / 92, 105 / 102, 120 / 124), 300 cells 1.01 / 0.95, 1.02 / 1.02, 1.11 / 1.09, 1.14 / 1.22; one table for all
+// sizes all the same.
 template <bool FWD>
 __host__ __device__ constexpr int step_cost(int sequences) {
     constexpr int cost[5] = {0, FWD ? 111 : 114, FWD ? 117 : 123, FWD ? 126 : 127, 128};
