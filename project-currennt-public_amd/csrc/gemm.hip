@@ -165,7 +165,7 @@ int pick_tile(const GemmArgs &a) {
 // order, the row sums of B (a dense layer's bias gradient) with them.  Nothing has to be cleared and nothing is added atomically.
 // Outputs of a few hundred splits (64 x 128 summed over 32 000 slots) would be bound by their atomic additions.  Wide outputs of a
 // few splits take as long either way (five 1024 x 1024 layers over 10 000 slots: pass 2143 us with clears and atomic additions,
-// 2152 so, of 33 MB of partial products a layer; the acoustic model 2615 and 2574, 32 sequences 2446 and 2469), but a clear in front of
+// 2152 so, of 33 MB of partial products a layer; the acoustic model 2610 and 2559, 32 sequences 2458 and 2448), but a clear in front of
 // atomic additions has once been seen to take a split's additions with it: on one run the bias gradient of a 1024 x 1028 layer came
 // out without its first split's share.  Nothing in the launches' order explains it, so no layer's weight gradient rests on it any
 // more, and all of them are the same bits in every call.
