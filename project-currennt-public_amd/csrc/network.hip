@@ -1612,6 +1612,30 @@ int cnt_network_calculate_error(cnt_network *net, void *stream_, float *loss_dev
     return cnt_mdn_calculate_error(post.mdn, stream, post.out, loss_dev);
 }
 
+// layers whose backward pass ends with a weight half
+static bool has_weight_half(const cnt::NetLayer &L) {
+    using namespace cnt;
+    return L.kind == K_DENSE || L.kind == K_LSTM || L.kind == K_CNN || (L.kind == K_WAVNETC && L.ctx_dim > 0);
+}
+
+// A small pass's weight halves stay on the caller's stream: a hop to another stream and back takes the host some 25 us and the
+// card 18, a product of few blocks over few slots 5 to 8.  The line goes by the multiply-adds of the weight gradients; a feed-forward
+// network, whose pass has no recursion to hide the host's time behind, has a later one.  Us per pass on other streams / in line, slots
+// in brackets: three layers of 256 (120) 142 / 90, (960) 146 / 104, (1920) 149 / 129; three of 1024 (480, 1.2e9) 187 / 169, (960, 2.4e9)
+// 248 / 263; 32 and blstm 128 (120) 161 / 130, (960) 393 / 384, (1920) 408 / 410; two lstm 256 (240, 2.4e8) 358 / 335, (480) 507 / 507, (960) 846 /
+// 851; the acoustic model (60) 443 / 411, (120, 4.4e8) 363 / 341, (240) 426 / 434, (480) 616 / 632.
+static bool weights_in_line(const cnt_network *net) {
+    using namespace cnt;
+    const long slots = static_cast<long>(net->S) * net->T;
+    if (slots > 2048) return false;
+    bool recurrent = false;
+    for (const NetLayer &L : net->layers) {
+        if (L.kind == K_CNN || L.kind == K_WAVNETC) return false;  // (their products are batched over layers)
+        recurrent = recurrent || L.kind == K_LSTM;
+    }
+    return static_cast<double>(net->n_weights) * static_cast<double>(slots) <= (recurrent ? 4.5e8 : 1.3e9);
+}
+
 int cnt_network_backward(cnt_network *net, void *stream_) {
     using namespace cnt;
     CNT_REQUIRE(net && net->T > 0, "network_backward: no fraction loaded");
@@ -1619,6 +1643,15 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     int next_side = 0;
     bool side_used[cnt_network::kMaxSide] = {};
+    const bool captured = capturing(stream);  // (a graph's products take the scratch that the side streams have reserved)
+    const bool overlap = net->overlap && (captured || !weights_in_line(net));
+    // Nothing runs on the caller's stream behind the error half of the lowest layer with weights, so its weight half, and what
+    // is still waiting by then, stays there: two hops between streams (9 us each) less in front of the optimizer.
+    // Mixture-density output over 6000 slots 189.5 -> 169 us per pass, eight small WaveNet blocks 316 -> 297.
+    size_t lowest = 0;
+    for (size_t j = net->layers.size() - 1; j >= 1; --j)
+        if (has_weight_half(net->layers[j])) lowest = j;
+    bool at_end = false;
 
     // The weight half of a layer's backward pass has no consumer before the optimizer, so it runs on a side stream
     // after the layer's error half.  Handing work to another stream costs the host two event calls; a network of
@@ -1676,6 +1709,10 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     int next_small = 0;
     cnt_lstm *after_recursion = nullptr;  // set: the side stream waits for this layer's recursion, just launched
     auto next_side_stream = [&](hipStream_t *ws, bool large) -> int {
+        if (at_end) {
+            *ws = stream;
+            return CNT_OK;
+        }
         int &cursor = large ? next_side : next_small;
         const int span = large ? net->n_side : std::min(net->n_side, 2);
         cursor %= span;
@@ -1790,7 +1827,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     auto hand_over_blocks = [&]() -> int {
         if (blocks.empty()) return CNT_OK;
         hipStream_t ws = stream;
-        if (net->overlap) {
+        if (overlap) {  // always the one stream: the launches share their scratch
             ws = net->side[0];
             CNT_HIP(hipEventRecord(net->ev_main, stream));
             CNT_HIP(hipStreamWaitEvent(ws, net->ev_main, 0));
@@ -1922,7 +1959,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                     static const bool early = [] { const char *e = std::getenv("CNT_NET_EARLY_WEIGHTS"); return !e || std::atoi(e) != 0; }();
                     if (errors_done[i]) goto weight_half_of_layer;
                     if (wanted) adds_to_side(prev);
-                    if (L.kind == K_DENSE && early && net->overlap && prev_err && (double)prev.size * L.size * N >= 4e8) {
+                    if (L.kind == K_DENSE && early && overlap && prev_err && (double)prev.size * L.size * N >= 4e8) {
                         // a large dense layer: deltas first, then its weight half starts on a side stream next to the
                         // product for the preceding layer's errors instead of after it
                         CNT_TRY(dense_backward_errors_fan(stream, prev.size, L.size, N, delta_done[i] ? ACT_IDENTITY : L.act, W,
@@ -1949,24 +1986,27 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                     fan_done[i - 1] = fused ? 1 : 0;
                 } else if (L.kind == K_LSTM) {
                     static const bool early = [] { const char *e = std::getenv("CNT_NET_EARLY_WEIGHTS"); return !e || std::atoi(e) != 0; }();
-                    if (early && net->overlap && prev_err) {
+                    if (prev_err && ((early && overlap) || (!overlap && net->overlap))) {
                         // The weight half starts right after the recursion, next to the product for the preceding
                         // layer's errors, instead of after it.  Each of these products alone keeps the matrix pipes about
                         // half busy (it waits on memory); two at once fill more of the machine, and the weight half is
                         // further along when the next layer's recursion starts: acoustic model 2.88 -> 2.78 ms.
                         CNT_TRY(cnt_lstm_backward_errors(L.lstm, stream, W, L.err, nullptr));
-                        pending.push_back(i);
-                        after_recursion = lstm_is_persistent(L.lstm) ? L.lstm : nullptr;
-                        const int handed = hand_over(true);
-                        after_recursion = nullptr;
-                        CNT_TRY(handed);
+                        if (overlap) {
+                            pending.push_back(i);
+                            after_recursion = lstm_is_persistent(L.lstm) ? L.lstm : nullptr;
+                            const int handed = hand_over(true);
+                            after_recursion = nullptr;
+                            CNT_TRY(handed);
+                        }
                         if (prev_err == prev.err && prev.N == N && delta_target(i - 1)) {
                             CNT_TRY(lstm_prev_errors_delta(L.lstm, stream, W, prev_err, prev.act, prev.out));
                             delta_done[i - 1] = 1;
                         } else {
                             CNT_TRY(cnt_lstm_backward_prev_errors(L.lstm, stream, W, prev_err));
                         }
-                        break;
+                        if (overlap) break;
+                        goto weight_half_of_layer;
                     }
                     CNT_TRY(cnt_lstm_backward_errors(L.lstm, stream, W, L.err, prev_err));
                 } else {
@@ -1988,8 +2028,9 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                     }
                 }
             weight_half_of_layer:
-                if (in_block[i] || (L.kind == K_WAVNETC && L.ctx_dim == 0)) break;
-                if (!net->overlap) {
+                if (in_block[i] || !has_weight_half(L)) break;
+                at_end = i == lowest && !captured;
+                if (!overlap) {
                     CNT_TRY(weight_half(i, stream));
                     break;
                 }

@@ -232,6 +232,47 @@ def test_weight_gradients_of_large_tiles_over_listed_slots(lengths):
     net.close()
 
 
+@pytest.mark.parametrize("layers,S,T", [
+    ([("feedforward_tanh", 32), ("blstm", 128)], 4, 30),                                  # in line
+    ([("feedforward_tanh", 16), ("lstm", 16)], 1, 2048), ([("feedforward_tanh", 16), ("lstm", 16)], 1, 2049),  # either side of the slots
+    ([("blstm", 512), ("blstm", 512)], 3, 48), ([("blstm", 512), ("blstm", 512)], 3, 50),  # 4.4e8 and 4.6e8 multiply-adds
+    ([("feedforward_logistic", 700), ("feedforward_tanh", 700)], 8, 160), ([("feedforward_logistic", 700), ("feedforward_tanh", 700)], 8, 320)])
+def test_weight_halves_on_other_streams_and_in_line(layers, S, T):
+    """Where the weight halves of a pass run is the sequencer's choice: the gradients, and those of a second pass over other
+    lengths, are the ones of a network told to use the caller's stream alone.  (The products sum over the same slots in the same
+    tiles but for batches of one shape, 2^-24 per addition over at most a tile's chain: 1e-6.)"""
+    import torch
+
+    print("weight halves", layers, S, T, flush=True)
+    capi = PC.pkg().capi
+    P, Q = 30, 7
+    doc = {"layers": [{"size": P, "name": "input", "type": "input"}] +
+           [{"size": n, "name": "l%d" % i, "type": t, "bias": 1.0} for i, (t, n) in enumerate(layers)] +
+           [{"size": Q, "name": "out", "type": "feedforward_identity", "bias": 1.0}, {"size": Q, "name": "post", "type": "sse"}]}
+    nets = [capi.Network(json.dumps(doc), S, T, overlap=overlap) for overlap in (True, False)]
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    nets[0].weights.uniform_(-0.1, 0.1, generator=gen)
+    nets[1].weights.copy_(nets[0].weights)
+    for shortest in (T, max(1, T // 3)):
+        lengths = [T - (T - shortest) * i // max(1, S - 1) for i in range(S)]
+        pat = PC.dev(make_pat_types(lengths, T))
+        valid = (pat != 0).reshape(-1, 1)
+        x = (torch.randn(S * T, P, device="cuda", generator=gen) * valid).reshape(-1)
+        target = (torch.randn(S * T, Q, device="cuda", generator=gen) * valid).reshape(-1)
+        updates = []
+        for net in nets:
+            net.load_sequences(pat, T, min(lengths), x, target)
+            net.forward()
+            net.calculate_error()
+            net.backward()
+            updates.append(net.updates.clone())
+        torch.cuda.synchronize()
+        assert float(updates[1].norm()) > 0
+        assert float((updates[0] - updates[1]).norm()) <= 1e-6 * float(updates[1].norm())
+    for net in nets:
+        net.close()
+
+
 @pytest.mark.parametrize("T", [40, 700])
 def test_weight_gradients_of_a_fraction_without_a_valid_slot(T):
     """Every weight gradient over an empty list of slots is zero, whatever the updates held: one split, several, narrow and wide."""
