@@ -606,7 +606,7 @@ template <typename Launch>
 int launch_in_order(cnt_lstm *h, hipStream_t stream, Launch launch) {
     RecursionOrder &o = recursion_order(h->device);
     std::lock_guard<std::mutex> lock(o.mu);
-    if (!o.done) CNT_HIP(hipEventCreateWithFlags(&o.done, hipEventDisableTiming));
+    if (!o.done) CNT_HIP(hipEventCreateWithFlags(&o.done, kOrderEvent));
     if (o.any && o.last != stream) CNT_HIP(hipStreamWaitEvent(stream, o.done, 0));
     launch();
     CNT_HIP(hipGetLastError());

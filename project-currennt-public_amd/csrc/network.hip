@@ -1123,10 +1123,10 @@ int finish_build(cnt_network *net, const json::Value *weights) {
         }
     if (const char *e = std::getenv("CNT_NET_SIDE_STREAMS"))
         net->n_side = std::max(1, std::min((int)cnt_network::kMaxSide, std::atoi(e)));
-    CNT_HIP(hipEventCreateWithFlags(&net->ev_main, hipEventDisableTiming));
+    CNT_HIP(hipEventCreateWithFlags(&net->ev_main, cnt::kOrderEvent));
     for (int k = 0; k < net->n_side; ++k) {
         CNT_HIP(hipStreamCreateWithFlags(&net->side[k], hipStreamNonBlocking));
-        CNT_HIP(hipEventCreateWithFlags(&net->ev_side[k], hipEventDisableTiming));
+        CNT_HIP(hipEventCreateWithFlags(&net->ev_side[k], cnt::kOrderEvent));
         CNT_TRY(cnt::gemm_reserve_stream(net->side[k]));  // the weight halves' split-K scratch, not inside a pass
     }
     return CNT_OK;
