@@ -330,6 +330,10 @@ void lstm_set_veto(cnt_lstm *h, int *veto);
 // launches that have already ended); the report clears the mark
 // cnt_lstm_backward_weights in two parts that write disjoint ranges (1: input weights, 2: the rest)
 int lstm_backward_weights_parts(cnt_lstm *h, hipStream_t stream, const float *x, float *weight_updates, int parts);
+// cnt_lstm_backward_errors whose recursion also sums up the bias and peephole gradients; the parts are then asked for with kSumsDone
+constexpr int kSumsDone = 4;
+int lstm_backward_errors_sums(cnt_lstm *h, hipStream_t stream, const float *weights, float *output_errors, float *prev_errors,
+                              float *weight_updates);
 int lstm_take_failure(cnt_lstm *h);
 // makes `other` wait for the recursion launched last on this handle's device (the event the library records behind
 // every recursion launch anyway): what a stream needs that consumes the recursion's results, without another event

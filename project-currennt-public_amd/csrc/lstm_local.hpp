@@ -379,7 +379,7 @@ struct BackwardShared {
     __attribute__((aligned(16))) float dl[2][NSQ][DP];      // [sequence][cell][gate]
     // element = cell * NSQ + sequence, as in the messages
     __attribute__((aligned(16))) float coef[RING][EL][4];      // of e in d_og and in the cell error, stored d_og, e
-    __attribute__((aligned(16))) float coef_own[RING][EL][4];  // of the cell error in d_ni, d_ig, d_fg
+    __attribute__((aligned(16))) float coef_own[RING][EL][4];  // of the cell error in d_ni, d_ig, d_fg; the cell state
     __attribute__((aligned(16))) float coef_fg[RING][EL][2];   // forget gate activation, 1: padding slot
     __attribute__((aligned(16))) float res[2][EL][2];       // summed output error, cell error
     int wait_failed;
@@ -463,7 +463,7 @@ __device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJo
                 // d_og = first * e + stored d_og, cell error = second * e + ...
                 *reinterpret_cast<f32x4 *>(coef[b][el]) = f32x4{logistic_deriv(x.og) * tc, x.og * tanh_deriv(tc), x.dog_old, x.e};
                 *reinterpret_cast<f32x4 *>(coef_own[b][el]) = f32x4{x.ig * tanh_deriv(x.ni), logistic_deriv(x.ig) * x.ni,
-                                                                    logistic_deriv(x.fg) * x.c_earlier, 0.0f};
+                                                                    logistic_deriv(x.fg) * x.c_earlier, x.c};
                 coef_fg[b][el][0] = x.fg;
                 coef_fg[b][el][1] = ((t >= p.Tmin) && (x.pat == 0)) ? 1.0f : 0.0f;
             }
@@ -496,7 +496,8 @@ __device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJo
         // ------------------------------------------------------------------ store wave
         const int s = part.order[min(ej, nseq - 1)], el = ec * NSQ + ej;
         f32x4 d = {0, 0, 0, 0};
-        float e = 0, ce = 0;
+        float e = 0, ce = 0, c = 0, c_earlier = 0;
+        double sums[kSmallSums] = {};  // over this lane's steps
         long long busy = 0;
         lds_barrier();  // start of the recursion
         for (int step = begin_step; step < end_step; ++step) {
@@ -507,6 +508,12 @@ __device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJo
             if (ahead == held) {
                 d = *reinterpret_cast<const f32x4 *>(&dl[b][ej][4 * ec]);
                 e = res[b][el][0]; ce = res[b][el][1];
+                if (p.sum_bias) {
+                    // the next step's coefficients have been there since before this step's barrier; behind a job's last step the
+                    // cell state is that of a padding slot or of none, whose delta is zero
+                    c = coef_own[(unsigned)(step - begin_step) % RING][el][3];
+                    c_earlier = step + 1 < end_step ? coef_own[(unsigned)(step + 1 - begin_step) % RING][el][3] : 0.0f;
+                }
             }
             for (int i = 0; i < p.mem_delay; ++i) __builtin_amdgcn_s_sleep(1);
             wait_all_vmem();  // the stores of the step before are done
@@ -517,6 +524,11 @@ __device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJo
                 D.cerr[gi] = ce;
                 if (p.herr_out) p.herr_out[gi] = e;
                 else D.herr[gi] = e;
+                if (p.sum_bias) {
+                    const double c64 = c, earlier64 = c_earlier, d_ig = d[1], d_fg = d[2], d_og = d[3];
+                    sums[0] += (double)d[0]; sums[1] += d_ig; sums[2] += d_fg; sums[3] += d_og;
+                    sums[4] += earlier64 * d_ig; sums[5] += earlier64 * d_fg; sums[6] += c64 * d_og;
+                }
             }
             if (step > part.first) {
                 // The words the cell waves consumed in this step (before the barrier) are empty again.  The slot is used
@@ -530,6 +542,16 @@ __device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJo
                                                                ((unsigned)me * RECV + (unsigned)(q * 64 + lane) * 4u) * 4u), 0, 0);
             }
             clock_add<CLOCKS>(busy, since);
+        }
+        if (p.sum_bias) {
+            // a cell's sums of the steps and sequences of an access, JB lanes apart
+#pragma unroll
+            for (int k = 0; k < kSmallSums; ++k) {
+                float v = (float)sums[k];
+#pragma unroll
+                for (int o = JB; o < 64; o *= 2) v += __shfl_xor(v, o);
+                if (lane < JB && j0 + ec < H) put_sum(p, dir, job % p.groups, k, j0 + ec, v);
+            }
         }
         if (lane == 0) clock_store<CLOCKS>(p, CLK_STORE, busy);
         return;
@@ -684,15 +706,29 @@ __device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJo
     }
 }
 
+// the sums of a job that takes no step
+template <int JB>
+__device__ __forceinline__ void no_sums(const ChainParams &p, int dir, int job, int me) {
+    const int u = me * JB + (int)threadIdx.x;
+    if (p.sum_bias && threadIdx.x < JB && u < p.H)
+        for (int k = 0; k < kSmallSums; ++k) put_sum(p, dir, job % p.groups, k, u, 0.0f);
+}
+
 template <int PW, int JB, int MOST, bool CLOCKS>
 __global__ __launch_bounds__(local_threads(PW, JB, MOST)) void lstm_backward_local(const ChainParams p) {
     __shared__ LocalPlan plan;
     __shared__ union Shared { BackwardShared<JB, 1> one; BackwardShared<JB, MOST < 2 ? 1 : 2> two; BackwardShared<JB, MOST> most; } sh;
-    int job = 0, me = 0;
+    int job = -1, me = 0;
     const LocalJob part = local_setup<MOST, false>(p, plan, job, me);
-    if (part.nseq == 0) return;
+    if (part.nseq == 0) {  // no job (-1), or a group that no sequence was left for
+        if (job >= 0) no_sums<JB>(p, part.dir, job, me);
+        return;
+    }
     fill_padding<JB, false>(p, part, me);
-    if (part.begin >= part.end) return;
+    if (part.begin >= part.end) {
+        no_sums<JB>(p, part.dir, job, me);
+        return;
+    }
     const unsigned mail_words = (unsigned)local_job_words(p.team, JB, MOST);
     if (threadIdx.x == 0) (part.nseq == 1 ? sh.one.wait_failed : part.nseq == 2 ? sh.two.wait_failed : sh.most.wait_failed) = 0;
     if (MOST == 1 || part.nseq == 1) backward_job<PW, JB, 1, CLOCKS>(p, part, job, me, mail_words, sh.one);

@@ -296,6 +296,7 @@ __global__ __launch_bounds__(solo_threads(NW)) __attribute__((amdgpu_waves_per_e
     __shared__ __attribute__((aligned(16))) float ds[2][kLocalSeqs][4][PITCH];
     __shared__ __attribute__((aligned(16))) float coef[2][NK][kLocalSeqs][ROW];
     __shared__ __attribute__((aligned(16))) float results[2][6][kLocalSeqs][ROW];  // d_ni, d_ig, d_fg, d_og, cell error, output error
+    __shared__ __attribute__((aligned(16))) float cells_ahead[4][kLocalSeqs][ROW];  // cell states of four steps, for the store wave's sums
     __shared__ unsigned pads[2][kLocalSeqs];
 
     const int H = p.H, S = p.S, T = p.T;
@@ -338,7 +339,8 @@ __global__ __launch_bounds__(solo_threads(NW)) __attribute__((amdgpu_waves_per_e
                 x.v[I_CNEXT] = solo_load4<CELLS>(r_c, step + 1 < T ? off : kSoloNowhere, last, (step + 1 < T ? t_of(step + 1) : 0) * row);
                 x.pat = __builtin_amdgcn_raw_buffer_load_b8(r_pat, (int)pat_off, t * S, 0);
             };
-            auto put = [&](int step, int parity, const StepIn &x) __attribute__((always_inline)) {
+            auto put = [&](int step, int i, const StepIn &x) __attribute__((always_inline)) {  // i: the launch's step, of kSoloAhead
+                const int parity = i & 1;
                 f32x4 v[NK];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
@@ -350,7 +352,8 @@ __global__ __launch_bounds__(solo_threads(NW)) __attribute__((amdgpu_waves_per_e
                     for (int i = 0; i < NK; ++i) v[i][q] = LOADER ? k[i] : in[i];
                 }
 #pragma unroll
-                for (int i = 0; i < NK; ++i) lds_store4<CELLS>(&coef[parity][i][j][cells], v[i]);
+                for (int n = 0; n < NK; ++n) lds_store4<CELLS>(&coef[parity][n][j][cells], v[n]);
+                lds_store4<CELLS>(&cells_ahead[i & 3][j][cells], x.v[I_C]);
                 pads[parity][j] = step < T && t_of(step) >= p.Tmin && (x.pat & 0xFFu) == 0 ? 1u : 0u;
             };
             StepIn in[kSoloAhead];
@@ -363,7 +366,7 @@ __global__ __launch_bounds__(solo_threads(NW)) __attribute__((amdgpu_waves_per_e
 #pragma unroll
                 for (int i = 1; i <= kSoloAhead; ++i) {
                     StepIn &now = in[i % kSoloAhead];
-                    put(sb + step + i, i & 1, now);
+                    put(sb + step + i, i, now);
                     request(sb + step + i + kSoloAhead, now);
                     lds_barrier();
                 }
@@ -373,17 +376,28 @@ __global__ __launch_bounds__(solo_threads(NW)) __attribute__((amdgpu_waves_per_e
         // ------------------------------------------------------------------ store wave
         const __amdgpu_buffer_rsrc_t r_dni = solo_array(D.dni, bytes), r_dig = solo_array(D.dig, bytes), r_dfg = solo_array(D.dfg, bytes),
                                      r_ce = solo_array(D.cerr, bytes), r_herr = solo_array(p.herr_out ? p.herr_out : D.herr, bytes);
+        double sums[kSmallSums][4] = {};
         auto store = [&](int step, int parity) __attribute__((always_inline)) {
             const bool on = step >= 0 && sb + step < se;
             const int t = on ? t_of(sb + step) : 0;
             const unsigned o = on ? off : kSoloNowhere;
             auto value = [&](int k) { return lds_load4<CELLS>(&results[parity][k][j][cells]); };
-            solo_store4<CELLS>(r_dni, o, last, t * row, value(0));
-            solo_store4<CELLS>(r_dig, o, last, t * row, value(1));
-            solo_store4<CELLS>(r_dfg, o, last, t * row, value(2));
-            solo_store4<CELLS>(r_dog, o, last, t * row, value(3));
+            const f32x4 d_ni = value(0), d_ig = value(1), d_fg = value(2), d_og = value(3);
+            solo_store4<CELLS>(r_dni, o, last, t * row, d_ni);
+            solo_store4<CELLS>(r_dig, o, last, t * row, d_ig);
+            solo_store4<CELLS>(r_dfg, o, last, t * row, d_fg);
+            solo_store4<CELLS>(r_dog, o, last, t * row, d_og);
             solo_store4<CELLS>(r_ce, o, last, t * row, value(4));
             solo_store4<CELLS>(r_herr, o, last, t * row, value(5));
+            if (!p.sum_bias || !on) return;
+            // the load wave is two steps ahead of this one; behind the last step the cell states it hands over are zeros
+            const f32x4 c = lds_load4<CELLS>(&cells_ahead[step & 3][j][cells]), earlier = lds_load4<CELLS>(&cells_ahead[(step + 1) & 3][j][cells]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const double ig = d_ig[q], fg = d_fg[q], og = d_og[q], before = earlier[q];
+                sums[0][q] += (double)d_ni[q]; sums[1][q] += ig; sums[2][q] += fg; sums[3][q] += og;
+                sums[4][q] += before * ig; sums[5][q] += before * fg; sums[6][q] += (double)c[q] * og;
+            }
         };
         __syncthreads();
         for (int step = 0; step < steps; ++step) {
@@ -391,6 +405,18 @@ __global__ __launch_bounds__(solo_threads(NW)) __attribute__((amdgpu_waves_per_e
             lds_barrier();
         }
         store(steps - 1, (steps + 1) & 1);
+        if (p.sum_bias) {
+#pragma unroll
+            for (int k = 0; k < kSmallSums; ++k)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    float v = valid ? (float)sums[k][q] : 0.0f;
+                    v += __shfl_xor(v, 16);
+                    v += __shfl_xor(v, 32);
+                    // (of cells that two lanes take both write the same)
+                    if (j == 0 && q < last) put_sum(p, dir, (int)blockIdx.x % p.groups, k, cells + q, v);
+                }
+        }
         return;
     }
 

@@ -1698,7 +1698,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
             const float *x = prev.out, *e = L.err;
             return dense_backward_weights_batch(ws, prev.size, L.size, L.N, 1, &L.bias, &x, &e, &dW, &L.order);
         }
-        if (L.kind == K_LSTM) return cnt_lstm_backward_weights(L.lstm, ws, prev.out, dW);
+        if (L.kind == K_LSTM) return lstm_backward_weights_parts(L.lstm, ws, prev.out, dW, 3 | kSumsDone);
         if (L.kind == K_CNN) return cnt_cnn_backward_weights(L.cnn, ws, L.pat, L.T, prev.out, L.err, dW);
         return cnt_wavnetc_backward_weights(ws, L.size, L.ctx_dim, L.N, net->ctx, L.cgrad, dW);
     };
@@ -1742,7 +1742,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                 CNT_TRY(lstm_backward_weights_parts(L.lstm, ws, net->layers[i - 1].out, net->updates + L.w_off, 1));
                 hipStream_t ws2;
                 CNT_TRY(next_side_stream(&ws2, large));
-                CNT_TRY(lstm_backward_weights_parts(L.lstm, ws2, net->layers[i - 1].out, net->updates + L.w_off, 2));
+                CNT_TRY(lstm_backward_weights_parts(L.lstm, ws2, net->layers[i - 1].out, net->updates + L.w_off, 2 | kSumsDone));
             } else {
                 CNT_TRY(weight_half(i, ws));
             }
@@ -1991,7 +1991,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                         // layer's errors, instead of after it.  Each of these products alone keeps the matrix pipes about
                         // half busy (it waits on memory); two at once fill more of the machine, and the weight half is
                         // further along when the next layer's recursion starts: acoustic model 2.88 -> 2.78 ms.
-                        CNT_TRY(cnt_lstm_backward_errors(L.lstm, stream, W, L.err, nullptr));
+                        CNT_TRY(lstm_backward_errors_sums(L.lstm, stream, W, L.err, nullptr, net->updates + L.w_off));
                         if (overlap) {
                             pending.push_back(i);
                             after_recursion = lstm_is_persistent(L.lstm) ? L.lstm : nullptr;
@@ -2008,7 +2008,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                         if (overlap) break;
                         goto weight_half_of_layer;
                     }
-                    CNT_TRY(cnt_lstm_backward_errors(L.lstm, stream, W, L.err, prev_err));
+                    CNT_TRY(lstm_backward_errors_sums(L.lstm, stream, W, L.err, prev_err, net->updates + L.w_off));
                 } else {
                     if (errors_done[i]) {
                         if (L.ctx_dim > 0 && net->flagged >= 0)

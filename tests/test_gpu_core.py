@@ -712,6 +712,52 @@ def test_lstm_recursion_resumes_between_batches_of_steps(L, bidir, S, T, cuts):
     test_lstm_recursion_in_several_launches_is_the_same_recursion(L, bidir, S, T, cuts)
 
 
+@pytest.mark.parametrize("L,bidir,lengths", [
+    (1, False, [1]), (3, False, [5, 2]), (8, True, [9, 9, 1]), (10, True, [6, 5, 4, 3, 2]), (50, False, [13] * 4), (128, True, [30, 8, 21, 3, 17]),
+    (65, False, [40]), (200, True, [7, 30, 2, 19]), (256, True, [11] * 33), (512, True, [29, 3, 3, 3, 3, 2, 2, 1, 1, 1]), (300, False, [12, 4, 8]),
+    (512, False, [21, 5]), (1024, True, [9, 9, 2]), (130, True, [3 + i % 9 for i in range(70)]), (520, False, [6, 4])])
+def test_lstm_small_gradients_of_a_whole_backward_call(L, bidir, lengths):
+    """In a whole backward call the recursion sums them up on the way (groups of sequences apart, some with no sequence; a job's last
+    steps where a batch of them is not full); after the error half alone a launch of their own reads the states.  Both against 64-bit
+    sums over the states, the call twice in a row over two fractions.  A sum is rounded once per lane, up to seven times between lanes and
+    once per group of sequences, the launch of its own up to 64 / 4 times per chunk of patterns: 24 + groups times 2^-24 of the terms."""
+    import torch
+
+    print("lstm small gradients", L, bidir, lengths, flush=True)
+    capi = PC.pkg().capi
+    S, T, P, bias, dirs = len(lengths), max(lengths), 5, 0.7, 2 if bidir else 1
+    H = L // dirs
+    gen = torch.Generator(device="cuda").manual_seed(L + S)
+    W = torch.empty(int(capi.lib().cnt_lstm_weight_count(P, L, int(bidir))), device="cuda").uniform_(-0.2, 0.2, generator=gen)
+    layer = capi.Lstm(P, L, bidir, S, T, bias)
+    for shift in (0, 1):
+        lens = [max(1, n - shift * (n // 2)) if shift else n for n in lengths]
+        pat = torch.tensor([[(1 if t == 0 else 3 if t == n - 1 else 2) if t < n else 0 for n in lens] for t in range(T)], dtype=torch.int8, device="cuda").reshape(-1)
+        valid = (pat != 0).reshape(-1, 1)
+        x = (torch.randn(T * S, P, device="cuda", generator=gen) * valid).reshape(-1)
+        errors = (torch.randn(T * S, L, device="cuda", generator=gen) * valid).reshape(-1)
+        out, prev = torch.zeros(T * S * L, device="cuda"), torch.zeros(T * S * P, device="cuda")
+        layer.load_sequences(pat, T, min(lens))
+        layer.forward(W, x, out)
+        dW = [torch.full_like(W, 7.0) for _ in range(2)]
+        layer.backward(W, x, out, errors.clone(), prev, dW[0])
+        states = [{n: layer.state(d, n).double().reshape(T, S, H) for n in ("dni", "dig", "dfg", "dog", "c")} for d in range(dirs)]
+        layer.backward_weights(x, dW[1])
+        layer.check()
+        at_bias, at_peep = 4 * P * L, 4 * P * L + 4 * L + 4 * L * H
+        for d, st in enumerate(states):
+            c, before = st["c"], torch.zeros(T, S, H, dtype=torch.float64, device="cuda")
+            if d == 0: before[1:] = c[:-1]
+            else: before[:-1] = c[1:]
+            terms = [bias * st[n] for n in ("dni", "dig", "dfg", "dog")] + [st["dig"] * before, st["dfg"] * before, st["dog"] * c]
+            for k, term in enumerate(terms):
+                at = (at_bias + k * L if k < 4 else at_peep + (k - 4) * L) + d * H
+                bound = (24 + S) * 2.0 ** -24 * term.abs().sum((0, 1))
+                for g in dW:
+                    assert bool(((g[at:at + H].double() - term.sum((0, 1))).abs() <= bound).all()), (d, k)
+    layer.close()
+
+
 def _product(m, n, k, tA, tB, A, B):
     import torch
     C = torch.empty(m * n, device="cuda")
