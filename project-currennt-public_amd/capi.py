@@ -2,6 +2,7 @@
 data_ptr()); every call checks the returned status and raises RuntimeError with cnt_last_error()."""
 import ctypes as C
 import os
+import threading
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libcurrennt_hip.so")
@@ -279,12 +280,64 @@ def sse_error(D, N, pat, y, tgt, result, stream=None):
     check(lib().cnt_sse_error(stream_ptr(stream), D, N, ptr(pat), ptr(y), ptr(tgt), ptr(result)))
 
 
+class _Lent:
+    """Memory of a pool under the arrays that are made on it; with the last of them it goes back."""
+
+    def __init__(self, pool, memory, shape, typestr):
+        self.pool, self.memory = pool, memory
+        self.__array_interface__ = {"shape": shape, "typestr": typestr, "data": (memory.ctypes.data, False), "version": 3}
+
+    def __del__(self):
+        self.pool.give_back(self.memory)
+
+
+class _HostBuffers:
+    """Memory of a data set's fractions, used again once nothing refers to the arrays on it: most of the time of a fraction of 14 MB into
+    fresh arrays, 416 us, was the kernel's faults and zeroing of their pages; 244 us into memory that is there.  Holds at most four unused
+    buffers of 256 MB in all, until the data set is closed.  Array owners give back from any thread, and from within a garbage
+    collection: `give_back` only appends, so that it may interrupt `array` at any point."""
+
+    MOST, MOST_BYTES, SMALL = 4, 256 << 20, 128 << 10
+
+    def __init__(self):
+        self.lock, self.free, self.closed = threading.RLock(), [], False
+
+    def array(self, count):
+        """count floats with any values"""
+        import numpy as np
+
+        need = 4 * count
+        if need < self.SMALL:  # from the heap, whose pages are there
+            return np.empty(count, np.float32)
+        memory = None
+        with self.lock:
+            fits = [i for i, m in enumerate(self.free) if m.nbytes >= need]
+            if fits:
+                memory = self.free.pop(min(fits, key=lambda i: self.free[i].nbytes))
+            elif len(self.free) >= self.MOST:
+                self.free.pop(min(range(self.MOST), key=lambda i: self.free[i].nbytes))
+        if memory is None:
+            memory = np.empty(need + need // 8, np.uint8)  # (fractions differ in length; what is not touched costs nothing)
+        return np.asarray(_Lent(self, memory, (count,), "<f4"))
+
+    def give_back(self, memory):
+        with self.lock:
+            if not self.closed and len(self.free) < self.MOST and sum(m.nbytes for m in self.free) + memory.nbytes <= self.MOST_BYTES:
+                self.free.append(memory)
+
+    def close(self):
+        with self.lock:
+            self.closed = True
+            del self.free[:]
+
+
 class Dataset:
     """One .nc file as the reference's data_sets::DataSet sees it; fractions come back as numpy arrays."""
 
     def __init__(self, path, parallel_sequences, training_mode=True, truncate_seq=0, fraction=1.0):
         self.handle = VP()
         self.S = parallel_sequences
+        self._buffers = _HostBuffers()
         desc = DatasetDesc(parallel_sequences, int(training_mode), truncate_seq, fraction)
         check(lib().cnt_dataset_open(path.encode(), C.byref(desc), C.byref(self.handle)))
         n, p, q, cls, mn, mx = I(), I(), I(), I(), I(), I()
@@ -312,8 +365,9 @@ class Dataset:
         check(lib().cnt_dataset_fraction_shape(self.handle, first_seq, C.byref(n), C.byref(mx), C.byref(mn), C.byref(tot)))
         slots = mx.value * self.S
         pat = np.zeros(slots, np.int8)
-        x = np.zeros(slots * self.input_size, np.float32)
-        tgt = np.zeros(slots * self.output_size, np.float32) if not self.is_classification else None
+        # (the call writes every value)
+        x = self._buffers.array(slots * self.input_size)
+        tgt = self._buffers.array(slots * self.output_size) if not self.is_classification else None
         cls = np.zeros(slots, np.int32) if self.is_classification else None
         as_ptr = lambda a: a.ctypes.data_as(VP) if a is not None else None
         check(lib().cnt_dataset_fraction_fill(self.handle, first_seq, as_ptr(pat), as_ptr(x), as_ptr(tgt), as_ptr(cls)))
@@ -324,6 +378,7 @@ class Dataset:
         if self.handle:
             lib().cnt_dataset_close(self.handle)
             self.handle = VP()
+        self._buffers.close()
 
 
 OPT_SGD, OPT_ADAGRAD, OPT_AVEGRAD, OPT_STOCHASTIC_ADAGRAD, OPT_SGD_DECAY, OPT_ADAM = 0, 1, 2, 3, 4, 5

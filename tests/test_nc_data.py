@@ -325,3 +325,55 @@ def test_refused_allocations_are_errors(tmp_path, lengths, P):
     r = subprocess.run([sys.executable, "-c", _REFUSED, ROOT, str(lib), p, str(len(lengths))], capture_output=True, text=True,
                        env=dict(os.environ, LD_PRELOAD=" ".join([str(lib)] + os.environ.get("LD_PRELOAD", "").split())))
     assert r.returncode == 0 and "survived" in r.stdout, (r.returncode, r.stdout, r.stderr)
+
+
+def test_fractions_share_memory_only_one_after_the_other(tmp_path):
+    """A fraction's arrays lie on memory that an earlier one has given back: never while any view of an earlier one is alive, also
+    from several threads, with lengths that differ; not more is kept than the pool's bounds, and nothing behind a close."""
+    import threading
+
+    capi = load_package().capi
+    p = str(tmp_path / "pool.nc")
+    lengths = [90, 300, 40, 310, 305, 7, 250, 260]
+    write_nc(p, lengths, 200, 130, 2, seed=5)
+    data = capi.Dataset(p, 2, False, 0, 1.0)
+    segs = NF.segments(p, training_mode=False)
+    want = {i: NF.make_fraction(p, segs, i, 2) for i in range(0, 8, 2)}
+    same = lambda f, i: (np.array_equal(f["inputs"], np.asarray(want[i]["inputs"]).reshape(-1)) and  # noqa: E731
+                         np.array_equal(f["targets"], np.asarray(want[i]["targets"]).reshape(-1)))
+    first = data.fraction(2)
+    at, view = first["inputs"].ctypes.data, first["inputs"].reshape(-1, 200)[1:]
+    second = data.fraction(2)
+    assert second["inputs"].ctypes.data != at and same(first, 2) and same(second, 2)
+    kept = view.copy()
+    del first
+    assert data.fraction(6)["inputs"].ctypes.data != at and np.array_equal(view, kept)  # the view keeps its memory
+    del view
+    third = data.fraction(2)
+    assert same(third, 2) and len(data._buffers.free) <= capi._HostBuffers.MOST
+    wrong = []
+
+    def walk(seed):
+        rng = np.random.default_rng(seed)
+        held = []
+        for _ in range(40):
+            i = int(rng.integers(0, 4)) * 2
+            held.append((i, data.fraction(i)))
+            if len(held) > int(rng.integers(1, 4)):
+                k, f = held.pop(0)
+                if not same(f, k):
+                    wrong.append((seed, k))
+        wrong.extend((seed, k) for k, f in held if not same(f, k))
+
+    threads = [threading.Thread(target=walk, args=(s,)) for s in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    pool = data._buffers
+    assert 0 < len(pool.free) <= pool.MOST and sum(m.nbytes for m in pool.free) <= pool.MOST_BYTES
+    data.close()
+    assert not pool.free
+    del second, third
+    assert not pool.free
