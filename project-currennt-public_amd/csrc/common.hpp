@@ -268,9 +268,30 @@ void gemm_plan(GemmArgs &args, hipStream_t stream);
 // products never do), and its launch
 bool direct_product(const GemmArgs &args);
 void gemm_direct_launch(const GemmArgs &args, hipStream_t stream);
+// Weight gradients of few blocks, of any sizes, as one launch: the products of a small pass, whose results nothing but the optimizer
+// waits for, and the two of a recurrent layer.  All through one list of k lines, or all without.  Their operands have to stay as they
+// are until the launch.
+constexpr int kGroupProducts = 32;
+struct DirectProduct {
+    const float *A[1], *B[1];
+    float *C, *rowsum_out;
+    int m, n, k, lda, ldb, ldc;
+    float rowsum_scale;
+    int rowsum, k_trim, k_shift;
+};
+struct DirectGroup {
+    int count, blocks;
+    const int *k_order, *k_count;
+    int first[kGroupProducts];  // block of the launch at which a product begins
+    DirectProduct product[kGroupProducts];
+};
+int gemm_group_add(hipStream_t stream, DirectGroup &group, const GemmArgs &planned);
+int gemm_group_launch(hipStream_t stream, DirectGroup &group);
 // whether a product with these operands can take the EPI_FAN epilogue (operand kinds, alignment)
 bool gemm_fan_supported(const GemmArgs &args);
-int gemm_launch(hipStream_t stream, const GemmArgs &args);
+struct DirectGroup;
+// group: a weight gradient that takes the few-block kernel waits there for others of its kind, until gemm_group_launch
+int gemm_launch(hipStream_t stream, const GemmArgs &args, DirectGroup *group = nullptr);
 // Frees the split-K scratch buffer that the launcher keeps for `stream` (for owners of a stream about to destroy
 // it; the stream must be idle).  Buffers of streams never released stay until the process ends.
 void gemm_release_stream(hipStream_t stream);
@@ -329,7 +350,8 @@ void lstm_set_veto(cnt_lstm *h, int *veto);
 // non-zero if a recursion of this handle has given up since the last report (no synchronisation: it only sees
 // launches that have already ended); the report clears the mark
 // cnt_lstm_backward_weights in two parts that write disjoint ranges (1: input weights, 2: the rest)
-int lstm_backward_weights_parts(cnt_lstm *h, hipStream_t stream, const float *x, float *weight_updates, int parts);
+int lstm_backward_weights_parts(cnt_lstm *h, hipStream_t stream, const float *x, float *weight_updates, int parts,
+                                DirectGroup *group = nullptr);
 // cnt_lstm_backward_errors whose recursion also sums up the bias and peephole gradients; the parts are then asked for with kSumsDone
 constexpr int kSumsDone = 4;
 int lstm_backward_errors_sums(cnt_lstm *h, hipStream_t stream, const float *weights, float *output_errors, float *prev_errors,
@@ -422,7 +444,8 @@ CnnTaps cnn_taps(const cnt_cnn *h);
 // same D, C, N and one context buffer, as the problems of one product.  Same results as `count` calls of
 // cnt_dense_backward_weights / cnt_wavnetc_backward_weights.
 int dense_backward_weights_batch(hipStream_t stream, int P, int D, int N, int count, const float *bias,
-                                 const float *const *x, const float *const *err, float *const *weight_updates, const SlotOrder *order = nullptr);
+                                 const float *const *x, const float *const *err, float *const *weight_updates, const SlotOrder *order = nullptr,
+                                 DirectGroup *group = nullptr);
 int wavnetc_backward_weights_batch(hipStream_t stream, int D, int C, int N, int count, const float *ctx,
                                    const float *const *ctx_tanh, float *const *weight_updates);
 // Convolution layers with one filter group each and the same sizes, window and causality (dilations may differ):

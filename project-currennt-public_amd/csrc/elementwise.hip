@@ -393,7 +393,7 @@ int cnt_dense_backward_weights(void *stream, int P, int D, int N, float bias, co
 
 extern "C++" int cnt::dense_backward_weights_batch(hipStream_t stream, int P, int D, int N, int count, const float *bias,
                                                    const float *const *x, const float *const *err,
-                                                   float *const *weight_updates, const SlotOrder *order) {
+                                                   float *const *weight_updates, const SlotOrder *order, DirectGroup *group) {
     CNT_REQUIRE(count >= 1 && count <= kGemmMaxProb, "dense_backward_weights: %d layers in one launch, supported 1..%d",
                 count, kGemmMaxProb);
     CNT_REQUIRE(bias && x && err && weight_updates, "dense_backward_weights: null argument");
@@ -424,7 +424,7 @@ extern "C++" int cnt::dense_backward_weights_batch(hipStream_t stream, int P, in
     ga.overwrite_ok = 1;
     ga.rowsum = 1;
     gemm_plan(ga, stream);
-    if (ga.epilogue != EPI_ATOMIC) return gemm_launch(stream, ga);
+    if (ga.epilogue != EPI_ATOMIC) return gemm_launch(stream, ga, group);
     for (int z = 0; z < count; ++z) CNT_TRY(fill_zero(stream, weight_updates[z], (size_t)P * D + D));
     CNT_TRY(gemm_launch(stream, ga));
     for (int z = 0; z < count && !ga.rowsum; ++z)

@@ -409,7 +409,7 @@ void gemm_plan(GemmArgs &args, hipStream_t stream) {
     }
 }
 
-int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
+int gemm_launch(hipStream_t stream, const GemmArgs &args_in, DirectGroup *group) {
     GemmArgs args = args_in;
     CNT_REQUIRE(args.m > 0 && args.n > 0 && args.k > 0, "gemm: empty problem %d x %d x %d", args.m, args.n,
                 args.k);
@@ -448,6 +448,8 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in) {
     static const bool use_lines = [] { const char *e = std::getenv("CNT_GEMM_K_ORDER"); return !e || std::atoi(e) != 0; }();
     if (!use_lines) args.k_order = nullptr;
     if (args.splitk == 1 && args.epilogue != EPI_PARTIAL && direct_product(args)) {
+        if (group && !args.a_kcontig && !args.b_kcontig && args.nseg == 1 && args.epilogue == EPI_STORE)
+            return gemm_group_add(stream, *group, args);
         ProfileScope prof(stream, args.label ? args.label : "gemm");
         gemm_direct_launch(args, stream);
         CNT_HIP(hipGetLastError());

@@ -16,6 +16,7 @@
 #include "gemm_kernel.hpp"
 
 #include <cstdlib>
+#include <limits>
 
 namespace cnt {
 namespace {
@@ -114,9 +115,11 @@ struct Piece {
     }
 };
 
-// GATHER: the k lines of both (row-contiguous) operands are those a list names (GemmArgs::k_order).
-template <bool AK, bool BK_, bool GATHER>
-__global__ __launch_bounds__(64 * kDirectWaves, 4) void gemm_direct_kernel(const GemmArgs args) {
+// One block.  GATHER: the k lines of both (row-contiguous) operands are those a list names (GemmArgs::k_order).  ARGS and PROBLEM: GemmArgs
+// and one of its problems, or a group of weight gradients (one operand pair, EPI_STORE) and one of those.
+template <bool AK, bool BK_, bool GATHER, typename ARGS, typename PROBLEM>
+__device__ __forceinline__ void direct_block(const ARGS &args, const PROBLEM &pb, unsigned block) {
+    constexpr bool GROUP = std::is_same<ARGS, DirectGroup>::value;
     typedef Piece<AK> PA;
     typedef Piece<BK_> PB;
     constexpr int STAGE = PA::UNITS + PB::UNITS;
@@ -127,16 +130,19 @@ __global__ __launch_bounds__(64 * kDirectWaves, 4) void gemm_direct_kernel(const
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint4 *const mine_a = lds[wave], *const mine_b = lds[wave] + PA::UNITS;
-    const int tiles_m = (args.m + 31) / 32;
-    const int m0 = (int)(blockIdx.x % (unsigned)tiles_m) * 32, n0 = (int)(blockIdx.x / (unsigned)tiles_m) * 32;
-    const GemmProblem &pb = args.prob[blockIdx.z];
+    const auto &size = sizes_of(args, pb);
+    int nseg = 1, has_sums = 0;
+    if constexpr (GROUP) has_sums = pb.rowsum;
+    else { nseg = args.nseg; has_sums = args.rowsum; }
+    const int tiles_m = (size.m + 31) / 32;
+    const int m0 = (int)(block % (unsigned)tiles_m) * 32, n0 = (int)(block / (unsigned)tiles_m) * 32;
 
     PA oa;
     PB ob;
-    oa.init(args.lda, m0, args.m, lane);
-    ob.init(args.ldb, n0, args.n, lane);
-    const size_t ka = kChunk * (AK ? 1 : (size_t)args.lda), kb = kChunk * (BK_ ? 1 : (size_t)args.ldb);  // floats per chunk
-    const bool rowsum = !AK && !BK_ && args.rowsum != 0 && m0 == 0;
+    oa.init(size.lda, m0, size.m, lane);
+    ob.init(size.ldb, n0, size.n, lane);
+    const size_t ka = kChunk * (AK ? 1 : (size_t)size.lda), kb = kChunk * (BK_ ? 1 : (size_t)size.ldb);  // floats per chunk
+    const bool rowsum = !AK && !BK_ && has_sums != 0 && m0 == 0;
     float rs[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // of the lane's four rows, over the k positions it loads
 
     f32x16 acc;
@@ -164,7 +170,7 @@ __global__ __launch_bounds__(64 * kDirectWaves, 4) void gemm_direct_kernel(const
         for (int t = 0; t < 6; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[QB[t]], fa[QA[t]], acc, 0, 0, 0);
     };
     // the k positions this problem takes: all of them, or the listed lines, all but the first / last time step's
-    int k_extent = args.k, k_lo = 0;
+    int k_extent = size.k, k_lo = 0;
     if (GATHER) {
         k_extent = args.k_count[0];
         if (pb.k_trim == 1) { k_lo = args.k_count[1]; k_extent -= k_lo; }
@@ -172,7 +178,7 @@ __global__ __launch_bounds__(64 * kDirectWaves, 4) void gemm_direct_kernel(const
         k_extent = max(k_extent, 0);
     }
     // the whole chunks of the concatenated operand pairs: wave, wave + 8, ...
-    const int per_seg = k_extent / kChunk, total = per_seg * args.nseg;
+    const int per_seg = k_extent / kChunk, total = per_seg * nseg;
     const int *const lines = GATHER ? args.k_order + k_lo : nullptr;
     const int shift = GATHER ? pb.k_shift : 0;
     auto lines_of = [&](int chunk, int (&idx)[2]) __attribute__((always_inline)) {
@@ -221,7 +227,7 @@ __global__ __launch_bounds__(64 * kDirectWaves, 4) void gemm_direct_kernel(const
     }
     // what is left of each pair, one wave each
     const int rest = k_extent % kChunk;
-    if (rest != 0 && wave < args.nseg) {
+    if (rest != 0 && wave < nseg) {
         float a[2][4], b[2][4];
         if constexpr (GATHER) {
             int idx[2];
@@ -284,12 +290,12 @@ __global__ __launch_bounds__(64 * kDirectWaves, 4) void gemm_direct_kernel(const
 #pragma unroll
     for (int q = 0; q < MINE; ++q) {
         const int r = MINE * wave + q, n = n0 + 8 * (r >> 2) + 4 * half + (r & 3);
-        finite = finite && (m >= args.m || n >= args.n || __builtin_fabsf(v[q]) <= lim::kMax);
+        finite = finite && (m >= size.m || n >= size.n || __builtin_fabsf(v[q]) <= lim::kMax);
     }
 #pragma unroll
     for (int r = 0; r < MINE; ++r) v[r] *= 1.0f / (kSplitScale * kSplitScale);
     if (__builtin_expect(__syncthreads_or(!finite), 0)) {
-        const int kt = (k_extent + BK - 1) / BK, all = kt * args.nseg, each = (all + kDirectWaves - 1) / kDirectWaves;
+        const int kt = (k_extent + BK - 1) / BK, all = kt * nseg, each = (all + kDirectWaves - 1) / kDirectWaves;
         // (every wave has read the sums above before this: the barrier in __syncthreads_or)
         leave(plain_sums<AK, BK_, false, GATHER>(args, pb, m0, n0, lane, min(all, wave * each), min(all, (wave + 1) * each), kt,
                                                    k_extent, k_lo));
@@ -297,21 +303,29 @@ __global__ __launch_bounds__(64 * kDirectWaves, 4) void gemm_direct_kernel(const
         gather(v);
     }
 
-    if (rowsum && threadIdx.x < 32 && n0 + (int)threadIdx.x < args.n) {
+    if (rowsum && threadIdx.x < 32 && n0 + (int)threadIdx.x < size.n) {
         float x[kDirectWaves];
 #pragma unroll
         for (int q = 0; q < kDirectWaves; ++q) x[q] = row_sums[q][threadIdx.x];
         const float s = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
         pb.rowsum_out[n0 + threadIdx.x] = pb.rowsum_scale * s;
     }
-    if (m >= args.m) return;
+    if (m >= size.m) return;
+    if constexpr (GROUP) {
+#pragma unroll
+        for (int q = 0; q < MINE; ++q) {
+            const int r = MINE * wave + q, n = n0 + 8 * (r >> 2) + 4 * half + (r & 3);
+            if (n < size.n) pb.C[(size_t)n * size.ldc + m] = v[q];
+        }
+        return;
+    } else {
     float bterm = 0.0f;
     if (args.epilogue == EPI_BIAS_ACT || args.epilogue == EPI_BIAS_ACT_SKIP) bterm = args.bias_scale * pb.bias_vec[m];
 #pragma unroll
     for (int q = 0; q < MINE; ++q) {
         const int r = MINE * wave + q, n = n0 + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (n >= args.n) continue;
-        const size_t idx = (size_t)n * args.ldc + m;
+        if (n >= size.n) continue;
+        const size_t idx = (size_t)n * size.ldc + m;
         float *dst = pb.C + idx;
         const float x = v[q];
         switch (args.epilogue) {
@@ -339,6 +353,24 @@ __global__ __launch_bounds__(64 * kDirectWaves, 4) void gemm_direct_kernel(const
             } break;
         }
     }
+    }
+}
+
+template <bool AK, bool BK_, bool GATHER>
+__global__ __launch_bounds__(64 * kDirectWaves, 4) void gemm_direct_kernel(const GemmArgs args) {
+    direct_block<AK, BK_, GATHER>(args, args.prob[blockIdx.z], blockIdx.x);
+}
+
+// The weight gradients of a small pass, or a recurrent layer's two, as one launch (DirectGroup).  One after the other each took 5 to 16 us
+// for blocks that leave most of the compute units idle; side by side they take little longer than the longest.  blstm 128 with dense
+// layers over 120 slots, four such launches: 115 -> 96 us per pass; one lstm layer of 256 cells over 800 slots, two: 362 -> 359.
+template <bool GATHER>
+__global__ __launch_bounds__(64 * kDirectWaves, 4) void gemm_direct_group_kernel(const DirectGroup group) {
+    // (the starts are a few scalar loads side by side; a search along them would wait for one after the other)
+    int i = 0;
+#pragma unroll
+    for (int q = 1; q < kGroupProducts; ++q) i += (int)blockIdx.x >= group.first[q] ? 1 : 0;
+    direct_block<false, false, GATHER>(group, group.product[i], blockIdx.x - (unsigned)group.first[i]);
 }
 
 }  // namespace
@@ -359,6 +391,35 @@ bool direct_product(const GemmArgs &a) {
     if (forced >= 0) return forced != 0;
     const long blocks = (long)((a.m + 31) / 32) * ((a.n + 31) / 32) * a.nprob;
     return a.splitk == 0 ? blocks <= kDirectGradientBlocks && (long)a.k * a.nseg <= kDirectGradientDepth : blocks <= kDirectBlocks;
+}
+
+int gemm_group_add(hipStream_t stream, DirectGroup &g, const GemmArgs &a) {
+    const bool listed = a.k_order && a.k_count;
+    const int *const order = listed ? a.k_order : nullptr;
+    if (g.count > 0 && (g.count + a.nprob > kGroupProducts || order != g.k_order)) CNT_TRY(gemm_group_launch(stream, g));
+    g.k_order = order; g.k_count = listed ? a.k_count : nullptr;
+    const int blocks = ((a.m + 31) / 32) * ((a.n + 31) / 32);
+    for (int z = 0; z < a.nprob; ++z) {
+        const GemmProblem &p = a.prob[z];
+        g.first[g.count] = g.blocks;
+        g.product[g.count] = {{p.A[0]}, {p.B[0]}, p.C, p.rowsum_out, a.m, a.n, a.k, a.lda, a.ldb, a.ldc, p.rowsum_scale, a.rowsum, p.k_trim,
+                              p.k_shift};
+        ++g.count;
+        g.blocks += blocks;
+    }
+    return CNT_OK;
+}
+
+int gemm_group_launch(hipStream_t stream, DirectGroup &g) {
+    if (g.count == 0) return CNT_OK;
+    for (int q = g.count; q < kGroupProducts; ++q) g.first[q] = std::numeric_limits<int>::max();
+    ProfileScope prof(stream, "gemm:weight_gradients");
+    const dim3 grid((unsigned)g.blocks), block(64 * kDirectWaves);
+    if (g.k_order) hipLaunchKernelGGL(gemm_direct_group_kernel<true>, grid, block, 0, stream, g);
+    else hipLaunchKernelGGL(gemm_direct_group_kernel<false>, grid, block, 0, stream, g);
+    g.count = g.blocks = 0;
+    CNT_HIP(hipGetLastError());
+    return CNT_OK;
 }
 
 void gemm_direct_launch(const GemmArgs &a, hipStream_t s) {

@@ -383,17 +383,23 @@ struct GatherStage {
     }
 };
 
+// where a product's sizes and leading dimensions stand
+__device__ __forceinline__ const GemmArgs &sizes_of(const GemmArgs &args, const GemmProblem &) { return args; }
+__device__ __forceinline__ const DirectProduct &sizes_of(const DirectGroup &, const DirectProduct &product) { return product; }
+
 // 32 x 32 sums of the product over the k tiles [it_begin, it_end), by one wave on the fp32 matrix instructions and straight
 // from memory, where the split product left sums that are not finite: scaled, an operand from 2^112 on is infinite and has
 // infinity minus infinity in its parts, and a sum from 2^96 on overflows.  Infinities and NaN come out as fp32 arithmetic has them.
 // A pass of a network that has diverged is full of NaN, which stay what they are: the walk along k ends when all sums are.  1024 x 6000 x 1024,
 // usually 107 us: 107 us with NaN throughout, 756 with one at the end of every sum; one thread per sum took 11 400.
-template <bool AK, bool BK_, bool MASKED, bool GATHER>
-__device__ __forceinline__ f32x16 plain_sums(const GemmArgs &args, const GemmProblem &pb, int m0, int n0, int lane, int it_begin,
+// ARGS and PROBLEM: GemmArgs and one of its problems, or a group of products and one of those.
+template <bool AK, bool BK_, bool MASKED, bool GATHER, typename ARGS, typename PROBLEM>
+__device__ __forceinline__ f32x16 plain_sums(const ARGS &args, const PROBLEM &pb, int m0, int n0, int lane, int it_begin,
                                              int it_end, int kt_per_seg, int k_extent, int k_lo) {
     constexpr int AHEAD = 4;  // matrix instructions whose operands are in flight together
     const int half = lane >> 5;
-    const int m = min(m0 + (lane & 31), args.m - 1), n = min(n0 + (lane & 31), args.n - 1);  // past an edge: sums that are not stored
+    const auto &size = sizes_of(args, pb);
+    const int m = min(m0 + (lane & 31), size.m - 1), n = min(n0 + (lane & 31), size.n - 1);  // past an edge: sums that are not stored
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
@@ -410,13 +416,13 @@ __device__ __forceinline__ f32x16 plain_sums(const GemmArgs &args, const GemmPro
                 const int k = GATHER ? args.k_order[k_lo + (on ? at : k0)] + pb.k_shift : on ? at : k0;
                 int bk = k, bn = n;
                 bool keep = on;
-                if (MASKED && args.pat) {
+                if constexpr (MASKED) if (args.pat) {
                     const int slot = args.b_time_on_k ? k : n, from = slot + pb.b_shift[seg], src = min(max(from, 0), args.n_slots - 1);
                     keep = on && args.pat[slot] != 0 && src == from && args.pat[src] != 0;
                     if (args.b_time_on_k) bk = src; else bn = src;
                 }
-                const float x = pb.A[seg][AK ? (size_t)m * args.lda + k : (size_t)k * args.lda + m];
-                const float y = pb.B[seg][BK_ ? (size_t)bn * args.ldb + bk : (size_t)bk * args.ldb + bn];
+                const float x = pb.A[seg][AK ? (size_t)m * size.lda + k : (size_t)k * size.lda + m];
+                const float y = pb.B[seg][BK_ ? (size_t)bn * size.ldb + bk : (size_t)bk * size.ldb + bn];
                 a[u] = on ? x : 0.0f;
                 b[u] = keep ? y : 0.0f;
             }

@@ -1690,15 +1690,18 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     for (size_t i = 5; i < net->layers.size(); ++i)
         if (block_at(i) && block_weights_at(net, i)) in_block[i] = in_block[i - 3] = in_block[i - 4] = in_block[i - 5] = 1;
     std::vector<size_t> pending;
+    DirectGroup in_line;  // products of few blocks on the caller's stream: one launch at the end of the pass
+    in_line.count = in_line.blocks = 0;
     auto weight_half = [&](size_t i, hipStream_t ws) -> int {
+        DirectGroup *const group = ws == stream ? &in_line : nullptr;
         NetLayer &L = net->layers[i];
         NetLayer &prev = net->layers[i - 1];
         float *dW = net->updates + L.w_off;
         if (L.kind == K_DENSE) {
             const float *x = prev.out, *e = L.err;
-            return dense_backward_weights_batch(ws, prev.size, L.size, L.N, 1, &L.bias, &x, &e, &dW, &L.order);
+            return dense_backward_weights_batch(ws, prev.size, L.size, L.N, 1, &L.bias, &x, &e, &dW, &L.order, group);
         }
-        if (L.kind == K_LSTM) return lstm_backward_weights_parts(L.lstm, ws, prev.out, dW, 3 | kSumsDone);
+        if (L.kind == K_LSTM) return lstm_backward_weights_parts(L.lstm, ws, prev.out, dW, 3 | kSumsDone, group);
         if (L.kind == K_CNN) return cnt_cnn_backward_weights(L.cnn, ws, L.pat, L.T, prev.out, L.err, dW);
         return cnt_wavnetc_backward_weights(ws, L.size, L.ctx_dim, L.N, net->ctx, L.cgrad, dW);
     };
@@ -1782,7 +1785,8 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
             colsum[z] = L.colsum; colsum_rows[z] = L.colsum_rows;
         }
         g.layers.clear();
-        if (g.kind == K_DENSE) return dense_backward_weights_batch(ws, g.a, g.b, g.n, count, bias, in0, in1, dW, &first.order);
+        if (g.kind == K_DENSE)
+            return dense_backward_weights_batch(ws, g.a, g.b, g.n, count, bias, in0, in1, dW, &first.order, ws == stream ? &in_line : nullptr);
         if (g.kind == K_CNN) return cnn_backward_weights_batch(cnn, count, ws, first.pat, first.T, in0, in1, dW, colsum, colsum_rows);
         return wavnetc_backward_weights_batch(ws, g.a, g.b, g.n, count, net->ctx, in0, dW);
     };
@@ -2105,6 +2109,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     CNT_TRY(hand_over_blocks());
     CNT_TRY(hand_over(false));
     for (ShapeGroup &g : groups) CNT_TRY(hand_over_group(g));
+    CNT_TRY(gemm_group_launch(stream, in_line));
     for (int k = 0; k < net->n_side; ++k) {
         if (!side_used[k]) continue;
         CNT_HIP(hipEventRecord(net->ev_side[k], net->side[k]));

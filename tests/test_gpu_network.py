@@ -273,6 +273,49 @@ def test_weight_halves_on_other_streams_and_in_line(layers, S, T):
         net.close()
 
 
+@pytest.mark.parametrize("lengths,count", [([30, 22, 13, 9], 3), ([30, 30], 3), ([17, 5, 1], 36), ([700, 650, 600], 5), ([1], 34)])
+def test_weight_gradients_of_a_small_pass_in_one_launch(lengths, count):
+    """Layers of other sizes, more of them than a launch holds, over listed slots and over all: every gradient against the 64-bit
+    product of the layer's inputs and deltas, bound of a sum in any order as for the products alone."""
+    import torch
+
+    print("one launch of gradients", lengths, count, flush=True)
+    capi = PC.pkg().capi
+    S, T, P, Q = len(lengths), max(lengths), 33, 6
+    sizes = [(5, 64, 31, 96, 4, 130)[i % 6] for i in range(count)]
+    doc = {"layers": [{"size": P, "name": "input", "type": "input"}] +
+           [{"size": n, "name": "l%d" % i, "type": "feedforward_tanh", "bias": 0.8} for i, n in enumerate(sizes)] +
+           [{"size": Q, "name": "out", "type": "feedforward_identity", "bias": 1.0}, {"size": Q, "name": "post", "type": "sse"}]}
+    net = capi.Network(json.dumps(doc), S, T)
+    gen = torch.Generator(device="cuda").manual_seed(count)
+    net.weights.uniform_(-0.3, 0.3, generator=gen)
+    pat = PC.dev(make_pat_types(lengths, T))
+    valid = (pat != 0).reshape(-1, 1)
+    x = (torch.randn(S * T, P, device="cuda", generator=gen) * valid).reshape(-1)
+    target = (torch.randn(S * T, Q, device="cuda", generator=gen) * valid).reshape(-1)
+    net.load_sequences(pat, T, min(lengths), x, target)
+    net.forward()
+    net.calculate_error()
+    net.updates.fill_(7.0)
+    net.backward()
+    torch.cuda.synchronize()
+    below, at = x.double().reshape(S * T, P), 0
+    for i, n in enumerate(sizes + [Q]):
+        name = "l%d" % i if i < count else "out"
+        layer = net.layer(name)
+        delta = layer["errors"].double().reshape(S * T, n)
+        bias = 0.8 if i < count else 1.0
+        w = below.shape[1] * n
+        got, got_bias = net.updates[at:at + w].double().reshape(n, -1), net.updates[at + w:at + w + n].double()
+        k = 2.0 ** -24 * (S * T + 2)
+        assert float(delta.abs().sum()) > 0
+        assert bool(((got - delta.T.contiguous() @ below).abs() <= k * (delta.abs().T.contiguous() @ below.abs())).all()), name
+        assert bool(((got_bias - bias * delta.sum(0)).abs() <= k * bias * delta.abs().sum(0)).all()), name
+        below, at = layer["outputs"].double().reshape(S * T, n), at + w + n
+    assert at == net.n_weights
+    net.close()
+
+
 @pytest.mark.parametrize("T", [40, 700])
 def test_weight_gradients_of_a_fraction_without_a_valid_slot(T):
     """Every weight gradient over an empty list of slots is zero, whatever the updates held: one split, several, narrow and wide."""
