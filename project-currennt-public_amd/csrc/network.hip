@@ -1619,21 +1619,18 @@ static bool has_weight_half(const cnt::NetLayer &L) {
 }
 
 // A small pass's weight halves stay on the caller's stream: a hop to another stream and back takes the host some 25 us and the
-// card 18, a product of few blocks over few slots 5 to 8.  The line goes by the multiply-adds of the weight gradients; a feed-forward
-// network, whose pass has no recursion to hide the host's time behind, has a later one.  Us per pass on other streams / in line, slots
-// in brackets: three layers of 256 (120) 142 / 90, (960) 146 / 104, (1920) 149 / 129; three of 1024 (480, 1.2e9) 187 / 169, (960, 2.4e9)
-// 248 / 263; 32 and blstm 128 (120) 161 / 130, (960) 393 / 384, (1920) 408 / 410; two lstm 256 (240, 2.4e8) 358 / 335, (480) 507 / 507, (960) 846 /
-// 851; the acoustic model (60) 443 / 411, (120, 4.4e8) 363 / 341, (240) 426 / 434, (480) 616 / 632.
+// card 18, and in line the products of few blocks are one launch.  The line goes by the multiply-adds of the weight gradients, and by the
+// slots, beyond which those products are cut along k.  Us per pass on other streams / in line, slots in brackets: three layers of 256
+// (120) 142 / 70, (960) 137 / 76, (1920) 142 / 90; three of 1024 (480, 1.2e9) 188 / 162, (960, 2.4e9) 267 / 256, (1920, 4.8e9) 312 / 332; 32 and
+// blstm 128 (240) 150 / 132, (960) 368 / 347, (1920) 382 / 359; two lstm 256 (240) 316 / 298, (960) 823 / 807, (1920, 2e9) 872 / 831; the acoustic
+// model (60) 395 / 374, (240) 435 / 396, (480, 1.8e9) 636 / 592, (960, 3.5e9) 977 / 974, (1920, 7e9) 1130 / 1162.
 static bool weights_in_line(const cnt_network *net) {
     using namespace cnt;
     const long slots = static_cast<long>(net->S) * net->T;
     if (slots > 2048) return false;
-    bool recurrent = false;
-    for (const NetLayer &L : net->layers) {
+    for (const NetLayer &L : net->layers)
         if (L.kind == K_CNN || L.kind == K_WAVNETC) return false;  // (their products are batched over layers)
-        recurrent = recurrent || L.kind == K_LSTM;
-    }
-    return static_cast<double>(net->n_weights) * static_cast<double>(slots) <= (recurrent ? 4.5e8 : 1.3e9);
+    return static_cast<double>(net->n_weights) * static_cast<double>(slots) <= 3e9;
 }
 
 int cnt_network_backward(cnt_network *net, void *stream_) {

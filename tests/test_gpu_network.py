@@ -235,8 +235,8 @@ def test_weight_gradients_of_large_tiles_over_listed_slots(lengths):
 @pytest.mark.parametrize("layers,S,T", [
     ([("feedforward_tanh", 32), ("blstm", 128)], 4, 30),                                  # in line
     ([("feedforward_tanh", 16), ("lstm", 16)], 1, 2048), ([("feedforward_tanh", 16), ("lstm", 16)], 1, 2049),  # either side of the slots
-    ([("blstm", 512), ("blstm", 512)], 3, 48), ([("blstm", 512), ("blstm", 512)], 3, 50),  # 4.4e8 and 4.6e8 multiply-adds
-    ([("feedforward_logistic", 700), ("feedforward_tanh", 700)], 8, 160), ([("feedforward_logistic", 700), ("feedforward_tanh", 700)], 8, 320)])
+    ([("blstm", 512), ("blstm", 512)], 8, 170), ([("blstm", 512), ("blstm", 512)], 8, 176),  # 2.9e9 and 3.1e9 multiply-adds
+    ([("feedforward_logistic", 1300), ("feedforward_tanh", 1300)], 8, 206), ([("feedforward_logistic", 1300), ("feedforward_tanh", 1300)], 8, 222)])
 def test_weight_halves_on_other_streams_and_in_line(layers, S, T):
     """Where the weight halves of a pass run is the sequencer's choice: the gradients, and those of a second pass over other
     lengths, are the ones of a network told to use the caller's stream alone.  (The products sum over the same slots in the same
