@@ -446,6 +446,7 @@ CnnTaps cnn_taps(const cnt_cnn *h);
 int dense_backward_weights_batch(hipStream_t stream, int P, int D, int N, int count, const float *bias,
                                  const float *const *x, const float *const *err, float *const *weight_updates, const SlotOrder *order = nullptr,
                                  DirectGroup *group = nullptr);
+bool dense_weights_direct(int P, int D, int N, int count);  // whether that is the kernel for few blocks
 int wavnetc_backward_weights_batch(hipStream_t stream, int D, int C, int N, int count, const float *ctx,
                                    const float *const *ctx_tanh, float *const *weight_updates);
 // Convolution layers with one filter group each and the same sizes, window and causality (dilations may differ):

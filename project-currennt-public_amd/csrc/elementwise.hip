@@ -432,6 +432,13 @@ extern "C++" int cnt::dense_backward_weights_batch(hipStream_t stream, int P, in
     return CNT_OK;
 }
 
+extern "C++" bool cnt::dense_weights_direct(int P, int D, int N, int count) {
+    GemmArgs ga = {};
+    ga.m = P; ga.n = D; ga.k = N;
+    ga.nseg = 1; ga.nprob = count; ga.splitk = 0;
+    return direct_product(ga);
+}
+
 int cnt_dense_backward_weights_static(void *stream, int P, int D, int N, float bias, const float *x, const float *err,
                                       float *weight_updates) {
     using namespace cnt;

@@ -1760,10 +1760,16 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         std::vector<size_t> layers;
     };
     std::vector<ShapeGroup> groups;
+    bool recurrent = false;
+    for (const NetLayer &L : net->layers) recurrent = recurrent || L.kind == K_LSTM;
     auto hand_over_group = [&](ShapeGroup &g) -> int {
         if (g.layers.empty()) return CNT_OK;
-        hipStream_t ws;
-        CNT_TRY(next_side_stream(&ws, false));
+        hipStream_t ws = stream;
+        // Dense layers' products of few blocks wait for the pass's end, where all of them are one launch, unless there are recursions to
+        // run them beside: a hop for each took the host longer than the card the product (eight small WaveNet blocks, whose
+        // pass the host bounds, 287 -> 267 us).
+        const bool waits = g.kind == K_DENSE && !recurrent && !captured && dense_weights_direct(g.a, g.b, g.n, (int)g.layers.size());
+        if (!waits) CNT_TRY(next_side_stream(&ws, false));
         const int count = (int)g.layers.size();
         const float *in0[kGemmMaxProb], *in1[kGemmMaxProb];
         float *dW[kGemmMaxProb], bias[kGemmMaxProb];
