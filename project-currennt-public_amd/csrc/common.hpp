@@ -247,6 +247,11 @@ struct GemmArgs {
     int fan_n;                   // EPI_FAN: device tables of fan_n targets and their flags
     float *const *fan_targets;
     const int *fan_is_skip;
+    // Columns of the output that may be left out (k-contiguous B, EPI_STORE and EPI_STORE_DELTA, one k range): column j of the product
+    // is column cols[j] of B and C, and from cols_count[0] on the columns get zeros, which is what their products come to
+    // (SlotOrder: the slots of a fraction, those of its padding behind the others).  The kernel for few blocks ignores the list.
+    const int *cols;
+    const int *cols_count;
     float *partial;        // scratch of splitk * partial_stride floats: the stream's buffer (set by gemm_plan) or the caller's
     size_t partial_stride;  // floats per split: nprob * m * n (+ nprob * n with rowsum), rounded up to a multiple of four
     int xcd_map;            // set by gemm_launch: workgroups pick their tile by XCD (gemm_kernel.hpp)
@@ -379,7 +384,7 @@ struct FanOut {
 // with several filter groups, leave it to the caller).
 int dense_backward_errors_fan(hipStream_t stream, int P, int D, int N, int act, const float *weights, const float *y,
                               float *err, float *prev_err, const FanOut *fan, bool *fused, int prev_act = ACT_IDENTITY,
-                              const float *prev_y = nullptr);
+                              const float *prev_y = nullptr, const SlotOrder *order = nullptr);
 // (prev_act, prev_y): the preceding layer is a dense layer with that activation and those outputs, and nothing but
 // this product writes its output errors: the product stores act'(prev_y) * error, the preceding layer's deltas, and
 // that layer's own backward step then runs with ACT_IDENTITY.  The same for a recurrent layer's error product:

@@ -347,7 +347,7 @@ int cnt_dense_backward_errors(void *stream, int P, int D, int N, int act, const 
 
 extern "C++" int cnt::dense_backward_errors_fan(hipStream_t stream, int P, int D, int N, int act, const float *weights,
                                                 const float *y, float *err, float *prev_err, const FanOut *fan,
-                                                bool *fused, int prev_act, const float *prev_y) {
+                                                bool *fused, int prev_act, const float *prev_y, const SlotOrder *order) {
     if (fused) *fused = false;
     CNT_REQUIRE(weights && y && err, "dense_backward_errors: null argument");
     CNT_REQUIRE(P > 0 && D > 0 && N > 0, "dense_backward_errors: non-positive size");
@@ -379,6 +379,7 @@ extern "C++" int cnt::dense_backward_errors_fan(hipStream_t stream, int P, int D
             ga.prob[0].aux_in = fan->from_skip;
             *fused = true;
         }
+        if (order) { ga.cols = order->order; ga.cols_count = order->count; }
         ga.label = "gemm:dense_prev_errors";
         CNT_TRY(gemm_launch(stream, ga));
     }

@@ -456,6 +456,7 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in, DirectGroup *group)
         return CNT_OK;
     }
     if (args.epilogue != EPI_PARTIAL && args.epilogue != EPI_ATOMIC && args.epilogue != EPI_STORE) args.rowsum = 0;
+    if (args.masked || !args.b_kcontig || args.splitk != 1 || (args.epilogue != EPI_STORE && args.epilogue != EPI_STORE_DELTA)) args.cols = nullptr;
     const int tile = pick_tile(args);
     const int edge = tile == kEightWaves ? 128 : tile;
     // a list of k lines is used where the kernel that reads through it exists, and ignored otherwise (the lines it leaves

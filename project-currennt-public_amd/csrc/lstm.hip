@@ -1115,6 +1115,8 @@ int cnt_lstm_forward(cnt_lstm *h, void *stream_, const float *weights, const flo
             pb.B[0] = x;
             pb.C = h->state[dir][g];
         }
+    // (the recursion leaves padding slots out; what it finds there as pre-activations reaches nothing)
+    ga.cols = h->slot_order.order; ga.cols_count = h->slot_order.count;
     ga.label = "gemm:lstm_input_projection";
     CNT_TRY(gemm_launch(stream, ga));
 
@@ -1225,6 +1227,7 @@ int cnt_lstm_backward_prev_errors_range(cnt_lstm *h, void *stream_, const float 
                 ga.prob[0].B[dir * 4 + g] = h->state[dir][7 + g] + first * H;
             }
         ga.prob[0].C = prev_errors + first * P;
+        if (t_begin == 0 && t_end == h->T) { ga.cols = h->slot_order.order; ga.cols_count = h->slot_order.count; }  // (no deltas on padding)
         ga.label = "gemm:lstm_prev_errors";
         CNT_TRY(gemm_launch(stream, ga));
     }
@@ -1253,6 +1256,7 @@ extern "C++" int cnt::lstm_prev_errors_delta(cnt_lstm *h, hipStream_t stream, co
         }
     ga.prob[0].C = prev_errors;
     ga.prob[0].aux_in = prev_y;
+    ga.cols = h->slot_order.order; ga.cols_count = h->slot_order.count;
     ga.label = "gemm:lstm_prev_errors";
     return gemm_launch(stream, ga);
 }

@@ -1976,7 +1976,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                         const bool below = !wanted && prev_err == prev.err && prev.N == N && delta_target(i - 1);
                         CNT_TRY(dense_backward_errors_fan(stream, prev.size, L.size, N, ACT_IDENTITY, W, L.out, L.err, prev_err,
                                                           wanted ? &fan : nullptr, &fused, below ? prev.act : ACT_IDENTITY,
-                                                          below ? prev.out : nullptr));
+                                                          below ? prev.out : nullptr, &L.order));
                         if (below) delta_done[i - 1] = 1;
                         fan_done[i - 1] = fused ? 1 : 0;
                         break;
@@ -1985,7 +1985,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                         const bool below = !wanted && prev_err && prev_err == prev.err && prev.N == N && delta_target(i - 1);
                         CNT_TRY(dense_backward_errors_fan(stream, prev.size, L.size, N, delta_done[i] ? ACT_IDENTITY : L.act, W,
                                                           L.out, L.err, prev_err, wanted ? &fan : nullptr, &fused,
-                                                          below ? prev.act : ACT_IDENTITY, below ? prev.out : nullptr));
+                                                          below ? prev.act : ACT_IDENTITY, below ? prev.out : nullptr, &L.order));
                         if (below) delta_done[i - 1] = 1;
                     } else
                         CNT_TRY(cnn_backward_errors_fan(L.cnn, stream, L.pat, L.T, W, L.out, L.err, prev_err,

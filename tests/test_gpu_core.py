@@ -758,6 +758,14 @@ def test_lstm_small_gradients_of_a_whole_backward_call(L, bidir, lengths):
     layer.close()
 
 
+@pytest.mark.parametrize("P,L,bidir,lengths", [
+    (61, 512, True, [130, 125] + [20] * 18), (382, 300, True, [513] + [70] * 9), (40, 256, False, [700, 1, 1, 1]), (128, 400, True, [65] * 30 + [17] * 8)])
+def test_lstm_products_of_a_fraction_with_padding(P, L, bidir, lengths):
+    """Input projections and errors of the layer below over the listed slots, against the oracle; slots of padding are zeros."""
+    print("lstm products with padding", P, L, bidir, lengths, flush=True)
+    assert PC.run_lstm_case(P, L, bidir, lengths, seed=P + L) < TOL
+
+
 def _product(m, n, k, tA, tB, A, B):
     import torch
     C = torch.empty(m * n, device="cuda")

@@ -316,6 +316,52 @@ def test_weight_gradients_of_a_small_pass_in_one_launch(lengths, count):
     net.close()
 
 
+@pytest.mark.parametrize("sizes,lengths", [
+    ([300, 700], [900, 700, 600, 500, 11]), ([299, 701], [900, 700, 600, 500, 11]), ([1024, 1028], [1700] + [900] * 6),  # three tiles
+    ([512, 512], [64] * 64 + [1] * 8), ([130, 640], [3000, 1, 1]), ([1024, 1024], [2100, 1000, 1000, 1000, 1000])])
+def test_errors_of_a_fraction_with_padding(sizes, lengths):
+    """Products over the listed columns: the deltas that reach a layer against the 64-bit product of those above, zeros on every padding
+    slot whatever stood there; column counts within, at and around tiles.  (k + 4) * 2^-24 of the terms: a sum in any order and the
+    factor of the activation."""
+    import torch
+
+    print("errors with padding", sizes, lengths, flush=True)
+    capi = PC.pkg().capi
+    S, T, P, Q = len(lengths), max(lengths), 21, 9
+    sizes = sizes + [450]
+    doc = {"layers": [{"size": P, "name": "input", "type": "input"}] +
+           [{"size": n, "name": "l%d" % i, "type": "feedforward_" + ("tanh", "logistic", "identity")[i % 3], "bias": 0.8} for i, n in enumerate(sizes)] +
+           [{"size": Q, "name": "out", "type": "feedforward_identity", "bias": 1.0}, {"size": Q, "name": "post", "type": "sse"}]}
+    net = capi.Network(json.dumps(doc), S, T)
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    net.weights.uniform_(-0.1, 0.1, generator=gen)
+    pat = PC.dev(make_pat_types(lengths, T))
+    valid = (pat != 0).reshape(-1, 1)
+    x = torch.randn(S * T * P, device="cuda", generator=gen)  # (anything on padding slots)
+    target = (torch.randn(S * T, Q, device="cuda", generator=gen) * valid).reshape(-1)
+    net.load_sequences(pat, T, min(lengths), x, target)
+    net.forward()
+    net.calculate_error()
+    for i in range(len(sizes)):
+        net.layer("l%d" % i)["errors"].fill_(7.0)
+    net.backward()
+    torch.cuda.synchronize()
+    above = net.layer("out")
+    for i in range(len(sizes) - 1, -1, -1):
+        layer = net.layer("l%d" % i)
+        n, m = sizes[i], above["size"]
+        W = above["weights"][:n * m].double().reshape(m, n)
+        delta, y = above["errors"].double().reshape(S * T, m), layer["outputs"].double().reshape(S * T, n)
+        slope = (1 - y * y, y * (1 - y), torch.ones_like(y))[i % 3]
+        got = layer["errors"].double().reshape(S * T, n)
+        assert not bool(got[~valid[:, 0]].any()), i
+        bound = (m + 4) * 2.0 ** -24 * (delta.abs() @ W.abs()) * slope.abs() + 2.0 ** -22 * (delta @ W).abs()  # (1 - y y in 32 bits)
+        assert bool(((got - delta @ W * slope).abs() <= bound).all()), i
+        assert float(got.abs().sum()) > 0
+        above = layer
+    net.close()
+
+
 @pytest.mark.parametrize("T", [40, 700])
 def test_weight_gradients_of_a_fraction_without_a_valid_slot(T):
     """Every weight gradient over an empty list of slots is zero, whatever the updates held: one split, several, narrow and wide."""
