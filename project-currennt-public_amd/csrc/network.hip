@@ -20,6 +20,8 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <new>
 #include <random>
 #include <string>
@@ -509,11 +511,11 @@ struct cnt_network {
     bool skip_padding = true;
     std::vector<LowRes> low_res;
     std::vector<void *> allocations;
-    // weight gradients go round-robin to these streams (default priority); CNT_NET_SIDE_STREAMS overrides the count
-    static constexpr int kMaxSide = 4;
-    hipStream_t side[kMaxSide] = {};
-    hipEvent_t ev_main = nullptr, ev_side[kMaxSide] = {};
-    int n_side = 3;
+    // Weight gradients go to a stream beside the caller's: the one that the device's networks share (SideStream), under capture one of the
+    // network's own, since a stream that takes part in a capture may take nothing else meanwhile.
+    int device = 0;
+    hipStream_t side = nullptr, capture_side = nullptr;
+    hipEvent_t ev_main = nullptr, ev_side = nullptr;
     int overlap = 1;
     // optimizer state (allocated by the first update)
     float *cur_updates = nullptr, *deltas = nullptr, *stats = nullptr;
@@ -527,6 +529,41 @@ struct cnt_network {
 
 namespace cnt {
 namespace {
+
+// The stream (default priority) on which the networks of a device run their weight gradients, from the first network's creation to the
+// last one's end.  One for all of them: the runtime deals streams to four hardware queues, and a stream that meets the caller's on one
+// of them runs nothing beside it.  With a stream per network every third or fourth network met that: us per pass of four acoustic
+// models side by side 2495, 2484, 2670, 2490.  And one per network, not three round-robin: products that fill the card are only in each
+// other's way and in the main stream's (3 / 2 / 1: feed-forward model 2102 / 2055 / 2037, acoustic model 2500 / 2485 / 2484, 150 and 200 cells with
+// twenty sequences 2095 / 2093 / 2080, 32 sequences 2247 / 2255 / 2267).  What different networks' threads enqueue here runs in the order it came;
+// each pass waits for its own share only.
+struct SideStream {
+    hipStream_t stream = nullptr;
+    int users = 0;
+};
+struct SideStreams {
+    std::mutex mu;
+    std::map<int, SideStream> of_device;
+};
+SideStreams &side_streams() {
+    static SideStreams all;
+    return all;
+}
+int acquire_side(int device, hipStream_t *stream) {
+    SideStreams &all = side_streams();
+    std::lock_guard<std::mutex> lock(all.mu);
+    SideStream &s = all.of_device[device];
+    if (s.users == 0) {
+        CNT_HIP(hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking));
+        if (cnt::gemm_reserve_stream(s.stream) != CNT_OK) {
+            (void)hipStreamDestroy(s.stream);
+            return CNT_ERR_HIP;
+        }
+    }
+    ++s.users;
+    *stream = s.stream;
+    return CNT_OK;
+}
 
 int device_alloc(cnt_network *n, void **p, size_t bytes, bool zero) {
     CNT_HIP(hipMalloc(p, bytes ? bytes : 4));
@@ -1121,15 +1158,24 @@ int finish_build(cnt_network *net, const json::Value *weights) {
             CNT_REQUIRE(L.size == (L.fb_end - L.fb_start) + net->mdn_classes, "network: feedback layer '%s' has size "
                         "%d, expected %d + %d classes", L.name.c_str(), L.size, L.fb_end - L.fb_start, net->mdn_classes);
         }
-    if (const char *e = std::getenv("CNT_NET_SIDE_STREAMS"))
-        net->n_side = std::max(1, std::min((int)cnt_network::kMaxSide, std::atoi(e)));
+    CNT_HIP(hipGetDevice(&net->device));
+    CNT_TRY(acquire_side(net->device, &net->side));
     CNT_HIP(hipEventCreateWithFlags(&net->ev_main, cnt::kOrderEvent));
-    for (int k = 0; k < net->n_side; ++k) {
-        CNT_HIP(hipStreamCreateWithFlags(&net->side[k], hipStreamNonBlocking));
-        CNT_HIP(hipEventCreateWithFlags(&net->ev_side[k], cnt::kOrderEvent));
-        CNT_TRY(cnt::gemm_reserve_stream(net->side[k]));  // the weight halves' split-K scratch, not inside a pass
-    }
+    CNT_HIP(hipEventCreateWithFlags(&net->ev_side, cnt::kOrderEvent));
+    CNT_HIP(hipStreamCreateWithFlags(&net->capture_side, hipStreamNonBlocking));
+    CNT_TRY(cnt::gemm_reserve_stream(net->capture_side));  // the weight halves' split-K scratch, not inside a pass
     return CNT_OK;
+}
+
+void release_side(int device) {
+    SideStreams &all = side_streams();
+    std::lock_guard<std::mutex> lock(all.mu);
+    SideStream &s = all.of_device[device];
+    if (--s.users > 0) return;
+    (void)hipStreamSynchronize(s.stream);
+    cnt::gemm_release_stream(s.stream);
+    (void)hipStreamDestroy(s.stream);
+    s.stream = nullptr;
 }
 
 }  // namespace
@@ -1146,15 +1192,17 @@ int cnt_network_destroy(cnt_network *net) {
         if (L.dft) cnt_dft_destroy(L.dft);
     }
     for (void *p : net->allocations) (void)hipFree(p);
-    for (int k = 0; k < cnt_network::kMaxSide; ++k) {
-        if (net->side[k]) {
-            // the product launcher keeps a scratch buffer per stream it has seen
-            (void)hipStreamSynchronize(net->side[k]);
-            cnt::gemm_release_stream(net->side[k]);
-            (void)hipStreamDestroy(net->side[k]);
-        }
-        if (net->ev_side[k]) (void)hipEventDestroy(net->ev_side[k]);
+    if (net->side) {
+        (void)hipStreamSynchronize(net->side);
+        cnt::release_side(net->device);
     }
+    if (net->capture_side) {
+        // the product launcher keeps a scratch buffer per stream it has seen
+        (void)hipStreamSynchronize(net->capture_side);
+        cnt::gemm_release_stream(net->capture_side);
+        (void)hipStreamDestroy(net->capture_side);
+    }
+    if (net->ev_side) (void)hipEventDestroy(net->ev_side);
     if (net->ev_main) (void)hipEventDestroy(net->ev_main);
     delete net;
     return CNT_OK;
@@ -1624,12 +1672,17 @@ static bool has_weight_half(const cnt::NetLayer &L) {
 // (120) 142 / 70, (960) 137 / 76, (1920) 142 / 90; three of 1024 (480, 1.2e9) 188 / 162, (960, 2.4e9) 267 / 256, (1920, 4.8e9) 312 / 332; 32 and
 // blstm 128 (240) 150 / 132, (960) 368 / 347, (1920) 382 / 359; two lstm 256 (240) 316 / 298, (960) 823 / 807, (1920, 2e9) 872 / 831; the acoustic
 // model (60) 395 / 374, (240) 435 / 396, (480, 1.8e9) 636 / 592, (960, 3.5e9) 977 / 974, (1920, 7e9) 1130 / 1162.
-static bool weights_in_line(const cnt_network *net) {
+// Blocks of 32 / 64 and 64 / 128 channels: 8 of them (2000) 249 / 235, (4000) 268 / 280, 20 (2000) 491 / 462, 10 wide ones (2000) 446 / 422,
+// (4000) 478 / 485.  Convolutions without the blocks' launches, whose products are batched over layers on another stream, stay there: 20 of
+// 48 channels (2000) 1095 / 1740.
+static bool weights_in_line(const cnt_network *net, const std::vector<char> &in_block) {
     using namespace cnt;
     const long slots = static_cast<long>(net->S) * net->T;
     if (slots > 2048) return false;
-    for (const NetLayer &L : net->layers)
-        if (L.kind == K_CNN || L.kind == K_WAVNETC) return false;  // (their products are batched over layers)
+    for (size_t i = 0; i < net->layers.size(); ++i) {
+        const NetLayer &L = net->layers[i];
+        if ((L.kind == K_CNN || L.kind == K_WAVNETC) && has_weight_half(L) && !in_block[i]) return false;
+    }
     return static_cast<double>(net->n_weights) * static_cast<double>(slots) <= 3e9;
 }
 
@@ -1638,10 +1691,9 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     CNT_REQUIRE(net && net->T > 0, "network_backward: no fraction loaded");
     CNT_TRY(report_failure(net, static_cast<hipStream_t>(stream_)));
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    int next_side = 0;
-    bool side_used[cnt_network::kMaxSide] = {};
+    bool side_used = false;
     const bool captured = capturing(stream);  // (a graph's products take the scratch that the side streams have reserved)
-    const bool overlap = net->overlap && (captured || !weights_in_line(net));
+    const hipStream_t side = captured ? net->capture_side : net->side;
     // Nothing runs on the caller's stream behind the error half of the lowest layer with weights, so its weight half, and what
     // is still waiting by then, stays there: two hops between streams (9 us each) less in front of the optimizer.
     // Mixture-density output over 6000 slots 189.5 -> 169 us per pass, eight small WaveNet blocks 316 -> 297.
@@ -1686,6 +1738,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     std::vector<char> in_block(net->layers.size(), 0);  // weight gradients in the blocks' common launches
     for (size_t i = 5; i < net->layers.size(); ++i)
         if (block_at(i) && block_weights_at(net, i)) in_block[i] = in_block[i - 3] = in_block[i - 4] = in_block[i - 5] = 1;
+    const bool overlap = net->overlap && (captured || !weights_in_line(net, in_block));
     std::vector<size_t> pending;
     DirectGroup in_line;  // products of few blocks on the caller's stream: one launch at the end of the pass
     in_line.count = in_line.blocks = 0;
@@ -1702,51 +1755,24 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         if (L.kind == K_CNN) return cnt_cnn_backward_weights(L.cnn, ws, L.pat, L.T, prev.out, L.err, dW);
         return cnt_wavnetc_backward_weights(ws, L.size, L.ctx_dim, L.N, net->ctx, L.cgrad, dW);
     };
-    // Large layers' weight halves go round-robin over all side streams, the collected small ones over the first two:
-    // measured on MI355X, a third stream gains 1% on the acoustic model (its last recurrent layer's and the dense
-    // layers' weight gradients end the pass side by side) and loses 2% on the WaveNet stack (three batched products
-    // at once crowd the error chain on the main stream).
-    int next_small = 0;
     cnt_lstm *after_recursion = nullptr;  // set: the side stream waits for this layer's recursion, just launched
-    auto next_side_stream = [&](hipStream_t *ws, bool large) -> int {
-        if (at_end) {
-            *ws = stream;
-            return CNT_OK;
-        }
-        int &cursor = large ? next_side : next_small;
-        const int span = large ? net->n_side : std::min(net->n_side, 2);
-        cursor %= span;
-        *ws = net->side[cursor];
+    auto weight_stream = [&](hipStream_t *ws) -> int {
+        *ws = at_end ? stream : side;
+        if (at_end) return CNT_OK;
         if (after_recursion) {
             CNT_TRY(lstm_wait_recursion(after_recursion, *ws));
         } else {
             CNT_HIP(hipEventRecord(net->ev_main, stream));
             CNT_HIP(hipStreamWaitEvent(*ws, net->ev_main, 0));
         }
-        side_used[cursor] = true;
-        cursor = (cursor + 1) % span;
+        side_used = true;
         return CNT_OK;
     };
-    auto hand_over = [&](bool large) -> int {
+    auto hand_over = [&]() -> int {
         if (pending.empty()) return CNT_OK;
         hipStream_t ws;
-        CNT_TRY(next_side_stream(&ws, large));
-        static const bool split_lstm = [] { const char *e = std::getenv("CNT_NET_SPLIT_LSTM_WEIGHTS"); return e && std::atoi(e) != 0; }();
-        for (size_t i : pending) {
-            NetLayer &L = net->layers[i];
-            if (L.kind == K_LSTM && split_lstm && net->n_side >= 2) {
-                // CNT_NET_SPLIT_LSTM_WEIGHTS=1: the input-weight product and the recurrent-weight product (with the bias /
-                // peephole sums) of a recurrent layer, which write disjoint ranges, side by side on two streams.  Off by
-                // default: one after the other on one stream they take less from the recursion of the layer below and from
-                // the error product beside them (acoustic model 2.51 -> 2.44 ms on MI355X).
-                CNT_TRY(lstm_backward_weights_parts(L.lstm, ws, net->layers[i - 1].out, net->updates + L.w_off, 1));
-                hipStream_t ws2;
-                CNT_TRY(next_side_stream(&ws2, large));
-                CNT_TRY(lstm_backward_weights_parts(L.lstm, ws2, net->layers[i - 1].out, net->updates + L.w_off, 2 | kSumsDone));
-            } else {
-                CNT_TRY(weight_half(i, ws));
-            }
-        }
+        CNT_TRY(weight_stream(&ws));
+        for (size_t i : pending) CNT_TRY(weight_half(i, ws));
         pending.clear();
         return CNT_OK;
     };
@@ -1769,7 +1795,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         // run them beside: a hop for each took the host longer than the card the product (eight small WaveNet blocks, whose
         // pass the host bounds, 287 -> 267 us).
         const bool waits = g.kind == K_DENSE && !recurrent && !captured && dense_weights_direct(g.a, g.b, g.n, (int)g.layers.size());
-        if (!waits) CNT_TRY(next_side_stream(&ws, false));
+        if (!waits) CNT_TRY(weight_stream(&ws));
         const int count = (int)g.layers.size();
         const float *in0[kGemmMaxProb], *in1[kGemmMaxProb];
         float *dW[kGemmMaxProb], bias[kGemmMaxProb];
@@ -1835,10 +1861,10 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         if (blocks.empty()) return CNT_OK;
         hipStream_t ws = stream;
         if (overlap) {  // always the one stream: the launches share their scratch
-            ws = net->side[0];
+            ws = side;
             CNT_HIP(hipEventRecord(net->ev_main, stream));
             CNT_HIP(hipStreamWaitEvent(ws, net->ev_main, 0));
-            side_used[0] = true;
+            side_used = true;
         }
         BlockGradients g[kBlockGradients];
         const NetLayer &first = net->layers[blocks[0]];
@@ -1972,7 +1998,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                         CNT_TRY(dense_backward_errors_fan(stream, prev.size, L.size, N, delta_done[i] ? ACT_IDENTITY : L.act, W,
                                                           L.out, L.err, nullptr, nullptr, nullptr));
                         pending.push_back(i);
-                        CNT_TRY(hand_over(true));
+                        CNT_TRY(hand_over());
                         const bool below = !wanted && prev_err == prev.err && prev.N == N && delta_target(i - 1);
                         CNT_TRY(dense_backward_errors_fan(stream, prev.size, L.size, N, ACT_IDENTITY, W, L.out, L.err, prev_err,
                                                           wanted ? &fan : nullptr, &fused, below ? prev.act : ACT_IDENTITY,
@@ -2002,7 +2028,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                         if (overlap) {
                             pending.push_back(i);
                             after_recursion = lstm_is_persistent(L.lstm) ? L.lstm : nullptr;
-                            const int handed = hand_over(true);
+                            const int handed = hand_over();
                             after_recursion = nullptr;
                             CNT_TRY(handed);
                         }
@@ -2054,7 +2080,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                     // measured best on the 30-block WaveNet stack (5.36 -> 5.23 ms; two: no gain, eight: 5.31 ms)
                     const double macs = (double)prev.size * L.size * N;
                     const bool large = L.kind == K_LSTM || macs >= 4e8;
-                    if (large || pending.size() >= 4) CNT_TRY(hand_over(large));
+                    if (large || pending.size() >= 4) CNT_TRY(hand_over());
                 }
                 break;
             case K_SKIPINI:
@@ -2110,13 +2136,12 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         }
     }
     CNT_TRY(hand_over_blocks());
-    CNT_TRY(hand_over(false));
+    CNT_TRY(hand_over());
     for (ShapeGroup &g : groups) CNT_TRY(hand_over_group(g));
     CNT_TRY(gemm_group_launch(stream, in_line));
-    for (int k = 0; k < net->n_side; ++k) {
-        if (!side_used[k]) continue;
-        CNT_HIP(hipEventRecord(net->ev_side[k], net->side[k]));
-        CNT_HIP(hipStreamWaitEvent(stream, net->ev_side[k], 0));
+    if (side_used) {
+        CNT_HIP(hipEventRecord(net->ev_side, side));
+        CNT_HIP(hipStreamWaitEvent(stream, net->ev_side, 0));
     }
     return CNT_OK;
 }

@@ -362,6 +362,82 @@ def test_errors_of_a_fraction_with_padding(sizes, lengths):
     net.close()
 
 
+def test_networks_share_the_stream_of_their_weight_gradients():
+    """Networks on streams and threads of their own, one of them destroyed while the others go on, a new one made, and one more pass
+    under capture beside them: every pass's gradients are those of a network that uses the caller's stream alone (1e-6, as
+    above)."""
+    import threading
+
+    import torch
+
+    capi = PC.pkg().capi
+    S, T, P, Q = 6, 500, 40, 30
+    doc = json.dumps({"layers": [{"size": P, "name": "input", "type": "input"}, {"size": 256, "name": "a", "type": "feedforward_tanh", "bias": 1.0},
+                                 {"size": 128, "name": "b", "type": "blstm", "bias": 1.0},
+                                 {"size": Q, "name": "out", "type": "feedforward_identity", "bias": 1.0}, {"size": Q, "name": "post", "type": "sse"}]})
+    pat = PC.dev(make_pat_types([T] * S, T))
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x, target = (torch.randn(S * T * n, device="cuda", generator=gen) for n in (P, Q))
+    weights = None
+
+    def made(overlap=True):
+        nonlocal weights
+        net = capi.Network(doc, S, T, overlap=overlap)
+        if weights is None:
+            weights = net.weights.uniform_(-0.1, 0.1, generator=gen).clone()
+        net.weights.copy_(weights)
+        return net
+
+    def passed(net, stream=None):
+        net.load_sequences(pat, T, T, x, target, stream=stream)
+        net.forward(stream=stream)
+        net.calculate_error(stream=stream)
+        net.backward(stream=stream)
+
+    alone = made(False)
+    passed(alone)
+    torch.cuda.synchronize()
+    want = alone.updates.clone()
+    nets = [made() for _ in range(3)]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(net):
+        stream = torch.cuda.Stream()
+        for _ in range(4):
+            net.updates.fill_(3.0)
+            torch.cuda.synchronize()
+            passed(net, stream)
+            stream.synchronize()
+            if not float((net.updates - want).norm()) <= 1e-6 * float(want.norm()):
+                wrong.append(net)
+
+    threads = [threading.Thread(target=work, args=(n,)) for n in nets[:2]]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    nets[0].close()
+    nets.append(made())
+    for net in nets[1:]:
+        passed(net)
+    torch.cuda.synchronize()
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        passed(nets[1], torch.cuda.current_stream())
+    for _ in range(3):
+        nets[1].updates.fill_(3.0)
+        nets[2].updates.fill_(3.0)
+        graph.replay()
+        passed(nets[2])
+        torch.cuda.synchronize()
+        for net in nets[1:]:
+            assert float((net.updates - want).norm()) <= 1e-6 * float(want.norm())
+    for net in nets[1:] + [alone]:
+        net.close()
+
+
 @pytest.mark.parametrize("T", [40, 700])
 def test_weight_gradients_of_a_fraction_without_a_valid_slot(T):
     """Every weight gradient over an empty list of slots is zero, whatever the updates held: one split, several, narrow and wide."""
