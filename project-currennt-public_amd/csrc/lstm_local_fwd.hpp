@@ -293,11 +293,14 @@ __device__ __forceinline__ void forward_job(const ChainParams &p, const LocalJob
     float wreg[4 * BLOCKS];
     {
         const int o = lane % ROWS, g = o % 4, jj = o / 4;
-        const float *wg = D.w_int + (size_t)g * p.L * H + (size_t)(j0 + jj) * H;
+        const bool has_row = j0 + jj < H;
+        const float *wg = D.w_int + (size_t)g * p.L * H + (size_t)(has_row ? j0 + jj : 0) * H;
+        const int from = 64 * pw + 4 * BLOCKS * (lane / ROWS);
+        if constexpr (JB == 16) {
+            load_weight_row(wg, has_row, from, H, wreg);
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4 * BLOCKS; ++i) {
-            const int from = 64 * pw + 4 * BLOCKS * (lane / ROWS) + i;
-            wreg[i] = from < H && j0 + jj < H ? wg[from] : 0.0f;
+            for (int i = 0; i < 4 * BLOCKS; ++i) wreg[i] = from + i < H && has_row ? wg[from + i] : 0.0f;
         }
     }
     // a lane past the end of the block polls the block's first vector instead and multiplies zeros

@@ -216,9 +216,13 @@ __global__ __launch_bounds__(solo_threads(NW)) __attribute__((amdgpu_waves_per_e
     // B operand: lane = 16 * gate + cell of the wave
     float wreg[K];
     {
-        const float *wg = D.w_int + (size_t)(lane >> 4) * p.L * H + (size_t)cell * H;
+        const float *wg = D.w_int + (size_t)(lane >> 4) * p.L * H + (size_t)(cell < H ? cell : 0) * H;
+        if constexpr (CELLS == kSingle) {
 #pragma unroll
-        for (int k = 0; k < K; ++k) wreg[k] = cell < H && k < H ? wg[k] : 0.0f;
+            for (int k = 0; k < K; ++k) wreg[k] = cell < H && k < H ? wg[k] : 0.0f;
+        } else {
+            load_weight_row(wg, cell < H, 0, H, wreg);
+        }
     }
     f32x4 bias = {0, 0, 0, 0};
     float p_ig = 0, p_fg = 0, p_og = 0;
