@@ -227,70 +227,84 @@ __global__ __launch_bounds__(NT, (CONV || K > 128) ? 1 : 2) void wavenet_block_e
     const bool ok = n_raw < a.N;
     const size_t n = ok ? n_raw : a.N - 1;  // lanes past the end compute on the last sample and store nothing
 
-    // every global read that does not depend on a product is requested up front
-    constexpr int T1 = K * R / 4, T2 = R * R / 4, TC = 2 * R * R / 4;  // 16-byte pieces
-    constexpr int F1 = (T1 + NT - 1) / NT, F2 = (T2 + NT - 1) / NT, FC = CONV ? (TC + NT - 1) / NT : 0;
-    float4 s1[F1], s2[F2];
+    // Every global read that does not depend on a product is requested up front, the weights first: with the folded convolution's
+    // requested behind the others' way into LDS the launch waited for memory three times over, one trip after the other.
+    // Weights: a thread takes four channels of four neighbouring k, so that what goes to LDS is 16 bytes of k per channel, side by
+    // side (one value at a time it was four times the stores, four to a bank).  Eight blocks of 32 and 64 channels over 2000 samples 226 -> 222 us
+    // per pass; 30 of 64 and 128 over 32 000, which the memory bounds, 3379 both ways.
+    constexpr int T1 = K * R / 16, T2 = R * R / 16, TC = CONV ? 2 * R * R / 16 : 0;  // such pieces
+    constexpr int F1 = (T1 + NT - 1) / NT, F2 = (T2 + NT - 1) / NT, FC = (TC + NT - 1) / NT;
+    auto request = [&](auto &s, auto pieces, const float *w, int ld) __attribute__((always_inline)) {
+        constexpr int T = decltype(pieces)::value;
 #pragma unroll
-    for (int q = 0; q < F1; ++q)
-        if (q * NT + tid < T1) s1[q] = reinterpret_cast<const float4 *>(a.w_skip)[q * NT + tid];
+        for (int q = 0; q < (T + NT - 1) / NT; ++q) {
+            const int at = q * NT + tid, k = at / (R / 4) * 4, ch = at % (R / 4) * 4;
+            if (T % NT == 0 || at < T)
 #pragma unroll
-    for (int q = 0; q < F2; ++q)
-        if (q * NT + tid < T2) s2[q] = reinterpret_cast<const float4 *>(a.w_out)[q * NT + tid];
+                for (int i = 0; i < 4; ++i) s[q][i] = *reinterpret_cast<const f32x4v *>(w + (size_t)(k + i) * ld + ch);
+        }
+    };
+    auto stage = [&](float *w, int J, const auto &s, auto pieces) __attribute__((always_inline)) {
+        constexpr int T = decltype(pieces)::value;
+#pragma unroll
+        for (int q = 0; q < (T + NT - 1) / NT; ++q) {
+            const int at = q * NT + tid, k = at / (R / 4) * 4, ch = at % (R / 4) * 4;
+            float *const dst = w + (((ch / 16 * J + k / 16) * 4 + (k >> 2 & 3)) * 16 + ch % 16) * 4;
+            if (T % NT == 0 || at < T)
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    *reinterpret_cast<f32x4v *>(dst + 4 * c) = f32x4v{s[q][0][c], s[q][1][c], s[q][2][c], s[q][3][c]};
+        }
+    };
+    const std::integral_constant<int, T1> t1; const std::integral_constant<int, T2> t2; const std::integral_constant<int, TC> tc;
+    f32x4v s1[F1][4], s2[F2][4], sc0[FC > 0 ? FC : 1][4];
+    f32x4v sc1[FC > 0 ? FC : 1][4];  // the second tap's weights wait in registers until the first tap's products are done
+    request(s1, t1, a.w_skip, R);
+    request(s2, t2, a.w_out, R);
+    if (CONV) {
+        request(sc0, tc, a.conv_w[0], a.conv_ld);
+        request(sc1, tc, a.conv_w[1], a.conv_ld);
+    }
     float4 b1[KJ];
     {
         const float4 *src = reinterpret_cast<const float4 *>(a.e_skip + n * K + 4 * quarter);
 #pragma unroll
         for (int j = 0; j < KJ; ++j) b1[j] = src[4 * j];
     }
+    const char own_pat = a.pat[n];
+    // folded convolution: tap q contributes sum_d Wc[d][tap q][p] * delta[slot n + shift q][d], counted only where both
+    // slots are inside the fraction and not padding (the rule of the convolution layer's own error product)
+    float4 bc[CONV ? 2 : 1][CONV ? CJ : 1];
+    char tap_pat[2] = {0, 0};
+    bool inside[2] = {false, false};
+    if (CONV) {
+#pragma unroll
+        for (int tap = 0; tap < 2; ++tap) {
+            const long long src = (long long)n + a.conv_shift[tap];
+            inside[tap] = src >= 0 && src < a.N;
+            const size_t sc = inside[tap] ? (size_t)src : n;
+            tap_pat[tap] = a.pat[sc];
+            const float4 *p = reinterpret_cast<const float4 *>(a.conv_deltas + sc * 2 * R + 4 * quarter);
+#pragma unroll
+            for (int j = 0; j < CJ; ++j) bc[tap][j] = p[4 * j];
+        }
+    }
     float4 side[RT];
     if (a.from_skip) {
 #pragma unroll
         for (int t = 0; t < RT; ++t) side[t] = *reinterpret_cast<const float4 *>(a.from_skip + n * R + 16 * t + 4 * quarter);
     }
-    const bool live = a.pat[n] != 0;
-    auto stage = [](float *w, int J, int idx4, const float4 &v) {
-        // element (k, ch .. ch+3): same k, four neighbouring channels of one tile
-        const int k = idx4 * 4 / R, ch = idx4 * 4 % R;
-        float *dst = w + ((((ch / 16) * J + k / 16) * 4 + ((k >> 2) & 3)) * 16 + ch % 16) * 4 + (k & 3);
-        dst[0] = v.x; dst[4] = v.y; dst[8] = v.z; dst[12] = v.w;
-    };
-#pragma unroll
-    for (int q = 0; q < F1; ++q)
-        if (q * NT + tid < T1) stage(w1, KJ, q * NT + tid, s1[q]);
-#pragma unroll
-    for (int q = 0; q < F2; ++q)
-        if (q * NT + tid < T2) stage(w2, RJ, q * NT + tid, s2[q]);
-    // folded convolution: tap q contributes sum_d Wc[d][tap q][p] * delta[slot n + shift q][d], counted only where both
-    // slots are inside the fraction and not padding (the rule of the convolution layer's own error product)
-    float4 bc[CONV ? 2 : 1][CONV ? CJ : 1];
-    float4 sc1[FC > 0 ? FC : 1];  // the second tap's weights wait in registers until the first tap's products are done
+    __builtin_amdgcn_sched_barrier(0);
+    stage(w1, KJ, s1, t1);
+    stage(w2, RJ, s2, t2);
+    if (CONV) stage(wc, CJ, sc0, tc);
+    const bool live = own_pat != 0;
     if (CONV) {
-        float4 sc0[FC > 0 ? FC : 1];
-#pragma unroll
-        for (int q = 0; q < FC; ++q) {
-            const int idx4 = q * NT + tid;
-            if (idx4 < TC) {
-                const size_t at = (size_t)(idx4 * 4 / R) * a.conv_ld + idx4 * 4 % R;
-                sc0[q] = *reinterpret_cast<const float4 *>(a.conv_w[0] + at);
-                sc1[q] = *reinterpret_cast<const float4 *>(a.conv_w[1] + at);
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < FC; ++q)
-            if (q * NT + tid < TC) stage(wc, CJ, q * NT + tid, sc0[q]);
 #pragma unroll
         for (int tap = 0; tap < 2; ++tap) {
-            const long long src = (long long)n + a.conv_shift[tap];
-            const bool inside = src >= 0 && src < a.N;
-            const size_t sc = inside ? (size_t)src : n;
-            const bool keep = live && inside && a.pat[sc] != 0;
-            const float4 *p = reinterpret_cast<const float4 *>(a.conv_deltas + sc * 2 * R + 4 * quarter);
+            const bool keep = live && inside[tap] && tap_pat[tap] != 0;
 #pragma unroll
-            for (int j = 0; j < CJ; ++j) {
-                const float4 v = p[4 * j];
-                bc[tap][j] = keep ? v : float4{0.0f, 0.0f, 0.0f, 0.0f};
-            }
+            for (int j = 0; j < CJ; ++j) bc[tap][j] = keep ? bc[tap][j] : float4{0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
     // the gate's operands and the first target's old values are requested before the products start, the four of SUM behind the
@@ -346,9 +360,7 @@ __global__ __launch_bounds__(NT, (CONV || K > 128) ? 1 : 2) void wavenet_block_e
     if (CONV) {
         if (LATE) request_gate();
         __syncthreads();  // every wave is done with the first tap's weights
-#pragma unroll
-        for (int q = 0; q < FC; ++q)
-            if (q * NT + tid < TC) stage(wc, CJ, q * NT + tid, sc1[q]);
+        stage(wc, CJ, sc1, tc);
         __syncthreads();
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
