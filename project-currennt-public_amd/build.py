@@ -26,7 +26,9 @@ FLAGS = [
 # Per-file additions.  The weight update is specified operation by operation (every product and sum rounded
 # on its own, as the reference's host and device code do), so its file is compiled without contraction into
 # fused multiply-adds; HIP's __fmul_rn / __fadd_rn are plain operators and do not prevent it.
-EXTRA_FLAGS = {"optimizer.hip": ["-ffp-contract=off"]}
+# The recursions' steps are loops of some hundred instructions by waves that have a SIMD to themselves: where their code falls on the
+# instruction cache's lines moves a step by 1 to 2 % with every change elsewhere in the kernel, so blocks that are jumped to begin a line.
+EXTRA_FLAGS = {"optimizer.hip": ["-ffp-contract=off"], "lstm.hip": ["-mllvm", "--align-all-nofallthru-blocks=6"]}
 
 
 def _compile(src):

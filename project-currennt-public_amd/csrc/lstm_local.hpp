@@ -53,10 +53,12 @@
 
 constexpr int kLocalSeqs = 4;     // sequences of a job at most
 constexpr int kLocalXcds = 8;
-// control words (zero before every launch): tickets per XCD, jobs claimed, per (XCD, team) arrivals and job; teams are
-// counted up to ChainParams::ctl_teams per XCD, which the launch makes large enough for all of its workgroups on one XCD
-constexpr int kCtlTickets = 0, kCtlClaimed = 8, kCtlArrived = 16;
-constexpr int ctl_words(int teams) { return kCtlArrived + 2 * kLocalXcds * teams; }
+// control words (zero before every launch): jobs claimed; per XCD its tickets, and per team arrivals and job.  What one XCD counts lies
+// on cache lines of its own: with all tickets on one line the eight L2s passed it around.  Teams are counted up to
+// ChainParams::ctl_teams per XCD, which the launch makes large enough for all of its workgroups on one XCD
+constexpr int kCtlLine = 32;
+constexpr int ctl_xcd_words(int teams) { return kCtlLine + (2 * teams + kCtlLine - 1) / kCtlLine * kCtlLine; }
+constexpr int ctl_words(int teams) { return kCtlLine + kLocalXcds * ctl_xcd_words(teams); }
 constexpr unsigned kNoJob = 0xFFFFFFFFu;
 
 // Elements (cell, sequence) of a workgroup of JB cells with NSQ sequences = words of a (receiver, sender) pair, the 16-byte
@@ -92,12 +94,15 @@ __device__ __forceinline__ unsigned ctl_load(const unsigned *p) {
 __device__ int local_claim_role(const ChainParams &p, int G) {
     const unsigned xcd = __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15u;  // XCC_ID, bits 3:0
     if (xcd >= 8u) return -1;
-    const unsigned ticket = __hip_atomic_fetch_add(p.ctl + kCtlTickets + xcd, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned *const claimed = p.ctl, *const own = p.ctl + kCtlLine + xcd * (unsigned)ctl_xcd_words(p.ctl_teams);
+    // (A workgroup that finds all jobs taken ends at once.  Those the compute units had no room for come when the recursion is over, and
+    // the launch lasts until they are gone.)
+    const unsigned taken = ctl_load(claimed);
+    const unsigned ticket = __hip_atomic_fetch_add(own, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (taken >= (unsigned)p.njobs) return -1;
     const unsigned team = ticket / (unsigned)G, member = ticket % (unsigned)G;
     if (team >= (unsigned)p.ctl_teams) return -1;
-    unsigned *arrived = p.ctl + kCtlArrived + xcd * (unsigned)p.ctl_teams + team;
-    unsigned *team_job = arrived + kLocalXcds * p.ctl_teams;
-    unsigned *claimed = p.ctl + kCtlClaimed;
+    unsigned *const arrived = own + kCtlLine + 2 * team, *const team_job = arrived + 1;
     const unsigned before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     unsigned job = 0;  // 0: undecided, j + 1: job j, kNoJob: none
     if (before == (unsigned)G - 1u) {
@@ -117,13 +122,13 @@ __device__ int local_claim_role(const ChainParams &p, int G) {
             job = ctl_load(team_job);
             if (job != 0u) break;
             // every job is taken and this team is still incomplete: whoever completes it will find none left
-            if (ctl_load(claimed) >= (unsigned)p.njobs && ctl_load(arrived) < (unsigned)G) { job = kNoJob; break; }
-            if (++spins > p.spin_limit || __hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+            if ((spins & 3u) == 3u && ctl_load(claimed) >= (unsigned)p.njobs && ctl_load(arrived) < (unsigned)G) { job = kNoJob; break; }
+            if (++spins > p.spin_limit || ((spins & 15u) == 0u && __hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
                 raise_abort(p);
                 job = kNoJob;
                 break;
             }
-            __builtin_amdgcn_s_sleep(4);
+            __builtin_amdgcn_s_sleep(2);
         }
     }
     if (job == kNoJob) return -1;
@@ -152,30 +157,88 @@ template <bool FWD>
 __host__ __device__ constexpr long long job_cost(int steps, int sequences) { return (long long)steps * step_cost<FWD>(sequences); }
 static_assert(job_cost<true>(0x7FFFFFFF, 4) == 0x7FFFFFFFLL * 128 && job_cost<false>(0x7FFFFFFF, 1) > 0x7FFFFFFFLL, "no wrap at any length");
 constexpr int kPlannedSeqs = 64;  // more parallel sequences are dealt evenly and in order, and take every step
+constexpr int kRoleOpen = -2;  // not decided yet (-1: none)
 struct LocalPlan {
     int role;
+    int gathered;              // waves that have looked at their share of the pattern types
     int length[kPlannedSeqs];  // steps until the last one that is no padding; then the same, longest first
     int order[kPlannedSeqs];
     int start[kPlannedSeqs + 1];  // first position in `order` of every group
 };
 
-// Called by all threads; wave 0 claims the role while the others look at the pattern types.
+// Called by all threads.  The role and the plan do not depend on each other and take some 5 us each, mostly trips to memory and a chain
+// of scalar steps: one wave claims the role while the others look at the pattern types and the last one, when they have, sorts and cuts.
+// One after the other, and with all XCDs' tickets on one line, the recursion began 12.5 us after the first workgroup (4 sequences of 150 to 200
+// steps) or 16 to 20 (10 of 300 to 600), 5.5 of it the role and 1 to 4 the plan.  One lstm layer 359 -> 350 us per pass, one utterance 1234 -> 1216, 150
+// and 200 cells with twenty sequences 2094 -> 2073, 32 sequences 2247 -> 2229, the acoustic model 2482 -> 2471.
 template <int MOST, bool FWD>
 __device__ __forceinline__ LocalJob local_setup(const ChainParams &p, LocalPlan &plan, int &job, int &me) {
     const int tid = threadIdx.x, lane = tid & 63, S = p.S, T = p.T, Tmin = min(p.Tmin, T);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), claims = (int)blockDim.x / 64 - 2;
     const bool planned = S <= kPlannedSeqs;
     if (tid < kPlannedSeqs) plan.length[tid] = Tmin;
+    if (tid == 0) { plan.gathered = 0; plan.role = kRoleOpen; }
     __syncthreads();
-    if (tid == 0) {
-        plan.role = local_claim_role(p, p.team);
-    } else if (tid >= 64 && planned && Tmin < T) {
-        const int threads = blockDim.x - 64, rows = threads / S, s = (tid - 64) % S, row = (tid - 64) / S;
-        if (row < rows) {
-            int length = 0;
-#pragma unroll 4
-            for (int t = Tmin + row; t < T; t += rows) length = p.pat[(size_t)t * S + s] != 0 ? t + 1 : length;
-            atomicMax(&plan.length[s], length);
+    if (wave == claims) {
+        if (lane == 0) __hip_atomic_store(&plan.role, local_claim_role(p, p.team), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    } else if (wave < claims) {
+        if (planned && Tmin < T) {
+            const int rows = 64 * claims / S, s = tid % S, row = tid / S;
+            if (row < rows) {
+                int length = 0;
+#pragma unroll 8
+                for (int t = Tmin + row; t < T; t += rows) length = p.pat[(size_t)t * S + s] != 0 ? t + 1 : length;
+                atomicMax(&plan.length[s], length);
+            }
         }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        if (lane == 0) atomicAdd(&plan.gathered, 1);
+    } else if (planned) {
+        while (__hip_atomic_load(&plan.gathered, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < claims) __builtin_amdgcn_s_sleep(1);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        const bool needed = __hip_atomic_load(&plan.role, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != -1;
+        const int mine = lane < S ? plan.length[lane] : -1;
+        int rank = 0;
+        for (int s = 0; s < S && needed; ++s) {
+            const int other = __builtin_amdgcn_readlane(mine, s);
+            rank += other > mine || (other == mine && s < lane) ? 1 : 0;
+        }
+        if (lane < S) { plan.order[rank] = lane; plan.length[rank] = mine; }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int sorted = lane < S ? plan.length[lane] : 0;
+        long long cost[MOST];  // of a job of this lane's sequence and the q behind it
+#pragma unroll
+        for (int q = 0; q < MOST; ++q) cost[q] = job_cost<FWD>(sorted, q + 1);
+        auto most_within = [&](long long bound) {  // sequences of a job that starts with this lane's
+            int n = 0;
+#pragma unroll
+            for (int q = 0; q < MOST; ++q) n = cost[q] <= bound ? q + 1 : n;
+            return n;
+        };
+        auto cut = [&](long long bound, bool keep) {
+            const int n = most_within(bound);
+            int at = 0, g = 0;
+            for (; at < S && g < p.groups; ++g) {
+                const int take = __builtin_amdgcn_readlane(n, at);
+                if (take == 0) break;
+                if (keep && lane == 0) plan.start[g] = at;
+                at = min(at + take, S);
+            }
+            if (keep)
+                for (; g <= p.groups; ++g)
+                    if (lane == 0) plan.start[g] = S;
+            return at >= S;
+        };
+        const int top = __builtin_amdgcn_readlane(sorted, 0);
+        long long low = job_cost<FWD>(top, 1) - 1, high = job_cost<FWD>(top, MOST);  // `high` always suffices
+        // (four in every job: nothing to choose)
+        for (int q = 0; q < 10 && needed && high - low > 1 && p.groups * MOST > S; ++q) {
+            const long long mid = (low + high) / 2;
+            if (cut(mid, false)) high = mid;
+            else low = mid;
+        }
+        if (needed) cut(high, true);
     }
     __syncthreads();
     LocalJob part = {0, 0, plan.order, 0, 0, 0, 0};
@@ -191,51 +254,6 @@ __device__ __forceinline__ LocalJob local_setup(const ChainParams &p, LocalPlan 
         // (jobs of more than kPlannedSeqs sequences in all still hold at most MOST each)
         if (tid < part.nseq) plan.order[tid] = group * each + min(group, more) + tid;
     } else {
-        if (tid < 64) {
-            const int mine = lane < S ? plan.length[lane] : -1;
-            int rank = 0;
-            for (int s = 0; s < S; ++s) {
-                const int other = __builtin_amdgcn_readlane(mine, s);
-                rank += other > mine || (other == mine && s < lane) ? 1 : 0;
-            }
-            if (lane < S) { plan.order[rank] = lane; plan.length[rank] = mine; }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            const int sorted = lane < S ? plan.length[lane] : 0;
-            long long cost[MOST];  // of a job of this lane's sequence and the q behind it
-#pragma unroll
-            for (int q = 0; q < MOST; ++q) cost[q] = job_cost<FWD>(sorted, q + 1);
-            auto most_within = [&](long long bound) {  // sequences of a job that starts with this lane's
-                int n = 0;
-#pragma unroll
-                for (int q = 0; q < MOST; ++q) n = cost[q] <= bound ? q + 1 : n;
-                return n;
-            };
-            auto cut = [&](long long bound, bool keep) {
-                const int n = most_within(bound);
-                int at = 0, g = 0;
-                for (; at < S && g < p.groups; ++g) {
-                    const int take = __builtin_amdgcn_readlane(n, at);
-                    if (take == 0) break;
-                    if (keep && lane == 0) plan.start[g] = at;
-                    at = min(at + take, S);
-                }
-                if (keep)
-                    for (; g <= p.groups; ++g)
-                        if (lane == 0) plan.start[g] = S;
-                return at >= S;
-            };
-            const int top = __builtin_amdgcn_readlane(sorted, 0);
-            long long low = job_cost<FWD>(top, 1) - 1, high = job_cost<FWD>(top, MOST);  // `high` always suffices
-            // (four in every job: nothing to choose)
-            for (int q = 0; q < 10 && high - low > 1 && p.groups * MOST > S; ++q) {
-                const long long mid = (low + high) / 2;
-                if (cut(mid, false)) high = mid;
-                else low = mid;
-            }
-            cut(high, true);
-        }
-        __syncthreads();
         const int from = __builtin_amdgcn_readfirstlane(plan.start[group]);
         part.nseq = __builtin_amdgcn_readfirstlane(plan.start[group + 1]) - from;
         part.order = plan.order + from;
