@@ -1673,8 +1673,8 @@ static bool has_weight_half(const cnt::NetLayer &L) {
 // blstm 128 (240) 150 / 132, (960) 368 / 347, (1920) 382 / 359; two lstm 256 (240) 316 / 298, (960) 823 / 807, (1920, 2e9) 872 / 831; the acoustic
 // model (60) 395 / 374, (240) 435 / 396, (480, 1.8e9) 636 / 592, (960, 3.5e9) 977 / 974, (1920, 7e9) 1130 / 1162.
 // Blocks of 32 / 64 and 64 / 128 channels: 8 of them (2000) 249 / 235, (4000) 268 / 280, 20 (2000) 491 / 462, 10 wide ones (2000) 446 / 422,
-// (4000) 478 / 485.  Convolutions without the blocks' launches, whose products are batched over layers on another stream, stay there: 20 of
-// 48 channels (2000) 1095 / 1740.
+// (4000) 478 / 485.  Convolutions without the blocks' launches, whose products are batched over layers on another stream, stay there: 20
+// blocks of 48 channels (2000) layer by layer 1095 / 1740.
 static bool weights_in_line(const cnt_network *net, const std::vector<char> &in_block) {
     using namespace cnt;
     const long slots = static_cast<long>(net->S) * net->T;

@@ -553,16 +553,22 @@ block_err_kernel_t block_errors_of(bool conv, bool sum, int threads) {
     return conv ? (sum ? wavenet_block_errors_kernel<R, K, true, true, 256> : wavenet_block_errors_kernel<R, K, true, false, 256>)
                 : (sum ? wavenet_block_errors_kernel<R, K, false, true, 256> : wavenet_block_errors_kernel<R, K, false, false, 256>);
 }
+// Widths that have the launch: the residual channels of the forward pass's launch with the usual numbers of skip channels.  All others go
+// layer by layer, and their weight gradients then do so as well.  us per pass layer by layer / with the launch, residual and skip channels, slots,
+// blocks: 48 and 96, 2001, 20 1019 / 560; 48 and 64, 16 200, 10 965 / 607; 48 and 128, 24 000, 30 3405 / 2291; 48 and 256, 32 000, 20 3017 /
+// 2259; 64 and 32, 4000, 8 550 / 344; 64 and 96, 16 000, 20 1980 / 1305; 32 and 96, 1000, 10 490 / 267; 32 and 256, 24 000, 20 2372 / 1676.
+// Gradients' 2-norm error against 64 bits there 1.2 to 6.5e-7, layer by layer 1.3 to 6.9e-7.
 block_err_kernel_t pick_block_errors_kernel(int R, int K, bool conv, bool sum, int threads) {
-#define CNT_BLOCK_KERNEL(r, k) \
-    if (R == r && K == k) return block_errors_of<r, k>(conv, sum, threads);
-    CNT_BLOCK_KERNEL(64, 128)
-    CNT_BLOCK_KERNEL(64, 256)
-    CNT_BLOCK_KERNEL(64, 64)
-    CNT_BLOCK_KERNEL(32, 128)
-    CNT_BLOCK_KERNEL(32, 64)
-    CNT_BLOCK_KERNEL(32, 32)
-#undef CNT_BLOCK_KERNEL
+#define CNT_BLOCK_KERNELS(r)                                            \
+    if (R == r && K == 32) return block_errors_of<r, 32>(conv, sum, threads);   \
+    if (R == r && K == 64) return block_errors_of<r, 64>(conv, sum, threads);   \
+    if (R == r && K == 96) return block_errors_of<r, 96>(conv, sum, threads);   \
+    if (R == r && K == 128) return block_errors_of<r, 128>(conv, sum, threads); \
+    if (R == r && K == 256) return block_errors_of<r, 256>(conv, sum, threads);
+    CNT_BLOCK_KERNELS(64)
+    CNT_BLOCK_KERNELS(48)
+    CNT_BLOCK_KERNELS(32)
+#undef CNT_BLOCK_KERNELS
     return nullptr;
 }
 
@@ -1022,7 +1028,7 @@ extern "C++" bool cnt::wavenet_block_errors_supported(int R, int K) { return pic
 // of 64 channels (80 KB of weights, one workgroup per compute unit) the smaller ones win as long as they are all resident at
 // once.  us per launch, products beside them, 256 / 512 threads: 64 channels, 2000 samples 24 / 33, 8000 25 / 34, 16 000 29 / 36,
 // 18 000 47 / 38, 32 000 58 / 47, 48 000 82 / 81; 32 channels, 2000 13.4 / 16.9, 16 000 15.4 / 18.3, 18 000 to 32 000 the same, 48 000
-// 29 / 37.
+// 29 / 37.  48 channels, us per pass: 30 blocks with 128 skip channels, 24 000 samples 2341 / 2291, 20 with 256, 32 000 samples 2377 / 2259.
 static int block_errors_threads(int R, int N, bool fold) { return fold && R > 32 && N > 64 * 256 ? 512 : 256; }
 
 extern "C++" int cnt::wavenet_block_rows(int R, int N, bool fold) {

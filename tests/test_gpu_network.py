@@ -607,6 +607,11 @@ def test_network_give_up_on_a_nonblocking_stream_keeps_weights_and_adam_state():
     # the other widths the fused block launch is built for
     (3, 1, 64, 256, 64, 20, [70, 52], 3, 20), (3, 0, 64, 64, 64, 20, [70, 52], 3, 20),
     (3, 1, 32, 128, 64, 20, [70, 52], 3, 20), (3, 0, 32, 32, 64, 20, [70, 52], 3, 20),
+    (3, 1, 64, 32, 64, 20, [70, 52], 3, 20), (3, 0, 64, 96, 64, 21, [70, 52], 3, 20), (3, 1, 32, 96, 64, 20, [70, 52], 3, 20),
+    (3, 1, 32, 256, 64, 22, [70, 52], 3, 20), (3, 0, 48, 32, 64, 20, [70, 52], 3, 20), (3, 1, 48, 64, 64, 45, [70, 52], 3, 20),
+    (3, 1, 48, 96, 64, 20, [70, 52], 3, 20), (3, 0, 48, 128, 64, 80, [70, 52], 3, 20), (3, 1, 48, 256, 64, 20, [70, 52], 3, 20),
+    # skip channels that it is not built for
+    (3, 1, 48, 80, 64, 20, [70, 52], 3, 20),
     (10, 1, 64, 128, 256, 80, [4000, 3300], 10, 80),
 ])
 def test_wavenet_network_file_against_oracle_graph(nb, cnn_tanh, R, K, Q, C, lengths, cycle, upsample):
@@ -669,7 +674,7 @@ def test_wavenet_network_file_against_oracle_graph(nb, cnn_tanh, R, K, Q, C, len
     torch.cuda.synchronize()
     launches = {k: n for k, (n, _) in capi.profile_read().items()}
     capi.profile_enable(False)
-    if (R, K) in [(64, 128), (64, 256), (64, 64), (32, 128), (32, 64), (32, 32)]:
+    if R in (32, 48, 64) and K in (32, 64, 96, 128, 256):
         assert launches.get("wavenet_block_errors") == 1 and launches.get("wavenet_block_errors+cnn") == nb - 1, launches
     else:
         assert "wavenet_block_errors" not in launches and "wavenet_block_errors+cnn" not in launches, launches
@@ -682,7 +687,8 @@ def test_wavenet_network_file_against_oracle_graph(nb, cnn_tanh, R, K, Q, C, len
 
 # block launches of 64 and of 128 samples per workgroup: a part of one workgroup, one and a sample more, and both sides of the line
 # between them at 64 channels (16 384 samples); 32 channels behind that line
-@pytest.mark.parametrize("R,K,lengths", [(64, 64, [1]), (64, 128, [64]), (32, 64, [65]), (64, 64, [8192, 8101]), (64, 64, [8193, 8050]), (32, 32, [8193, 8192])])
+@pytest.mark.parametrize("R,K,lengths", [(64, 64, [1]), (64, 128, [64]), (32, 64, [65]), (64, 64, [8192, 8101]), (64, 64, [8193, 8050]), (32, 32, [8193, 8192]),
+                                         (48, 96, [1]), (48, 32, [65]), (48, 128, [8192, 8101]), (48, 96, [8193, 8050])])
 def test_wavenet_block_errors_of_both_workgroup_sizes(R, K, lengths):
     test_wavenet_network_file_against_oracle_graph(2, 1, R, K, 16, 4, lengths, 2, 5)
 
@@ -976,7 +982,7 @@ def test_first_optimizer_step_under_capture(option, rate, sgd_before):
 # conditioning part of layers whose pre-activations are kept: its gradient takes the place of its values.
 @pytest.mark.parametrize("cnn_tanh,R,K,C,lengths,conditioning_again", [
     (1, 32, 64, 20, [120, 90], True), (1, 64, 128, 81, [700, 333], True), (1, 64, 256, 7, [16500], True), (0, 32, 64, 20, [120, 90], False),
-    (1, 64, 64, 0, [70, 52], True),
+    (1, 64, 64, 0, [70, 52], True), (1, 48, 96, 20, [120, 90], True),
 ])
 def test_second_backward_pass_of_a_wavenet_stack(cnn_tanh, R, K, C, lengths, conditioning_again):
     import torch
