@@ -492,6 +492,108 @@ __global__ __launch_bounds__(NT, (CONV || K > 128) ? 1 : 2) void wavenet_block_e
     }
 }
 
+// The same for short waveforms, one block folded in and the pre-activations formed again: a workgroup owns 16 samples and has a wave per
+// sixteen residual channels, as in the forward pass's launch.  What bounds the launch above there is its chain, the products of all channels
+// (64 residual and 128 skip channels: 448 matrix instructions, 6 us) behind the weights' way into LDS, on an eighth of the compute units.  Here a wave
+// has a quarter of the products and takes its channels' weights straight into registers, all requested up front; the errors behind the first product
+// pass through LDS, a tile of channels per wave.  Every sum is formed in the launch above's order: the same values bit for bit.
+template <int R, int K>
+__global__ __launch_bounds__(4 * R, 1) void wavenet_block_errors_narrow_kernel(const BlockErrArgs a) {
+    constexpr int KJ = K / 16, RJ = R / 16, CJ = 2 * R / 16, ROW = 17;
+    __shared__ __attribute__((aligned(16))) f32x4v es[4 * RJ * ROW];  // [four channels][sample]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int quarter = lane >> 4, col = lane & 15;
+    const int n_raw = blockIdx.x * 16 + col;
+    const bool ok = n_raw < a.N;
+    const size_t n = ok ? n_raw : a.N - 1;  // lanes past the end compute on the last sample and store nothing
+    // A operands: element i of j is the weight of input 16j + 4*quarter + i and this wave's channel `col`
+    auto weights = [&](auto &w, const float *from, int ld) __attribute__((always_inline)) {
+        const float *const at = from + (size_t)(4 * quarter) * ld + 16 * wave + col;
+#pragma unroll
+        for (int j = 0; j < (int)(sizeof(w) / sizeof(w[0])); ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[j][i] = at[(size_t)(16 * j + i) * ld];
+    };
+    f32x4v b1[KJ], w1[KJ], bc[2][CJ], wc[2][CJ], w2[RJ];
+#pragma unroll
+    for (int j = 0; j < KJ; ++j) b1[j] = *reinterpret_cast<const f32x4v *>(a.e_skip + n * K + 16 * j + 4 * quarter);
+    weights(w1, a.w_skip, R);
+    const char own_pat = a.pat[n];
+    char tap_pat[2];
+    bool inside[2];
+#pragma unroll
+    for (int tap = 0; tap < 2; ++tap) {
+        const long long src = (long long)n + a.conv_shift[tap];
+        inside[tap] = src >= 0 && src < a.N;
+        const size_t sc = inside[tap] ? (size_t)src : n;
+        tap_pat[tap] = a.pat[sc];
+#pragma unroll
+        for (int j = 0; j < CJ; ++j) bc[tap][j] = *reinterpret_cast<const f32x4v *>(a.conv_deltas + sc * 2 * R + 16 * j + 4 * quarter);
+        weights(wc[tap], a.conv_w[tap], a.conv_ld);
+    }
+    weights(w2, a.w_out, R);
+    const size_t one = n * R + 16 * wave + 4 * quarter, at = n * 2 * R + 16 * wave + 4 * quarter;
+    const f32x4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    const f32x4v side = a.from_skip ? *reinterpret_cast<const f32x4v *>(a.from_skip + one) : zero;
+    const f32x4v y1 = *reinterpret_cast<const f32x4v *>(a.conv_tanh + at), y2 = *reinterpret_cast<const f32x4v *>(a.conv_tanh + at + R);
+    const f32x4v c1 = *reinterpret_cast<const f32x4v *>(a.ctx_tanh + at), c2 = *reinterpret_cast<const f32x4v *>(a.ctx_tanh + at + R);
+    const f32x4v old0 = a.fan_n > 0 && a.fan_is_skip[0] != 0 ? *reinterpret_cast<const f32x4v *>(a.fan_targets[0] + one) : zero;
+    __builtin_amdgcn_sched_barrier(0);
+    const bool live = own_pat != 0;
+
+    auto product = [](f32x4v &acc0, f32x4v &acc1, const auto &w, const auto &b, int count, bool keep) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < count; ++j) {
+            f32x4v x;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = keep ? b[j][i] : 0.0f;
+            acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][0], x[0], acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][1], x[1], acc1, 0, 0, 0);
+            acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][2], x[2], acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][3], x[3], acc1, 0, 0, 0);
+        }
+    };
+    f32x4v acc0 = zero, acc1 = zero;
+    product(acc0, acc1, w1, b1, KJ, true);
+    product(acc0, acc1, wc[0], bc[0], CJ, live && inside[0] && tap_pat[0] != 0);
+    acc0 = acc0 + acc1;
+    acc1 = zero;
+    product(acc0, acc1, wc[1], bc[1], CJ, live && inside[1] && tap_pat[1] != 0);
+    f32x4v e = acc0 + acc1;
+    if (a.from_skip) e += side;
+    es[(4 * wave + quarter) * ROW + col] = e;
+    __syncthreads();
+    f32x4v be[RJ];
+#pragma unroll
+    for (int j = 0; j < RJ; ++j) be[j] = es[(4 * j + quarter) * ROW + col];
+    if (ok) {
+        *reinterpret_cast<f32x4v *>(a.total + one) = e;
+        for (int q = 0; q < a.fan_n; ++q) {
+            f32x4v *const to = reinterpret_cast<f32x4v *>(a.fan_targets[q] + one);
+            *to = a.fan_is_skip[q] ? e + (q == 0 ? old0 : *to) : e;
+        }
+    }
+    acc0 = acc1 = zero;
+    product(acc0, acc1, w2, be, RJ, true);
+    const f32x4v u = acc0 + acc1;
+
+    // the gated unit, as above
+    f32x4v o1, o2, q1, q2;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const float th = tanh_act(y1[v] + c1[v]), sg = logistic(y2[v] + c2[v]);
+        const float g1 = live ? (1.0f - th * th) * sg * u[v] : 0.0f, g2 = live ? th * (sg * (1.0f - sg)) * u[v] : 0.0f;
+        o1[v] = tanh_deriv(y1[v]) * g1; o2[v] = tanh_deriv(y2[v]) * g2;
+        q1[v] = tanh_deriv(c1[v]) * g1; q2[v] = tanh_deriv(c2[v]) * g2;
+    }
+    if (ok) {
+        *reinterpret_cast<f32x4v *>(a.deltas + at) = o1;
+        *reinterpret_cast<f32x4v *>(a.deltas + at + R) = o2;
+        *reinterpret_cast<f32x4v *>(a.ctx_grad + at) = q1;
+        *reinterpret_cast<f32x4v *>(a.ctx_grad + at + R) = q2;
+    }
+}
+
 // out[d] = scale * sum over rows of partial[row][d] (the second half of a column sum whose first half rode in
 // wavenet_block_errors_kernel), for the layers of a list; overwrites
 constexpr int kColsumGroups = 4;
@@ -570,6 +672,15 @@ block_err_kernel_t pick_block_errors_kernel(int R, int K, bool conv, bool sum, i
     CNT_BLOCK_KERNELS(32)
 #undef CNT_BLOCK_KERNELS
     return nullptr;
+}
+template <int R>
+block_err_kernel_t narrow_block_errors_of(int K) {
+    return K == 32 ? wavenet_block_errors_narrow_kernel<R, 32> : K == 64 ? wavenet_block_errors_narrow_kernel<R, 64>
+         : K == 96 ? wavenet_block_errors_narrow_kernel<R, 96> : K == 128 ? wavenet_block_errors_narrow_kernel<R, 128>
+         : K == 256 ? wavenet_block_errors_narrow_kernel<R, 256> : nullptr;
+}
+block_err_kernel_t pick_narrow_block_errors_kernel(int R, int K) {
+    return R == 64 ? narrow_block_errors_of<64>(K) : R == 48 ? narrow_block_errors_of<48>(K) : R == 32 ? narrow_block_errors_of<32>(K) : nullptr;
 }
 
 __global__ void sum_context_grad_kernel(int C, int S, int resolution, size_t count, int N,
@@ -1031,6 +1142,13 @@ extern "C++" bool cnt::wavenet_block_errors_supported(int R, int K) { return pic
 // 29 / 37.  48 channels, us per pass: 30 blocks with 128 skip channels, 24 000 samples 2341 / 2291, 20 with 256, 32 000 samples 2377 / 2259.
 static int block_errors_threads(int R, int N, bool fold) { return fold && R > 32 && N > 64 * 256 ? 512 : 256; }
 
+// Up to 8192 samples (512 workgroups) the narrow launch.  us per pass of twelve blocks, the launch above / narrow, residual and skip channels and
+// samples: 64 and 128, 700 443 / 347, 2000 472 / 377, 4000 532 / 450, 8000 651 / 634, 10 000 765 / 779, 16 000 865 / 925; 64 and 256,
+// 3000 604 / 502, 8000 736 / 738, 12 000 920 / 994; 64 and 32, 2000 426 / 339, 8000 579 / 542, 12 000 690 / 696; 48 and 96, 1000
+// 351 / 294, 8000 518 / 496, 12 000 608 / 622; 32 and 64, 700 286 / 250, 4000 367 / 321, 8000 420 / 406, 16 000 525 / 524; 32 and 256, 6000
+// 517 / 500, 12 000 608 / 615.
+static bool narrow_block_errors(int N) { return N <= 8192; }
+
 extern "C++" int cnt::wavenet_block_rows(int R, int N, bool fold) {
     const int samples = block_errors_threads(R, N, fold) / 4;
     return (N + samples - 1) / samples;
@@ -1051,8 +1169,9 @@ extern "C++" int cnt::wavenet_block_errors(hipStream_t stream, int R, int K, int
                                            float *total, const FanOut *fan, const float *core_buf, const float *ctx_tanh,
                                            float *ctx_grad, const float *conv_tanh_outputs, float *conv_errors, const cnt_cnn *fold,
                                            const float *fold_weights, const float *fold_deltas, float *colsum_partial) {
-    const int threads = block_errors_threads(R, N, fold != nullptr);
-    block_err_kernel_t k = pick_block_errors_kernel(R, K, fold != nullptr, core_buf == nullptr, threads);
+    const bool narrow = narrow_block_errors(N) && fold && !core_buf && !colsum_partial;  // (it leaves no sums of the deltas)
+    const int threads = narrow ? 4 * R : block_errors_threads(R, N, fold != nullptr);
+    block_err_kernel_t k = narrow ? pick_narrow_block_errors_kernel(R, K) : pick_block_errors_kernel(R, K, fold != nullptr, core_buf == nullptr, threads);
     CNT_REQUIRE(k != nullptr, "wavenet_block_errors: no kernel for %d residual and %d skip channels", R, K);
     CNT_REQUIRE(N > 0 && patTypes && skip_weights && out_weights && skip_errors && total && (core_buf || (ctx_tanh && conv_tanh_outputs)) &&
                 conv_errors && (!ctx_tanh || ctx_grad) && (core_buf || ctx_grad != ctx_tanh),
@@ -1081,7 +1200,7 @@ extern "C++" int cnt::wavenet_block_errors(hipStream_t stream, int R, int K, int
                 aligned(a.from_skip) && aligned(core_buf) && aligned(ctx_tanh) && aligned(ctx_grad) &&
                 aligned(conv_tanh_outputs) && aligned(conv_errors), "wavenet_block_errors: buffers must be 16-byte aligned");
     ProfileScope prof(stream, fold ? "wavenet_block_errors+cnn" : "wavenet_block_errors");
-    hipLaunchKernelGGL(k, dim3(wavenet_block_rows(R, N, fold != nullptr)), dim3(threads), 0, stream, a);
+    hipLaunchKernelGGL(k, dim3(narrow ? (N + 15) / 16 : wavenet_block_rows(R, N, fold != nullptr)), dim3(threads), 0, stream, a);
     CNT_HIP(hipGetLastError());
     return CNT_OK;
 }

@@ -685,9 +685,10 @@ def test_wavenet_network_file_against_oracle_graph(nb, cnn_tanh, R, K, Q, C, len
     net.close()
 
 
-# block launches of 64 and of 128 samples per workgroup: a part of one workgroup, one and a sample more, and both sides of the line
-# between them at 64 channels (16 384 samples); 32 channels behind that line
+# block launches of 16, 64 and 128 samples per workgroup: a part of one workgroup, one and a sample more, and both sides of the lines
+# between them (8192 samples, at 64 and 48 channels also 16 384); 32 channels behind the second line
 @pytest.mark.parametrize("R,K,lengths", [(64, 64, [1]), (64, 128, [64]), (32, 64, [65]), (64, 64, [8192, 8101]), (64, 64, [8193, 8050]), (32, 32, [8193, 8192]),
+                                         (64, 128, [15]), (64, 128, [4096, 4001]), (64, 32, [4097, 4003]), (32, 256, [17]), (48, 64, [4096, 4093]),
                                          (48, 96, [1]), (48, 32, [65]), (48, 128, [8192, 8101]), (48, 96, [8193, 8050])])
 def test_wavenet_block_errors_of_both_workgroup_sizes(R, K, lengths):
     test_wavenet_network_file_against_oracle_graph(2, 1, R, K, 16, 4, lengths, 2, 5)
