@@ -433,7 +433,7 @@ struct BlockGradients {
     int shift;                                                   // the earlier tap reads slot n - shift
 };
 bool wavenet_block_weights_supported(int R, int K, int C, long N);
-size_t wavenet_block_weights_scratch();  // floats; one launch at a time
+size_t wavenet_block_weights_scratch(int R, int K, int C);  // floats; one launch at a time
 int wavenet_block_weights(hipStream_t stream, int R, int K, int C, int N, int count, const BlockGradients *blocks, const float *ctx,
                           const char *patTypes, float *scratch);
 // the shift, the bias gradient's place behind the weights and its factor, of a layer that cnn_foldable accepts

@@ -1097,11 +1097,13 @@ int finish_build(cnt_network *net, const json::Value *weights) {
         const size_t rows = ((size_t)net->S * C.maxTr + 63) / 64;
         CNT_TRY(device_alloc(net, (void **)&C.colsum, rows * C.size * sizeof(float), false));
     }
-    for (size_t i = 5; i < net->layers.size() && !net->block_sums; ++i)
+    size_t block_sums = 0;
+    for (size_t i = 5; i < net->layers.size(); ++i)
         if (net->layers[i].kind == K_DENSE && net->layers[i - 4].kind == K_WAVNETC &&
             wavenet_block_errors_supported(net->layers[i - 4].size, net->layers[i].size) &&
             wavenet_block_weights_supported(net->layers[i - 4].size, net->layers[i].size, net->layers[i - 4].ctx_dim, 1))
-            CNT_TRY(device_alloc(net, (void **)&net->block_sums, wavenet_block_weights_scratch() * sizeof(float), false));
+            block_sums = std::max(block_sums, wavenet_block_weights_scratch(net->layers[i - 4].size, net->layers[i].size, net->layers[i - 4].ctx_dim));
+    if (block_sums) CNT_TRY(device_alloc(net, (void **)&net->block_sums, block_sums * sizeof(float), false));
     // the slots of a fraction with the valid ones first: the weight gradients of the dense and recurrent layers sum over
     // those only (CNT_NET_SKIP_PADDING=0: over all slots)
     {

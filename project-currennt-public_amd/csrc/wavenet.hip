@@ -658,25 +658,26 @@ block_err_kernel_t block_errors_of(bool conv, bool sum, int threads) {
 // Widths that have the launch: the residual channels of the forward pass's launch with the usual numbers of skip channels.  All others go
 // layer by layer, and their weight gradients then do so as well.  us per pass layer by layer / with the launch, residual and skip channels, slots,
 // blocks: 48 and 96, 2001, 20 1019 / 560; 48 and 64, 16 200, 10 965 / 607; 48 and 128, 24 000, 30 3405 / 2291; 48 and 256, 32 000, 20 3017 /
-// 2259; 64 and 32, 4000, 8 550 / 344; 64 and 96, 16 000, 20 1980 / 1305; 32 and 96, 1000, 10 490 / 267; 32 and 256, 24 000, 20 2372 / 1676.
+// 2259; 64 and 96, 16 000, 20 1980 / 1305; 32 and 96, 1000, 10 490 / 267; 32 and 256, 24 000, 20 2372 / 1676.
 // Gradients' 2-norm error against 64 bits there 1.2 to 6.5e-7, layer by layer 1.3 to 6.9e-7.
 block_err_kernel_t pick_block_errors_kernel(int R, int K, bool conv, bool sum, int threads) {
-#define CNT_BLOCK_KERNELS(r)                                            \
-    if (R == r && K == 32) return block_errors_of<r, 32>(conv, sum, threads);   \
-    if (R == r && K == 64) return block_errors_of<r, 64>(conv, sum, threads);   \
-    if (R == r && K == 96) return block_errors_of<r, 96>(conv, sum, threads);   \
-    if (R == r && K == 128) return block_errors_of<r, 128>(conv, sum, threads); \
-    if (R == r && K == 256) return block_errors_of<r, 256>(conv, sum, threads);
+#define CNT_BLOCK_KERNEL(r, k) \
+    if (R == r && K == k) return block_errors_of<r, k>(conv, sum, threads);
+#define CNT_BLOCK_KERNELS(r) CNT_BLOCK_KERNEL(r, 64) CNT_BLOCK_KERNEL(r, 96) CNT_BLOCK_KERNEL(r, 128) CNT_BLOCK_KERNEL(r, 256)
     CNT_BLOCK_KERNELS(64)
     CNT_BLOCK_KERNELS(48)
     CNT_BLOCK_KERNELS(32)
+    CNT_BLOCK_KERNEL(48, 32)
+    CNT_BLOCK_KERNEL(32, 32)
+#undef CNT_BLOCK_KERNEL
 #undef CNT_BLOCK_KERNELS
     return nullptr;
 }
 template <int R>
 block_err_kernel_t narrow_block_errors_of(int K) {
-    return K == 32 ? wavenet_block_errors_narrow_kernel<R, 32> : K == 64 ? wavenet_block_errors_narrow_kernel<R, 64>
-         : K == 96 ? wavenet_block_errors_narrow_kernel<R, 96> : K == 128 ? wavenet_block_errors_narrow_kernel<R, 128>
+    if constexpr (R < 64)
+        if (K == 32) return wavenet_block_errors_narrow_kernel<R, 32>;
+    return K == 64 ? wavenet_block_errors_narrow_kernel<R, 64> : K == 96 ? wavenet_block_errors_narrow_kernel<R, 96> : K == 128 ? wavenet_block_errors_narrow_kernel<R, 128>
          : K == 256 ? wavenet_block_errors_narrow_kernel<R, 256> : nullptr;
 }
 block_err_kernel_t pick_narrow_block_errors_kernel(int R, int K) {
@@ -1144,7 +1145,7 @@ static int block_errors_threads(int R, int N, bool fold) { return fold && R > 32
 
 // Up to 8192 samples (512 workgroups) the narrow launch.  us per pass of twelve blocks, the launch above / narrow, residual and skip channels and
 // samples: 64 and 128, 700 443 / 347, 2000 472 / 377, 4000 532 / 450, 8000 651 / 634, 10 000 765 / 779, 16 000 865 / 925; 64 and 256,
-// 3000 604 / 502, 8000 736 / 738, 12 000 920 / 994; 64 and 32, 2000 426 / 339, 8000 579 / 542, 12 000 690 / 696; 48 and 96, 1000
+// 3000 604 / 502, 8000 736 / 738, 12 000 920 / 994; 48 and 96, 1000
 // 351 / 294, 8000 518 / 496, 12 000 608 / 622; 32 and 64, 700 286 / 250, 4000 367 / 321, 8000 420 / 406, 16 000 525 / 524; 32 and 256, 6000
 // 517 / 500, 12 000 608 / 615.
 static bool narrow_block_errors(int N) { return N <= 8192; }

@@ -50,6 +50,7 @@ struct TallArgs {
     int n, R, K, C;         // slots, residual and skip channels, conditioning features
     int conv_ld;            // distance of two filters' weights
     int jobs;               // per block: convolution, conditioning projection, 1x1 layer, 128 skip channels each
+    int sums;               // 32 x 32 blocks of sums that a workgroup has room for in `partial`
     int first[kTallMaxJobs + 1];  // workgroup of a block with which a job's splits begin
     const float *ctx;
     const char *pat;
@@ -339,7 +340,7 @@ __global__ __launch_bounds__(kTallThreads, 4) void wavenet_block_weights_kernel(
             sum[t] = plain_block(segment_of(a, b, job, m >> 1), segment_of(a, b, job, 2 + (n >> 1)), a.pat, 32 * (m & 1) + frag_row,
                                  32 * (n & 1) + frag_row, begin, end, half);
         }
-        float4 *const to = reinterpret_cast<float4 *>(a.partial) + (group * kTallBlocks + at) * 256 + lane;
+        float4 *const to = reinterpret_cast<float4 *>(a.partial) + (group * a.sums + at) * 256 + lane;
 #pragma unroll
         for (int g = 0; g < 4; ++g) to[64 * g] = float4{sum[t][4 * g], sum[t][4 * g + 1], sum[t][4 * g + 2], sum[t][4 * g + 3]};
     }
@@ -375,18 +376,18 @@ __global__ __launch_bounds__(256) void wavenet_block_weights_sum_kernel(const Ta
     const int mask_m = row_blocks(rows0, rows1), mask_n = row_blocks(rows2, rows3);
     const int count_n = __builtin_popcount(mask_n), count = __builtin_popcount(mask_m) * count_n;
     if (at >= count) return;
-    const float4 *const p = reinterpret_cast<const float4 *>(a.partial) + (first * kTallBlocks + at) * 256 + tid;
+    const float4 *const p = reinterpret_cast<const float4 *>(a.partial) + (first * a.sums + at) * 256 + tid;
     const auto add = [](const float4 &x, const float4 &y) { return float4{x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w}; };
     float4 v0 = {0, 0, 0, 0};
     int s = 0;
     for (; s + 8 <= splits; s += 8) {
         float4 x[8];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) x[q] = p[(size_t)(s + q) * kTallBlocks * 256];
+        for (int q = 0; q < 8; ++q) x[q] = p[(size_t)(s + q) * a.sums * 256];
         v0 = add(v0, add(add(add(x[0], x[1]), add(x[2], x[3])), add(add(x[4], x[5]), add(x[6], x[7]))));
     }
     float4 v1 = {0, 0, 0, 0};
-    for (; s < splits; ++s) v1 = add(v1, p[(size_t)s * kTallBlocks * 256]);
+    for (; s < splits; ++s) v1 = add(v1, p[(size_t)s * a.sums * 256]);
     v0 = add(v0, v1);
     const int mb = ith_bit(mask_m, at / count_n), nb = ith_bit(mask_n, at % count_n);
     const int m = 32 * (mb & 1) + (lane & 31), n = 32 * nb + 8 * g + 4 * (lane >> 5);
@@ -418,7 +419,13 @@ bool wavenet_block_weights_supported(int R, int K, int C, long N) {
            K >= 4 && K <= 256 && K % 4 == 0 && C >= 4 && C <= 128;
 }
 
-size_t wavenet_block_weights_scratch() { return (size_t)kTallWorkgroups * (kTallBlocks * 1024 + 256); }
+// 32 x 32 blocks of sums of the job that has the most: 16 with 64 residual channels, 12 with 48
+static int most_sums(int R, int K, int C) {
+    const auto blocks_of = [](int rows) { return (rows + 31) / 32; };
+    return std::max({2 * blocks_of(R) * blocks_of(2 * R), blocks_of(C) * blocks_of(2 * R), blocks_of(R) * blocks_of(R),
+                     blocks_of(R) * blocks_of(std::min(K, 128))});
+}
+size_t wavenet_block_weights_scratch(int R, int K, int C) { return (size_t)kTallWorkgroups * (most_sums(R, K, C) * 1024 + 256); }
 
 int wavenet_block_weights(hipStream_t stream, int R, int K, int C, int N, int count, const BlockGradients *blocks, const float *ctx,
                           const char *patTypes, float *scratch) {
@@ -434,7 +441,8 @@ int wavenet_block_weights(hipStream_t stream, int R, int K, int C, int N, int co
     a.jobs = 3 + (K + 127) / 128;
     a.ctx = ctx; a.pat = patTypes;
     a.partial = scratch;
-    a.rows = scratch + (size_t)kTallWorkgroups * kTallBlocks * 1024;
+    a.sums = most_sums(R, K, C);
+    a.rows = scratch + (size_t)kTallWorkgroups * a.sums * 1024;
     // The launch is one generation, two workgroups per compute unit; a block's share is dealt to its jobs by what a tile of theirs
     // takes: 16 rows to convert weigh about as much as a block of sums to multiply, and a tile's barriers and the wait for its loads
     // about eight times that.  Pass without this constant / with 3 / 5 / 8, us: 20 blocks of 32 and 32 channels, 80 features, 24 000

@@ -607,11 +607,11 @@ def test_network_give_up_on_a_nonblocking_stream_keeps_weights_and_adam_state():
     # the other widths the fused block launch is built for
     (3, 1, 64, 256, 64, 20, [70, 52], 3, 20), (3, 0, 64, 64, 64, 20, [70, 52], 3, 20),
     (3, 1, 32, 128, 64, 20, [70, 52], 3, 20), (3, 0, 32, 32, 64, 20, [70, 52], 3, 20),
-    (3, 1, 64, 32, 64, 20, [70, 52], 3, 20), (3, 0, 64, 96, 64, 21, [70, 52], 3, 20), (3, 1, 32, 96, 64, 20, [70, 52], 3, 20),
+    (3, 0, 64, 96, 64, 21, [70, 52], 3, 20), (3, 1, 32, 96, 64, 20, [70, 52], 3, 20),
     (3, 1, 32, 256, 64, 22, [70, 52], 3, 20), (3, 0, 48, 32, 64, 20, [70, 52], 3, 20), (3, 1, 48, 64, 64, 45, [70, 52], 3, 20),
     (3, 1, 48, 96, 64, 20, [70, 52], 3, 20), (3, 0, 48, 128, 64, 80, [70, 52], 3, 20), (3, 1, 48, 256, 64, 20, [70, 52], 3, 20),
     # skip channels that it is not built for
-    (3, 1, 48, 80, 64, 20, [70, 52], 3, 20),
+    (3, 1, 48, 80, 64, 20, [70, 52], 3, 20), (3, 1, 64, 32, 64, 20, [70, 52], 3, 20),
     (10, 1, 64, 128, 256, 80, [4000, 3300], 10, 80),
 ])
 def test_wavenet_network_file_against_oracle_graph(nb, cnn_tanh, R, K, Q, C, lengths, cycle, upsample):
@@ -674,7 +674,7 @@ def test_wavenet_network_file_against_oracle_graph(nb, cnn_tanh, R, K, Q, C, len
     torch.cuda.synchronize()
     launches = {k: n for k, (n, _) in capi.profile_read().items()}
     capi.profile_enable(False)
-    if R in (32, 48, 64) and K in (32, 64, 96, 128, 256):
+    if R in (32, 48, 64) and K in (32, 64, 96, 128, 256) and (R, K) != (64, 32):
         assert launches.get("wavenet_block_errors") == 1 and launches.get("wavenet_block_errors+cnn") == nb - 1, launches
     else:
         assert "wavenet_block_errors" not in launches and "wavenet_block_errors+cnn" not in launches, launches
@@ -688,7 +688,7 @@ def test_wavenet_network_file_against_oracle_graph(nb, cnn_tanh, R, K, Q, C, len
 # block launches of 16, 64 and 128 samples per workgroup: a part of one workgroup, one and a sample more, and both sides of the lines
 # between them (8192 samples, at 64 and 48 channels also 16 384); 32 channels behind the second line
 @pytest.mark.parametrize("R,K,lengths", [(64, 64, [1]), (64, 128, [64]), (32, 64, [65]), (64, 64, [8192, 8101]), (64, 64, [8193, 8050]), (32, 32, [8193, 8192]),
-                                         (64, 128, [15]), (64, 128, [4096, 4001]), (64, 32, [4097, 4003]), (32, 256, [17]), (48, 64, [4096, 4093]),
+                                         (64, 128, [15]), (64, 128, [4096, 4001]), (64, 96, [4097, 4003]), (32, 256, [17]), (48, 64, [4096, 4093]),
                                          (48, 96, [1]), (48, 32, [65]), (48, 128, [8192, 8101]), (48, 96, [8193, 8050])])
 def test_wavenet_block_errors_of_both_workgroup_sizes(R, K, lengths):
     test_wavenet_network_file_against_oracle_graph(2, 1, R, K, 16, 4, lengths, 2, 5)
