@@ -492,12 +492,12 @@ __global__ __launch_bounds__(NT, (CONV || K > 128) ? 1 : 2) void wavenet_block_e
     }
 }
 
-// The same for short waveforms, one block folded in and the pre-activations formed again: a workgroup owns 16 samples and has a wave per
+// The same for short waveforms where the pre-activations are formed again: a workgroup owns 16 samples and has a wave per
 // sixteen residual channels, as in the forward pass's launch.  What bounds the launch above there is its chain, the products of all channels
 // (64 residual and 128 skip channels: 448 matrix instructions, 6 us) behind the weights' way into LDS, on an eighth of the compute units.  Here a wave
 // has a quarter of the products and takes its channels' weights straight into registers, all requested up front; the errors behind the first product
 // pass through LDS, a tile of channels per wave.  Every sum is formed in the launch above's order: the same values bit for bit.
-template <int R, int K>
+template <int R, int K, bool CONV>
 __global__ __launch_bounds__(4 * R, 1) void wavenet_block_errors_narrow_kernel(const BlockErrArgs a) {
     constexpr int KJ = K / 16, RJ = R / 16, CJ = 2 * R / 16, ROW = 17;
     __shared__ __attribute__((aligned(16))) f32x4v es[4 * RJ * ROW];  // [four channels][sample]
@@ -514,23 +514,24 @@ __global__ __launch_bounds__(4 * R, 1) void wavenet_block_errors_narrow_kernel(c
 #pragma unroll
             for (int i = 0; i < 4; ++i) w[j][i] = at[(size_t)(16 * j + i) * ld];
     };
-    f32x4v b1[KJ], w1[KJ], bc[2][CJ], wc[2][CJ], w2[RJ];
+    f32x4v b1[KJ], w1[KJ], bc[2][CONV ? CJ : 1], wc[2][CONV ? CJ : 1], w2[RJ];
 #pragma unroll
     for (int j = 0; j < KJ; ++j) b1[j] = *reinterpret_cast<const f32x4v *>(a.e_skip + n * K + 16 * j + 4 * quarter);
     weights(w1, a.w_skip, R);
     const char own_pat = a.pat[n];
-    char tap_pat[2];
-    bool inside[2];
+    char tap_pat[2] = {0, 0};
+    bool inside[2] = {false, false};
+    if constexpr (CONV)
 #pragma unroll
-    for (int tap = 0; tap < 2; ++tap) {
-        const long long src = (long long)n + a.conv_shift[tap];
-        inside[tap] = src >= 0 && src < a.N;
-        const size_t sc = inside[tap] ? (size_t)src : n;
-        tap_pat[tap] = a.pat[sc];
+        for (int tap = 0; tap < 2; ++tap) {
+            const long long src = (long long)n + a.conv_shift[tap];
+            inside[tap] = src >= 0 && src < a.N;
+            const size_t sc = inside[tap] ? (size_t)src : n;
+            tap_pat[tap] = a.pat[sc];
 #pragma unroll
-        for (int j = 0; j < CJ; ++j) bc[tap][j] = *reinterpret_cast<const f32x4v *>(a.conv_deltas + sc * 2 * R + 16 * j + 4 * quarter);
-        weights(wc[tap], a.conv_w[tap], a.conv_ld);
-    }
+            for (int j = 0; j < CJ; ++j) bc[tap][j] = *reinterpret_cast<const f32x4v *>(a.conv_deltas + sc * 2 * R + 16 * j + 4 * quarter);
+            weights(wc[tap], a.conv_w[tap], a.conv_ld);
+        }
     weights(w2, a.w_out, R);
     const size_t one = n * R + 16 * wave + 4 * quarter, at = n * 2 * R + 16 * wave + 4 * quarter;
     const f32x4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -555,10 +556,12 @@ __global__ __launch_bounds__(4 * R, 1) void wavenet_block_errors_narrow_kernel(c
     };
     f32x4v acc0 = zero, acc1 = zero;
     product(acc0, acc1, w1, b1, KJ, true);
-    product(acc0, acc1, wc[0], bc[0], CJ, live && inside[0] && tap_pat[0] != 0);
-    acc0 = acc0 + acc1;
-    acc1 = zero;
-    product(acc0, acc1, wc[1], bc[1], CJ, live && inside[1] && tap_pat[1] != 0);
+    if constexpr (CONV) {
+        product(acc0, acc1, wc[0], bc[0], CJ, live && inside[0] && tap_pat[0] != 0);
+        acc0 = acc0 + acc1;
+        acc1 = zero;
+        product(acc0, acc1, wc[1], bc[1], CJ, live && inside[1] && tap_pat[1] != 0);
+    }
     f32x4v e = acc0 + acc1;
     if (a.from_skip) e += side;
     es[(4 * wave + quarter) * ROW + col] = e;
@@ -673,15 +676,19 @@ block_err_kernel_t pick_block_errors_kernel(int R, int K, bool conv, bool sum, i
 #undef CNT_BLOCK_KERNELS
     return nullptr;
 }
-template <int R>
+template <int R, bool CONV>
 block_err_kernel_t narrow_block_errors_of(int K) {
     if constexpr (R < 64)
-        if (K == 32) return wavenet_block_errors_narrow_kernel<R, 32>;
-    return K == 64 ? wavenet_block_errors_narrow_kernel<R, 64> : K == 96 ? wavenet_block_errors_narrow_kernel<R, 96> : K == 128 ? wavenet_block_errors_narrow_kernel<R, 128>
-         : K == 256 ? wavenet_block_errors_narrow_kernel<R, 256> : nullptr;
+        if (K == 32) return wavenet_block_errors_narrow_kernel<R, 32, CONV>;
+    return K == 64 ? wavenet_block_errors_narrow_kernel<R, 64, CONV> : K == 96 ? wavenet_block_errors_narrow_kernel<R, 96, CONV>
+         : K == 128 ? wavenet_block_errors_narrow_kernel<R, 128, CONV> : K == 256 ? wavenet_block_errors_narrow_kernel<R, 256, CONV> : nullptr;
 }
-block_err_kernel_t pick_narrow_block_errors_kernel(int R, int K) {
-    return R == 64 ? narrow_block_errors_of<64>(K) : R == 48 ? narrow_block_errors_of<48>(K) : R == 32 ? narrow_block_errors_of<32>(K) : nullptr;
+template <bool CONV>
+block_err_kernel_t narrow_block_errors_of(int R, int K) {
+    return R == 64 ? narrow_block_errors_of<64, CONV>(K) : R == 48 ? narrow_block_errors_of<48, CONV>(K) : R == 32 ? narrow_block_errors_of<32, CONV>(K) : nullptr;
+}
+block_err_kernel_t pick_narrow_block_errors_kernel(int R, int K, bool conv) {
+    return conv ? narrow_block_errors_of<true>(R, K) : narrow_block_errors_of<false>(R, K);
 }
 
 __global__ void sum_context_grad_kernel(int C, int S, int resolution, size_t count, int N,
@@ -1147,7 +1154,7 @@ static int block_errors_threads(int R, int N, bool fold) { return fold && R > 32
 // samples: 64 and 128, 700 443 / 347, 2000 472 / 377, 4000 532 / 450, 8000 651 / 634, 10 000 765 / 779, 16 000 865 / 925; 64 and 256,
 // 3000 604 / 502, 8000 736 / 738, 12 000 920 / 994; 48 and 96, 1000
 // 351 / 294, 8000 518 / 496, 12 000 608 / 622; 32 and 64, 700 286 / 250, 4000 367 / 321, 8000 420 / 406, 16 000 525 / 524; 32 and 256, 6000
-// 517 / 500, 12 000 608 / 615.
+// 517 / 500, 12 000 608 / 615.  The top block, whose errors come without a convolution above, too: 20 blocks of 64 and 128 over 800 521 -> 515.
 static bool narrow_block_errors(int N) { return N <= 8192; }
 
 extern "C++" int cnt::wavenet_block_rows(int R, int N, bool fold) {
@@ -1170,9 +1177,9 @@ extern "C++" int cnt::wavenet_block_errors(hipStream_t stream, int R, int K, int
                                            float *total, const FanOut *fan, const float *core_buf, const float *ctx_tanh,
                                            float *ctx_grad, const float *conv_tanh_outputs, float *conv_errors, const cnt_cnn *fold,
                                            const float *fold_weights, const float *fold_deltas, float *colsum_partial) {
-    const bool narrow = narrow_block_errors(N) && fold && !core_buf && !colsum_partial;  // (it leaves no sums of the deltas)
+    const bool narrow = narrow_block_errors(N) && !core_buf && !colsum_partial;  // (it leaves no sums of the deltas)
     const int threads = narrow ? 4 * R : block_errors_threads(R, N, fold != nullptr);
-    block_err_kernel_t k = narrow ? pick_narrow_block_errors_kernel(R, K) : pick_block_errors_kernel(R, K, fold != nullptr, core_buf == nullptr, threads);
+    block_err_kernel_t k = narrow ? pick_narrow_block_errors_kernel(R, K, fold != nullptr) : pick_block_errors_kernel(R, K, fold != nullptr, core_buf == nullptr, threads);
     CNT_REQUIRE(k != nullptr, "wavenet_block_errors: no kernel for %d residual and %d skip channels", R, K);
     CNT_REQUIRE(N > 0 && patTypes && skip_weights && out_weights && skip_errors && total && (core_buf || (ctx_tanh && conv_tanh_outputs)) &&
                 conv_errors && (!ctx_tanh || ctx_grad) && (core_buf || ctx_grad != ctx_tanh),
