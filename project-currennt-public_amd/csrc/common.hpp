@@ -249,7 +249,8 @@ struct GemmArgs {
     const int *fan_is_skip;
     // Columns of the output that may be left out (k-contiguous B, EPI_STORE and EPI_STORE_DELTA, one k range): column j of the product
     // is column cols[j] of B and C, and from cols_count[0] on the columns get zeros, which is what their products come to
-    // (SlotOrder: the slots of a fraction, those of its padding behind the others).  The kernel for few blocks ignores the list.
+    // (SlotOrder: the slots of a fraction, those of its padding behind the others).  The kernel for few blocks has no use for the list:
+    // gemm_launch takes it away.
     const int *cols;
     const int *cols_count;
     float *partial;        // scratch of splitk * partial_stride floats: the stream's buffer (set by gemm_plan) or the caller's

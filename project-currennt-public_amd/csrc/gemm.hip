@@ -450,6 +450,8 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in, DirectGroup *group)
     if (args.splitk == 1 && args.epilogue != EPI_PARTIAL && direct_product(args)) {
         if (group && !args.a_kcontig && !args.b_kcontig && args.nseg == 1 && args.epilogue == EPI_STORE)
             return gemm_group_add(stream, *group, args);
+        // It multiplies all columns, each in its place, and so do the sums it forms again in fp32, which go by the list where there is one.
+        args.cols = args.cols_count = nullptr;
         ProfileScope prof(stream, args.label ? args.label : "gemm");
         gemm_direct_launch(args, stream);
         CNT_HIP(hipGetLastError());

@@ -362,6 +362,60 @@ def test_errors_of_a_fraction_with_padding(sizes, lengths):
     net.close()
 
 
+@pytest.mark.parametrize("sizes,lengths", [
+    ((40, 64, 36), [30, 21, 8]), ((96, 130, 64), [50, 50, 3, 1]),  # products of few blocks
+    ((512, 512, 512), [130, 125] + [20] * 18)])                     # in tiles
+@pytest.mark.parametrize("where,value", [
+    ("padding", 3e38), ("padding", float("nan")), ("padding", float("-inf")), ("valid", 2.0 ** 113), ("valid", float("nan")),
+    ("target", float("nan")), ("target", 3e38)])
+def test_values_without_a_split_stay_in_their_slot(sizes, lengths, where, value):
+    """A fraction with padding whose products have an operand that the bf16 split has no finite parts for: on a padding slot
+    nothing but that slot changes, on a valid one nothing but its own sequence and the gradients.  Blocks of sums that were infinite are summed again in
+    fp32, (k + 2) * 2^-24 of the terms beside the split's; through the recursion's steps 1e-5 in the 2-norm."""
+    import torch
+
+    print("values without a split", sizes, lengths, where, value, flush=True)
+    capi = PC.pkg().capi
+    S, T, P, Q = len(lengths), max(lengths), 32, 8
+    a, b, c = sizes
+    doc = {"layers": [{"size": P, "name": "input", "type": "input"}, {"size": a, "name": "a", "type": "blstm", "bias": 0.8},
+                      {"size": b, "name": "b", "type": "blstm", "bias": 1.0}, {"size": c, "name": "c", "type": "feedforward_logistic", "bias": 1.0},
+                      {"size": Q, "name": "out", "type": "feedforward_identity", "bias": 1.0}, {"size": Q, "name": "post", "type": "sse"}]}
+    net = capi.Network(json.dumps(doc), S, T)
+    gen = torch.Generator(device="cuda").manual_seed(b)
+    net.weights.uniform_(-0.1, 0.1, generator=gen)
+    types = make_pat_types(lengths, T)
+    pat = PC.dev(types)
+    valid = (pat != 0).reshape(-1, 1)
+    x = (torch.randn(S * T, P, device="cuda", generator=gen) * valid).reshape(-1)
+    target = (torch.randn(S * T, Q, device="cuda", generator=gen) * valid).reshape(-1)
+    # the first slot of padding of the shortest sequence, or a slot of the first sequence beside it
+    step = min(lengths) if where == "padding" else min(lengths) - 1
+    slot = step * S + (lengths.index(min(lengths)) if where == "padding" else 0)
+    assert (types.reshape(-1)[slot] == 0) == (where == "padding")
+    others = valid[:, 0].clone()
+    if where != "padding":
+        others[0::S] = False
+
+    def passed():
+        net.load_sequences(pat, T, min(lengths), x, target)
+        net.forward()
+        net.calculate_error()
+        net.backward()
+        torch.cuda.synchronize()
+        return {"%s.%s" % (n, kind): net.layer(n)[kind].reshape(S * T, -1)[others].clone() for n in ("a", "b", "c", "out") for kind in ("outputs", "errors")}, net.updates.clone()
+
+    want, gradients = passed()
+    (target if where == "target" else x).reshape(S * T, -1)[slot, 5] = value
+    got, changed = passed()
+    for name in want:
+        assert float(want[name].norm()) > 0
+        assert float((got[name] - want[name]).norm()) <= 1e-5 * float(want[name].norm()), name
+    if where == "padding" and np.isfinite(value):  # (a forget gate that is NaN on a slot of padding is multiplied with the zero error there)
+        assert float((changed - gradients).norm()) <= 1e-5 * float(gradients.norm())
+    net.close()
+
+
 def test_networks_share_the_stream_of_their_weight_gradients():
     """Networks on streams and threads of their own, one of them destroyed while the others go on, a new one made, and one more pass
     under capture beside them: every pass's gradients are those of a network that uses the caller's stream alone (1e-6, as
