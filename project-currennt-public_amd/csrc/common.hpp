@@ -333,6 +333,20 @@ __device__ __forceinline__ float sum_of_parts(const float *__restrict__ parts, s
 // stream comes between what it launches.  false: no buffer of that size (as for gemm_plan), nothing was called.
 constexpr size_t kSplitScratchFloats = (size_t)9 << 20;  // 36 MB per (device, stream)
 bool with_split_scratch(hipStream_t stream, size_t floats, const std::function<void(float *)> &enqueue);
+// While it lives, everything that this thread enqueues on `stream` and that would take the stream's split-K scratch takes `buffer` instead
+// (kSplitScratchFloats floats, or null: nothing changes).  For a handle whose products run on a stream of the caller's, which it
+// can neither reserve nor release: the buffer is the handle's, also in a graph that is captured meanwhile.
+class ScratchLoan {
+public:
+    ScratchLoan(hipStream_t stream, float *buffer);
+    ~ScratchLoan();
+    ScratchLoan(const ScratchLoan &) = delete;
+    ScratchLoan &operator=(const ScratchLoan &) = delete;
+
+private:
+    hipStream_t outer_stream_;
+    float *outer_buffer_;
+};
 // number of split-K scratch buffers the library holds at the moment (one per stream that has needed or reserved one)
 int gemm_scratch_buffers();
 // cnt_dense_backward_weights with the partial products in a scratch array that is part of the code object

@@ -187,9 +187,13 @@ bool partial_on() {
     return on;
 }
 
+thread_local hipStream_t t_loan_stream = nullptr;
+thread_local float *t_loan_buffer = nullptr;  // of the thread's ScratchLoan, or null
+
 // One scratch buffer per stream: launches on a stream execute in order, so the next product on the same stream
 // cannot overwrite partial sums that a reduction has yet to read.  Kept until gemm_release_stream.
 float *split_scratch_find(hipStream_t stream) {
+    if (t_loan_buffer && t_loan_stream == stream) return t_loan_buffer;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
     for (const SplitScratch &e : g_split_scratch)
@@ -336,6 +340,16 @@ bool with_split_scratch(hipStream_t stream, size_t floats, const std::function<v
     if (!buf && !capturing(stream)) buf = split_scratch(stream);
     if (buf) enqueue(buf);
     return buf != nullptr;
+}
+
+ScratchLoan::ScratchLoan(hipStream_t stream, float *buffer) : outer_stream_(t_loan_stream), outer_buffer_(t_loan_buffer) {
+    t_loan_stream = stream;
+    t_loan_buffer = buffer;
+}
+
+ScratchLoan::~ScratchLoan() {
+    t_loan_stream = outer_stream_;
+    t_loan_buffer = outer_buffer_;
 }
 
 int gemm_scratch_buffers() {

@@ -515,6 +515,7 @@ struct cnt_network {
     // network's own, since a stream that takes part in a capture may take nothing else meanwhile.
     int device = 0;
     hipStream_t side = nullptr, capture_side = nullptr;
+    float *main_scratch = nullptr;  // split-K scratch of the products on the caller's stream
     hipEvent_t ev_main = nullptr, ev_side = nullptr;
     int overlap = 1;
     // optimizer state (allocated by the first update)
@@ -1165,7 +1166,9 @@ int finish_build(cnt_network *net, const json::Value *weights) {
     CNT_HIP(hipEventCreateWithFlags(&net->ev_main, cnt::kOrderEvent));
     CNT_HIP(hipEventCreateWithFlags(&net->ev_side, cnt::kOrderEvent));
     CNT_HIP(hipStreamCreateWithFlags(&net->capture_side, hipStreamNonBlocking));
-    CNT_TRY(cnt::gemm_reserve_stream(net->capture_side));  // the weight halves' split-K scratch, not inside a pass
+    // the weight halves' split-K scratch, not inside a pass and not the caller's streams'
+    CNT_TRY(cnt::gemm_reserve_stream(net->capture_side));
+    CNT_TRY(device_alloc(net, (void **)&net->main_scratch, kSplitScratchFloats * sizeof(float), false));
     return CNT_OK;
 }
 
@@ -1693,6 +1696,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     CNT_REQUIRE(net && net->T > 0, "network_backward: no fraction loaded");
     CNT_TRY(report_failure(net, static_cast<hipStream_t>(stream_)));
     hipStream_t stream = static_cast<hipStream_t>(stream_);
+    const ScratchLoan loan(stream, net->main_scratch);
     bool side_used = false;
     const bool captured = capturing(stream);  // (a graph's products take the scratch that the side streams have reserved)
     const hipStream_t side = captured ? net->capture_side : net->side;

@@ -416,6 +416,69 @@ def test_values_without_a_split_stay_in_their_slot(sizes, lengths, where, value)
     net.close()
 
 
+@pytest.mark.parametrize("layers,P,S,T", [
+    ([("feedforward_tanh", 512), ("feedforward_tanh", 512)], 382, 12, 500), ([("blstm", 200), ("lstm", 96)], 61, 10, 300),
+    ([("feedforward_tanh", 1024)], 1300, 1, 2048)])  # (in line, its product cut along k)
+@pytest.mark.parametrize("overlap", [True, False])
+@pytest.mark.parametrize("own_stream", [True, False])
+def test_a_pass_takes_no_scratch_of_the_callers_stream(layers, P, S, T, overlap, own_stream):
+    """Products that are cut along k and run on the caller's stream find their scratch with the network: a pass on a stream that has none
+    leaves it so, and the gradients are those of a stream that has.  The same under capture, whose replays give the same bits."""
+    import torch
+
+    print("scratch of the caller's stream", layers, P, S, T, overlap, own_stream, flush=True)
+    capi = PC.pkg().capi
+    Q = 7
+    doc = {"layers": [{"size": P, "name": "input", "type": "input"}] +
+           [{"size": n, "name": "l%d" % i, "type": t, "bias": 1.0} for i, (t, n) in enumerate(layers)] +
+           [{"size": Q, "name": "out", "type": "feedforward_identity", "bias": 1.0}, {"size": Q, "name": "post", "type": "sse"}]}
+    net = capi.Network(json.dumps(doc), S, T, overlap=overlap)
+    gen = torch.Generator(device="cuda").manual_seed(P)
+    net.weights.uniform_(-0.1, 0.1, generator=gen)
+    pat = PC.dev(make_pat_types([T] * S, T))
+    x, target = (torch.randn(S * T * n, device="cuda", generator=gen) for n in (P, Q))
+    stream = torch.cuda.Stream() if own_stream else None
+
+    def passed(stream):
+        net.load_sequences(pat, T, T, x, target, stream=stream)
+        net.forward(stream=stream)
+        net.calculate_error(stream=stream)
+        net.backward(stream=stream)
+
+    torch.cuda.synchronize()
+    capi.gemm_release(stream)
+    held, got = capi.lib().cnt_gemm_scratch_buffers(), []
+    for reserved in (False, True):
+        if reserved:
+            capi.gemm_reserve(stream)
+        net.updates.fill_(3.0)
+        torch.cuda.synchronize()
+        passed(stream)
+        torch.cuda.synchronize()
+        got.append(net.updates.clone())
+        assert capi.lib().cnt_gemm_scratch_buffers() == held + reserved
+    capi.gemm_release(stream)
+    assert float(got[0].norm()) > 0 and torch.equal(got[0], got[1])
+    if own_stream:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+            passed(stream)
+        assert capi.lib().cnt_gemm_scratch_buffers() == held
+        for _ in range(3):
+            net.updates.fill_(3.0)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            # (captured passes keep other batches of products: 1e-6, as above)
+            assert float((net.updates - got[0]).norm()) <= 1e-6 * float(got[0].norm())
+        again = net.updates.clone()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(again, net.updates)
+        del graph
+    net.close()
+
+
 def test_networks_share_the_stream_of_their_weight_gradients():
     """Networks on streams and threads of their own, one of them destroyed while the others go on, a new one made, and one more pass
     under capture beside them: every pass's gradients are those of a network that uses the caller's stream alone (1e-6, as
