@@ -511,17 +511,18 @@ struct cnt_network {
     bool skip_padding = true;
     std::vector<LowRes> low_res;
     std::vector<void *> allocations;
-    // Weight gradients go to a stream beside the caller's: the one that the device's networks share (SideStream), under capture one of the
-    // network's own, since a stream that takes part in a capture may take nothing else meanwhile.
+    // Weight gradients go to a stream beside the caller's: the one that the device's networks have on one of the caller's streams
+    // (SideStream), on others and under capture one of the network's own, since a stream that takes part in a capture may take nothing else meanwhile.
     int device = 0;
-    hipStream_t side = nullptr, capture_side = nullptr;
+    bool side_user = false;
+    hipStream_t own_side = nullptr;
     float *main_scratch = nullptr;  // split-K scratch of the products on the caller's stream
     hipEvent_t ev_main = nullptr, ev_side = nullptr;
     int overlap = 1;
     // optimizer state (allocated by the first update)
     float *cur_updates = nullptr, *deltas = nullptr, *stats = nullptr;
     int stats_option = -1;
-    float *block_sums = nullptr;  // of wavenet_block_weights, whose launches go to the first side stream one after the other
+    float *block_sums = nullptr;  // of wavenet_block_weights, whose launches go to one stream one after the other
     float *adam_accum = nullptr;  // beta1^t, beta2^t of Adam's bias correction (device)
     int mdn_target_start = 0, mdn_classes = 0;
     // set on the device by an LSTM recursion that gives up; the optimizer step looks at it and leaves the weights alone
@@ -531,16 +532,21 @@ struct cnt_network {
 namespace cnt {
 namespace {
 
-// The stream (default priority) on which the networks of a device run their weight gradients, from the first network's creation to the
-// last one's end.  One for all of them: the runtime deals streams to four hardware queues, and a stream that meets the caller's on one
-// of them runs nothing beside it.  With a stream per network every third or fourth network met that: us per pass of four acoustic
-// models side by side 2495, 2484, 2670, 2490.  And one per network, not three round-robin: products that fill the card are only in each
-// other's way and in the main stream's (3 / 2 / 1: feed-forward model 2102 / 2055 / 2037, acoustic model 2500 / 2485 / 2484, 150 and 200 cells with
-// twenty sequences 2095 / 2093 / 2080, 32 sequences 2247 / 2255 / 2267).  What different networks' threads enqueue here runs in the order it came;
-// each pass waits for its own share only.
+// A stream (default priority) on which networks of a device run their weight gradients, from the first network's creation to the
+// last one's end.  One for the networks on a stream of the caller's: the runtime deals streams to four hardware queues, and a stream
+// that meets the caller's on one of them runs nothing beside it.  With a stream per network every third or fourth network met that: us per pass of
+// four acoustic models side by side 2495, 2484, 2670, 2490.  And one per network, not three round-robin: products that fill the card are only
+// in each other's way and in the main stream's (3 / 2 / 1: feed-forward model 2102 / 2055 / 2037, acoustic model 2500 / 2485 / 2484, 150 and 200 cells
+// with twenty sequences 2095 / 2093 / 2080, 32 sequences 2247 / 2255 / 2267).
+// Passes on one stream of the caller's are in order anyway, so those may share.  A network on another one has its weight gradients on its own
+// stream: here they would wait for the other caller's stream, whatever that waits for.  Two networks on threads and streams of their own, all on
+// the one stream / as it is, us per pass of each: three dense layers of 256 over 4800 slots beside the feed-forward model 2232 beside 2389 / 418 beside
+// 2850, beside the acoustic model 2071 beside 2795 / 261 beside 3275, two of them 367 / 269 and 218.
 struct SideStream {
     hipStream_t stream = nullptr;
     int users = 0;
+    const cnt_network *last = nullptr;  // the network that used it last, or null (none, or gone), and on which stream of the caller's
+    hipStream_t caller = nullptr;
 };
 struct SideStreams {
     std::mutex mu;
@@ -550,10 +556,10 @@ SideStreams &side_streams() {
     static SideStreams all;
     return all;
 }
-int acquire_side(int device, hipStream_t *stream) {
+int acquire_side(cnt_network *net) {
     SideStreams &all = side_streams();
     std::lock_guard<std::mutex> lock(all.mu);
-    SideStream &s = all.of_device[device];
+    SideStream &s = all.of_device[net->device];
     if (s.users == 0) {
         CNT_HIP(hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking));
         if (cnt::gemm_reserve_stream(s.stream) != CNT_OK) {
@@ -562,8 +568,25 @@ int acquire_side(int device, hipStream_t *stream) {
         }
     }
     ++s.users;
-    *stream = s.stream;
+    net->side_user = true;
     return CNT_OK;
+}
+
+// The stream beside `caller` for a pass of this network, or null: a graph that has the network's own stream is still being captured.
+hipStream_t side_beside(const cnt_network *net, hipStream_t caller, bool captured) {
+    if (captured) return net->own_side;
+    {
+        SideStreams &all = side_streams();
+        std::lock_guard<std::mutex> lock(all.mu);
+        SideStream &s = all.of_device[net->device];
+        // (a network's passes are in order on whichever streams; hipStreamPerThread is another stream in every thread)
+        if (caller != hipStreamPerThread && (!s.last || s.last == net || s.caller == caller)) {
+            s.last = net;
+            s.caller = caller;
+            return s.stream;
+        }
+    }
+    return capturing(net->own_side) ? nullptr : net->own_side;
 }
 
 int device_alloc(cnt_network *n, void **p, size_t bytes, bool zero) {
@@ -1162,20 +1185,21 @@ int finish_build(cnt_network *net, const json::Value *weights) {
                         "%d, expected %d + %d classes", L.name.c_str(), L.size, L.fb_end - L.fb_start, net->mdn_classes);
         }
     CNT_HIP(hipGetDevice(&net->device));
-    CNT_TRY(acquire_side(net->device, &net->side));
+    CNT_TRY(acquire_side(net));
     CNT_HIP(hipEventCreateWithFlags(&net->ev_main, cnt::kOrderEvent));
     CNT_HIP(hipEventCreateWithFlags(&net->ev_side, cnt::kOrderEvent));
-    CNT_HIP(hipStreamCreateWithFlags(&net->capture_side, hipStreamNonBlocking));
+    CNT_HIP(hipStreamCreateWithFlags(&net->own_side, hipStreamNonBlocking));
     // the weight halves' split-K scratch, not inside a pass and not the caller's streams'
-    CNT_TRY(cnt::gemm_reserve_stream(net->capture_side));
+    CNT_TRY(cnt::gemm_reserve_stream(net->own_side));
     CNT_TRY(device_alloc(net, (void **)&net->main_scratch, kSplitScratchFloats * sizeof(float), false));
     return CNT_OK;
 }
 
-void release_side(int device) {
+void release_side(const cnt_network *net) {
     SideStreams &all = side_streams();
     std::lock_guard<std::mutex> lock(all.mu);
-    SideStream &s = all.of_device[device];
+    SideStream &s = all.of_device[net->device];
+    if (s.last == net) s.last = nullptr;
     if (--s.users > 0) return;
     (void)hipStreamSynchronize(s.stream);
     cnt::gemm_release_stream(s.stream);
@@ -1197,15 +1221,12 @@ int cnt_network_destroy(cnt_network *net) {
         if (L.dft) cnt_dft_destroy(L.dft);
     }
     for (void *p : net->allocations) (void)hipFree(p);
-    if (net->side) {
-        (void)hipStreamSynchronize(net->side);
-        cnt::release_side(net->device);
-    }
-    if (net->capture_side) {
+    if (net->side_user) cnt::release_side(net);
+    if (net->own_side) {
         // the product launcher keeps a scratch buffer per stream it has seen
-        (void)hipStreamSynchronize(net->capture_side);
-        cnt::gemm_release_stream(net->capture_side);
-        (void)hipStreamDestroy(net->capture_side);
+        (void)hipStreamSynchronize(net->own_side);
+        cnt::gemm_release_stream(net->own_side);
+        (void)hipStreamDestroy(net->own_side);
     }
     if (net->ev_side) (void)hipEventDestroy(net->ev_side);
     if (net->ev_main) (void)hipEventDestroy(net->ev_main);
@@ -1699,7 +1720,6 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     const ScratchLoan loan(stream, net->main_scratch);
     bool side_used = false;
     const bool captured = capturing(stream);  // (a graph's products take the scratch that the side streams have reserved)
-    const hipStream_t side = captured ? net->capture_side : net->side;
     // Nothing runs on the caller's stream behind the error half of the lowest layer with weights, so its weight half, and what
     // is still waiting by then, stays there: two hops between streams (9 us each) less in front of the optimizer.
     // Mixture-density output over 6000 slots 189.5 -> 169 us per pass, eight small WaveNet blocks 316 -> 297.
@@ -1744,7 +1764,8 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     std::vector<char> in_block(net->layers.size(), 0);  // weight gradients in the blocks' common launches
     for (size_t i = 5; i < net->layers.size(); ++i)
         if (block_at(i) && block_weights_at(net, i)) in_block[i] = in_block[i - 3] = in_block[i - 4] = in_block[i - 5] = 1;
-    const bool overlap = net->overlap && (captured || !weights_in_line(net, in_block));
+    const hipStream_t side = net->overlap && (captured || !weights_in_line(net, in_block)) ? side_beside(net, stream, captured) : nullptr;
+    const bool overlap = side != nullptr;
     std::vector<size_t> pending;
     DirectGroup in_line;  // products of few blocks on the caller's stream: one launch at the end of the pass
     in_line.count = in_line.blocks = 0;

@@ -480,9 +480,9 @@ def test_a_pass_takes_no_scratch_of_the_callers_stream(layers, P, S, T, overlap,
 
 
 def test_networks_share_the_stream_of_their_weight_gradients():
-    """Networks on streams and threads of their own, one of them destroyed while the others go on, a new one made, and one more pass
-    under capture beside them: every pass's gradients are those of a network that uses the caller's stream alone (1e-6, as
-    above)."""
+    """Networks on one stream, on streams and threads of their own, one of them destroyed while the others go on, a new one made, and one more
+    pass under capture beside them: every pass's gradients are those of the same network, weights, inputs and targets on the caller's
+    stream alone (1e-6, as above).  No two networks have the same, so that one's sums in another's are seen."""
     import threading
 
     import torch
@@ -493,65 +493,178 @@ def test_networks_share_the_stream_of_their_weight_gradients():
                                  {"size": 128, "name": "b", "type": "blstm", "bias": 1.0},
                                  {"size": Q, "name": "out", "type": "feedforward_identity", "bias": 1.0}, {"size": Q, "name": "post", "type": "sse"}]})
     pat = PC.dev(make_pat_types([T] * S, T))
-    gen = torch.Generator(device="cuda").manual_seed(5)
-    x, target = (torch.randn(S * T * n, device="cuda", generator=gen) for n in (P, Q))
-    weights = None
 
-    def made(overlap=True):
-        nonlocal weights
-        net = capi.Network(doc, S, T, overlap=overlap)
-        if weights is None:
-            weights = net.weights.uniform_(-0.1, 0.1, generator=gen).clone()
-        net.weights.copy_(weights)
-        return net
+    class Run:
+        def __init__(self, seed):
+            gen = torch.Generator(device="cuda").manual_seed(seed)
+            self.x, self.target = (torch.randn(S * T * n, device="cuda", generator=gen) for n in (P, Q))
+            self.net = capi.Network(doc, S, T, overlap=False)
+            weights = self.net.weights.uniform_(-0.1, 0.1, generator=gen).clone()
+            self.go()
+            torch.cuda.synchronize()
+            self.want = self.net.updates.clone()
+            self.net.close()
+            self.net = capi.Network(doc, S, T)
+            self.net.weights.copy_(weights)
+            torch.cuda.synchronize()
 
-    def passed(net, stream=None):
-        net.load_sequences(pat, T, T, x, target, stream=stream)
-        net.forward(stream=stream)
-        net.calculate_error(stream=stream)
-        net.backward(stream=stream)
+        def go(self, stream=None):
+            self.net.load_sequences(pat, T, T, self.x, self.target, stream=stream)
+            self.net.forward(stream=stream)
+            self.net.calculate_error(stream=stream)
+            self.net.backward(stream=stream)
 
-    alone = made(False)
-    passed(alone)
-    torch.cuda.synchronize()
-    want = alone.updates.clone()
-    nets = [made() for _ in range(3)]
-    torch.cuda.synchronize()
+        def right(self):
+            return float((self.net.updates - self.want).norm()) <= 1e-6 * float(self.want.norm())
+
+    runs = [Run(seed) for seed in range(5, 8)]
+    for a in runs:
+        for b in runs:
+            assert a is b or float((a.want - b.want).norm()) > 0.1 * float(a.want.norm())
     wrong = []
 
-    def work(net):
+    def work(run):
         stream = torch.cuda.Stream()
         for _ in range(4):
-            net.updates.fill_(3.0)
+            run.net.updates.fill_(3.0)
             torch.cuda.synchronize()
-            passed(net, stream)
+            run.go(stream)
             stream.synchronize()
-            if not float((net.updates - want).norm()) <= 1e-6 * float(want.norm()):
-                wrong.append(net)
+            if not run.right():
+                wrong.append(run)
 
-    threads = [threading.Thread(target=work, args=(n,)) for n in nets[:2]]
+    threads = [threading.Thread(target=work, args=(r,)) for r in runs]
     for t in threads:
         t.start()
     for t in threads:
         t.join()
     assert not wrong
-    nets[0].close()
-    nets.append(made())
-    for net in nets[1:]:
-        passed(net)
+    runs.pop(0).net.close()
+    runs.append(Run(8))
+    for _ in range(2):
+        for run in runs:
+            run.net.updates.fill_(3.0)
+            run.go()
     torch.cuda.synchronize()
+    assert all(run.right() for run in runs)
     graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
     with torch.cuda.graph(graph, stream=stream):
-        passed(nets[1], torch.cuda.current_stream())
+        runs[0].go(torch.cuda.current_stream())
     for _ in range(3):
-        nets[1].updates.fill_(3.0)
-        nets[2].updates.fill_(3.0)
+        for run in runs[:2]:
+            run.net.updates.fill_(3.0)
         graph.replay()
-        passed(nets[2])
+        runs[1].go()
         torch.cuda.synchronize()
-        for net in nets[1:]:
-            assert float((net.updates - want).norm()) <= 1e-6 * float(want.norm())
-    for net in nets[1:] + [alone]:
+        assert all(run.right() for run in runs)
+    for run in runs:
+        run.net.close()
+
+
+def dense_network(capi, seed, S=8, T=512, P=64, n=256, Q=32):
+    """A feed-forward network whose pass is too large for weight gradients in line, and what a pass of it takes."""
+    import torch
+
+    doc = {"layers": [{"size": P, "name": "input", "type": "input"}] +
+           [{"size": n, "name": "l%d" % i, "type": "feedforward_tanh", "bias": 1.0} for i in range(3)] +
+           [{"size": Q, "name": "out", "type": "feedforward_identity", "bias": 1.0}, {"size": Q, "name": "post", "type": "sse"}]}
+    net = capi.Network(json.dumps(doc), S, T)
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    net.weights.uniform_(-0.1, 0.1, generator=gen)
+    pat = PC.dev(make_pat_types([T] * S, T))
+    x, target = (torch.randn(S * T * k, device="cuda", generator=gen) for k in (P, Q))
+
+    def go(stream):
+        net.load_sequences(pat, T, T, x, target, stream=stream)
+        net.forward(stream=stream)
+        net.calculate_error(stream=stream)
+        net.backward(stream=stream)
+
+    return net, go
+
+
+def test_a_network_does_not_wait_for_another_callers_stream():
+    """Two networks on two streams, one of which is busy with something else first: the other one's pass ends meanwhile.  (Streams that the
+    runtime puts on one hardware queue do wait for each other, so several pairs of streams and networks are tried; one is enough.)"""
+    import torch
+
+    capi = PC.pkg().capi
+    first, first_go = dense_network(capi, 1)
+    others = [dense_network(capi, seed) for seed in (2, 3)]
+    begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    for go in [first_go] + [o[1] for o in others]:
+        go(None)
+    torch.cuda.synchronize()
+    begin.record()
+    torch.cuda._sleep(1 << 20)
+    end.record()
+    torch.cuda.synchronize()
+    cycles = int((1 << 20) * 40.0 / max(begin.elapsed_time(end), 1e-3))  # 40 ms
+    free = []
+    for k in range(12):
+        mine, busy = torch.cuda.Stream(), torch.cuda.Stream()
+        other_go = others[k % 2][1]
+        with torch.cuda.stream(busy):
+            torch.cuda._sleep(cycles)
+        other_go(busy)
+        first_go(mine)
+        mine.synchronize()
+        free.append(not busy.query())
+        torch.cuda.synchronize()
+        if free[-1]:
+            break
+    assert any(free), free
+    for net in [first] + [o[0] for o in others]:
+        net.close()
+
+
+def test_the_stream_beside_the_callers_is_one_for_a_callers_stream():
+    """The gradients of passes that alternate between networks and streams, of a pass between a capture's pass and its end, and of
+    networks whose predecessor on the shared stream is gone: bit for bit those of the network's first pass."""
+    import torch
+
+    capi = PC.pkg().capi
+    nets = [dense_network(capi, seed) for seed in (1, 2, 3)]
+    want = []
+    for net, go in nets:
+        go(None)
+        torch.cuda.synchronize()
+        want.append(net.updates.clone())
+    streams = [None, torch.cuda.Stream(), torch.cuda.Stream()]
+
+    def check(order):
+        torch.cuda.synchronize()
+        for i, stream in order:
+            nets[i][0].updates.fill_(3.0)
+            torch.cuda.synchronize()
+        for i, stream in order:
+            nets[i][1](stream)
+        torch.cuda.synchronize()
+        for i, _ in order:
+            assert torch.equal(nets[i][0].updates, want[i]), (i, order)
+
+    for order in ([0, 1, 2], [1, 2, 0], [2, 2, 1], [0, 0, 0], [1, 1, 2]):
+        check([(i, streams[s]) for i, s in enumerate(order)])
+    # a network's own stream that takes part in a capture may take nothing else before the capture's end
+    check([(0, streams[1]), (1, streams[2])])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream(), capture_error_mode="relaxed"):
+        nets[1][1](torch.cuda.current_stream())
+        nets[1][1](streams[2])
+    torch.cuda.synchronize()
+    assert float((nets[1][0].updates - want[1]).norm()) <= 1e-6 * float(want[1].norm())  # (in line: other batches of products)
+    for _ in range(3):
+        nets[1][0].updates.fill_(3.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((nets[1][0].updates - want[1]).norm()) <= 1e-6 * float(want[1].norm())
+    del graph
+    check([(0, streams[1])])
+    nets[0][0].close()
+    nets.pop(0)
+    want.pop(0)
+    check([(0, streams[2]), (1, streams[1])])
+    for net, _ in nets:
         net.close()
 
 
