@@ -2,6 +2,7 @@
 turned into the layer list, and forward pass, error, backward pass and optimizer step of a fraction are compared
 with the CPU oracle doing the same steps.  Tolerance 1e-4 on L2-normalised differences (fp32, different summation
 orders), the tolerance of the layer kernels themselves."""
+import itertools
 import json
 
 import numpy as np
@@ -594,26 +595,28 @@ def test_a_network_does_not_wait_for_another_callers_stream():
     begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
     for go in [first_go] + [o[1] for o in others]:
         go(None)
+    for _ in range(2):  # (the first sleep loads its code)
+        torch.cuda.synchronize()
+        begin.record()
+        torch.cuda._sleep(1 << 20)
+        end.record()
     torch.cuda.synchronize()
-    begin.record()
-    torch.cuda._sleep(1 << 20)
-    end.record()
-    torch.cuda.synchronize()
-    cycles = int((1 << 20) * 40.0 / max(begin.elapsed_time(end), 1e-3))  # 40 ms
+    cycles = int((1 << 20) * 20.0 / begin.elapsed_time(end))  # 20 ms
+    streams = [torch.cuda.Stream() for _ in range(5)]
     free = []
-    for k in range(12):
-        mine, busy = torch.cuda.Stream(), torch.cuda.Stream()
-        other_go = others[k % 2][1]
+    for (_, other_go), busy, mine in itertools.product(others, streams, streams):
+        if busy is mine or any(free):
+            continue
         with torch.cuda.stream(busy):
             torch.cuda._sleep(cycles)
+            slept = torch.cuda.Event()
+            slept.record()
         other_go(busy)
         first_go(mine)
         mine.synchronize()
-        free.append(not busy.query())
+        free.append(not slept.query())
         torch.cuda.synchronize()
-        if free[-1]:
-            break
-    assert any(free), free
+    assert any(free)
     for net in [first] + [o[0] for o in others]:
         net.close()
 
