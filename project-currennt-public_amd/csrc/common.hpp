@@ -295,7 +295,6 @@ int gemm_group_add(hipStream_t stream, DirectGroup &group, const GemmArgs &plann
 int gemm_group_launch(hipStream_t stream, DirectGroup &group);
 // whether a product with these operands can take the EPI_FAN epilogue (operand kinds, alignment)
 bool gemm_fan_supported(const GemmArgs &args);
-struct DirectGroup;
 // group: a weight gradient that takes the few-block kernel waits there for others of its kind, until gemm_group_launch
 int gemm_launch(hipStream_t stream, const GemmArgs &args, DirectGroup *group = nullptr);
 // Frees the split-K scratch buffer that the launcher keeps for `stream` (for owners of a stream about to destroy
@@ -367,15 +366,14 @@ int opt_step_guarded(hipStream_t stream, int option, long n, float *weights, con
 int opt_adam_advance(hipStream_t stream, float *accum_dev, const int *veto);
 // LSTM handles of a network share one such flag: a recursion that gives up also sets *veto (until the owner clears it).
 void lstm_set_veto(cnt_lstm *h, int *veto);
-// non-zero if a recursion of this handle has given up since the last report (no synchronisation: it only sees
-// launches that have already ended); the report clears the mark
-// cnt_lstm_backward_weights in two parts that write disjoint ranges (1: input weights, 2: the rest)
-int lstm_backward_weights_parts(cnt_lstm *h, hipStream_t stream, const float *x, float *weight_updates, int parts,
-                                DirectGroup *group = nullptr);
-// cnt_lstm_backward_errors whose recursion also sums up the bias and peephole gradients; the parts are then asked for with kSumsDone
-constexpr int kSumsDone = 4;
+// cnt_lstm_backward_weights; sums_done: the error half was lstm_backward_errors_sums.  group: products of few blocks wait there.
+int lstm_backward_weights_grouped(cnt_lstm *h, hipStream_t stream, const float *x, float *weight_updates, bool sums_done,
+                                  DirectGroup *group = nullptr);
+// cnt_lstm_backward_errors whose recursion also sums up the bias and peephole gradients
 int lstm_backward_errors_sums(cnt_lstm *h, hipStream_t stream, const float *weights, float *output_errors, float *prev_errors,
                               float *weight_updates);
+// non-zero if a recursion of this handle has given up since the last report (no synchronisation: it only sees
+// launches that have already ended); the report clears the mark
 int lstm_take_failure(cnt_lstm *h);
 // makes `other` wait for the recursion launched last on this handle's device (the event the library records behind
 // every recursion launch anyway): what a stream needs that consumes the recursion's results, without another event

@@ -1154,7 +1154,7 @@ int cnt_lstm_backward_errors(cnt_lstm *h, void *stream_, const float *weights, f
     return cnt::lstm_backward_errors_sums(h, static_cast<hipStream_t>(stream_), weights, output_errors, prev_errors, nullptr);
 }
 
-// weight_updates: the bias and peephole gradients are summed up on the way, for lstm_backward_weights_parts with kSumsDone; only within
+// weight_updates: the bias and peephole gradients are summed up on the way, for lstm_backward_weights_grouped with sums_done; only within
 // one call of this library's, between whose halves nobody can change the states
 extern "C++" int cnt::lstm_backward_errors_sums(cnt_lstm *h, hipStream_t stream, const float *weights, float *output_errors,
                                                 float *prev_errors, float *weight_updates) {
@@ -1283,18 +1283,16 @@ extern "C++" int cnt::lstm_prev_errors_delta(cnt_lstm *h, hipStream_t stream, co
 }
 
 int cnt_lstm_backward_weights(cnt_lstm *h, void *stream, const float *x, float *weight_updates) {
-    return cnt::lstm_backward_weights_parts(h, static_cast<hipStream_t>(stream), x, weight_updates, 3);
+    return cnt::lstm_backward_weights_grouped(h, static_cast<hipStream_t>(stream), x, weight_updates, false);
 }
 
-// parts: 1 = input weights, 2 = bias, recurrent and peephole weights; the two parts write disjoint ranges of the
-// weight updates and may run on different streams.  With kSumsDone the error half was lstm_backward_errors_sums.
-extern "C++" int cnt::lstm_backward_weights_parts(cnt_lstm *h, hipStream_t stream, const float *x, float *weight_updates,
-                                                  int parts, DirectGroup *group) {
+extern "C++" int cnt::lstm_backward_weights_grouped(cnt_lstm *h, hipStream_t stream, const float *x, float *weight_updates, bool sums_done,
+                                                    DirectGroup *group) {
     DirectGroup own;
     own.count = own.blocks = 0;
     if (!group) {
         // products of few blocks: both in one launch (a layer of 256 cells over 800 slots 14 + 9.5 us one after the other)
-        CNT_TRY(lstm_backward_weights_parts(h, stream, x, weight_updates, parts, &own));
+        CNT_TRY(lstm_backward_weights_grouped(h, stream, x, weight_updates, sums_done, &own));
         return gemm_group_launch(stream, own);
     }
     CNT_REQUIRE(h && x && weight_updates, "lstm_backward_weights: null argument");
@@ -1307,8 +1305,7 @@ extern "C++" int cnt::lstm_backward_weights_parts(cnt_lstm *h, hipStream_t strea
     const size_t nW = weight_count(P, L, d.bidir);
     const size_t off_bias = (size_t)4 * P * L, off_int = off_bias + (size_t)4 * L;
     const size_t off_peep = off_int + (size_t)4 * L * H;
-    const bool summed = (parts & kSumsDone) && h->sums;
-    if ((parts & 2) && summed) {
+    if (sums_done && h->sums) {
         if (h->groups > 1) {
             SmallGradDirs sp = {};
             sp.H = H; sp.L = L; sp.parts = h->sums;
@@ -1320,7 +1317,7 @@ extern "C++" int cnt::lstm_backward_weights_parts(cnt_lstm *h, hipStream_t strea
                                h->ndir, h->groups);
             CNT_HIP(hipGetLastError());
         }
-    } else if (parts & 2) {
+    } else {
         // In front of the products: reading all states is bound by memory and goes by beside another stream's products, while behind them,
         // at a pass's end, the card had nothing else to do (32 sequences 2485 -> 2448 us per pass, acoustic model 2572 -> 2559).
         SmallGradDirs sp;
@@ -1353,7 +1350,7 @@ extern "C++" int cnt::lstm_backward_weights_parts(cnt_lstm *h, hipStream_t strea
         }
         CNT_HIP(hipGetLastError());
     }
-    if (parts & 1) {
+    {
         // input weights: dW_in[g,dir] (P x H) = x (P x N) * delta^T
         GemmArgs ga = {};
         ga.m = P; ga.n = H; ga.k = N;
@@ -1380,7 +1377,6 @@ extern "C++" int cnt::lstm_backward_weights_parts(cnt_lstm *h, hipStream_t strea
         if (ga.epilogue == EPI_ATOMIC) CNT_TRY(fill_zero(stream, weight_updates, off_bias));
         CNT_TRY(gemm_launch(stream, ga, group));
     }
-    if (!(parts & 2)) return CNT_OK;
     if (h->T > 1) {
         // recurrent weights: dW_int[g,dir][src + to*H] = sum h[src] at the earlier step * delta[to]
         GemmArgs ga = {};
@@ -1426,7 +1422,7 @@ int cnt_lstm_backward(cnt_lstm *h, void *stream, const float *weights, const flo
     CNT_REQUIRE(x && weight_updates, "lstm_backward_weights: null argument");
     hipStream_t s = static_cast<hipStream_t>(stream);
     CNT_TRY(lstm_backward_errors_sums(h, s, weights, output_errors, prev_errors, weight_updates));
-    return lstm_backward_weights_parts(h, s, x, weight_updates, 3 | kSumsDone);
+    return lstm_backward_weights_grouped(h, s, x, weight_updates, true);
 }
 
 }  // extern "C"

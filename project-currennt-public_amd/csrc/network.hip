@@ -1778,7 +1778,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
             const float *x = prev.out, *e = L.err;
             return dense_backward_weights_batch(ws, prev.size, L.size, L.N, 1, &L.bias, &x, &e, &dW, &L.order, group);
         }
-        if (L.kind == K_LSTM) return lstm_backward_weights_parts(L.lstm, ws, prev.out, dW, 3 | kSumsDone, group);
+        if (L.kind == K_LSTM) return lstm_backward_weights_grouped(L.lstm, ws, prev.out, dW, true, group);
         if (L.kind == K_CNN) return cnt_cnn_backward_weights(L.cnn, ws, L.pat, L.T, prev.out, L.err, dW);
         return cnt_wavnetc_backward_weights(ws, L.size, L.ctx_dim, L.N, net->ctx, L.cgrad, dW);
     };
