@@ -90,6 +90,12 @@ __device__ __forceinline__ unsigned ctl_load(const unsigned *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Rounds of a wait for the team's job in which the thread also looks whether all jobs are taken: every fourth, and the one before it gives up,
+// so that a team that stays incomplete is no failure, however small the limit.
+__host__ __device__ constexpr bool looks_at_claims(unsigned spins, unsigned spin_limit) { return (spins & 3u) == 3u || spins >= spin_limit; }
+static_assert(looks_at_claims(0, 0) && looks_at_claims(1, 1) && looks_at_claims(2, 2) && looks_at_claims(3, 100) && !looks_at_claims(4, 5) &&
+              looks_at_claims(5, 5), "the last round before giving up looks");
+
 // Role of this workgroup: job * 64 + member (a team has at most 32 workgroups), or -1.  Called by one thread.
 __device__ int local_claim_role(const ChainParams &p, int G) {
     const unsigned xcd = __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15u;  // XCC_ID, bits 3:0
@@ -122,7 +128,7 @@ __device__ int local_claim_role(const ChainParams &p, int G) {
             job = ctl_load(team_job);
             if (job != 0u) break;
             // every job is taken and this team is still incomplete: whoever completes it will find none left
-            if ((spins & 3u) == 3u && ctl_load(claimed) >= (unsigned)p.njobs && ctl_load(arrived) < (unsigned)G) { job = kNoJob; break; }
+            if (looks_at_claims(spins, p.spin_limit) && ctl_load(claimed) >= (unsigned)p.njobs && ctl_load(arrived) < (unsigned)G) { job = kNoJob; break; }
             if (++spins > p.spin_limit || ((spins & 15u) == 0u && __hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
                 raise_abort(p);
                 job = kNoJob;
