@@ -1693,11 +1693,17 @@ static bool has_weight_half(const cnt::NetLayer &L) {
 }
 
 // A small pass's weight halves stay on the caller's stream: a hop to another stream and back takes the host some 25 us and the
-// card 18, and in line the products of few blocks are one launch.  The line goes by the multiply-adds of the weight gradients, and by the
-// slots, beyond which those products are cut along k.  Us per pass on other streams / in line, slots in brackets: three layers of 256
-// (120) 142 / 70, (960) 137 / 76, (1920) 142 / 90; three of 1024 (480, 1.2e9) 188 / 162, (960, 2.4e9) 267 / 256, (1920, 4.8e9) 312 / 332; 32 and
-// blstm 128 (240) 150 / 132, (960) 368 / 347, (1920) 382 / 359; two lstm 256 (240) 316 / 298, (960) 823 / 807, (1920, 2e9) 872 / 831; the acoustic
-// model (60) 395 / 374, (240) 435 / 396, (480, 1.8e9) 636 / 592, (960, 3.5e9) 977 / 974, (1920, 7e9) 1130 / 1162.
+// card 18, and in line the products of few blocks are one launch.  The line goes by the slots, beyond which those products are cut along k, and
+// by the multiply-adds of the weight gradients.  Us per pass on another stream / in line, slots in brackets.
+// With recursions, which run while another stream's products do: 32 and blstm 128 (120) 107 / 90, (960) 357 / 341, (2048) 395 / 375, (2400) 461 /
+// 468, (4800) 467 / 476; two lstm 256 (120) 214 / 195, (960) 801 / 778, (2048, 1.9e9) 872 / 855, (2400) 1005 / 1026, (4800) 1130 / 1160; lstm 512 (1440,
+// 1.8e9) 514 / 500, (2000, 2.6e9) 671 / 656; the acoustic model (60 to 480, up to 1.8e9) the same, (720, 2.7e9) 755 / 764, (960, 3.6e9) 938 / 940,
+// (1200, 4.4e9) 798 / 812, (1920, 7.1e9) 1140 / 1203: to 3e9.
+// Dense layers alone, whose products of few blocks are one launch at the pass's end either way: the lowest one's gradient stays in line too, so
+// those above it count.  Three of 1024 (120) 108 / 99, (480, 1.1e9) 147 / 145, (720, 1.6e9) 213 / 232, (840, 1.8e9) 219 / 237, (1200, 2.6e9) 257 /
+// 286; five of 512 (960, 1.1e9) 174 / 151, (1440, 1.6e9) 265 / 248, (1680, 1.8e9) 252 / 256; three of 512 (2400) 203 / 224; four of 640 (720, 1e9) 171 /
+// 147, (1440, 1.9e9) 256 / 264, (2000, 2.7e9) 296 / 315; three of 800 (720, 1e9) 155 / 166, (1440, 1.9e9) 215 / 244; three of 256 (960) 66 / 67, (2400)
+// 115 / 144; five of 64 (1920) 82 / 82, (4800) 144 / 166: to 1.7e9.
 // Blocks of 32 / 64 and 64 / 128 channels: 8 of them (2000) 249 / 235, (4000) 268 / 280, 20 (2000) 491 / 462, 10 wide ones (2000) 446 / 422,
 // (4000) 478 / 485.  Convolutions without the blocks' launches, whose products are batched over layers on another stream, stay there: 20
 // blocks of 48 channels (2000) layer by layer 1095 / 1740.
@@ -1705,11 +1711,17 @@ static bool weights_in_line(const cnt_network *net, const std::vector<char> &in_
     using namespace cnt;
     const long slots = static_cast<long>(net->S) * net->T;
     if (slots > 2048) return false;
-    for (size_t i = 0; i < net->layers.size(); ++i) {
+    bool dense_only = true, lowest = true;
+    double above = 0;  // weights of the dense layers above the lowest one
+    for (size_t i = 1; i < net->layers.size(); ++i) {
         const NetLayer &L = net->layers[i];
-        if ((L.kind == K_CNN || L.kind == K_WAVNETC) && has_weight_half(L) && !in_block[i]) return false;
+        if (!has_weight_half(L)) continue;
+        if ((L.kind == K_CNN || L.kind == K_WAVNETC) && !in_block[i]) return false;
+        if (L.kind != K_DENSE) dense_only = false;
+        else if (!lowest) above += static_cast<double>(net->layers[i - 1].size) * L.size;
+        lowest = false;
     }
-    return static_cast<double>(net->n_weights) * static_cast<double>(slots) <= 3e9;
+    return static_cast<double>(net->n_weights) * static_cast<double>(slots) <= 3e9 && !(dense_only && above * static_cast<double>(slots) > 1.7e9);
 }
 
 int cnt_network_backward(cnt_network *net, void *stream_) {

@@ -562,14 +562,14 @@ def test_networks_share_the_stream_of_their_weight_gradients():
         run.net.close()
 
 
-def dense_network(capi, seed, S=8, T=512, P=64, n=256, Q=32):
-    """A feed-forward network whose pass is too large for weight gradients in line, and what a pass of it takes."""
+def dense_network(capi, seed, S=8, T=512, P=64, n=256, Q=32, overlap=True):
+    """A feed-forward network, by itself one whose pass is too large for weight gradients in line, and what a pass of it takes."""
     import torch
 
     doc = {"layers": [{"size": P, "name": "input", "type": "input"}] +
            [{"size": n, "name": "l%d" % i, "type": "feedforward_tanh", "bias": 1.0} for i in range(3)] +
            [{"size": Q, "name": "out", "type": "feedforward_identity", "bias": 1.0}, {"size": Q, "name": "post", "type": "sse"}]}
-    net = capi.Network(json.dumps(doc), S, T)
+    net = capi.Network(json.dumps(doc), S, T, overlap=overlap)
     gen = torch.Generator(device="cuda").manual_seed(seed)
     net.weights.uniform_(-0.1, 0.1, generator=gen)
     pat = PC.dev(make_pat_types([T] * S, T))
@@ -619,6 +619,24 @@ def test_a_network_does_not_wait_for_another_callers_stream():
     assert any(free)
     for net in [first] + [o[0] for o in others]:
         net.close()
+
+
+@pytest.mark.parametrize("T", [781, 782, 2048, 2049])  # 1.7e9 multiply-adds above the lowest layer, and the slots' line
+def test_gradients_in_line_and_beside_the_callers_stream(T):
+    """Feed-forward gradients at the lines between weight halves on the caller's stream and on the one beside it, against all on the
+    caller's (1e-6, as above)."""
+    import torch
+
+    capi = PC.pkg().capi
+    got = []
+    for overlap in (True, False):
+        net, go = dense_network(capi, 4, 1, T, 16, 1024 if T < 2000 else 256, 76 if T < 2000 else 32, overlap)
+        net.updates.fill_(3.0)
+        go(None)
+        torch.cuda.synchronize()
+        got.append(net.updates.clone())
+        net.close()
+    assert float(got[1].norm()) > 0 and float((got[0] - got[1]).norm()) <= 1e-6 * float(got[1].norm())
 
 
 def test_the_stream_beside_the_callers_is_one_for_a_callers_stream():
