@@ -476,9 +476,10 @@ int cnn_backward_weights_batch(cnt_cnn *const *h, int count, hipStream_t stream,
                                const float *const *x, const float *const *output_errors, float *const *weight_updates,
                                const float *const *colsum_partial = nullptr, const int *colsum_rows = nullptr);
 
-// Flags of the events that order this library's streams among each other: the consumer is always a kernel of the same device, and a
-// kernel's end makes its results visible to that.  Without the record's system-wide fence, which is for readers on the host or
-// other devices, a launch behind a record starts 2 to 3 us earlier: acoustic model 2539 -> 2525 us per pass, one lstm layer 372 -> 368,
+// Flags of the events that order this library's streams among each other: what such an event orders is always a kernel of the same device, and a
+// kernel's end makes its results visible to that.  The host only asks whether such an event is over (lstm_take_failure); what it then reads, a
+// recursion's latch, is stored at system scope and needs no fence either.  Without the record's system-wide fence, which is for readers on the host
+// or other devices, a launch behind a record starts 2 to 3 us earlier: acoustic model 2539 -> 2525 us per pass, one lstm layer 372 -> 368,
 // eight small WaveNet blocks 298 -> 284.
 constexpr unsigned kOrderEvent = hipEventDisableTiming | hipEventDisableSystemFence;
 

@@ -658,8 +658,11 @@ block_err_kernel_t block_errors_of(bool conv, bool sum, int threads) {
     return conv ? (sum ? wavenet_block_errors_kernel<R, K, true, true, 256> : wavenet_block_errors_kernel<R, K, true, false, 256>)
                 : (sum ? wavenet_block_errors_kernel<R, K, false, true, 256> : wavenet_block_errors_kernel<R, K, false, false, 256>);
 }
-// Widths that have the launch: the residual channels of the forward pass's launch with the usual numbers of skip channels.  All others go
-// layer by layer, and their weight gradients then do so as well.  us per pass layer by layer / with the launch, residual and skip channels, slots,
+// Widths that have the launch: a kernel of its own for each, which is why there is a table: the residual channels of the forward pass's launch with
+// 64, 96, 128 or 256 skip channels, up to 48 residual channels with 32 as well.  Skip channels between those, which the forward launch takes in
+// any multiple of 16, go layer by layer, and their weight gradients then do so as well.  So do 64 and 32, which a kernel would take from 550 to
+// 344 us per pass (8 blocks, 4000 samples): the scratch of its weight gradients, by the largest job's sums for every workgroup, would be 34 MB
+// where the sums that are dealt need 18.  us per pass layer by layer / with the launch, residual and skip channels, slots,
 // blocks: 48 and 96, 2001, 20 1019 / 560; 48 and 64, 16 200, 10 965 / 607; 48 and 128, 24 000, 30 3405 / 2291; 48 and 256, 32 000, 20 3017 /
 // 2259; 64 and 96, 16 000, 20 1980 / 1305; 32 and 96, 1000, 10 490 / 267; 32 and 256, 24 000, 20 2372 / 1676.
 // Gradients' 2-norm error against 64 bits there 1.2 to 6.5e-7, layer by layer 1.3 to 6.9e-7.

@@ -130,9 +130,10 @@ def test_block_weight_gradients_under_capture():
     net.close()
 
 
-@pytest.mark.parametrize("R,K,scratch", [(64, 128, True), (48, 96, False), (64, 32, False), (32, 256, False)])
-def test_scratch_of_the_common_launches_only_where_they_are_made(R, K, scratch):
-    """A stack whose block sizes have no launch for the errors sums its weight gradients without the blocks' scratch (34 MB)."""
+@pytest.mark.parametrize("R,K,sums", [(64, 128, 16), (48, 96, 12), (32, 256, 4), (64, 32, 0), (48, 80, 0)])
+def test_scratch_of_the_common_launches_only_where_they_are_made(R, K, sums):
+    """The blocks' scratch of a stack whose widths have the launch for the errors holds 32 x 32 blocks of sums, as many as the job with the most
+    has, and 256 more for each of 512 workgroups: 34, 26 and 9 MB.  A stack of other widths sums its weight gradients without."""
     import torch
 
     pkg = PC.pkg()
@@ -146,5 +147,7 @@ def test_scratch_of_the_common_launches_only_where_they_are_made(R, K, scratch):
         net.close()
         return before - after
 
-    # (beside the same stack without conditioning features, which never has it)
-    assert (taken(20) - taken(0) >= 32 << 20) == scratch
+    # (beside the same stack without conditioning features, which never has it; the layers' own buffers and what an allocation is rounded up
+    # to differ by less than 4 MB)
+    need = 512 * (sums * 1024 + 256) * 4 if sums else 0
+    assert abs(taken(20) - taken(0) - need) < 4 << 20
