@@ -70,8 +70,8 @@ def run(args, pkg):
     roof = {"bound": "hbm", "kernel": dom, "traffic": None, "peak": PEAK_HBM_GBS, "unit": "GB/s"}
     if dom == "wavenet_block_errors+cnn" and (R, K, N) == (64, 128, 32000):
         # two rocprofv3 --pmc runs (FETCH_SIZE x 2.00 by a copy of known size, WRITE_SIZE x 1.00) of this workload:
-        # 82.0 MB read + 44.6 MB written per launch of wavenet_block_errors_kernel<64, 128, true, true, 512>
-        roof["traffic"] = 126.6e6
+        # 82.3 MB read + 44.5 MB written per launch of wavenet_block_errors_kernel<64, 128, true, true, 512>
+        roof["traffic"] = 126.8e6
         roof["traffic_source"] = "profiles/wavenet_c4_backward_kernel_stats.md"
     if dom == "wavenet_block_errors+cnn":
         # one residual block's error path: reads the skip errors (K), what the later block handed on (R), the deltas of

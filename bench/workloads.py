@@ -92,8 +92,8 @@ def lstm_c1(args, pkg):
     hop_us = capi.probe_hop_latency(same_xcd=True, with_compute=True, rounds=2000)
     roof = {"bound": "mfma", "achieved": ach, "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s", "frac": ach / PEAK_FP32_MFMA_TFLOPS,
             # two rocprofv3 --pmc runs of this workload (FETCH_SIZE x 2.00 by a copy of known size, WRITE_SIZE x 1.00):
-            # 10.6 MB read + 5.5 MB written per launch of lstm_backward_local<4, 8, 1, false>; algorithmic 12.5 MB
-            "traffic": 16.1e6, "traffic_source": "profiles/lstm_c1_backward_kernel_stats.md",
+            # 10.3 MB read + 5.4 MB written per launch of lstm_backward_local<4, 8, 1, false>; algorithmic 12.5 MB
+            "traffic": 15.7e6, "traffic_source": "profiles/lstm_c1_backward_kernel_stats.md",
             "kernel": dom, "us_per_step": us_per_step, "latency_floor_us_per_step": hop_us,
             "frac_of_latency_floor": hop_us / us_per_step,
             "note": "latency-bound recursion (T sequential steps, four jobs of one sequence, each on one XCD): `frac` is against the "
