@@ -551,7 +551,9 @@ __device__ __forceinline__ void backward_job(const ChainParams &p, const LocalJo
                 if (p.sum_bias) {
                     const double c64 = c, earlier64 = c_earlier, d_ig = d[1], d_fg = d[2], d_og = d[3];
                     sums[0] += (double)d[0]; sums[1] += d_ig; sums[2] += d_fg; sums[3] += d_og;
-                    sums[4] += earlier64 * d_ig; sums[5] += earlier64 * d_fg; sums[6] += c64 * d_og;
+                    sums[6] += c64 * d_og;
+                    // (a job's last step has no earlier state: a zero in its place would be NaN with a delta that is not finite)
+                    if (step - held + ahead + 1 < end_step) { sums[4] += earlier64 * d_ig; sums[5] += earlier64 * d_fg; }
                 }
             }
             if (step > part.first) {

@@ -394,13 +394,16 @@ __global__ __launch_bounds__(solo_threads(NW)) __attribute__((amdgpu_waves_per_e
             solo_store4<CELLS>(r_ce, o, last, t * row, value(4));
             solo_store4<CELLS>(r_herr, o, last, t * row, value(5));
             if (!p.sum_bias || !on) return;
-            // the load wave is two steps ahead of this one; behind the last step the cell states it hands over are zeros
+            // the load wave is two steps ahead of this one; the last step has no earlier state, and a zero in its place would be NaN with a
+            // delta that is not finite
+            const bool has_earlier = sb + step + 1 < se;
             const f32x4 c = lds_load4<CELLS>(&cells_ahead[step & 3][j][cells]), earlier = lds_load4<CELLS>(&cells_ahead[(step + 1) & 3][j][cells]);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const double ig = d_ig[q], fg = d_fg[q], og = d_og[q], before = earlier[q];
                 sums[0][q] += (double)d_ni[q]; sums[1][q] += ig; sums[2][q] += fg; sums[3][q] += og;
-                sums[4][q] += before * ig; sums[5][q] += before * fg; sums[6][q] += (double)c[q] * og;
+                sums[6][q] += (double)c[q] * og;
+                if (has_earlier) { sums[4][q] += before * ig; sums[5][q] += before * fg; }
             }
         };
         __syncthreads();

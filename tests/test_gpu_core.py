@@ -758,6 +758,43 @@ def test_lstm_small_gradients_of_a_whole_backward_call(L, bidir, lengths):
     layer.close()
 
 
+@pytest.mark.parametrize("L,bidir,lengths", [
+    (3, False, [5, 2]), (6, True, [7, 7]), (50, False, [13] * 4), (128, True, [30, 8, 21, 30, 17]), (130, False, [9]), (200, True, [7, 7, 2, 5]),
+    (512, True, [29, 29, 3, 3, 3, 2, 2, 1, 1, 1]), (300, False, [12, 4, 12]), (130, True, [9 - i % 3 for i in range(70)])])
+def test_lstm_peephole_gradients_where_the_last_delta_is_not_finite(L, bidir, lengths):
+    """The step a recursion ends with has no earlier cell state, so its delta is in no gradient of an input or forget gate's peephole, whatever
+    it is; those gradients are what they are with a finite delta there, bit for bit."""
+    import torch
+
+    print("lstm last delta", L, bidir, lengths, flush=True)
+    capi = PC.pkg().capi
+    S, T, P, dirs = len(lengths), max(lengths), 5, 2 if bidir else 1
+    H = L // dirs
+    gen = torch.Generator(device="cuda").manual_seed(L + S)
+    W = torch.empty(int(capi.lib().cnt_lstm_weight_count(P, L, int(bidir))), device="cuda").uniform_(-0.2, 0.2, generator=gen)
+    pat = PC.dev(PC.make_pat_types(lengths, T))
+    valid = (pat != 0).reshape(-1, 1)
+    layer = capi.Lstm(P, L, bidir, S, T, 0.7)
+    x = (torch.randn(T * S, P, device="cuda", generator=gen) * valid).reshape(-1)
+    errors = torch.randn(T * S, L, device="cuda", generator=gen) * valid
+    out, prev = torch.zeros(T * S * L, device="cuda"), torch.zeros(T * S * P, device="cuda")
+    got = []
+    for value in (1.0, float("nan")):
+        layer.load_sequences(pat, T, min(lengths))
+        layer.forward(W, x, out)
+        e, dW = errors.clone(), torch.full_like(W, 7.0)
+        e[:S, :H] = value
+        if bidir:
+            e[(T - 1) * S:, H:][valid[(T - 1) * S:, 0]] = value
+        layer.backward(W, x, out, e.reshape(-1), prev, dW)
+        layer.check()
+        got.append(dW[4 * P * L + 4 * L + 4 * L * H:].clone())
+        bias = dW[4 * P * L:4 * P * L + 4 * L]
+        assert bool(bias.isfinite().all()) == (value == 1.0)
+    assert bool(got[0].isfinite().all()) and torch.equal(got[0][:2 * L], got[1][:2 * L])
+    layer.close()
+
+
 @pytest.mark.parametrize("P,L,bidir,lengths", [
     (61, 512, True, [130, 125] + [20] * 18), (382, 300, True, [513] + [70] * 9), (40, 256, False, [700, 1, 1, 1]), (128, 400, True, [65] * 30 + [17] * 8)])
 def test_lstm_products_of_a_fraction_with_padding(P, L, bidir, lengths):
