@@ -436,6 +436,12 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in, DirectGroup *group)
                 "gemm: split-K needs the atomic epilogue");
     CNT_REQUIRE(args.epilogue != EPI_STORE_DELTA || (args.splitk == 1 && args.prob[0].aux_in != nullptr),
                 "gemm: the delta epilogue needs the preceding layer's outputs and no split");
+    CNT_REQUIRE((args.epilogue != EPI_BIAS_ACT && args.epilogue != EPI_BIAS_ACT_SKIP && args.epilogue != EPI_CONTEXT) || args.a_kcontig,
+                "gemm: the forward epilogues are for two k-contiguous operands");
+    CNT_REQUIRE((args.epilogue != EPI_BIAS_ACT_SKIP || args.masked) && (args.epilogue != EPI_CONTEXT || !args.masked),
+                "gemm: an epilogue that goes by the pattern types has one loader");
+    CNT_REQUIRE(args.epilogue != EPI_STORE_DELTA || (!args.a_kcontig && args.b_kcontig),
+                "gemm: the delta epilogue is for a row-contiguous A and a k-contiguous B");
     CNT_REQUIRE(args.epilogue != EPI_FAN || (gemm_fan_supported(args) && args.splitk == 1),
                 "gemm: the fan epilogue exists for one unsplit problem with 16-byte row-contiguous A and k-contiguous B");
     CNT_REQUIRE(args.epilogue != EPI_PARTIAL || (args.splitk >= 1 && args.partial_stride > 0 && args.partial),

@@ -443,6 +443,17 @@ __device__ __forceinline__ f32x16 plain_sums(const ARGS &args, const PROBLEM &pb
     return acc;
 }
 
+// step(the activation function as a constant)
+template <typename STEP>
+__device__ __forceinline__ void by_activation(int act, STEP &&step) {
+    switch (act) {
+        case ACT_TANH: step(std::integral_constant<int, ACT_TANH>()); break;
+        case ACT_LOGISTIC: step(std::integral_constant<int, ACT_LOGISTIC>()); break;
+        case ACT_RELU: step(std::integral_constant<int, ACT_RELU>()); break;
+        default: step(std::integral_constant<int, ACT_IDENTITY>()); break;
+    }
+}
+
 // VA, VB: vector widths of the masked loader, 16-byte alignment included; unmasked: 4 where the operand's lines are a
 // multiple of four long, at any alignment, else 1.
 // MASKED selects the time-shifted, padding-masked B loader at compile time: its per-element predication is a lot
@@ -714,25 +725,6 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (VA * VB
             }
         }
     }
-    if (args.epilogue == EPI_PARTIAL) {
-        // this split's partial product, m x n column-major without padding, after those of the problems before it
-        float *__restrict__ P = args.partial + (size_t)split_id * args.partial_stride +
-                                (size_t)prob_id * args.m * args.n;
-#pragma unroll
-        for (int i = 0; i < NBM; ++i) {
-            const int m = m0 + wm * WM + i * 32 + frag_row;
-            if (m >= args.m) continue;
-#pragma unroll
-            for (int j = 0; j < NBN; ++j) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int n = n0 + wn * WN + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-                    if (n < args.n) P[(size_t)n * args.m + m] = acc[i][j][r];
-                }
-            }
-        }
-        return;
-    }
     if (FAN) {
         // All loads of a 32 x 32 tile's sixteen values per lane are issued before anything is stored: the compiler
         // cannot know that the buffers do not overlap and would otherwise wait for memory once per value.
@@ -774,53 +766,124 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (VA * VB
         }
         return;
     }
-    const float *const old = args.epilogue == EPI_STORE_DELTA || args.epilogue == EPI_CONTEXT ? pb.aux_in
-                                        : args.epilogue == EPI_ADD ? C : nullptr;
+    // The other epilogues: what becomes of the sums first, in registers, one kind of step after the other, then the stores.  Every step is
+    // straight code over a wave's sums with the choices outside.  With a switch and the edges' conditions per sum the kernels were 7 to
+    // 28 thousand instructions, and what bounded a tile's end was fetching them: 1024 x 32000 x 128 103 -> 58 us (128 x 128 tiles, four
+    // waves), 79 -> 72 (64 x 64), 1936 x 6000 x 256 51 -> 42, 1024 x 12000 x 1024 161 -> 151, 512 x 6000 x 512 33 -> 31; the feed-forward
+    // model's pass 2018 -> 1924, mixture output 171 -> 158.
+    const int epilogue = args.epilogue;
+    int ldc = args.ldc;
+    if (epilogue == EPI_PARTIAL) {
+        // this split's partial product, m x n column-major without padding, after those of the problems before it
+        C = args.partial + (size_t)split_id * args.partial_stride + (size_t)prob_id * args.m * args.n;
+        ldc = args.m;
+    }
+    const int wave_m = m0 + wm * WM, wave_n = wn * WN;  // the wave's first row, its first column inside the tile
+    auto in_tile = [&](int j, int r) __attribute__((always_inline)) { return wave_n + 32 * j + 8 * (r >> 2) + 4 * half + (r & 3); };
+    // the column of C for a column of the tile (clamped into the matrix)
+    auto column = [&](int at) __attribute__((always_inline)) { return listed ? col_of[at] : min(n0 + at, args.n - 1); };
+    auto all_sums = [&](auto &&step) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NBM; ++i) {
-        const int m = m0 + wm * WM + i * 32 + frag_row;
-        if (m >= args.m) continue;
-        float bterm = 0.0f;
-        if (args.epilogue == EPI_BIAS_ACT || args.epilogue == EPI_BIAS_ACT_SKIP)
-            bterm = args.bias_scale * pb.bias_vec[m];
+        for (int i = 0; i < NBM; ++i)
 #pragma unroll
-        for (int j = 0; j < NBN; ++j) {
-            // What the sums meet in memory is requested for sixteen of them at a time: the compiler cannot know that it does not
-            // overlap the output and would wait for one load per sum (a dense layer's deltas in the epilogue of the product above
-            // it: the feed-forward model's pass, four such products, 2260 -> 2183 us).
-            float met[16];
-            if (old) {
+            for (int j = 0; j < NBN; ++j)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int in_tile = wn * WN + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-                    const int n = listed ? col_of[in_tile] : min(n0 + in_tile, args.n - 1);
-                    met[r] = old[(size_t)n * args.ldc + m];
+                for (int r = 0; r < 16; ++r) acc[i][j][r] = step(acc[i][j][r], i, j, r);
+    };
+    if (listed && n0 + BN > listed_n)  // behind the listed columns there are zeros
+        all_sums([&](float v, int, int j, int r) { return n0 + in_tile(j, r) < listed_n ? v : 0.0f; });
+    // (which operand kinds come with which epilogue: gemm_launch)
+    constexpr bool FORWARD = AK && BK_, BACKWARD = !AK && BK_;
+    if (FORWARD && (epilogue == EPI_BIAS_ACT || epilogue == EPI_BIAS_ACT_SKIP)) {
+#pragma unroll
+        for (int i = 0; i < NBM; ++i) {
+            const float bterm = args.bias_scale * pb.bias_vec[min(wave_m + 32 * i + frag_row, args.m - 1)];
+#pragma unroll
+            for (int j = 0; j < NBN; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][j][r] += bterm;
+        }
+        by_activation(args.act, [&](auto act) { all_sums([&](float v, int, int, int) { return act_fn(decltype(act)::value, v); }); });
+    } else if ((BACKWARD && epilogue == EPI_STORE_DELTA) || (FORWARD && !MASKED && epilogue == EPI_CONTEXT) || epilogue == EPI_ADD) {
+        // What the sums meet in memory is requested for sixteen of them at a time: the compiler cannot know that it does not
+        // overlap the output and would wait for one load per sum (a dense layer's deltas in the epilogue of the product above
+        // it: the feed-forward model's pass, four such products, 2260 -> 2183 us).
+        const float *const old = epilogue == EPI_ADD ? C : pb.aux_in;
+#pragma unroll
+        for (int j = 0; j < NBN; ++j)
+#pragma unroll
+            for (int i = 0; i < NBM; ++i) {
+                const int m = min(wave_m + 32 * i + frag_row, args.m - 1);
+                float met[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) met[r] = old[(size_t)column(in_tile(j, r)) * ldc + m];
+                f32x16 &v = acc[i][j];
+                if (epilogue == EPI_ADD) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) v[r] = met[r] + v[r];
+                } else if constexpr (BACKWARD) {
+                    by_activation(args.act, [&](auto act) {
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) v[r] *= act_deriv(decltype(act)::value, met[r]);
+                    });
+                } else if constexpr (FORWARD && !MASKED) {
+                    bool valid[16];
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) valid[r] = args.pat[column(in_tile(j, r))] != 0;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const float th = valid[r] ? tanh_act(v[r]) : 0.0f;
+                        met[r] = valid[r] ? met[r] + th : 0.0f;
+                        v[r] = th;
+                    }
+                    if (pb.aux_out)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            const int n = n0 + in_tile(j, r);
+                            if (n < args.n && wave_m + 32 * i + frag_row < args.m) pb.aux_out[(size_t)n * ldc + m] = v[r];
+                        }
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) v[r] = met[r];
                 }
             }
+    }
+    // A wave whose sums all lie inside the matrix stores them through one offset per lane beside an address per sum that is uniform.
+    if (epilogue != EPI_ATOMIC && epilogue != EPI_BIAS_ACT_SKIP && !listed && wave_m + WM <= args.m && n0 + wave_n + WN <= args.n) {
+        const unsigned mine = ((unsigned)(4 * half) * (unsigned)ldc + (unsigned)frag_row) * (unsigned)sizeof(float);
+        char *at = reinterpret_cast<char *>(C + (size_t)(n0 + wave_n) * ldc + wave_m);
+        const size_t line = (size_t)ldc * sizeof(float);
+#pragma unroll
+        for (int j = 0; j < NBN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int in_tile = wn * WN + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3), n = n0 + in_tile;
-                if (n >= args.n) continue;
-                const size_t idx = (size_t)(listed ? col_of[in_tile] : n) * args.ldc + m;
-                float *dst = C + idx;
-                const float v = n < listed_n ? acc[i][j][r] : 0.0f;
-                switch (args.epilogue) {
-                    case EPI_STORE: *dst = v; break;
-                    case EPI_STORE_DELTA: *dst = v * act_deriv(args.act, met[r]); break;
-                    case EPI_ADD: *dst = met[r] + v; break;
-                    case EPI_ATOMIC: atomicAdd(dst, v); break;
-
-                    case EPI_BIAS_ACT: *dst = act_fn(args.act, v + bterm); break;
-                    case EPI_BIAS_ACT_SKIP:
-                        if (args.pat[n] != 0) *dst = act_fn(args.act, v + bterm);
-                        break;
-                    default: {  // EPI_CONTEXT
-                        const bool valid = args.pat[n] != 0;
-                        const float th = valid ? tanh_act(v) : 0.0f;
-                        if (pb.aux_out) pb.aux_out[idx] = th;
-                        *dst = valid ? met[r] + th : 0.0f;
-                    } break;
-                }
+#pragma unroll
+                for (int i = 0; i < NBM; ++i) *reinterpret_cast<float *>(at + mine + 128 * i) = acc[i][j][r];
+                at += (r & 3) == 3 ? 5 * line : line;
+                asm volatile("" : "+s"(at));  // (one address that moves along, not one per column)
+            }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < NBN; ++j) {
+        bool keep[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            keep[r] = n0 + in_tile(j, r) < args.n;
+            if constexpr (FORWARD && MASKED)
+                if (epilogue == EPI_BIAS_ACT_SKIP) keep[r] = keep[r] && args.pat[column(in_tile(j, r))] != 0;
+        }
+#pragma unroll
+        for (int i = 0; i < NBM; ++i) {
+            const int m = wave_m + 32 * i + frag_row;
+            if (m >= args.m) continue;
+            if (epilogue == EPI_ATOMIC) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (keep[r]) atomicAdd(C + (size_t)column(in_tile(j, r)) * ldc + m, acc[i][j][r]);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (keep[r]) C[(size_t)column(in_tile(j, r)) * ldc + m] = acc[i][j][r];
             }
         }
     }
