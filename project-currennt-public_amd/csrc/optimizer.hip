@@ -35,51 +35,109 @@ struct OptArgs {
 };
 
 __device__ __forceinline__ bool bad(float g) { return isnan(g) || isinf(g); }
+// (the options that keep statistics, and how many floats of them per weight)
+__device__ __forceinline__ bool with_statistics(const OptArgs &a) { return a.option == 1 || a.option == 3 || a.option == 5; }
 
-__device__ __forceinline__ float adjust_one(const OptArgs &a, size_t i, float g) {
+// The gradient that the update uses; s: the weight's statistics (Adam: m and v).
+__device__ __forceinline__ float adjust_one(const OptArgs &a, float g, float mask, float (&s)[2]) {
     if (a.option == 2) return g / a.frac_length;
-    if (a.option != 1 && a.option != 3 && a.option != 5) return g;
+    if (!with_statistics(a)) return g;
     if (bad(g)) g = 0.0f;
-    if (a.mask && a.mask[i] < 1.0f) return g;
+    if (mask < 1.0f) return g;
     const float ave = g / a.frac_length;
     if (a.option == 5) {
-        const float m = (float)(a.stats[2 * i] * kBeta1 + ave * (1 - kBeta1));
-        const float v = (float)(a.stats[2 * i + 1] * kBeta2 + (double)(ave * ave) * (1 - kBeta2));
-        a.stats[2 * i] = m;
-        a.stats[2 * i + 1] = v;
+        const float m = (float)(s[0] * kBeta1 + ave * (1 - kBeta1));
+        const float v = (float)(s[1] * kBeta2 + (double)(ave * ave) * (1 - kBeta2));
+        s[0] = m;
+        s[1] = v;
         const float b1 = a.accum_dev ? a.accum_dev[0] : a.beta1_accum, b2 = a.accum_dev ? a.accum_dev[1] : a.beta2_accum;
         const float mh = m / (1 - b1);
         const float vh = v / (1 - b2);
         return (float)(mh / (sqrtf(vh) + kEps));
     }
-    const float acc = a.stats[i] + (ave * ave);
-    a.stats[i] = acc;
+    const float acc = s[0] + (ave * ave);
+    s[0] = acc;
     return a.option == 1 ? ave / sqrtf(acc) : g;
 }
 
-__device__ __forceinline__ float update_one(const OptArgs &a, size_t i, float g) {
+__device__ __forceinline__ float update_one(const OptArgs &a, float g, float mask, float &delta, float &w) {
     if (bad(g)) g = 0.0f;
-    const float delta = a.momentum * a.deltas[i] - a.learning_rate * g;
-    a.deltas[i] = delta;
-    const float w = a.weights[i] + delta;
-    a.weights[i] = a.mask ? w * a.mask[i] : w;
+    delta = a.momentum * delta - a.learning_rate * g;
+    w = w + delta;
+    if (a.mask) w = w * mask;
     return g;
 }
 
-// MODE 0 accumulate, 1 adjust, 2 update, 3 all three in one pass
+// N neighbouring floats, at any address that a float may have
+template <int N>
+__device__ __forceinline__ void fetch(const float *p, float (&v)[N]) {
+    typedef float vec __attribute__((ext_vector_type(N), aligned(4)));
+    const vec x = *reinterpret_cast<const vec *>(p);
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] = x[q];
+}
+template <int N>
+__device__ __forceinline__ void put(float *p, const float (&v)[N]) {
+    typedef float vec __attribute__((ext_vector_type(N), aligned(4)));
+    vec x;
+#pragma unroll
+    for (int q = 0; q < N; ++q) x[q] = v[q];
+    *reinterpret_cast<vec *>(p) = x;
+}
+
+// MODE 0 accumulate, 1 adjust, 2 update, 3 all three in one pass; N weights from i on: everything is asked for before anything is
+// worked out, so that a wave has up to six accesses in flight.
+template <int MODE, int N>
+__device__ __forceinline__ void optimize(const OptArgs &a, size_t i) {
+    constexpr bool LAYER = MODE == 0 || MODE == 3, ADJUST = MODE == 1 || MODE == 3, UPDATE = MODE == 2 || MODE == 3;
+    float g[N], cur[N], mask[N], delta[N], w[N], s[N * 2];
+    const bool moments = ADJUST && a.option == 5, squares = ADJUST && (a.option == 1 || a.option == 3);
+    if (LAYER) fetch<N>(a.layer_updates + i, g);
+    if (!LAYER || a.add) fetch<N>(a.cur + i, cur);
+    if (moments) fetch<N * 2>(a.stats + 2 * i, s);
+    if (squares) {
+        float t[N];
+        fetch<N>(a.stats + i, t);
+#pragma unroll
+        for (int q = 0; q < N; ++q) s[2 * q] = t[q];
+    }
+    if (UPDATE) { fetch<N>(a.deltas + i, delta); fetch<N>(a.weights + i, w); }
+    if (a.mask) fetch<N>(a.mask + i, mask);
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        float x = !LAYER ? cur[q] : a.add ? g[q] + cur[q] : g[q];
+        const float m = a.mask ? mask[q] : 1.0f;
+        if (ADJUST) {
+            float own[2] = {s[2 * q], s[2 * q + 1]};
+            x = adjust_one(a, x, m, own);
+            s[2 * q] = own[0];
+            s[2 * q + 1] = own[1];
+        }
+        if (UPDATE) x = update_one(a, x, m, delta[q], w[q]);
+        cur[q] = x;
+    }
+    if (moments) put<N * 2>(a.stats + 2 * i, s);
+    if (squares) {
+        float t[N];
+#pragma unroll
+        for (int q = 0; q < N; ++q) t[q] = s[2 * q];
+        put<N>(a.stats + i, t);
+    }
+    if (UPDATE) { put<N>(a.deltas + i, delta); put<N>(a.weights + i, w); }
+    put<N>(a.cur + i, cur);
+}
+
+// kAtOnce weights per thread; those that are left over at the end go one by one.  What bounds it is memory: with a weight per thread
+// and so four-byte accesses a step in a training pass took 44.8 us (Adam, 4.8 million weights) and 21.0 (steepest descent, 3.0 million), in
+// fours 38.1 and 19.4; one step after another 5.9 to 6.7 TB/s.  Two per thread are 0 to 7 % slower, eight 3 to 24 %.
+constexpr int kAtOnce = 4;
 template <int MODE>
 __global__ __launch_bounds__(256) void optimizer_kernel(const OptArgs a) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    const size_t first = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
     if (a.veto && *a.veto != 0) return;
-    for (; i < a.n; i += stride) {
-        float g;
-        if (MODE == 0 || MODE == 3) g = a.add ? a.layer_updates[i] + a.cur[i] : a.layer_updates[i];
-        else g = a.cur[i];
-        if (MODE == 1 || MODE == 3) g = adjust_one(a, i, g);
-        if (MODE == 2 || MODE == 3) g = update_one(a, i, g);
-        a.cur[i] = g;
-    }
+    const size_t whole = a.n / kAtOnce;
+    for (size_t i = first; i < whole; i += stride) optimize<MODE, kAtOnce>(a, i * kAtOnce);
+    if (first < a.n % kAtOnce) optimize<MODE, 1>(a, whole * kAtOnce + first);
 }
 
 // Adam's bias-correction products beta1^t, beta2^t kept in device memory, advanced in stream order in front of a step
@@ -91,7 +149,7 @@ __global__ void adam_advance_kernel(float *accum, const int *veto) {
 }
 
 int blocks_for(size_t n) {
-    size_t b = (n + 255) / 256;
+    size_t b = (n / kAtOnce + 255) / 256;
     if (b > 8192) b = 8192;
     return (int)(b < 1 ? 1 : b);
 }

@@ -97,3 +97,42 @@ def test_negative_learning_rate_skips_update_and_bad_arguments():
         capi.opt_adjust_gradient(5, g, None, None, 1.0, 0.9, 0.999)   # Adam without a statistics buffer
     with pytest.raises(RuntimeError):
         capi.opt_adjust_gradient(9, g, d, None, 1.0)
+
+
+@pytest.mark.parametrize("option,with_mask,add", [(0, False, False), (1, True, True), (2, False, True), (3, True, False), (5, True, False), (5, False, True)])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 7, 1023, 1026])
+def test_a_weight_is_updated_the_same_wherever_it_stands(option, with_mask, add, n):
+    # Several weights per thread, and the last ones by themselves: every array begins at another place behind an aligned address, and the
+    # result is bit for bit that of the same weights at the front of arrays of one more vector, and nothing beside an array changes.
+    import torch
+
+    capi = PC.pkg().capi
+    rng = np.random.default_rng(n)
+    per = {"w": 1, "g": 1, "cur": 1, "stats": 2 if option == 5 else 1, "deltas": 1, "mask": 1}
+    host = {k: np.abs(rng.standard_normal(n * p)).astype(np.float32) for k, p in per.items()}
+    host["mask"] = np.where(rng.random(n) < 0.3, 0.0, 1.0).astype(np.float32)
+    host["g"][n // 2] = np.nan
+    results = []
+    for shifted in (False, True):
+        whole = {}
+        view = {}
+        for at, (k, p) in enumerate(per.items()):
+            skip, behind = (1 + at % 3, 8) if shifted else (0, 8 + 3 * n)  # (the second form has a full vector behind every weight)
+            whole[k] = torch.full((skip + n * p + behind,), 7.0, device="cuda")
+            whole[k][skip:skip + n * p] = torch.from_numpy(host[k]).cuda()
+            view[k] = whole[k][skip:skip + (n * p if shifted else (n + 4 - n % 4) * p)]
+        args = (option, view["cur"], view["stats"], view["mask"] if with_mask else None, 41.0, 0.9, 0.999)
+        if add:  # the three calls, the first of them accumulating; else the one that does all
+            capi.opt_accumulate(view["g"], view["cur"], True)
+            capi.opt_adjust_gradient(*args)
+            capi.opt_update_weights(view["w"], view["cur"], view["deltas"], args[3], 3e-3, 0.9)
+        else:
+            capi.opt_step(option, view["w"], view["g"], view["cur"], view["stats"], view["deltas"], args[3], 41.0, 0.9, 0.999, 3e-3, 0.9)
+        torch.cuda.synchronize()
+        if shifted:
+            for k, p in per.items():
+                skip = whole[k].numel() - n * p - 8
+                assert torch.all(whole[k][:skip] == 7.0) and torch.all(whole[k][skip + n * p:] == 7.0), k
+        results.append({k: view[k][:n * p].cpu().numpy().view(np.int32) for k, p in per.items()})
+    for k in per:
+        assert np.array_equal(results[0][k], results[1][k]), k
