@@ -127,17 +127,14 @@ __device__ __forceinline__ void optimize(const OptArgs &a, size_t i) {
     put<N>(a.cur + i, cur);
 }
 
-// kAtOnce weights per thread; those that are left over at the end go one by one.  What bounds it is memory: with a weight per thread
-// and so four-byte accesses a step in a training pass took 44.8 us (Adam, 4.8 million weights) and 21.0 (steepest descent, 3.0 million), in
-// fours 38.1 and 19.4; one step after another 5.9 to 6.7 TB/s.  Two per thread are 0 to 7 % slower, eight 3 to 24 %.
-constexpr int kAtOnce = 4;
-template <int MODE>
+// N weights per thread; those that are left over at the end go one by one.
+template <int MODE, int N>
 __global__ __launch_bounds__(256) void optimizer_kernel(const OptArgs a) {
     const size_t first = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
     if (a.veto && *a.veto != 0) return;
-    const size_t whole = a.n / kAtOnce;
-    for (size_t i = first; i < whole; i += stride) optimize<MODE, kAtOnce>(a, i * kAtOnce);
-    if (first < a.n % kAtOnce) optimize<MODE, 1>(a, whole * kAtOnce + first);
+    const size_t whole = a.n / N;
+    for (size_t i = first; i < whole; i += stride) optimize<MODE, N>(a, i * N);
+    if (first < a.n % N) optimize<MODE, 1>(a, whole * N + first);
 }
 
 // Adam's bias-correction products beta1^t, beta2^t kept in device memory, advanced in stream order in front of a step
@@ -148,10 +145,19 @@ __global__ void adam_advance_kernel(float *accum, const int *veto) {
     accum[1] = (float)(accum[1] * kBeta2);
 }
 
-int blocks_for(size_t n) {
-    size_t b = (n / kAtOnce + 255) / 256;
-    if (b > 8192) b = 8192;
-    return (int)(b < 1 ? 1 : b);
+// One weight per thread while a full grid holds them, four beyond that.  What bounds a step is memory: with four-byte accesses and a
+// second round of the grid a step in a training pass took 44.8 us (Adam, 4.8 million weights) and 21.0 (steepest descent, 3.0 million),
+// in fours 38.1 and 19.4; one step after another 5.9 to 6.7 TB/s (two per thread 0 to 7 % less, eight 3 to 24 %).  Below the line
+// the shorter threads finish first: Adam, 0.8 million 7.2 us and 8.6 in fours, 40 thousand in a small network's pass 3.2 and 3.6.
+constexpr size_t kMostBlocks = 8192, kFours = kMostBlocks * 256;
+template <int MODE>
+int launch_optimizer(hipStream_t stream, const OptArgs &a) {
+    const bool fours = a.n > kFours;
+    const size_t blocks = ((fours ? a.n / 4 : a.n) + 255) / 256;
+    void (*const kernel)(const OptArgs) = fours ? optimizer_kernel<MODE, 4> : optimizer_kernel<MODE, 1>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(blocks, kMostBlocks)), dim3(256), 0, stream, a);
+    CNT_HIP(hipGetLastError());
+    return CNT_OK;
 }
 
 bool known_option(int o) { return o == 0 || o == 1 || o == 2 || o == 3 || o == 4 || o == 5; }
@@ -168,9 +174,7 @@ int cnt_opt_accumulate(void *stream, long n, const float *layer_updates, float *
     OptArgs a = {};
     a.n = (size_t)n; a.layer_updates = layer_updates; a.cur = cur_updates; a.add = add;
     ProfileScope prof(static_cast<hipStream_t>(stream), "opt_accumulate");
-    hipLaunchKernelGGL(optimizer_kernel<0>, dim3(blocks_for(a.n)), dim3(256), 0, static_cast<hipStream_t>(stream), a);
-    CNT_HIP(hipGetLastError());
-    return CNT_OK;
+    return launch_optimizer<0>(static_cast<hipStream_t>(stream), a);
 }
 
 int cnt_opt_adjust_gradient(void *stream, int option, long n, float *cur_updates, float *stats, const float *mask,
@@ -185,9 +189,7 @@ int cnt_opt_adjust_gradient(void *stream, int option, long n, float *cur_updates
     a.n = (size_t)n; a.cur = cur_updates; a.stats = stats; a.mask = mask; a.option = option;
     a.frac_length = frac_length; a.beta1_accum = beta1_accum; a.beta2_accum = beta2_accum;
     ProfileScope prof(static_cast<hipStream_t>(stream), "opt_adjust_gradient");
-    hipLaunchKernelGGL(optimizer_kernel<1>, dim3(blocks_for(a.n)), dim3(256), 0, static_cast<hipStream_t>(stream), a);
-    CNT_HIP(hipGetLastError());
-    return CNT_OK;
+    return launch_optimizer<1>(static_cast<hipStream_t>(stream), a);
 }
 
 int cnt_opt_update_weights(void *stream, long n, float *weights, float *cur_updates, float *weight_deltas,
@@ -200,9 +202,7 @@ int cnt_opt_update_weights(void *stream, long n, float *weights, float *cur_upda
     a.n = (size_t)n; a.cur = cur_updates; a.deltas = weight_deltas; a.weights = weights; a.mask = mask;
     a.learning_rate = learning_rate; a.momentum = momentum;
     ProfileScope prof(static_cast<hipStream_t>(stream), "opt_update_weights");
-    hipLaunchKernelGGL(optimizer_kernel<2>, dim3(blocks_for(a.n)), dim3(256), 0, static_cast<hipStream_t>(stream), a);
-    CNT_HIP(hipGetLastError());
-    return CNT_OK;
+    return launch_optimizer<2>(static_cast<hipStream_t>(stream), a);
 }
 
 int cnt_opt_step(void *stream, int option, long n, float *weights, const float *layer_updates, float *cur_updates,
@@ -237,9 +237,7 @@ extern "C++" int cnt::opt_step_guarded(hipStream_t stream, int option, long n, f
     a.veto = veto;
     a.accum_dev = accum_dev;
     ProfileScope prof(stream, "opt_step");
-    hipLaunchKernelGGL(optimizer_kernel<3>, dim3(blocks_for(a.n)), dim3(256), 0, stream, a);
-    CNT_HIP(hipGetLastError());
-    return CNT_OK;
+    return launch_optimizer<3>(stream, a);
 }
 
 float cnt_opt_next_beta_accum(float accum, int which) { return (float)(accum * (which == 1 ? cnt::kBeta1 : cnt::kBeta2)); }

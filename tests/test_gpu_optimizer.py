@@ -100,10 +100,10 @@ def test_negative_learning_rate_skips_update_and_bad_arguments():
 
 
 @pytest.mark.parametrize("option,with_mask,add", [(0, False, False), (1, True, True), (2, False, True), (3, True, False), (5, True, False), (5, False, True)])
-@pytest.mark.parametrize("n", [1, 3, 4, 5, 7, 1023, 1026])
+@pytest.mark.parametrize("n", [1, 5, 1023, 2 ** 21 - 2, 2 ** 21 + 1, 2 ** 21 + 4, 2 ** 21 + 1027])
 def test_a_weight_is_updated_the_same_wherever_it_stands(option, with_mask, add, n):
-    # Several weights per thread, and the last ones by themselves: every array begins at another place behind an aligned address, and the
-    # result is bit for bit that of the same weights at the front of arrays of one more vector, and nothing beside an array changes.
+    # A few weights go one per thread, more than 2^21 in fours and the last ones by themselves: every array begins at another place behind
+    # an aligned address, and the result is bit for bit that of the same weights, a part at a time, one by one; nothing beside an array changes.
     import torch
 
     capi = PC.pkg().capi
@@ -117,17 +117,21 @@ def test_a_weight_is_updated_the_same_wherever_it_stands(option, with_mask, add,
         whole = {}
         view = {}
         for at, (k, p) in enumerate(per.items()):
-            skip, behind = (1 + at % 3, 8) if shifted else (0, 8 + 3 * n)  # (the second form has a full vector behind every weight)
-            whole[k] = torch.full((skip + n * p + behind,), 7.0, device="cuda")
+            skip = 1 + at % 3 if shifted else 0
+            whole[k] = torch.full((skip + n * p + 8,), 7.0, device="cuda")
             whole[k][skip:skip + n * p] = torch.from_numpy(host[k]).cuda()
-            view[k] = whole[k][skip:skip + (n * p if shifted else (n + 4 - n % 4) * p)]
-        args = (option, view["cur"], view["stats"], view["mask"] if with_mask else None, 41.0, 0.9, 0.999)
-        if add:  # the three calls, the first of them accumulating; else the one that does all
-            capi.opt_accumulate(view["g"], view["cur"], True)
-            capi.opt_adjust_gradient(*args)
-            capi.opt_update_weights(view["w"], view["cur"], view["deltas"], args[3], 3e-3, 0.9)
-        else:
-            capi.opt_step(option, view["w"], view["g"], view["cur"], view["stats"], view["deltas"], args[3], 41.0, 0.9, 0.999, 3e-3, 0.9)
+            view[k] = whole[k][skip:skip + n * p]
+        for part in range(1 if shifted else 3):
+            cut = n if shifted else (n + 2) // 3
+            sub = {k: v[part * cut * per[k]:(part + 1) * cut * per[k]] for k, v in view.items()}
+            if sub["w"].numel() == 0: continue
+            args = (option, sub["cur"], sub["stats"], sub["mask"] if with_mask else None, 41.0, 0.9, 0.999)
+            if add:  # the three calls, the first of them accumulating; else the one that does all
+                capi.opt_accumulate(sub["g"], sub["cur"], True)
+                capi.opt_adjust_gradient(*args)
+                capi.opt_update_weights(sub["w"], sub["cur"], sub["deltas"], args[3], 3e-3, 0.9)
+            else:
+                capi.opt_step(option, sub["w"], sub["g"], sub["cur"], sub["stats"], sub["deltas"], args[3], 41.0, 0.9, 0.999, 3e-3, 0.9)
         torch.cuda.synchronize()
         if shifted:
             for k, p in per.items():
