@@ -416,7 +416,7 @@ struct BlockForward {
 };
 bool wavenet_block_forward_supported(const cnt_cnn *cnn, int R, int K, int C);
 int wavenet_block_forward(hipStream_t stream, const cnt_cnn *cnn, int R, int K, int C, int N, const char *patTypes,
-                          const BlockForward &block);
+                          const BlockForward &block, int from, int to);
 // Error path of one WaveNet residual block in one launch (skip 1x1 layer, the skip layer in front of it, the 1x1
 // layer behind the gated unit, the gated unit): see wavenet_block_errors_kernel.
 bool wavenet_block_errors_supported(int R, int K);

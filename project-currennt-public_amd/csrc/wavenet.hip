@@ -1104,14 +1104,15 @@ extern "C++" bool cnt::wavenet_block_forward_supported(const cnt_cnn *cnn, int R
 }
 
 extern "C++" int cnt::wavenet_block_forward(hipStream_t stream, const cnt_cnn *cnn, int R, int K, int C, int N,
-                                            const char *patTypes, const BlockForward &b) {
+                                            const char *patTypes, const BlockForward &b, int from, int to) {
     CNT_REQUIRE(wavenet_block_forward_supported(cnn, R, K, C), "wavenet_block_forward: no kernel for this block");
-    CNT_REQUIRE(N > 0 && patTypes && b.x && b.conv_weights && b.out_weights && b.skip_weights && b.conv && b.gated &&
+    CNT_REQUIRE(N > 0 && from >= 0 && from < to && to <= N, "wavenet_block_forward: slots %d..%d of %d", from, to, N);
+    CNT_REQUIRE(patTypes && b.x && b.conv_weights && b.out_weights && b.skip_weights && b.conv && b.gated &&
                 b.out && b.sum && b.skip && (C == 0 || (b.ctx && b.ctx_weights && b.ctx_tanh)),
                 "wavenet_block_forward: null argument");
     const cnt_cnn_group &g = cnn->groups[0];
     BlockFwdArgs a = {};
-    a.N = N; a.K = K; a.C = C; a.pat = patTypes; a.x = b.x; a.ctx = b.ctx;
+    a.first = from; a.N = to; a.K = K; a.C = C; a.pat = patTypes; a.x = b.x; a.ctx = b.ctx;
     a.shift = g.dil * cnn->desc.S;
     a.conv_ld = (2 * g.hw + 1) * R;
     for (int tap = 0; tap < 2; ++tap) a.conv_w[tap] = b.conv_weights + (size_t)(g.col0 + g.hw + tap - 1) * R;
@@ -1138,7 +1139,7 @@ extern "C++" int cnt::wavenet_block_forward(hipStream_t stream, const cnt_cnn *c
     if (lds > 65536)
         CNT_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     ProfileScope prof(stream, "wavenet_block_forward");
-    hipLaunchKernelGGL(kernel, dim3((N + 16 * st - 1) / (16 * st)), dim3(4 * R), lds, stream, a);
+    hipLaunchKernelGGL(kernel, dim3((to - from + 16 * st - 1) / (16 * st)), dim3(4 * R), lds, stream, a);
     CNT_HIP(hipGetLastError());
     return CNT_OK;
 }

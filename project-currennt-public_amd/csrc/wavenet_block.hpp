@@ -10,13 +10,14 @@ namespace cnt {
 namespace {
 
 struct BlockFwdArgs {
-    int N, K, C;
+    int N, K, C;             // (N: the end of the launch's slots)
     int shift;               // the earlier tap reads slot n - shift, the later one slot n
     const char *pat;
     const float *x;          // R x N: the block's input, also the residual
     const float *ctx;        // C x N conditioning features
     const float *conv_w[2];  // weight of (filter 0, channel 0) of the earlier and of the later tap
     int conv_ld;             // filter d at + d * conv_ld
+    int first;               // the launch's first slot
     const float *conv_bias;
     const float *ctx_w;      // [2R][C]
     const float *out_w, *out_bias;    // [R][R]
@@ -76,7 +77,7 @@ __global__ __launch_bounds__(R * 4, 2) void wavenet_block_forward_kernel(const B
     constexpr int CB = (4 * CJ * NS + NT - 1) / NT;
     f32x4 x0[XF], x1[XF], xc[CB];
     char p1[XF], pc[CB], pl[ST];
-    const int n0 = blockIdx.x * NS;
+    const int n0 = a.first + blockIdx.x * NS;
     {
 #pragma unroll
         for (int q = 0; q < XF; ++q) {

@@ -1654,3 +1654,62 @@ def test_mixture_density_network_file():
     net.close()
     with pytest.raises(RuntimeError, match="mdn config"):
         capi.Network(json.dumps(doc), S, T)
+
+
+# either side of the line from which a stack of blocks runs as two halves of the samples, a middle that is no workgroup's edge, dilations that
+# reach from the later half to the earlier one's beginning and past it, one and several blocks, several sequences
+@pytest.mark.parametrize("R,K,nb,cycle,lengths", [(64, 64, 2, 2, [8192, 8100]), (64, 64, 2, 2, [8193, 8100]), (64, 32, 1, 1, [17000]),
+                                                  (48, 64, 3, 14, [7301, 7282, 7000]), (32, 64, 15, 15, [33001]), (64, 128, 4, 4, [21111])])
+def test_blocks_in_two_halves_of_the_samples(R, K, nb, cycle, lengths):
+    """Both ways give the same values bit for bit, in every layer: on the caller's stream alone, with the later half beside it, on another
+    stream of the caller's, and replayed from a graph between eager passes."""
+    import torch
+
+    print("block halves", R, K, nb, cycle, lengths, flush=True)
+    capi = PC.pkg().capi
+    Q, C, S, T = 64, 20, len(lengths), max(lengths)
+    N = S * T
+    pat, onehot, ctx, target, _ = WD.make(lengths, Q, C, upsample=20, seed=2)
+    doc = json.dumps(PC.pkg().specs.wavenet_network_doc(nb, Q, R, K, C, 1, cycle))
+    fraction = (PC.dev(pat), T, min(lengths), torch.zeros(N, device="cuda"), PC.dev(target))
+    ctx = PC.dev(ctx)
+    want = None
+    for overlap in (False, True):
+        net = capi.Network(doc, S, T, mdn_config=[1, 0, Q, 0, 1, -1], overlap=overlap)
+        net.randomize(7, 0.1)
+        net.set_context(ctx)
+        net.load_sequences(*fraction)
+        layers = [L for L in net.layers if L["outputs"] is not None]
+        values = lambda: [L["outputs"][: N * L["size"]].clone() for L in layers]
+        if not overlap:
+            net.forward()
+            want = values()
+            net.close()
+            continue
+
+        def same():
+            torch.cuda.synchronize()
+            for L, a, b in zip(layers, values(), want):
+                assert torch.equal(a.view(torch.int32), b.view(torch.int32)), L["name"]
+
+        def spoil():
+            for L in layers[1:]:
+                if L["type"] != layers[-1]["type"] and L["outputs"].data_ptr() != layers[-1]["outputs"].data_ptr():
+                    L["outputs"].zero_()  # (padding slots of some layers stay as they are: zeros, as in a new network)
+        net.forward()
+        same()
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            net.forward()
+        same()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            net.forward()
+        for _ in range(3):
+            spoil()
+            graph.replay()
+            same()
+            net.forward()
+            same()
+        net.close()
