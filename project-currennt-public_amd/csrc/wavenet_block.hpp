@@ -47,8 +47,9 @@ constexpr int block_forward_lds_words(int R, int st, int C) { return (3 * (R / 4
 // of one sample per lane) go back into the same layout with one 16-byte write for the next product.  A wave holds
 // channel c of the tanh half and channel R + c of the sigmoid half, so the gate needs no exchange.
 //
-// What bounds it: FP32 matrix issue and the stores of the seven activation buffers, about equally (64 residual, 128 skip
-// channels, 80 conditioning features, per sample: 78 kFLOP and 2.8 KB).
+// What bounds it: the chain of its phases.  64 residual, 128 skip channels, 80 conditioning features (per sample 78 kFLOP and 2.8 KB), 32 000
+// samples in one launch, 39 us: FP32 matrix instructions 20 (without seven eighths of the convolution's 32), the gate's arithmetic 5, the stores of the
+// activation buffers 2, the rest loads, barriers and the launch itself.
 template <int R, int ST>
 __global__ __launch_bounds__(R * 4, 2) void wavenet_block_forward_kernel(const BlockFwdArgs a) {
     constexpr int CJ = kBlockMaxContext / 16;
