@@ -55,9 +55,6 @@ int cnt_probe_activation(void *stream, int which, long n, const float *x, float 
  * along k) with 16-byte aligned operands.  plan[0]: edge of an output tile (32, 64 or 128), plan[1]: waves of a workgroup,
  * plan[2]: splits of k.  Needs no device. */
 int cnt_probe_gemm_plan(int m, int n, int k, int problems, int a_kcontig, int b_kcontig, int weight_gradient, int *plan);
-/* Test hook: cnt_matrix_product with two fp16 parts per value, as the recurrent and dense layers multiply (where the product is neither
- * of few blocks nor over fewer than 128 values of k). */
-int cnt_probe_product_of_halves(void *stream, float *C, int m, int n, int k, const float *A, int transA, const float *B, int transB);
 
 /* ---- helpers::Matrix product seam -------------------------------------------------------------
  * Replaces helpers::Matrix<Gpu>::assignProduct / addProduct (helpers/Matrix.cu:353-377, which call

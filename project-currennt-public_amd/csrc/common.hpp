@@ -234,7 +234,6 @@ struct GemmArgs {
     int epilogue, act;
     float bias_scale;
     int masked, b_time_on_k, n_slots;
-    int halves;        // two fp16 parts per value instead of three bf16 ones, for operands whose rows hold values of about one size (gemm.hip)
     const char *pat;  // masked mode and the *_SKIP / CONTEXT epilogues
     GemmProblem prob[kGemmMaxProb];
     const char *label;  // name under which the launch is timed when profiling is on (may be NULL)
@@ -355,7 +354,7 @@ int gemm_dense_weights_static(hipStream_t stream, int P, int D, int N, float bia
 
 // Convenience: single problem, BLAS-like transposes on column-major matrices.
 int gemm_simple(hipStream_t stream, float *C, int m, int n, int k, const float *A, bool transA,
-                const float *B, bool transB, bool accumulate, bool halves = false);
+                const float *B, bool transB, bool accumulate);
 
 // cnt_opt_step with a device flag in front of it: when *veto is non-zero at the time the kernel runs (a recursion of
 // the pass that produced the gradients gave up), the step changes nothing.
@@ -398,7 +397,7 @@ struct FanOut {
 // with several filter groups, leave it to the caller).
 int dense_backward_errors_fan(hipStream_t stream, int P, int D, int N, int act, const float *weights, const float *y,
                               float *err, float *prev_err, const FanOut *fan, bool *fused, int prev_act = ACT_IDENTITY,
-                              const float *prev_y = nullptr, const SlotOrder *order = nullptr, bool even = false);
+                              const float *prev_y = nullptr, const SlotOrder *order = nullptr);
 // (prev_act, prev_y): the preceding layer is a dense layer with that activation and those outputs, and nothing but
 // this product writes its output errors: the product stores act'(prev_y) * error, the preceding layer's deltas, and
 // that layer's own backward step then runs with ACT_IDENTITY.  The same for a recurrent layer's error product:
@@ -464,7 +463,7 @@ CnnTaps cnn_taps(const cnt_cnn *h);
 // cnt_dense_backward_weights / cnt_wavnetc_backward_weights.
 int dense_backward_weights_batch(hipStream_t stream, int P, int D, int N, int count, const float *bias,
                                  const float *const *x, const float *const *err, float *const *weight_updates, const SlotOrder *order = nullptr,
-                                 DirectGroup *group = nullptr, bool even = false);
+                                 DirectGroup *group = nullptr);
 bool dense_weights_direct(int P, int D, int N, int count);  // whether that is the kernel for few blocks
 int wavnetc_backward_weights_batch(hipStream_t stream, int D, int C, int N, int count, const float *ctx,
                                    const float *const *ctx_tanh, float *const *weight_updates);

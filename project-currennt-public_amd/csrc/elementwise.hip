@@ -335,7 +335,6 @@ int cnt_dense_forward(void *stream_, int P, int D, int N, int act, float bias, c
     ga.epilogue = EPI_BIAS_ACT; ga.act = act; ga.bias_scale = bias;
     ga.prob[0].A[0] = weights; ga.prob[0].B[0] = x; ga.prob[0].C = y;
     ga.prob[0].bias_vec = weights + (size_t)P * D;
-    ga.halves = 1;
     ga.label = "gemm:dense_forward";
     return gemm_launch(static_cast<hipStream_t>(stream_), ga);
 }
@@ -348,7 +347,7 @@ int cnt_dense_backward_errors(void *stream, int P, int D, int N, int act, const 
 
 extern "C++" int cnt::dense_backward_errors_fan(hipStream_t stream, int P, int D, int N, int act, const float *weights,
                                                 const float *y, float *err, float *prev_err, const FanOut *fan,
-                                                bool *fused, int prev_act, const float *prev_y, const SlotOrder *order, bool even) {
+                                                bool *fused, int prev_act, const float *prev_y, const SlotOrder *order) {
     if (fused) *fused = false;
     CNT_REQUIRE(weights && y && err, "dense_backward_errors: null argument");
     CNT_REQUIRE(P > 0 && D > 0 && N > 0, "dense_backward_errors: non-positive size");
@@ -381,7 +380,6 @@ extern "C++" int cnt::dense_backward_errors_fan(hipStream_t stream, int P, int D
             *fused = true;
         }
         if (order) { ga.cols = order->order; ga.cols_count = order->count; }
-        ga.halves = even;
         ga.label = "gemm:dense_prev_errors";
         CNT_TRY(gemm_launch(stream, ga));
     }
@@ -396,7 +394,7 @@ int cnt_dense_backward_weights(void *stream, int P, int D, int N, float bias, co
 
 extern "C++" int cnt::dense_backward_weights_batch(hipStream_t stream, int P, int D, int N, int count, const float *bias,
                                                    const float *const *x, const float *const *err,
-                                                   float *const *weight_updates, const SlotOrder *order, DirectGroup *group, bool even) {
+                                                   float *const *weight_updates, const SlotOrder *order, DirectGroup *group) {
     CNT_REQUIRE(count >= 1 && count <= kGemmMaxProb, "dense_backward_weights: %d layers in one launch, supported 1..%d",
                 count, kGemmMaxProb);
     CNT_REQUIRE(bias && x && err && weight_updates, "dense_backward_weights: null argument");
@@ -419,7 +417,6 @@ extern "C++" int cnt::dense_backward_weights_batch(hipStream_t stream, int P, in
         ga.k_order = order->order;
         ga.k_count = order->count;
     }
-    ga.halves = even;
     ga.label = "gemm:dense_dW";
     // The launcher sums partial products in a fixed order, which overwrites the updates; it adds atomically, to updates that are cleared
     // here, only where it has no scratch (gemm.hip).  The bias part (row sums of the errors) comes along either way: a column sum behind

@@ -31,18 +31,6 @@
 // in turn (162 us); LDS stores without bank conflicts (a third of the LDS clocks less, no difference); instructions of
 // 16 x 16 x 32, which alone run a third faster (150 us: twice as many of them hold the vector instructions up).
 //
-// Two parts: where the caller says that the values of an operand's row are of about one size (GemmArgs::halves: weights, activations, the
-// errors of recurrent and dense layers; not what a mixture or a softmax hands down) and k is 128 or more, a value is split into
-// two fp16 parts, 2^s x = h + 2^-11 l, with one s per row, and three part products are added up, h*h in one accumulator and h*l, l*h in
-// another: half the matrix instructions, two thirds of the LDS traffic and half of the conversions' vector instructions.  23 of 24 bits
-// of a value are kept, but a third of the roundings remain: 2-norm error against 64 bits, three parts / two, at k = 128 1.63e-7 / 1.12e-7,
-// 256 2.36 / 1.33, 512 3.39 / 1.67, 1024 4.85 / 2.20, 6000 12.3 / 4.98; below 128 three parts are the closer ones (emulated, 64: 0.77 /
-// 0.88).  s comes from 64 values of a row (`run` in gemm_kernel.hpp); a value 2^17 times as large as those has infinite parts, and
-// its block is formed again in fp32 (1024 x 12000 x 1024 with one such value 110 -> 240 to 440 us).  us, three parts / two:
-//   1024 x 12000 x 1024 151 / 95 (265 TFLOP/s), 512 x 6000 x 512 31 / 24, 1024 x 6000 x 512 51 / 34, 1024 x 9600 x 512 74 / 51, 512 x 9600 x 1024
-//   81 / 54, 425 x 12000 x 1024 98 / 58, 1936 x 6000 x 256 42 / 33, 300 x 10000 x 425 33 / 26; every fifth row zeros: 110 / 134 at the first.
-// Passes: feed-forward model 1924 -> 1338, 32 sequences 2152 -> 1871, acoustic model 2444 -> 2279, mixture output 158 -> 147.
-//
 // Tiling: T x T x 32 per workgroup with T = 128 or 64, four 64-lane waves in a 2 x 2 arrangement, each wave
 // owning a T/2 x T/2 block as tiles of v_mfma_f32_32x32x16_bf16.  The parts lie in LDS in the order the instruction takes
 // them (TileLayout); 50 KB (T = 128) and 26 KB (T = 64) per workgroup leave room for three and five of them per compute unit, whose
@@ -110,7 +98,6 @@ inline bool eight_waves(long tiles, long run) {
 // (least and most over 512, 1024 and 2048 rows and both orders of A): k = 768 0.84-0.87 / 0.86-0.89 / 1.00-1.04 / 1.08-1.13 / 1.04 /
 // 1.23-1.25 / 0.97-0.99 / 1.10-1.12, k = 3072 0.95-1.01 / 0.96-1.02 / 1.12-1.18 / 1.22-1.28 / 1.12 / 1.32-1.35 / 1.06 / 1.17-1.20.  Lines
 // of odd length (loads of single values at the edges): from 600 tiles and 512 values on.
-constexpr long kHalvesDepth = 128;
 inline long large_tiles(const GemmArgs &a) { return (long)((a.m + 127) / 128) * ((a.n + 127) / 128) * a.nprob; }
 
 // The weight gradient of one dense layer of 64 to 256 large tiles (1024 x 1024 weights and more) also takes the large tile, and
@@ -148,31 +135,14 @@ inline bool level_gradient(const GemmArgs &a) {
            20L * a.m * a.n * a.nprob >= 19L * 16384 * tiles && (long)a.k * a.nseg * tiles >= kLevelGradientSplit * kLevelGradientGroups;
 }
 
-// Two fp16 parts: 128 x 128 on eight waves or 64 x 64 (128 x 128 on four waves was the slower one everywhere: two accumulators per sum leave two
-// such workgroups per compute unit).  Times as fast on eight waves as 64 x 64, k-contiguous / row-contiguous A, 1024 rows:
-//   tiles       160       192       224       256       288       320       384       448       512       544       640       768       1024      2048
-//   k = 128  .96/.95   .96/.94  1.07/1.01 1.05/.98   .88/.86   .88/.86  1.02/.96  1.06/1.06 1.14/1.12  .96/.87  1.04/.97  1.16/1.07 1.20/1.14 1.21/1.09
-//   256     1.02/.97  1.01/.95  1.10/1.05 1.10/1.04  .94/.91   .97/.92  1.09/1.02 1.16/1.13 1.22/1.18 1.01/.95  1.12/1.07 1.24/1.19 1.26/1.23 1.28/1.23
-//   512     1.07/1.01 1.06/.99  1.19/1.12 1.15/1.11 1.01/.97  1.01/.99  1.15/1.10 1.22/1.21 1.28/1.27 1.04/.99  1.15/1.11 1.28/1.25 1.30/1.28 1.31/1.28
-//   768     1.00/.94   .98/.93  1.12/1.04 1.14/1.07  .99/.99  1.03/1.01 1.16/1.13 1.25/1.24 1.30/1.28 1.05/1.01 1.18/1.13 1.29/1.27 1.31/1.29 1.31/1.28
-//   2048    1.02/.94  1.07/1.00 1.26/1.15 1.23/1.17 1.02/1.04 1.04/1.06 1.20/1.17 1.28/1.29 1.33/1.34 1.08/1.04 1.19/1.16 1.32/1.30 1.33/1.32
-// What decides is how full the last level of one tile per compute unit is.  Outputs that leave more than an eighth of the large tiles' rows
-// and columns empty stay on the small ones (425 x 12000 x 1024, 376 tiles, an eighth empty: 64 / 58 us).
-inline int pick_tile_of_halves(long tiles, long small, long run) {
-    if (8 * small < 7 * 4 * tiles || tiles < 224) return 64;
-    const long percent = 100 * tiles / ((tiles + 255) / 256 * 256);
-    return percent >= (tiles <= 256 ? 87 : run >= 768 ? 56 : 72) ? kEightWaves : 64;
-}
-
 int pick_tile(const GemmArgs &a) {
     static const int forced = [] { const char *e = std::getenv("CNT_GEMM_TILE"); return e ? std::atoi(e) : 0; }();
     if (a.masked || a.epilogue == EPI_FAN) return 64;
-    if (forced == 64 || forced == 128 || forced == kEightWaves) return forced == 128 && a.halves ? kEightWaves : forced;
+    if (forced == 64 || forced == 128 || forced == kEightWaves) return forced;
     const long t128 = large_tiles(a) * a.splitk;
     if ((wide_gradient(a) && t128 >= kWideGradientGroups / 2) || (level_gradient(a) && t128 >= kLevelGradientGroups / 2)) return kEightWaves;
     const long run = (long)a.k * a.nseg / a.splitk;
     const long t64 = (long)((a.m + 63) / 64) * ((a.n + 63) / 64) * a.nprob * a.splitk;
-    if (a.halves) return a.a_kcontig || a.b_kcontig || t128 >= 600 ? pick_tile_of_halves(t128, t64, run) : 64;
     // (outputs that leave more than a twelfth of the large tiles' rows and columns empty stay on the small ones: 300 x 10 000 x 425
     // and the like, 2207 -> 2276 us per pass with them on the large ones.  Up to an eighth empty, 600 tiles and more of 512 to 767
     // values are better off on the large ones, us with 64 x 64 / 128 on four waves / on eight: 430 rows, k = 640, 608 tiles 89 / 85 / 87,
@@ -509,7 +479,6 @@ int gemm_launch(hipStream_t stream, const GemmArgs &args_in, DirectGroup *group)
     }
     if (args.epilogue != EPI_PARTIAL && args.epilogue != EPI_ATOMIC && args.epilogue != EPI_STORE) args.rowsum = 0;
     if (args.masked || !args.b_kcontig || args.splitk != 1 || (args.epilogue != EPI_STORE && args.epilogue != EPI_STORE_DELTA)) args.cols = nullptr;
-    if (args.masked || args.epilogue == EPI_FAN || (long)args.k * args.nseg < kHalvesDepth) args.halves = 0;
     const int tile = pick_tile(args);
     const int edge = tile == kEightWaves ? 128 : tile;
     // a list of k lines is used where the kernel that reads through it exists, and ignored otherwise (the lines it leaves
@@ -590,7 +559,7 @@ int gemm_dense_weights_static(hipStream_t stream, int P, int D, int N, float bia
 }
 
 int gemm_simple(hipStream_t stream, float *C, int m, int n, int k, const float *A, bool transA,
-                const float *B, bool transB, bool accumulate, bool halves) {
+                const float *B, bool transB, bool accumulate) {
     GemmArgs a = {};
     a.m = m; a.n = n; a.k = k;
     // column-major A (m x k, lda=m) is row-contiguous; transposed storage (k x m, lda=k) is k-contiguous
@@ -601,7 +570,6 @@ int gemm_simple(hipStream_t stream, float *C, int m, int n, int k, const float *
     a.ldb = transB ? n : k;
     a.ldc = m;
     a.nseg = 1; a.nprob = 1; a.splitk = 1;
-    a.halves = halves;
     a.epilogue = accumulate ? EPI_ADD : EPI_STORE;
     a.prob[0].A[0] = A;
     a.prob[0].B[0] = B;
@@ -610,12 +578,6 @@ int gemm_simple(hipStream_t stream, float *C, int m, int n, int k, const float *
 }
 
 }  // namespace cnt
-
-extern "C" int cnt_probe_product_of_halves(void *stream, float *C, int m, int n, int k, const float *A, int transA, const float *B, int transB) {
-    using namespace cnt;
-    CNT_REQUIRE(C && A && B && !(transA && transB), "probe_product_of_halves: bad argument");
-    return gemm_simple(static_cast<hipStream_t>(stream), C, m, n, k, A, transA != 0, B, transB != 0, false, true);
-}
 
 extern "C" int cnt_probe_gemm_plan(int m, int n, int k, int problems, int a_kcontig, int b_kcontig, int weight_gradient, int *plan) {
     using namespace cnt;

@@ -17,21 +17,12 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 // workgroup barrier that orders LDS traffic only; global loads issued before it stay in flight
 __device__ __forceinline__ void lds_only_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// the lane's number, worked out where it is asked for: nothing of it is kept in registers through a loop in front
-__device__ __forceinline__ int lane_asked_for_here() {
-    int n;
-    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(n));
-    return n;
 }
 
 template <int V>
@@ -63,53 +54,18 @@ __device__ __forceinline__ void split_pair(float x0, float x1, unsigned (&part)[
     }
 }
 
-// Two fp32 values as two fp16 pairs: 2^s x = h + 2^-11 l, s a number of the operand's row.  h is the nearest fp16 value (11 bits of
-// significand), l the nearest one to 2^11 times what it leaves: 23 of 24 bits wherever 2^s x is 2^-12 or more in size, steps of
-// 2^-36 below, infinite parts from 65520 on.  `factor` is 2^(s + 11), so that the two steps are exact.
-constexpr float kHalfLow = 2048.0f;  // 2^11
-constexpr int kHalfLowBits = 11;
-__device__ __forceinline__ unsigned nearest_f16(float x0, float x1) {
-    return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x0, x1}), f16x2));
-}
-__device__ __forceinline__ void split_pair(float x0, float x1, float factor0, float factor1, unsigned (&part)[2]) {
-    x0 *= factor0; x1 *= factor1;
-    part[0] = nearest_f16(x0 * (1.0f / kHalfLow), x1 * (1.0f / kHalfLow));
-    const f16x2 h = __builtin_bit_cast(f16x2, part[0]);
-    part[1] = nearest_f16(__builtin_fmaf((float)h[0], -kHalfLow, x0), __builtin_fmaf((float)h[1], -kHalfLow, x1));
-}
-// The row's number from its largest value (as bits) among those looked at, the peak: peaks lie between 2^-2 and 2^-1, which leaves a
-// factor of 2^17 for values that were not looked at, 10 binades below the peak with all 23 bits, and steps of 2^-34 of it below those.
-constexpr int kPeakAt = -2;
-__device__ __forceinline__ int exponent_of_peak(unsigned bits) { return min(kPeakAt + 127 - (int)(bits >> 23), 127 - kHalfLowBits); }
-__device__ __forceinline__ float factor_of_peak(unsigned bits) {
-    return __uint_as_float((unsigned)(exponent_of_peak(bits) + kHalfLowBits + 127) << 23);
-}
-// largest of |a|, |b| and m; infinite or not a number where one of them is infinite or a signalling NaN
-__device__ __forceinline__ float larger_size(float a, float b, float m) {
-    float v;
-    asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(v) : "v"(a), "v"(b), "v"(m));
-    return v;
-}
-__device__ __forceinline__ float finite_size(float x) {
-    const float v = __builtin_fabsf(x);
-    return v <= lim::kMax ? v : 0.0f;
-}
-// whether a peak says something about its row: no zeros only, nothing infinite
-__device__ __forceinline__ bool known(unsigned bits) { return bits - 1u < 0x7f7fffffu; }
-
 // Where the parts of a ROWS-row x BK-k operand tile lie in LDS.  The 16-byte unit is what one lane of a matrix instruction
 // takes: eight consecutive k of one row.  Units are ordered [part][k / 8][position of the row]; the position of a row is the
 // row itself where a thread loads along k, and r * GROUP + t for row VEC * t + r where it loads VEC rows at once, so that in
 // both cases the lanes of one store, and those of one read, fall on distinct banks (the pads of GROUP and LINE see to it).
-template <int VEC, bool KCONTIG, int ROWS, int NT = NTHREADS, int PARTS = 3>
+template <int VEC, bool KCONTIG, int ROWS, int NT = NTHREADS>
 struct TileLayout {
     static constexpr int NLOAD = (ROWS * BK) / (NT * VEC);  // vectors per thread
     static_assert(NLOAD >= 1, "tile too small for this vector width");
     static constexpr int GROUP = ROWS / VEC + (VEC == 4 ? 4 : VEC == 2 ? 8 : 0);
     static constexpr int LINE = KCONTIG ? ROWS + 4 : VEC * GROUP;  // units per k / 8
     static constexpr int PART = (BK / 8) * LINE;                   // units per part
-    static constexpr int UNITS = PARTS * PART;
-    static constexpr int FACTORS = KCONTIG ? NLOAD : VEC;  // rows of a thread's vectors
+    static constexpr int UNITS = 3 * PART;
     typedef typename VecT<VEC>::type vec_t;
 
     // k-contiguous: the thread's vectors start at k position first_k of the rows row(p); row-contiguous: they hold the VEC
@@ -128,40 +84,11 @@ struct TileLayout {
     static __device__ __forceinline__ int first_row(int tid) { return KCONTIG ? tid / TPR : column(tid) * VEC; }
     static __device__ __forceinline__ int row(int tid, int p) { return KCONTIG ? tid / TPR + p * RPP : column(tid) * VEC; }
 
-    // The factors of the rows of a thread's vectors (two parts): in registers, or, where they are one 16-byte read, in LDS (registers are
-    // what the kernels for two row-contiguous operands are short of).
-    struct Factors {
-        float mine[KCONTIG ? FACTORS : 1];
-        const float *at;
-        __device__ __forceinline__ void init(const unsigned *peak, const float *all, int tid) {
-            at = all + first_row(tid);
-            if constexpr (KCONTIG)
-#pragma unroll
-                for (int f = 0; f < FACTORS; ++f) mine[f] = factor_of_peak(peak[row(tid, f)]);
-        }
-        __device__ __forceinline__ void get(float (&f)[FACTORS]) const {
-            if constexpr (PARTS == 3) return;
-            else if constexpr (KCONTIG) {
-#pragma unroll
-                for (int q = 0; q < FACTORS; ++q) f[q] = mine[q];
-            } else {
-                const float4 x = *reinterpret_cast<const float4 *>(at);
-                f[0] = x.x; f[1] = x.y; f[2] = x.z; f[3] = x.w;
-            }
-        }
-    };
-    static __device__ __forceinline__ void put(uint4 *__restrict__ lds, int tid, const vec_t (&v)[NLOAD], const Factors &factors) {
-        float factor[FACTORS];
-        factors.get(factor);
-        auto split = [&](float x0, float x1, int f, unsigned (&x)[PARTS]) __attribute__((always_inline)) {
-            if constexpr (PARTS == 3) split_pair(x0, x1, x);
-            else split_pair(x0, x1, factor[f], factor[f], x);
-        };
+    static __device__ __forceinline__ void put(uint4 *__restrict__ lds, int tid, const vec_t (&v)[NLOAD]) {
         const int k = first_k(tid);
         if (KCONTIG) {
             char *at = reinterpret_cast<char *>(lds + (k / 8) * LINE + tid / TPR) + 2 * (k % 8);
             if constexpr (VEC == 1) {
-                static_assert(PARTS == 3, "vectors of one float hold one value of each of two rows");
 #pragma unroll
                 for (int p = 0; p < NLOAD; p += 2) {
                     unsigned x[3];
@@ -176,11 +103,11 @@ struct TileLayout {
 #pragma unroll
                 for (int p = 0; p < NLOAD; ++p) {
                     const float *e = reinterpret_cast<const float *>(&v[p]);
-                    unsigned x[VEC / 2][PARTS];
+                    unsigned x[VEC / 2][3];
 #pragma unroll
-                    for (int j = 0; j < VEC / 2; ++j) split(e[2 * j], e[2 * j + 1], p, x[j]);
+                    for (int j = 0; j < VEC / 2; ++j) split_pair(e[2 * j], e[2 * j + 1], x[j]);
 #pragma unroll
-                    for (int q = 0; q < PARTS; ++q) {
+                    for (int q = 0; q < 3; ++q) {
                         char *to = at + 16 * (q * PART + p * RPP);
                         if constexpr (VEC == 4) *reinterpret_cast<uint2 *>(to) = uint2{x[0][q], x[1][q]};
                         else *reinterpret_cast<unsigned *>(to) = x[0][q];
@@ -191,12 +118,12 @@ struct TileLayout {
             char *at = reinterpret_cast<char *>(lds + (k / 8) * LINE + column(tid)) + 2 * (k % 8);
 #pragma unroll
             for (int r = 0; r < VEC; ++r) {
-                unsigned x[NLOAD / 2][PARTS];
+                unsigned x[NLOAD / 2][3];
 #pragma unroll
                 for (int p = 0; p < NLOAD; p += 2)
-                    split(reinterpret_cast<const float *>(&v[p])[r], reinterpret_cast<const float *>(&v[p + 1])[r], r, x[p / 2]);
+                    split_pair(reinterpret_cast<const float *>(&v[p])[r], reinterpret_cast<const float *>(&v[p + 1])[r], x[p / 2]);
 #pragma unroll
-                for (int q = 0; q < PARTS; ++q) {
+                for (int q = 0; q < 3; ++q) {
                     char *to = at + 16 * (q * PART + r * GROUP);
                     if constexpr (NLOAD == 2) *reinterpret_cast<unsigned *>(to) = x[0][q];
                     else if constexpr (NLOAD == 4) *reinterpret_cast<uint2 *>(to) = uint2{x[0][q], x[1][q]};
@@ -211,44 +138,11 @@ struct TileLayout {
         }
     }
 
-    // the parts of k positions [8 * k8, 8 * k8 + 8) of tile row `row`
-    typedef typename std::conditional<PARTS == 3, bf16x8, f16x8>::type part_t;
-    static __device__ __forceinline__ void fragment(const uint4 *__restrict__ lds, int row, int k8, part_t (&f)[PARTS]) {
+    // the three parts of k positions [8 * k8, 8 * k8 + 8) of tile row `row`
+    static __device__ __forceinline__ void fragment(const uint4 *__restrict__ lds, int row, int k8, bf16x8 (&f)[3]) {
         const uint4 *at = lds + k8 * LINE + (KCONTIG ? row : (row % VEC) * GROUP + row / VEC);
 #pragma unroll
-        for (int q = 0; q < PARTS; ++q) f[q] = __builtin_bit_cast(part_t, at[q * PART]);
-    }
-
-    // Peaks of a tile in registers: the largest value of each of the thread's rows over its k positions, joined with the other
-    // threads' in `peak` (bits of a float per row of the tile, cleared before; their order is that of the values).  k-contiguous: a row's
-    // eight threads are neighbours.
-    static __device__ __forceinline__ void row_peaks(const vec_t (&v)[NLOAD], float (&size)[FACTORS]) {
-        static_assert(VEC == 4, "the unmasked loaders");
-        if constexpr (KCONTIG) {
-#pragma unroll
-            for (int p = 0; p < NLOAD; ++p) size[p] = larger_size(v[p].z, v[p].w, larger_size(v[p].x, v[p].y, size[p]));
-        } else {
-#pragma unroll
-            for (int p = 0; p < NLOAD; p += 2) {
-                size[0] = larger_size(v[p].x, v[p + 1].x, size[0]); size[1] = larger_size(v[p].y, v[p + 1].y, size[1]);
-                size[2] = larger_size(v[p].z, v[p + 1].z, size[2]); size[3] = larger_size(v[p].w, v[p + 1].w, size[3]);
-            }
-        }
-    }
-    static __device__ __forceinline__ void join_peaks(unsigned *__restrict__ peak, int tid, const float (&size)[FACTORS]) {
-#pragma unroll
-        for (int f = 0; f < FACTORS; ++f) {
-            unsigned bits = __float_as_uint(size[f]);
-            if (KCONTIG) {
-                static_assert(TPR == 8 || !KCONTIG, "lanes of a row");
-                bits = max(bits, (unsigned)__builtin_amdgcn_update_dpp(0, (int)bits, 0xb1, 0xf, 0xf, false));   // the other lane of a pair,
-                bits = max(bits, (unsigned)__builtin_amdgcn_update_dpp(0, (int)bits, 0x4e, 0xf, 0xf, false));   // the other pair of four,
-                bits = max(bits, (unsigned)__builtin_amdgcn_update_dpp(0, (int)bits, 0x141, 0xf, 0xf, false));  // the other four of eight
-                if (tid % TPR == 0) peak[row(tid, f)] = bits;
-            } else {
-                atomicMax(peak + first_row(tid) + f, bits);
-            }
-        }
+        for (int q = 0; q < 3; ++q) f[q] = __builtin_bit_cast(bf16x8, at[q * PART]);
     }
 };
 
@@ -358,7 +252,7 @@ struct TileStage {
         typename VecT<VEC>::type v[NLOAD];
 #pragma unroll
         for (int p = 0; p < NLOAD; ++p) v[p] = kept(p);
-        L::put(lds, tid, v, typename L::Factors());
+        L::put(lds, tid, v);
     }
 };
 
@@ -387,12 +281,11 @@ __device__ __forceinline__ void add_tile_rows(float (&sum)[4], const float4 (&r)
 }
 
 // WHOLE: the lines are a multiple of four long, so that no vector crosses the end of one.
-template <bool WHOLE, bool KCONTIG, int ROWS, int NT, int PARTS>
+template <bool WHOLE, bool KCONTIG, int ROWS, int NT>
 struct FastStage {
-    typedef TileLayout<4, KCONTIG, ROWS, NT, PARTS> L;
+    typedef TileLayout<4, KCONTIG, ROWS, NT> L;
     static constexpr int NLOAD = L::NLOAD;
     float4 r[NLOAD];
-    typename L::Factors factor;
     unsigned voff[NLOAD];
     int ld, row0, rows_total;  // uniform
 
@@ -415,48 +308,20 @@ struct FastStage {
         if (left >= (KCONTIG || WHOLE ? BK : BK + 3)) {
 #pragma unroll
             for (int p = 0; p < NLOAD; ++p) {
-                asm volatile("" : "+v"(voff[p]));  // (else the loop keeps the offsets in 64 bits, in twice the registers)
                 const f32x4u v = *reinterpret_cast<const f32x4u *>(b + voff[p]);
                 r[p] = float4{v[0], v[1], v[2], v[3]};
             }
         } else if (WHOLE) {
-            int line = ld;
-            asm volatile("" : "+s"(line));
-            asm volatile("" : "+v"(tid));  // what follows is worked out here, not kept in registers through the loop
 #pragma unroll
             for (int p = 0; p < NLOAD; ++p) {
                 const int k = kpos(tid, p);
-                const unsigned back = (unsigned)(k * (KCONTIG ? 1 : line)) * (unsigned)sizeof(float);  // to k position 0
+                const unsigned back = (unsigned)(k * (KCONTIG ? 1 : ld)) * (unsigned)sizeof(float);  // to k position 0
                 const f32x4u v = *reinterpret_cast<const f32x4u *>(b + (k < left ? voff[p] : voff[p] - back));
                 r[p] = k < left ? float4{v[0], v[1], v[2], v[3]} : float4{0.0f, 0.0f, 0.0f, 0.0f};
             }
-        } else if (PARTS == 2 && (KCONTIG || rows_total >= 4)) {
-            // (two parts: k is kHalvesDepth at least.)  A vector that would reach beyond its line is the line's last one, moved into place.
-            int line = ld;
-            asm volatile("" : "+s"(line));
-            asm volatile("" : "+v"(tid));
-#pragma unroll
-            for (int p = 0; p < NLOAD; ++p) {
-                const int k = kpos(tid, p), over = KCONTIG ? max(k + 4 - left, 0) : max(min(row0 + L::row(tid, p), rows_total) + 4 - rows_total, 0);
-                unsigned back = (unsigned)(KCONTIG ? over : k < left ? 0 : k * line);
-                // (row-contiguous: rows past the edge stand for the first one in voff, which has its line to itself)
-                if (!KCONTIG) back += row0 + L::row(tid, p) < rows_total ? over : 0;
-                // (in 64 bits: the operand's first line may end within the first three values of a tile, in front of which its last vector begins)
-                const f32x4u v = *reinterpret_cast<const f32x4u *>(b + ((long)voff[p] - (long)back * (long)sizeof(float)));
-                float e[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    float x = v[3];
-#pragma unroll
-                    for (int d = 2; d >= q; --d) x = over <= d - q ? v[d] : x;
-                    e[q] = KCONTIG ? (k + q < left ? x : 0.0f) : k < left ? x : 0.0f;
-                }
-                r[p] = float4{e[0], e[1], e[2], e[3]};
-            }
         } else {
             int line = ld;
-            if (PARTS == 2) asm volatile("" : "+s"(line));
-            if (PARTS == 2) asm volatile("" : "+v"(tid));
+            asm volatile("" : "+s"(line));  // the addresses below are formed here, not kept in registers through the loop
 #pragma unroll
             for (int p = 0; p < NLOAD; ++p) {
                 float e[4];
@@ -472,8 +337,7 @@ struct FastStage {
             }
         }
     }
-    __device__ __forceinline__ void store(uint4 *__restrict__ lds, int tid) const { L::put(lds, tid, r, factor); }
-    __device__ __forceinline__ void row_peaks(float (&size)[L::FACTORS]) const { L::row_peaks(r, size); }
+    __device__ __forceinline__ void store(uint4 *__restrict__ lds, int tid) const { L::put(lds, tid, r); }
     // adds the tile in registers to the sums of the thread's four rows (row-contiguous operands)
     __device__ __forceinline__ void add_rows(float (&sum)[4]) const { add_tile_rows<NLOAD>(sum, r); }
 };
@@ -481,12 +345,11 @@ struct FastStage {
 // The unmasked loader for row-contiguous operands whose k lines are picked through a list (16-byte vectors only): tile k
 // line j is line idx[j] of the operand.  The indices of a tile are loaded one iteration ahead by the kernel (both operands
 // share them) and handed to load(); everything else is FastStage.
-template <int ROWS, int NT, int PARTS>
+template <int ROWS, int NT>
 struct GatherStage {
-    typedef TileLayout<4, false, ROWS, NT, PARTS> L;
+    typedef TileLayout<4, false, ROWS, NT> L;
     static constexpr int NLOAD = L::NLOAD;
     float4 r[NLOAD];
-    typename L::Factors factor;
     unsigned roff;   // byte offset of the thread's four rows inside a k line (clamped into the matrix)
     int kk;          // the thread's first k line inside a tile; its others follow
     int k_valid;     // uniform: k lines of the tile in registers that are listed
@@ -510,16 +373,10 @@ struct GatherStage {
             float4 v[NLOAD];
 #pragma unroll
             for (int p = 0; p < NLOAD; ++p) v[p] = kk + p < k_valid ? r[p] : float4{0.0f, 0.0f, 0.0f, 0.0f};
-            L::put(lds, tid, v, factor);
+            L::put(lds, tid, v);
         } else {
-            L::put(lds, tid, r, factor);
+            L::put(lds, tid, r);
         }
-    }
-    __device__ __forceinline__ void row_peaks(float (&size)[4]) const {
-        float4 v[NLOAD];
-#pragma unroll
-        for (int p = 0; p < NLOAD; ++p) v[p] = kk + p < k_valid ? r[p] : float4{0.0f, 0.0f, 0.0f, 0.0f};
-        L::row_peaks(v, size);
     }
     __device__ __forceinline__ void add_rows(float (&sum)[4]) const {
         float4 v[NLOAD];
@@ -597,7 +454,6 @@ __device__ __forceinline__ void by_activation(int act, STEP &&step) {
     }
 }
 
-// PARTS: three bf16 parts of a value or two fp16 ones (gemm.hip has when and why).
 // VA, VB: vector widths of the masked loader, 16-byte alignment included; unmasked: 4 where the operand's lines are a
 // multiple of four long, at any alignment, else 1.
 // MASKED selects the time-shifted, padding-masked B loader at compile time: its per-element predication is a lot
@@ -610,21 +466,16 @@ __device__ __forceinline__ void by_activation(int act, STEP &&step) {
 // behind another's matrix instructions.  128 x 128 tiles of two row-contiguous operands take 55 KB each, so two: where three were
 // asked for, the compiler held operands in accumulator registers and a small change made it miss two as well (the feed-forward
 // model 2213 -> 2293 us per pass).
-template <int VA, bool AK, int VB, bool BK_, bool MASKED, int TILE, int PARTS, bool FAN = false, bool GATHER = false, int WAVES = 4>
-__global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS == 3 && VA * VB == 16 && (AK || BK_) ? 3 : 2) : VA * VB == 16 ? 5 : 4) void gemm_split_kernel(const GemmArgs args) {
-    constexpr bool HALVES = PARTS == 2;
-    static_assert(!HALVES || (!MASKED && !FAN), "kernels that exist");
+template <int VA, bool AK, int VB, bool BK_, bool MASKED, int TILE, bool FAN = false, bool GATHER = false, int WAVES = 4>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (VA * VB == 16 && (AK || BK_) ? 3 : 2) : VA * VB == 16 ? 5 : 4) void gemm_split_kernel(const GemmArgs args) {
     constexpr int BM = TILE, BN = TILE;
     constexpr int NT = 64 * WAVES;
     static_assert(WAVES == 4 || !MASKED, "the masked loader is for four waves");
     constexpr int WM = TILE / 2, WN = 2 * TILE / WAVES;  // a wave's block (waves are arranged 2 x 2 or 2 x 4)
     constexpr int NBM = WM / 32, NBN = WN / 32;          // 32 x 32 MFMA tiles per wave and dimension
-    typedef TileLayout<MASKED ? VA : 4, AK, TILE, NT, PARTS> LA;
-    typedef TileLayout<MASKED ? VB : 4, BK_, TILE, NT, PARTS> LB;
+    typedef TileLayout<MASKED ? VA : 4, AK, TILE, NT> LA;
+    typedef TileLayout<MASKED ? VB : 4, BK_, TILE, NT> LB;
     __shared__ uint4 lds[LA::UNITS + LB::UNITS];
-    __shared__ unsigned peak[HALVES ? 2 * TILE : 1];  // of the rows of A, then of B
-    __shared__ __align__(16) float factor[HALVES ? 2 * TILE : 1];
-    __shared__ unsigned missing[HALVES ? 2 * TILE : 1];
     uint4 *const lds_a = lds, *const lds_b = lds + LA::UNITS;
 
     const int tid = threadIdx.x;
@@ -705,17 +556,13 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
     // (a split left without k lines by a short list still has its zeros to write)
     if (it_begin >= it_end && !(GATHER && args.epilogue != EPI_ATOMIC)) return;
 
-    // the products of the high parts, and those with a low part, which stand for 2^-11 of their size (halves)
-    f32x16 acc[NBM][NBN], low[HALVES ? NBM : 1][HALVES ? NBN : 1];
+    f32x16 acc[NBM][NBN];
 #pragma unroll
     for (int i = 0; i < NBM; ++i)
 #pragma unroll
         for (int j = 0; j < NBN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                acc[i][j][r] = 0.0f;
-                if constexpr (HALVES) low[i][j][r] = 0.0f;
-            }
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
     const char *mask_pat = MASKED ? args.pat : nullptr;
 
@@ -732,172 +579,36 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
     // again, so that the count of loads in flight is the same on every path.  The loads of tile it+1 are in flight during
     // the matrix instructions of tile it; the barriers order LDS only (__syncthreads() would also wait for those loads).
     auto loop = [&](auto &ra, auto &rb, auto &fetch_next, auto sums) __attribute__((always_inline)) {
+        fetch_next(ra, rb);
         for (int it = it_begin; it < it_end; ++it) {
-            if constexpr (decltype(sums)::value)
-                if (!HALVES || rowsum) rb.add_rows(rs);
+            if constexpr (decltype(sums)::value) rb.add_rows(rs);
             ra.store(lds_a, tid);
             rb.store(lds_b, tid);
             fetch_next(ra, rb);
             lds_only_barrier();
 #pragma unroll
             for (int s = 0; s < BK / 16; ++s) {
-                typename LA::part_t fa[NBM][PARTS], fb[NBN][PARTS];
+                bf16x8 fa[NBM][3], fb[NBN][3];
 #pragma unroll
                 for (int i = 0; i < NBM; ++i) LA::fragment(lds_a, wm * WM + i * 32 + frag_row, 2 * s + half, fa[i]);
 #pragma unroll
                 for (int j = 0; j < NBN; ++j) LB::fragment(lds_b, wn * WN + j * 32 + frag_row, 2 * s + half, fb[j]);
-                if constexpr (HALVES) {
-                    // l*h, h*l, h*h
+                // h*l, l*h, m*m, h*m, m*h, h*h: the small terms first
+                constexpr int QA[6] = {0, 2, 1, 0, 1, 0}, QB[6] = {2, 0, 1, 1, 0, 0};
 #pragma unroll
-                    for (int t = 0; t < 2; ++t)
-#pragma unroll
-                        for (int i = 0; i < NBM; ++i)
-#pragma unroll
-                            for (int j = 0; j < NBN; ++j)
-                                low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[j][1 - t], fa[i][t], low[i][j], 0, 0, 0);
+                for (int t = 0; t < 6; ++t)
 #pragma unroll
                     for (int i = 0; i < NBM; ++i)
 #pragma unroll
                         for (int j = 0; j < NBN; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[j][0], fa[i][0], acc[i][j], 0, 0, 0);
-                } else {
-                    // h*l, l*h, m*m, h*m, m*h, h*h: the small terms first
-                    constexpr int QA[6] = {0, 2, 1, 0, 1, 0}, QB[6] = {2, 0, 1, 1, 0, 0};
-#pragma unroll
-                    for (int t = 0; t < 6; ++t)
-#pragma unroll
-                        for (int i = 0; i < NBM; ++i)
-#pragma unroll
-                            for (int j = 0; j < NBN; ++j)
-                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j][QB[t]], fa[i][QA[t]], acc[i][j], 0, 0, 0);
-                }
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j][QB[t]], fa[i][QA[t]], acc[i][j], 0, 0, 0);
             }
             lds_only_barrier();
         }
     };
-    // Two parts: the peaks of an operand's rows from all their values, for the rows that have none.  Every thread has eight loads of four
-    // values in flight; rows past an edge hold the last one.
-    auto missing_peaks = [&](auto kcontig, bool of_a, int ld, int row0, int rows_total, const int *rows, int first) __attribute__((always_inline)) {
-        constexpr bool KC = decltype(kcontig)::value;
-        constexpr int PER_ROW = KC ? NT / TILE : 4 * NT / TILE;  // threads that share a row (k-contiguous) or four
-        constexpr int LOADS = 8;
-        const int row = KC ? tid / PER_ROW : 4 * (tid % (TILE / 4)), c = KC ? tid % PER_ROW : tid / (TILE / 4);
-        const int line = rows ? rows[row] : min(row0 + row, rows_total - 1);
-        const bool whole = KC || row0 + row + 4 <= rows_total;
-        float size[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 1
-        for (int it = it_begin; it < it_end;) {
-            const int seg = it / kt_per_seg, kin = it % kt_per_seg, run = min(kt_per_seg - kin, it_end - it);
-            const int k0 = kin * BK, k1 = min(k0 + run * BK, k_extent);
-            const float *const base = of_a ? pb.A[seg] : pb.B[seg];
-            if constexpr (KC) {
-                const float *const from = base + (size_t)line * ld;
-                int k = k0 + 4 * c;
-                for (; k + 4 * PER_ROW * (LOADS - 1) + 4 <= k1; k += 4 * PER_ROW * LOADS) {
-                    f32x4u v[LOADS];
-#pragma unroll
-                    for (int u = 0; u < LOADS; ++u) v[u] = *reinterpret_cast<const f32x4u *>(from + k + 4 * PER_ROW * u);
-#pragma unroll
-                    for (int u = 0; u < LOADS; ++u)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) size[q] = fmaxf(size[q], finite_size(v[u][q]));
-                }
-                for (; k < k1; k += 4 * PER_ROW)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) size[q] = fmaxf(size[q], finite_size(from[min(k + q, k1 - 1)]));
-            } else {
-                for (int k = k0 + c; k < k1; k += PER_ROW * LOADS) {
-                    float v[LOADS][4];
-#pragma unroll
-                    for (int u = 0; u < LOADS; ++u) {
-                        int at = min(k + PER_ROW * u, k1 - 1);
-                        if constexpr (GATHER) at = args.k_order[k_lo + at] + pb.k_shift;
-                        const float *const from = base + (size_t)at * ld;
-                        if (whole) {
-                            const f32x4u x = *reinterpret_cast<const f32x4u *>(from + line);
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) v[u][q] = x[q];
-                        } else {
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) v[u][q] = from[min(row0 + row + q, rows_total - 1)];
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < LOADS; ++u)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) size[q] = fmaxf(size[q], finite_size(v[u][q]));
-                }
-            }
-            it += run;
-        }
-        if constexpr (KC) {
-            const float all = fmaxf(fmaxf(size[0], size[1]), fmaxf(size[2], size[3]));
-            atomicMax(missing + first + row, __float_as_uint(all));
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                atomicMax(missing + first + row + q, __float_as_uint(size[q]));
-        }
-    };
-    // Two parts: a row's peak is the smaller one of its largest values in the walk's first tile and in the one in its middle, so that one
-    // value far larger than the others is not taken for the row's size (its parts are infinite then and the sums formed again).  Where both
-    // are zeros or infinite it comes from all of the row's values: rows of padding, inputs that are mostly zeros.
-    // `load_tile(it, a, b)` loads a tile beside the walk.
-    auto run = [&](auto &ra, auto &rb, auto &fetch_next, auto &load_tile) __attribute__((always_inline)) {
-        fetch_next(ra, rb);
-        if constexpr (HALVES) {
-            unsigned *const second = missing;  // of the tile in the middle; then the sizes of rows without a peak
-            if (tid < 2 * TILE) peak[tid] = second[tid] = 0;
-            float size_a[2][LA::FACTORS] = {}, size_b[2][LB::FACTORS] = {};
-            {
-                auto ma = ra;
-                auto mb = rb;
-                load_tile((it_begin + it_end) / 2, ma, mb);
-                ma.row_peaks(size_a[1]);
-                mb.row_peaks(size_b[1]);
-            }
-            ra.row_peaks(size_a[0]);
-            rb.row_peaks(size_b[0]);
-            lds_only_barrier();
-            LA::join_peaks(peak, tid, size_a[0]);
-            LB::join_peaks(peak + TILE, tid, size_b[0]);
-            LA::join_peaks(second, tid, size_a[1]);
-            LB::join_peaks(second + TILE, tid, size_b[1]);
-            lds_only_barrier();
-            // (every wave looks at all rows: no barrier for their answer)
-            unsigned mine = 0;
-            bool none[2] = {false, false};
-#pragma unroll
-            for (int q = 0; q < 2 * TILE / 64; ++q) {
-                const unsigned x = peak[64 * q + lane], y = second[64 * q + lane];
-                const unsigned both = !known(x) ? y : !known(y) ? x : min(x, y);
-                none[q / (TILE / 64)] = none[q / (TILE / 64)] || !known(both);
-                mine = q == wave ? both : mine;
-            }
-            static_assert(2 * TILE / 64 <= WAVES, "a wave takes 64 rows");
-            lds_only_barrier();
-            if (wave < 2 * TILE / 64) {
-                peak[64 * wave + lane] = known(mine) ? mine : 0;
-                factor[64 * wave + lane] = factor_of_peak(known(mine) ? mine : 0);
-                missing[64 * wave + lane] = 0;
-            }
-            lds_only_barrier();
-            const bool none_a = __builtin_amdgcn_ballot_w64(none[0]) != 0, none_b = __builtin_amdgcn_ballot_w64(none[1]) != 0;
-            if (__builtin_expect(none_a || none_b, 0)) {
-                if (none_a) missing_peaks(std::integral_constant<bool, AK>(), true, args.lda, m0, args.m, nullptr, 0);
-                if (none_b) missing_peaks(std::integral_constant<bool, BK_>(), false, args.ldb, n0, args.n, listed ? col_of : nullptr, TILE);
-                lds_only_barrier();
-                if (wave < 2 * TILE / 64 && peak[64 * wave + lane] == 0) {
-                    peak[64 * wave + lane] = missing[64 * wave + lane];
-                    factor[64 * wave + lane] = factor_of_peak(missing[64 * wave + lane]);
-                }
-                lds_only_barrier();
-            }
-            ra.factor.init(peak, factor, tid);
-            rb.factor.init(peak + TILE, factor + TILE, tid);
-        }
+    auto run = [&](auto &ra, auto &rb, auto &fetch_next) __attribute__((always_inline)) {
         if constexpr (!AK && !BK_ && !MASKED) {
-            if (HALVES || rowsum) {  // (two parts: a second loop left too few registers for either)
+            if (rowsum) {
                 loop(ra, rb, fetch_next, std::true_type());
                 return;
             }
@@ -906,11 +617,10 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
     };
     if constexpr (GATHER) {
         static_assert(VA == 4 && VB == 4 && !AK && !BK_ && !MASKED, "the gathering loader is for two row-contiguous operands");
-        typedef GatherStage<TILE, NT, PARTS> Stage;
-        Stage ga, gb;
+        GatherStage<TILE, NT> ga, gb;
         ga.init(m0, args.m, tid);
         gb.init(n0, args.n, tid);
-        constexpr int NL = Stage::NLOAD;
+        constexpr int NL = GatherStage<TILE, NT>::NLOAD;
         const int *__restrict__ order = args.k_order + k_lo;
         const int k_shift = pb.k_shift;
         const unsigned a_line = (unsigned)(args.lda * sizeof(float)), b_line = (unsigned)(args.ldb * sizeof(float));
@@ -918,19 +628,12 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
         const float *pa = pb.A[seg], *pbb = pb.B[seg];
         // the k lines of the cursor's tile, loaded while the tile before it is being requested
         int idx[NL];
-        auto lines_of = [&](int tile, int (&to)[NL]) __attribute__((always_inline)) {
+        auto lines_of = [&](int tile) __attribute__((always_inline)) {
 #pragma unroll
-            for (int p = 0; p < NL; ++p) to[p] = order[max(min(tile * BK + ga.kk + p, k_extent - 1), 0)] + k_shift;
+            for (int p = 0; p < NL; ++p) idx[p] = order[max(min(tile * BK + ga.kk + p, k_extent - 1), 0)] + k_shift;
         };
-        lines_of(kin, idx);
-        auto load_tile = [&](int it, Stage &qa, Stage &qb) __attribute__((always_inline)) {
-            int lines[NL];
-            const int s = it / kt_per_seg, tile = it % kt_per_seg, kv = min(BK, k_extent - tile * BK);
-            lines_of(tile, lines);
-            qa.load(pb.A[s], a_line, lines, kv);
-            qb.load(pb.B[s], b_line, lines, kv);
-        };
-        auto fetch_next = [&](Stage &qa, Stage &qb) __attribute__((always_inline)) {
+        lines_of(kin);
+        auto fetch_next = [&](GatherStage<TILE, NT> &qa, GatherStage<TILE, NT> &qb) __attribute__((always_inline)) {
             const int kv = min(BK, k_extent - kin * BK);
             qa.load(pa, a_line, idx, kv);
             qb.load(pbb, b_line, idx, kv);
@@ -941,9 +644,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
                     pa = pb.A[seg]; pbb = pb.B[seg];
                 }
             }
-            lines_of(kin, idx);
+            lines_of(kin);
         };
-        if (it_begin < it_end) run(ga, gb, fetch_next, load_tile);
+        if (it_begin < it_end) run(ga, gb, fetch_next);
     } else if constexpr (MASKED) {
         TileStage<VA, AK, TILE> sa;
         TileStage<VB, BK_, TILE> sb;
@@ -957,26 +660,18 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
             rb.load(pb.B[seg], args.ldb, n0, k0, args.n, args.k, tid, mask_pat, pb.b_shift[seg], args.n_slots,
                     args.b_time_on_k != 0);
         };
-        auto none = [] {};
-        run(sa, sb, fetch_next, none);
+        run(sa, sb, fetch_next);
     } else {
         // the tile cursor: operand pair `seg`, k tile `kin` inside it; the operands' base pointers are looked up only
         // when the pair changes
-        typedef FastStage<VA == 4, AK, TILE, NT, PARTS> StageA;
-        typedef FastStage<VB == 4, BK_, TILE, NT, PARTS> StageB;
-        StageA sa;
-        StageB sb;
+        FastStage<VA == 4, AK, TILE, NT> sa;
+        FastStage<VB == 4, BK_, TILE, NT> sb;
         sa.init(args.lda, m0, args.m, tid);
         sb.init(args.ldb, n0, args.n, tid, listed ? col_of : nullptr);
         int seg = it_begin / kt_per_seg, kin = it_begin % kt_per_seg, left = it_end - it_begin - 1;
         const float *pa = pb.A[seg], *pbb = pb.B[seg];
         const size_t ka = AK ? 1 : (size_t)args.lda, kb = BK_ ? 1 : (size_t)args.ldb;  // floats per k step
-        auto load_tile = [&](int it, StageA &qa, StageB &qb) __attribute__((always_inline)) {
-            const int s = it / kt_per_seg, at = it % kt_per_seg;
-            qa.load(pb.A[s] + (size_t)at * BK * ka, args.k - at * BK, tid);
-            qb.load(pb.B[s] + (size_t)at * BK * kb, args.k - at * BK, tid);
-        };
-        auto fetch_next = [&](StageA &qa, StageB &qb) __attribute__((always_inline)) {
+        auto fetch_next = [&](FastStage<VA == 4, AK, TILE, NT> &qa, FastStage<VB == 4, BK_, TILE, NT> &qb) __attribute__((always_inline)) {
             qa.load(pa + (size_t)kin * BK * ka, args.k - kin * BK, tid);
             qb.load(pbb + (size_t)kin * BK * kb, args.k - kin * BK, tid);
             if (left > 0) {
@@ -987,62 +682,46 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
                 }
             }
         };
-        run(sa, sb, fetch_next, load_tile);
+        run(sa, sb, fetch_next);
     }
 
-    const int lane_at = lane_asked_for_here(), thread = 64 * wave + lane_at;
-    const int row_at = lane_at & 31, half_at = lane_at >> 5;
     // what came out infinite or not a number is formed again (plain_sums)
 #pragma unroll
-    for (int j = 0; j < NBN; ++j) {
-        int exponent[16];
-        if constexpr (HALVES)
+    for (int i = 0; i < NBM; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) exponent[r] = -exponent_of_peak(peak[TILE + wn * WN + 32 * j + 8 * (r >> 2) + 4 * half_at + (r & 3)]);
-#pragma unroll
-        for (int i = 0; i < NBM; ++i) {
+        for (int j = 0; j < NBN; ++j) {
             bool finite = true;
-            int of_row = 0;
-            if constexpr (HALVES) {
-                of_row = exponent_of_peak(peak[wm * WM + 32 * i + row_at]);
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] += (1.0f / kHalfLow) * low[i][j][r];
-            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) finite = finite && __builtin_fabsf(acc[i][j][r]) <= lim::kMax;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                if constexpr (HALVES) acc[i][j][r] = __builtin_ldexpf(acc[i][j][r], exponent[r] - of_row);
-                else acc[i][j][r] *= 1.0f / (kSplitScale * kSplitScale);
-            }
+            for (int r = 0; r < 16; ++r) acc[i][j][r] *= 1.0f / (kSplitScale * kSplitScale);
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(!finite) != 0, 0))
-                acc[i][j] = plain_sums<AK, BK_, MASKED, GATHER>(args, pb, m0 + wm * WM + 32 * i, n0 + wn * WN + 32 * j, lane_at, it_begin,
+                acc[i][j] = plain_sums<AK, BK_, MASKED, GATHER>(args, pb, m0 + wm * WM + 32 * i, n0 + wn * WN + 32 * j, lane, it_begin,
                                                                 it_end, kt_per_seg, k_extent, k_lo);
         }
-    }
 
     // epilogue: lane%32 runs along m (contiguous), the 16 accumulators along n
     float *__restrict__ C = pb.C;
     if constexpr (!AK && !BK_ && !MASKED) {
         if (rowsum) {
             // the threads that loaded different k positions of the same rows add up through LDS, in a fixed order
-            constexpr int SHARES = BK / LB::NLOAD;
-            static_assert(SHARES * BN * sizeof(float) <= sizeof(lds), "the row sums fit the tile's buffer");
+            constexpr int PARTS = BK / LB::NLOAD;
+            static_assert(PARTS * BN * sizeof(float) <= sizeof(lds), "the row sums fit the tile's buffer");
             float *const sums = reinterpret_cast<float *>(lds);
             __syncthreads();
-            *reinterpret_cast<float4 *>(sums + LB::first_k(thread) / LB::NLOAD * BN + LB::first_row(thread)) = float4{rs[0], rs[1], rs[2], rs[3]};
+            *reinterpret_cast<float4 *>(sums + LB::first_k(tid) / LB::NLOAD * BN + LB::first_row(tid)) = float4{rs[0], rs[1], rs[2], rs[3]};
             __syncthreads();
-            if (thread < BN && n0 + thread < args.n) {
+            if (tid < BN && n0 + tid < args.n) {
                 float s = 0.0f;
 #pragma unroll
-                for (int q = 0; q < SHARES; ++q) s += sums[q * BN + thread];
+                for (int q = 0; q < PARTS; ++q) s += sums[q * BN + tid];
                 if (args.epilogue == EPI_PARTIAL)
                     args.partial[(size_t)split_id * args.partial_stride + (size_t)args.nprob * args.m * args.n +
-                                 (size_t)prob_id * args.n + n0 + thread] = s;
+                                 (size_t)prob_id * args.n + n0 + tid] = s;
                 else if (args.epilogue == EPI_STORE)
-                    pb.rowsum_out[n0 + thread] = pb.rowsum_scale * s;
+                    pb.rowsum_out[n0 + tid] = pb.rowsum_scale * s;
                 else
-                    atomicAdd(pb.rowsum_out + n0 + thread, pb.rowsum_scale * s);
+                    atomicAdd(pb.rowsum_out + n0 + tid, pb.rowsum_scale * s);
             }
         }
     }
@@ -1051,7 +730,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
         // cannot know that the buffers do not overlap and would otherwise wait for memory once per value.
 #pragma unroll
         for (int i = 0; i < NBM; ++i) {
-            const int m = m0 + wm * WM + i * 32 + row_at;
+            const int m = m0 + wm * WM + i * 32 + frag_row;
 #pragma unroll
             for (int j = 0; j < NBN; ++j) {
                 size_t idx[16];
@@ -1059,7 +738,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
                 float e[16], old[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int n = n0 + wn * WN + j * 32 + 8 * (r >> 2) + 4 * half_at + (r & 3);
+                    const int n = n0 + wn * WN + j * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
                     ok[r] = m < args.m && n < args.n;
                     idx[r] = ok[r] ? (size_t)n * args.ldc + m : 0;
                     old[r] = (ok[r] && pb.aux_in) ? pb.aux_in[idx[r]] : 0.0f;
@@ -1100,7 +779,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
         ldc = args.m;
     }
     const int wave_m = m0 + wm * WM, wave_n = wn * WN;  // the wave's first row, its first column inside the tile
-    auto in_tile = [&](int j, int r) __attribute__((always_inline)) { return wave_n + 32 * j + 8 * (r >> 2) + 4 * half_at + (r & 3); };
+    auto in_tile = [&](int j, int r) __attribute__((always_inline)) { return wave_n + 32 * j + 8 * (r >> 2) + 4 * half + (r & 3); };
     // the column of C for a column of the tile (clamped into the matrix)
     auto column = [&](int at) __attribute__((always_inline)) { return listed ? col_of[at] : min(n0 + at, args.n - 1); };
     auto all_sums = [&](auto &&step) __attribute__((always_inline)) {
@@ -1118,7 +797,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
     if (FORWARD && (epilogue == EPI_BIAS_ACT || epilogue == EPI_BIAS_ACT_SKIP)) {
 #pragma unroll
         for (int i = 0; i < NBM; ++i) {
-            const float bterm = args.bias_scale * pb.bias_vec[min(wave_m + 32 * i + row_at, args.m - 1)];
+            const float bterm = args.bias_scale * pb.bias_vec[min(wave_m + 32 * i + frag_row, args.m - 1)];
 #pragma unroll
             for (int j = 0; j < NBN; ++j)
 #pragma unroll
@@ -1134,7 +813,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
         for (int j = 0; j < NBN; ++j)
 #pragma unroll
             for (int i = 0; i < NBM; ++i) {
-                const int m = min(wave_m + 32 * i + row_at, args.m - 1);
+                const int m = min(wave_m + 32 * i + frag_row, args.m - 1);
                 float met[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) met[r] = old[(size_t)column(in_tile(j, r)) * ldc + m];
@@ -1161,28 +840,26 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
 #pragma unroll
                         for (int r = 0; r < 16; ++r) {
                             const int n = n0 + in_tile(j, r);
-                            if (n < args.n && wave_m + 32 * i + row_at < args.m) pb.aux_out[(size_t)n * ldc + m] = v[r];
+                            if (n < args.n && wave_m + 32 * i + frag_row < args.m) pb.aux_out[(size_t)n * ldc + m] = v[r];
                         }
 #pragma unroll
                     for (int r = 0; r < 16; ++r) v[r] = met[r];
                 }
             }
     }
-    // A wave whose sums all lie inside the matrix stores them through an offset per lane that moves along beside one uniform address (32 bits
-    // of it, so lines of less than 2^32 / (4 * TILE) values).
-    if (epilogue != EPI_ATOMIC && epilogue != EPI_BIAS_ACT_SKIP && !listed && wave_m + WM <= args.m && n0 + wave_n + WN <= args.n &&
-        ldc < (1 << 30) / TILE) {
-        const unsigned line = (unsigned)ldc * (unsigned)sizeof(float);
-        unsigned mine = (unsigned)(4 * half_at) * line + (unsigned)row_at * (unsigned)sizeof(float);
-        char *const at = reinterpret_cast<char *>(C + (size_t)(n0 + wave_n) * ldc + wave_m);
+    // A wave whose sums all lie inside the matrix stores them through one offset per lane beside an address per sum that is uniform.
+    if (epilogue != EPI_ATOMIC && epilogue != EPI_BIAS_ACT_SKIP && !listed && wave_m + WM <= args.m && n0 + wave_n + WN <= args.n) {
+        const unsigned mine = ((unsigned)(4 * half) * (unsigned)ldc + (unsigned)frag_row) * (unsigned)sizeof(float);
+        char *at = reinterpret_cast<char *>(C + (size_t)(n0 + wave_n) * ldc + wave_m);
+        const size_t line = (size_t)ldc * sizeof(float);
 #pragma unroll
         for (int j = 0; j < NBN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
 #pragma unroll
                 for (int i = 0; i < NBM; ++i) *reinterpret_cast<float *>(at + mine + 128 * i) = acc[i][j][r];
-                mine += (r & 3) == 3 ? 5 * line : line;
-                asm volatile("" : "+v"(mine));  // (one offset, not one per column)
+                at += (r & 3) == 3 ? 5 * line : line;
+                asm volatile("" : "+s"(at));  // (one address that moves along, not one per column)
             }
         return;
     }
@@ -1197,7 +874,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
         }
 #pragma unroll
         for (int i = 0; i < NBM; ++i) {
-            const int m = wave_m + 32 * i + row_at;
+            const int m = wave_m + 32 * i + frag_row;
             if (m >= args.m) continue;
             if (epilogue == EPI_ATOMIC) {
 #pragma unroll
@@ -1212,14 +889,6 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : TILE == 128 ? (PARTS =
     }
 }
 
-template <int VA, bool AK, int VB, bool BK_, int PARTS, bool GATHER>
-void launch_tile(const GemmArgs &a, dim3 grid, hipStream_t s, int tile) {
-    if (tile == kEightWaves)
-        hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128, PARTS, false, GATHER, 8>), grid, dim3(2 * NTHREADS), 0, s, a);
-    else if (PARTS == 3 && tile == 128)  // (pick_tile: not of two parts)
-        hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128, 3, false, GATHER>), grid, dim3(NTHREADS), 0, s, a);
-    else hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64, PARTS, false, GATHER>), grid, dim3(NTHREADS), 0, s, a);
-}
 template <int VA, bool AK, int VB, bool BK_>
 void launch_t(const GemmArgs &a, dim3 grid, hipStream_t s, int tile) {
     // gemm_launch has checked the operand kinds of the two special products and that they, and the masked one, come with
@@ -1227,20 +896,26 @@ void launch_t(const GemmArgs &a, dim3 grid, hipStream_t s, int tile) {
     if (a.epilogue == EPI_FAN) {
         if constexpr (VA == 4 && !AK && VB == 4 && BK_) {
             if (a.masked)
-                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, true, 64, 3, true>), grid, dim3(NTHREADS), 0, s, a);
+                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, true, 64, true>), grid, dim3(NTHREADS), 0, s, a);
             else
-                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64, 3, true>), grid, dim3(NTHREADS), 0, s, a);
+                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64, true>), grid, dim3(NTHREADS), 0, s, a);
         }
     } else if (a.k_order) {
         if constexpr (VA == 4 && !AK && VB == 4 && !BK_) {
-            if (a.halves) launch_tile<VA, AK, VB, BK_, 2, true>(a, grid, s, tile);
-            else launch_tile<VA, AK, VB, BK_, 3, true>(a, grid, s, tile);
+            if (tile == kEightWaves)
+                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128, false, true, 8>), grid, dim3(2 * NTHREADS), 0, s, a);
+            else if (tile == 128)
+                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128, false, true>), grid, dim3(NTHREADS), 0, s, a);
+            else
+                hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64, false, true>), grid, dim3(NTHREADS), 0, s, a);
         }
     } else if (a.masked) {
-        hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, true, 64, 3>), grid, dim3(NTHREADS), 0, s, a);
+        hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, true, 64>), grid, dim3(NTHREADS), 0, s, a);
     } else if constexpr (VA != 2 && VB != 2) {
-        if (a.halves) launch_tile<VA, AK, VB, BK_, 2, false>(a, grid, s, tile);
-        else launch_tile<VA, AK, VB, BK_, 3, false>(a, grid, s, tile);
+        if (tile == kEightWaves)
+            hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128, false, false, 8>), grid, dim3(2 * NTHREADS), 0, s, a);
+        else if (tile == 128) hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 128>), grid, dim3(NTHREADS), 0, s, a);
+        else hipLaunchKernelGGL((gemm_split_kernel<VA, AK, VB, BK_, false, 64>), grid, dim3(NTHREADS), 0, s, a);
     }
 }
 template <int VA, bool AK, int VB>

@@ -1138,7 +1138,6 @@ int cnt_lstm_forward(cnt_lstm *h, void *stream_, const float *weights, const flo
         }
     // (the recursion leaves padding slots out; what it finds there as pre-activations reaches nothing)
     ga.cols = h->slot_order.order; ga.cols_count = h->slot_order.count;
-    ga.halves = 1;
     ga.label = "gemm:lstm_input_projection";
     CNT_TRY(gemm_launch(stream, ga));
 
@@ -1250,7 +1249,6 @@ int cnt_lstm_backward_prev_errors_range(cnt_lstm *h, void *stream_, const float 
             }
         ga.prob[0].C = prev_errors + first * P;
         if (t_begin == 0 && t_end == h->T) { ga.cols = h->slot_order.order; ga.cols_count = h->slot_order.count; }  // (no deltas on padding)
-        ga.halves = 1;
         ga.label = "gemm:lstm_prev_errors";
         CNT_TRY(gemm_launch(stream, ga));
     }
@@ -1280,7 +1278,6 @@ extern "C++" int cnt::lstm_prev_errors_delta(cnt_lstm *h, hipStream_t stream, co
     ga.prob[0].C = prev_errors;
     ga.prob[0].aux_in = prev_y;
     ga.cols = h->slot_order.order; ga.cols_count = h->slot_order.count;
-    ga.halves = 1;
     ga.label = "gemm:lstm_prev_errors";
     return gemm_launch(stream, ga);
 }
@@ -1374,7 +1371,6 @@ extern "C++" int cnt::lstm_backward_weights_grouped(cnt_lstm *h, hipStream_t str
             ga.k_order = h->slot_order.order;
             ga.k_count = h->slot_order.count;
         }
-        ga.halves = 1;
         ga.label = "gemm:lstm_dW_input";
         ga.overwrite_ok = 1;  // the problems cover all input weights
         gemm_plan(ga, stream);
@@ -1408,7 +1404,6 @@ extern "C++" int cnt::lstm_backward_weights_grouped(cnt_lstm *h, hipStream_t str
             ga.k_order = h->slot_order.order;
             ga.k_count = h->slot_order.count;
         }
-        ga.halves = 1;
         ga.label = "gemm:lstm_dW_internal";
         ga.overwrite_ok = 1;  // the problems cover all recurrent weights
         gemm_plan(ga, stream);

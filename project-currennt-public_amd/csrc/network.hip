@@ -1730,15 +1730,6 @@ static bool has_weight_half(const cnt::NetLayer &L) {
     return L.kind == K_DENSE || L.kind == K_LSTM || L.kind == K_CNN || (L.kind == K_WAVNETC && L.ctx_dim > 0);
 }
 
-// Whether a layer's errors are of about one size along the slots and along its outputs.  A mixture's or a softmax's are not: a component
-// that explains no frame of a tile has errors of 1e-20 there and of 1 elsewhere.
-static bool even_errors(const cnt_network *net, size_t i) {
-    return i + 1 >= net->layers.size() || net->layers[i + 1].kind != cnt::K_MDN;
-}
-// The same of the operands of its weight gradient.  Behind a feedback layer the inputs are one-hot: two parts would look at all of them twice, since the
-// tiles that a row's size is taken from hold zeros (1024 inputs, 64 outputs, 32 000 samples: 59.7 us, three parts 47.1).
-static bool even_weights(const cnt_network *net, size_t i) { return even_errors(net, i) && net->layers[i - 1].kind != cnt::K_FEEDBACK; }
-
 // A small pass's weight halves stay on the caller's stream: a hop to another stream and back takes the host some 25 us and the
 // card 18, and in line the products of few blocks are one launch.  The line goes by the slots, beyond which those products are cut along k, and
 // by the multiply-adds of the weight gradients.  Us per pass on another stream / in line, slots in brackets.
@@ -1835,7 +1826,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         float *dW = net->updates + L.w_off;
         if (L.kind == K_DENSE) {
             const float *x = prev.out, *e = L.err;
-            return dense_backward_weights_batch(ws, prev.size, L.size, L.N, 1, &L.bias, &x, &e, &dW, &L.order, group, even_weights(net, i));
+            return dense_backward_weights_batch(ws, prev.size, L.size, L.N, 1, &L.bias, &x, &e, &dW, &L.order, group);
         }
         if (L.kind == K_LSTM) return lstm_backward_weights_grouped(L.lstm, ws, prev.out, dW, true, group);
         if (L.kind == K_CNN) return cnt_cnn_backward_weights(L.cnn, ws, L.pat, L.T, prev.out, L.err, dW);
@@ -1889,8 +1880,6 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         const float *colsum[kGemmMaxProb];
         int colsum_rows[kGemmMaxProb];
         const NetLayer &first = net->layers[g.layers[0]];
-        bool even = true;
-        for (size_t i : g.layers) even = even && even_weights(net, i);
         for (int z = 0; z < count; ++z) {
             NetLayer &L = net->layers[g.layers[(size_t)z]];
             NetLayer &prev = net->layers[g.layers[(size_t)z] - 1];
@@ -1903,7 +1892,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         }
         g.layers.clear();
         if (g.kind == K_DENSE)
-            return dense_backward_weights_batch(ws, g.a, g.b, g.n, count, bias, in0, in1, dW, &first.order, ws == stream ? &in_line : nullptr, even);
+            return dense_backward_weights_batch(ws, g.a, g.b, g.n, count, bias, in0, in1, dW, &first.order, ws == stream ? &in_line : nullptr);
         if (g.kind == K_CNN) return cnn_backward_weights_batch(cnn, count, ws, first.pat, first.T, in0, in1, dW, colsum, colsum_rows);
         return wavnetc_backward_weights_batch(ws, g.a, g.b, g.n, count, net->ctx, in0, dW);
     };
@@ -2090,7 +2079,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                         const bool below = !wanted && prev_err == prev.err && prev.N == N && delta_target(i - 1);
                         CNT_TRY(dense_backward_errors_fan(stream, prev.size, L.size, N, ACT_IDENTITY, W, L.out, L.err, prev_err,
                                                           wanted ? &fan : nullptr, &fused, below ? prev.act : ACT_IDENTITY,
-                                                          below ? prev.out : nullptr, &L.order, even_errors(net, i)));
+                                                          below ? prev.out : nullptr, &L.order));
                         if (below) delta_done[i - 1] = 1;
                         fan_done[i - 1] = fused ? 1 : 0;
                         break;
@@ -2099,8 +2088,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
                         const bool below = !wanted && prev_err && prev_err == prev.err && prev.N == N && delta_target(i - 1);
                         CNT_TRY(dense_backward_errors_fan(stream, prev.size, L.size, N, delta_done[i] ? ACT_IDENTITY : L.act, W,
                                                           L.out, L.err, prev_err, wanted ? &fan : nullptr, &fused,
-                                                          below ? prev.act : ACT_IDENTITY, below ? prev.out : nullptr, &L.order,
-                                                          even_errors(net, i)));
+                                                          below ? prev.act : ACT_IDENTITY, below ? prev.out : nullptr, &L.order));
                         if (below) delta_done[i - 1] = 1;
                     } else
                         CNT_TRY(cnn_backward_errors_fan(L.cnn, stream, L.pat, L.T, W, L.out, L.err, prev_err,
