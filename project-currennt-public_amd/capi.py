@@ -73,6 +73,7 @@ _SIGNATURES = {
     "cnt_probe_hop_message": (I, [VP, I, I, C.POINTER(F)]),
     "cnt_probe_activation": (I, [VP, I, C.c_long, VP, VP]),
     "cnt_probe_gemm_plan": (I, [I, I, I, I, I, I, I, C.POINTER(I)]),
+    "cnt_probe_halves_order": (I, [I, I, C.POINTER(I), I]),
     "cnt_gemm_reserve": (I, [VP]),
     "cnt_gemm_release": (I, [VP]),
     "cnt_gemm_scratch_buffers": (I, []),
@@ -262,6 +263,13 @@ def probe_gemm_plan(m, n, k, problems=1, a_kcontig=False, b_kcontig=False, weigh
     out = (C.c_int * 3)()
     check(lib().cnt_probe_gemm_plan(m, n, k, problems, int(a_kcontig), int(b_kcontig), int(weight_gradient), out))
     return tuple(out)
+
+
+def probe_halves_order(blocks, fails=-1):
+    """(whether it succeeded, the steps up to its return): see cnt_probe_halves_order."""
+    steps = (C.c_int * (3 * blocks + 1))()
+    status = lib().cnt_probe_halves_order(blocks, fails, steps, len(steps))
+    return status == 0, [s for s in steps if s >= 0]
 
 
 def gemm_reserve(stream=None):

@@ -1509,10 +1509,79 @@ bool block_weights_at(const cnt_network *net, size_t i) {
 // 808, 64 000 1777 / 1718; 32 and 64, 32 000 692 / 716, 48 000 1004 / 937; 64 and 256, 32 000 1485 / 1466.
 constexpr long kBlockHalves = 1L << 20;
 
+// The stream beside the caller's, as a pass uses it: handed work by fork(), behind all that the caller's stream has been given so far, and
+// waited for by join().  Whatever happens in between, a call that has handed work over does not return before the caller's stream waits for
+// it: what follows on that stream meets the same buffers, and a capture must not end with a stream that has not come back.
+template <typename STREAMS>
+class Beside {
+    STREAMS &streams;
+    bool away = false;
+
+public:
+    explicit Beside(STREAMS &streams_) : streams(streams_) {}
+    Beside(const Beside &) = delete;
+    Beside &operator=(const Beside &) = delete;
+    ~Beside() { if (away) (void)streams.join(); }
+    void handed() { away = true; }  // work that was ordered by other means
+    hipError_t fork() {
+        const hipError_t status = streams.fork();
+        if (status == hipSuccess) away = true;
+        return status;
+    }
+    hipError_t join() {
+        if (!away) return hipSuccess;
+        away = false;
+        return streams.join();
+    }
+};
+
+struct NetStreams {
+    const cnt_network *net;
+    hipStream_t caller, side;
+    hipError_t fork() {
+        const hipError_t status = hipEventRecord(net->ev_main, caller);
+        return status == hipSuccess ? hipStreamWaitEvent(side, net->ev_main, 0) : status;
+    }
+    hipError_t join() {
+        const hipError_t status = hipEventRecord(net->ev_side, side);
+        return status == hipSuccess ? hipStreamWaitEvent(caller, net->ev_side, 0) : status;
+    }
+};
+
+// The blocks from `first` on, each as launch(block, whether the later half): the later half behind the earlier half of the block in front.
+template <typename STREAMS, typename BEHIND, typename LAUNCH>
+int blocks_in_halves(STREAMS &streams, size_t first, BEHIND &&behind, LAUNCH &&launch) {
+    Beside<STREAMS> side(streams);
+    for (size_t at = first; at; at = behind(at)) {
+        CNT_HIP(side.fork());
+        CNT_TRY(launch(at, false));
+        CNT_TRY(launch(at, true));
+    }
+    CNT_HIP(side.join());
+    return CNT_OK;
+}
+
 }  // namespace
 }  // namespace cnt
 
 extern "C" {
+
+int cnt_probe_halves_order(int blocks, int fails, int *steps, int room) {
+    using namespace cnt;
+    CNT_REQUIRE(blocks >= 1 && steps && room >= 3 * blocks + 1, "probe_halves_order: bad argument");
+    struct Recorder {
+        int fails, count, *steps;
+        bool step(int what) {
+            steps[count] = what;
+            return count++ != fails;
+        }
+        hipError_t fork() { return step(0) ? hipSuccess : hipErrorUnknown; }
+        hipError_t join() { return step(3) ? hipSuccess : hipErrorUnknown; }
+    } log = {fails, 0, steps};
+    for (int k = 0; k < room; ++k) steps[k] = -1;
+    return blocks_in_halves(log, 1, [&](size_t at) { return at < (size_t)blocks ? at + 1 : 0; },
+                            [&](size_t, bool later) { return log.step(later ? 2 : 1) ? CNT_OK : CNT_ERR_STATE; });
+}
 
 int cnt_network_forward(cnt_network *net, void *stream_) {
     using namespace cnt;
@@ -1634,7 +1703,7 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
                         return block_at(at) && net->layers[at].N == N ? at : 0;
                     };
                     CNT_TRY(conditioning(i + 1));
-                    size_t next = behind(i);
+                    const size_t next = behind(i);
                     const hipStream_t side = next ? side_beside(net, stream, capturing(stream)) : nullptr;
                     if (!side) {
                         CNT_TRY(block_forward(stream, i, 0, N));
@@ -1643,16 +1712,13 @@ int cnt_network_forward(cnt_network *net, void *stream_) {
                     }
                     for (size_t at = next; at; at = behind(at)) CNT_TRY(conditioning(at + 1));
                     const int middle = (N / 2 + 63) / 64 * 64;
-                    for (size_t at = i; at; at = next) {
-                        next = behind(at);
-                        CNT_HIP(hipEventRecord(net->ev_main, stream));  // the earlier half of the block in front
-                        CNT_HIP(hipStreamWaitEvent(side, net->ev_main, 0));
-                        CNT_TRY(block_forward(stream, at, 0, middle));
-                        CNT_TRY(block_forward(side, at, middle, N));
-                        i = at + 5;
-                    }
-                    CNT_HIP(hipEventRecord(net->ev_side, side));
-                    CNT_HIP(hipStreamWaitEvent(stream, net->ev_side, 0));
+                    NetStreams streams = {net, stream, side};
+                    size_t last = i;
+                    CNT_TRY(blocks_in_halves(streams, i, behind, [&](size_t at, bool later) {
+                        last = at;
+                        return later ? block_forward(side, at, middle, N) : block_forward(stream, at, 0, middle);
+                    }));
+                    i = last + 5;
                     break;
                 }
                 CNT_TRY(cnt_cnn_forward(L.cnn, stream, L.pat, L.T, W, prev.out, L.out));
@@ -1768,7 +1834,6 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     CNT_TRY(report_failure(net, static_cast<hipStream_t>(stream_)));
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     const ScratchLoan loan(stream, net->main_scratch);
-    bool side_used = false;
     const bool captured = capturing(stream);  // (a graph's products take the scratch that the side streams have reserved)
     // Nothing runs on the caller's stream behind the error half of the lowest layer with weights, so its weight half, and what
     // is still waiting by then, stays there: two hops between streams (9 us each) less in front of the optimizer.
@@ -1816,6 +1881,8 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         if (block_at(i) && block_weights_at(net, i)) in_block[i] = in_block[i - 3] = in_block[i - 4] = in_block[i - 5] = 1;
     const hipStream_t side = net->overlap && (captured || !weights_in_line(net, in_block)) ? side_beside(net, stream, captured) : nullptr;
     const bool overlap = side != nullptr;
+    NetStreams streams = {net, stream, side};
+    Beside<NetStreams> beside(streams);
     std::vector<size_t> pending;
     DirectGroup in_line;  // products of few blocks on the caller's stream: one launch at the end of the pass
     in_line.count = in_line.blocks = 0;
@@ -1836,13 +1903,12 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     auto weight_stream = [&](hipStream_t *ws) -> int {
         *ws = at_end ? stream : side;
         if (at_end) return CNT_OK;
-        if (after_recursion) {
-            CNT_TRY(lstm_wait_recursion(after_recursion, *ws));
-        } else {
-            CNT_HIP(hipEventRecord(net->ev_main, stream));
-            CNT_HIP(hipStreamWaitEvent(*ws, net->ev_main, 0));
+        if (!after_recursion) {
+            CNT_HIP(beside.fork());
+            return CNT_OK;
         }
-        side_used = true;
+        CNT_TRY(lstm_wait_recursion(after_recursion, *ws));
+        beside.handed();
         return CNT_OK;
     };
     auto hand_over = [&]() -> int {
@@ -1939,9 +2005,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
         hipStream_t ws = stream;
         if (overlap) {  // always the one stream: the launches share their scratch
             ws = side;
-            CNT_HIP(hipEventRecord(net->ev_main, stream));
-            CNT_HIP(hipStreamWaitEvent(ws, net->ev_main, 0));
-            side_used = true;
+            CNT_HIP(beside.fork());
         }
         BlockGradients g[kBlockGradients];
         const NetLayer &first = net->layers[blocks[0]];
@@ -2216,10 +2280,7 @@ int cnt_network_backward(cnt_network *net, void *stream_) {
     CNT_TRY(hand_over());
     for (ShapeGroup &g : groups) CNT_TRY(hand_over_group(g));
     CNT_TRY(gemm_group_launch(stream, in_line));
-    if (side_used) {
-        CNT_HIP(hipEventRecord(net->ev_side, side));
-        CNT_HIP(hipStreamWaitEvent(stream, net->ev_side, 0));
-    }
+    CNT_HIP(beside.join());
     return CNT_OK;
 }
 
