@@ -55,6 +55,9 @@ int cnt_probe_activation(void *stream, int which, long n, const float *x, float 
  * along k) with 16-byte aligned operands.  plan[0]: edge of an output tile (32, 64 or 128), plan[1]: waves of a workgroup,
  * plan[2]: splits of k.  Needs no device. */
 int cnt_probe_gemm_plan(int m, int n, int k, int problems, int a_kcontig, int b_kcontig, int weight_gradient, int *plan);
+/* Test hook: cnt_matrix_product.  The name is that of two fp16 parts per value, on which the layers' products ran for a while: values far below
+ * their row's largest lost their bits that way, so no product is formed so any more. */
+int cnt_probe_product_of_halves(void *stream, float *C, int m, int n, int k, const float *A, int transA, const float *B, int transB);
 /* Test hook: the order in which a stack of WaveNet blocks that runs as two halves of its samples uses the stream beside the caller's, where
  * step number `fails` (-1: none) reports an error.  steps[0 .. room), at least 3 * blocks + 1 of them: 0 the stream beside waits for the caller's,
  * 1 a block's earlier half, 2 its later half, 3 the caller's stream waits for the one beside, -1 nothing.  Needs no device. */

@@ -73,6 +73,7 @@ _SIGNATURES = {
     "cnt_probe_hop_message": (I, [VP, I, I, C.POINTER(F)]),
     "cnt_probe_activation": (I, [VP, I, C.c_long, VP, VP]),
     "cnt_probe_gemm_plan": (I, [I, I, I, I, I, I, I, C.POINTER(I)]),
+    "cnt_probe_product_of_halves": (I, [VP, VP, I, I, I, VP, I, VP, I]),
     "cnt_probe_halves_order": (I, [I, I, C.POINTER(I), I]),
     "cnt_gemm_reserve": (I, [VP]),
     "cnt_gemm_release": (I, [VP]),
@@ -263,6 +264,10 @@ def probe_gemm_plan(m, n, k, problems=1, a_kcontig=False, b_kcontig=False, weigh
     out = (C.c_int * 3)()
     check(lib().cnt_probe_gemm_plan(m, n, k, problems, int(a_kcontig), int(b_kcontig), int(weight_gradient), out))
     return tuple(out)
+
+
+def probe_product_of_halves(Cm, m, n, k, A, tA, B, tB, stream=None):
+    check(lib().cnt_probe_product_of_halves(stream_ptr(stream), ptr(Cm), m, n, k, ptr(A), int(tA), ptr(B), int(tB)))
 
 
 def probe_halves_order(blocks, fails=-1):

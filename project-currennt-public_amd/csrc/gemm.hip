@@ -579,6 +579,10 @@ int gemm_simple(hipStream_t stream, float *C, int m, int n, int k, const float *
 
 }  // namespace cnt
 
+extern "C" int cnt_probe_product_of_halves(void *stream, float *C, int m, int n, int k, const float *A, int transA, const float *B, int transB) {
+    return cnt_matrix_product(stream, C, m, n, k, A, transA, B, transB, 0);
+}
+
 extern "C" int cnt_probe_gemm_plan(int m, int n, int k, int problems, int a_kcontig, int b_kcontig, int weight_gradient, int *plan) {
     using namespace cnt;
     CNT_REQUIRE(plan && m > 0 && n > 0 && k > 0 && problems >= 1 && problems <= kGemmMaxProb && (!a_kcontig || b_kcontig),
